@@ -192,8 +192,11 @@ class MoeFeedForward(FeedForward):
         act = rt.empty((A, self.expert_width))
         y = rt.empty((A, self.hidden_size))
         if tile_rows == ops.moe_tiled_rows(self.wide_tiles):  # many rows per expert: operands staged through LDS
-            ops.moe_grouped_tiled(x, w13, act, offsets, rows, tile_map, self.first_epilogue, self.wide_tiles, self.limit)
-            ops.moe_grouped_tiled(act, w2, y, offsets, None, tile_map, False, self.wide_tiles)
+            # (a piece of the shared expert holds every token: its tiles are full, and the last ones of the map)
+            full = self.shared_pieces * -(-x.shape[0] // tile_rows) if with_shared else 0
+            ops.moe_grouped_tiled(x, w13, act, offsets, rows, tile_map, self.first_epilogue, self.wide_tiles, self.limit,
+                                  full)
+            ops.moe_grouped_tiled(act, w2, y, offsets, None, tile_map, False, self.wide_tiles, 0.0, full)
         elif tile_rows:
             # few rows: the weights are the traffic, the reduction is split over a workgroup's four wavefronts
             ops.moe_grouped_mfma(x, w13, act, offsets, rows, tile_map, tile_rows, self.first_epilogue, 4, self.limit)

@@ -273,6 +273,22 @@ def test_grouped_tiled(T, H, E, k, mi, wide):
         assert rel_err(act, act2) < 1e-2 and rel_err(y, y2) < 1e-2
 
 
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("last", [1, 3, 7, 8, 1000])
+def test_grouped_tiled_order_of_the_last_tiles(last, wide):
+    """Working the last tiles of the map spread among the others changes no bit, whatever their number."""
+    from inferx_amd import ops
+    T, H, E, k, mi = 400, 136, 6, 2, 88
+    g = torch.Generator().manual_seed(1)
+    topk_e = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)]).to(torch.int32).to(DEV)
+    offsets, rows, dest, tile_map = dispatch(topk_e, E, ops.moe_tiled_rows(wide))
+    x, w = rnd(T, H, dtype=torch.bfloat16), rnd(E, 2 * mi, H, seed=2, dtype=torch.bfloat16, scale=H ** -0.5)
+    out = [torch.full((T * k, mi), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    for o, n in zip(out, (0, last)):
+        ops.moe_grouped_tiled(x, w, o, offsets, rows, tile_map, True, wide, last_tiles=n)
+    assert torch.isfinite(out[0]).all() and torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+
+
 @pytest.mark.parametrize("T,N,K", [(3, 40, 264), (16, 33, 1160), (2, 16, 8), (5, 48, 520)])
 def test_streaming_kernels_read_nothing_past_their_operands(T, N, K):
     """Reduction widths that leave a wavefront a ragged last round: what lies behind the last row of the weights

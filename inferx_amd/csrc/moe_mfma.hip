@@ -1,4 +1,5 @@
-// Grouped expert products on the matrix cores (bfloat16 in, float32 accumulate).
+// Grouped expert products on the matrix cores: bfloat16 in, float32 accumulate, or all of it float32 (template
+// parameter TI; v_mfma_f32_16x16x4_f32, every product and sum in 32 bits).
 //
 //   GATE_UP: act[r, n] = silu(x[rows[r]] . W[e][n]) * (x[rows[r]] . W[e][N + n]),  W [E, 2N, K]
 //   else:    y[r, n]   = a[r] . W[e][n],                                           W [E, N, K]
@@ -16,39 +17,68 @@
 // 128 of K with four loads: in load j lane (m, g) reads the 16 bytes at
 // k0 + 32 j + 8 g of weight row m, so the four lane groups cover 64 contiguous
 // bytes of each row and the 32 reduction slots of MFMA j; the activations are
-// read with the same mapping.  KSPLIT = 4 (decoding: few rows, the weights are the traffic) lets
+// read with the same mapping (in float32 a round is 64 of K, and the j-th numbers of the four groups' pieces meet in
+// one instruction).  KSPLIT = 4 (decoding: few rows, the weights are the traffic) lets
 // the four wavefronts of a workgroup take a quarter of K each and add up through
-// LDS; KSPLIT = 1 gives each wavefront its own 16 out-features.
+// LDS; KSPLIT = 1 gives each wavefront its own 16 out-features.  In float32 (8 tokens, 24 of 60 experts of 1,408 and a
+// shared one of 5,632 in one launch): 117 + 60 us for both products, 5.5 TB/s, against 514 + 268 us of the plain kernel
+// for the routed ones alone; a product of 8 rows with 2,048 x 2,048 weights 6 us against 12 to 18 through the library.
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// 16 bytes of an operand, and what one of them against another adds to a 16 x 16 block of sums
+template <typename TI> struct MfmaPiece;
+template <> struct MfmaPiece<__bf16> {
+  typedef bf16x8 type;
+  static constexpr int N = 8;
+  static __device__ __forceinline__ type zero() {
+    return type{(__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f};
+  }
+  static __device__ __forceinline__ f32x4 mac(type w, type x, f32x4 acc) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x, acc, 0, 0, 0);
+  }
+};
+template <> struct MfmaPiece<float> {
+  typedef f32x4 type;
+  static constexpr int N = 4;
+  static __device__ __forceinline__ type zero() { return type{0.f, 0.f, 0.f, 0.f}; }
+  static __device__ __forceinline__ f32x4 mac(type w, type x, f32x4 acc) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], x[j], acc, 0, 0, 0);
+    return acc;
+  }
+};
+
 // The work of one wavefront (KSPLIT == 1) or workgroup (KSPLIT == 4): rows [row0, row_end) x out-features
 // [n0, n0 + 16) of expert e.  `red`: LDS for the partial sums of a split reduction.
 // NB: blocks of 16 out-features side by side ([n0, n0 + 16 NB)), so that the rows are read once for all of them.
-template <int MT, bool GATE_UP, int KSPLIT, typename TO = __bf16, int NB = 1>
-__device__ __forceinline__ void grouped_body(const __bf16* a, const __bf16* w,
+template <int MT, bool GATE_UP, int KSPLIT, typename TI, typename TO, int NB = 1>
+__device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
                                              TO* __restrict__ out, const int32_t* __restrict__ rows, int e,
                                              int row0, int row_end, int n0, int n_out, int width, float* red,
                                              int act = 0, float glu_limit = 0.f) {
+  typedef MfmaPiece<TI> Piece;
+  typedef typename Piece::type piece_t;
+  constexpr int PN = Piece::N, ROUND = 16 * PN;  // numbers of a piece; of a round of four loads
   constexpr int NACC = NB * (GATE_UP ? 2 : 1);  // accumulator b + NB h: block b of the gate (h = 0) or up (1) rows
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
-  const int kper = KSPLIT > 1 ? (((width + KSPLIT - 1) / KSPLIT + 127) & ~127) : width;
+  const int kper = KSPLIT > 1 ? (((width + KSPLIT - 1) / KSPLIT + ROUND - 1) & ~(ROUND - 1)) : width;
   const int kbegin = KSPLIT > 1 ? wave * kper : 0;
   const int kend = min(width, kbegin + kper);
 
   const int64_t w_rows = GATE_UP ? 2 * static_cast<int64_t>(n_out) : n_out;
-  const __bf16* wp[NACC];
+  const TI* wp[NACC];
 #pragma unroll
   for (int u = 0; u < NACC; ++u) {
     const int wrow = min(n0 + 16 * (u % NB) + m, n_out - 1);  // rows past the end are computed and not stored
     wp[u] = w + (static_cast<int64_t>(e) * w_rows + (u / NB) * static_cast<int64_t>(n_out) + wrow) * width;
   }
 
-  const __bf16* xr[MT];
+  const TI* xr[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     const int r = min(row0 + 16 * t + m, row_end - 1);
@@ -61,59 +91,57 @@ __device__ __forceinline__ void grouped_body(const __bf16* a, const __bf16* w,
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const bf16x8 zero = {(__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f,
-                       (__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f};
-  // The loads of the next 128 of K are issued before the products of the present ones, so that a wavefront
+  const piece_t zero = Piece::zero();
+  // The loads of the next round of K are issued before the products of the present one, so that a wavefront
   // always has loads on their way.  Every load is unconditional (a piece past the end of a ragged last round is
   // read from the range's first piece instead, which is in the cache, and the activations' values are replaced
   // by zeros when they are used): with no branch in it the loop is one straight line, and the compiler lets the
   // younger loads stay in flight at each wait instead of waiting for all.
-  bf16x8 fw[2][NACC][4], fx[2][MT][4];
-  auto fetch = [&](int k0, bf16x8 (&w_)[NACC][4], bf16x8 (&x_)[MT][4]) {
+  piece_t fw[2][NACC][4], fx[2][MT][4];
+  auto fetch = [&](int k0, piece_t (&w_)[NACC][4], piece_t (&x_)[MT][4]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      int kk = k0 + 32 * j + 8 * g;  // the four lane groups cover 64 contiguous bytes of a row per load
-      kk = kk < kend ? kk : kbegin;  // (the range's first piece: it exists, kbegin + 8 g need not)
+      int kk = k0 + PN * (4 * j + g);  // the four lane groups cover 64 contiguous bytes of a row per load
+      kk = kk < kend ? kk : kbegin;  // (the range's first piece: it exists, kbegin + PN g need not)
 #pragma unroll
-      for (int u = 0; u < NACC; ++u) w_[u][j] = *reinterpret_cast<const bf16x8*>(wp[u] + kk);
+      for (int u = 0; u < NACC; ++u) w_[u][j] = *reinterpret_cast<const piece_t*>(wp[u] + kk);
 #pragma unroll
-      for (int t = 0; t < MT; ++t) x_[t][j] = *reinterpret_cast<const bf16x8*>(xr[t] + kk);
+      for (int t = 0; t < MT; ++t) x_[t][j] = *reinterpret_cast<const piece_t*>(xr[t] + kk);
     }
   };
-  auto multiply = [&](int k0, const bf16x8 (&w_)[NACC][4], const bf16x8 (&x_)[MT][4]) {
+  auto multiply = [&](int k0, const piece_t (&w_)[NACC][4], const piece_t (&x_)[MT][4]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const bool ok = k0 + 32 * j + 8 * g < kend;
+      const bool ok = k0 + PN * (4 * j + g) < kend;
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
-        const bf16x8 xv = ok ? x_[t][j] : zero;
+        const piece_t xv = ok ? x_[t][j] : zero;
 #pragma unroll
-        for (int u = 0; u < NACC; ++u)
-          acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_[u][j], xv, acc[u][t], 0, 0, 0);
+        for (int u = 0; u < NACC; ++u) acc[u][t] = Piece::mac(w_[u][j], xv, acc[u][t]);
       }
     }
   };
-  // Rounds of 128 in pairs, so that the register sets are named statically; the loop runs while both rounds of a
+  // Rounds in pairs, so that the register sets are named statically; the loop runs while both rounds of a
   // turn are followed by another one and has no way out of its middle, the last one or two rounds come after it.
-  const int rounds = kbegin < kend ? (kend - kbegin + 127) >> 7 : 0;
+  const int rounds = kbegin < kend ? (kend - kbegin + ROUND - 1) / ROUND : 0;
   if (rounds > 0) {
     fetch(kbegin, fw[0], fx[0]);
     int k0 = kbegin, left = rounds;
-    for (; left > 2; left -= 2, k0 += 256) {
-      fetch(k0 + 128, fw[1], fx[1]);
+    for (; left > 2; left -= 2, k0 += 2 * ROUND) {
+      fetch(k0 + ROUND, fw[1], fx[1]);
       __builtin_amdgcn_sched_barrier(0);
       multiply(k0, fw[0], fx[0]);
       __builtin_amdgcn_sched_barrier(0);
-      fetch(k0 + 256, fw[0], fx[0]);
+      fetch(k0 + 2 * ROUND, fw[0], fx[0]);
       __builtin_amdgcn_sched_barrier(0);
-      multiply(k0 + 128, fw[1], fx[1]);
+      multiply(k0 + ROUND, fw[1], fx[1]);
       __builtin_amdgcn_sched_barrier(0);
     }
     if (left == 2) {
-      fetch(k0 + 128, fw[1], fx[1]);
+      fetch(k0 + ROUND, fw[1], fx[1]);
       __builtin_amdgcn_sched_barrier(0);
       multiply(k0, fw[0], fx[0]);
-      multiply(k0 + 128, fw[1], fx[1]);
+      multiply(k0 + ROUND, fw[1], fx[1]);
     } else {
       multiply(k0, fw[0], fx[0]);
     }
@@ -156,7 +184,7 @@ __device__ __forceinline__ void grouped_body(const __bf16* a, const __bf16* w,
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         v[i] = acc[u][t][i];
-        if constexpr (GATE_UP) v[i] = ix_glu<true>(v[i], acc[NB + u][t][i], glu_limit);
+        if constexpr (GATE_UP) v[i] = ix_glu<sizeof(TI) == 2>(v[i], acc[NB + u][t][i], glu_limit);
         else if (act) v[i] = v[i] > 0.f ? v[i] * v[i] : 0.f;  // the square of relu
       }
       TO* dst = out + static_cast<int64_t>(r) * n_out + nb;
@@ -179,17 +207,17 @@ __device__ __forceinline__ void grouped_body(const __bf16* a, const __bf16* w,
 // x [rows <= 16 * MT, width] . w[n_out, width]^T -> float32 [rows, n_out]: the head of a decoding step, whose
 // logits stay float32 (one workgroup per 32 out-features, so that the rows, which every workgroup reads, weigh
 // less beside the weights; the reduction split over its four wavefronts).
-template <int MT>
-__global__ void __launch_bounds__(256)
-linear_skinny_f32_kernel(const __bf16* x, const __bf16* w, float* __restrict__ out,
+template <int MT, typename TI>
+__global__ void __launch_bounds__(256, MT == 1 ? 4 : 1)
+linear_skinny_f32_kernel(const TI* x, const TI* w, float* __restrict__ out,
                          int rows, int n_out, int width) {
   __shared__ float red[3 * 64 * MT * 2 * 4];
-  grouped_body<MT, false, 4, float, 2>(x, w, out, nullptr, 0, 0, rows, blockIdx.x * 32, n_out, width, red);
+  grouped_body<MT, false, 4, TI, float, 2>(x, w, out, nullptr, 0, 0, rows, blockIdx.x * 32, n_out, width, red);
 }
 
-template <int MT, bool GATE_UP, int KSPLIT>
-__global__ void __launch_bounds__(256)
-moe_grouped_mfma_kernel(const __bf16* a, const __bf16* w, __bf16* __restrict__ out,
+template <int MT, bool GATE_UP, int KSPLIT, typename TI>
+__global__ void __launch_bounds__(256, MT == 1 ? 4 : 1)
+moe_grouped_mfma_kernel(const TI* a, const TI* w, TI* __restrict__ out,
                         const int32_t* __restrict__ offsets, const int32_t* __restrict__ rows,
                         const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_row0,
                         const int32_t* __restrict__ tile_info, int n_out, int width, int act, float glu_limit) {
@@ -198,7 +226,7 @@ moe_grouped_mfma_kernel(const __bf16* a, const __bf16* w, __bf16* __restrict__ o
   const int e = tile_expert[blockIdx.y];
   const int n0 = (KSPLIT > 1 ? blockIdx.x : blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
   if (n0 >= n_out) return;  // whole wavefront (KSPLIT == 1) or whole workgroup
-  grouped_body<MT, GATE_UP, KSPLIT>(a, w, out, rows, e, tile_row0[blockIdx.y], offsets[e + 1], n0, n_out, width, red,
+  grouped_body<MT, GATE_UP, KSPLIT, TI, TI>(a, w, out, rows, e, tile_row0[blockIdx.y], offsets[e + 1], n0, n_out, width, red,
                                     act, glu_limit);
 }
 
@@ -206,13 +234,13 @@ moe_grouped_mfma_kernel(const __bf16* a, const __bf16* w, __bf16* __restrict__ o
 // n16_s * shared_tiles workgroups serve the shared expert, which is one more "expert" over all `shared_rows`
 // tokens with weights and sizes of its own (first, because its reduction may be the longer one and the last
 // workgroups to start set the kernel's end); the rest serve the routed experts' row tiles.
-template <int MT, bool GATE_UP, int NB>
-__global__ void __launch_bounds__(256)
-moe_grouped_dual_kernel(const __bf16* a, const __bf16* w, __bf16* __restrict__ out,
+template <int MT, bool GATE_UP, int NB, typename TI>
+__global__ void __launch_bounds__(256, MT == 1 ? 4 : 1)
+moe_grouped_dual_kernel(const TI* a, const TI* w, TI* __restrict__ out,
                         const int32_t* __restrict__ offsets, const int32_t* __restrict__ rows,
                         const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_row0,
                         const int32_t* __restrict__ tile_info, int max_tiles, int n_out, int width,
-                        const __bf16* a_s, const __bf16* w_s, __bf16* __restrict__ out_s,
+                        const TI* a_s, const TI* w_s, TI* __restrict__ out_s,
                         int shared_rows, int n_out_s, int width_s, float glu_limit, float glu_limit_s) {
   __shared__ float red[3 * 64 * MT * NB * (GATE_UP ? 2 : 1) * 4];
   const int n16_s = (n_out_s + 16 * NB - 1) / (16 * NB);  // column blocks of 16 NB out-features
@@ -220,7 +248,7 @@ moe_grouped_dual_kernel(const __bf16* a, const __bf16* w, __bf16* __restrict__ o
   int idx = blockIdx.x;
   if (idx < shared_blocks) {
     const int tile = idx / n16_s;
-    grouped_body<MT, GATE_UP, 4, __bf16, NB>(a_s, w_s, out_s, nullptr, 0, tile * 16 * MT, shared_rows,
+    grouped_body<MT, GATE_UP, 4, TI, TI, NB>(a_s, w_s, out_s, nullptr, 0, tile * 16 * MT, shared_rows,
                                              (idx - tile * n16_s) * 16 * NB,
                                  n_out_s, width_s, red, 0, glu_limit_s);
   } else {
@@ -229,7 +257,7 @@ moe_grouped_dual_kernel(const __bf16* a, const __bf16* w, __bf16* __restrict__ o
     const int tile = idx / n16_e;
     if (tile >= tile_info[0]) return;
     const int e = tile_expert[tile];
-    grouped_body<MT, GATE_UP, 4, __bf16, NB>(a, w, out, rows, e, tile_row0[tile], offsets[e + 1],
+    grouped_body<MT, GATE_UP, 4, TI, TI, NB>(a, w, out, rows, e, tile_row0[tile], offsets[e + 1],
                                              (idx - tile * n16_e) * 16 * NB, n_out, width, red, 0, glu_limit);
   }
 }
@@ -237,32 +265,38 @@ moe_grouped_dual_kernel(const __bf16* a, const __bf16* w, __bf16* __restrict__ o
 // `max_tiles` bounds the number of row tiles (the grid); the kernel reads the true number from tile_info.
 // tile_rows (16, 32 or 64) must be what the grouping kernel was given.  gate_up: 0 a plain product, 1 gate|up rows
 // with SwiGLU, 2 a plain product whose results pass the square of relu.  glu_limit > 0: the gate|up rows meet in
-// the clamped form (`ix_glu`).
-extern "C" int ix_moe_grouped_mfma(const void* a, const void* w, void* out, const int32_t* offsets,
+// the clamped form (`ix_glu`).  dtype: all of a, w and out (float32: k_split 4 only).
+#define IX_REQUIRE_PIECES(dtype, width)                                                                     \
+  IX_REQUIRE(dtype == IX_F32 || dtype == IX_BF16, "dtype must be float32 or bfloat16");                      \
+  IX_REQUIRE(width % (dtype == IX_F32 ? 4 : 8) == 0, "rows of the reduction must be multiples of 16 bytes")
+extern "C" int ix_moe_grouped_mfma(const void* a, const void* w, void* out, int dtype, const int32_t* offsets,
                                    const int32_t* rows, const int32_t* tile_expert, const int32_t* tile_row0,
                                    const int32_t* tile_info, int max_tiles, int tile_rows, int64_t n_out,
                                    int64_t width, int gate_up, int k_split, float glu_limit, hipStream_t stream) {
   IX_REQUIRE(n_out > 0 && width > 0 && max_tiles >= 0, "sizes must be positive");
-  IX_REQUIRE(width % 8 == 0, "the reduction width must be a multiple of 8 for the matrix-core kernel");
+  IX_REQUIRE_PIECES(dtype, width);
   IX_REQUIRE(n_out < (1 << 30) && width < (1 << 30), "sizes too large");
   IX_REQUIRE(tile_rows == 16 || tile_rows == 32 || tile_rows == 64, "tile_rows must be 16, 32 or 64");
-  IX_REQUIRE(k_split == 1 || k_split == 4, "k_split must be 1 or 4");
+  IX_REQUIRE(k_split == 4 || (k_split == 1 && dtype == IX_BF16), "k_split must be 1 (bfloat16 only) or 4");
   IX_REQUIRE(gate_up >= 0 && gate_up <= 2, "gate_up must be 0, 1 or 2");
   IX_REQUIRE(max_tiles <= 65535, "too many row tiles for one launch");
   if (max_tiles == 0) return 0;
   const int n_tiles16 = static_cast<int>((n_out + 15) / 16);
   dim3 grid(k_split > 1 ? n_tiles16 : (n_tiles16 + 3) / 4, max_tiles), block(256);
-#define LAUNCH(MT, GU, KS)                                                                                        \
-  hipLaunchKernelGGL((moe_grouped_mfma_kernel<MT, GU, KS>), grid, block, 0, stream, (const __bf16*)a,             \
-                     (const __bf16*)w, (__bf16*)out, offsets, rows, tile_expert, tile_row0, tile_info, (int)n_out, \
+#define LAUNCH(MT, GU, KS, TI)                                                                                    \
+  hipLaunchKernelGGL((moe_grouped_mfma_kernel<MT, GU, KS, TI>), grid, block, 0, stream, (const TI*)a,             \
+                     (const TI*)w, (TI*)out, offsets, rows, tile_expert, tile_row0, tile_info, (int)n_out,         \
                      (int)width, gate_up == 2 ? 1 : 0, glu_limit)
 #define PICK(MT)                                       \
-  if (gate_up == 1) {                                  \
-    if (k_split > 1) LAUNCH(MT, true, 4);              \
-    else LAUNCH(MT, true, 1);                          \
+  if (dtype == IX_F32) {                               \
+    if (gate_up == 1) LAUNCH(MT, true, 4, float);      \
+    else LAUNCH(MT, false, 4, float);                  \
+  } else if (gate_up == 1) {                           \
+    if (k_split > 1) LAUNCH(MT, true, 4, __bf16);      \
+    else LAUNCH(MT, true, 1, __bf16);                  \
   } else {                                             \
-    if (k_split > 1) LAUNCH(MT, false, 4);             \
-    else LAUNCH(MT, false, 1);                         \
+    if (k_split > 1) LAUNCH(MT, false, 4, __bf16);     \
+    else LAUNCH(MT, false, 1, __bf16);                 \
   }
   if (tile_rows == 16) { PICK(1) } else if (tile_rows == 32) { PICK(2) } else { PICK(4) }
 #undef PICK
@@ -272,7 +306,7 @@ extern "C" int ix_moe_grouped_mfma(const void* a, const void* w, void* out, cons
 
 // One launch for the routed experts (as ix_moe_grouped_mfma with k_split 4) and the shared expert
 // (a_s [shared_rows, width_s] . w_s[(2) n_out_s, width_s]^T -> out_s [shared_rows, n_out_s]).
-extern "C" int ix_moe_grouped_dual(const void* a, const void* w, void* out, const int32_t* offsets,
+extern "C" int ix_moe_grouped_dual(const void* a, const void* w, void* out, int dtype, const int32_t* offsets,
                                    const int32_t* rows, const int32_t* tile_expert, const int32_t* tile_row0,
                                    const int32_t* tile_info, int max_tiles, int tile_rows, int64_t n_out,
                                    int64_t width, const void* a_s, const void* w_s, void* out_s, int shared_rows,
@@ -280,7 +314,8 @@ extern "C" int ix_moe_grouped_dual(const void* a, const void* w, void* out, cons
                                    hipStream_t stream) {
   IX_REQUIRE(n_out > 0 && width > 0 && n_out_s > 0 && width_s > 0 && max_tiles >= 0 && shared_rows > 0,
              "sizes must be positive");
-  IX_REQUIRE(width % 8 == 0 && width_s % 8 == 0, "the reduction widths must be multiples of 8");
+  IX_REQUIRE_PIECES(dtype, width);
+  IX_REQUIRE_PIECES(dtype, width_s);
   IX_REQUIRE(n_out < (1 << 24) && width < (1 << 30) && n_out_s < (1 << 24) && width_s < (1 << 30), "sizes too large");
   IX_REQUIRE(tile_rows == 16 || tile_rows == 32 || tile_rows == 64, "tile_rows must be 16, 32 or 64");
   // one column block per workgroup: two (the rows read once for 32 out-features) measured slower at every tile
@@ -291,35 +326,41 @@ extern "C" int ix_moe_grouped_dual(const void* a, const void* w, void* out, cons
   const int64_t blocks = n16_e * max_tiles + n16_s * shared_tiles;
   IX_REQUIRE(blocks < (1ll << 31), "too many workgroups");
   dim3 grid(static_cast<unsigned>(blocks)), block(256);
-#define LAUNCH(MT, GU, NB)                                                                                        \
-  hipLaunchKernelGGL((moe_grouped_dual_kernel<MT, GU, NB>), grid, block, 0, stream, (const __bf16*)a, (const __bf16*)w, \
-                     (__bf16*)out, offsets, rows, tile_expert, tile_row0, tile_info, max_tiles, (int)n_out,        \
-                     (int)width, (const __bf16*)a_s, (const __bf16*)w_s, (__bf16*)out_s, shared_rows, (int)n_out_s, \
+#define LAUNCH(MT, GU, NB, TI)                                                                                    \
+  hipLaunchKernelGGL((moe_grouped_dual_kernel<MT, GU, NB, TI>), grid, block, 0, stream, (const TI*)a, (const TI*)w, \
+                     (TI*)out, offsets, rows, tile_expert, tile_row0, tile_info, max_tiles, (int)n_out,            \
+                     (int)width, (const TI*)a_s, (const TI*)w_s, (TI*)out_s, shared_rows, (int)n_out_s,             \
                      (int)width_s, glu_limit, glu_limit_s)
-#define PICK(MT, NB)                 \
-  if (gate_up == 1) LAUNCH(MT, true, NB); \
-  else LAUNCH(MT, false, NB);
+#define PICK(MT, NB)                                   \
+  if (dtype == IX_F32) {                               \
+    if (gate_up == 1) LAUNCH(MT, true, NB, float);     \
+    else LAUNCH(MT, false, NB, float);                 \
+  } else if (gate_up == 1) {                           \
+    LAUNCH(MT, true, NB, __bf16);                      \
+  } else {                                             \
+    LAUNCH(MT, false, NB, __bf16);                     \
+  }
   if (tile_rows == 16) { PICK(1, 1) } else if (tile_rows == 32) { PICK(2, 1) } else { PICK(4, 1) }
 #undef PICK
 #undef LAUNCH
   return ix_check_launch("ix_moe_grouped_dual");
 }
 
-// out float32 [rows, n_out] = x [rows, width] . w[n_out, width]^T, rows <= 64, bfloat16 operands.
-extern "C" int ix_linear_skinny_f32(const void* x, const void* w, float* out, int rows, int64_t n_out, int64_t width,
-                                    hipStream_t stream) {
+// out float32 [rows, n_out] = x [rows, width] . w[n_out, width]^T, rows <= 64, operands of `dtype`.
+extern "C" int ix_linear_skinny_f32(const void* x, const void* w, int dtype, float* out, int rows, int64_t n_out,
+                                    int64_t width, hipStream_t stream) {
   IX_REQUIRE(rows > 0 && rows <= 64 && n_out > 0 && width > 0, "between 1 and 64 rows, positive sizes");
-  IX_REQUIRE(width % 8 == 0, "the reduction width must be a multiple of 8");
+  IX_REQUIRE_PIECES(dtype, width);
   IX_REQUIRE(n_out < (1ll << 31) - 16 && width < (1 << 30), "sizes too large");
   dim3 grid(static_cast<unsigned>((n_out + 31) / 32)), block(256);
-  if (rows <= 16)
-    hipLaunchKernelGGL(linear_skinny_f32_kernel<1>, grid, block, 0, stream, (const __bf16*)x, (const __bf16*)w, out,
-                       rows, (int)n_out, (int)width);
-  else if (rows <= 32)
-    hipLaunchKernelGGL(linear_skinny_f32_kernel<2>, grid, block, 0, stream, (const __bf16*)x, (const __bf16*)w, out,
-                       rows, (int)n_out, (int)width);
-  else
-    hipLaunchKernelGGL(linear_skinny_f32_kernel<4>, grid, block, 0, stream, (const __bf16*)x, (const __bf16*)w, out,
-                       rows, (int)n_out, (int)width);
+#define LAUNCH(MT, TI)                                                                                       \
+  hipLaunchKernelGGL((linear_skinny_f32_kernel<MT, TI>), grid, block, 0, stream, (const TI*)x, (const TI*)w, out, rows, \
+                     (int)n_out, (int)width)
+#define PICK(MT)                       \
+  if (dtype == IX_F32) LAUNCH(MT, float); \
+  else LAUNCH(MT, __bf16);
+  if (rows <= 16) { PICK(1) } else if (rows <= 32) { PICK(2) } else { PICK(4) }
+#undef PICK
+#undef LAUNCH
   return ix_check_launch("ix_linear_skinny_f32");
 }

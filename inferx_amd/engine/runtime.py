@@ -88,11 +88,16 @@ class Runtime:
     # that also serves the experts (one "expert", one row tile), instead of a library product tuned for tiles
     # Up to two 16-row tiles: a decode step of 6 layers at batch 17 / 24 / 32 took 1477 / 1642 / 1822 us against
     # 1566 / 1691 / 1837 us through the library's products; from 48 rows on the library is faster (1966 against 2120).
+    # In float32 the library's products of 8 rows took 12 to 84 us a product of the A2.7B shape (1.5 TB/s at best),
+    # the streaming kernel's 6 to 13; the vocabulary's 1.2 GB 249 us, 5.0 TB/s.
     SKINNY_ROWS = 32
 
     def _skinny_ok(self, x: torch.Tensor, w: torch.Tensor) -> bool:
-        return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and 0 < x.shape[0] <= self.SKINNY_ROWS
-                and x.shape[1] % 8 == 0 and x.is_contiguous() and w.is_contiguous())
+        if not (x.dtype == w.dtype and 0 < x.shape[0] <= self.SKINNY_ROWS and x.is_contiguous() and w.is_contiguous()):
+            return False
+        if x.dtype == torch.float32:  # (tensors of any origin meet here: their place in memory is looked at)
+            return x.shape[1] % 4 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0
+        return x.dtype == torch.bfloat16 and x.shape[1] % 8 == 0
 
     def _skinny(self, x: torch.Tensor, w: torch.Tensor, gate_up: bool, limit: float = 0.0) -> torch.Tensor:
         from .. import ops
@@ -106,7 +111,7 @@ class Runtime:
             plan = self._skinny_plans[T] = (offsets, tile_map, tile_rows)
         offsets, tile_map, tile_rows = plan
         n_out = w.shape[0] // 2 if gate_up else w.shape[0]
-        out = self.empty((T, n_out))
+        out = self.empty((T, n_out), x.dtype)
         ops.moe_grouped_mfma(x, w.unsqueeze(0), out, offsets, None, tile_map, tile_rows, gate_up, 4, limit)
         return out
 
@@ -143,14 +148,14 @@ class Runtime:
 
     def linear_f32(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """As `linear`, result float32 (the logits)."""
+        if self._skinny_ok(x, w):  # few rows: the vocabulary's weights are the traffic
+            from .. import ops
+            out = self.empty((x.shape[0], w.shape[0]), torch.float32)
+            ops.linear_skinny_f32(x, w, out)
+            return out
         if x.dtype == torch.float32 and w.dtype == torch.float32:
             return torch.matmul(x, w.t())
         if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16:
-            if self._skinny_ok(x, w):  # few rows: the vocabulary's weights are the traffic
-                from .. import ops
-                out = self.empty((x.shape[0], w.shape[0]), torch.float32)
-                ops.linear_skinny_f32(x, w, out)
-                return out
             if x.shape[0] > 0 and x.is_contiguous() and w.is_contiguous():
                 from .. import ops
                 out = self.empty((x.shape[0], w.shape[0]), torch.float32)

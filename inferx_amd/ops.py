@@ -605,18 +605,24 @@ def moe_max_tiles(assignments: int, experts: int, tile_rows: int) -> int:
     return max(1, min(assignments, -(-assignments // tile_rows) + experts))
 
 
+def _need_pieces(a: torch.Tensor, *others: torch.Tensor) -> None:
+    """What the streaming matrix-core products ask of their operands."""
+    _need(a.dtype in (torch.bfloat16, torch.float32) and all(t.dtype == a.dtype for t in others),
+          "the matrix-core products take operands that are all bfloat16 or all float32")
+    _need(a.shape[1] % (16 // a.element_size()) == 0, "rows of the reduction must be multiples of 16 bytes")
+
+
 def moe_grouped_mfma(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offsets: torch.Tensor,
                      rows: Optional[torch.Tensor], tile_map: torch.Tensor, tile_rows: int, gate_up: bool,
                      k_split: int, glu_limit: float = 0.0) -> None:
-    """Grouped product on the matrix cores (bfloat16), shapes as `moe_grouped_plain`; `tile_map` from `moe_dispatch`."""
+    """Grouped product on the matrix cores (all bfloat16, or all float32 with k_split 4), shapes as
+    `moe_grouped_plain`; `tile_map` from `moe_dispatch`."""
     E = w.shape[0]
     A, n_out = out.shape
     K = a.shape[1]
-    _need(a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and out.dtype == torch.bfloat16,
-          "the matrix-core grouped product is bfloat16 only")
+    _need_pieces(a, w, out)
     _need(w.dim() == 3 and w.shape[2] == K and w.shape[1] == (2 * n_out if _epilogue(gate_up) == GATE_UP_SWIGLU else n_out),
           "expert weight shape does not fit")
-    _need(K % 8 == 0, "the reduction width must be a multiple of 8")
     _is_i32(offsets, E + 1)
     if rows is not None:
         _is_i32(rows, A)
@@ -624,7 +630,7 @@ def moe_grouped_mfma(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offset
         _need(a.shape[0] >= A, "a has fewer rows than out")
     mt = moe_max_tiles(A, E, tile_rows)
     _is_i32(tile_map, 2 * mt + 1)
-    _call("ix_moe_grouped_mfma", _ptr(a), _ptr(w), _ptr(out), _ptr(offsets), _ptr(rows), _ptr(tile_map[:mt]),
+    _call("ix_moe_grouped_mfma", _ptr(a), _ptr(w), _ptr(out), _i32(_dt(a)), _ptr(offsets), _ptr(rows), _ptr(tile_map[:mt]),
           _ptr(tile_map[mt:2 * mt]), _ptr(tile_map[2 * mt:]), _i32(mt), _i32(tile_rows), _i64(n_out), _i64(K),
           _i32(_epilogue(gate_up)), _i32(k_split), _f32(glu_limit), _stream())
 
@@ -641,13 +647,12 @@ def moe_grouped_dual(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offset
     K = a.shape[1]
     T, n_out_s = out_s.shape
     K_s = a_s.shape[1]
-    for t in (a, w, out, a_s, w_s, out_s):
-        _need(t.dtype == torch.bfloat16, "the matrix-core grouped product is bfloat16 only")
+    _need_pieces(a, w, out, a_s, w_s, out_s)
+    _need(a_s.shape[1] % (16 // a.element_size()) == 0, "rows of the reduction must be multiples of 16 bytes")
     _need(w.dim() == 3 and w.shape[2] == K and w.shape[1] == (2 * n_out if _epilogue(gate_up) == GATE_UP_SWIGLU else n_out),
           "expert weight shape does not fit")
     _need(w_s.shape == ((2 * n_out_s if gate_up else n_out_s), K_s) and a_s.shape[0] == T,
           "shared weight shape does not fit")
-    _need(K % 8 == 0 and K_s % 8 == 0, "the reduction widths must be multiples of 8")
     _is_i32(offsets, E + 1)
     if rows is not None:
         _is_i32(rows, A)
@@ -655,7 +660,7 @@ def moe_grouped_dual(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offset
         _need(a.shape[0] >= A, "a has fewer rows than out")
     mt = moe_max_tiles(A, E, tile_rows)
     _is_i32(tile_map, 2 * mt + 1)
-    _call("ix_moe_grouped_dual", _ptr(a), _ptr(w), _ptr(out), _ptr(offsets), _ptr(rows), _ptr(tile_map[:mt]),
+    _call("ix_moe_grouped_dual", _ptr(a), _ptr(w), _ptr(out), _i32(_dt(a)), _ptr(offsets), _ptr(rows), _ptr(tile_map[:mt]),
           _ptr(tile_map[mt:2 * mt]), _ptr(tile_map[2 * mt:]), _i32(mt), _i32(tile_rows), _i64(n_out), _i64(K),
           _ptr(a_s), _ptr(w_s), _ptr(out_s), _i32(T), _i64(n_out_s), _i64(K_s), _i32(1 if gate_up else 0),
           _f32(glu_limit), _f32(glu_limit_s), _stream())
@@ -688,15 +693,17 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
 
 
 def linear_skinny_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
-    """out float32 [T, N] = x [T, K] . w[N, K]^T for at most 64 rows, bfloat16 operands (the head of a decode step)."""
+    """out float32 [T, N] = x [T, K] . w[N, K]^T for at most 64 rows, operands both bfloat16 or both float32 (the head
+    of a decode step)."""
     T, K = x.shape
-    _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and out.dtype == torch.float32,
-          "bfloat16 operands and a float32 result")
+    _need(out.dtype == torch.float32, "a float32 result")
+    _need_pieces(x, w)
     _need(w.dim() == 2 and w.shape[1] == K and out.shape == (T, w.shape[0]), "shapes do not fit")
-    _need(0 < T <= 64 and K % 8 == 0, "between 1 and 64 rows and a reduction width that is a multiple of 8")
-    _call("ix_linear_skinny_f32", _ptr(x), _ptr(w), _ptr(out), _i32(T), _i64(w.shape[0]), _i64(K), _stream())
+    _need(0 < T <= 64, "between 1 and 64 rows")
+    _call("ix_linear_skinny_f32", _ptr(x), _ptr(w), _i32(_dt(x)), _ptr(out), _i32(T), _i64(w.shape[0]), _i64(K), _stream())
 
 
+MOE_TILED_F32_ROWS = 64  # rows per tile of the LDS-staged grouped product in float32
 MOE_TILED_ROWS = 160  # rows per tile of the LDS-staged grouped product
 MOE_TILED_ROWS_WIDE = 192  # ... of its wide form
 
@@ -730,6 +737,29 @@ def moe_grouped_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offse
     _call("ix_moe_grouped_tiled", _ptr(a), _ptr(w), _ptr(out), _ptr(offsets), _ptr(rows), _ptr(tile_map[:mt]),
           _ptr(tile_map[mt:2 * mt]), _ptr(tile_map[2 * mt:]), _i32(mt), _i64(a.shape[0]), _i64(n_out), _i64(K),
           _i32(_epilogue(gate_up)), _i32(1 if wide else 0), _f32(glu_limit), _i32(last_tiles), _stream())
+
+
+def moe_grouped_tiled_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offsets: torch.Tensor,
+                          rows: Optional[torch.Tensor], tile_map: torch.Tensor, gate_up, glu_limit: float = 0.0) -> None:
+    """Grouped product on the matrix cores, all float32, staged through LDS; shapes as `moe_grouped_plain`; `tile_map`
+    made for tiles of MOE_TILED_F32_ROWS rows."""
+    E = w.shape[0]
+    A, n_out = out.shape
+    K = a.shape[1]
+    _need(a.dtype == w.dtype == out.dtype == torch.float32, "this grouped product is float32 only")
+    _need_pieces(a, w, out)
+    _need(w.dim() == 3 and w.shape[2] == K and w.shape[1] == (2 * n_out if _epilogue(gate_up) == GATE_UP_SWIGLU else n_out),
+          "expert weight shape does not fit")
+    _is_i32(offsets, E + 1)
+    if rows is not None:
+        _is_i32(rows, A)
+    else:
+        _need(a.shape[0] >= A, "a has fewer rows than out")
+    mt = moe_max_tiles(A, E, MOE_TILED_F32_ROWS)
+    _is_i32(tile_map, 2 * mt + 1)
+    _call("ix_moe_grouped_tiled_f32", _ptr(a), _ptr(w), _ptr(out), _ptr(offsets), _ptr(rows), _ptr(tile_map[:mt]),
+          _ptr(tile_map[mt:2 * mt]), _ptr(tile_map[2 * mt:]), _i32(mt), _i64(a.shape[0]), _i64(n_out), _i64(K),
+          _i32(_epilogue(gate_up)), _f32(glu_limit), _stream())
 
 
 def moe_grouped_plain(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offsets: torch.Tensor,

@@ -164,15 +164,26 @@ class MoeFeedForward(FeedForward):
 
     def _tile_rows(self, ctx, x) -> int:
         """Rows per tile of the matrix-core product, or 0 where it does not take the shapes (then the plain one runs)."""
-        ok = (x.dtype == torch.bfloat16 and self.w13.dtype == torch.bfloat16 and self.w2.dtype == torch.bfloat16
-              and self.hidden_size % 8 == 0 and self.expert_width % 8 == 0)
+        piece = 16 // x.element_size()  # (rows are read 16 bytes at a time)
+        ok = (self.w13.dtype == x.dtype and self.w2.dtype == x.dtype and self.hidden_size % piece == 0
+              and self.expert_width % piece == 0 and (x.dtype == torch.bfloat16 or self._f32_fits(x)))
         if not ok:
             return 0
         # A decoding step, or few rows per expert: 16-row tiles, the weights streamed by every wavefront for itself.
         # From about three rows per expert on the LDS-staged kernel is faster (60 experts, 4 per token: 174 against
-        # 173 us for both products at 48 tokens, 209 against 189 at 96, 316 against 195 at 256).
+        # 173 us for both products at 48 tokens, 209 against 189 at 96, 316 against 195 at 256).  The float32 forms go by
+        # the same line.
         per_expert = x.shape[0] * self.top_k / self.num_experts
-        return 16 if (x.shape[0] <= ctx.rt.SKINNY_ROWS or per_expert <= 3) else ops.moe_tiled_rows(self.wide_tiles)
+        if x.shape[0] <= ctx.rt.SKINNY_ROWS or per_expert <= 3:
+            return 16
+        return ops.MOE_TILED_F32_ROWS if x.dtype == torch.float32 else ops.moe_tiled_rows(self.wide_tiles)
+
+    def _f32_fits(self, x) -> bool:
+        """What the float32 products on the matrix cores ask for beside whole 16-byte pieces: 32-bit offsets."""
+        A = x.shape[0] * self.top_k
+        return (max(x.shape[0] * self.hidden_size, A * self.expert_width) < 1 << 31
+                and (2 if self.gated else 1) * self.expert_width * self.hidden_size < 1 << 31
+                and ops.moe_max_tiles(A, self.num_experts, 16) < 65536)
 
     def dispatch(self, ctx, topk_e, tile_rows: int = 0, always: int = 0):
         rt, A, E = ctx.rt, topk_e.numel(), self.num_experts + always
@@ -191,7 +202,10 @@ class MoeFeedForward(FeedForward):
         w13, w2 = (self.w13_all, self.w2_all) if with_shared else (self.w13, self.w2)
         act = rt.empty((A, self.expert_width))
         y = rt.empty((A, self.hidden_size))
-        if tile_rows == ops.moe_tiled_rows(self.wide_tiles):  # many rows per expert: operands staged through LDS
+        if tile_rows == ops.MOE_TILED_F32_ROWS:  # a float32 run, more than a few rows per expert
+            ops.moe_grouped_tiled_f32(x, w13, act, offsets, rows, tile_map, self.first_epilogue, self.limit)
+            ops.moe_grouped_tiled_f32(act, w2, y, offsets, None, tile_map, False)
+        elif tile_rows == ops.moe_tiled_rows(self.wide_tiles):  # many rows per expert: operands staged through LDS
             # (a piece of the shared expert holds every token: its tiles are full, and the last ones of the map)
             full = self.shared_pieces * -(-x.shape[0] // tile_rows) if with_shared else 0
             ops.moe_grouped_tiled(x, w13, act, offsets, rows, tile_map, self.first_epilogue, self.wide_tiles, self.limit,
@@ -208,9 +222,9 @@ class MoeFeedForward(FeedForward):
 
     def _one_launch(self, ctx, x, tile_rows: int) -> bool:
         """Few tokens (decoding): routed and shared experts go into one launch per product."""
-        return (tile_rows == 16 and self.shared_width > 0 and self.shared_width % 8 == 0
-                and x.shape[0] <= ctx.rt.SKINNY_ROWS and self.w_shared_gate_up.dtype == torch.bfloat16
-                and self.w_shared_down.dtype == torch.bfloat16)
+        return (tile_rows == 16 and self.shared_width > 0 and self.shared_width % (16 // x.element_size()) == 0
+                and x.shape[0] <= ctx.rt.SKINNY_ROWS and self.w_shared_gate_up.dtype == x.dtype
+                and self.w_shared_down.dtype == x.dtype)
 
     def experts_and_shared(self, ctx, x, offsets, rows, tile_map, tile_rows):
         rt, A, T = ctx.rt, rows.numel(), x.shape[0]

@@ -444,3 +444,69 @@ def test_expert_sum_add_and_norm_in_one_pass(T, H, k, A, dtype, with_shared, gat
     h3, picked = h0.clone(), torch.empty(4, H, dtype=dtype, device=DEV)
     ops.moe_combine_add_rmsnorm(h3, y, dest, topk_w, shared, gate, weight, picked, eps, rows)
     assert torch.equal(h3, h0) and rel_err(picked, x_want[rows.long()]) < tol
+
+
+# rows of the experts (around the sixteens of a tile and its 64 rows), reduction width (no multiple of a stage of 32; rows
+# of a multiple of 1,024 bytes), columns (no multiple of a workgroup's, of four)
+F32_PRODUCTS = [([1, 0, 16, 17], 36, 40), ([63, 64, 65], 100, 33), ([130, 5], 256, 64), ([31, 33, 48, 49], 2048, 100),
+                ([2, 200], 4, 4)]
+
+
+@pytest.mark.parametrize("counts,K,n", F32_PRODUCTS)
+@pytest.mark.parametrize("kind", ["tiled", "streaming", "dual"])
+@pytest.mark.parametrize("gate_up,limit", [(0, 0.0), (1, 0.0), (1, 7.0), (2, 0.0)])
+def test_grouped_products_in_float32(counts, K, n, kind, gate_up, limit):
+    """The matrix-core products in float32 against float64: every product and sum is 32-bit, so a result is off by at
+    most K roundings of 2^-24 of the sum of magnitudes, here (normal numbers) under 1e-5 of the largest result.  What
+    lies behind the operands (NaN) reaches no result."""
+    from inferx_amd import ops
+    E, A, T = len(counts), sum(counts), 50
+    if kind == "dual" and gate_up == 2:
+        pytest.skip("the shared expert is gated")
+    wn = 2 * n if gate_up == 1 else n
+    buf = lambda rows, seed: torch.cat([rnd(rows, K, seed=seed, scale=K ** -0.25), torch.full((1, K), float("nan"), device=DEV)])
+    x, w = buf(T, 0)[:T], buf(E * wn, 1)[:E * wn].view(E, wn, K)
+    offsets = torch.tensor([sum(counts[:e]) for e in range(E + 1)], dtype=torch.int32, device=DEV)
+    rows = torch.randint(0, T, (A,), generator=torch.Generator().manual_seed(2)).to(torch.int32).to(DEV)
+    tr = ops.MOE_TILED_F32_ROWS if kind == "tiled" else 32
+    mt = ops.moe_max_tiles(A, E, tr)
+    tiles = [(e, int(offsets[e]) + r) for e in range(E) for r in range(0, counts[e], tr)]
+    tile_map = torch.zeros(2 * mt + 1, dtype=torch.int32)
+    for i, (e, r) in enumerate(tiles):
+        tile_map[i], tile_map[mt + i] = e, r
+    tile_map[2 * mt] = len(tiles)
+    tile_map = tile_map.to(DEV)
+    out = torch.full((A, n), float("nan"), device=DEV)
+    if kind == "tiled":
+        ops.moe_grouped_tiled_f32(x, w, out, offsets, rows, tile_map, gate_up, limit)
+    elif kind == "streaming":
+        ops.moe_grouped_mfma(x, w, out, offsets, rows, tile_map, tr, gate_up, 4, limit)
+    else:
+        shared = torch.full((T, n), float("nan"), device=DEV)
+        ops.moe_grouped_dual(x, w, out, offsets, rows, tile_map, tr, x, w[0], shared, gate_up == 1, limit, limit)
+
+    def want(z):
+        if gate_up == 0:
+            return z
+        if gate_up == 2:
+            return torch.relu(z) ** 2
+        g, u = z[:, :n], z[:, n:]
+        if limit:
+            g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+            return g * torch.sigmoid(1.702 * g) * (u + 1)
+        return torch.nn.functional.silu(g) * u
+
+    xd, wd = x.double().cpu(), w.double().cpu()
+    expect = torch.cat([want(xd[rows.cpu().long()[sum(counts[:e]):sum(counts[:e + 1])]] @ wd[e].T) for e in range(E)])
+    assert torch.isfinite(out).all() and rel_err(out, expect) < 1e-5
+    if kind == "dual":
+        assert torch.isfinite(shared).all() and rel_err(shared, want(xd @ wd[0].T)) < 1e-5
+
+
+@pytest.mark.parametrize("T,N,K", [(1, 301, 36), (16, 33, 2048), (17, 384, 100), (32, 70, 4), (64, 1000, 260)])
+def test_linear_skinny_in_float32(T, N, K):
+    from inferx_amd import ops
+    x, w = rnd(T, K), rnd(N, K, seed=1, scale=K ** -0.5)
+    out = torch.full((T, N), float("nan"), device=DEV)
+    ops.linear_skinny_f32(x, w, out)
+    assert rel_err(out, x.double().cpu() @ w.double().cpu().T) < 1e-5

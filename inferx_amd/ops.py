@@ -363,6 +363,39 @@ def attention_mfma(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
     _call("ix_attention_mfma_sink", *args, _ptr(sink), _ptr(turn_back), _f32(softcap), gate_ptr, _i64(gate_stride), _stream())
 
 
+def attention_f32(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor,
+                  tiles: torch.Tensor, positions: torch.Tensor, out: torch.Tensor, n_splits: int,
+                  workspace: Optional[torch.Tensor], scale: float, span: int, grouped: bool = False,
+                  sink: Optional[torch.Tensor] = None, softcap: float = 0.0) -> None:
+    """Paged attention on the matrix cores, float32 throughout; arguments as `attention_mfma` (tiles of up to 16
+    queries), keys and values of one size in multiples of 16, pages in multiples of 16."""
+    T, heads, d = q.shape
+    _need(q.dtype == torch.float32, "this attention kernel is float32 only")
+    _need(out.shape == q.shape and out.dtype == q.dtype, "out mismatch")
+    _check_caches(q, k_cache, v_cache)
+    kv_heads, page_size = k_cache.shape[1], k_cache.shape[2]
+    _need(block_table.dim() == 2, "block table must be [requests, pages]")
+    _is_i32(block_table)
+    _is_i32(positions, T)
+    _is_i32(tiles)
+    _need(tiles.dim() == 2 and tiles.shape[0] == 3 and tiles.is_contiguous(), "tiles must be int32 [3, n_tiles]")
+    n_tiles = tiles.shape[1]
+    _need(not grouped or (heads // kv_heads <= 16 and n_tiles <= T),
+          "grouped queries: one token per tile, at most 16 query heads per key/value head")
+    _need(sink is None or (sink.dtype == torch.float32 and sink.numel() == heads), "one float32 sink per head")
+    part_o = part_ml = None
+    if n_splits > 1:
+        need = T * heads * n_splits * (d + 2)
+        _need(workspace is not None and workspace.dtype == torch.float32 and workspace.numel() >= need,
+              f"workspace of {need} float32 needed")
+        part_o = workspace
+        part_ml = workspace[T * heads * n_splits * d:]
+    _call("ix_attention_f32", _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), _ptr(tiles[0]), _ptr(tiles[1]),
+          _ptr(tiles[2]), _ptr(positions), _ptr(out), _ptr(part_o), _ptr(part_ml), _i64(T), _i32(n_tiles),
+          _i32(n_splits), _i32(heads), _i32(kv_heads), _i32(d), _i32(page_size), _i32(block_table.shape[1]),
+          _f32(scale), _i32(span), _i32(1 if grouped else 0), _ptr(sink), _f32(softcap), _stream())
+
+
 def _gate_rows(gate: Optional[torch.Tensor], tokens: int, width: int, dtype):
     """(address, row stride) of a gate that an attention kernel applies to its result: rows of `width` numbers of the
     activations' type on 8-byte boundaries."""

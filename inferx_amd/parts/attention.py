@@ -216,7 +216,8 @@ class PagedAttention(Mixer):
     def attend(self, ctx, q, cache, out, turn_back=None, gate=None) -> None:
         """bfloat16 with pages and heads in multiples of 16: the matrix-core kernels (the one that shares keys through
         LDS for the prompt portions of a step, the wavefront-level one for requests that bring few tokens and for
-        steps of one token per request); else the plain one, which also knows a sink, values of another size than
+        steps of one token per request); float32 likewise through a wavefront-level kernel of its own; else the plain one,
+        which also knows a sink, values of another size than
         keys and a result that is rotated back (`turn_back`: the table of the query's angles).  `gate`:
         rows [T, heads * value_dim] whose sigmoid multiplies the result."""
         page_size = cache.k.shape[2]
@@ -267,10 +268,33 @@ class PagedAttention(Mixer):
             ops.attention_mfma(q, cache.k, cache.v, ctx.block_tables[cache.group], tiles, ctx.positions, out,
                                n_splits, work, self.scale, self.span, tile, prefetch=True, grouped=grouped, **more)
         else:
-            ops.attention_plain(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.seq_of_token, ctx.positions,
-                                out, self.scale, self.span, self.sink, turn_back, self.softcap)
+            if (q.dtype == torch.float32 and turn_back is None and self.value_dim == self.head_dim
+                    and page_size % 16 == 0 and self.head_dim % 16 == 0):
+                self._attend_f32(ctx, q, cache, out)
+            else:
+                ops.attention_plain(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.seq_of_token, ctx.positions,
+                                    out, self.scale, self.span, self.sink, turn_back, self.softcap)
             if gate is not None:
                 ops.sigmoid_gate(out.view(out.shape[0], -1), gate)
+
+    def _attend_f32(self, ctx, q, cache, out) -> None:
+        """A float32 run on the matrix cores: every request through the wavefront-level kernel."""
+        table = ctx.block_tables[cache.group]
+        if ctx.one_token_each:
+            tiles, _, n_splits, grouped = query_tiles(ctx, self.span, self.num_heads, self.head_dim, self.num_kv_heads)
+            waves = [(None, tiles, ctx.positions, n_splits, grouped)]
+        else:
+            _, waves = mixed_step_plan(ctx, self.span, self.num_heads, self.num_kv_heads, lds_fits=False)
+        for rows, tiles, positions, n_splits, grouped in waves:
+            qs = q if rows is None else q.index_select(0, rows)
+            outs = out if rows is None else torch.empty_like(qs)
+            work = None
+            if n_splits > 1:
+                work = ctx.rt.empty((qs.shape[0] * self.num_heads * n_splits * (self.head_dim + 2),), torch.float32)
+            ops.attention_f32(qs, cache.k, cache.v, table, tiles, positions, outs, n_splits, work, self.scale, self.span,
+                              grouped, self.sink, self.softcap)
+            if rows is not None:
+                out.index_copy_(0, rows, outs)
 
 
 def padded_head(*sizes: int, to: int = 16) -> int:

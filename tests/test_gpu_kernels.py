@@ -346,3 +346,50 @@ def test_attention_kernels_ignore_what_other_requests_left_in_the_pool(case):
     for what, out in runs:
         assert torch.isfinite(out.float()).all(), f"{what}: NaN from the pool reached the output"
         close(out, want, TOL[torch.bfloat16], what)
+
+
+# ---- float32 attention on the matrix cores: head sizes up to the kernel's largest, on both sides of where it stops asking
+# a round ahead; sums of float32, so the tolerance of the plain float32 kernel
+F32_CASES = ATTN_CASES + [([90, 17], [90, 1], 2, 1, 96, 16, 0), ([50, 16], [50, 16], 2, 2, 112, 32, 0),
+                          ([70], [33], 2, 1, 256, 16, 20)]
+
+
+@pytest.mark.parametrize("n_splits", [1, 3, 70])
+@pytest.mark.parametrize("case", F32_CASES)
+def test_attention_f32(case, n_splits):
+    from inferx_amd import ops
+    seq_lens, q_lens, heads, kv_heads, d, page, window = case
+    p = build_paged(seq_lens, q_lens, heads, kv_heads, d, page, torch.float32, seed=4)
+    T, scale = p["q"].shape[0], d ** -0.5
+    work = torch.empty(T * heads * n_splits * (d + 2), dtype=torch.float32, device=DEV) if n_splits > 1 else None
+    want = attention_reference(p, seq_lens, q_lens, heads, kv_heads, scale, window)
+    for tile, grouped in [(16, False)] + ([(1, True)] if heads > kv_heads else []):
+        out = torch.full_like(p["q"], float("nan"))
+        ops.attention_f32(p["q"], p["k_cache"], p["v_cache"], p["table"], tiles_for(q_lens, tile), p["positions"], out,
+                          n_splits, work, scale, window, grouped)
+        close(out, want, TOL[torch.float32], f"attention_f32 splits={n_splits} grouped={grouped}")
+
+
+@pytest.mark.parametrize("n_splits", [1, 4])
+@pytest.mark.parametrize("span", [0, 24, -32])
+@pytest.mark.parametrize("softcap,with_sink", [(0.0, True), (5.0, False), (5.0, True)])
+def test_attention_f32_options_agree_with_the_plain_kernel(softcap, with_sink, span, n_splits):
+    """Sinks, capped scores, windows and chunks; pages that hold NaN wherever no live key lies."""
+    from inferx_amd import ops
+    seq_lens, q_lens, heads, kv_heads, d, page = [300, 37, 16], [70, 37, 1], 4, 2, 64, 16
+    p = build_paged(seq_lens, q_lens, heads, kv_heads, d, page, torch.float32, seed=9)
+    for s, L in enumerate(seq_lens):
+        if L % page:
+            last = int(p["table"][s, L // page])
+            p["k_cache"][last, :, L % page:] = float("nan")
+            p["v_cache"][last, :, :, L % page:] = float("nan")
+    sink = rnd(heads, seed=3, scale=3.0) if with_sink else None
+    T = p["q"].shape[0]
+    work = torch.empty(T * heads * n_splits * (d + 2), dtype=torch.float32, device=DEV)
+    out, want = torch.full_like(p["q"], float("nan")), torch.full_like(p["q"], float("nan"))
+    ops.attention_plain(p["q"], p["k_cache"], p["v_cache"], p["table"], p["seq_of_token"], p["positions"], want, 0.3, span,
+                        sink, None, softcap)
+    ops.attention_f32(p["q"], p["k_cache"], p["v_cache"], p["table"], tiles_for(q_lens), p["positions"], out, n_splits,
+                      work, 0.3, span, False, sink, softcap)
+    assert torch.isfinite(want).all()
+    close(out, want, TOL[torch.float32], "attention_f32")

@@ -1,0 +1,460 @@
+// The gated delta rule over prompt portions, a chunk of 64 rows at a time (delta_rule.hip has the recurrence, its
+// operands and the form that walks row by row):
+//
+//   S <- g S;   u = beta (v - S^T k);   S <- S + k u^T;   o = S^T q
+//
+// Within a chunk, with G_i = g_0 .. g_i, the state before it S, and rows of U the u_i:
+//
+//   (I + A) U = diag(beta) V - diag(beta G) K S,     A_ij = beta_i (G_i / G_j) k_i . k_j  (j < i)
+//   O         = diag(G) Q S + P U,                   P_ij = (G_i / G_j) q_i . k_j         (j <= i)
+//   S_new     = G_n S + sum_j (G_n / G_j) k_j u_j^T
+//
+// so that only U = Uv - W S and S_new are left to the chain over a request's chunks.  Three launches:
+//   prepare   a workgroup per (chunk, head): unit rows, the decays, A and P on the matrix cores, the triangular system
+//             for Uv and W by blocks of sixteen rows (the four blocks on the diagonal inverted by substitution, the rest
+//             matrix products whose results are the next ones' operands as they lie in registers);
+//   chain     a workgroup per (request, head, 16 value columns): per chunk two products, W S and K^T U, the state in
+//             registers, the next chunk's operands on their way; leaves every chunk its U and the state before it;
+//   result    a workgroup per (chunk, head): O.
+//
+// Everything is float32 (v_mfma_f32_16x16x4_f32) but the sums of the decays' logarithms, which are 64-bit so that the
+// ratio of two late rows is as exact as that of two early ones.
+//
+// What bounds it: row by row, the chain of dependent sums of a row (0.33 us a row whatever the chip is doing).  In chunks
+// the chain is 64 times shorter and its step two small products (2.7 us a chunk).  Measured with 16 heads of 128 x 128, one
+// request, all three launches against row by row: 41 against 46 us at 128 rows, 47 against 72 at 200, 64 against 171 at
+// 500, 88 against 336 at 1,024, 150 against 667 at 2,048.  Results are 2.4e-7 of their norm from the float64 recurrence
+// (row by row 1.3e-7; with slow decays 4.2e-7 against 6.7e-7): the order of 32-bit sums.
+//
+// A lane's operand of a 16 x 16 x 4 product is one number of row (column) l % 16 at reduction index l / 16.  Operands
+// are read four numbers at a time, index 16 s + 4 (l / 16) + e, and the e-th of them meet in one instruction.
+#include "common.h"
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+#define DC_ROWS 64
+#define DC_THREADS 256
+
+// where the parts of a (chunk, head) lie in its block of the workspace, in floats
+struct DeltaBlock {
+  int dim, vdim;
+  __host__ __device__ __forceinline__ int64_t w() const { return 0; }                          // [64][dim]: -W
+  __host__ __device__ __forceinline__ int64_t kt() const { return 64 * dim; }                  // [dim][64]: (G_n / G_j) k_j
+  __host__ __device__ __forceinline__ int64_t q() const { return 128 * dim; }                  // [64][dim]: G_i q_i
+  __host__ __device__ __forceinline__ int64_t p() const { return 192 * dim; }                  // [64][64]: P, tiles j <= i
+  __host__ __device__ __forceinline__ int64_t u() const { return 192 * dim + 4096; }           // [vdim][64]: Uv, then U
+  __host__ __device__ __forceinline__ int64_t s() const { return u() + 64 * vdim; }            // [vdim][dim]: S before
+  __host__ __device__ __forceinline__ int64_t g() const { return s() + static_cast<int64_t>(dim) * vdim; }  // [dim]: G_n
+  __host__ __device__ __forceinline__ int64_t size() const { return g() + dim; }
+};
+
+__device__ __forceinline__ f32x4 dc_mac(f32x4 a, f32x4 b, f32x4 acc) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], acc, 0, 0, 0);
+  return acc;
+}
+
+template <int DIM>
+__global__ void __launch_bounds__(DC_THREADS, 2)
+delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, int64_t q_stride, int64_t k_stride,
+                            int64_t v_stride, const float* __restrict__ ab, const float* __restrict__ a_log,
+                            const float* __restrict__ dt_bias, const int32_t* __restrict__ chunk_row0,
+                            const int32_t* __restrict__ chunk_rows, float* __restrict__ work, int heads, int kv_heads,
+                            int vdim) {
+  constexpr int LD = DIM + 4, LA = DC_ROWS + 4;
+  __shared__ __attribute__((aligned(16))) float k_s[DC_ROWS * LD];
+  // the queries, and once they are done with A in their place (two workgroups fit a compute unit so)
+  __shared__ __attribute__((aligned(16))) float qa_s[DC_ROWS * (LD > LA ? LD : LA)];
+  float *const q_s = qa_s, *const a_s = qa_s;
+  __shared__ __attribute__((aligned(16))) float t_s[4][16][20];  // inverses of the blocks on the diagonal of I + A
+  __shared__ double c_s[DC_ROWS];                                // log G_i
+  __shared__ float beta_s[DC_ROWS], g_s[DC_ROWS], rest_s[DC_ROWS];  // beta_i, G_i, G_n / G_i
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m = lane & 15, g = lane >> 4;
+  const int head = blockIdx.x, chunk = blockIdx.y;
+  const int kv = head / (heads / kv_heads);
+  const int64_t row0 = chunk_row0[chunk];
+  const int n = chunk_rows[chunk];
+  const DeltaBlock blk{DIM, vdim};
+  float* mine = work + (static_cast<int64_t>(chunk) * heads + head) * blk.size();
+
+  // ---- unit rows into LDS: four threads a row, a quarter of its numbers each; rows past the chunk's end are zeros
+  {
+    constexpr int QUARTER = DIM / 4;
+    const int row = tid >> 2, part = tid & 3;
+    const int64_t src = row0 + min(row, n - 1);
+    const bf16_t* rows[2] = {k + src * k_stride + kv * DIM + part * QUARTER, q + src * q_stride + kv * DIM + part * QUARTER};
+    uint4 raw[2][QUARTER / 8];
+#pragma unroll
+    for (int which = 0; which < 2; ++which)
+#pragma unroll
+      for (int i = 0; i < QUARTER / 8; ++i) raw[which][i] = *reinterpret_cast<const uint4*>(rows[which] + 8 * i);
+#pragma unroll
+    for (int which = 0; which < 2; ++which) {
+      float x[QUARTER], ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < QUARTER / 8; ++i) {
+        const uint32_t u[4] = {raw[which][i].x, raw[which][i].y, raw[which][i].z, raw[which][i].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[8 * i + 2 * e] = __uint_as_float(u[e] << 16);
+          x[8 * i + 2 * e + 1] = __uint_as_float(u[e] & 0xffff0000u);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < QUARTER; ++i) ss += x[i] * x[i];
+      ss += ix_dpp<IX_DPP_XOR1>(ss);
+      ss += ix_dpp<IX_DPP_XOR2>(ss);
+      const float f = row < n ? (which ? 1.0f / sqrtf(static_cast<float>(DIM)) : 1.0f) / sqrtf(ss + 1e-6f) : 0.f;
+      float* dst = (which ? q_s : k_s) + row * LD + part * QUARTER;
+#pragma unroll
+      for (int i = 0; i < QUARTER; i += 4)
+        *reinterpret_cast<f32x4*>(dst + i) = f32x4{x[i] * f, x[i + 1] * f, x[i + 2] * f, x[i + 3] * f};
+    }
+  }
+  if (wave == 0) {
+    const bool live = lane < n;
+    const int64_t row = row0 + min(lane, n - 1);
+    const float x = ab[row * 2 * heads + head] + dt_bias[head];
+    const float lg = live ? -expf(a_log[head]) * (x > 20.f ? x : log1pf(expf(x))) : 0.f;
+    double c = lg;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const double below = __shfl_up(c, off, 64);
+      if (lane >= off) c += below;
+    }
+    const double last = __shfl(c, 63, 64);
+    c_s[lane] = c;
+    g_s[lane] = expf(static_cast<float>(c));
+    rest_s[lane] = expf(static_cast<float>(last - c));
+    beta_s[lane] = live ? 1.0f / (1.0f + expf(-ab[row * 2 * heads + heads + head])) : 0.f;
+  }
+  __syncthreads();
+
+  // ---- q_i . k_j, then k_i . k_j: the ten tiles on and below the diagonal of each
+  auto score = [&](const float* rows, int pair, auto&& put) {
+    const int rt = pair < 1 ? 0 : (pair < 3 ? 1 : (pair < 6 ? 2 : 3)), ct = pair - rt * (rt + 1) / 2;
+    const float* ar = rows + (16 * rt + m) * LD + 4 * g;
+    const float* br = k_s + (16 * ct + m) * LD + 4 * g;
+    f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+    for (int c = 0; c < DIM / 16; c += 2) {
+      s0 = dc_mac(*reinterpret_cast<const f32x4*>(ar + 16 * c), *reinterpret_cast<const f32x4*>(br + 16 * c), s0);
+      s1 = dc_mac(*reinterpret_cast<const f32x4*>(ar + 16 * c + 16), *reinterpret_cast<const f32x4*>(br + 16 * c + 16), s1);
+    }
+    const int j = 16 * ct + m;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = 16 * rt + 4 * g + e;
+      const float ratio = expf(static_cast<float>(fmin(c_s[i] - c_s[j], 0.0)));  // (above the diagonal: not used)
+      put(i, j, ratio * (s0[e] + s1[e]));
+    }
+  };
+#pragma unroll 1
+  for (int pair = wave; pair < 10; pair += 4)
+    score(q_s, pair, [&](int i, int j, float x) { mine[blk.p() + i * 64 + j] = j <= i ? x : 0.f; });
+  // ---- what the chain and the result take as they are
+  for (int id = tid; id < DIM * 16; id += DC_THREADS) {
+    const int row = id / (DIM / 4), d = 4 * (id % (DIM / 4));
+    const f32x4 x = *reinterpret_cast<const f32x4*>(q_s + row * LD + d);
+    *reinterpret_cast<f32x4*>(mine + blk.q() + row * DIM + d) = x * g_s[row];
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int pair = 3 - wave; pair < 10; pair += 4)  // (the wavefronts that had three tiles above have two)
+    score(k_s, pair, [&](int i, int j, float x) { a_s[i * LA + j] = j < i ? beta_s[i] * x : 0.f; });
+  for (int id = tid; id < DIM * 16; id += DC_THREADS) {
+    const int d = id >> 4, jq = 4 * (id & 15);
+    f32x4 x;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = k_s[(jq + e) * LD + d] * rest_s[jq + e];
+    *reinterpret_cast<f32x4*>(mine + blk.kt() + d * 64 + jq) = x;
+  }
+  for (int d = tid; d < DIM; d += DC_THREADS) mine[blk.g() + d] = g_s[DC_ROWS - 1];
+  __syncthreads();
+
+  // ---- the diagonal blocks' inverses: lane (block, column), sixteen steps of substitution
+  if (wave == 0) {
+    const int b = g, col = m;
+    float x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      float s = i == col ? 1.f : 0.f;
+      const float* ar = a_s + (16 * b + i) * LA + 16 * b;
+#pragma unroll
+      for (int j = 0; j < i; ++j) s = fmaf(-ar[j], x[j], s);
+      x[i] = s;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t_s[b][i][col] = x[i];
+  }
+  __syncthreads();
+
+  // ---- (I + A) [W | Uv] = [diag(beta G) K | diag(beta) V], four tiles of sixteen columns at a time and wavefront
+  const int tiles = (DIM + vdim) / 16;
+#pragma unroll 1
+  for (int t0 = 4 * wave; t0 < tiles; t0 += 16) {
+    f32x4 x[4][4];  // [tile][block of rows]
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int t = min(t0 + u, tiles - 1);
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int row = 16 * b + 4 * g + e;
+          if (16 * t < DIM) x[u][b][e] = beta_s[row] * g_s[row] * k_s[row * LD + 16 * t + m];
+          else x[u][b][e] = beta_s[row] * ix_load(v + (row0 + min(row, n - 1)) * v_stride + head * vdim + 16 * t - DIM + m);
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+#pragma unroll
+      for (int a = 0; a < b; ++a) {
+        const f32x4 na = -*reinterpret_cast<const f32x4*>(a_s + (16 * b + m) * LA + 16 * a + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) x[u][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(na[e], x[u][a][e], x[u][b], 0, 0, 0);
+      }
+      const f32x4 inv = *reinterpret_cast<const f32x4*>(&t_s[b][m][4 * g]);
+      f32x4 y[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) y[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) y[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(inv[e], x[u][b][e], y[u], 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u][b] = y[u];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int t = t0 + u;
+      if (t >= tiles) continue;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        if (16 * t < DIM) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) mine[blk.w() + (16 * b + 4 * g + e) * DIM + 16 * t + m] = -x[u][b][e];
+        } else {
+          *reinterpret_cast<f32x4*>(mine + blk.u() + (16 * t - DIM + m) * 64 + 16 * b + 4 * g) = x[u][b];
+        }
+      }
+    }
+  }
+}
+
+// request blockIdx.z's chunks [first, first + count) one after the other, value columns 16 blockIdx.y ..
+template <int DIM>
+__global__ void __launch_bounds__(DC_THREADS)
+delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, const int32_t* __restrict__ seq_first,
+                          const int32_t* __restrict__ seq_count, const int32_t* __restrict__ state_slots,
+                          float* __restrict__ state, int64_t state_stride, int heads, int vdim) {
+  constexpr int LD = DIM + 4, LU = DC_ROWS + 4;
+  constexpr int TILES = DIM / 16;                  // tiles of sixteen rows of the state
+  constexpr int TS = TILES >= 4 ? TILES / 4 : 1;   // ... per wavefront (with two tiles in all two wavefronts have none)
+  __shared__ __attribute__((aligned(16))) float s_s[16 * LD];
+  __shared__ __attribute__((aligned(16))) float u_s[16 * LU];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m = lane & 15, g = lane >> 4;
+  // (heads first: workgroups go to the chip's eight dies in turn, so a head's column blocks, which read the same W and
+  // K^T, share a die's L2 where the heads come in eights: 67 against 70 us at 1,437 rows)
+  const int head = blockIdx.x, seq = blockIdx.z;
+  const int col = 16 * blockIdx.y + m;
+  const int first = seq_first[seq], count = seq_count[seq];
+  if (count <= 0) return;
+  const bool owns = wave * TS < TILES;
+  const DeltaBlock blk{DIM, vdim};
+  const int64_t size = blk.size(), step = heads * size;
+  float* at0 = work + (static_cast<int64_t>(first) * heads + head) * size;
+  float* sp = state + static_cast<int64_t>(state_slots[seq_ids[seq]]) * state_stride +
+              (static_cast<int64_t>(head) * vdim + col) * DIM;
+  int row[TS];  // this lane's four rows of the state in each of its tiles
+  f32x4 st[TS];
+#pragma unroll
+  for (int t = 0; t < TS; ++t) {
+    row[t] = owns ? 16 * (wave * TS + t) + 4 * g : 0;
+    st[t] = *reinterpret_cast<const f32x4*>(sp + row[t]);
+  }
+  struct Operands { f32x4 w[TILES], kt[TS][4], u, gn[TS]; };
+  auto ask = [&](const float* p, Operands& o) {
+#pragma unroll
+    for (int c = 0; c < TILES; ++c)
+      o.w[c] = *reinterpret_cast<const f32x4*>(p + blk.w() + (16 * wave + m) * DIM + 16 * c + 4 * g);
+#pragma unroll
+    for (int t = 0; t < TS; ++t) {
+      const int d = (owns ? 16 * (wave * TS + t) : 0) + m;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) o.kt[t][s] = *reinterpret_cast<const f32x4*>(p + blk.kt() + d * 64 + 16 * s + 4 * g);
+      o.gn[t] = *reinterpret_cast<const f32x4*>(p + blk.g() + row[t]);
+    }
+    o.u = *reinterpret_cast<const f32x4*>(p + blk.u() + col * 64 + 16 * wave + 4 * g);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto work_chunk = [&](float* p, const Operands& o) {
+    if (owns) {
+#pragma unroll
+      for (int t = 0; t < TS; ++t) {
+        *reinterpret_cast<f32x4*>(s_s + m * LD + row[t]) = st[t];
+        *reinterpret_cast<f32x4*>(p + blk.s() + static_cast<int64_t>(col) * DIM + row[t]) = st[t];
+      }
+    }
+    __syncthreads();
+    // (all of a product's operands are asked for before the first is used: left to itself the compiler takes them two by
+    // two and waits for each pair)
+    f32x4 b[TILES > 4 ? TILES : 4];
+#pragma unroll
+    for (int c = 0; c < TILES; ++c) b[c] = *reinterpret_cast<const f32x4*>(s_s + m * LD + 16 * c + 4 * g);
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 ua = o.u, ub = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < TILES; c += 2) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        ua = __builtin_amdgcn_mfma_f32_16x16x4f32(o.w[c][e], b[c][e], ua, 0, 0, 0);
+        ub = __builtin_amdgcn_mfma_f32_16x16x4f32(o.w[c + 1][e], b[c + 1][e], ub, 0, 0, 0);
+      }
+    }
+    ua += ub;
+    *reinterpret_cast<f32x4*>(u_s + m * LU + 16 * wave + 4 * g) = ua;
+    *reinterpret_cast<f32x4*>(p + blk.u() + col * 64 + 16 * wave + 4 * g) = ua;
+#pragma unroll
+    for (int t = 0; t < TS; ++t) st[t] *= o.gn[t];
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < 4; ++s) b[s] = *reinterpret_cast<const f32x4*>(u_s + m * LU + 16 * s + 4 * g);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int t = 0; t < TS; ++t) st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kt[t][s][e], b[s][e], st[t], 0, 0, 0);
+  };
+  Operands one, two;  // the next chunk's operands on their way while this one is worked
+  ask(at0, one);
+  for (int c = 0; c < count; c += 2) {
+    float* p = at0 + c * step;
+    ask(at0 + min(c + 1, count - 1) * step, two);
+    work_chunk(p, one);
+    if (c + 1 < count) {
+      ask(at0 + min(c + 2, count - 1) * step, one);
+      work_chunk(p + step, two);
+    }
+  }
+  if (owns) {
+#pragma unroll
+    for (int t = 0; t < TS; ++t) *reinterpret_cast<f32x4*>(sp + row[t]) = st[t];
+  }
+}
+
+// O^T = S^T (diag(G) Q)^T + U^T P^T: a lane ends up with four consecutive columns of a row
+template <int DIM>
+__global__ void __launch_bounds__(DC_THREADS, 2)
+delta_chunks_result_kernel(const float* __restrict__ work, const int32_t* __restrict__ chunk_row0,
+                           const int32_t* __restrict__ chunk_rows, float* __restrict__ out, int heads, int vdim) {
+  constexpr int LD = DIM + 4, LP = DC_ROWS + 4;
+  __shared__ __attribute__((aligned(16))) float q_s[DC_ROWS * LD];
+  __shared__ __attribute__((aligned(16))) float p_s[DC_ROWS * LP];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m = lane & 15, g = lane >> 4;
+  const int head = blockIdx.x, chunk = blockIdx.y;
+  const int64_t row0 = chunk_row0[chunk];
+  const int n = chunk_rows[chunk];
+  const DeltaBlock blk{DIM, vdim};
+  const float* mine = work + (static_cast<int64_t>(chunk) * heads + head) * blk.size();
+#pragma unroll
+  for (int id = tid; id < DC_ROWS * DIM / 4; id += DC_THREADS) {
+    const int row = id / (DIM / 4), d = 4 * (id % (DIM / 4));
+    *reinterpret_cast<f32x4*>(q_s + row * LD + d) = *reinterpret_cast<const f32x4*>(mine + blk.q() + row * DIM + d);
+  }
+#pragma unroll
+  for (int id = tid; id < DC_ROWS * 16; id += DC_THREADS) {
+    const int row = id >> 4, j = 4 * (id & 15);  // (tiles above the diagonal hold nothing and are not read below)
+    if ((j >> 4) <= (row >> 4))
+      *reinterpret_cast<f32x4*>(p_s + row * LP + j) = *reinterpret_cast<const f32x4*>(mine + blk.p() + row * 64 + j);
+  }
+  __syncthreads();
+  const int tiles = vdim / 16;
+  for (int t0 = 2 * wave; t0 < tiles; t0 += 8) {
+    f32x4 acc[2][4];  // [tile of columns][tile of rows]
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[u][r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int t1 = min(t0 + 1, tiles - 1);
+    const float* s0 = mine + blk.s() + static_cast<int64_t>(16 * t0 + m) * DIM + 4 * g;
+    const float* s1 = mine + blk.s() + static_cast<int64_t>(16 * t1 + m) * DIM + 4 * g;
+#pragma unroll
+    for (int c = 0; c < DIM / 16; ++c) {
+      const f32x4 a0 = *reinterpret_cast<const f32x4*>(s0 + 16 * c), a1 = *reinterpret_cast<const f32x4*>(s1 + 16 * c);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const f32x4 b = *reinterpret_cast<const f32x4*>(q_s + (16 * r + m) * LD + 16 * c + 4 * g);
+        acc[0][r] = dc_mac(a0, b, acc[0][r]);
+        acc[1][r] = dc_mac(a1, b, acc[1][r]);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const f32x4 a0 = *reinterpret_cast<const f32x4*>(mine + blk.u() + (16 * t0 + m) * 64 + 16 * s + 4 * g);
+      const f32x4 a1 = *reinterpret_cast<const f32x4*>(mine + blk.u() + (16 * t1 + m) * 64 + 16 * s + 4 * g);
+#pragma unroll
+      for (int r = s; r < 4; ++r) {
+        const f32x4 b = *reinterpret_cast<const f32x4*>(p_s + (16 * r + m) * LP + 16 * s + 4 * g);
+        acc[0][r] = dc_mac(a0, b, acc[0][r]);
+        acc[1][r] = dc_mac(a1, b, acc[1][r]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (t0 + u >= tiles) continue;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * r + m;
+        if (row < n)
+          *reinterpret_cast<f32x4*>(out + ((row0 + row) * heads + head) * vdim + 16 * (t0 + u) + 4 * g) = acc[u][r];
+      }
+    }
+  }
+}
+
+// q, k, v, ab, a_log, dt_bias, state, out as ix_delta_rule takes them (bfloat16, a decay per head).  chunk_row0 /
+// chunk_rows [chunks]: first row in the step and number of rows (1 to 64) of every chunk; request seq_ids[s] of the
+// step has the chunks seq_first[s] .. + seq_count[s], in order; its state is read before them and written after them.
+// work: chunks * heads blocks as `DeltaBlock` has them (work_floats: how many floats there are).
+extern "C" int ix_delta_chunks(const void* q, const void* k, const void* v, int64_t q_stride, int64_t k_stride,
+                               int64_t v_stride, const float* ab, const float* a_log, const float* dt_bias, float* state,
+                               int64_t state_stride, const int32_t* state_slots, const int32_t* chunk_row0,
+                               const int32_t* chunk_rows, int chunks, const int32_t* seq_ids, const int32_t* seq_first,
+                               const int32_t* seq_count, int seqs, float* work, int64_t work_floats, float* out,
+                               int heads, int kv_heads, int dim, int vdim, hipStream_t stream) {
+  IX_REQUIRE(chunks >= 0 && seqs >= 0 && heads > 0 && kv_heads > 0 && vdim > 0, "sizes must be positive");
+  IX_REQUIRE(heads % kv_heads == 0, "heads must be a multiple of kv_heads");
+  IX_REQUIRE(dim == 32 || dim == 64 || dim == 128, "key heads of 32, 64 or 128 numbers");
+  IX_REQUIRE(vdim % 16 == 0, "value heads in multiples of 16 numbers");
+  IX_REQUIRE(state_stride >= static_cast<int64_t>(heads) * dim * vdim && state_stride % 4 == 0, "state blocks too small");
+  IX_REQUIRE(q_stride % 8 == 0 && k_stride % 8 == 0, "rows must lie on 16-byte boundaries");
+  IX_REQUIRE(((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(state) |
+               reinterpret_cast<uintptr_t>(work) | reinterpret_cast<uintptr_t>(out)) & 15) == 0,
+             "operands must lie on 16-byte boundaries");
+  IX_REQUIRE(heads < 65536 && chunks < 65536 && seqs < 65536 && vdim / 16 < 65536, "too many heads, chunks or requests");
+  IX_REQUIRE(work_floats >= static_cast<int64_t>(chunks) * heads * (DeltaBlock{dim, vdim}).size(), "workspace too small");
+  if (chunks == 0 || seqs == 0) return 0;
+#define RUN(DIM)                                                                                                         \
+  hipLaunchKernelGGL(delta_chunks_prepare_kernel<DIM>, dim3(heads, chunks), dim3(DC_THREADS), 0, stream, (const bf16_t*)q, \
+                     (const bf16_t*)k, (const bf16_t*)v, q_stride, k_stride, v_stride, ab, a_log, dt_bias, chunk_row0,   \
+                     chunk_rows, work, heads, kv_heads, vdim);                                                           \
+  if (ix_check_launch("ix_delta_chunks: prepare")) return 1;                                                             \
+  hipLaunchKernelGGL(delta_chunks_chain_kernel<DIM>, dim3(heads, vdim / 16, seqs), dim3(DC_THREADS), 0, stream, work,    \
+                     seq_ids, seq_first, seq_count, state_slots, state, state_stride, heads, vdim);                      \
+  if (ix_check_launch("ix_delta_chunks: chain")) return 1;                                                               \
+  hipLaunchKernelGGL(delta_chunks_result_kernel<DIM>, dim3(heads, chunks), dim3(DC_THREADS), 0, stream, work, chunk_row0, \
+                     chunk_rows, out, heads, vdim)
+  if (dim == 32) { RUN(32); }
+  else if (dim == 64) { RUN(64); }
+  else { RUN(128); }
+#undef RUN
+  return ix_check_launch("ix_delta_chunks");
+}

@@ -49,14 +49,14 @@ delta_rule_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __r
                   const float* __restrict__ a_log,
                   const float* __restrict__ dt_bias, float* __restrict__ state, int64_t state_stride,
                   const int32_t* __restrict__ q_start, const int32_t* __restrict__ state_slots,
-                  float* __restrict__ out, int heads, int kv_heads, int dim, int vdim) {
+                  float* __restrict__ out, int heads, int kv_heads, int dim, int vdim, int max_rows) {
   const int lane = threadIdx.x;
   const int col = blockIdx.x * DELTA_COLS + lane / DELTA_SPLIT, part = lane % DELTA_SPLIT;
   const int head = blockIdx.y, seq = blockIdx.z;
   const int kv = head / (heads / kv_heads);
   const int64_t row0 = q_start[seq];
   const int n = q_start[seq + 1] - static_cast<int>(row0);
-  if (n <= 0) return;
+  if (n <= 0 || (max_rows > 0 && n > max_rows)) return;
   const bool live = col < vdim;
   const int cj = live ? col : vdim - 1;  // lanes past the last column repeat it and store nothing
 
@@ -244,7 +244,7 @@ delta_rule_chunk_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, int64
                         int64_t v_stride, const float* ab, const float* ach, const float* __restrict__ a_log,
                         const float* __restrict__ dt_bias, float* __restrict__ state, int64_t state_stride,
                         const int32_t* __restrict__ q_start, const int32_t* __restrict__ state_slots,
-                        float* __restrict__ out, int heads, int kv_heads, int vdim) {
+                        float* __restrict__ out, int heads, int kv_heads, int vdim, int max_rows) {
   constexpr int DIM = SP * RPL;
   constexpr int COLS = 64 / SP;                      // value columns of a wavefront
   constexpr int PIECES = DIM / 8;                    // 16-byte pieces of a q or k row (4, 8 or 16: a power of two)
@@ -263,7 +263,7 @@ delta_rule_chunk_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, int64
   const int kv = head / (heads / kv_heads);
   const int64_t row0 = q_start[seq];
   const int n = q_start[seq + 1] - static_cast<int>(row0);
-  if (n <= 0) return;
+  if (n <= 0 || (max_rows > 0 && n > max_rows)) return;
   const bool live = col < vdim;
   const int cj = live ? col : vdim - 1;
 
@@ -417,12 +417,12 @@ delta_rule_chunk_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, int64
 // q, k [T, kv_heads * dim] and v [T, heads * vdim] of the run's type with their row strides; ab float32 [T, 2 heads]
 // (a then b); a_log, dt_bias float32 [heads]; or, with a decay per key channel, ach float32 [T, heads * dim] (the
 // decays themselves) and ab float32 [T, heads] (b alone); state: slot s at state + s * state_stride, [heads, vdim, dim] (a column's rows side by side);
-// out float32 [T, heads, vdim].
+// out float32 [T, heads, vdim].  Requests that bring more than `max_rows` rows are left to others (0: none).
 extern "C" int ix_delta_rule(const void* q, const void* k, const void* v, int dtype, int64_t q_stride,
                              int64_t k_stride, int64_t v_stride, const float* ab, const float* ach, const float* a_log,
                              const float* dt_bias, float* state, int64_t state_stride, const int32_t* q_start,
                              const int32_t* state_slots, float* out, int64_t tokens, int requests, int heads,
-                             int kv_heads, int dim, int vdim, hipStream_t stream) {
+                             int kv_heads, int dim, int vdim, int max_rows, hipStream_t stream) {
   IX_REQUIRE(tokens >= 0 && requests >= 0 && heads > 0 && kv_heads > 0 && dim > 0 && vdim > 0, "sizes must be positive");
   IX_REQUIRE(heads % kv_heads == 0, "heads must be a multiple of kv_heads");
   IX_REQUIRE(dim <= 256, "at most 256 numbers per query and key head");
@@ -441,7 +441,7 @@ extern "C" int ix_delta_rule(const void* q, const void* k, const void* v, int dt
 #define LAUNCH_CH(TT, RPL, VEC, CH)                                                                                         \
   hipLaunchKernelGGL((delta_rule_kernel<TT, RPL, VEC, CH>), grid, block, 0, stream, (const TT*)q, (const TT*)k, (const TT*)v, \
                      q_stride, k_stride, v_stride, ab, ach, a_log, dt_bias, state, state_stride, q_start, state_slots, out,   \
-                     heads, kv_heads, dim, vdim)
+                     heads, kv_heads, dim, vdim, max_rows)
 #define LAUNCH(TT, RPL, VEC)                \
   do {                                      \
     if (ach) LAUNCH_CH(TT, RPL, VEC, true); \
@@ -457,7 +457,7 @@ extern "C" int ix_delta_rule(const void* q, const void* k, const void* v, int dt
 #define CHUNKED_CH(SP, RPL, CH)                                                                                               \
   hipLaunchKernelGGL((delta_rule_chunk_kernel<SP, RPL, CH>), dim3((vdim + 64 / SP - 1) / (64 / SP), heads, requests), block, \
                      0, stream, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, q_stride, k_stride, v_stride, ab, ach, \
-                     a_log, dt_bias, state, state_stride, q_start, state_slots, out, heads, kv_heads, vdim)
+                     a_log, dt_bias, state, state_stride, q_start, state_slots, out, heads, kv_heads, vdim, max_rows)
 #define CHUNKED(SP, RPL)                \
   do {                                  \
     if (ach) CHUNKED_CH(SP, RPL, true); \

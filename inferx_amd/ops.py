@@ -1222,12 +1222,14 @@ def short_conv(x: torch.Tensor, bias: Optional[torch.Tensor], weight: torch.Tens
 
 def delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ab: torch.Tensor, a_log: torch.Tensor,
                dt_bias: torch.Tensor, state: torch.Tensor, rows: StepRows, out: torch.Tensor, heads: int,
-               kv_heads: int, dim: int, vdim: int, channel_decays: Optional[torch.Tensor] = None) -> None:
+               kv_heads: int, dim: int, vdim: int, channel_decays: Optional[torch.Tensor] = None,
+               max_rows: int = 0) -> None:
     """The gated delta rule over the rows of a step, request by request, from and to `state` (a float32 view
     [slots, >= heads * dim * vdim]).  q, k [T, kv_heads * dim], v [T, heads * vdim] (rows may be strided);
     ab float32 [T, 2 heads]: the decay's and the step size's logits; out float32 [T, heads, vdim].
     `channel_decays` float32 [T, heads * dim]: a decay per key channel (the decays themselves, see
-    `channel_decays`); ab is then float32 [T, heads], the step size's logits alone, and dt_bias is not read."""
+    `channel_decays`); ab is then float32 [T, heads], the step size's logits alone, and dt_bias is not read.
+    `max_rows` > 0: requests that bring more rows are left out."""
     T = q.shape[0]
     channel_logits = channel_decays
     for t, n in ((q, kv_heads * dim), (k, kv_heads * dim), (v, heads * vdim)):
@@ -1249,6 +1251,46 @@ def delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ab: torch.Tens
     _call("ix_delta_rule", q.data_ptr(), k.data_ptr(), v.data_ptr(), _i32(_dt(q)), _i64(q.stride(0)), _i64(k.stride(0)),
           _i64(v.stride(0)), _ptr(ab), _ptr(channel_logits), _ptr(a_log), _ptr(dt_bias), state.data_ptr(), _i64(state.stride(0)),
           _ptr(rows.q_start), _ptr(rows.state_slots), _ptr(out), _i64(T), _i32(S), _i32(heads), _i32(kv_heads),
+          _i32(dim), _i32(vdim), _i32(max_rows), _stream())
+
+
+def delta_chunks_fits(q: torch.Tensor, k: torch.Tensor, state: torch.Tensor, dim: int, vdim: int) -> bool:
+    """Whether `delta_chunks` takes these operands: bfloat16, key heads of 32, 64 or 128 numbers, value heads in
+    sixteens, rows and state on 16-byte boundaries."""
+    return (q.dtype == torch.bfloat16 and dim in (32, 64, 128) and vdim % 16 == 0 and q.stride(0) % 8 == 0
+            and k.stride(0) % 8 == 0 and state.stride(0) % 4 == 0
+            and (q.data_ptr() | k.data_ptr() | state.data_ptr()) % 16 == 0)
+
+
+def delta_chunks_floats(dim: int, vdim: int) -> int:
+    """Floats of workspace that `delta_chunks` takes per chunk and head (the entry point checks it)."""
+    return 193 * dim + 4096 + 64 * vdim + dim * vdim
+
+
+def delta_chunks(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ab: torch.Tensor, a_log: torch.Tensor,
+                 dt_bias: torch.Tensor, state: torch.Tensor, state_slots: torch.Tensor, chunks: torch.Tensor,
+                 seqs: torch.Tensor, out: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int) -> None:
+    """`delta_rule` with a decay per head for the requests that `seqs` names, their rows in chunks whose products are
+    worked at the same time.  `chunks`, `seqs`: as `linear_chunks` takes them."""
+    T = q.shape[0]
+    for t, n in ((q, kv_heads * dim), (k, kv_heads * dim), (v, heads * vdim)):
+        _need(t.dim() == 2 and t.shape == (T, n) and t.stride(1) == 1 and t.dtype == q.dtype and t.is_cuda, "q, k or v shape")
+    _need(ab.dtype == torch.float32 and ab.shape == (T, 2 * heads) and ab.is_contiguous(), "ab must be float32 [T, 2 heads]")
+    _need(a_log.dtype == torch.float32 and a_log.numel() == heads and dt_bias.dtype == torch.float32
+          and dt_bias.numel() == heads and dt_bias.is_contiguous(), "a_log and dt_bias must be float32 [heads]")
+    _need(state.dtype == torch.float32 and state.dim() == 2 and state.stride(1) == 1
+          and state.shape[1] >= heads * dim * vdim, "the state must be float32 [slots, >= heads * dim * vdim]")
+    _need(out.dtype == torch.float32 and out.shape == (T, heads, vdim), "out must be float32 [T, heads, vdim]")
+    _need(delta_chunks_fits(q, k, state, dim, vdim), "operands that the chunked form does not take")
+    _is_i32(state_slots)
+    for t, n in ((chunks, 2), (seqs, 3)):
+        _is_i32(t)
+        _need(t.dim() == 2 and t.shape[0] == n and t.is_contiguous(), "chunks int32 [2, n], seqs int32 [3, m]")
+    work = torch.empty((chunks.shape[1] * heads * delta_chunks_floats(dim, vdim),), dtype=torch.float32, device=q.device)
+    _call("ix_delta_chunks", q.data_ptr(), k.data_ptr(), v.data_ptr(), _i64(q.stride(0)), _i64(k.stride(0)),
+          _i64(v.stride(0)), _ptr(ab), _ptr(a_log), _ptr(dt_bias), state.data_ptr(), _i64(state.stride(0)),
+          _ptr(state_slots), _ptr(chunks[0]), _ptr(chunks[1]), _i32(chunks.shape[1]), _ptr(seqs[0]), _ptr(seqs[1]),
+          _ptr(seqs[2]), _i32(seqs.shape[1]), _ptr(work), _i64(work.numel()), _ptr(out), _i32(heads), _i32(kv_heads),
           _i32(dim), _i32(vdim), _stream())
 
 

@@ -129,6 +129,32 @@ def decayed_state(ctx, q, k, v, state, out, heads: int, dim: int, vdim: int, dec
         ops.linear_chunks(q, k, v, state, ctx.state_slots, chunks, seqs, out, heads, dim, vdim, **more)
 
 
+def chunk_slices(ctx, min_rows: int, most: int):
+    """The step's portions of at least `min_rows` rows cut into chunks, as a list of (chunks, requests) like `chunk_plan`'s
+    with at most `most` chunks each: a request whose chunks lie in two of them goes on in the second from the state that
+    the first left.  Planned on the host, once per step."""
+    key = ("chunk_slices", min_rows, most)
+    if key not in ctx.memo:
+        n = (ctx.host.q_start[1:] - ctx.host.q_start[:-1]).astype(np.int64)
+        seqs = np.flatnonzero(n >= min_rows)
+        size = ops.LINEAR_CHUNK_ROWS
+        count = -(-n[seqs] // size)
+        first = np.cumsum(count) - count
+        total = int(count.sum())
+        which = np.repeat(np.arange(len(seqs)), count)
+        off = (np.arange(total) - first[which]) * size
+        row0, rows = ctx.host.q_start[seqs][which] + off, np.minimum(size, n[seqs][which] - off)
+        dev = lambda a: torch.from_numpy(np.ascontiguousarray(a.astype(np.int32))).to(ctx.rt.device)
+        out = []
+        for a in range(0, total, most):
+            b = min(total, a + most)
+            lo, hi = np.maximum(first, a), np.minimum(first + count, b)
+            here = hi > lo
+            out.append((dev(np.stack([row0[a:b], rows[a:b]])), dev(np.stack([seqs[here], lo[here] - a, (hi - lo)[here]]))))
+        ctx.memo[key] = out
+    return ctx.memo[key]
+
+
 class LightningAttention(Mixer):
     graph_safe = True
 

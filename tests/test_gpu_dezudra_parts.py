@@ -593,3 +593,79 @@ def test_one_key_stands_out_for_every_query_of_a_portion(kernel):
             seen = np.array([key <= p and (p - key < window or key < keep) for p in positions])
             assert np.array_equal(err < 3e-2, seen), \
                 f"portion ending at {last}, key {key}: queries {np.flatnonzero((err < 3e-2) != seen).tolist()} of the portion are wrong"
+
+
+# ---- the delta rule in chunks ---------------------------------------------------------------------------------------------
+# rows of the requests of a step (one of them without any), around chunks of 64 and the sixteens within them
+@pytest.mark.parametrize("lengths", [[1, 15, 0, 16], [17, 64, 63], [65, 130], [200]])
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(4, 2, 32, 48), (3, 1, 64, 16), (8, 2, 128, 128), (2, 2, 128, 144)])
+@pytest.mark.parametrize("decay", [0.0, -6.0])
+def test_delta_rule_in_chunks(lengths, heads, kv_heads, dim, vdim, decay):
+    """The chunked form against the float64 recurrence, from a state that is not zero, its last state too; in one call and
+    cut into slices of two chunks.  float32 sums of at most dim + 64 products of numbers up to the results' size: 1e-5
+    of the largest."""
+    from inferx_amd import ops
+    T, S = sum(lengths), len(lengths)
+    q, k = (rnd((T, kv_heads * dim), s, 1.0, torch.bfloat16) for s in (1, 2))
+    v, ab = rnd((T, heads * vdim), 3, 1.0, torch.bfloat16), rnd((T, 2 * heads), 4, 1.5)
+    ab[:, :heads] += decay
+    a_log, dt_bias = rnd((heads,), 5, 0.7), rnd((heads,), 6, 0.7)
+    before = rnd((S + 1, heads * dim * vdim + 4), 7, 0.3)
+    starts = [sum(lengths[:s]) for s in range(S + 1)]
+    row0 = [(s, starts[s] + at, min(64, n - at)) for s, n in enumerate(lengths) for at in range(0, n, 64)]
+    slots = i32([S - s for s in range(S)])
+
+    def slices(most):
+        for a in range(0, len(row0), most):
+            part = row0[a:a + most]
+            live = sorted({s for s, _, _ in part})
+            first = [[p[0] for p in part].index(s) for s in live]
+            yield (i32([[p[1] for p in part], [p[2] for p in part]]),
+                   i32([live, first, [sum(p[0] == s for p in part) for s in live]]))
+
+    for most in (1000, 2):
+        state = before.to(DEV)
+        out = torch.full((T, heads, vdim), float("nan"), device=DEV)
+        for chunks, seqs in slices(most):
+            ops.delta_chunks(q.to(DEV), k.to(DEV), v.to(DEV), ab.to(DEV), a_log.to(DEV), dt_bias.to(DEV), state, slots,
+                             chunks, seqs, out, heads, kv_heads, dim, vdim)
+        for s, n in enumerate(lengths):
+            sl, at = S - s, slice(starts[s], starts[s] + n)
+            if n == 0:
+                assert torch.equal(state[sl].cpu(), before[sl])
+                continue
+            g = np.exp(-np.exp(f64(a_log)) * np.logaddexp(0.0, f64(ab[at, :heads]) + f64(dt_bias)))
+            beta = 1.0 / (1.0 + np.exp(-f64(ab[at, heads:])))
+            unit = lambda x: x / np.sqrt((x * x).sum(-1, keepdims=True) + 1e-6)
+            qn, kn = (unit(f64(x[at]).reshape(n, kv_heads, dim)).repeat(heads // kv_heads, 1) for x in (q, k))
+            M = f64(before[sl][:heads * dim * vdim]).reshape(heads, vdim, dim)
+            want = np.zeros((n, heads, vdim))
+            for t in range(n):
+                M = M * g[t][:, None, None]
+                u = beta[t][:, None] * (f64(v[at])[t].reshape(heads, vdim) - np.einsum("hvd,hd->hv", M, kn[t]))
+                M = M + u[:, :, None] * kn[t][:, None, :]
+                want[t] = np.einsum("hvd,hd->hv", M, qn[t]) * dim ** -0.5
+            close(out[at].cpu(), want, 1e-5, f"request {s}, slices of {most}")
+            close(state[sl].cpu()[:heads * dim * vdim], M.reshape(-1), 1e-5, f"state of request {s}, slices of {most}")
+            assert torch.equal(state[sl].cpu()[heads * dim * vdim:], before[sl][heads * dim * vdim:])
+
+
+def test_delta_rule_leaves_long_requests_to_others():
+    """`max_rows`: requests with more rows keep their state, and their rows of the result are not written."""
+    from inferx_amd import ops
+    lengths, heads, dim, vdim = [3, 40, 16], 2, 32, 16
+    T = sum(lengths)
+    q, k, v = (rnd((T, heads * n), s, 1.0, torch.bfloat16).to(DEV) for s, n in ((1, dim), (2, dim), (3, vdim)))
+    ab, a_log, dt_bias = rnd((T, 2 * heads), 4).to(DEV), rnd((heads,), 5).to(DEV), rnd((heads,), 6).to(DEV)
+    q_start, seq = i32([0, 3, 43, 59]), i32([0] * 3 + [1] * 40 + [2] * 16)
+    results = []
+    for max_rows in (0, 16):
+        state = rnd((3, heads * dim * vdim), 7).to(DEV)
+        out = torch.full((T, heads, vdim), 7.0, device=DEV)
+        ops.delta_rule(q, k, v, ab, a_log, dt_bias, state, ops.StepRows(seq, q_start, i32([0, 1, 2])), out, heads, heads, dim,
+                       vdim, max_rows=max_rows)
+        results.append((out.cpu(), state.cpu()))
+    (all_out, all_state), (some_out, some_state) = results
+    assert torch.equal(all_out[:3], some_out[:3]) and torch.equal(all_out[43:], some_out[43:])
+    assert torch.equal(all_state[[0, 2]], some_state[[0, 2]])
+    assert (some_out[3:43] == 7.0).all() and torch.equal(some_state[1], rnd((3, heads * dim * vdim), 7)[1])

@@ -212,11 +212,9 @@ extern "C" int ix_latent_attention_plain(const void* ql, int64_t ql_t, int64_t q
 // 8 (l / 16) .. + 7 of its column: the B operand of the second product as it stands.  Softmax online, float32, per
 // column; a lane's accumulators all belong to its column, so rescaling is a multiplication by the lane's factor.
 //
-// What a column is: prompt portions (DEC false): a workgroup takes 16 consecutive rows of the step and four heads,
-// a wavefront one head, a column one row.  Rows of several requests in a tile are worked request by request (the
-// other rows' keys all masked: they change nothing).  One token per request (DEC true): a workgroup takes one token
-// and one slice of its keys, a wavefront sixteen heads, a column one head; slices leave (max, sum, unnormalised
-// sums) for `attn_combine_kernel`.  The next round's rows are on their way from memory while a round is multiplied.
+// One token per request (steps that bring more go through latent_prefill.hip): a workgroup takes one token and one slice
+// of its keys, a wavefront sixteen heads, a column one head; slices leave (max, sum, unnormalised sums) for
+// `attn_combine_kernel`.  The next round's rows are on their way from memory while a round is multiplied.
 typedef __bf16 lat_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 lat_bf16x4 __attribute__((ext_vector_type(4)));
 typedef float lat_f32x4 __attribute__((ext_vector_type(4)));
@@ -225,14 +223,14 @@ typedef float lat_f32x4 __attribute__((ext_vector_type(4)));
 #define LATM_KPAD 8      // numbers between key rows in LDS (keeps 16-byte pieces aligned, spreads the banks)
 #define LATM_VSTRIDE 40  // numbers per transposed row: 32 keys and 8 spare
 
-template <int NW, int NR, bool DEC>  // rank + rot_dim <= 32 NW, rank <= 16 NR
+template <int NW, int NR>  // rank + rot_dim <= 32 NW, rank <= 16 NR
 __global__ void __launch_bounds__(256)
 latent_attn_mfma_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_h, const __bf16* __restrict__ qr,
                         int64_t qr_t, int64_t qr_h, const __bf16* __restrict__ cache,
                         const int32_t* __restrict__ block_table, const int32_t* __restrict__ seq_of_token,
                         const int32_t* __restrict__ positions, __bf16* __restrict__ out, int64_t out_t, int64_t out_h,
                         float* __restrict__ part_o, float* __restrict__ part_ml, int n_splits, int tokens, int heads,
-                        int rank, int rot_dim, int page_size, int max_blocks, float scale_log2, int n_tiles,
+                        int rank, int rot_dim, int page_size, int max_blocks, float scale_log2,
                         int window, const __bf16* __restrict__ head_gate, int64_t gate_stride) {
   extern __shared__ __attribute__((aligned(16))) unsigned char latm_lds[];
   constexpr int NP = (4 * NW + 7) / 8;  // 16-byte pieces of a round's rows that a thread moves
@@ -248,24 +246,9 @@ latent_attn_mfma_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, g = lane >> 4;
-  int row, head, r0, r1;
-  bool wave_on;
-  if constexpr (DEC) {
-    r0 = blockIdx.x;
-    r1 = r0 + 1;
-    row = r0;
-    head = (blockIdx.y * 4 + wave) * 16 + n;
-    wave_on = (blockIdx.y * 4 + wave) * 16 < heads;
-  } else {
-    // one row of workgroups, the tiles with the most keys first, a tile's groups of four heads side by side
-    const int head_groups = (heads + 3) / 4;
-    r0 = (n_tiles - 1 - static_cast<int>(blockIdx.x) / head_groups) * 16;
-    r1 = min(r0 + 16, tokens);
-    row = r0 + n;
-    head = (static_cast<int>(blockIdx.x) % head_groups) * 4 + wave;
-    wave_on = head < heads;
-  }
-  const bool col_ok = row < r1 && head < heads;
+  const int row = blockIdx.x, head = (blockIdx.y * 4 + wave) * 16 + n;
+  const bool wave_on = (blockIdx.y * 4 + wave) * 16 < heads;
+  const bool col_ok = head < heads;
 
   lat_bf16x8 qf[NW];
 #pragma unroll
@@ -284,26 +267,15 @@ latent_attn_mfma_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_
   float m = -1e30f, l = 0.f;
   const int ka0 = 8 * (n >> 2) + (n & 3), ka1 = ka0 + 4;  // the keys of this lane's rows of the two A operands
 
-  int seg = r0;
-  while (seg < r1) {  // (every decision in this loop is the same for the whole workgroup)
-    const int seq = seq_of_token[seg];
-    int end = seg + 1;
-    if constexpr (!DEC)
-      while (end < r1 && seq_of_token[end] == seq) ++end;
-    int k_end = positions[end - 1] + 1;  // a request's rows come in the order of their positions
-    // with a window W the first of these rows reads from key k_lo on, and no row reads an earlier one (whose page
-    // may be gone); rounds start at multiples of their length
-    const int k_lo = window > 0 ? max(positions[seg] + 1 - window, 0) : 0;
-    int k_begin = k_lo & ~(LATM_KEYS - 1);
-    if constexpr (DEC) {
-      const int per = ((k_end - k_begin + n_splits - 1) / n_splits + LATM_KEYS - 1) & ~(LATM_KEYS - 1);
-      k_begin += static_cast<int>(blockIdx.z) * per;
-      k_end = min(k_end, k_begin + per);
-    }
-    const int my_pos = (col_ok && row >= seg && row < end) ? positions[row] : -1;
-    const int my_lo = window > 0 ? my_pos - window : -1;  // the last key that this column does not read
-    const int32_t* table = block_table + static_cast<int64_t>(seq) * max_blocks;
-
+  const int my_pos = positions[row];
+  // with a window W the query reads from key k_lo on (earlier pages may be gone); rounds start at multiples of their length
+  const int k_lo = window > 0 ? max(my_pos + 1 - window, 0) : 0;
+  int k_begin = k_lo & ~(LATM_KEYS - 1), k_end = my_pos + 1;
+  const int per = ((k_end - k_begin + n_splits - 1) / n_splits + LATM_KEYS - 1) & ~(LATM_KEYS - 1);
+  k_begin += static_cast<int>(blockIdx.z) * per;
+  k_end = min(k_end, k_begin + per);
+  const int32_t* table = block_table + static_cast<int64_t>(seq_of_token[row]) * max_blocks;
+  {  // (every decision in here is the same for the whole workgroup)
     uint4 st[NP];
     const int my_key = tid >> 3, my_sub = tid & 7;  // a thread moves pieces my_sub, my_sub + 8, .. of one key's row
     auto ask = [&](int k0) {
@@ -370,8 +342,8 @@ latent_attn_mfma_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int j = k0 + 8 * g + i;
-          p[i] = (j <= my_pos && j > my_lo && j < k_end) ? s0[i] * scale_log2 : -INFINITY;
-          p[4 + i] = (j + 4 <= my_pos && j + 4 > my_lo && j + 4 < k_end) ? s1[i] * scale_log2 : -INFINITY;
+          p[i] = (j >= k_lo && j < k_end) ? s0[i] * scale_log2 : -INFINITY;
+          p[4 + i] = (j + 4 >= k_lo && j + 4 < k_end) ? s1[i] * scale_log2 : -INFINITY;
           mx = fmaxf(mx, fmaxf(p[i], p[4 + i]));
         }
         mx = fmaxf(mx, __shfl_xor(mx, 16));
@@ -399,14 +371,13 @@ latent_attn_mfma_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_
         }
       }
     }
-    seg = end;
   }
 
   if (!wave_on) return;
   float lt = l + __shfl_xor(l, 16);
   lt += __shfl_xor(lt, 32);
   if (!col_ok) return;
-  if (DEC && n_splits > 1) {
+  if (n_splits > 1) {
     const int64_t p = (static_cast<int64_t>(row) * heads + head) * n_splits + blockIdx.z;
 #pragma unroll
     for (int d = 0; d < NR; ++d)
@@ -432,6 +403,11 @@ latent_attn_mfma_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_
 // decode != 0: one token per request (tokens == requests); with n_splits > 1 the keys are cut into that many slices,
 // part_o float32 [tokens * heads * n_splits, rank] and part_ml float32 [tokens * heads * n_splits, 2] take what the
 // slices leave, and out must be contiguous [tokens, heads, rank].  head_gate as for the plain kernel (bfloat16).
+int ix_latent_prefill(const void* ql, int64_t ql_t, int64_t ql_h, const void* qr, int64_t qr_t, int64_t qr_h,
+                      const void* cache, const int32_t* block_table, const int32_t* seq_of_token, const int32_t* positions,
+                      void* out, int64_t out_t, int64_t out_h, int tokens, int heads, int rank, int rot_dim, int page_size,
+                      int max_blocks, float scale_log2, int window, const void* head_gate, int64_t gate_stride,
+                      hipStream_t stream);  // latent_prefill.hip
 extern "C" int ix_latent_attention_mfma(const void* ql, int64_t ql_t, int64_t ql_h, const void* qr, int64_t qr_t,
                                         int64_t qr_h, const void* cache, const int32_t* block_table,
                                         const int32_t* seq_of_token, const int32_t* positions, void* out,
@@ -453,14 +429,16 @@ extern "C" int ix_latent_attention_mfma(const void* ql, int64_t ql_t, int64_t ql
              "slices need their workspace and a contiguous result");
   IX_REQUIRE(heads < 65536 * 4, "too many heads for one launch");
   if (tokens == 0) return 0;
-  const int n_tiles = static_cast<int>((tokens + 15) / 16);
+  if (!decode)
+    return ix_latent_prefill(ql, ql_t, ql_h, qr, qr_t, qr_h, cache, block_table, seq_of_token, positions, out, out_t, out_h,
+                             static_cast<int>(tokens), heads, rank, rot_dim, page_size, max_blocks,
+                             scale * 1.4426950408889634f, window, head_gate, gate_stride, stream);
   const size_t lds = (static_cast<size_t>(LATM_KEYS) * (((width + 63) & ~63) + LATM_KPAD) + static_cast<size_t>(rank) * LATM_VSTRIDE) * 2;
-  const dim3 grid = decode ? dim3(static_cast<unsigned>(tokens), (heads + 63) / 64, n_splits)
-                           : dim3(static_cast<unsigned>(n_tiles) * ((heads + 3) / 4), 1, 1);
+  const dim3 grid(static_cast<unsigned>(tokens), (heads + 63) / 64, n_splits);
   const float scale_log2 = scale * 1.4426950408889634f;
-#define LAUNCH(NW, NR, DEC)                                                                                             \
+#define LAUNCH(NW, NR)                                                                                                  \
   do {                                                                                                                  \
-    auto kernel = latent_attn_mfma_kernel<NW, NR, DEC>;                                                                 \
+    auto kernel = latent_attn_mfma_kernel<NW, NR>;                                                                      \
     if (lds > 48 * 1024) {                                                                                              \
       static bool raised = false;                                                                                       \
       if (!raised) {                                                                                                    \
@@ -474,14 +452,11 @@ extern "C" int ix_latent_attention_mfma(const void* ql, int64_t ql_t, int64_t ql
     hipLaunchKernelGGL(kernel, grid, dim3(256), lds, stream, (const __bf16*)ql, ql_t, ql_h, (const __bf16*)qr, qr_t,     \
                        qr_h, (const __bf16*)cache, block_table, seq_of_token, positions, (__bf16*)out, out_t, out_h,     \
                        part_o, part_ml, n_splits, static_cast<int>(tokens), heads, rank, rot_dim, page_size, max_blocks, \
-                       scale_log2, n_tiles, window, (const __bf16*)head_gate, gate_stride);                              \
+                       scale_log2, window, (const __bf16*)head_gate, gate_stride);                                       \
   } while (0)
-#define BY_SIZE(DEC)                                        \
-  if (width <= 128 && rank <= 128) LAUNCH(4, 8, DEC);       \
-  else if (width <= 320 && rank <= 256) LAUNCH(10, 16, DEC); \
-  else LAUNCH(18, 32, DEC)
-  if (decode) { BY_SIZE(true); } else { BY_SIZE(false); }
-#undef BY_SIZE
+  if (width <= 128 && rank <= 128) LAUNCH(4, 8);
+  else if (width <= 320 && rank <= 256) LAUNCH(10, 16);
+  else LAUNCH(18, 32);
 #undef LAUNCH
   if (ix_check_launch("ix_latent_attention_mfma")) return 1;
   if (n_splits > 1)

@@ -279,3 +279,31 @@ def test_norm_with_one_number():
     h = x.float().to(DEV)
     ops.add_rmsnorm(h, None, torch.full((24,), 1.3, dtype=torch.float32, device=DEV), out, 1e-5, None)
     assert torch.allclose(out.cpu().double(), want, atol=1e-5)
+
+
+# head groups that are not full, pages that eight keys do not share, all numbers of a row in its first 64 pieces or not
+@pytest.mark.parametrize("H,rank,rot,page", [(1, 512, 64, 16), (7, 512, 64, 12), (4, 256, 0, 8), (9, 480, 64, 16), (3, 16, 16, 4),
+                                             (16, 512, 32, 32)])
+@pytest.mark.parametrize("window,gated", [(0, False), (40, True)])
+def test_latent_attention_of_prompts(H, rank, rot, page, window, gated):
+    """Portions long enough for several rounds of 32 keys and both buffers, requests that share a tile of rows, portions on
+    contexts; against the plain kernel in float32 on the same numbers.  Weights and results are bfloat16: 2e-2."""
+    from inferx_amd import ops
+    contexts, lengths = [200, 33, 64, 97], [200, 20, 1, 40]
+    paged = Paged(contexts, rank + rot, page, torch.bfloat16, seed=5)
+    T, scale = sum(lengths), (rank + rot) ** -0.5
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=DEV)
+    seq = i32(np.repeat(np.arange(4), lengths).tolist())
+    pos = i32(np.concatenate([np.arange(c - n, c) for c, n in zip(contexts, lengths)]).tolist())
+    q = rnd((T, H, rank + 64), 6, 2.0, torch.bfloat16).to(DEV)
+    qr = rnd((T, H, max(rot, 8)), 7, 2.0, torch.bfloat16).to(DEV)[:, :, :rot] if rot else q
+    gate = rnd((T, H + 8), 8, 1.0, torch.bfloat16).to(DEV)[:, :H] if gated else None
+    cache, table = paged.cache.to(DEV), paged.table.to(DEV)
+    out = torch.full((H, T, rank), float("nan"), dtype=torch.bfloat16, device=DEV).transpose(0, 1)
+    assert ops.latent_mfma_fits(q[:, :, :rank], qr, out, rank, rot)
+    ops.latent_attention_mfma(q[:, :, :rank], qr, cache, table, seq, pos, out, rank, rot, scale, False, 1, None, window, gate)
+    want = torch.empty(T, H, rank, device=DEV)
+    f32 = lambda t: None if t is None else t.float().contiguous()
+    ops.latent_attention_plain(f32(q[:, :, :rank]), f32(qr), f32(cache), table, seq, pos, want, rank, rot, scale, window, f32(gate))
+    err = float((out.float() - want).abs().max()) / float(want.abs().max())
+    assert torch.isfinite(out).all() and err <= 2e-2, f"{err:.2e}"

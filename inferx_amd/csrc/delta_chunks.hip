@@ -17,14 +17,30 @@
 //             registers, the next chunk's operands on their way; leaves every chunk its U and the state before it;
 //   result    a workgroup per (chunk, head): O.
 //
+// The generalized delta rule (linear_state.hip has it: a decay w per row and key channel, a correction a (b^T S)),
+//
+//   S <- diag(w) S - a (b^T S) + k v^T;   o = S^T r
+//
+// goes the same way with y_i = b_i^T S_(i-1) and, per channel, G_i = w_0 .. w_i: b_i G_(i-1), a_j / G_j, k_j / G_j and
+// r_i G_i take the keys' places in
+//
+//   (I + A) Y = (B G) S + C V,  A_ij = (b_i G_(i-1)) . (a_j / G_j), C_ij with k_j for a_j  (j < i);   U = -Y
+//   O = (R G) S + P U + Q V,    P_ij = (r_i G_i) . (a_j / G_j), Q_ij with k_j              (j <= i)
+//   S_new = diag(G_n) S + sum_j (G_n / G_j) (a_j u_j^T + k_j v_j^T)
+//
+// where Q V and the k_j v_j^T, which need no state, are formed by the first launch.  The caller answers for 1 / G_63 being
+// a float32 number (a decay no smaller than e^-1).
+//
 // Everything is float32 (v_mfma_f32_16x16x4_f32) but the sums of the decays' logarithms, which are 64-bit so that the
-// ratio of two late rows is as exact as that of two early ones.
+// ratio of two late rows is as exact as that of two early ones (per channel: the decays' products).
 //
 // What bounds it: row by row, the chain of dependent sums of a row (0.33 us a row whatever the chip is doing).  In chunks
 // the chain is 64 times shorter and its step two small products (2.7 us a chunk).  Measured with 16 heads of 128 x 128, one
 // request, all three launches against row by row: 41 against 46 us at 128 rows, 47 against 72 at 200, 64 against 171 at
 // 500, 88 against 336 at 1,024, 150 against 667 at 2,048.  Results are 2.4e-7 of their norm from the float64 recurrence
-// (row by row 1.3e-7; with slow decays 4.2e-7 against 6.7e-7): the order of 32-bit sums.
+// (row by row 1.3e-7; with slow decays 4.2e-7 against 6.7e-7): the order of 32-bit sums.  The generalized rule, 32 heads
+// of 64 x 64: 34 against 44 us at 160 rows, 37 against 67 at 256, 130 against 493 at 2,048, where the first launch takes
+// 60, the chain 39 and the result 29; 1.2e-7 against 0.8e-7 of the result's norm.
 //
 // A lane's operand of a 16 x 16 x 4 product is one number of row (column) l % 16 at reduction index l / 16.  Operands
 // are read four numbers at a time, index 16 s + 4 (l / 16) + e, and the e-th of them meet in one instruction.
@@ -37,7 +53,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // where the parts of a (chunk, head) lie in its block of the workspace, in floats
 struct DeltaBlock {
-  int dim, vdim;
+  int dim, vdim, more;  // more: the generalized rule
   __host__ __device__ __forceinline__ int64_t w() const { return 0; }                          // [64][dim]: -W
   __host__ __device__ __forceinline__ int64_t kt() const { return 64 * dim; }                  // [dim][64]: (G_n / G_j) k_j
   __host__ __device__ __forceinline__ int64_t q() const { return 128 * dim; }                  // [64][dim]: G_i q_i
@@ -45,13 +61,56 @@ struct DeltaBlock {
   __host__ __device__ __forceinline__ int64_t u() const { return 192 * dim + 4096; }           // [vdim][64]: Uv, then U
   __host__ __device__ __forceinline__ int64_t s() const { return u() + 64 * vdim; }            // [vdim][dim]: S before
   __host__ __device__ __forceinline__ int64_t g() const { return s() + static_cast<int64_t>(dim) * vdim; }  // [dim]: G_n
-  __host__ __device__ __forceinline__ int64_t size() const { return g() + dim; }
+  __host__ __device__ __forceinline__ int64_t m() const { return g() + dim; }  // [vdim][dim]: sum_j (G_n / G_j) k_j v_j^T
+  __host__ __device__ __forceinline__ int64_t size() const { return m() + (more ? static_cast<int64_t>(dim) * vdim : 0); }
 };
 
 __device__ __forceinline__ f32x4 dc_mac(f32x4 a, f32x4 b, f32x4 acc) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], acc, 0, 0, 0);
   return acc;
+}
+
+// A (in LDS, strictly lower) -> the inverses of the blocks on the diagonal of I + A; one wavefront, lane (block, column)
+template <int LA>
+__device__ __forceinline__ void dc_invert_diagonal(const float* a_s, float (*t_s)[16][20], int b, int col) {
+  float x[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    float s = i == col ? 1.f : 0.f;
+    const float* ar = a_s + (16 * b + i) * LA + 16 * b;
+#pragma unroll
+    for (int j = 0; j < i; ++j) s = fmaf(-ar[j], x[j], s);
+    x[i] = s;
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) t_s[b][i][col] = x[i];
+}
+
+// x <- (I + A)^-1 x for NT tiles of sixteen columns: [tile][block of sixteen rows], a lane's numbers rows 4 g + e of column m
+template <int LA, int NT>
+__device__ __forceinline__ void dc_solve(const float* a_s, const float (*t_s)[16][20], int m, int g, f32x4 (&x)[NT][4]) {
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+#pragma unroll
+    for (int a = 0; a < b; ++a) {
+      const f32x4 na = -*reinterpret_cast<const f32x4*>(a_s + (16 * b + m) * LA + 16 * a + 4 * g);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) x[u][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(na[e], x[u][a][e], x[u][b], 0, 0, 0);
+    }
+    const f32x4 inv = *reinterpret_cast<const f32x4*>(&t_s[b][m][4 * g]);
+    f32x4 y[NT];
+#pragma unroll
+    for (int u = 0; u < NT; ++u) y[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int u = 0; u < NT; ++u) y[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(inv[e], x[u][b][e], y[u], 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < NT; ++u) x[u][b] = y[u];
+  }
 }
 
 template <int DIM>
@@ -75,7 +134,7 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
   const int kv = head / (heads / kv_heads);
   const int64_t row0 = chunk_row0[chunk];
   const int n = chunk_rows[chunk];
-  const DeltaBlock blk{DIM, vdim};
+  const DeltaBlock blk{DIM, vdim, 0};
   float* mine = work + (static_cast<int64_t>(chunk) * heads + head) * blk.size();
 
   // ---- unit rows into LDS: four threads a row, a quarter of its numbers each; rows past the chunk's end are zeros
@@ -174,20 +233,7 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
   __syncthreads();
 
   // ---- the diagonal blocks' inverses: lane (block, column), sixteen steps of substitution
-  if (wave == 0) {
-    const int b = g, col = m;
-    float x[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      float s = i == col ? 1.f : 0.f;
-      const float* ar = a_s + (16 * b + i) * LA + 16 * b;
-#pragma unroll
-      for (int j = 0; j < i; ++j) s = fmaf(-ar[j], x[j], s);
-      x[i] = s;
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) t_s[b][i][col] = x[i];
-  }
+  if (wave == 0) dc_invert_diagonal<LA>(a_s, t_s, g, m);
   __syncthreads();
 
   // ---- (I + A) [W | Uv] = [diag(beta G) K | diag(beta) V], four tiles of sixteen columns at a time and wavefront
@@ -207,27 +253,7 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
           else x[u][b][e] = beta_s[row] * ix_load(v + (row0 + min(row, n - 1)) * v_stride + head * vdim + 16 * t - DIM + m);
         }
     }
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-#pragma unroll
-      for (int a = 0; a < b; ++a) {
-        const f32x4 na = -*reinterpret_cast<const f32x4*>(a_s + (16 * b + m) * LA + 16 * a + 4 * g);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) x[u][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(na[e], x[u][a][e], x[u][b], 0, 0, 0);
-      }
-      const f32x4 inv = *reinterpret_cast<const f32x4*>(&t_s[b][m][4 * g]);
-      f32x4 y[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) y[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) y[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(inv[e], x[u][b][e], y[u], 0, 0, 0);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) x[u][b] = y[u];
-    }
+    dc_solve<LA, 4>(a_s, t_s, m, g, x);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int t = t0 + u;
@@ -245,8 +271,220 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
   }
 }
 
-// request blockIdx.z's chunks [first, first + count) one after the other, value columns 16 blockIdx.y ..
+// The generalized rule's first launch.  w, a, b float32 [T, heads * DIM]; r, k, v bfloat16 rows.
 template <int DIM>
+__global__ void __launch_bounds__(DC_THREADS, DIM <= 64 ? 2 : 1)
+general_chunks_prepare_kernel(const bf16_t* r, const bf16_t* k, const bf16_t* v, int64_t r_stride, int64_t k_stride,
+                              int64_t v_stride, const float* __restrict__ w_rows, const float* __restrict__ a_rows,
+                              const float* __restrict__ b_rows, const int32_t* __restrict__ chunk_row0,
+                              const int32_t* __restrict__ chunk_rows, float* __restrict__ work, float* __restrict__ out,
+                              int heads, int vdim) {
+  constexpr int LD = (DIM > DC_ROWS ? DIM : DC_ROWS) + 4;  // (a buffer also holds 64 x 64 scores)
+  constexpr int SEG = DIM / 4;                             // rows per thread: 256 / DIM threads share a channel
+  __shared__ __attribute__((aligned(16))) float x_s[4][DC_ROWS * LD];  // b G, a / G (then A), k / G (then C), r G (then Q)
+  __shared__ __attribute__((aligned(16))) float t_s[4][16][20];
+  __shared__ double seg_s[DC_THREADS / DIM][DIM];
+  __shared__ float gn_s[DIM];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m = lane & 15, g = lane >> 4;
+  const int head = blockIdx.x, chunk = blockIdx.y;
+  const int64_t row0 = chunk_row0[chunk];
+  const int n = chunk_rows[chunk];
+  const DeltaBlock blk{DIM, vdim, 1};
+  float* mine = work + (static_cast<int64_t>(chunk) * heads + head) * blk.size();
+  float *const b_s = x_s[0], *const a_s = x_s[1], *const k_s = x_s[2], *const r_s = x_s[3];
+
+  // ---- the decays' products down the rows, and the four operands scaled by them (everything is asked for before the first
+  // use and under no condition: loads that a condition guards come one after the other, 18 against 26 us for one chunk)
+  {
+    constexpr int PART = SEG < 16 ? SEG : 16;  // rows whose numbers are asked for together
+    const int d = tid % DIM, seg = tid / DIM;
+    const int64_t c = static_cast<int64_t>(head) * DIM + d, wide = static_cast<int64_t>(heads) * DIM;
+    auto at = [&](int i) { return row0 + min(seg * SEG + i, n - 1); };
+    float w[SEG];
+#pragma unroll
+    for (int i = 0; i < SEG; ++i) w[i] = w_rows[at(i) * wide + c];
+    float av[PART], bv[PART], kv[PART], rv[PART];
+    auto ask = [&](int i0) {
+#pragma unroll
+      for (int i = 0; i < PART; ++i) {
+        const int64_t t = at(i0 + i);
+        av[i] = a_rows[t * wide + c];
+        bv[i] = b_rows[t * wide + c];
+        kv[i] = ix_load(k + t * k_stride + c);
+        rv[i] = ix_load(r + t * r_stride + c);
+      }
+    };
+    ask(0);
+    __builtin_amdgcn_sched_barrier(0);
+    double p = 1.0;
+#pragma unroll
+    for (int i = 0; i < SEG; ++i) {
+      w[i] = seg * SEG + i < n ? w[i] : 1.0f;
+      p *= w[i];
+    }
+    seg_s[seg][d] = p;
+    __syncthreads();
+    p = 1.0;
+    for (int s = 0; s < seg; ++s) p *= seg_s[s][d];
+#pragma unroll
+    for (int i0 = 0; i0 < SEG; i0 += PART) {
+      if (i0 > 0) ask(i0);
+#pragma unroll
+      for (int i = 0; i < PART; ++i) {
+        const int row = seg * SEG + i0 + i;
+        const bool live = row < n;  // (one rounding each: the products are 64-bit)
+        b_s[row * LD + d] = live ? static_cast<float>(bv[i] * p) : 0.f;
+        p *= w[i0 + i];
+        const double over = 1.0 / p;
+        a_s[row * LD + d] = live ? static_cast<float>(av[i] * over) : 0.f;
+        k_s[row * LD + d] = live ? static_cast<float>(kv[i] * over) : 0.f;
+        const float rg = live ? static_cast<float>(rv[i] * p) : 0.f;
+        r_s[row * LD + d] = rg;
+        mine[blk.q() + row * DIM + d] = rg;
+        if (row == DC_ROWS - 1) {
+          gn_s[d] = static_cast<float>(p);
+          mine[blk.g() + d] = static_cast<float>(p);
+        }
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- the four score matrices, ten tiles on and below the diagonal each: P to the workspace, the others into registers
+  // (at most three tiles of each a wavefront) until their operands' buffers are free
+  auto score = [&](const float* left, const float* right, int pair, int& rt, int& ct) {
+    rt = pair < 1 ? 0 : (pair < 3 ? 1 : (pair < 6 ? 2 : 3));
+    ct = pair - rt * (rt + 1) / 2;
+    const float* ar = left + (16 * rt + m) * LD + 4 * g;
+    const float* br = right + (16 * ct + m) * LD + 4 * g;
+    f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+    for (int c = 0; c < DIM / 16; c += 2) {
+      s0 = dc_mac(*reinterpret_cast<const f32x4*>(ar + 16 * c), *reinterpret_cast<const f32x4*>(br + 16 * c), s0);
+      s1 = dc_mac(*reinterpret_cast<const f32x4*>(ar + 16 * c + 16), *reinterpret_cast<const f32x4*>(br + 16 * c + 16), s1);
+    }
+    return s0 + s1;
+  };
+  f32x4 qv[3], av[3], cv[3];
+#pragma unroll
+  for (int u = 0; u < 3; ++u) {
+    const int pair = wave + 4 * u, back = 3 - wave + 4 * u;  // (who has three tiles of two matrices has two of the others)
+    int rt, ct;
+    if (pair < 10) {
+      const f32x4 s = score(r_s, a_s, pair, rt, ct);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 16 * rt + 4 * g + e, j = 16 * ct + m;
+        mine[blk.p() + i * 64 + j] = j <= i ? s[e] : 0.f;
+      }
+      av[u] = score(b_s, a_s, pair, rt, ct);
+    }
+    if (back < 10) {
+      qv[u] = score(r_s, k_s, back, rt, ct);
+      cv[u] = score(b_s, k_s, back, rt, ct);
+    }
+  }
+  // ---- (G_n / G_j) a_j for the chain, and what k and v alone add to the state, a wavefront per tile of value columns
+  for (int id = tid; id < DIM * 16; id += DC_THREADS) {
+    const int d = id >> 4, jq = 4 * (id & 15);
+    f32x4 x;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = a_s[(jq + e) * LD + d] * gn_s[d];
+    *reinterpret_cast<f32x4*>(mine + blk.kt() + d * 64 + jq) = x;
+  }
+  const int vtiles = vdim / 16;
+  auto load_v = [&](int t, f32x4 (&x)[4]) {
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = 16 * b + 4 * g + e;
+        x[b][e] = ix_load(v + (row0 + min(row, n - 1)) * v_stride + head * vdim + 16 * t + m);  // (past the end: times 0)
+      }
+  };
+#pragma unroll 1
+  for (int t = wave; t < vtiles; t += 4) {
+    f32x4 x[4];
+    load_v(t, x);
+#pragma unroll 1
+    for (int dt = 0; dt < DIM / 16; ++dt) {
+      f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+      const float gn = gn_s[16 * dt + m];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        f32x4 kk;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) kk[e] = k_s[(16 * b + 4 * g + e) * LD + 16 * dt + m] * gn;
+        s = dc_mac(kk, x[b], s);
+      }
+      *reinterpret_cast<f32x4*>(mine + blk.m() + static_cast<int64_t>(16 * t + m) * DIM + 16 * dt + 4 * g) = s;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 3; ++u) {
+    const int pair = wave + 4 * u, back = 3 - wave + 4 * u;
+    auto place = [&](int pr, float* to, const f32x4& s, bool diagonal) {
+      const int rt = pr < 1 ? 0 : (pr < 3 ? 1 : (pr < 6 ? 2 : 3)), ct = pr - rt * (rt + 1) / 2;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 16 * rt + 4 * g + e, j = 16 * ct + m;
+        to[i * LD + j] = (j < i || (diagonal && j == i)) ? s[e] : 0.f;
+      }
+    };
+    if (pair < 10) place(pair, a_s, av[u], false);
+    if (back < 10) {
+      place(back, k_s, cv[u], false);
+      place(back, r_s, qv[u], true);
+    }
+  }
+  __syncthreads();
+  if (wave == 0) dc_invert_diagonal<LD>(a_s, t_s, g, m);
+  __syncthreads();
+
+  // ---- -W = -(I + A)^-1 (B G)
+#pragma unroll 1
+  for (int t = wave; t < DIM / 16; t += 4) {
+    f32x4 x[1][4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[0][b][e] = b_s[(16 * b + 4 * g + e) * LD + 16 * t + m];
+    dc_solve<LD, 1>(a_s, t_s, m, g, x);
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mine[blk.w() + (16 * b + 4 * g + e) * DIM + 16 * t + m] = -x[0][b][e];
+  }
+  // ---- Q V into the result, -(I + A)^-1 C V into U's place
+#pragma unroll 1
+  for (int t = wave; t < vtiles; t += 4) {
+    f32x4 x[4], z[1][4];
+    load_v(t, x);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f}, c = o;
+#pragma unroll
+      for (int a = 0; a <= b; ++a) {
+        o = dc_mac(*reinterpret_cast<const f32x4*>(r_s + (16 * b + m) * LD + 16 * a + 4 * g), x[a], o);
+        c = dc_mac(*reinterpret_cast<const f32x4*>(k_s + (16 * b + m) * LD + 16 * a + 4 * g), x[a], c);
+      }
+      z[0][b] = -c;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = 16 * b + 4 * g + e;
+        if (row < n) out[((row0 + row) * heads + head) * vdim + 16 * t + m] = o[e];
+      }
+    }
+    dc_solve<LD, 1>(a_s, t_s, m, g, z);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) *reinterpret_cast<f32x4*>(mine + blk.u() + (16 * t + m) * 64 + 16 * b + 4 * g) = z[0][b];
+  }
+}
+
+// request blockIdx.z's chunks [first, first + count) one after the other, value columns 16 blockIdx.y ..
+template <int DIM, bool MORE>
 __global__ void __launch_bounds__(DC_THREADS)
 delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, const int32_t* __restrict__ seq_first,
                           const int32_t* __restrict__ seq_count, const int32_t* __restrict__ state_slots,
@@ -265,7 +503,7 @@ delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, cons
   const int first = seq_first[seq], count = seq_count[seq];
   if (count <= 0) return;
   const bool owns = wave * TS < TILES;
-  const DeltaBlock blk{DIM, vdim};
+  const DeltaBlock blk{DIM, vdim, MORE};
   const int64_t size = blk.size(), step = heads * size;
   float* at0 = work + (static_cast<int64_t>(first) * heads + head) * size;
   float* sp = state + static_cast<int64_t>(state_slots[seq_ids[seq]]) * state_stride +
@@ -277,7 +515,7 @@ delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, cons
     row[t] = owns ? 16 * (wave * TS + t) + 4 * g : 0;
     st[t] = *reinterpret_cast<const f32x4*>(sp + row[t]);
   }
-  struct Operands { f32x4 w[TILES], kt[TS][4], u, gn[TS]; };
+  struct Operands { f32x4 w[TILES], kt[TS][4], u, gn[TS], add[MORE ? TS : 1]; };
   auto ask = [&](const float* p, Operands& o) {
 #pragma unroll
     for (int c = 0; c < TILES; ++c)
@@ -288,6 +526,7 @@ delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, cons
 #pragma unroll
       for (int s = 0; s < 4; ++s) o.kt[t][s] = *reinterpret_cast<const f32x4*>(p + blk.kt() + d * 64 + 16 * s + 4 * g);
       o.gn[t] = *reinterpret_cast<const f32x4*>(p + blk.g() + row[t]);
+      if constexpr (MORE) o.add[t] = *reinterpret_cast<const f32x4*>(p + blk.m() + static_cast<int64_t>(col) * DIM + row[t]);
     }
     o.u = *reinterpret_cast<const f32x4*>(p + blk.u() + col * 64 + 16 * wave + 4 * g);
     __builtin_amdgcn_sched_barrier(0);
@@ -320,7 +559,10 @@ delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, cons
     *reinterpret_cast<f32x4*>(u_s + m * LU + 16 * wave + 4 * g) = ua;
     *reinterpret_cast<f32x4*>(p + blk.u() + col * 64 + 16 * wave + 4 * g) = ua;
 #pragma unroll
-    for (int t = 0; t < TS; ++t) st[t] *= o.gn[t];
+    for (int t = 0; t < TS; ++t) {
+      st[t] *= o.gn[t];
+      if constexpr (MORE) st[t] += o.add[t];
+    }
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < 4; ++s) b[s] = *reinterpret_cast<const f32x4*>(u_s + m * LU + 16 * s + 4 * g);
@@ -350,7 +592,7 @@ delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, cons
 }
 
 // O^T = S^T (diag(G) Q)^T + U^T P^T: a lane ends up with four consecutive columns of a row
-template <int DIM>
+template <int DIM, bool MORE>
 __global__ void __launch_bounds__(DC_THREADS, 2)
 delta_chunks_result_kernel(const float* __restrict__ work, const int32_t* __restrict__ chunk_row0,
                            const int32_t* __restrict__ chunk_rows, float* __restrict__ out, int heads, int vdim) {
@@ -362,7 +604,7 @@ delta_chunks_result_kernel(const float* __restrict__ work, const int32_t* __rest
   const int head = blockIdx.x, chunk = blockIdx.y;
   const int64_t row0 = chunk_row0[chunk];
   const int n = chunk_rows[chunk];
-  const DeltaBlock blk{DIM, vdim};
+  const DeltaBlock blk{DIM, vdim, MORE};
   const float* mine = work + (static_cast<int64_t>(chunk) * heads + head) * blk.size();
 #pragma unroll
   for (int id = tid; id < DC_ROWS * DIM / 4; id += DC_THREADS) {
@@ -413,8 +655,11 @@ delta_chunks_result_kernel(const float* __restrict__ work, const int32_t* __rest
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = 16 * r + m;
-        if (row < n)
-          *reinterpret_cast<f32x4*>(out + ((row0 + row) * heads + head) * vdim + 16 * (t0 + u) + 4 * g) = acc[u][r];
+        if (row < n) {
+          f32x4* to = reinterpret_cast<f32x4*>(out + ((row0 + row) * heads + head) * vdim + 16 * (t0 + u) + 4 * g);
+          if constexpr (MORE) *to += acc[u][r];  // (Q V is there already)
+          else *to = acc[u][r];
+        }
       }
     }
   }
@@ -440,21 +685,56 @@ extern "C" int ix_delta_chunks(const void* q, const void* k, const void* v, int6
                reinterpret_cast<uintptr_t>(work) | reinterpret_cast<uintptr_t>(out)) & 15) == 0,
              "operands must lie on 16-byte boundaries");
   IX_REQUIRE(heads < 65536 && chunks < 65536 && seqs < 65536 && vdim / 16 < 65536, "too many heads, chunks or requests");
-  IX_REQUIRE(work_floats >= static_cast<int64_t>(chunks) * heads * (DeltaBlock{dim, vdim}).size(), "workspace too small");
+  IX_REQUIRE(work_floats >= static_cast<int64_t>(chunks) * heads * (DeltaBlock{dim, vdim, 0}).size(), "workspace too small");
   if (chunks == 0 || seqs == 0) return 0;
 #define RUN(DIM)                                                                                                         \
   hipLaunchKernelGGL(delta_chunks_prepare_kernel<DIM>, dim3(heads, chunks), dim3(DC_THREADS), 0, stream, (const bf16_t*)q, \
                      (const bf16_t*)k, (const bf16_t*)v, q_stride, k_stride, v_stride, ab, a_log, dt_bias, chunk_row0,   \
                      chunk_rows, work, heads, kv_heads, vdim);                                                           \
   if (ix_check_launch("ix_delta_chunks: prepare")) return 1;                                                             \
-  hipLaunchKernelGGL(delta_chunks_chain_kernel<DIM>, dim3(heads, vdim / 16, seqs), dim3(DC_THREADS), 0, stream, work,    \
+  hipLaunchKernelGGL((delta_chunks_chain_kernel<DIM, false>), dim3(heads, vdim / 16, seqs), dim3(DC_THREADS), 0, stream, work, \
                      seq_ids, seq_first, seq_count, state_slots, state, state_stride, heads, vdim);                      \
   if (ix_check_launch("ix_delta_chunks: chain")) return 1;                                                               \
-  hipLaunchKernelGGL(delta_chunks_result_kernel<DIM>, dim3(heads, chunks), dim3(DC_THREADS), 0, stream, work, chunk_row0, \
+  hipLaunchKernelGGL((delta_chunks_result_kernel<DIM, false>), dim3(heads, chunks), dim3(DC_THREADS), 0, stream, work, chunk_row0, \
                      chunk_rows, out, heads, vdim)
   if (dim == 32) { RUN(32); }
   else if (dim == 64) { RUN(64); }
   else { RUN(128); }
 #undef RUN
   return ix_check_launch("ix_delta_chunks");
+}
+
+// The generalized rule: r, k [T, heads * dim] and v [T, heads * vdim] bfloat16 rows, w, a, b float32 [T, heads * dim] as
+// ix_linear_state takes them (every decay between e^-1 and 1); the rest as above, blocks of the workspace with `m`.
+extern "C" int ix_general_delta_chunks(const void* r, const void* k, const void* v, int64_t r_stride, int64_t k_stride,
+                                       int64_t v_stride, const float* w_rows, const float* a_rows, const float* b_rows,
+                                       float* state, int64_t state_stride, const int32_t* state_slots,
+                                       const int32_t* chunk_row0, const int32_t* chunk_rows, int chunks,
+                                       const int32_t* seq_ids, const int32_t* seq_first, const int32_t* seq_count, int seqs,
+                                       float* work, int64_t work_floats, float* out, int heads, int dim, int vdim,
+                                       hipStream_t stream) {
+  IX_REQUIRE(chunks >= 0 && seqs >= 0 && heads > 0 && vdim > 0, "sizes must be positive");
+  IX_REQUIRE(dim == 32 || dim == 64 || dim == 128, "key heads of 32, 64 or 128 numbers");
+  IX_REQUIRE(vdim % 16 == 0, "value heads in multiples of 16 numbers");
+  IX_REQUIRE(state_stride >= static_cast<int64_t>(heads) * dim * vdim && state_stride % 4 == 0, "state blocks too small");
+  IX_REQUIRE(((reinterpret_cast<uintptr_t>(state) | reinterpret_cast<uintptr_t>(work) | reinterpret_cast<uintptr_t>(out)) & 15) == 0,
+             "state, workspace and result must lie on 16-byte boundaries");
+  IX_REQUIRE(heads < 65536 && chunks < 65536 && seqs < 65536 && vdim / 16 < 65536, "too many heads, chunks or requests");
+  IX_REQUIRE(work_floats >= static_cast<int64_t>(chunks) * heads * (DeltaBlock{dim, vdim, 1}).size(), "workspace too small");
+  if (chunks == 0 || seqs == 0) return 0;
+#define RUN(DIM)                                                                                                         \
+  hipLaunchKernelGGL(general_chunks_prepare_kernel<DIM>, dim3(heads, chunks), dim3(DC_THREADS), 0, stream,               \
+                     (const bf16_t*)r, (const bf16_t*)k, (const bf16_t*)v, r_stride, k_stride, v_stride, w_rows, a_rows, \
+                     b_rows, chunk_row0, chunk_rows, work, out, heads, vdim);                                            \
+  if (ix_check_launch("ix_general_delta_chunks: prepare")) return 1;                                                     \
+  hipLaunchKernelGGL((delta_chunks_chain_kernel<DIM, true>), dim3(heads, vdim / 16, seqs), dim3(DC_THREADS), 0, stream,  \
+                     work, seq_ids, seq_first, seq_count, state_slots, state, state_stride, heads, vdim);                \
+  if (ix_check_launch("ix_general_delta_chunks: chain")) return 1;                                                       \
+  hipLaunchKernelGGL((delta_chunks_result_kernel<DIM, true>), dim3(heads, chunks), dim3(DC_THREADS), 0, stream, work,    \
+                     chunk_row0, chunk_rows, out, heads, vdim)
+  if (dim == 32) { RUN(32); }
+  else if (dim == 64) { RUN(64); }
+  else { RUN(128); }
+#undef RUN
+  return ix_check_launch("ix_general_delta_chunks");
 }

@@ -1294,6 +1294,46 @@ def delta_chunks(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ab: torch.Te
           _i32(dim), _i32(vdim), _stream())
 
 
+def general_delta_fits(r: torch.Tensor, state: torch.Tensor, dim: int, vdim: int) -> bool:
+    """Whether `general_delta_chunks` takes these operands: bfloat16, key heads of 32, 64 or 128 numbers, value heads in
+    sixteens, the state on 16-byte boundaries."""
+    return (r.dtype == torch.bfloat16 and dim in (32, 64, 128) and vdim % 16 == 0 and state.stride(0) % 4 == 0
+            and state.data_ptr() % 16 == 0)
+
+
+def general_delta_floats(dim: int, vdim: int) -> int:
+    """Floats of workspace that `general_delta_chunks` takes per chunk and head (the entry point checks it)."""
+    return delta_chunks_floats(dim, vdim) + dim * vdim
+
+
+def general_delta_chunks(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Tensor, state_slots: torch.Tensor,
+                         chunks: torch.Tensor, seqs: torch.Tensor, out: torch.Tensor, heads: int, dim: int, vdim: int,
+                         w_rows: torch.Tensor, a_rows: torch.Tensor, b_rows: torch.Tensor) -> None:
+    """`linear_state` with decays and corrections per row, for the requests that `seqs` names, their rows in chunks whose
+    products are worked at the same time.  No decay may be below e^-1: 64 of them are divided by.  `chunks`, `seqs`: as
+    `linear_chunks` takes them."""
+    T = r.shape[0]
+    for t, n in ((r, heads * dim), (k, heads * dim), (v, heads * vdim)):
+        _need(t.dim() == 2 and t.shape == (T, n) and t.stride(1) == 1 and t.dtype == r.dtype and t.is_cuda, "r, k or v shape")
+    for t in (w_rows, a_rows, b_rows):
+        _need(t.dtype == torch.float32 and t.shape == (T, heads * dim) and t.is_contiguous(),
+              "the rows of decays and corrections must be float32 [T, heads * dim]")
+    _need(state.dtype == torch.float32 and state.dim() == 2 and state.stride(1) == 1
+          and state.shape[1] >= heads * dim * vdim, "the state must be float32 [slots, >= heads * dim * vdim]")
+    _need(out.dtype == torch.float32 and out.shape == (T, heads, vdim), "out must be float32 [T, heads, vdim]")
+    _need(general_delta_fits(r, state, dim, vdim), "operands that the chunked form does not take")
+    _is_i32(state_slots)
+    for t, n in ((chunks, 2), (seqs, 3)):
+        _is_i32(t)
+        _need(t.dim() == 2 and t.shape[0] == n and t.is_contiguous(), "chunks int32 [2, n], seqs int32 [3, m]")
+    work = torch.empty((chunks.shape[1] * heads * general_delta_floats(dim, vdim),), dtype=torch.float32, device=r.device)
+    _call("ix_general_delta_chunks", r.data_ptr(), k.data_ptr(), v.data_ptr(), _i64(r.stride(0)), _i64(k.stride(0)),
+          _i64(v.stride(0)), _ptr(w_rows), _ptr(a_rows), _ptr(b_rows), state.data_ptr(), _i64(state.stride(0)),
+          _ptr(state_slots), _ptr(chunks[0]), _ptr(chunks[1]), _i32(chunks.shape[1]), _ptr(seqs[0]), _ptr(seqs[1]),
+          _ptr(seqs[2]), _i32(seqs.shape[1]), _ptr(work), _i64(work.numel()), _ptr(out), _i32(heads), _i32(dim), _i32(vdim),
+          _stream())
+
+
 def channel_decays(logits: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor, heads: int, dim: int) -> None:
     """logits float32 [T, heads * dim] in place: exp(-exp(a_log[h]) softplus(logit + dt_bias[h, i])), the decay of
     every head's every key channel."""

@@ -25,7 +25,7 @@ import torch
 from .. import ops
 from .base import Mixer, ParamSpec, StateNeed, register_part
 from .dense_mlp import stack_rows
-from .linear_state import chunk_slices
+from .linear_state import CHUNK_WORKSPACE, chunk_slices
 from .short_conv import ShortConv
 
 # A step goes through the chunked form if some request brings at least CHUNKED_FROM_ROWS rows (16 heads of 128 x 128: 41
@@ -33,7 +33,6 @@ from .short_conv import ShortConv
 # others row by row.
 CHUNKED_FROM_ROWS = 112
 CHUNKED_MIN_ROWS = 16
-CHUNK_WORKSPACE = 128 << 20  # bytes that the chunks worked at the same time may take; longer steps go in slices
 
 
 class GatedDeltaMixer(Mixer):

@@ -19,8 +19,8 @@
     q, k, v = x . W^T;   q, k rotated by the token's position;   S <- decay_h S + (k dim^(-1/2)) v^T;   o = S^T q
     y = (o / rms(o over the head) * silu(x . Wg^T)) . Wo^T
 
-With a decay per head, the portions of a step that bring many rows are worked in chunks of 64 rows at the same time
-(`ops.linear_chunks`), the others row by row.
+The portions of a step that bring many rows are worked in chunks of 64 rows (`ops.linear_chunks`,
+`ops.general_delta_chunks`), the others row by row.
 
 State, decays, rates, unit keys, the recurrence and the norms are float32 in every run; nothing is kept in pages.
 """
@@ -36,6 +36,13 @@ from .. import ops
 from ..config.spec import PartSpec
 from .base import Mixer, ParamSpec, StateNeed, build_part, register_part
 from .dense_mlp import stack_rows
+
+
+# A step goes through the generalized delta rule's chunked form if some request brings at least this many rows, where it
+# is no slower at any size of head (rows against chunks at 160 rows: 27 and 26 us for 32 heads of 32 numbers, 44 and 34
+# for 32 of 64, 58 and 58 for 16 of 128; at 112 rows 22 and 25, 34 and 32, 42 and 55).
+CORRECTED_FROM_ROWS = 160
+CHUNK_WORKSPACE = 128 << 20  # bytes that the chunks worked at the same time may take; longer steps go in slices
 
 
 class GeneralizedDelta(Mixer):
@@ -79,8 +86,19 @@ class GeneralizedDelta(Mixer):
         w, a, u = (rt.empty((T, C), torch.float32) for _ in range(3))
         ops.delta_operands(w_logit, self.w0, rate, self.a_bias, k, w, a, u, H, D, self.decay_scale, self.unit_eps)
         o = rt.empty((T, H, D), torch.float32)
-        ops.linear_state(r, k, v, cache.state, ops.StepRows(ctx.seq_of_token, ctx.q_start, ctx.state_slots), o, H, D, D,
-                         w_rows=w, a_rows=a, b_rows=u)
+        rows = ops.StepRows(ctx.seq_of_token, ctx.q_start, ctx.state_slots)
+        n = None if ctx.one_token_each else ctx.host.q_start[1:] - ctx.host.q_start[:-1]
+        # (a decay below e^-1 would take the products of 64 of them out of float32's range)
+        if (n is not None and n.max() >= CORRECTED_FROM_ROWS and 0.0 <= self.decay_scale <= 1.0
+                and ops.general_delta_fits(r, cache.state, D, D)):
+            if ((n > 0) & (n < CHUNKED_MIN_ROWS)).any():
+                ops.linear_state(r, k, v, cache.state, rows, o, H, D, D, w_rows=w, a_rows=a, b_rows=u,
+                                 max_rows=CHUNKED_MIN_ROWS - 1)
+            most = max(1, CHUNK_WORKSPACE // (4 * H * ops.general_delta_floats(D, D)))
+            for chunks, seqs in chunk_slices(ctx, CHUNKED_MIN_ROWS, most):
+                ops.general_delta_chunks(r, k, v, cache.state, ctx.state_slots, chunks, seqs, o, H, D, D, w, a, u)
+        else:
+            ops.linear_state(r, k, v, cache.state, rows, o, H, D, D, w_rows=w, a_rows=a, b_rows=u)
         y = rt.empty((T, C))
         ops.head_norm_gate(o, y, self.norm_eps, weight=self.norm_weight, gate=gate, weight_per_head=True,
                            gate_sigmoid=True)

@@ -101,6 +101,56 @@ def test_recurrence_over_steps_and_slots(H, D, V, corrected, dtype):
     assert bool(torch.isnan(state[1]).all()), "a slot of no request was written"
 
 
+# rows of the requests of a step (one of them without any), around chunks of 64 and the sixteens within them
+@pytest.mark.parametrize("lengths", [[1, 15, 0, 16], [17, 64, 63], [65, 130]])
+@pytest.mark.parametrize("H,D,V", [(3, 32, 48), (2, 64, 64), (1, 128, 144)])
+@pytest.mark.parametrize("decay,same_key", [(0.6, False), (1.0, False), (1e-3, False), (0.6, True)])
+def test_generalized_delta_rule_in_chunks(lengths, H, D, V, decay, same_key):
+    """The chunked form against the float64 recurrence, from a state that is not zero, its last state too; in one call and
+    cut into slices of two chunks; with the strongest decays that it takes (e^-1 a row), hardly any, and one unit key
+    for all rows.  float32 sums of at most D + 64 products of numbers up to the results' size: 1e-5 of the largest."""
+    from inferx_amd import ops
+    T, S = sum(lengths), len(lengths)
+    strided = rnd((T, 3 * H * (D + 1)), 1, 0.7, torch.bfloat16)  # rows neither dense nor on 16-byte boundaries
+    r, k = strided[:, 1:1 + H * D], strided[:, H * (D + 1):H * (D + 1) + H * D]
+    v = rnd((T, H * V), 3, 1.0, torch.bfloat16)
+    logit = rnd((T, H * D), 4, 3.0)
+    w = torch.exp(-decay * (torch.ones_like(logit) if decay == 1.0 else torch.sigmoid(logit)))
+    u = rnd((1 if same_key else T, H, D), 5).expand(T, H, D)
+    u = (u / u.norm(dim=2, keepdim=True)).reshape(T, H * D).contiguous()
+    a = (u * torch.sigmoid(rnd((T, H * D), 6))).contiguous()
+    before = rnd((S + 1, H * D * V + 4), 7, 0.3)
+    starts = [sum(lengths[:s]) for s in range(S + 1)]
+    row0 = [(s, starts[s] + at, min(64, n - at)) for s, n in enumerate(lengths) for at in range(0, n, 64)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    slots = i32([S - s for s in range(S)])
+    on = strided.to(DEV)
+    r_dev, k_dev = on[:, 1:1 + H * D], on[:, H * (D + 1):H * (D + 1) + H * D]
+    for most in (1000, 2):
+        state = before.to(DEV)
+        out = torch.full((T, H, V), float("nan"), device=DEV)
+        for first in range(0, len(row0), most):
+            part = row0[first:first + most]
+            live = sorted({s for s, _, _ in part})
+            ops.general_delta_chunks(r_dev, k_dev, v.to(DEV), state, slots,
+                                     i32([[x[1] for x in part], [x[2] for x in part]]),
+                                     i32([live, [[x[0] for x in part].index(s) for s in live],
+                                          [sum(x[0] == s for x in part) for s in live]]),
+                                     out, H, D, V, w.to(DEV), a.to(DEV), u.to(DEV))
+        for s, n in enumerate(lengths):
+            slot, at = S - s, slice(starts[s], starts[s] + n)
+            if n == 0:
+                assert torch.equal(state[slot].cpu(), before[slot])
+                continue
+            M = before[slot, :H * D * V].double().view(H, V, D).transpose(1, 2).clone()
+            rows = [x[at].double().view(n, H, -1) for x in (r, k, v, w, a, u)]
+            want = plain_recurrence(*rows, M)
+            assert float((out[at].cpu().double() - want).abs().max()) <= 1e-5 * float(want.abs().max()), f"request {s}"
+            left = state[slot, :H * D * V].cpu().double().view(H, V, D).transpose(1, 2)
+            assert float((left - M).abs().max()) <= 1e-5 * float(M.abs().max()), f"state of request {s}"
+            assert torch.equal(state[slot, H * D * V:].cpu(), before[slot, H * D * V:])
+
+
 def test_delta_operands_and_the_plain_mixer_agree():
     """decay, removal and unit key as the kernel makes them against the plain mixer's formulas."""
     from inferx_amd import ops

@@ -747,11 +747,11 @@ def moe_tiled_rows(wide: bool) -> int:
 
 def moe_grouped_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offsets: torch.Tensor,
                       rows: Optional[torch.Tensor], tile_map: torch.Tensor, gate_up: bool, wide: bool = False,
-                      glu_limit: float = 0.0, last_tiles: int = 0) -> None:
+                      glu_limit: float = 0.0, last_tiles: int = 0, last_each: int = 1) -> None:
     """Grouped product staged through LDS (bfloat16, many rows per expert); `tile_map` made for tiles of
     `moe_tiled_rows(wide)` rows.  `wide`: 256 instead of 128 weight rows per workgroup (the same sums in the same
-    order; which rows share a tile, and with it where a row's sum starts, differs).  `last_tiles`: so many tiles at
-    the end of the map are worked spread among the others (any number gives the same results)."""
+    order).  `last_tiles`: so many tiles at the end of the map are worked spread among the others, `last_each`
+    consecutive ones of them belong to one expert (any number gives the same results)."""
     E = w.shape[0]
     A, n_out = out.shape
     K = a.shape[1]
@@ -769,7 +769,7 @@ def moe_grouped_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offse
     _is_i32(tile_map, 2 * mt + 1)
     _call("ix_moe_grouped_tiled", _ptr(a), _ptr(w), _ptr(out), _ptr(offsets), _ptr(rows), _ptr(tile_map[:mt]),
           _ptr(tile_map[mt:2 * mt]), _ptr(tile_map[2 * mt:]), _i32(mt), _i64(a.shape[0]), _i64(n_out), _i64(K),
-          _i32(_epilogue(gate_up)), _i32(1 if wide else 0), _f32(glu_limit), _i32(last_tiles), _stream())
+          _i32(_epilogue(gate_up)), _i32(1 if wide else 0), _f32(glu_limit), _i32(last_tiles), _i32(last_each), _stream())
 
 
 def moe_grouped_tiled_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offsets: torch.Tensor,

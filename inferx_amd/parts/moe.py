@@ -37,8 +37,8 @@ SHARED_BESIDE_TOKENS = 512
 # shared expert stays on the main stream (a wide workgroup fills a compute unit's LDS, the library's kernels find
 # no place beside it).  Measured, prompt portions at a width of 3,584 (64 experts of 2,560, 8 per token): 14.9 against
 # 15.5 ms for a mixed step of 1,056 tokens and 8 layers, 2.86 against 3.03 s for 193,000 tokens of long prompts; at a
-# width of 2,048 (60 experts of 1,408, 4 per token) the narrow form beside the shared expert is ahead, 15.2 against
-# 16.0 ms for 2,048 tokens and 24 layers.
+# width of 2,048 (60 experts of 1,408, 4 per token) the narrow form beside the shared expert is ahead, 5.19 against
+# 5.30 ms for 2,048 tokens and 8 layers.
 WIDE_TILES_WIDTH = 3072
 # Between the few rows of a decoding step (where routed and shared experts already share a launch) and the portions
 # from which the shared expert's library products run beside the routed experts, the shared expert is cut into
@@ -206,11 +206,12 @@ class MoeFeedForward(FeedForward):
             ops.moe_grouped_tiled_f32(x, w13, act, offsets, rows, tile_map, self.first_epilogue, self.limit)
             ops.moe_grouped_tiled_f32(act, w2, y, offsets, None, tile_map, False)
         elif tile_rows == ops.moe_tiled_rows(self.wide_tiles):  # many rows per expert: operands staged through LDS
+            wide = self.wide_tiles
             # (a piece of the shared expert holds every token: its tiles are full, and the last ones of the map)
-            full = self.shared_pieces * -(-x.shape[0] // tile_rows) if with_shared else 0
-            ops.moe_grouped_tiled(x, w13, act, offsets, rows, tile_map, self.first_epilogue, self.wide_tiles, self.limit,
-                                  full)
-            ops.moe_grouped_tiled(act, w2, y, offsets, None, tile_map, False, self.wide_tiles, 0.0, full)
+            each = -(-x.shape[0] // tile_rows)
+            full = self.shared_pieces * each if with_shared else 0
+            ops.moe_grouped_tiled(x, w13, act, offsets, rows, tile_map, self.first_epilogue, wide, self.limit, full, each)
+            ops.moe_grouped_tiled(act, w2, y, offsets, None, tile_map, False, wide, 0.0, full, each)
         elif tile_rows:
             # few rows: the weights are the traffic, the reduction is split over a workgroup's four wavefronts
             ops.moe_grouped_mfma(x, w13, act, offsets, rows, tile_map, tile_rows, self.first_epilogue, 4, self.limit)

@@ -289,6 +289,34 @@ def test_grouped_tiled_order_of_the_last_tiles(last, wide):
     assert torch.isfinite(out[0]).all() and torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
 
 
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("T,E,mi", [(30, 12, 160), (330, 5, 520), (500, 9, 72)])
+@pytest.mark.parametrize("pieces", [1, 2, 4])
+def test_grouped_tiled_last_tiles_of_one_expert_together(T, E, mi, pieces, wide):
+    """The last experts hold every row (one to four tiles each); their tiles, worked expert by expert and spread over the
+    dies, with more and with fewer tiles than the others have, change no bit.  Reductions of 1 to 9 stages of 64, whole
+    and not."""
+    from inferx_amd import ops
+    g = torch.Generator().manual_seed(1)
+    top = torch.stack([torch.randperm(E, generator=g)[:1] for _ in range(T)])
+    always = torch.arange(E, E + pieces).expand(T, pieces)
+    topk_e = torch.cat([top, always], 1).to(torch.int32).to(DEV)
+    offsets, rows, dest, tile_map = dispatch(topk_e, E + pieces, ops.moe_tiled_rows(wide))
+    each = -(-T // ops.moe_tiled_rows(wide))
+    for H in (64, 200, 256, 320, 512, 576):
+        x = rnd(T, H, dtype=torch.bfloat16)
+        w = rnd(E + pieces, mi, H, seed=2, dtype=torch.bfloat16, scale=H ** -0.5)
+        out = [torch.full((topk_e.numel(), mi), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+        ops.moe_grouped_tiled(x, w, out[0], offsets, rows, tile_map, False, wide)
+        ops.moe_grouped_tiled(x, w, out[1], offsets, rows, tile_map, False, wide, last_tiles=pieces * each, last_each=each)
+        assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+        for t in (0, T // 2, T - 1):
+            for c in range(1 + pieces):
+                want = x[t].double().cpu() @ w[int(topk_e[t, c])].double().cpu().T
+                got = out[0][int(dest[t * (1 + pieces) + c])].double().cpu()
+                assert float((got - want).abs().max()) <= 2 ** -8 * float(want.abs().max()) + 1e-5, (H, t, c)
+
+
 @pytest.mark.parametrize("T,N,K", [(3, 40, 264), (16, 33, 1160), (2, 16, 8), (5, 48, 520)])
 def test_streaming_kernels_read_nothing_past_their_operands(T, N, K):
     """Reduction widths that leave a wavefront a ragged last round: what lies behind the last row of the weights

@@ -59,7 +59,8 @@ template <int MT, bool GATE_UP, int KSPLIT, typename TI, typename TO, int NB = 1
 __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
                                              TO* __restrict__ out, const int32_t* __restrict__ rows, int e,
                                              int row0, int row_end, int n0, int n_out, int width, float* red,
-                                             int act = 0, float glu_limit = 0.f) {
+                                             int act = 0, float glu_limit = 0.f, const void* bias = nullptr,
+                                             int bias_dtype = 0) {
   typedef MfmaPiece<TI> Piece;
   typedef typename Piece::type piece_t;
   constexpr int PN = Piece::N, ROUND = 16 * PN;  // numbers of a piece; of a round of four loads
@@ -148,7 +149,7 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
   }
 
   if (KSPLIT > 1) {
-    // wavefronts 1..3 hand their partial sums to wavefront 0
+    // the other wavefronts hand their partial sums to wavefront 0
     if (wave > 0) {
       float* dst = red + ((wave - 1) * 64 + lane) * (MT * NACC * 4);
 #pragma unroll
@@ -184,8 +185,14 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         v[i] = acc[u][t][i];
-        if constexpr (GATE_UP) v[i] = ix_glu<sizeof(TI) == 2>(v[i], acc[NB + u][t][i], glu_limit);
-        else if (act) v[i] = v[i] > 0.f ? v[i] * v[i] : 0.f;  // the square of relu
+        const int c = min(nb + i, n_out - 1);
+        if (bias) v[i] += ix_load_rt(bias, bias_dtype, c);
+        if constexpr (GATE_UP) {
+          float up = acc[NB + u][t][i];
+          if (bias) up += ix_load_rt(bias, bias_dtype, static_cast<int64_t>(n_out) + c);
+          v[i] = ix_glu<sizeof(TI) == 2>(v[i], up, glu_limit);
+        }
+        if (!GATE_UP && act) v[i] = v[i] > 0.f ? v[i] * v[i] : 0.f;  // the square of relu
       }
       TO* dst = out + static_cast<int64_t>(r) * n_out + nb;
       if (nb + 4 <= n_out && (n_out & 3) == 0) {
@@ -204,15 +211,15 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
   }
 }
 
-// x [rows <= 16 * MT, width] . w[n_out, width]^T -> float32 [rows, n_out]: the head of a decoding step, whose
-// logits stay float32 (one workgroup per 32 out-features, so that the rows, which every workgroup reads, weigh
-// less beside the weights; the reduction split over its four wavefronts).
-template <int MT, typename TI>
-__global__ void __launch_bounds__(256, MT == 1 ? 4 : 1)
-linear_skinny_f32_kernel(const TI* x, const TI* w, float* __restrict__ out,
-                         int rows, int n_out, int width) {
-  __shared__ float red[3 * 64 * MT * 2 * 4];
-  grouped_body<MT, false, 4, TI, float, 2>(x, w, out, nullptr, 0, 0, rows, blockIdx.x * 32, n_out, width, red);
+// x [rows <= 16 * MT, width] . w^T -> [rows, n_out], the products of a decoding step: 16 NB out-features a workgroup, the
+// reduction split over its KSPLIT wavefronts.
+template <int MT, bool GATE_UP, int KSPLIT, int NB, typename TI, typename TO>
+__global__ void __launch_bounds__(64 * KSPLIT, MT == 1 ? 4 : 1)
+linear_skinny_kernel(const TI* x, const TI* w, TO* __restrict__ out, const void* bias, int bias_dtype, int rows, int n_out,
+                     int width, float glu_limit) {
+  __shared__ float red[(KSPLIT - 1) * 64 * MT * NB * (GATE_UP ? 2 : 1) * 4];
+  grouped_body<MT, GATE_UP, KSPLIT, TI, TO, NB>(x, w, out, nullptr, 0, 0, rows, blockIdx.x * 16 * NB, n_out, width, red, 0,
+                                                glu_limit, bias, bias_dtype);
 }
 
 template <int MT, bool GATE_UP, int KSPLIT, typename TI>
@@ -346,21 +353,49 @@ extern "C" int ix_moe_grouped_dual(const void* a, const void* w, void* out, int 
   return ix_check_launch("ix_moe_grouped_dual");
 }
 
-// out float32 [rows, n_out] = x [rows, width] . w[n_out, width]^T, rows <= 64, operands of `dtype`.
-extern "C" int ix_linear_skinny_f32(const void* x, const void* w, int dtype, float* out, int rows, int64_t n_out,
-                                    int64_t width, hipStream_t stream) {
+// out [rows, n_out] = x [rows, width] . w[n_out, width]^T, rows <= 64, operands of `dtype`; out of `dtype` or float32.
+// gate_up 1: w is [2 n_out, width], gate rows and then up rows, which meet in the gated unit (`ix_glu` with glu_limit).
+// `bias`: as many numbers as w has rows, added to the sums (to both before they meet), or null.
+//
+// What bounds it: the weights, and where they are few the launch itself and how many bytes a compute unit has on their
+// way.  A product of the run's type is a workgroup of 16 out-features; with no more of them than the chip has compute
+// units eight wavefronts split its reduction instead of four.  The float32 result (the logits) has so many out-features
+// that 32 a workgroup are better: the rows, which every workgroup reads, weigh less beside the weights.
+// Eight rows: 2,048 features of 2,048 numbers 5.7 us (6.3 with four wavefronts, by way of a grouping of one expert, whose
+// tables a workgroup reads before its weights); a gated unit with biases saves the launch behind it, 6.2 us.
+extern "C" int ix_linear_skinny(const void* x, const void* w, int dtype, void* out, int out_f32, const void* bias,
+                                int bias_dtype, int rows, int64_t n_out, int64_t width, int gate_up, float glu_limit,
+                                hipStream_t stream) {
   IX_REQUIRE(rows > 0 && rows <= 64 && n_out > 0 && width > 0, "between 1 and 64 rows, positive sizes");
   IX_REQUIRE_PIECES(dtype, width);
-  IX_REQUIRE(n_out < (1ll << 31) - 16 && width < (1 << 30), "sizes too large");
-  dim3 grid(static_cast<unsigned>((n_out + 31) / 32)), block(256);
-#define LAUNCH(MT, TI)                                                                                       \
-  hipLaunchKernelGGL((linear_skinny_f32_kernel<MT, TI>), grid, block, 0, stream, (const TI*)x, (const TI*)w, out, rows, \
-                     (int)n_out, (int)width)
-#define PICK(MT)                       \
-  if (dtype == IX_F32) LAUNCH(MT, float); \
-  else LAUNCH(MT, __bf16);
-  if (rows <= 16) { PICK(1) } else if (rows <= 32) { PICK(2) } else { PICK(4) }
-#undef PICK
+  IX_REQUIRE(n_out < (1ll << 31) - 32 && width < (1 << 30), "sizes too large");
+  IX_REQUIRE(!out_f32 || !gate_up, "the gated unit's result is of the operands' type");
+  const int per = out_f32 ? 32 : 16;
+  const unsigned blocks = static_cast<unsigned>((n_out + per - 1) / per);
+  const bool split8 = !out_f32 && blocks <= 256 && rows <= 32;
+#define LAUNCH(MT, GU, KS, NB, TI, TO)                                                                                      \
+  hipLaunchKernelGGL((linear_skinny_kernel<MT, GU, KS, NB, TI, TO>), dim3(blocks), dim3(64 * KS), 0, stream, (const TI*)x, \
+                     (const TI*)w, (TO*)out, bias, bias_dtype, rows, (int)n_out, (int)width, glu_limit)
+#define BY_FORM(MT, KS, TI)                        \
+  if (gate_up) LAUNCH(MT, true, KS, 1, TI, TI);    \
+  else LAUNCH(MT, false, KS, 1, TI, TI)
+#define BY_ROWS(TI)                                      \
+  if (split8 && rows <= 16) { BY_FORM(1, 8, TI); }       \
+  else if (split8) { BY_FORM(2, 8, TI); }                \
+  else if (rows <= 16) { BY_FORM(1, 4, TI); }            \
+  else if (rows <= 32) { BY_FORM(2, 4, TI); }            \
+  else { BY_FORM(4, 4, TI); }
+#define LOGITS(TI)                                              \
+  if (rows <= 16) LAUNCH(1, false, 4, 2, TI, float);            \
+  else if (rows <= 32) LAUNCH(2, false, 4, 2, TI, float);       \
+  else LAUNCH(4, false, 4, 2, TI, float)
+  if (out_f32 && dtype == IX_F32) { LOGITS(float); }
+  else if (out_f32) { LOGITS(__bf16); }
+  else if (dtype == IX_F32) { BY_ROWS(float) }
+  else { BY_ROWS(__bf16) }
+#undef LOGITS
+#undef BY_ROWS
+#undef BY_FORM
 #undef LAUNCH
-  return ix_check_launch("ix_linear_skinny_f32");
+  return ix_check_launch("ix_linear_skinny");
 }

@@ -41,7 +41,6 @@ class Runtime:
         from .. import ops
         ops.lib()  # fail now, loudly, if the HIP library cannot be had
         self._mm_out_dtype_ok: Optional[bool] = None
-        self._skinny_plans: Dict[int, Any] = {}
         self._side_stream: Optional[torch.cuda.Stream] = None
 
     @property
@@ -99,20 +98,11 @@ class Runtime:
             return x.shape[1] % 4 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0
         return x.dtype == torch.bfloat16 and x.shape[1] % 8 == 0
 
-    def _skinny(self, x: torch.Tensor, w: torch.Tensor, gate_up: bool, limit: float = 0.0) -> torch.Tensor:
+    def _skinny(self, x: torch.Tensor, w: torch.Tensor, gate_up: bool, limit: float = 0.0,
+                bias: Optional[torch.Tensor] = None) -> torch.Tensor:
         from .. import ops
-        T = x.shape[0]
-        plan = self._skinny_plans.get(T)
-        if plan is None:
-            tile_rows = 16 if T <= 16 else (32 if T <= 32 else 64)
-            mt = ops.moe_max_tiles(T, 1, tile_rows)
-            tile_map = torch.tensor([0] * (2 * mt) + [1], dtype=torch.int32, device=self.device)
-            offsets = torch.tensor([0, T], dtype=torch.int32, device=self.device)
-            plan = self._skinny_plans[T] = (offsets, tile_map, tile_rows)
-        offsets, tile_map, tile_rows = plan
-        n_out = w.shape[0] // 2 if gate_up else w.shape[0]
-        out = self.empty((T, n_out), x.dtype)
-        ops.moe_grouped_mfma(x, w.unsqueeze(0), out, offsets, None, tile_map, tile_rows, gate_up, 4, limit)
+        out = self.empty((x.shape[0], w.shape[0] // 2 if gate_up else w.shape[0]), x.dtype)
+        ops.linear_skinny(x, w, out, gate_up, limit, bias)
         return out
 
     def linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -136,8 +126,8 @@ class Runtime:
         """silu(x . Wg^T) * (x . Wu^T) for w_gate_up = [Wg; Wu] of shape [2 n, in] -> [T, n].  `bias` (2 n numbers) is
         added to both products first; with `limit` other than 0 they meet in another form (see `ops.glu_bias`)."""
         from .. import ops
-        if bias is None and self._skinny_ok(x, w_gate_up):
-            return self._skinny(x, w_gate_up, True, limit)
+        if self._skinny_ok(x, w_gate_up):
+            return self._skinny(x, w_gate_up, True, limit, bias)
         gate_up = self.linear(x, w_gate_up)
         act = self.empty((x.shape[0], w_gate_up.shape[0] // 2))
         if bias is None and limit == 0:

@@ -725,15 +725,32 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
     return True
 
 
+def linear_skinny(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate_up: bool = False, glu_limit: float = 0.0,
+                  bias: Optional[torch.Tensor] = None) -> None:
+    """out [T, N] = x [T, K] . w[N, K]^T for at most 64 rows, all three bfloat16 or all float32.  `gate_up`: w is [2 N, K],
+    gate rows and then up rows, which meet as in `glu_bias` with `glu_limit`.  `bias` (as many numbers as w has rows) is
+    added to the sums, to both before they meet."""
+    _need(out.dtype == x.dtype, "a result of the operands' type")
+    _linear_skinny(x, w, out, gate_up, glu_limit, bias)
+
+
 def linear_skinny_f32(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
     """out float32 [T, N] = x [T, K] . w[N, K]^T for at most 64 rows, operands both bfloat16 or both float32 (the head
     of a decode step)."""
-    T, K = x.shape
     _need(out.dtype == torch.float32, "a float32 result")
+    _linear_skinny(x, w, out, False, 0.0, None, True)
+
+
+def _linear_skinny(x, w, out, gate_up, glu_limit, bias, out_f32: bool = False) -> None:
+    T, K = x.shape
     _need_pieces(x, w)
-    _need(w.dim() == 2 and w.shape[1] == K and out.shape == (T, w.shape[0]), "shapes do not fit")
+    _need(w.dim() == 2 and w.shape[1] == K and out.shape == (T, w.shape[0] // 2 if gate_up else w.shape[0])
+          and (not gate_up or w.shape[0] % 2 == 0), "shapes do not fit")
+    _need(bias is None or bias.numel() == w.shape[0], "one bias per row of the weights")
     _need(0 < T <= 64, "between 1 and 64 rows")
-    _call("ix_linear_skinny_f32", _ptr(x), _ptr(w), _i32(_dt(x)), _ptr(out), _i32(T), _i64(w.shape[0]), _i64(K), _stream())
+    _call("ix_linear_skinny", _ptr(x), _ptr(w), _i32(_dt(x)), _ptr(out), _i32(1 if out_f32 else 0), _ptr(bias),
+          _i32(_dt(bias) if bias is not None else F32), _i32(T), _i64(out.shape[1]), _i64(K), _i32(1 if gate_up else 0),
+          _f32(glu_limit), _stream())
 
 
 MOE_TILED_F32_ROWS = 64  # rows per tile of the LDS-staged grouped product in float32

@@ -317,6 +317,35 @@ def test_grouped_tiled_last_tiles_of_one_expert_together(T, E, mi, pieces, wide)
                 assert float((got - want).abs().max()) <= 2 ** -8 * float(want.abs().max()) + 1e-5, (H, t, c)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T", [1, 17, 64])
+@pytest.mark.parametrize("N,K", [(33, 8), (4096, 1160), (4100, 264)])  # at most 256 blocks of sixteen, and more
+@pytest.mark.parametrize("form", [None, 0.0, 1.5, -1.0])  # a plain product; gate|up rows by the unit's limit
+@pytest.mark.parametrize("biased", [False, True])
+def test_dense_products_of_few_rows(dtype, T, N, K, form, biased):
+    """x . w^T in one launch with the gated unit and the biases behind it, against float64.  The bound is the result's own
+    rounding (half of a bfloat16's last place, at most 2^-8 of the number) and that of K float32 sums on both of a unit's sides."""
+    from inferx_amd import ops
+    rows = N if form is None else 2 * N
+    x, w = rnd(T, K, dtype=dtype), rnd(rows, K, seed=1, dtype=dtype, scale=K ** -0.5)
+    bias = rnd(rows, seed=2, dtype=dtype) if biased else None
+    out = torch.full((T, N), float("nan"), dtype=dtype, device=DEV)
+    ops.linear_skinny(x, w, out, form is not None, form or 0.0, bias)
+    want = x.double() @ w.double().T + (bias.double() if biased else 0.0)
+    if form is not None:
+        g, u = want[:, :N], want[:, N:]
+        if form > 0:
+            g, u = g.clamp(max=form), u.clamp(-form, form) + 1.0
+            want = g * torch.sigmoid(1.702 * g) * u
+        elif form < 0:
+            want = torch.nn.functional.gelu(g, approximate="tanh") * u
+        else:
+            want = torch.nn.functional.silu(g) * u
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -22
+    err = (out.double() - want).abs()
+    assert float((err - eps * want.abs()).max()) <= 4e-5, float(err.max())
+
+
 @pytest.mark.parametrize("T,N,K", [(3, 40, 264), (16, 33, 1160), (2, 16, 8), (5, 48, 520)])
 def test_streaming_kernels_read_nothing_past_their_operands(T, N, K):
     """Reduction widths that leave a wavefront a ragged last round: what lies behind the last row of the weights

@@ -25,7 +25,7 @@ import torch
 from .. import ops
 from .base import Mixer, ParamSpec, StateNeed, register_part
 from .dense_mlp import stack_rows
-from .linear_state import CHUNK_WORKSPACE, chunk_slices
+from .linear_state import CHUNK_WORKSPACE, chunk_slices, longest_portion, shorter_portions
 from .short_conv import ShortConv
 
 # A step goes through the chunked form if some request brings at least CHUNKED_FROM_ROWS rows (16 heads of 128 x 128: 41
@@ -118,10 +118,9 @@ class GatedDeltaMixer(Mixer):
         o = rt.empty((T, self.num_heads, self.value_dim), torch.float32)
         sizes = (self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim)
         rows = ops.StepRows(ctx.seq_of_token, ctx.q_start, ctx.state_slots)
-        n = None if ctx.one_token_each else ctx.host.q_start[1:] - ctx.host.q_start[:-1]
-        if (n is not None and channel_logits is None and n.max() >= CHUNKED_FROM_ROWS
+        if (channel_logits is None and longest_portion(ctx) >= CHUNKED_FROM_ROWS
                 and ops.delta_chunks_fits(q, k, matrices, self.head_dim, self.value_dim)):
-            if ((n > 0) & (n < CHUNKED_MIN_ROWS)).any():
+            if shorter_portions(ctx, CHUNKED_MIN_ROWS):
                 ops.delta_rule(q, k, v, ab, self.a_log, self.dt_bias, matrices, rows, o, *sizes, max_rows=CHUNKED_MIN_ROWS - 1)
             most = max(1, CHUNK_WORKSPACE // (4 * self.num_heads * ops.delta_chunks_floats(self.head_dim, self.value_dim)))
             for chunks, seqs in chunk_slices(ctx, CHUNKED_MIN_ROWS, most):

@@ -87,11 +87,10 @@ class GeneralizedDelta(Mixer):
         ops.delta_operands(w_logit, self.w0, rate, self.a_bias, k, w, a, u, H, D, self.decay_scale, self.unit_eps)
         o = rt.empty((T, H, D), torch.float32)
         rows = ops.StepRows(ctx.seq_of_token, ctx.q_start, ctx.state_slots)
-        n = None if ctx.one_token_each else ctx.host.q_start[1:] - ctx.host.q_start[:-1]
         # (a decay below e^-1 would take the products of 64 of them out of float32's range)
-        if (n is not None and n.max() >= CORRECTED_FROM_ROWS and 0.0 <= self.decay_scale <= 1.0
+        if (longest_portion(ctx) >= CORRECTED_FROM_ROWS and 0.0 <= self.decay_scale <= 1.0
                 and ops.general_delta_fits(r, cache.state, D, D)):
-            if ((n > 0) & (n < CHUNKED_MIN_ROWS)).any():
+            if shorter_portions(ctx, CHUNKED_MIN_ROWS):
                 ops.linear_state(r, k, v, cache.state, rows, o, H, D, D, w_rows=w, a_rows=a, b_rows=u,
                                  max_rows=CHUNKED_MIN_ROWS - 1)
             most = max(1, CHUNK_WORKSPACE // (4 * H * ops.general_delta_floats(D, D)))
@@ -106,6 +105,22 @@ class GeneralizedDelta(Mixer):
 
 
 CHUNKED_MIN_ROWS = 16  # portions of at least this many rows are worked in chunks
+
+
+def longest_portion(ctx) -> int:
+    """The most rows that a request of the step brings, as far as the choice of a recurrence's form goes (0 in a step of
+    one token per request, which may have no host data)."""
+    if ctx.one_token_each:
+        return 0
+    if "longest_portion" not in ctx.memo:
+        ctx.memo["longest_portion"] = int((ctx.host.q_start[1:] - ctx.host.q_start[:-1]).max())
+    return ctx.memo["longest_portion"]
+
+
+def shorter_portions(ctx, rows: int) -> bool:
+    """Whether some request of the step brings fewer rows than `rows`."""
+    n = ctx.host.q_start[1:] - ctx.host.q_start[:-1]
+    return bool(((n > 0) & (n < rows)).any())
 
 
 def _on_device(ctx, chunks, seqs):

@@ -175,7 +175,10 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
     const bool live = lane < n;
     const int64_t row = row0 + min(lane, n - 1);
     const float x = ab[row * 2 * heads + head] + dt_bias[head];
-    const float lg = live ? -expf(a_log[head]) * (x > 20.f ? x : log1pf(expf(x))) : 0.f;
+    float lg = live ? -expf(a_log[head]) * (x > 20.f ? x : log1pf(expf(x))) : 0.f;
+    // (a decay of e^-200 is zero in float32; below that, and at minus infinity, the differences of the sums, which are the
+    // ratios of the rows that come after, would lose those rows' own logarithms.  NaN stays.)
+    if (lg < -200.f) lg = -200.f;
     double c = lg;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {

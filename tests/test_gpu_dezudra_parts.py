@@ -669,3 +669,36 @@ def test_delta_rule_leaves_long_requests_to_others():
     assert torch.equal(all_out[:3], some_out[:3]) and torch.equal(all_out[43:], some_out[43:])
     assert torch.equal(all_state[[0, 2]], some_state[[0, 2]])
     assert (some_out[3:43] == 7.0).all() and torch.equal(some_state[1], rnd((3, heads * dim * vdim), 7)[1])
+
+
+@pytest.mark.parametrize("how", ["infinite logit", "rate that overflows", "huge rate"])
+def test_delta_rule_in_chunks_forgets_all_at_once(how):
+    """A decay of exactly zero in the middle of a chunk: the rows after it go on from what it left, each with its own
+    decay, as row by row.  Both forms are float32: their sums' orders differ by less than 1e-5 of the largest number."""
+    from inferx_amd import ops
+    T, heads, dim, vdim, at = 100, 2, 64, 32, (5, 40, 70)
+    q, k, v = (rnd((T, heads * n), s, 1.0, torch.bfloat16).to(DEV) for s, n in ((1, dim), (2, dim), (3, vdim)))
+    ab, a_log, dt_bias = rnd((T, 2 * heads), 4, 1.5), rnd((heads,), 5), rnd((heads,), 6)
+    if how == "infinite logit":
+        ab[list(at), :heads] = math.inf
+    else:  # the other rows forget next to nothing beside it
+        a_log[:] = 80.0 if how == "rate that overflows" else 40.0
+        ab[:, :heads] = -80.0 if how == "rate that overflows" else -40.0
+        ab[list(at), :heads] = 3e4
+        dt_bias[:] = 0.0
+    ab, a_log, dt_bias = ab.to(DEV), a_log.to(DEV), dt_bias.to(DEV)
+    before = rnd((1, heads * dim * vdim), 7, 0.3)
+    slots, results = i32([0]), []
+    for chunked in (False, True):
+        state, out = before.to(DEV), torch.full((T, heads, vdim), float("nan"), device=DEV)
+        if chunked:
+            ops.delta_chunks(q, k, v, ab, a_log, dt_bias, state, slots, i32([[0, 64], [64, 36]]), i32([[0], [0], [2]]), out,
+                             heads, heads, dim, vdim)
+        else:
+            ops.delta_rule(q, k, v, ab, a_log, dt_bias, state, ops.StepRows(i32([0] * T), i32([0, T]), slots), out, heads,
+                           heads, dim, vdim)
+        results.append((out.cpu(), state.cpu()))
+    (want, left), (out, state) = results
+    assert torch.isfinite(want).all() and torch.isfinite(left).all()
+    close(out, f64(want), 1e-5, "result")
+    close(state, f64(left), 1e-5, "state")

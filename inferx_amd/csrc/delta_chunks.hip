@@ -71,6 +71,48 @@ __device__ __forceinline__ f32x4 dc_mac(f32x4 a, f32x4 b, f32x4 acc) {
   return acc;
 }
 
+// Numbers that are not finite stay with their row and the later ones, as row by row.  A triangular block of sixteen rows
+// keeps zeros for the rows that a row does not see, but zero times NaN is NaN: where a block's operand holds such numbers,
+// it is multiplied without them, and the results that see one of them become NaN.  `seen`: this lane's numbers of a matrix
+// that holds 1 where the triangle does.
+__device__ __forceinline__ bool dc_odd(const f32x4 x) {  // is any of them not finite?  (the products are 0 or NaN)
+  return !(x[0] * 0.f + x[1] * 0.f + (x[2] * 0.f + x[3] * 0.f) == 0.f);
+}
+__device__ __forceinline__ f32x4 dc_seen(int row, int first, bool own) {  // rows first + e that `row` sees, its own with `own`
+  f32x4 s;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) s[e] = first + e < row + (own ? 1 : 0) ? 1.f : 0.f;
+  return s;
+}
+// the operand x without its numbers that are not finite, and where they were
+__device__ __forceinline__ void dc_part(const f32x4 x, f32x4& clean, f32x4& odd) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const bool bad = !(x[e] * 0.f == 0.f);
+    clean[e] = bad ? 0.f : x[e];
+    odd[e] = bad ? 1.f : 0.f;
+  }
+}
+__device__ __forceinline__ f32x4 dc_spoil(const f32x4 x, const f32x4 count) {
+  f32x4 y;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = count[e] > 0.f ? __builtin_nanf("") : x[e];
+  return y;
+}
+// acc + the product of a triangular block with x: the block is the first operand, or the second one
+__device__ __forceinline__ f32x4 dc_mac_block(f32x4 block, f32x4 x, f32x4 seen, f32x4 acc) {
+  const f32x4 none = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 clean, odd;
+  dc_part(x, clean, odd);
+  return dc_spoil(dc_mac(block, clean, acc), dc_mac(seen, odd, none));
+}
+__device__ __forceinline__ f32x4 dc_mac_block_second(f32x4 x, f32x4 block, f32x4 seen, f32x4 acc) {
+  const f32x4 none = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 clean, odd;
+  dc_part(x, clean, odd);
+  return dc_spoil(dc_mac(clean, block, acc), dc_mac(odd, seen, none));
+}
+
 // A (in LDS, strictly lower) -> the inverses of the blocks on the diagonal of I + A; one wavefront, lane (block, column)
 template <int LA>
 __device__ __forceinline__ void dc_invert_diagonal(const float* a_s, float (*t_s)[16][20], int b, int col) {
@@ -104,10 +146,18 @@ __device__ __forceinline__ void dc_solve(const float* a_s, const float (*t_s)[16
     f32x4 y[NT];
 #pragma unroll
     for (int u = 0; u < NT; ++u) y[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bool odd = false;
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
+    for (int u = 0; u < NT; ++u) odd = odd || dc_odd(x[u][b]);
+    if (__any(odd)) {
 #pragma unroll
-      for (int u = 0; u < NT; ++u) y[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(inv[e], x[u][b][e], y[u], 0, 0, 0);
+      for (int u = 0; u < NT; ++u) y[u] = dc_mac_block(inv, x[u][b], dc_seen(m, 4 * g, true), y[u]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) y[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(inv[e], x[u][b][e], y[u], 0, 0, 0);
+    }
 #pragma unroll
     for (int u = 0; u < NT; ++u) x[u][b] = y[u];
   }
@@ -470,8 +520,15 @@ general_chunks_prepare_kernel(const bf16_t* r, const bf16_t* k, const bf16_t* v,
       f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f}, c = o;
 #pragma unroll
       for (int a = 0; a <= b; ++a) {
-        o = dc_mac(*reinterpret_cast<const f32x4*>(r_s + (16 * b + m) * LD + 16 * a + 4 * g), x[a], o);
-        c = dc_mac(*reinterpret_cast<const f32x4*>(k_s + (16 * b + m) * LD + 16 * a + 4 * g), x[a], c);
+        const f32x4 ra = *reinterpret_cast<const f32x4*>(r_s + (16 * b + m) * LD + 16 * a + 4 * g);
+        const f32x4 ka = *reinterpret_cast<const f32x4*>(k_s + (16 * b + m) * LD + 16 * a + 4 * g);
+        if (a == b && __any(dc_odd(x[a]))) {
+          o = dc_mac_block(ra, x[a], dc_seen(m, 4 * g, true), o);
+          c = dc_mac_block(ka, x[a], dc_seen(m, 4 * g, false), c);
+        } else {
+          o = dc_mac(ra, x[a], o);
+          c = dc_mac(ka, x[a], c);
+        }
       }
       z[0][b] = -c;
 #pragma unroll
@@ -645,11 +702,18 @@ delta_chunks_result_kernel(const float* __restrict__ work, const int32_t* __rest
     for (int s = 0; s < 4; ++s) {
       const f32x4 a0 = *reinterpret_cast<const f32x4*>(mine + blk.u() + (16 * t0 + m) * 64 + 16 * s + 4 * g);
       const f32x4 a1 = *reinterpret_cast<const f32x4*>(mine + blk.u() + (16 * t1 + m) * 64 + 16 * s + 4 * g);
+      const bool odd = __any(dc_odd(a0) || dc_odd(a1));
 #pragma unroll
       for (int r = s; r < 4; ++r) {
         const f32x4 b = *reinterpret_cast<const f32x4*>(p_s + (16 * r + m) * LP + 16 * s + 4 * g);
-        acc[0][r] = dc_mac(a0, b, acc[0][r]);
-        acc[1][r] = dc_mac(a1, b, acc[1][r]);
+        if (r == s && odd) {
+          const f32x4 seen = dc_seen(m, 4 * g, true);
+          acc[0][r] = dc_mac_block_second(a0, b, seen, acc[0][r]);
+          acc[1][r] = dc_mac_block_second(a1, b, seen, acc[1][r]);
+        } else {
+          acc[0][r] = dc_mac(a0, b, acc[0][r]);
+          acc[1][r] = dc_mac(a1, b, acc[1][r]);
+        }
       }
     }
 #pragma unroll

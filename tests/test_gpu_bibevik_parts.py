@@ -357,3 +357,44 @@ def test_latent_attention_of_prompts(H, rank, rot, page, window, gated):
     ops.latent_attention_plain(f32(q[:, :, :rank]), f32(qr), f32(cache), table, seq, pos, want, rank, rot, scale, window, f32(gate))
     err = float((out.float() - want).abs().max()) / float(want.abs().max())
     assert torch.isfinite(out).all() and err <= 2e-2, f"{err:.2e}"
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("row", [0, 7, 37, 64, 99])
+def test_generalized_delta_rule_in_chunks_keeps_what_is_not_finite_to_later_rows(row, bad):
+    """A number that is not finite reaches what the recurrence lets it reach and nothing else: a value its column from its row
+    on, a reading vector its row, a key, a decay, a removal vector or a direction all columns from its row on.
+    Everything else keeps its bits."""
+    from inferx_amd import ops
+    T, H, D, V = 100, 3, 64, 48  # one chunk and the next one, 36 rows
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=DEV)
+    before = rnd((1, H * D * V), 7, 0.3)
+
+    def run(where=None):
+        ops_ = [rnd((T, H * D), 1, 0.7, torch.bfloat16), rnd((T, H * D), 2, 0.7, torch.bfloat16), rnd((T, H * V), 3, 1.0, torch.bfloat16),
+                torch.exp(-0.6 * torch.sigmoid(rnd((T, H * D), 4))), rnd((T, H * D), 5, D ** -0.5), rnd((T, H * D), 6, D ** -0.5)]
+        if where is not None:
+            ops_[where][row, (V if where == 2 else D) + 5] = bad  # head 1, number 5
+        r, k, v, w, a, b = (t.to(DEV) for t in ops_)
+        state, out = before.to(DEV), torch.full((T, H, V), 7.0, device=DEV)
+        ops.general_delta_chunks(r, k, v, state, i32([0]), i32([[0, 64], [64, 36]]), i32([[0], [0], [2]]), out, H, D, V, w, a, b)
+        return out.cpu(), state.cpu().view(H, V, D)
+
+    want, left = run()
+    assert torch.isfinite(want).all() and torch.isfinite(left).all()
+    for where in range(6):
+        out, state = run(where)
+        before_it = torch.ones(T, dtype=torch.bool)
+        before_it[row:] = False
+        assert torch.equal(out[before_it], want[before_it]), f"operand {where}: an earlier row"
+        assert torch.equal(out[:, [0, 2]], want[:, [0, 2]]) and torch.equal(state[[0, 2]], left[[0, 2]]), "another head"
+        if where == 2:
+            others = torch.arange(V) != 5
+            assert torch.equal(out[:, 1, others], want[:, 1, others]) and torch.equal(state[1, others], left[1, others])
+            assert not torch.isfinite(out[row:, 1, 5]).any() and not torch.isfinite(state[1, 5, 5]).any()
+        elif where == 0:
+            later = torch.arange(T) != row
+            assert torch.equal(out[later], want[later]) and torch.equal(state, left)
+            assert not torch.isfinite(out[row, 1]).any()
+        else:
+            assert not torch.isfinite(out[row:, 1]).any()

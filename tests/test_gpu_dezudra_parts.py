@@ -702,3 +702,40 @@ def test_delta_rule_in_chunks_forgets_all_at_once(how):
     assert torch.isfinite(want).all() and torch.isfinite(left).all()
     close(out, f64(want), 1e-5, "result")
     close(state, f64(left), 1e-5, "state")
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("row", [0, 7, 37, 64, 99])
+def test_delta_rule_in_chunks_keeps_what_is_not_finite_to_later_rows(row, bad):
+    """A value, a key or a query that is not finite reaches what the recurrence lets it reach and nothing else: a value its
+    column from its row on, a key all columns from its row on, a query its row; everything else keeps its bits."""
+    from inferx_amd import ops
+    T, heads, dim, vdim = 100, 3, 64, 48  # one chunk and the next one, 36 rows
+    a_log, dt_bias, before = rnd((heads,), 5).to(DEV), rnd((heads,), 6).to(DEV), rnd((1, heads * dim * vdim), 7, 0.3)
+    ab = rnd((T, 2 * heads), 4, 1.5).to(DEV)
+
+    def run(where=None):
+        qkv = [rnd((T, heads * n), s, 1.0, torch.bfloat16) for s, n in ((1, dim), (2, dim), (3, vdim))]
+        if where is not None:
+            n = (dim, dim, vdim)[where]
+            qkv[where][row, n + 5] = bad  # head 1, number 5
+        q, k, v = (t.to(DEV) for t in qkv)
+        state, out = before.to(DEV), torch.full((T, heads, vdim), 7.0, device=DEV)
+        ops.delta_chunks(q, k, v, ab, a_log, dt_bias, state, i32([0]), i32([[0, 64], [64, 36]]), i32([[0], [0], [2]]), out, heads,
+                         heads, dim, vdim)
+        return out.cpu(), state.cpu().view(heads, vdim, dim)
+
+    want, left = run()
+    assert torch.isfinite(want).all() and torch.isfinite(left).all()
+    for where in range(3):
+        out, state = run(where)
+        reached = torch.zeros(T, heads, vdim, dtype=torch.bool)
+        reached_state = torch.zeros(heads, vdim, dim, dtype=torch.bool)
+        if where == 0:
+            reached[row, 1] = True
+        elif where == 1:
+            reached[row:, 1], reached_state[1] = True, True
+        else:
+            reached[row:, 1, 5], reached_state[1, 5] = True, True
+        for got, full, on in ((out, want, reached), (state, left, reached_state)):
+            assert not torch.isfinite(got[on]).any() and torch.equal(got[~on], full[~on]), f"operand {where}"

@@ -25,8 +25,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define AF_KEYS 16  // keys per round
 
-// head_dim = 16 NB
-template <int NB, bool GQ>
+// head_dim = 16 NB.  MANY: a tile may hold several queries (tiles of one do without the registers of that case: a decoding
+// step of eight requests, 4 layers, takes 1,353 us, with them 1,391)
+template <int NB, bool GQ, bool MANY>
 __global__ void __launch_bounds__(256)
 attn_f32_kernel(const float* q, const float* k_cache, const float* v_cache, const int32_t* __restrict__ block_table,
                 const int32_t* __restrict__ tile_seq, const int32_t* __restrict__ tile_q0,
@@ -65,6 +66,7 @@ attn_f32_kernel(const float* q, const float* k_cache, const float* v_cache, cons
                    : f32x4{0.f, 0.f, 0.f, 0.f};
   const int my_pos = pos0 + (GQ ? 0 : n);
   const int my_lo = GQ ? lo : ix_first_key(my_pos, span);
+  const int last_lo = GQ ? lo : ix_first_key(pos0 + rows - 1, span);  // the first key of the tile's last query
 
   f32x4 o[NB];
 #pragma unroll
@@ -129,6 +131,37 @@ attn_f32_kernel(const float* q, const float* k_cache, const float* v_cache, cons
 #pragma unroll
           for (int b = 0; b < NB; ++b) vf[b][i] = 0.f;
         }
+      }
+    }
+    // Likewise a key of the request itself that some queries of the tile see and others do not: where its value is not
+    // finite, the others' zero weights would take it up.
+    if (MANY && rows > 1 && (kb + AF_KEYS - 1 > pos0 || kb < last_lo)) {
+      float z = 0.f;  // (0 or NaN)
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z = fmaf(vf[b][i], 0.f, z);
+      if (__any(z != 0.f)) {
+        f32x4 seen;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = kb + 4 * g + i;
+          seen[i] = key >= my_lo && key <= my_pos ? 1.f : 0.f;
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          f32x4 clean = o[b], count = f32x4{0.f, 0.f, 0.f, 0.f};  // without such values; how many of them a query sees
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const bool odd = !(vf[b][i] * 0.f == 0.f);
+            clean = __builtin_amdgcn_mfma_f32_16x16x4f32(odd ? 0.f : vf[b][i], p[i], clean, 0, 0, 0);
+            count = __builtin_amdgcn_mfma_f32_16x16x4f32(odd ? 1.f : 0.f, seen[i], count, 0, 0, 0);
+            o[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[b][i], p[i], o[b], 0, 0, 0);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[b][i] = count[i] > 0.f ? o[b][i] : clean[i];
+        }
+        return;
       }
     }
 #pragma unroll
@@ -248,11 +281,15 @@ extern "C" int ix_attention_f32(const float* q, const float* k_cache, const floa
 #define CASE(NB)                                                                                                     \
   case NB:                                                                                                           \
     if (grouped)                                                                                                     \
-      hipLaunchKernelGGL((attn_f32_kernel<NB, true>), grid, block, 0, stream, q, k_cache, v_cache, block_table, tile_seq, \
+      hipLaunchKernelGGL((attn_f32_kernel<NB, true, false>), grid, block, 0, stream, q, k_cache, v_cache, block_table, tile_seq, \
+                         tile_q0, tile_rows, positions, out, part_o, part_ml, n_tiles, n_splits, heads, kv_heads,    \
+                         page_size, max_blocks, scale, span, sink, softcap);                                         \
+    else if (n_tiles >= tokens) /* tiles of one query each */                                                         \
+      hipLaunchKernelGGL((attn_f32_kernel<NB, false, false>), grid, block, 0, stream, q, k_cache, v_cache, block_table, tile_seq, \
                          tile_q0, tile_rows, positions, out, part_o, part_ml, n_tiles, n_splits, heads, kv_heads,    \
                          page_size, max_blocks, scale, span, sink, softcap);                                         \
     else                                                                                                             \
-      hipLaunchKernelGGL((attn_f32_kernel<NB, false>), grid, block, 0, stream, q, k_cache, v_cache, block_table, tile_seq, \
+      hipLaunchKernelGGL((attn_f32_kernel<NB, false, true>), grid, block, 0, stream, q, k_cache, v_cache, block_table, tile_seq, \
                          tile_q0, tile_rows, positions, out, part_o, part_ml, n_tiles, n_splits, heads, kv_heads,    \
                          page_size, max_blocks, scale, span, sink, softcap);                                         \
     break;

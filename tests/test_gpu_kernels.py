@@ -393,3 +393,44 @@ def test_attention_f32_options_agree_with_the_plain_kernel(softcap, with_sink, s
                       work, 0.3, span, False, sink, softcap)
     assert torch.isfinite(want).all()
     close(out, want, TOL[torch.float32], "attention_f32")
+
+
+@pytest.mark.parametrize("span", [0, 5, -6])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", ["key", "value"])
+@pytest.mark.parametrize("row", [0, 9, 21, 39])
+def test_attention_f32_keeps_what_is_not_finite_to_the_queries_that_see_it(row, where, bad, span):
+    """One number of a portion's keys or values that is not finite: the queries that see it are what the plain kernel says,
+    to the last one, and the others keep their bits."""
+    from inferx_amd import ops
+    heads, kv_heads, d, page, n, before = 2, 1, 32, 16, 40, 20
+    p = build_paged([before + n], [n], heads, kv_heads, d, page, torch.float32, seed=6)
+    pg, off = int(p["table"][0, (before + row) // page]), (before + row) % page
+    outs = {}
+    for spoilt in (False, True):
+        if spoilt:
+            (p["k_cache"][pg, 0, off] if where == "key" else p["v_cache"][pg, 0, :, off])[7] = bad
+        for name in ("plain", "mfma"):
+            out = torch.full_like(p["q"], float("inf"))
+            if name == "plain":
+                ops.attention_plain(p["q"], p["k_cache"], p["v_cache"], p["table"], p["seq_of_token"], p["positions"], out, 0.3,
+                                    span, None, None, 0.0)
+            else:
+                ops.attention_f32(p["q"], p["k_cache"], p["v_cache"], p["table"], tiles_for([n]), p["positions"], out, 1, None,
+                                  0.3, span)
+            outs[name, spoilt] = out.cpu()
+    pos = torch.arange(before, before + n)
+    start = (pos - span + 1).clamp(min=0) if span > 0 else (pos - pos % -span if span < 0 else torch.zeros_like(pos))
+    sees = (pos >= before + row) & (start <= before + row)
+    assert 0 < int(sees.sum())
+    assert torch.equal(outs["mfma", True][~sees], outs["mfma", False][~sees]), "a query that does not see it"
+    if where == "value":
+        hit = torch.zeros_like(outs["mfma", True], dtype=torch.bool)
+        hit[sees, :, 7] = True
+        assert torch.equal(outs["mfma", True][~hit], outs["mfma", False][~hit]), "another column"
+        assert not torch.isfinite(outs["mfma", True][hit]).any() and not torch.isfinite(outs["plain", True][hit]).any()
+    else:
+        finite = torch.isfinite(outs["plain", True])
+        assert torch.equal(torch.isfinite(outs["mfma", True]), finite)
+        if finite.any():
+            close(outs["mfma", True][finite], outs["plain", True][finite], TOL[torch.float32], "beside it")

@@ -3,11 +3,11 @@
 //
 //   S <- g S;   u = beta (v - S^T k);   S <- S + k u^T;   o = S^T q
 //
-// Within a chunk, with G_i = g_0 .. g_i, the state before it S, and rows of U the u_i:
+// Within a chunk, with G_i = g_0 .. g_i, the state before it S, and rows of U the u_i / beta_i (so that V enters as it is):
 //
-//   (I + A) U = diag(beta) V - diag(beta G) K S,     A_ij = beta_i (G_i / G_j) k_i . k_j  (j < i)
-//   O         = diag(G) Q S + P U,                   P_ij = (G_i / G_j) q_i . k_j         (j <= i)
-//   S_new     = G_n S + sum_j (G_n / G_j) k_j u_j^T
+//   (I + A) U = V - diag(G) K S,       A_ij = (G_i / G_j) beta_j k_i . k_j  (j < i)
+//   O         = diag(G) Q S + P U,     P_ij = (G_i / G_j) beta_j q_i . k_j  (j <= i)
+//   S_new     = G_n S + sum_j (G_n / G_j) beta_j k_j u_j^T
 //
 // so that only U = Uv - W S and S_new are left to the chain over a request's chunks.  Three launches:
 //   prepare   a workgroup per (chunk, head): unit rows, the decays, A and P on the matrix cores, the triangular system
@@ -31,14 +31,18 @@
 // where Q V and the k_j v_j^T, which need no state, are formed by the first launch.  The caller answers for 1 / G_63 being
 // a float32 number (a decay no smaller than e^-1).
 //
-// Everything is float32 (v_mfma_f32_16x16x4_f32) but the sums of the decays' logarithms, which are 64-bit so that the
-// ratio of two late rows is as exact as that of two early ones (per channel: the decays' products).
+// Everything is held in float32.  The matrix cores' 32-bit sums (v_mfma_f32_16x16x4_f32, in order) are kept to sixteen or 32
+// terms each, what is added to a number is summed up before it; the keys' inner products and the state's sums are 64-bit
+// (v_mfma_f64_16x16x4_f64), as are the sums of the decays' logarithms, so that the ratio of two late rows is as exact as that
+// of two early ones (per channel: the decays' products), and what rows are multiplied by is rounded once.  So no result and
+// no state is further from the float64 recurrence than row by row: of their norms, 16 requests of 8 heads of 128 x 128, 1.0e-7
+// and 0.6e-7 against 1.2e-7 and 0.7e-7 with the quickest decays, 1.5e-7 and 1.0e-7 against 5.8e-7 and 7.3e-7 with slow ones
+// (32-bit sums one after the other throughout: 2.4e-7 and 1.5e-7).
 //
 // What bounds it: row by row, the chain of dependent sums of a row (0.33 us a row whatever the chip is doing).  In chunks
-// the chain is 64 times shorter and its step two small products (2.7 us a chunk).  Measured with 16 heads of 128 x 128, one
-// request, all three launches against row by row: 41 against 46 us at 128 rows, 47 against 72 at 200, 64 against 171 at
-// 500, 88 against 336 at 1,024, 150 against 667 at 2,048.  Results are 2.4e-7 of their norm from the float64 recurrence
-// (row by row 1.3e-7; with slow decays 4.2e-7 against 6.7e-7): the order of 32-bit sums.  The generalized rule, 32 heads
+// the chain is 64 times shorter and its step two small products (3.6 us a chunk).  Measured with 16 heads of 128 x 128, one
+// request, all three launches against row by row: 51 against 46 us at 128 rows, 59 against 72 at 200, 81 against 172 at
+// 500, 155 against 474 at 1,437, 190 against 672 at 2,048 (with 32-bit sums throughout 151).  The generalized rule, 32 heads
 // of 64 x 64: 34 against 44 us at 160 rows, 37 against 67 at 256, 130 against 493 at 2,048, where the first launch takes
 // 60, the chain 39 and the result 29; 1.2e-7 against 0.8e-7 of the result's norm.
 //
@@ -47,6 +51,7 @@
 #include "common.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef double f64x4 __attribute__((ext_vector_type(4), aligned(16)));
 
 #define DC_ROWS 64
 #define DC_THREADS 256
@@ -55,20 +60,36 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 struct DeltaBlock {
   int dim, vdim, more;  // more: the generalized rule
   __host__ __device__ __forceinline__ int64_t w() const { return 0; }                          // [64][dim]: -W
-  __host__ __device__ __forceinline__ int64_t kt() const { return 64 * dim; }                  // [dim][64]: (G_n / G_j) k_j
+  __host__ __device__ __forceinline__ int64_t kt() const { return 64 * dim; }                  // [dim][64]: k_j, or (G_n / G_j) a_j
   __host__ __device__ __forceinline__ int64_t q() const { return 128 * dim; }                  // [64][dim]: G_i q_i
   __host__ __device__ __forceinline__ int64_t p() const { return 192 * dim; }                  // [64][64]: P, tiles j <= i
   __host__ __device__ __forceinline__ int64_t u() const { return 192 * dim + 4096; }           // [vdim][64]: Uv, then U
   __host__ __device__ __forceinline__ int64_t s() const { return u() + 64 * vdim; }            // [vdim][dim]: S before
   __host__ __device__ __forceinline__ int64_t g() const { return s() + static_cast<int64_t>(dim) * vdim; }  // [dim]: G_n
   __host__ __device__ __forceinline__ int64_t m() const { return g() + dim; }  // [vdim][dim]: sum_j (G_n / G_j) k_j v_j^T
-  __host__ __device__ __forceinline__ int64_t size() const { return m() + (more ? static_cast<int64_t>(dim) * vdim : 0); }
+  __host__ __device__ __forceinline__ int64_t rest() const { return m(); }  // [64] double: (G_n / G_j) beta_j (the gated rule)
+  __host__ __device__ __forceinline__ int64_t size() const { return m() + (more ? static_cast<int64_t>(dim) * vdim : 128); }
 };
 
 __device__ __forceinline__ f32x4 dc_mac(f32x4 a, f32x4 b, f32x4 acc) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], acc, 0, 0, 0);
   return acc;
+}
+
+// The same with 64-bit sums (v_mfma_f64_16x16x4_f64, half the rate).  Its result e of a lane is row 4 e + l / 16: with the
+// first operand's rows handed over in the order of `dc_turn` a lane has the rows 4 (l / 16) + e, as in 32 bits.
+__device__ __forceinline__ int dc_turn(int m) { return 4 * (m & 3) + (m >> 2); }
+__device__ __forceinline__ f64x4 dc_mac64(f32x4 a, f32x4 b, f64x4 acc) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(a[e]), static_cast<double>(b[e]), acc, 0, 0, 0);
+  return acc;
+}
+// e^c, c <= 0, without the rounding of c
+__device__ __forceinline__ float dc_exp(double c) {
+  const float hi = static_cast<float>(c), e = expf(hi);
+  return fmaf(e, static_cast<float>(c - hi), e);
 }
 
 // Numbers that are not finite stay with their row and the later ones, as row by row.  A triangular block of sixteen rows
@@ -113,7 +134,7 @@ __device__ __forceinline__ f32x4 dc_mac_block_second(f32x4 x, f32x4 block, f32x4
   return dc_spoil(dc_mac(clean, block, acc), dc_mac(odd, seen, none));
 }
 
-// A (in LDS, strictly lower) -> the inverses of the blocks on the diagonal of I + A; one wavefront, lane (block, column)
+// A (in LDS, strictly lower) -> the inverses of the blocks on the diagonal of I + A, less I; one wavefront, lane (block, column)
 template <int LA>
 __device__ __forceinline__ void dc_invert_diagonal(const float* a_s, float (*t_s)[16][20], int b, int col) {
   float x[16];
@@ -126,21 +147,32 @@ __device__ __forceinline__ void dc_invert_diagonal(const float* a_s, float (*t_s
     x[i] = s;
   }
 #pragma unroll
-  for (int i = 0; i < 16; ++i) t_s[b][i][col] = x[i];
+  for (int i = 0; i < 16; ++i) t_s[b][i][col] = i == col ? 0.f : x[i];
 }
 
-// x <- (I + A)^-1 x for NT tiles of sixteen columns: [tile][block of sixteen rows], a lane's numbers rows 4 g + e of column m
+// x <- (I + A)^-1 x for NT tiles of sixteen columns: [tile][block of sixteen rows], a lane's numbers rows 4 g + e of column m.
+// What is added to a row is summed up by itself, sixteen terms at a time, and rounds at its own size.
 template <int LA, int NT>
 __device__ __forceinline__ void dc_solve(const float* a_s, const float (*t_s)[16][20], int m, int g, f32x4 (&x)[NT][4]) {
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
+    f32x4 sum[NT];
 #pragma unroll
     for (int a = 0; a < b; ++a) {
       const f32x4 na = -*reinterpret_cast<const f32x4*>(a_s + (16 * b + m) * LA + 16 * a + 4 * g);
+      f32x4 part[NT];
+#pragma unroll
+      for (int u = 0; u < NT; ++u) part[u] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int u = 0; u < NT; ++u) x[u][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(na[e], x[u][a][e], x[u][b], 0, 0, 0);
+        for (int u = 0; u < NT; ++u) part[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(na[e], x[u][a][e], part[u], 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < NT; ++u) sum[u] = a == 0 ? part[u] : sum[u] + part[u];
+    }
+    if (b > 0) {
+#pragma unroll
+      for (int u = 0; u < NT; ++u) x[u][b] += sum[u];
     }
     const f32x4 inv = *reinterpret_cast<const f32x4*>(&t_s[b][m][4 * g]);
     f32x4 y[NT];
@@ -151,7 +183,7 @@ __device__ __forceinline__ void dc_solve(const float* a_s, const float (*t_s)[16
     for (int u = 0; u < NT; ++u) odd = odd || dc_odd(x[u][b]);
     if (__any(odd)) {
 #pragma unroll
-      for (int u = 0; u < NT; ++u) y[u] = dc_mac_block(inv, x[u][b], dc_seen(m, 4 * g, true), y[u]);
+      for (int u = 0; u < NT; ++u) y[u] = dc_mac_block(inv, x[u][b], dc_seen(m, 4 * g, false), y[u]);
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
@@ -159,7 +191,7 @@ __device__ __forceinline__ void dc_solve(const float* a_s, const float (*t_s)[16
         for (int u = 0; u < NT; ++u) y[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(inv[e], x[u][b][e], y[u], 0, 0, 0);
     }
 #pragma unroll
-    for (int u = 0; u < NT; ++u) x[u][b] = y[u];
+    for (int u = 0; u < NT; ++u) x[u][b] += y[u];
   }
 }
 
@@ -177,7 +209,7 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
   float *const q_s = qa_s, *const a_s = qa_s;
   __shared__ __attribute__((aligned(16))) float t_s[4][16][20];  // inverses of the blocks on the diagonal of I + A
   __shared__ double c_s[DC_ROWS];                                // log G_i
-  __shared__ float beta_s[DC_ROWS], g_s[DC_ROWS], rest_s[DC_ROWS];  // beta_i, G_i, G_n / G_i
+  __shared__ double beta_s[DC_ROWS], g_s[DC_ROWS], rest_s[DC_ROWS];  // beta_i, G_i, G_n / G_i (products with them round once)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m = lane & 15, g = lane >> 4;
   const int head = blockIdx.x, chunk = blockIdx.y;
@@ -200,7 +232,8 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
       for (int i = 0; i < QUARTER / 8; ++i) raw[which][i] = *reinterpret_cast<const uint4*>(rows[which] + 8 * i);
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
-      float x[QUARTER], ss = 0.f;
+      float x[QUARTER];
+      double sum = 0.;  // (a row's factor is one error for all its numbers)
 #pragma unroll
       for (int i = 0; i < QUARTER / 8; ++i) {
         const uint32_t u[4] = {raw[which][i].x, raw[which][i].y, raw[which][i].z, raw[which][i].w};
@@ -211,7 +244,8 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
         }
       }
 #pragma unroll
-      for (int i = 0; i < QUARTER; ++i) ss += x[i] * x[i];
+      for (int i = 0; i < QUARTER; ++i) sum += static_cast<double>(x[i]) * static_cast<double>(x[i]);
+      float ss = static_cast<float>(sum);
       ss += ix_dpp<IX_DPP_XOR1>(ss);
       ss += ix_dpp<IX_DPP_XOR2>(ss);
       const float f = row < n ? (which ? 1.0f / sqrtf(static_cast<float>(DIM)) : 1.0f) / sqrtf(ss + 1e-6f) : 0.f;
@@ -237,8 +271,8 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
     }
     const double last = __shfl(c, 63, 64);
     c_s[lane] = c;
-    g_s[lane] = expf(static_cast<float>(c));
-    rest_s[lane] = expf(static_cast<float>(last - c));
+    g_s[lane] = exp(c);
+    rest_s[lane] = exp(last - c);
     beta_s[lane] = live ? 1.0f / (1.0f + expf(-ab[row * 2 * heads + heads + head])) : 0.f;
   }
   __syncthreads();
@@ -246,50 +280,53 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
   // ---- q_i . k_j, then k_i . k_j: the ten tiles on and below the diagonal of each
   auto score = [&](const float* rows, int pair, auto&& put) {
     const int rt = pair < 1 ? 0 : (pair < 3 ? 1 : (pair < 6 ? 2 : 3)), ct = pair - rt * (rt + 1) / 2;
-    const float* ar = rows + (16 * rt + m) * LD + 4 * g;
+    const float* ar = rows + (16 * rt + dc_turn(m)) * LD + 4 * g;
     const float* br = k_s + (16 * ct + m) * LD + 4 * g;
-    f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+    f64x4 s0 = f64x4{0., 0., 0., 0.}, s1 = s0;
 #pragma unroll
     for (int c = 0; c < DIM / 16; c += 2) {
-      s0 = dc_mac(*reinterpret_cast<const f32x4*>(ar + 16 * c), *reinterpret_cast<const f32x4*>(br + 16 * c), s0);
-      s1 = dc_mac(*reinterpret_cast<const f32x4*>(ar + 16 * c + 16), *reinterpret_cast<const f32x4*>(br + 16 * c + 16), s1);
+      s0 = dc_mac64(*reinterpret_cast<const f32x4*>(ar + 16 * c), *reinterpret_cast<const f32x4*>(br + 16 * c), s0);
+      s1 = dc_mac64(*reinterpret_cast<const f32x4*>(ar + 16 * c + 16), *reinterpret_cast<const f32x4*>(br + 16 * c + 16), s1);
     }
     const int j = 16 * ct + m;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int i = 16 * rt + 4 * g + e;
-      const float ratio = expf(static_cast<float>(fmin(c_s[i] - c_s[j], 0.0)));  // (above the diagonal: not used)
+      const float ratio = dc_exp(fmin(c_s[i] - c_s[j], 0.0));  // (above the diagonal: not used)
       put(i, j, ratio * (s0[e] + s1[e]));
     }
   };
 #pragma unroll 1
   for (int pair = wave; pair < 10; pair += 4)
-    score(q_s, pair, [&](int i, int j, float x) { mine[blk.p() + i * 64 + j] = j <= i ? x : 0.f; });
+    score(q_s, pair, [&](int i, int j, double x) { mine[blk.p() + i * 64 + j] = j <= i ? static_cast<float>(beta_s[j] * x) : 0.f; });
   // ---- what the chain and the result take as they are
   for (int id = tid; id < DIM * 16; id += DC_THREADS) {
     const int row = id / (DIM / 4), d = 4 * (id % (DIM / 4));
-    const f32x4 x = *reinterpret_cast<const f32x4*>(q_s + row * LD + d);
-    *reinterpret_cast<f32x4*>(mine + blk.q() + row * DIM + d) = x * g_s[row];
+    f32x4 x = *reinterpret_cast<const f32x4*>(q_s + row * LD + d);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = static_cast<float>(x[e] * g_s[row]);
+    *reinterpret_cast<f32x4*>(mine + blk.q() + row * DIM + d) = x;
   }
   __syncthreads();
 #pragma unroll 1
   for (int pair = 3 - wave; pair < 10; pair += 4)  // (the wavefronts that had three tiles above have two)
-    score(k_s, pair, [&](int i, int j, float x) { a_s[i * LA + j] = j < i ? beta_s[i] * x : 0.f; });
+    score(k_s, pair, [&](int i, int j, double x) { a_s[i * LA + j] = j < i ? static_cast<float>(beta_s[j] * x) : 0.f; });
   for (int id = tid; id < DIM * 16; id += DC_THREADS) {
     const int d = id >> 4, jq = 4 * (id & 15);
     f32x4 x;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] = k_s[(jq + e) * LD + d] * rest_s[jq + e];
+    for (int e = 0; e < 4; ++e) x[e] = k_s[(jq + e) * LD + d];
     *reinterpret_cast<f32x4*>(mine + blk.kt() + d * 64 + jq) = x;
   }
-  for (int d = tid; d < DIM; d += DC_THREADS) mine[blk.g() + d] = g_s[DC_ROWS - 1];
+  if (tid < DC_ROWS) reinterpret_cast<double*>(mine + blk.rest())[tid] = rest_s[tid] * beta_s[tid];
+  for (int d = tid; d < DIM; d += DC_THREADS) mine[blk.g() + d] = static_cast<float>(g_s[DC_ROWS - 1]);
   __syncthreads();
 
   // ---- the diagonal blocks' inverses: lane (block, column), sixteen steps of substitution
   if (wave == 0) dc_invert_diagonal<LA>(a_s, t_s, g, m);
   __syncthreads();
 
-  // ---- (I + A) [W | Uv] = [diag(beta G) K | diag(beta) V], four tiles of sixteen columns at a time and wavefront
+  // ---- (I + A) [W | Uv] = [diag(G) K | V], four tiles of sixteen columns at a time and wavefront
   const int tiles = (DIM + vdim) / 16;
 #pragma unroll 1
   for (int t0 = 4 * wave; t0 < tiles; t0 += 16) {
@@ -302,8 +339,8 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int row = 16 * b + 4 * g + e;
-          if (16 * t < DIM) x[u][b][e] = beta_s[row] * g_s[row] * k_s[row * LD + 16 * t + m];
-          else x[u][b][e] = beta_s[row] * ix_load(v + (row0 + min(row, n - 1)) * v_stride + head * vdim + 16 * t - DIM + m);
+          if (16 * t < DIM) x[u][b][e] = static_cast<float>(g_s[row] * k_s[row * LD + 16 * t + m]);
+          else x[u][b][e] = ix_load(v + (row0 + min(row, n - 1)) * v_stride + head * vdim + 16 * t - DIM + m);
         }
     }
     dc_solve<LA, 4>(a_s, t_s, m, g, x);
@@ -543,17 +580,20 @@ general_chunks_prepare_kernel(const bf16_t* r, const bf16_t* k, const bf16_t* v,
   }
 }
 
-// request blockIdx.z's chunks [first, first + count) one after the other, value columns 16 blockIdx.y ..
+// request blockIdx.z's chunks [first, first + count) one after the other, value columns 16 blockIdx.y ..  The state's sums are
+// 64-bit: row by row the state is left with fewer roundings than 32-bit sums over a chunk have, 0.8e-7 of its norm after
+// quick decays against 0.9e-7 (the generalized rule's, whose terms cancel, 0.5e-7 against 1.8e-7); they cost a chunk's step
+// 3.6 instead of 2.8 us.
 template <int DIM, bool MORE>
 __global__ void __launch_bounds__(DC_THREADS)
 delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, const int32_t* __restrict__ seq_first,
                           const int32_t* __restrict__ seq_count, const int32_t* __restrict__ state_slots,
                           float* __restrict__ state, int64_t state_stride, int heads, int vdim) {
-  constexpr int LD = DIM + 4, LU = DC_ROWS + 4;
+  constexpr int LD = DIM + 4, LU = DC_ROWS + 2;
   constexpr int TILES = DIM / 16;                  // tiles of sixteen rows of the state
   constexpr int TS = TILES >= 4 ? TILES / 4 : 1;   // ... per wavefront (with two tiles in all two wavefronts have none)
   __shared__ __attribute__((aligned(16))) float s_s[16 * LD];
-  __shared__ __attribute__((aligned(16))) float u_s[16 * LU];
+  __shared__ __attribute__((aligned(16))) double u_s[16 * LU];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
   // (heads first: workgroups go to the chip's eight dies in turn, so a head's column blocks, which read the same W and
@@ -575,20 +615,21 @@ delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, cons
     row[t] = owns ? 16 * (wave * TS + t) + 4 * g : 0;
     st[t] = *reinterpret_cast<const f32x4*>(sp + row[t]);
   }
-  struct Operands { f32x4 w[TILES], kt[TS][4], u, gn[TS], add[MORE ? TS : 1]; };
+  struct Operands { f32x4 w[TILES], kt[TS][4], u, gn[TS], add[MORE ? TS : 1]; f64x4 rest; };
   auto ask = [&](const float* p, Operands& o) {
 #pragma unroll
     for (int c = 0; c < TILES; ++c)
       o.w[c] = *reinterpret_cast<const f32x4*>(p + blk.w() + (16 * wave + m) * DIM + 16 * c + 4 * g);
 #pragma unroll
     for (int t = 0; t < TS; ++t) {
-      const int d = (owns ? 16 * (wave * TS + t) : 0) + m;
+      const int d = (owns ? 16 * (wave * TS + t) : 0) + dc_turn(m);
 #pragma unroll
       for (int s = 0; s < 4; ++s) o.kt[t][s] = *reinterpret_cast<const f32x4*>(p + blk.kt() + d * 64 + 16 * s + 4 * g);
       o.gn[t] = *reinterpret_cast<const f32x4*>(p + blk.g() + row[t]);
       if constexpr (MORE) o.add[t] = *reinterpret_cast<const f32x4*>(p + blk.m() + static_cast<int64_t>(col) * DIM + row[t]);
     }
     o.u = *reinterpret_cast<const f32x4*>(p + blk.u() + col * 64 + 16 * wave + 4 * g);
+    if constexpr (!MORE) o.rest = *reinterpret_cast<const f64x4*>(reinterpret_cast<const double*>(p + blk.rest()) + 16 * wave + 4 * g);
     __builtin_amdgcn_sched_barrier(0);
   };
   auto work_chunk = [&](float* p, const Operands& o) {
@@ -602,37 +643,59 @@ delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, cons
     __syncthreads();
     // (all of a product's operands are asked for before the first is used: left to itself the compiler takes them two by
     // two and waits for each pair)
-    f32x4 b[TILES > 4 ? TILES : 4];
+    f32x4 b[TILES];
 #pragma unroll
     for (int c = 0; c < TILES; ++c) b[c] = *reinterpret_cast<const f32x4*>(s_s + m * LD + 16 * c + 4 * g);
     __builtin_amdgcn_sched_barrier(0);
-    f32x4 ua = o.u, ub = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int PARTS = TILES < 4 ? TILES : 4;
+    f32x4 part[PARTS];
 #pragma unroll
-    for (int c = 0; c < TILES; c += 2) {
+    for (int i = 0; i < PARTS; ++i) part[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < TILES; c += PARTS)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < PARTS; ++i)
+          part[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.w[c + i][e], b[c + i][e], part[i], 0, 0, 0);
+    f32x4 ws = part[0] + part[1], u;
+    if constexpr (PARTS == 4) ws += part[2] + part[3];
+    f64x4 us;  // (the state takes U, and what its rows are multiplied by, unrounded)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      us[e] = static_cast<double>(ws[e]) + static_cast<double>(o.u[e]);
+      u[e] = static_cast<float>(us[e]);
+      if constexpr (!MORE) us[e] *= o.rest[e];
+    }
+    *reinterpret_cast<f64x4*>(u_s + m * LU + 16 * wave + 4 * g) = us;
+    *reinterpret_cast<f32x4*>(p + blk.u() + col * 64 + 16 * wave + 4 * g) = u;
+    f64x4 sum[2];  // two tiles' sums, or the halves of one's
+#pragma unroll
+    for (int t = 0; t < TS; ++t)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        ua = __builtin_amdgcn_mfma_f32_16x16x4f32(o.w[c][e], b[c][e], ua, 0, 0, 0);
-        ub = __builtin_amdgcn_mfma_f32_16x16x4f32(o.w[c + 1][e], b[c + 1][e], ub, 0, 0, 0);
+        sum[t][e] = static_cast<double>(st[t][e]) * static_cast<double>(o.gn[t][e]);
+        if constexpr (MORE) sum[t][e] += static_cast<double>(o.add[t][e]);
       }
-    }
-    ua += ub;
-    *reinterpret_cast<f32x4*>(u_s + m * LU + 16 * wave + 4 * g) = ua;
-    *reinterpret_cast<f32x4*>(p + blk.u() + col * 64 + 16 * wave + 4 * g) = ua;
-#pragma unroll
-    for (int t = 0; t < TS; ++t) {
-      st[t] *= o.gn[t];
-      if constexpr (MORE) st[t] += o.add[t];
-    }
+    if constexpr (TS == 1) sum[1] = f64x4{0., 0., 0., 0.};
     __syncthreads();
+    f64x4 bu[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) b[s] = *reinterpret_cast<const f32x4*>(u_s + m * LU + 16 * s + 4 * g);
+    for (int s = 0; s < 4; ++s) bu[s] = *reinterpret_cast<const f64x4*>(u_s + m * LU + 16 * s + 4 * g);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int t = 0; t < TS; ++t) st[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.kt[t][s][e], b[s][e], st[t], 0, 0, 0);
+        for (int t = 0; t < TS; ++t) {
+          f64x4& to = sum[TS == 1 ? s & 1 : t];
+          to = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(o.kt[t][s][e]), bu[s][e], to, 0, 0, 0);
+        }
+#pragma unroll
+    for (int t = 0; t < TS; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) st[t][e] = static_cast<float>(TS == 1 ? sum[0][e] + sum[1][e] : sum[t][e]);
   };
   Operands one, two;  // the next chunk's operands on their way while this one is worked
   ask(at0, one);
@@ -679,6 +742,7 @@ delta_chunks_result_kernel(const float* __restrict__ work, const int32_t* __rest
   }
   __syncthreads();
   const int tiles = vdim / 16;
+  const f32x4 none = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int t0 = 2 * wave; t0 < tiles; t0 += 8) {
     f32x4 acc[2][4];  // [tile of columns][tile of rows]
 #pragma unroll
@@ -688,33 +752,49 @@ delta_chunks_result_kernel(const float* __restrict__ work, const int32_t* __rest
     const int t1 = min(t0 + 1, tiles - 1);
     const float* s0 = mine + blk.s() + static_cast<int64_t>(16 * t0 + m) * DIM + 4 * g;
     const float* s1 = mine + blk.s() + static_cast<int64_t>(16 * t1 + m) * DIM + 4 * g;
+    // (S is asked for at once, U half-way; a sixteen of the reduction is worked before the next one is read from LDS, or the
+    // registers do not hold what the compiler asks for ahead)
+    f32x4 sa[2][DIM / 16], ua[2][4];
 #pragma unroll
     for (int c = 0; c < DIM / 16; ++c) {
-      const f32x4 a0 = *reinterpret_cast<const f32x4*>(s0 + 16 * c), a1 = *reinterpret_cast<const f32x4*>(s1 + 16 * c);
+      sa[0][c] = *reinterpret_cast<const f32x4*>(s0 + 16 * c);
+      sa[1][c] = *reinterpret_cast<const f32x4*>(s1 + 16 * c);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < DIM / 16; ++c) {
+      if (c == DIM / 32) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          ua[0][s] = *reinterpret_cast<const f32x4*>(mine + blk.u() + (16 * t0 + m) * 64 + 16 * s + 4 * g);
+          ua[1][s] = *reinterpret_cast<const f32x4*>(mine + blk.u() + (16 * t1 + m) * 64 + 16 * s + 4 * g);
+        }
+      }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const f32x4 b = *reinterpret_cast<const f32x4*>(q_s + (16 * r + m) * LD + 16 * c + 4 * g);
-        acc[0][r] = dc_mac(a0, b, acc[0][r]);
-        acc[1][r] = dc_mac(a1, b, acc[1][r]);
+        acc[0][r] += dc_mac(sa[0][c], b, none);
+        acc[1][r] += dc_mac(sa[1][c], b, none);
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      const f32x4 a0 = *reinterpret_cast<const f32x4*>(mine + blk.u() + (16 * t0 + m) * 64 + 16 * s + 4 * g);
-      const f32x4 a1 = *reinterpret_cast<const f32x4*>(mine + blk.u() + (16 * t1 + m) * 64 + 16 * s + 4 * g);
+      const f32x4 a0 = ua[0][s], a1 = ua[1][s];
       const bool odd = __any(dc_odd(a0) || dc_odd(a1));
 #pragma unroll
       for (int r = s; r < 4; ++r) {
         const f32x4 b = *reinterpret_cast<const f32x4*>(p_s + (16 * r + m) * LP + 16 * s + 4 * g);
         if (r == s && odd) {
           const f32x4 seen = dc_seen(m, 4 * g, true);
-          acc[0][r] = dc_mac_block_second(a0, b, seen, acc[0][r]);
-          acc[1][r] = dc_mac_block_second(a1, b, seen, acc[1][r]);
+          acc[0][r] += dc_mac_block_second(a0, b, seen, none);
+          acc[1][r] += dc_mac_block_second(a1, b, seen, none);
         } else {
-          acc[0][r] = dc_mac(a0, b, acc[0][r]);
-          acc[1][r] = dc_mac(a1, b, acc[1][r]);
+          acc[0][r] += dc_mac(a0, b, none);
+          acc[1][r] += dc_mac(a1, b, none);
         }
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {

@@ -28,10 +28,10 @@ from .dense_mlp import stack_rows
 from .linear_state import CHUNK_WORKSPACE, chunk_slices, longest_portion, shorter_portions
 from .short_conv import ShortConv
 
-# A step goes through the chunked form if some request brings at least CHUNKED_FROM_ROWS rows (16 heads of 128 x 128: 41
-# against 46 us row by row at 128 rows, 40 against 35 at 96); with it go all that bring CHUNKED_MIN_ROWS or more, the
+# A step goes through the chunked form if some request brings at least CHUNKED_FROM_ROWS rows (16 heads of 128 x 128: 51
+# against 46 us row by row at 128 rows, 59 against 72 at 200); with it go all that bring CHUNKED_MIN_ROWS or more, the
 # others row by row.
-CHUNKED_FROM_ROWS = 112
+CHUNKED_FROM_ROWS = 160
 CHUNKED_MIN_ROWS = 16
 
 

@@ -739,3 +739,48 @@ def test_delta_rule_in_chunks_keeps_what_is_not_finite_to_later_rows(row, bad):
             reached[row:, 1, 5], reached_state[1, 5] = True, True
         for got, full, on in ((out, want, reached), (state, left, reached_state)):
             assert not torch.isfinite(got[on]).any() and torch.equal(got[~on], full[~on]), f"operand {where}"
+
+
+@pytest.mark.parametrize("heads,dim,vdim", [(8, 32, 48), (8, 64, 64), (8, 128, 128)])
+@pytest.mark.parametrize("decay", [3.0, 2.0, 0.0, -2.0, -5.0, -9.0])
+def test_delta_rule_in_chunks_is_no_less_exact_than_row_by_row(heads, dim, vdim, decay):
+    """The distance of the chunked form's results and last states from the float64 recurrence, over sixteen requests, is at
+    most that of the form that walks row by row, from decays that forget within a row to some that keep thousands."""
+    from inferx_amd import ops
+    f64_ = lambda x: x.to(torch.float64)
+    lengths = [65 + 13 * s for s in range(16)]
+    S, T, starts = len(lengths), sum(lengths), [0]
+    for n in lengths:
+        starts.append(starts[-1] + n)
+    q, k, v = (rnd((T, heads * n), s, 1.0, torch.bfloat16).to(DEV) for s, n in ((1, dim), (2, dim), (3, vdim)))
+    ab, a_log, dt_bias = rnd((T, 2 * heads), 4, 1.5).to(DEV), rnd((heads,), 5, 0.7).to(DEV), rnd((heads,), 6, 0.7).to(DEV)
+    ab[:, :heads] += decay
+    before = rnd((S, heads * dim * vdim), 7, 0.3).to(DEV)
+    g = torch.exp(-torch.exp(f64_(a_log)) * torch.nn.functional.softplus(f64_(ab[:, :heads]) + f64_(dt_bias)))
+    beta = torch.sigmoid(f64_(ab[:, heads:]))
+    unit = lambda x: x * torch.rsqrt((x * x).sum(-1, keepdim=True) + 1e-6)
+    qn, kn = (unit(f64_(x).view(T, heads, 1, dim)) for x in (q, k))
+    vd, M = f64_(v).view(T, heads, vdim), f64_(before).view(S, heads, vdim, dim).clone()
+    want = torch.empty((T, heads, vdim), dtype=torch.float64, device=DEV)
+    for t in range(max(lengths)):  # every request's row t
+        on = torch.tensor([s for s, n in enumerate(lengths) if t < n], device=DEV)
+        at = torch.tensor(starts[:-1], device=DEV)[on] + t
+        now = M[on] * g[at][:, :, None, None]
+        u = beta[at][:, :, None] * (vd[at] - (now * kn[at]).sum(-1))
+        now = now + u[..., None] * kn[at]
+        want[at] = (now * qn[at]).sum(-1) * dim ** -0.5
+        M[on] = now
+    row0 = [(s, starts[s] + at, min(64, n - at)) for s, n in enumerate(lengths) for at in range(0, n, 64)]
+    count = [-(-n // 64) for n in lengths]
+    off, slots = [], i32(list(range(S)))
+    for chunked in (False, True):
+        state, out = before.clone(), torch.empty((T, heads, vdim), device=DEV)
+        if chunked:
+            ops.delta_chunks(q, k, v, ab, a_log, dt_bias, state, slots, i32([[x[1] for x in row0], [x[2] for x in row0]]),
+                             i32([list(range(S)), [sum(count[:s]) for s in range(S)], count]), out, heads, heads, dim, vdim)
+        else:
+            rows = ops.StepRows(i32([s for s, n in enumerate(lengths) for _ in range(n)]), i32(starts), slots)
+            ops.delta_rule(q, k, v, ab, a_log, dt_bias, state, rows, out, heads, heads, dim, vdim)
+        off.append([float((f64_(a).view(b.shape) - b).norm() / b.norm()) for a, b in ((out, want), (state, M))])
+    print(f"decay {decay}, {dim} x {vdim}: rows {off[0][0]:.3e} {off[0][1]:.3e}, chunks {off[1][0]:.3e} {off[1][1]:.3e}")
+    assert off[1][0] <= off[0][0] and off[1][1] <= off[0][1], off

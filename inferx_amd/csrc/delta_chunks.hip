@@ -34,17 +34,18 @@
 // Everything is held in float32.  The matrix cores' 32-bit sums (v_mfma_f32_16x16x4_f32, in order) are kept to sixteen or 32
 // terms each, what is added to a number is summed up before it; the keys' inner products and the state's sums are 64-bit
 // (v_mfma_f64_16x16x4_f64), as are the sums of the decays' logarithms, so that the ratio of two late rows is as exact as that
-// of two early ones (per channel: the decays' products), and what rows are multiplied by is rounded once.  So no result and
-// no state is further from the float64 recurrence than row by row: of their norms, 16 requests of 8 heads of 128 x 128, 1.0e-7
+// of two early ones (per channel: the decays' products), and what rows are multiplied by is rounded once.  So results and
+// states are no further from the float64 recurrence than row by row: of their norms, 16 requests of 8 heads of 128 x 128, 1.0e-7
 // and 0.6e-7 against 1.2e-7 and 0.7e-7 with the quickest decays, 1.5e-7 and 1.0e-7 against 5.8e-7 and 7.3e-7 with slow ones
-// (32-bit sums one after the other throughout: 2.4e-7 and 1.5e-7).
+// (32-bit sums one after the other throughout: 2.4e-7 and 1.5e-7).  The generalized rule, decays e^(-0.61 sigmoid(normal)):
+// 0.59e-7 and 0.37e-7 against 0.87e-7 and 0.46e-7 (1.4e-7 and 1.5e-7), slow ones 1.1e-7 and 0.7e-7 against 2.2e-7 and 2.3e-7;
+// only where every channel of every row forgets as fast as it can (e^-0.61) the state is 0.36e-7 off against 0.34e-7.
 //
 // What bounds it: row by row, the chain of dependent sums of a row (0.33 us a row whatever the chip is doing).  In chunks
 // the chain is 64 times shorter and its step two small products (3.6 us a chunk).  Measured with 16 heads of 128 x 128, one
 // request, all three launches against row by row: 51 against 46 us at 128 rows, 59 against 72 at 200, 81 against 172 at
 // 500, 155 against 474 at 1,437, 190 against 672 at 2,048 (with 32-bit sums throughout 151).  The generalized rule, 32 heads
-// of 64 x 64: 34 against 44 us at 160 rows, 37 against 67 at 256, 130 against 493 at 2,048, where the first launch takes
-// 60, the chain 39 and the result 29; 1.2e-7 against 0.8e-7 of the result's norm.
+// of 64 x 64: 42 against 43 us at 160 rows, 46 against 66 at 256, 169 against 492 at 2,048 (with 32-bit sums 130).
 //
 // A lane's operand of a 16 x 16 x 4 product is one number of row (column) l % 16 at reduction index l / 16.  Operands
 // are read four numbers at a time, index 16 s + 4 (l / 16) + e, and the e-th of them meet in one instruction.
@@ -66,9 +67,9 @@ struct DeltaBlock {
   __host__ __device__ __forceinline__ int64_t u() const { return 192 * dim + 4096; }           // [vdim][64]: Uv, then U
   __host__ __device__ __forceinline__ int64_t s() const { return u() + 64 * vdim; }            // [vdim][dim]: S before
   __host__ __device__ __forceinline__ int64_t g() const { return s() + static_cast<int64_t>(dim) * vdim; }  // [dim]: G_n
-  __host__ __device__ __forceinline__ int64_t m() const { return g() + dim; }  // [vdim][dim]: sum_j (G_n / G_j) k_j v_j^T
+  __host__ __device__ __forceinline__ int64_t m() const { return g() + dim; }  // [vdim][dim] double: sum_j (G_n / G_j) k_j v_j^T
   __host__ __device__ __forceinline__ int64_t rest() const { return m(); }  // [64] double: (G_n / G_j) beta_j (the gated rule)
-  __host__ __device__ __forceinline__ int64_t size() const { return m() + (more ? static_cast<int64_t>(dim) * vdim : 128); }
+  __host__ __device__ __forceinline__ int64_t size() const { return m() + (more ? 2 * static_cast<int64_t>(dim) * vdim : 128); }
 };
 
 __device__ __forceinline__ f32x4 dc_mac(f32x4 a, f32x4 b, f32x4 acc) {
@@ -126,6 +127,19 @@ __device__ __forceinline__ f32x4 dc_mac_block(f32x4 block, f32x4 x, f32x4 seen, 
   f32x4 clean, odd;
   dc_part(x, clean, odd);
   return dc_spoil(dc_mac(block, clean, acc), dc_mac(seen, odd, none));
+}
+__device__ __forceinline__ f64x4 dc_mac64_block(f32x4 block, f32x4 x, f32x4 seen, f64x4 acc) {  // (the block's rows in the order of `dc_turn`)
+  const f32x4 none = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 clean, odd;
+  dc_part(x, clean, odd);
+  acc = dc_mac64(block, clean, acc);
+  const f32x4 count = dc_mac(seen, odd, none);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc[e] = count[e] > 0.f ? __builtin_nan("") : acc[e];
+  return acc;
+}
+__device__ __forceinline__ f32x4 dc_narrow(const f64x4 x) {
+  return f32x4{static_cast<float>(x[0]), static_cast<float>(x[1]), static_cast<float>(x[2]), static_cast<float>(x[3])};
 }
 __device__ __forceinline__ f32x4 dc_mac_block_second(f32x4 x, f32x4 block, f32x4 seen, f32x4 acc) {
   const f32x4 none = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -374,7 +388,7 @@ general_chunks_prepare_kernel(const bf16_t* r, const bf16_t* k, const bf16_t* v,
   __shared__ __attribute__((aligned(16))) float x_s[4][DC_ROWS * LD];  // b G, a / G (then A), k / G (then C), r G (then Q)
   __shared__ __attribute__((aligned(16))) float t_s[4][16][20];
   __shared__ double seg_s[DC_THREADS / DIM][DIM];
-  __shared__ float gn_s[DIM];
+  __shared__ double gn_s[DIM];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int m = lane & 15, g = lane >> 4;
   const int head = blockIdx.x, chunk = blockIdx.y;
@@ -415,8 +429,14 @@ general_chunks_prepare_kernel(const bf16_t* r, const bf16_t* k, const bf16_t* v,
     }
     seg_s[seg][d] = p;
     __syncthreads();
+    double all = 1.0;  // G_n
     p = 1.0;
-    for (int s = 0; s < seg; ++s) p *= seg_s[s][d];
+#pragma unroll
+    for (int s = 0; s < DC_THREADS / DIM; ++s) {
+      p *= s < seg ? seg_s[s][d] : 1.0;
+      all *= seg_s[s][d];
+    }
+    f32x4 kt;
 #pragma unroll
     for (int i0 = 0; i0 < SEG; i0 += PART) {
       if (i0 > 0) ask(i0);
@@ -432,11 +452,13 @@ general_chunks_prepare_kernel(const bf16_t* r, const bf16_t* k, const bf16_t* v,
         const float rg = live ? static_cast<float>(rv[i] * p) : 0.f;
         r_s[row * LD + d] = rg;
         mine[blk.q() + row * DIM + d] = rg;
-        if (row == DC_ROWS - 1) {
-          gn_s[d] = static_cast<float>(p);
-          mine[blk.g() + d] = static_cast<float>(p);
-        }
+        kt[i & 3] = live ? static_cast<float>(av[i] * (all * over)) : 0.f;
+        if ((i & 3) == 3) *reinterpret_cast<f32x4*>(mine + blk.kt() + d * 64 + row - 3) = kt;
       }
+    }
+    if (seg == 0) {
+      gn_s[d] = all;
+      mine[blk.g() + d] = static_cast<float>(all);
     }
   }
   __syncthreads();
@@ -446,15 +468,15 @@ general_chunks_prepare_kernel(const bf16_t* r, const bf16_t* k, const bf16_t* v,
   auto score = [&](const float* left, const float* right, int pair, int& rt, int& ct) {
     rt = pair < 1 ? 0 : (pair < 3 ? 1 : (pair < 6 ? 2 : 3));
     ct = pair - rt * (rt + 1) / 2;
-    const float* ar = left + (16 * rt + m) * LD + 4 * g;
+    const float* ar = left + (16 * rt + dc_turn(m)) * LD + 4 * g;
     const float* br = right + (16 * ct + m) * LD + 4 * g;
-    f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+    f64x4 s0 = f64x4{0., 0., 0., 0.}, s1 = s0;
 #pragma unroll
     for (int c = 0; c < DIM / 16; c += 2) {
-      s0 = dc_mac(*reinterpret_cast<const f32x4*>(ar + 16 * c), *reinterpret_cast<const f32x4*>(br + 16 * c), s0);
-      s1 = dc_mac(*reinterpret_cast<const f32x4*>(ar + 16 * c + 16), *reinterpret_cast<const f32x4*>(br + 16 * c + 16), s1);
+      s0 = dc_mac64(*reinterpret_cast<const f32x4*>(ar + 16 * c), *reinterpret_cast<const f32x4*>(br + 16 * c), s0);
+      s1 = dc_mac64(*reinterpret_cast<const f32x4*>(ar + 16 * c + 16), *reinterpret_cast<const f32x4*>(br + 16 * c + 16), s1);
     }
-    return s0 + s1;
+    return dc_narrow(s0 + s1);
   };
   f32x4 qv[3], av[3], cv[3];
 #pragma unroll
@@ -469,20 +491,15 @@ general_chunks_prepare_kernel(const bf16_t* r, const bf16_t* k, const bf16_t* v,
         mine[blk.p() + i * 64 + j] = j <= i ? s[e] : 0.f;
       }
       av[u] = score(b_s, a_s, pair, rt, ct);
+      __builtin_amdgcn_sched_barrier(0);
     }
     if (back < 10) {
       qv[u] = score(r_s, k_s, back, rt, ct);
       cv[u] = score(b_s, k_s, back, rt, ct);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
-  // ---- (G_n / G_j) a_j for the chain, and what k and v alone add to the state, a wavefront per tile of value columns
-  for (int id = tid; id < DIM * 16; id += DC_THREADS) {
-    const int d = id >> 4, jq = 4 * (id & 15);
-    f32x4 x;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] = a_s[(jq + e) * LD + d] * gn_s[d];
-    *reinterpret_cast<f32x4*>(mine + blk.kt() + d * 64 + jq) = x;
-  }
+  // ---- what k and v alone add to the state, a wavefront per tile of value columns
   const int vtiles = vdim / 16;
   auto load_v = [&](int t, f32x4 (&x)[4]) {
 #pragma unroll
@@ -499,16 +516,15 @@ general_chunks_prepare_kernel(const bf16_t* r, const bf16_t* k, const bf16_t* v,
     load_v(t, x);
 #pragma unroll 1
     for (int dt = 0; dt < DIM / 16; ++dt) {
-      f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
-      const float gn = gn_s[16 * dt + m];
+      f64x4 s = f64x4{0., 0., 0., 0.};
+      const int d = 16 * dt + dc_turn(m);
+      const double gn = gn_s[d];
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        f32x4 kk;
+      for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) kk[e] = k_s[(16 * b + 4 * g + e) * LD + 16 * dt + m] * gn;
-        s = dc_mac(kk, x[b], s);
-      }
-      *reinterpret_cast<f32x4*>(mine + blk.m() + static_cast<int64_t>(16 * t + m) * DIM + 16 * dt + 4 * g) = s;
+        for (int e = 0; e < 4; ++e)
+          s = __builtin_amdgcn_mfma_f64_16x16x4f64(k_s[(16 * b + 4 * g + e) * LD + d] * gn, static_cast<double>(x[b][e]), s, 0, 0, 0);
+      *reinterpret_cast<f64x4*>(reinterpret_cast<double*>(mine + blk.m()) + static_cast<int64_t>(16 * t + m) * DIM + 16 * dt + 4 * g) = s;
     }
   }
   __syncthreads();
@@ -554,25 +570,26 @@ general_chunks_prepare_kernel(const bf16_t* r, const bf16_t* k, const bf16_t* v,
     load_v(t, x);
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-      f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f}, c = o;
+      f64x4 o = f64x4{0., 0., 0., 0.}, c = o;
 #pragma unroll
       for (int a = 0; a <= b; ++a) {
-        const f32x4 ra = *reinterpret_cast<const f32x4*>(r_s + (16 * b + m) * LD + 16 * a + 4 * g);
-        const f32x4 ka = *reinterpret_cast<const f32x4*>(k_s + (16 * b + m) * LD + 16 * a + 4 * g);
+        const f32x4 ra = *reinterpret_cast<const f32x4*>(r_s + (16 * b + dc_turn(m)) * LD + 16 * a + 4 * g);
+        const f32x4 ka = *reinterpret_cast<const f32x4*>(k_s + (16 * b + dc_turn(m)) * LD + 16 * a + 4 * g);
         if (a == b && __any(dc_odd(x[a]))) {
-          o = dc_mac_block(ra, x[a], dc_seen(m, 4 * g, true), o);
-          c = dc_mac_block(ka, x[a], dc_seen(m, 4 * g, false), c);
+          o = dc_mac64_block(ra, x[a], dc_seen(m, 4 * g, true), o);
+          c = dc_mac64_block(ka, x[a], dc_seen(m, 4 * g, false), c);
         } else {
-          o = dc_mac(ra, x[a], o);
-          c = dc_mac(ka, x[a], c);
+          o = dc_mac64(ra, x[a], o);
+          c = dc_mac64(ka, x[a], c);
         }
       }
-      z[0][b] = -c;
+      z[0][b] = -dc_narrow(c);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int row = 16 * b + 4 * g + e;
-        if (row < n) out[((row0 + row) * heads + head) * vdim + 16 * t + m] = o[e];
+        if (row < n) out[((row0 + row) * heads + head) * vdim + 16 * t + m] = static_cast<float>(o[e]);
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
     dc_solve<LD, 1>(a_s, t_s, m, g, z);
 #pragma unroll
@@ -615,7 +632,7 @@ delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, cons
     row[t] = owns ? 16 * (wave * TS + t) + 4 * g : 0;
     st[t] = *reinterpret_cast<const f32x4*>(sp + row[t]);
   }
-  struct Operands { f32x4 w[TILES], kt[TS][4], u, gn[TS], add[MORE ? TS : 1]; f64x4 rest; };
+  struct Operands { f32x4 w[TILES], kt[TS][4], u, gn[TS]; f64x4 more[MORE ? TS : 1]; };  // more: M, or (G_n / G_j) beta_j
   auto ask = [&](const float* p, Operands& o) {
 #pragma unroll
     for (int c = 0; c < TILES; ++c)
@@ -626,10 +643,10 @@ delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, cons
 #pragma unroll
       for (int s = 0; s < 4; ++s) o.kt[t][s] = *reinterpret_cast<const f32x4*>(p + blk.kt() + d * 64 + 16 * s + 4 * g);
       o.gn[t] = *reinterpret_cast<const f32x4*>(p + blk.g() + row[t]);
-      if constexpr (MORE) o.add[t] = *reinterpret_cast<const f32x4*>(p + blk.m() + static_cast<int64_t>(col) * DIM + row[t]);
+      if constexpr (MORE) o.more[t] = *reinterpret_cast<const f64x4*>(reinterpret_cast<const double*>(p + blk.m()) + static_cast<int64_t>(col) * DIM + row[t]);
     }
     o.u = *reinterpret_cast<const f32x4*>(p + blk.u() + col * 64 + 16 * wave + 4 * g);
-    if constexpr (!MORE) o.rest = *reinterpret_cast<const f64x4*>(reinterpret_cast<const double*>(p + blk.rest()) + 16 * wave + 4 * g);
+    if constexpr (!MORE) o.more[0] = *reinterpret_cast<const f64x4*>(reinterpret_cast<const double*>(p + blk.rest()) + 16 * wave + 4 * g);
     __builtin_amdgcn_sched_barrier(0);
   };
   auto work_chunk = [&](float* p, const Operands& o) {
@@ -665,7 +682,7 @@ delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, cons
     for (int e = 0; e < 4; ++e) {
       us[e] = static_cast<double>(ws[e]) + static_cast<double>(o.u[e]);
       u[e] = static_cast<float>(us[e]);
-      if constexpr (!MORE) us[e] *= o.rest[e];
+      if constexpr (!MORE) us[e] *= o.more[0][e];
     }
     *reinterpret_cast<f64x4*>(u_s + m * LU + 16 * wave + 4 * g) = us;
     *reinterpret_cast<f32x4*>(p + blk.u() + col * 64 + 16 * wave + 4 * g) = u;
@@ -675,7 +692,7 @@ delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, cons
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         sum[t][e] = static_cast<double>(st[t][e]) * static_cast<double>(o.gn[t][e]);
-        if constexpr (MORE) sum[t][e] += static_cast<double>(o.add[t][e]);
+        if constexpr (MORE) sum[t][e] += o.more[t][e];
       }
     if constexpr (TS == 1) sum[1] = f64x4{0., 0., 0., 0.};
     __syncthreads();

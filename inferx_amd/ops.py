@@ -1320,7 +1320,7 @@ def general_delta_fits(r: torch.Tensor, state: torch.Tensor, dim: int, vdim: int
 
 def general_delta_floats(dim: int, vdim: int) -> int:
     """Floats of workspace that `general_delta_chunks` takes per chunk and head (the entry point checks it)."""
-    return 193 * dim + 4096 + 64 * vdim + 2 * dim * vdim
+    return 193 * dim + 4096 + 64 * vdim + 3 * dim * vdim
 
 
 def general_delta_chunks(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Tensor, state_slots: torch.Tensor,

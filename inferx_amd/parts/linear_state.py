@@ -39,9 +39,9 @@ from .dense_mlp import stack_rows
 
 
 # A step goes through the generalized delta rule's chunked form if some request brings at least this many rows, where it
-# is no slower at any size of head (rows against chunks at 160 rows: 27 and 26 us for 32 heads of 32 numbers, 44 and 34
-# for 32 of 64, 58 and 58 for 16 of 128; at 112 rows 22 and 25, 34 and 32, 42 and 55).
-CORRECTED_FROM_ROWS = 160
+# is no slower at any size of head (one request, rows against chunks at 256 rows: 42 and 35 us for 32 heads of 32 numbers, 66
+# and 46 for 32 of 64, 88 and 87 for 16 of 128; at 192 rows 32 and 33, 51 and 42, 68 and 80).
+CORRECTED_FROM_ROWS = 256
 CHUNK_WORKSPACE = 128 << 20  # bytes that the chunks worked at the same time may take; longer steps go in slices
 
 

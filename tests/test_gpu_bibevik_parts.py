@@ -398,3 +398,47 @@ def test_generalized_delta_rule_in_chunks_keeps_what_is_not_finite_to_later_rows
             assert not torch.isfinite(out[row, 1]).any()
         else:
             assert not torch.isfinite(out[row:, 1]).any()
+
+
+@pytest.mark.parametrize("H,D,V", [(8, 32, 48), (8, 64, 64), (8, 128, 128)])
+@pytest.mark.parametrize("decay", [1.0, 0.6065, 0.05, 1e-3])
+def test_generalized_delta_rule_in_chunks_is_no_less_exact_than_row_by_row(H, D, V, decay):
+    """The distance of the chunked form's results and last states from the float64 recurrence, over sixteen requests, is at
+    most that of the form that walks row by row, for decays e^(-decay sigmoid(normal numbers))."""
+    from inferx_amd import ops
+    lengths = [65 + 13 * s for s in range(16)]
+    S, T, starts = len(lengths), sum(lengths), [0]
+    for n in lengths:
+        starts.append(starts[-1] + n)
+    r, k, v = (rnd((T, H * n), s, 0.7, torch.bfloat16).to(DEV) for s, n in ((1, D), (2, D), (3, V)))
+    logit = rnd((T, H * D), 4, 2.0)
+    w = torch.exp(-decay * torch.sigmoid(logit)).to(DEV)
+    u = rnd((T, H, D), 5)
+    u = (u / u.norm(dim=2, keepdim=True)).reshape(T, H * D).to(DEV)
+    a = (u * torch.sigmoid(rnd((T, H * D), 6)).to(DEV)).contiguous()
+    before = rnd((S, H * D * V), 7, 0.3).to(DEV)
+    rd, kd, vd, wd, ad, ud = (x.double().view(T, H, -1) for x in (r, k, v, w, a, u))
+    M = before.double().view(S, H, V, D).clone()
+    want = torch.empty((T, H, V), dtype=torch.float64, device=DEV)
+    for t in range(max(lengths)):  # every request's row t
+        on = torch.tensor([s for s, n in enumerate(lengths) if t < n], device=DEV)
+        at = torch.tensor(starts[:-1], device=DEV)[on] + t
+        y = (M[on] * ud[at][:, :, None]).sum(-1)
+        now = M[on] * wd[at][:, :, None] - ad[at][:, :, None] * y[..., None] + kd[at][:, :, None] * vd[at][..., None]
+        want[at] = (now * rd[at][:, :, None]).sum(-1)
+        M[on] = now
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    row0 = [(s, starts[s] + at, min(64, n - at)) for s, n in enumerate(lengths) for at in range(0, n, 64)]
+    count = [-(-n // 64) for n in lengths]
+    off, slots = [], i32(list(range(S)))
+    for chunked in (False, True):
+        state, out = before.clone(), torch.empty((T, H, V), device=DEV)
+        if chunked:
+            ops.general_delta_chunks(r, k, v, state, slots, i32([[x[1] for x in row0], [x[2] for x in row0]]),
+                                     i32([list(range(S)), [sum(count[:s]) for s in range(S)], count]), out, H, D, V, w, a, u)
+        else:
+            rows = ops.StepRows(i32([s for s, n in enumerate(lengths) for _ in range(n)]), i32(starts), slots)
+            ops.linear_state(r, k, v, state, rows, out, H, D, V, w_rows=w, a_rows=a, b_rows=u)
+        off.append([float((x.double().view(y.shape) - y).norm() / y.norm()) for x, y in ((out, want), (state, M))])
+    print(f"decay {decay}, {D} x {V}: rows {off[0][0]:.3e} {off[0][1]:.3e}, chunks {off[1][0]:.3e} {off[1][1]:.3e}")
+    assert off[1][0] <= off[0][0] and off[1][1] <= off[0][1], off

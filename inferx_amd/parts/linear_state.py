@@ -42,7 +42,7 @@ from .dense_mlp import stack_rows
 # is no slower at any size of head (one request, rows against chunks at 256 rows: 42 and 35 us for 32 heads of 32 numbers, 66
 # and 46 for 32 of 64, 88 and 87 for 16 of 128; at 192 rows 32 and 33, 51 and 42, 68 and 80).
 CORRECTED_FROM_ROWS = 256
-CHUNK_WORKSPACE = 128 << 20  # bytes that the chunks worked at the same time may take; longer steps go in slices
+CHUNK_WORKSPACE = 160 << 20  # bytes that the chunks worked at the same time may take (32 chunks of 32 heads of 64 x 64: 134 MB); longer steps go in slices
 
 
 class GeneralizedDelta(Mixer):

@@ -1271,6 +1271,12 @@ def delta_rule(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ab: torch.Tens
           _i32(dim), _i32(vdim), _i32(max_rows), _stream())
 
 
+def _lines(t: torch.Tensor):
+    """The addresses of the lines of a contiguous int32 matrix."""
+    at, step = _ptr(t), 4 * t.shape[1]
+    return [at + step * i for i in range(t.shape[0])]
+
+
 def delta_chunks_fits(q: torch.Tensor, k: torch.Tensor, state: torch.Tensor, dim: int, vdim: int) -> bool:
     """Whether `delta_chunks` takes these operands: bfloat16, key heads of 32, 64 or 128 numbers, value heads in
     sixteens, rows and state on 16-byte boundaries."""
@@ -1306,9 +1312,8 @@ def delta_chunks(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ab: torch.Te
     work = torch.empty((chunks.shape[1] * heads * delta_chunks_floats(dim, vdim),), dtype=torch.float32, device=q.device)
     _call("ix_delta_chunks", q.data_ptr(), k.data_ptr(), v.data_ptr(), _i64(q.stride(0)), _i64(k.stride(0)),
           _i64(v.stride(0)), _ptr(ab), _ptr(a_log), _ptr(dt_bias), state.data_ptr(), _i64(state.stride(0)),
-          _ptr(state_slots), _ptr(chunks[0]), _ptr(chunks[1]), _i32(chunks.shape[1]), _ptr(seqs[0]), _ptr(seqs[1]),
-          _ptr(seqs[2]), _i32(seqs.shape[1]), _ptr(work), _i64(work.numel()), _ptr(out), _i32(heads), _i32(kv_heads),
-          _i32(dim), _i32(vdim), _stream())
+          _ptr(state_slots), *_lines(chunks), _i32(chunks.shape[1]), *_lines(seqs), _i32(seqs.shape[1]), _ptr(work),
+          _i64(work.numel()), _ptr(out), _i32(heads), _i32(kv_heads), _i32(dim), _i32(vdim), _stream())
 
 
 def general_delta_fits(r: torch.Tensor, state: torch.Tensor, dim: int, vdim: int) -> bool:
@@ -1346,9 +1351,8 @@ def general_delta_chunks(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, stat
     work = torch.empty((chunks.shape[1] * heads * general_delta_floats(dim, vdim),), dtype=torch.float32, device=r.device)
     _call("ix_general_delta_chunks", r.data_ptr(), k.data_ptr(), v.data_ptr(), _i64(r.stride(0)), _i64(k.stride(0)),
           _i64(v.stride(0)), _ptr(w_rows), _ptr(a_rows), _ptr(b_rows), state.data_ptr(), _i64(state.stride(0)),
-          _ptr(state_slots), _ptr(chunks[0]), _ptr(chunks[1]), _i32(chunks.shape[1]), _ptr(seqs[0]), _ptr(seqs[1]),
-          _ptr(seqs[2]), _i32(seqs.shape[1]), _ptr(work), _i64(work.numel()), _ptr(out), _i32(heads), _i32(dim), _i32(vdim),
-          _stream())
+          _ptr(state_slots), *_lines(chunks), _i32(chunks.shape[1]), *_lines(seqs), _i32(seqs.shape[1]), _ptr(work),
+          _i64(work.numel()), _ptr(out), _i32(heads), _i32(dim), _i32(vdim), _stream())
 
 
 def channel_decays(logits: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor, heads: int, dim: int) -> None:

@@ -25,14 +25,11 @@ import torch
 from .. import ops
 from .base import Mixer, ParamSpec, StateNeed, register_part
 from .dense_mlp import stack_rows
-from .linear_state import CHUNK_WORKSPACE, chunk_slices, longest_portion, shorter_portions
+from .linear_state import CHUNK_WORKSPACE, CHUNKED_MIN_ROWS, chunk_slices, chunks_pay, shorter_portions
 from .short_conv import ShortConv
 
-# A step goes through the chunked form if some request brings at least CHUNKED_FROM_ROWS rows (16 heads of 128 x 128: 51
-# against 46 us row by row at 128 rows, 59 against 72 at 200); with it go all that bring CHUNKED_MIN_ROWS or more, the
-# others row by row.
-CHUNKED_FROM_ROWS = 160
-CHUNKED_MIN_ROWS = 16
+# What the two forms of the gated delta rule take, by the key heads' size (see `chunks_pay`).
+GATED_COSTS = {32: (0.235, 0.6, 30, 1.2, 60), 64: (0.235, 1.7, 33, 1.8, 125), 128: (0.34, 9.9, 47, 3.8, 310)}
 
 
 class GatedDeltaMixer(Mixer):
@@ -118,7 +115,7 @@ class GatedDeltaMixer(Mixer):
         o = rt.empty((T, self.num_heads, self.value_dim), torch.float32)
         sizes = (self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim)
         rows = ops.StepRows(ctx.seq_of_token, ctx.q_start, ctx.state_slots)
-        if (channel_logits is None and longest_portion(ctx) >= CHUNKED_FROM_ROWS
+        if (channel_logits is None and chunks_pay(ctx, self.num_heads, self.head_dim, self.value_dim, GATED_COSTS)
                 and ops.delta_chunks_fits(q, k, matrices, self.head_dim, self.value_dim)):
             if shorter_portions(ctx, CHUNKED_MIN_ROWS):
                 ops.delta_rule(q, k, v, ab, self.a_log, self.dt_bias, matrices, rows, o, *sizes, max_rows=CHUNKED_MIN_ROWS - 1)

@@ -38,11 +38,10 @@ from .base import Mixer, ParamSpec, StateNeed, build_part, register_part
 from .dense_mlp import stack_rows
 
 
-# A step goes through the generalized delta rule's chunked form if some request brings at least this many rows, where it
-# is no slower at any size of head (one request, rows against chunks at 256 rows: 42 and 35 us for 32 heads of 32 numbers, 66
-# and 46 for 32 of 64, 88 and 87 for 16 of 128; at 192 rows 32 and 33, 51 and 42, 68 and 80).
-CORRECTED_FROM_ROWS = 256
-CHUNK_WORKSPACE = 160 << 20  # bytes that the chunks worked at the same time may take (32 chunks of 32 heads of 64 x 64: 134 MB); longer steps go in slices
+# What the two forms of the generalized delta rule take, by the key heads' size (see `chunks_pay`).
+CORRECTED_COSTS = {32: (0.16, 0.42, 29, 1.2, 77), 64: (0.25, 3.5, 36, 1.9, 150), 128: (0.34, 12.2, 72, 4.2, 450)}
+# Bytes that the chunks worked at the same time may take (32 chunks of 32 heads of 64 x 64: 134 MB); longer steps go in slices.
+CHUNK_WORKSPACE = 160 << 20
 
 
 class GeneralizedDelta(Mixer):
@@ -88,7 +87,7 @@ class GeneralizedDelta(Mixer):
         o = rt.empty((T, H, D), torch.float32)
         rows = ops.StepRows(ctx.seq_of_token, ctx.q_start, ctx.state_slots)
         # (a decay below e^-1 would take the products of 64 of them out of float32's range)
-        if (longest_portion(ctx) >= CORRECTED_FROM_ROWS and 0.0 <= self.decay_scale <= 1.0
+        if (0.0 <= self.decay_scale <= 1.0 and chunks_pay(ctx, H, D, D, CORRECTED_COSTS)
                 and ops.general_delta_fits(r, cache.state, D, D)):
             if shorter_portions(ctx, CHUNKED_MIN_ROWS):
                 ops.linear_state(r, k, v, cache.state, rows, o, H, D, D, w_rows=w, a_rows=a, b_rows=u,
@@ -105,28 +104,69 @@ class GeneralizedDelta(Mixer):
 
 
 CHUNKED_MIN_ROWS = 16  # portions of at least this many rows are worked in chunks
+CHUNKS_HOST_US = 25    # a step's plan and two more launches a layer, which a step that waits for the host pays
 
 
-def longest_portion(ctx) -> int:
-    """The most rows that a request of the step brings, as far as the choice of a recurrence's form goes (0 in a step of
-    one token per request, which may have no host data)."""
-    if ctx.one_token_each:
-        return 0
-    if "longest_portion" not in ctx.memo:
-        ctx.memo["longest_portion"] = int((ctx.host.q_start[1:] - ctx.host.q_start[:-1]).max())
-    return ctx.memo["longest_portion"]
+def portions(ctx):
+    """How many rows each request of the step brings.  Once per step; none in a step of one token per request, which may
+    have no host data."""
+    lengths = ctx.memo.get("portions")
+    if lengths is None:
+        starts = [] if ctx.one_token_each else ctx.host.q_start.tolist()
+        lengths = ctx.memo["portions"] = [b - a for a, b in zip(starts, starts[1:])]
+    return lengths
 
 
 def shorter_portions(ctx, rows: int) -> bool:
     """Whether some request of the step brings fewer rows than `rows`."""
-    n = ctx.host.q_start[1:] - ctx.host.q_start[:-1]
-    return bool(((n > 0) & (n < rows)).any())
+    return any(0 < n < rows for n in portions(ctx))
+
+
+def chunks_pay(ctx, heads: int, dim: int, vdim: int, costs) -> bool:
+    """Whether a delta rule's step is worked faster in chunks than row by row.  Row by row the requests and heads run beside
+    each other: the time follows the longest portion until they fill the chip, then all rows.  In chunks it follows the
+    longest portion's chain of chunks, then all chunks.  `costs`, by `dim`: us a row of the longest portion and ns a row of a
+    head; us for the three launches, us a chunk of the chain and ns a chunk of a head.  Chunks are taken if they save
+    CHUNKS_HOST_US at least.
+
+    Measured, rows / chunks in us, the gated rule with 16 heads of 128 x 128: one request of 128 rows 46 / 51, of 256 87 / 59;
+    eight of 64 88 / 76, of 320 404 / 192.  The generalized one with 32 heads of 32 x 32: one of 256 42 / 35, eight of 320
+    59 / 102, 32 of 160 69 / 232; of 64 x 64: one of 160 43 / 42, of 320 81 / 48, 32 of 128 455 / 308."""
+    lengths = portions(ctx)
+    if dim not in costs or not lengths or max(lengths) < CHUNKED_MIN_ROWS:
+        return False
+    us_row, ns_row, us_chunks, us_chunk, ns_chunk = costs[dim]
+    longest, size = max(lengths), ops.LINEAR_CHUNK_ROWS
+    wide = vdim / dim
+    by_rows = max(us_row * longest, 1e-3 * ns_row * heads * wide * sum(lengths) + us_row * longest / 3)
+    chunks = sum(-(-n // size) for n in lengths if n >= CHUNKED_MIN_ROWS)
+    in_chunks = max(us_chunks * (0.8 + 0.2 * wide) + us_chunk * -(-longest // size),
+                    1e-3 * ns_chunk * heads * (1 + wide) / 2 * chunks)
+    return in_chunks + CHUNKS_HOST_US < by_rows
+
+
+def _cut(ctx, min_rows: int):
+    """The step's portions of at least `min_rows` rows cut into chunks: every chunk's first row and number of rows; the
+    requests, their first chunks and numbers of chunks."""
+    size, at = ops.LINEAR_CHUNK_ROWS, 0
+    row0, rows, seqs, first, count = [], [], [], [], []
+    for s, n in enumerate(portions(ctx)):
+        if n >= min_rows:
+            seqs.append(s)
+            first.append(len(row0))
+            row0 += range(at, at + n, size)
+            rows += [size] * (n // size)
+            if n % size:
+                rows.append(n % size)
+            count.append(len(row0) - first[-1])
+        at += n
+    return row0, rows, seqs, first, count
 
 
 def _on_device(ctx, chunks, seqs):
-    """Two lists of equally long arrays as int32 matrices on the device, in one copy from pinned memory that the host does
+    """Two lists of equally long lists as int32 matrices on the device, in one copy from pinned memory that the host does
     not wait for (two from pageable memory, each of which it waits for, cost a step of 1 ms a tenth)."""
-    flat = np.concatenate([np.asarray(a, np.int32) for a in chunks + seqs])
+    flat = np.array([x for part in chunks + seqs for x in part], np.int32)
     dev = torch.from_numpy(flat).pin_memory().to(ctx.rt.device, non_blocking=True)
     n = len(chunks) * len(chunks[0])
     return dev[:n].view(len(chunks), -1), dev[n:].view(len(seqs), -1)
@@ -140,20 +180,9 @@ def chunk_plan(ctx):
         return None, None, True
     plan = ctx.memo.get("linear_chunks")
     if plan is None:
-        n = (ctx.host.q_start[1:] - ctx.host.q_start[:-1]).astype(np.int64)
-        seqs = np.flatnonzero(n >= CHUNKED_MIN_ROWS)
-        others = bool(((n > 0) & (n < CHUNKED_MIN_ROWS)).any())
-        if len(seqs) == 0:
-            plan = (None, None, others)
-        else:
-            size = ops.LINEAR_CHUNK_ROWS
-            count = -(-n[seqs] // size)
-            first = np.cumsum(count) - count
-            which = np.repeat(np.arange(len(seqs)), count)
-            off = (np.arange(int(count.sum())) - first[which]) * size
-            rows = np.minimum(size, n[seqs][which] - off)
-            plan = _on_device(ctx, [ctx.host.q_start[seqs][which] + off, rows], [seqs, first, count]) + (others,)
-        ctx.memo["linear_chunks"] = plan
+        row0, rows, seqs, first, count = _cut(ctx, CHUNKED_MIN_ROWS)
+        plan = _on_device(ctx, [row0, rows], [seqs, first, count]) if seqs else (None, None)
+        plan = ctx.memo["linear_chunks"] = plan + (shorter_portions(ctx, CHUNKED_MIN_ROWS),)
     return plan
 
 
@@ -181,21 +210,13 @@ def chunk_slices(ctx, min_rows: int, most: int):
             if chunks is not None and chunks.shape[1] <= most:
                 ctx.memo[key] = [(chunks, seqs)]
                 return ctx.memo[key]
-        n = (ctx.host.q_start[1:] - ctx.host.q_start[:-1]).astype(np.int64)
-        seqs = np.flatnonzero(n >= min_rows)
-        size = ops.LINEAR_CHUNK_ROWS
-        count = -(-n[seqs] // size)
-        first = np.cumsum(count) - count
-        total = int(count.sum())
-        which = np.repeat(np.arange(len(seqs)), count)
-        off = (np.arange(total) - first[which]) * size
-        row0, rows = ctx.host.q_start[seqs][which] + off, np.minimum(size, n[seqs][which] - off)
+        row0, rows, seqs, first, count = _cut(ctx, min_rows)
         out = []
-        for a in range(0, total, most):
-            b = min(total, a + most)
-            lo, hi = np.maximum(first, a), np.minimum(first + count, b)
-            here = hi > lo
-            out.append(_on_device(ctx, [row0[a:b], rows[a:b]], [seqs[here], lo[here] - a, (hi - lo)[here]]))
+        for a in range(0, len(row0), most):
+            b = min(len(row0), a + most)
+            here = [(s, max(f, a) - a, min(f + c, b) - max(f, a))
+                    for s, f, c in zip(seqs, first, count) if f < b and f + c > a]
+            out.append(_on_device(ctx, [row0[a:b], rows[a:b]], [list(x) for x in zip(*here)]))
         ctx.memo[key] = out
     return ctx.memo[key]
 

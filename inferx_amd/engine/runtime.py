@@ -94,8 +94,8 @@ class Runtime:
     def _skinny_ok(self, x: torch.Tensor, w: torch.Tensor) -> bool:
         if not (x.dtype == w.dtype and 0 < x.shape[0] <= self.SKINNY_ROWS and x.is_contiguous() and w.is_contiguous()):
             return False
-        if x.dtype == torch.float32:  # (tensors of any origin meet here: their place in memory is looked at)
-            return x.shape[1] % 4 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0
+        if x.dtype == torch.float32:  # (tensors of any origin and size meet here: their place in memory is looked at)
+            return x.shape[1] % 4 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0 and w.numel() > 0
         return x.dtype == torch.bfloat16 and x.shape[1] % 8 == 0
 
     def _skinny(self, x: torch.Tensor, w: torch.Tensor, gate_up: bool, limit: float = 0.0,

@@ -259,6 +259,17 @@ def test_moe_part(dtype, tol, H, E, k, mi, si, renorm, gated, T):
                        again.view(torch.int16 if dtype == "bfloat16" else torch.int32))
 
 
+@pytest.mark.parametrize("T", [3, 33])
+def test_float32_products_without_numbers(T):
+    """An empty reduction gives zeros, no features an empty result, at every number of rows."""
+    from inferx_amd.engine.runtime import Runtime
+    rt = Runtime("float32")
+    for N, K in ((5, 0), (0, 8), (0, 0)):
+        x, w = torch.ones(T, K, device=DEV), torch.ones(N, K, device=DEV)
+        for y in (rt.linear(x, w), rt.linear_f32(x, w)):
+            assert y.shape == (T, N) and y.dtype == torch.float32 and not y.any()
+
+
 def test_moe_part_with_wide_expert_tiles():
     """The expert products' wide form (chosen by the part from a width of 3,072 on; forced here at a small one)
     gives the bits of the narrow form, with the shared expert on the main stream."""

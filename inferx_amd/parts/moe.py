@@ -179,9 +179,10 @@ class MoeFeedForward(FeedForward):
         return ops.MOE_TILED_F32_ROWS if x.dtype == torch.float32 else ops.moe_tiled_rows(self.wide_tiles)
 
     def _f32_fits(self, x) -> bool:
-        """What the float32 products on the matrix cores ask for beside whole 16-byte pieces: 32-bit offsets."""
+        """What the float32 products on the matrix cores ask for beside whole 16-byte pieces: rows on 16-byte boundaries
+        and 32-bit offsets."""
         A = x.shape[0] * self.top_k
-        return (max(x.shape[0] * self.hidden_size, A * self.expert_width) < 1 << 31
+        return (x.data_ptr() % 16 == 0 and max(x.shape[0] * self.hidden_size, A * self.expert_width) < 1 << 31
                 and (2 if self.gated else 1) * self.expert_width * self.hidden_size < 1 << 31
                 and ops.moe_max_tiles(A, self.num_experts, 16) < 65536)
 
@@ -225,7 +226,8 @@ class MoeFeedForward(FeedForward):
         """Few tokens (decoding): routed and shared experts go into one launch per product."""
         return (tile_rows == 16 and self.shared_width > 0 and self.shared_width % (16 // x.element_size()) == 0
                 and x.shape[0] <= ctx.rt.SKINNY_ROWS and self.w_shared_gate_up.dtype == x.dtype
-                and self.w_shared_down.dtype == x.dtype)
+                and self.w_shared_down.dtype == x.dtype
+                and (x.dtype == torch.bfloat16 or self.w_shared_down.data_ptr() % 16 == 0))
 
     def experts_and_shared(self, ctx, x, offsets, rows, tile_map, tile_rows):
         rt, A, T = ctx.rt, rows.numel(), x.shape[0]

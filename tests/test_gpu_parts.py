@@ -270,6 +270,28 @@ def test_float32_products_without_numbers(T):
             assert y.shape == (T, N) and y.dtype == torch.float32 and not y.any()
 
 
+@pytest.mark.parametrize("T", [3, 17, 70])
+def test_float32_experts_on_rows_at_any_place(T):
+    """Rows and a shared expert's weights that do not lie on 16-byte boundaries give what those that do give, to the order of
+    float32 sums."""
+    from inferx_amd.config import PartSpec
+    from inferx_amd.engine.runtime import Runtime
+    from inferx_amd.parts import build_part, resolve_delta
+    rt, H = Runtime("float32"), 64
+    part = build_part("feed_forward", PartSpec("moe", {"hidden_size": H, "num_experts": 4, "top_k": 2, "expert_width": 32,
+                                                       "shared_width": 64, "init_std": 0.15}))
+    w = {n: t.to(DEV) for n, t in tensors_for(part, rt, seed=8).items()}
+    place = lambda t, off: torch.cat([t.new_zeros(off), t.reshape(-1)])[off:].view(t.shape)
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(9)).to(DEV)
+    ctx, _ = make_ctx(rt, [T], [T], 16, T // 16 + 2)
+    part.bind(dict(w), rt)
+    want = resolve_delta(ctx, part.forward(ctx, x))
+    name = "shared_expert.down_proj.weight"
+    part.bind(dict(w, **{name: place(w[name], 1)}), rt)
+    for off in (0, 1, 3):
+        assert err(resolve_delta(ctx, part.forward(ctx, place(x, off))), want) < 1e-5, f"rows {off} numbers off"
+
+
 def test_moe_part_with_wide_expert_tiles():
     """The expert products' wide form (chosen by the part from a width of 3,072 on; forced here at a small one)
     gives the bits of the narrow form, with the shared expert on the main stream."""

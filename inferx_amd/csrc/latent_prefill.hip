@@ -22,8 +22,13 @@
 // A workgroup takes sixteen consecutive rows of the step and four heads.  Rows of several requests in a tile are worked
 // request by request (the other rows' keys all masked: they change nothing).
 //
-// Measured at 2,048 tokens of 16 heads, rank 512 with 64 rotated numbers: 168 us, against 390 with a head's sixteen columns
-// in one wavefront through both products and the rows written transposed, 314 with the products split as here.
+// There are three forms by the size of a row; the smaller ones take less LDS, and more workgroups share a compute unit.
+//
+// Measured with 16 heads, one prompt of 2,048 tokens | 32 prompts of 160, us, against a head's sixteen columns in one
+// wavefront through both products and the rows written transposed (latent + rotated numbers): 512 + 64 148 | 72 (378 | 145),
+// 448 + 64 155 | 73 (353 | 137), 256 + 64 118 | 46 (216 | 88), 128 + 64 112 | 39 (163 | 69), 64 + 32 85 | 22 (109 | 25),
+// 32 + 32 85 | 20.5 (86 | 21).  One form of 78 KB of LDS for all sizes took 113 | 35 and 111 | 33 us at the last two;
+// branches past the products that a smaller row does without, 258 | 104 us at 448 + 64.
 #include "common.h"
 
 typedef __bf16 lp_bf16x8 __attribute__((ext_vector_type(8)));
@@ -31,13 +36,17 @@ typedef __bf16 lp_bf16x4 __attribute__((ext_vector_type(4)));
 typedef float lp_f32x4 __attribute__((ext_vector_type(4)));
 
 #define LP_KEYS 32
-#define LP_MAIN 512  // numbers of a row's first 64 pieces of 16 bytes; the rest, at most eight pieces, lie in rows of 64
-#define LP_TAIL 64
+// A row's numbers in LDS, by the size of the form: its first 16, 32 or 64 pieces of 16 bytes, and where there are more (at
+// most eight) the rest in rows of their own.
+constexpr int lp_main(int nw) { return nw <= 4 ? 128 : nw <= 10 ? 256 : 512; }
+constexpr int lp_tail(int nw) { return 32 * nw > lp_main(nw) ? 64 : 0; }
+constexpr int lp_lds_bytes(int nw) { return 256 + 2 * LP_KEYS * (64 + 2 * (lp_main(nw) + lp_tail(nw))); }
+constexpr int lp_per_unit(int nw) { return nw <= 4 ? 4 : 2; }  // workgroups that a compute unit holds
 
-// Where piece p of key row r lies among the rows' first 64 pieces (or among their last eight), in numbers: a row's pieces
-// are permuted so that the sixteen rows that one product reads at one piece (8 a + b, or 8 a + 4 + b; a, b < 4) fall on
-// all banks.  A row is brought by one instruction that fills 64 pieces in the order of the lanes, so it is the lanes'
-// source addresses that are permuted.
+// Where piece p of key row r lies among the rows' first pieces (or among their last eight): a row's pieces are permuted
+// so that the sixteen rows that one product reads at one piece (8 a + b, or 8 a + 4 + b; a, b < 4) fall on all banks.
+// One instruction fills 64 pieces in the order of the lanes (one, two or four rows), so it is the lanes' source
+// addresses that are permuted.
 __device__ __forceinline__ int lp_swap(int r) { return ((r >> 3) << 2) | (r & 3); }
 __device__ __forceinline__ int lp_swap_tail(int r) { return ((r >> 3) << 1) | ((r >> 1) & 1); }
 // 16 bytes of every live lane from memory into LDS, side by side in the order of the lanes
@@ -51,9 +60,11 @@ __device__ __forceinline__ lp_s16x4 lp_read_turned(const __bf16* at) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) lp_s16x4*)at);
 }
 
-// rank + rot_dim <= 32 NW, rank <= 16 NR; FULL: both are these sizes
+// rank + rot_dim <= 32 NW, rank <= 16 NR.  The loops over a row always run to these sizes (behind a smaller row lie zeros):
+// with a branch at each product the compiler waits for every operand.  FULL: both are these sizes, which are then numbers
+// that the compiler knows (148 us instead of 157 at 2,048 tokens of 512 + 64, the largest form and the usual latent).
 template <int NW, int NR, bool FULL>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, lp_per_unit(NW))
 latent_prefill_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_h, const __bf16* __restrict__ qr,
                       int64_t qr_t, int64_t qr_h, const __bf16* __restrict__ cache,
                       const int32_t* __restrict__ block_table, const int32_t* __restrict__ seq_of_token,
@@ -62,18 +73,20 @@ latent_prefill_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_h,
                       int n_tiles, int inwards, int window, const __bf16* __restrict__ head_gate, int64_t gate_stride) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lp_lds[];
   constexpr int DT = NR / 4;  // tiles of sixteen numbers of the latent that a wavefront sums up
+  constexpr int MAIN = lp_main(NW), TAIL = lp_tail(NW);
+  constexpr int PIECES = MAIN / 8, TOGETHER = 64 / PIECES;  // rows that one instruction brings
   const int width = FULL ? 32 * NW : rank + rot_dim;
   if (FULL) rank = 16 * NR;
   const int p8 = width / 8, nw = width / 32, nr = rank / 16;
   float* const alpha_s = reinterpret_cast<float*>(lp_lds);             // [4][16]: the factor of a column's sums; at the end 1 / sum
   __bf16* const p_s = reinterpret_cast<__bf16*>(alpha_s + 64);         // [4][16][32]: weights
-  __bf16* const k_s = p_s + 4 * 16 * LP_KEYS;  // two buffers of rows: [32][LP_MAIN], then [32][LP_TAIL]
-  constexpr int BUFFER = LP_KEYS * (LP_MAIN + LP_TAIL);
+  __bf16* const k_s = p_s + 4 * 16 * LP_KEYS;  // two buffers of rows: [32][MAIN], then [32][TAIL]
+  constexpr int BUFFER = LP_KEYS * (MAIN + TAIL);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, g = lane >> 4;
   // one row of workgroups, a tile's groups of four heads side by side; the tiles with the most keys first, or (inwards:
-  // all workgroups are resident at once, two to a compute unit) the second half of them in the order of rising length,
+  // all workgroups are resident at once) the second half of them in the order of rising length,
   // so that a compute unit gets a long and a short one
   const int head_groups = (heads + 3) / 4;
   const int at = static_cast<int>(blockIdx.x) / head_groups, half = (n_tiles + 1) / 2;
@@ -100,6 +113,10 @@ latent_prefill_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_h,
 #pragma unroll
     for (int d = 0; d < DT; ++d) acc[c][d] = lp_f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -1e30f, l = 0.f;
+  if (!FULL && width < 32 * NW) {  // (what no row fills is zero; the barrier before the first rows orders these writes)
+    const lp_bf16x8 zero = {(__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f};
+    for (int i = tid; i < 2 * BUFFER / 8; i += 256) *reinterpret_cast<lp_bf16x8*>(k_s + 8 * i) = zero;
+  }
 
   int seg = r0;
   while (seg < r1) {  // (every decision in this loop is the same for the whole workgroup)
@@ -126,13 +143,15 @@ latent_prefill_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_h,
         return (static_cast<int64_t>(table[j / page_size]) * page_size + j % page_size) * width;
       };
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int r = 8 * wave + u, piece = lane ^ lp_swap(r);
-        const int64_t from = row_at(u);
-        if (FULL || piece < p8) lp_bring(cache + from + 8 * piece, to + r * LP_MAIN);
+      for (int u = 0; u < 8; u += TOGETHER) {
+        const int v = TOGETHER > 1 ? u + lane / PIECES : u, r = 8 * wave + v, piece = (lane % PIECES) ^ lp_swap(r);
+        const int64_t from = row_at(v);
+        if (FULL || piece < p8) lp_bring(cache + from + 8 * piece, to + (8 * wave + u) * MAIN);
       }
-      const int r = 8 * wave + (lane >> 3), piece = 64 + ((lane & 7) ^ lp_swap_tail(r));
-      if (piece < p8) lp_bring(cache + row_at(lane >> 3) + 8 * piece, to + LP_KEYS * LP_MAIN + 8 * wave * LP_TAIL);
+      if constexpr (TAIL > 0) {
+        const int r = 8 * wave + (lane >> 3), piece = PIECES + ((lane & 7) ^ lp_swap_tail(r));
+        if (piece < p8) lp_bring(cache + row_at(lane >> 3) + 8 * piece, to + LP_KEYS * MAIN + 8 * wave * TAIL);
+      }
     };
     __syncthreads();  // (the request before: its last round has been read)
     if (k_begin < k_end) bring(k_begin, k_s, lane);
@@ -154,28 +173,26 @@ latent_prefill_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_h,
         // piece's number (a tail's on the last three), so pieces 4 q + g of q = i, i + 4, .. are a constant apart
         const int r = 8 * (n_ >> 2) + (n_ & 3);
         const __bf16* main_at[4];
-        const __bf16* tail_at[2];
+        const __bf16* tail_at[2];  // (not used where there are none)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) main_at[i] = rows + r * LP_MAIN + (((4 * i + g_) ^ lp_swap(r)) << 3);
+        for (int i = 0; i < 4; ++i) main_at[i] = rows + r * MAIN + (((4 * i + g_) ^ lp_swap(r)) << 3);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) tail_at[i] = rows + LP_KEYS * LP_MAIN + r * LP_TAIL + (((4 * i + g_) ^ lp_swap_tail(r)) << 3);
+        for (int i = 0; i < 2; ++i) tail_at[i] = rows + LP_KEYS * MAIN + r * TAIL + (((4 * i + g_) ^ lp_swap_tail(r)) << 3);
         // (two pairs of operands on their way while one is multiplied; left to itself the compiler waits for every pair)
         lp_bf16x8 a0[3], a1[3];
         auto read = [&](int q) {
-          const __bf16* at = q < 16 ? main_at[q & 3] + 128 * (q >> 2) : tail_at[q & 1];
+          const __bf16* at = q < MAIN / 32 ? main_at[q & 3] + 128 * (q >> 2) : tail_at[q & 1];
           a0[q % 3] = *reinterpret_cast<const lp_bf16x8*>(at);
-          a1[q % 3] = *reinterpret_cast<const lp_bf16x8*>(at + 4 * (q < 16 ? LP_MAIN : LP_TAIL));
+          a1[q % 3] = *reinterpret_cast<const lp_bf16x8*>(at + 4 * (q < MAIN / 32 ? MAIN : TAIL));
         };
         read(0);
-        if (FULL || 1 < nw) read(1);
+        read(1);
 #pragma unroll
         for (int q = 0; q < NW; ++q) {
-          if (q + 2 < NW && (FULL || q + 2 < nw)) read(q + 2);
+          if (q + 2 < NW) read(q + 2);
           __builtin_amdgcn_sched_barrier(0);
-          if (FULL || q < nw) {
-            s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[q % 3], qf[q], s0, 0, 0, 0);
-            s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[q % 3], qf[q], s1, 0, 0, 0);
-          }
+          s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[q % 3], qf[q], s0, 0, 0, 0);
+          s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[q % 3], qf[q], s1, 0, 0, 0);
         }
         float p[8], mx = -INFINITY;
 #pragma unroll
@@ -224,23 +241,21 @@ latent_prefill_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_h,
       // this lane's part of the transposed reads: key 8 g + n / 4 (and four keys on), numbers 4 (n % 4) .. of a tile's
       // sixteen; they lie in piece 2 D + (n % 4) / 2 of the row (D the tile), and D and D + 8 are a constant apart
       const int r = 8 * g_ + (n_ >> 2), in_piece = 4 * (n_ & 1);
-      const __bf16* at = rows + r * LP_MAIN + in_piece;
+      const __bf16* at = rows + r * MAIN + in_piece;
       lp_s16x4 lo[2], hi[2];
       auto read = [&](int d) {
         const __bf16* from = at + (((2 * (wave * DT + d) + ((n_ >> 1) & 1)) ^ lp_swap(r)) << 3);
         lo[d & 1] = lp_read_turned(from);
-        hi[d & 1] = lp_read_turned(from + 4 * LP_MAIN);
+        hi[d & 1] = lp_read_turned(from + 4 * MAIN);
       };
-      if (FULL || wave * DT < nr) read(0);
+      read(0);
 #pragma unroll
       for (int d = 0; d < DT; ++d) {
-        if (d + 1 < DT && (FULL || wave * DT + d + 1 < nr)) read(d + 1);
+        if (d + 1 < DT) read(d + 1);
         __builtin_amdgcn_sched_barrier(0);
-        if (FULL || wave * DT + d < nr) {
-          const lp_bf16x8 a = __builtin_bit_cast(lp_bf16x8, __builtin_shufflevector(lo[d & 1], hi[d & 1], 0, 1, 2, 3, 4, 5, 6, 7));
+        const lp_bf16x8 a = __builtin_bit_cast(lp_bf16x8, __builtin_shufflevector(lo[d & 1], hi[d & 1], 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
-          for (int c = 0; c < 4; ++c) acc[c][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb[c], acc[c][d], 0, 0, 0);
-        }
+        for (int c = 0; c < 4; ++c) acc[c][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb[c], acc[c][d], 0, 0, 0);
       }
     }
     seg = end;
@@ -277,14 +292,14 @@ int ix_latent_prefill(const void* ql, int64_t ql_t, int64_t ql_h, const void* qr
                       int max_blocks, float scale_log2, int window, const void* head_gate, int64_t gate_stride,
                       hipStream_t stream) {
   const int width = rank + rot_dim, n_tiles = (tokens + 15) / 16;
-  const size_t lds = 256 + 2 * static_cast<size_t>(LP_KEYS) * (64 + 2 * (LP_MAIN + LP_TAIL));
   const int64_t groups = static_cast<int64_t>(n_tiles) * ((heads + 3) / 4);
   IX_REQUIRE(groups < (int64_t(1) << 31), "too many workgroups for one launch");
   const dim3 grid(static_cast<unsigned>(groups));
-  const int inwards = groups <= 512;  // (two workgroups on each of 256 compute units)
 #define LAUNCH(NW, NR, FULL)                                                                                            \
   do {                                                                                                                  \
     auto kernel = latent_prefill_kernel<NW, NR, FULL>;                                                                  \
+    constexpr size_t lds = lp_lds_bytes(NW);                                                                            \
+    const int inwards = groups <= 256 * lp_per_unit(NW); /* (all of them on the 256 compute units at once) */           \
     if (lds > 48 * 1024) {                                                                                              \
       static bool raised = false;                                                                                       \
       if (!raised) {                                                                                                    \
@@ -300,7 +315,7 @@ int ix_latent_prefill(const void* ql, int64_t ql_t, int64_t ql_h, const void* qr
                        tokens, heads, rank, rot_dim, page_size, max_blocks, scale_log2, n_tiles, inwards, window,       \
                        (const __bf16*)head_gate, gate_stride);                                                          \
   } while (0)
-  if (width <= 128 && rank <= 128) LAUNCH(4, 8, false);
+  if (width <= 128) LAUNCH(4, 8, false);
   else if (width <= 320 && rank <= 256) LAUNCH(10, 16, false);
   else if (width == 576 && rank == 512) LAUNCH(18, 32, true);
   else LAUNCH(18, 32, false);

@@ -359,6 +359,35 @@ def test_latent_attention_of_prompts(H, rank, rot, page, window, gated):
     assert torch.isfinite(out).all() and err <= 2e-2, f"{err:.2e}"
 
 
+# the smallest sizes of the kernel's three forms and their largest (128, 320 with a latent of 256, 576), one row of each
+# with fewer numbers than the form has room for
+@pytest.mark.parametrize("rank,rot", [(16, 16), (96, 0), (112, 16), (128, 32), (144, 48), (256, 64), (272, 16), (512, 0), (512, 64)])
+def test_latent_attention_of_prompts_behind_a_launch_that_left_nan(rank, rot):
+    """What is behind a row in LDS (here what a launch on a cache of nothing but NaN left there) reaches no result."""
+    from inferx_amd import ops
+    T, H, page = 75, 6, 16
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=DEV)
+    seq, pos, table = i32([0] * T), i32(list(range(T))), i32([[2, 0, 1, 4, 3]])
+
+    def run(rank, rot, seed, fill=None, op=ops.latent_attention_mfma):
+        cache = rnd((5, 1, page, rank + rot), seed, 1.0, torch.bfloat16).to(DEV)
+        if fill is not None:
+            cache.fill_(fill)
+        q = rnd((T, H, rank + 64), seed + 1, 2.0, torch.bfloat16).to(DEV)
+        out = torch.full((T, H, rank), float("nan"), dtype=torch.bfloat16, device=DEV)
+        args = (q[:, :, :rank], q[:, :, rank:rank + rot] if rot else q, cache)
+        if op is ops.latent_attention_plain:
+            out, args = out.float(), tuple(t.float().contiguous() for t in args)
+        op(*args, table, seq, pos, out, rank, rot, (rank + rot) ** -0.5)
+        return out.float()
+
+    for _ in range(20):  # (every compute unit's LDS)
+        run(512, 64, 5, float("nan"))
+    got, want = run(rank, rot, 7), run(rank, rot, 7, op=ops.latent_attention_plain)
+    err = float((got - want).abs().max()) / float(want.abs().max())
+    assert torch.isfinite(got).all() and err <= 2e-2, f"{err:.2e}"
+
+
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
 @pytest.mark.parametrize("row", [0, 7, 37, 64, 99])
 def test_generalized_delta_rule_in_chunks_keeps_what_is_not_finite_to_later_rows(row, bad):

@@ -83,22 +83,19 @@ class Runtime:
             return t.to(self.device, torch.float32)
         return t.to(self.device, torch.bfloat16)
 
-    # ---- few rows (decoding): the weights are the traffic, so they are streamed (`ops.linear_skinny`) instead of going
-    # through a library product tuned for tiles.
-    # bfloat16, up to two 16-row tiles: a decode step of 6 layers at batch 17 / 24 / 32 took 1477 / 1642 / 1822 us against
+    # ---- few rows (decoding): the weights are the traffic, so they are streamed by the matrix-core kernel
+    # that also serves the experts (one "expert", one row tile), instead of a library product tuned for tiles
+    # Up to two 16-row tiles: a decode step of 6 layers at batch 17 / 24 / 32 took 1477 / 1642 / 1822 us against
     # 1566 / 1691 / 1837 us through the library's products; from 48 rows on the library is faster (1966 against 2120).
+    # In float32 the library's products of 8 rows took 12 to 84 us a product of the A2.7B shape (1.5 TB/s at best),
+    # the streaming kernel's 6 to 13; the vocabulary's 1.2 GB 249 us, 5.0 TB/s.
     SKINNY_ROWS = 32
-    # float32, whose matrix instructions do a sixteenth of the work: a decode step of the A2.7B shape, 4 layers, at batch
-    # 2 / 4 / 6 / 8 took 863 / 1026 / 1190 / 1329 us against 916 / 1070 / 1221 / 1342 through the library's, at 10 / 12 / 16 /
-    # 32 1483 / 1620 / 1773 / 2335 against 1470 / 1596 / 1726 / 2194.
-    SKINNY_ROWS_F32 = 8
 
     def _skinny_ok(self, x: torch.Tensor, w: torch.Tensor) -> bool:
         if not (x.dtype == w.dtype and 0 < x.shape[0] <= self.SKINNY_ROWS and x.is_contiguous() and w.is_contiguous()):
             return False
         if x.dtype == torch.float32:  # (tensors of any origin and size meet here: their place in memory is looked at)
-            return (x.shape[0] <= self.SKINNY_ROWS_F32 and x.shape[1] % 4 == 0 and w.numel() > 0
-                    and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+            return x.shape[1] % 4 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0 and w.numel() > 0
         return x.dtype == torch.bfloat16 and x.shape[1] % 8 == 0
 
     def _skinny(self, x: torch.Tensor, w: torch.Tensor, gate_up: bool, limit: float = 0.0,

@@ -400,14 +400,15 @@ latent_attn_mfma_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_
   }
 }
 
-// decode != 0: one token per request (tokens == requests); with n_splits > 1 the keys are cut into that many slices,
-// part_o float32 [tokens * heads * n_splits, rank] and part_ml float32 [tokens * heads * n_splits, 2] take what the
-// slices leave, and out must be contiguous [tokens, heads, rank].  head_gate as for the plain kernel (bfloat16).
 int ix_latent_prefill(const void* ql, int64_t ql_t, int64_t ql_h, const void* qr, int64_t qr_t, int64_t qr_h,
                       const void* cache, const int32_t* block_table, const int32_t* seq_of_token, const int32_t* positions,
                       void* out, int64_t out_t, int64_t out_h, int tokens, int heads, int rank, int rot_dim, int page_size,
                       int max_blocks, float scale_log2, int window, const void* head_gate, int64_t gate_stride,
                       hipStream_t stream);  // latent_prefill.hip
+
+// decode != 0: one token per request (tokens == requests); with n_splits > 1 the keys are cut into that many slices,
+// part_o float32 [tokens * heads * n_splits, rank] and part_ml float32 [tokens * heads * n_splits, 2] take what the
+// slices leave, and out must be contiguous [tokens, heads, rank].  head_gate as for the plain kernel (bfloat16).
 extern "C" int ix_latent_attention_mfma(const void* ql, int64_t ql_t, int64_t ql_h, const void* qr, int64_t qr_t,
                                         int64_t qr_h, const void* cache, const int32_t* block_table,
                                         const int32_t* seq_of_token, const int32_t* positions, void* out,

@@ -272,7 +272,8 @@ moe_grouped_dual_kernel(const TI* a, const TI* w, TI* __restrict__ out,
 // `max_tiles` bounds the number of row tiles (the grid); the kernel reads the true number from tile_info.
 // tile_rows (16, 32 or 64) must be what the grouping kernel was given.  gate_up: 0 a plain product, 1 gate|up rows
 // with SwiGLU, 2 a plain product whose results pass the square of relu.  glu_limit > 0: the gate|up rows meet in
-// the clamped form (`ix_glu`).  dtype: all of a, w and out (float32: k_split 4 only).
+// the clamped form (`ix_glu`).  dtype: all of a, w and out (float32: tiles of 16 rows and k_split 4 only, which is what
+// steps of few rows take).
 #define IX_REQUIRE_PIECES(dtype, width)                                                                     \
   IX_REQUIRE(dtype == IX_F32 || dtype == IX_BF16, "dtype must be float32 or bfloat16");                      \
   IX_REQUIRE(width % (dtype == IX_F32 ? 4 : 8) == 0, "rows of the reduction must be multiples of 16 bytes")
@@ -284,7 +285,8 @@ extern "C" int ix_moe_grouped_mfma(const void* a, const void* w, void* out, int 
   IX_REQUIRE_PIECES(dtype, width);
   IX_REQUIRE(n_out < (1 << 30) && width < (1 << 30), "sizes too large");
   IX_REQUIRE(tile_rows == 16 || tile_rows == 32 || tile_rows == 64, "tile_rows must be 16, 32 or 64");
-  IX_REQUIRE(k_split == 4 || (k_split == 1 && dtype == IX_BF16), "k_split must be 1 (bfloat16 only) or 4");
+  IX_REQUIRE(k_split == 1 || k_split == 4, "k_split must be 1 or 4");
+  IX_REQUIRE(dtype == IX_BF16 || (tile_rows == 16 && k_split == 4), "float32: tiles of 16 rows and k_split 4 only");
   IX_REQUIRE(gate_up >= 0 && gate_up <= 2, "gate_up must be 0, 1 or 2");
   IX_REQUIRE(max_tiles <= 65535, "too many row tiles for one launch");
   if (max_tiles == 0) return 0;
@@ -295,17 +297,17 @@ extern "C" int ix_moe_grouped_mfma(const void* a, const void* w, void* out, int 
                      (const TI*)w, (TI*)out, offsets, rows, tile_expert, tile_row0, tile_info, (int)n_out,         \
                      (int)width, gate_up == 2 ? 1 : 0, glu_limit)
 #define PICK(MT)                                       \
-  if (dtype == IX_F32) {                               \
-    if (gate_up == 1) LAUNCH(MT, true, 4, float);      \
-    else LAUNCH(MT, false, 4, float);                  \
-  } else if (gate_up == 1) {                           \
+  if (gate_up == 1) {                                  \
     if (k_split > 1) LAUNCH(MT, true, 4, __bf16);      \
     else LAUNCH(MT, true, 1, __bf16);                  \
   } else {                                             \
     if (k_split > 1) LAUNCH(MT, false, 4, __bf16);     \
     else LAUNCH(MT, false, 1, __bf16);                 \
   }
-  if (tile_rows == 16) { PICK(1) } else if (tile_rows == 32) { PICK(2) } else { PICK(4) }
+  if (dtype == IX_F32) {
+    if (gate_up == 1) LAUNCH(1, true, 4, float);
+    else LAUNCH(1, false, 4, float);
+  } else if (tile_rows == 16) { PICK(1) } else if (tile_rows == 32) { PICK(2) } else { PICK(4) }
 #undef PICK
 #undef LAUNCH
   return ix_check_launch("ix_moe_grouped_mfma");
@@ -325,6 +327,7 @@ extern "C" int ix_moe_grouped_dual(const void* a, const void* w, void* out, int 
   IX_REQUIRE_PIECES(dtype, width_s);
   IX_REQUIRE(n_out < (1 << 24) && width < (1 << 30) && n_out_s < (1 << 24) && width_s < (1 << 30), "sizes too large");
   IX_REQUIRE(tile_rows == 16 || tile_rows == 32 || tile_rows == 64, "tile_rows must be 16, 32 or 64");
+  IX_REQUIRE(dtype == IX_BF16 || tile_rows == 16, "float32: tiles of 16 rows only");
   // one column block per workgroup: two (the rows read once for 32 out-features) measured slower at every tile
   // height, 64 against 60 us for the gate|up product of a decoding step, for want of wavefronts in flight
   const int nb = 1;
@@ -338,16 +341,13 @@ extern "C" int ix_moe_grouped_dual(const void* a, const void* w, void* out, int 
                      (TI*)out, offsets, rows, tile_expert, tile_row0, tile_info, max_tiles, (int)n_out,            \
                      (int)width, (const TI*)a_s, (const TI*)w_s, (TI*)out_s, shared_rows, (int)n_out_s,             \
                      (int)width_s, glu_limit, glu_limit_s)
-#define PICK(MT, NB)                                   \
-  if (dtype == IX_F32) {                               \
-    if (gate_up == 1) LAUNCH(MT, true, NB, float);     \
-    else LAUNCH(MT, false, NB, float);                 \
-  } else if (gate_up == 1) {                           \
-    LAUNCH(MT, true, NB, __bf16);                      \
-  } else {                                             \
-    LAUNCH(MT, false, NB, __bf16);                     \
-  }
-  if (tile_rows == 16) { PICK(1, 1) } else if (tile_rows == 32) { PICK(2, 1) } else { PICK(4, 1) }
+#define PICK(MT, NB)                          \
+  if (gate_up == 1) LAUNCH(MT, true, NB, __bf16); \
+  else LAUNCH(MT, false, NB, __bf16);
+  if (dtype == IX_F32) {
+    if (gate_up == 1) LAUNCH(1, true, 1, float);
+    else LAUNCH(1, false, 1, float);
+  } else if (tile_rows == 16) { PICK(1, 1) } else if (tile_rows == 32) { PICK(2, 1) } else { PICK(4, 1) }
 #undef PICK
 #undef LAUNCH
   return ix_check_launch("ix_moe_grouped_dual");

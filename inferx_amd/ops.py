@@ -648,8 +648,8 @@ def _need_pieces(a: torch.Tensor, *others: torch.Tensor) -> None:
 def moe_grouped_mfma(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offsets: torch.Tensor,
                      rows: Optional[torch.Tensor], tile_map: torch.Tensor, tile_rows: int, gate_up: bool,
                      k_split: int, glu_limit: float = 0.0) -> None:
-    """Grouped product on the matrix cores (all bfloat16, or all float32 with k_split 4), shapes as
-    `moe_grouped_plain`; `tile_map` from `moe_dispatch`."""
+    """Grouped product on the matrix cores (all bfloat16, or all float32 with tiles of 16 rows and k_split 4),
+    shapes as `moe_grouped_plain`; `tile_map` from `moe_dispatch`."""
     E = w.shape[0]
     A, n_out = out.shape
     K = a.shape[1]

@@ -525,7 +525,7 @@ def test_grouped_products_in_float32(counts, K, n, kind, gate_up, limit):
     x, w = buf(T, 0)[:T], buf(E * wn, 1)[:E * wn].view(E, wn, K)
     offsets = torch.tensor([sum(counts[:e]) for e in range(E + 1)], dtype=torch.int32, device=DEV)
     rows = torch.randint(0, T, (A,), generator=torch.Generator().manual_seed(2)).to(torch.int32).to(DEV)
-    tr = ops.MOE_TILED_F32_ROWS if kind == "tiled" else 32
+    tr = ops.MOE_TILED_F32_ROWS if kind == "tiled" else 16
     mt = ops.moe_max_tiles(A, E, tr)
     tiles = [(e, int(offsets[e]) + r) for e in range(E) for r in range(0, counts[e], tr)]
     tile_map = torch.zeros(2 * mt + 1, dtype=torch.int32)

@@ -23,14 +23,13 @@
 // adds to them.  The reduction runs in stages of 64 through two LDS buffers, and a stage in halves of 32: while a half is
 // multiplied, the next half's operands are already on their way from LDS into other registers, also over the end of the
 // stage, and the next stage's writes and the loads of the stages after it stand between the products.  One barrier a
-// stage, between its halves.  Both products, us, against operands read behind the barrier and each use waited for:
-// 60 experts of 1,408, rows of 2,048 numbers: 136 rows each 183 + 106 (190 + 107); 23 rows and four experts of 340
-// rows 140 + 79 (163 + 87); one expert of 2,048 rows 123 + 66 (158 + 84).  64 experts of 2,560, rows of 3,584, wide: 64 rows
-// each 404 + 241 (409 + 241); with eight experts of 512 rows 562 + 307 (570 + 315), 85 rows and eight of 682 608 + 348
-// (680 + 379).  (Weights straight into registers as operands, past LDS: sixteen rows of 64 bytes a load are half as
-// fast for one compute unit as eight of 128.  One wavefront a SIMD with 512 registers: no better.)
-// LDS rows are 128 bytes with their 16-byte
-// pieces permuted, so that operand reads and writes fall on distinct banks.
+// stage, between its halves.  Both products, us, against operands read behind the barrier, each use waited for, and row
+// tiles dealt to the dies as wholes: 60 experts of 1,408, rows of 2,048 numbers: 136 rows each 166 + 98 (185 + 104); 23 rows
+// and four experts of 340 rows 143 + 77 (169 + 93); one expert of 5,632 with 2,048 rows 109 + 60 (150 + 82).  64 experts of
+// 2,560, rows of 3,584, wide: 64 rows each 403 + 241 (406 + 241); with eight experts of 512 rows 543 + 305 (579 + 328), 85
+// rows and eight of 682 587 + 348 (684 + 387).  (Weights straight into registers as operands, past LDS: sixteen rows of 64
+// bytes a load are half as fast for one compute unit as eight of 128.  One wavefront a SIMD with 512 registers: no better.)
+// LDS rows are 128 bytes with their 16-byte pieces permuted, so that operand reads and writes fall on distinct banks.
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));

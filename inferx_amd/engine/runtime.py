@@ -83,12 +83,16 @@ class Runtime:
             return t.to(self.device, torch.float32)
         return t.to(self.device, torch.bfloat16)
 
-    # ---- few rows (decoding): the weights are the traffic, so they are streamed by the matrix-core kernel
-    # that also serves the experts (one "expert", one row tile), instead of a library product tuned for tiles
-    # Up to two 16-row tiles: a decode step of 6 layers at batch 17 / 24 / 32 took 1477 / 1642 / 1822 us against
+    # ---- few rows (decoding): the weights are the traffic, so they are streamed (`ops.linear_skinny`) instead of going
+    # through a library product tuned for tiles.
+    # bfloat16, up to two 16-row tiles: a decode step of 6 layers at batch 17 / 24 / 32 took 1477 / 1642 / 1822 us against
     # 1566 / 1691 / 1837 us through the library's products; from 48 rows on the library is faster (1966 against 2120).
-    # In float32 the library's products of 8 rows took 12 to 84 us a product of the A2.7B shape (1.5 TB/s at best),
-    # the streaming kernel's 6 to 13; the vocabulary's 1.2 GB 249 us, 5.0 TB/s.
+    # 8 layers with the kernel as it is now, batch 8 / 16 / 17 / 24 / 32: 743 / 936 / 1001 / 1124 / 1243 us against 840 /
+    # 1009 / 1018 / 1126 / 1225.
+    # float32: a decode step of the A2.7B shape, 4 layers, at batch 2 / 4 / 6 / 8 took 863 / 1026 / 1190 / 1329 us against
+    # 916 / 1070 / 1221 / 1342 through the library's products, at 10 / 16 / 32 1483 / 1773 / 2335 against 1470 / 1726 / 2194.
+    # The line is bfloat16's all the same: with one at 8 rows, portions of 9 to 32 rows are summed up in the library's
+    # order, in which two scores of a router 1.8e-6 apart fell the other way from the 64-bit result.
     SKINNY_ROWS = 32
 
     def _skinny_ok(self, x: torch.Tensor, w: torch.Tensor) -> bool:

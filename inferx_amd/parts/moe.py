@@ -48,7 +48,12 @@ WIDE_TILES_WIDTH = 3072
 # that is a multiple of the experts' width; keeps the shared expert's weights a second time, in that layout.
 # Measured at the A2.7B shape (24 layers), with against without: decoding at batch 64 11.22 against 11.59 ms a step; a
 # portion of 256 tokens 6.58 against 7.19 ms, of 512 8.16 against 9.17, of 768 9.50 against 9.47, of 1,024 10.88
-# against 10.42; at the 57B shape (8 layers) 512 tokens 9.41 against 10.26 ms, 1,024 13.41 against 13.29.
+# against 10.42; at the 57B shape (8 layers) 512 tokens 9.41 against 10.26 ms, 1,024 13.41 against 13.29.  With the
+# grouped products' stages pipelined and their tiles cut over the dies, ms of a whole prompt: A2.7B shape (8 layers), folded
+# / beside / after: 256 tokens 2.48 / 2.75 / 2.79, 512 2.99 / 3.18 / 3.19, 768 3.33 / 3.50 / 3.60, 1,024 3.78 / 3.97 / 3.99,
+# 1,536 4.48 / 4.47 / 4.68, 2,048 5.35 / 5.11 / 5.35, 4,096 9.37 / 8.56 / 8.87; 57B shape (4 layers), folded / after: 256
+# 3.98 / 4.34, 512 4.52 / 5.15, 768 5.10 / 5.61, 1,024 5.97 / 6.60, 2,048 9.86 / 9.78: the line could now lie higher, and
+# has not been moved.
 FOLD_SHARED_BELOW_TOKENS = 768
 
 
@@ -172,7 +177,7 @@ class MoeFeedForward(FeedForward):
         # A decoding step, or few rows per expert: 16-row tiles, the weights streamed by every wavefront for itself.
         # From about three rows per expert on the LDS-staged kernel is faster (60 experts, 4 per token: 174 against
         # 173 us for both products at 48 tokens, 209 against 189 at 96, 316 against 195 at 256).  The float32 forms go by
-        # the same line.
+        # the same line (33 tokens 345 against 334, 48 358 against 349, 96 411 against 371, 256 645 against 397).
         per_expert = x.shape[0] * self.top_k / self.num_experts
         if x.shape[0] <= ctx.rt.SKINNY_ROWS or per_expert <= 3:
             return 16

@@ -14,15 +14,25 @@
 // of row l%16, i.e. four consecutive numbers of one output row.
 //
 // A wavefront owns 16 out-features x (16 * MT) rows.  Per iteration it covers
-// 128 of K with four loads: in load j lane (m, g) reads the 16 bytes at
-// k0 + 32 j + 8 g of weight row m, so the four lane groups cover 64 contiguous
-// bytes of each row and the 32 reduction slots of MFMA j; the activations are
-// read with the same mapping (in float32 a round is 64 of K, and the j-th numbers of the four groups' pieces meet in
-// one instruction).  KSPLIT = 4 (decoding: few rows, the weights are the traffic) lets
-// the four wavefronts of a workgroup take a quarter of K each and add up through
-// LDS; KSPLIT = 1 gives each wavefront its own 16 out-features.  In float32 (8 tokens, 24 of 60 experts of 1,408 and a
-// shared one of 5,632 in one launch): 117 + 60 us for both products, 5.5 TB/s, against 514 + 268 us of the plain kernel
-// for the routed ones alone; a product of 8 rows with 2,048 x 2,048 weights 6 us against 12 to 18 through the library.
+// 128 of K (in float32 64: 256 bytes of a row either way).  The matrix cores want
+// 64 contiguous bytes of sixteen rows at once, memory wants whole lines of 128:
+// so a load brings 128 contiguous bytes of eight weight rows, past the caches
+// (non-temporal: a weight is used once a step), and the wavefront turns them over
+// through 4 KB of LDS of its own, with no barrier.  The activations, which every
+// workgroup reads, come from the caches as operands: in load j lane (m, g) reads
+// the 16 bytes at k0 + 32 j + 8 g of row m (in float32 the j-th numbers of the four
+// groups' pieces meet in one instruction).  KSPLIT = 4 (decoding: few rows, the
+// weights are the traffic) lets the four wavefronts of a workgroup take a quarter
+// of K each and add up through LDS; KSPLIT = 1 gives each wavefront its own 16
+// out-features.
+//
+// What bounds it is the weights.  Against half lines straight into the operands' registers, through the caches, us (the
+// same bits; non-temporal half lines are slower than either: a line's other half is gone when it is asked for):
+// experts of 1,408 and a shared one of 5,632, rows of 2,048 numbers, both products: one row 16.3 + 10.9 (20.8 + 12.8), eight
+// rows on 24 experts 49.5 + 25.8 (59.1 + 30.2; 6.5 TB/s), 32 rows on 43 experts 90 + 46 (106 + 56); experts of 2,560 and a
+// shared one of 20,480, rows of 3,584, eight rows on 41 experts 264 + 130 (322 + 166).  The logits of a vocabulary of
+// 151,936, rows of 2,048: one 95 (111), eight 98 (134), sixteen 110 (154), 32 153 (184); of 3,584: sixteen 197 (273).  Two
+// blocks of weights a wavefront (gate|up, logits) take three wavefronts a SIMD, in whose registers nothing is spilled.
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -52,13 +62,16 @@ template <> struct MfmaPiece<float> {
   }
 };
 
-// The work of one wavefront (KSPLIT == 1) or workgroup (KSPLIT == 4): rows [row0, row_end) x out-features
-// [n0, n0 + 16) of expert e.  `red`: LDS for the partial sums of a split reduction.
-// NB: blocks of 16 out-features side by side ([n0, n0 + 16 NB)), so that the rows are read once for all of them.
+// LDS that a wavefront turns its weights over in, bytes: a round of each of its blocks of sixteen rows
+#define IX_TURN_BYTES(NACC) (4096 * (NACC))
+
+// The work of one wavefront (KSPLIT == 1) or workgroup (KSPLIT > 1): rows [row0, row_end) x out-features
+// [n0, n0 + 16) of expert e.  `lds`: IX_TURN_BYTES for each wavefront; the partial sums of a split reduction go the same
+// way.  NB: blocks of 16 out-features side by side ([n0, n0 + 16 NB)), so that the rows are read once for all of them.
 template <int MT, bool GATE_UP, int KSPLIT, typename TI, typename TO, int NB = 1>
 __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
                                              TO* __restrict__ out, const int32_t* __restrict__ rows, int e,
-                                             int row0, int row_end, int n0, int n_out, int width, float* red,
+                                             int row0, int row_end, int n0, int n_out, int width, char* lds,
                                              int act = 0, float glu_limit = 0.f, const void* bias = nullptr,
                                              int bias_dtype = 0) {
   typedef MfmaPiece<TI> Piece;
@@ -72,12 +85,23 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
   const int kend = min(width, kbegin + kper);
 
   const int64_t w_rows = GATE_UP ? 2 * static_cast<int64_t>(n_out) : n_out;
-  const TI* wp[NACC];
+  // In load j lane l reads piece 8 (j / 2) + l % 8 of row 8 (j % 2) + l / 8: whole lines of 128 bytes.  (A block's rows
+  // start at an address that is the same for all lanes; beside it 32 bits are enough.)
+  const char* wbase[NACC];
+  unsigned wrow[NB][2];
 #pragma unroll
   for (int u = 0; u < NACC; ++u) {
-    const int wrow = min(n0 + 16 * (u % NB) + m, n_out - 1);  // rows past the end are computed and not stored
-    wp[u] = w + (static_cast<int64_t>(e) * w_rows + (u / NB) * static_cast<int64_t>(n_out) + wrow) * width;
+    const int first = min(n0 + 16 * (u % NB), n_out - 1);  // (rows past the end: the last one, computed and not stored)
+    wbase[u] = reinterpret_cast<const char*>(w + (static_cast<int64_t>(e) * w_rows + (u / NB) * static_cast<int64_t>(n_out) + first) * width);
+    if (u < NB)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        wrow[u][h] = static_cast<unsigned>(min(8 * h + (lane >> 3), n_out - 1 - first)) * static_cast<unsigned>(width) * sizeof(TI);
   }
+  // Piece p of row r of a round lies at piece p ^ (r / 2 + 8 (r % 2)) of its 256 bytes: the rows that sixteen lanes read at
+  // one piece, and the pieces of two rows that they write, fall on sixteen different groups of four banks.
+  char* const turn = lds + wave * IX_TURN_BYTES(NACC);
+  auto turn_at = [&](int r, int p) { return turn + 256 * r + 16 * (p ^ ((r >> 1) | ((r & 1) << 3))); };
 
   const TI* xr[MT];
 #pragma unroll
@@ -104,13 +128,30 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
     for (int j = 0; j < 4; ++j) {
       int kk = k0 + PN * (4 * j + g);  // the four lane groups cover 64 contiguous bytes of a row per load
       kk = kk < kend ? kk : kbegin;  // (the range's first piece: it exists, kbegin + PN g need not)
+      int kw = k0 + PN * (8 * (j >> 1) + (lane & 7));
+      kw = kw < kend ? kw : kbegin;
 #pragma unroll
-      for (int u = 0; u < NACC; ++u) w_[u][j] = *reinterpret_cast<const piece_t*>(wp[u] + kk);
+      for (int u = 0; u < NACC; ++u)
+        w_[u][j] = __builtin_nontemporal_load(
+            reinterpret_cast<const piece_t*>(wbase[u] + (wrow[u % NB][j & 1] + static_cast<unsigned>(kw) * sizeof(TI))));
 #pragma unroll
       for (int t = 0; t < MT; ++t) x_[t][j] = *reinterpret_cast<const piece_t*>(xr[t] + kk);
     }
   };
-  auto multiply = [&](int k0, const piece_t (&w_)[NACC][4], const piece_t (&x_)[MT][4]) {
+  // (a wavefront's LDS operations are carried out in their order: what the last round left is read before it is written over)
+  auto turn_over = [&](piece_t (&w_)[NACC][4]) {
+#pragma unroll
+    for (int u = 0; u < NACC; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<piece_t*>(turn_at(8 * (j & 1) + (lane >> 3), 8 * (j >> 1) + (lane & 7)) + 4096 * u) = w_[u][j];
+  };
+  auto multiply = [&](int k0, const piece_t (&x_)[MT][4]) {
+    piece_t w_[NACC][4];
+#pragma unroll
+    for (int u = 0; u < NACC; ++u)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w_[u][j] = *reinterpret_cast<const piece_t*>(turn_at(m, 4 * j + g) + 4096 * u);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const bool ok = k0 + PN * (4 * j + g) < kend;
@@ -131,27 +172,32 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
     for (; left > 2; left -= 2, k0 += 2 * ROUND) {
       fetch(k0 + ROUND, fw[1], fx[1]);
       __builtin_amdgcn_sched_barrier(0);
-      multiply(k0, fw[0], fx[0]);
+      turn_over(fw[0]);
+      multiply(k0, fx[0]);
       __builtin_amdgcn_sched_barrier(0);
       fetch(k0 + 2 * ROUND, fw[0], fx[0]);
       __builtin_amdgcn_sched_barrier(0);
-      multiply(k0 + ROUND, fw[1], fx[1]);
+      turn_over(fw[1]);
+      multiply(k0 + ROUND, fx[1]);
       __builtin_amdgcn_sched_barrier(0);
     }
     if (left == 2) {
       fetch(k0 + ROUND, fw[1], fx[1]);
       __builtin_amdgcn_sched_barrier(0);
-      multiply(k0, fw[0], fx[0]);
-      multiply(k0 + ROUND, fw[1], fx[1]);
+      turn_over(fw[0]);
+      multiply(k0, fx[0]);
+      turn_over(fw[1]);
+      multiply(k0 + ROUND, fx[1]);
     } else {
-      multiply(k0, fw[0], fx[0]);
+      turn_over(fw[0]);
+      multiply(k0, fx[0]);
     }
   }
 
   if (KSPLIT > 1) {
     // the other wavefronts hand their partial sums to wavefront 0
     if (wave > 0) {
-      float* dst = red + ((wave - 1) * 64 + lane) * (MT * NACC * 4);
+      float* dst = reinterpret_cast<float*>(turn) + lane * (MT * NACC * 4);
 #pragma unroll
       for (int u = 0; u < NACC; ++u)
 #pragma unroll
@@ -163,7 +209,7 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
     if (wave > 0) return;
 #pragma unroll
     for (int s = 0; s < KSPLIT - 1; ++s) {
-      const float* src = red + (s * 64 + lane) * (MT * NACC * 4);
+      const float* src = reinterpret_cast<const float*>(lds + (s + 1) * IX_TURN_BYTES(NACC)) + lane * (MT * NACC * 4);
 #pragma unroll
       for (int u = 0; u < NACC; ++u)
 #pragma unroll
@@ -214,26 +260,26 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
 // x [rows <= 16 * MT, width] . w^T -> [rows, n_out], the products of a decoding step: 16 NB out-features a workgroup, the
 // reduction split over its KSPLIT wavefronts.
 template <int MT, bool GATE_UP, int KSPLIT, int NB, typename TI, typename TO>
-__global__ void __launch_bounds__(64 * KSPLIT, MT == 1 ? 4 : 1)
+__global__ void __launch_bounds__(64 * KSPLIT, MT > 1 ? 1 : NB * (GATE_UP ? 2 : 1) > 1 ? 3 : 4)
 linear_skinny_kernel(const TI* x, const TI* w, TO* __restrict__ out, const void* bias, int bias_dtype, int rows, int n_out,
                      int width, float glu_limit) {
-  __shared__ float red[(KSPLIT - 1) * 64 * MT * NB * (GATE_UP ? 2 : 1) * 4];
-  grouped_body<MT, GATE_UP, KSPLIT, TI, TO, NB>(x, w, out, nullptr, 0, 0, rows, blockIdx.x * 16 * NB, n_out, width, red, 0,
+  __shared__ __attribute__((aligned(16))) char lds[KSPLIT * IX_TURN_BYTES(NB * (GATE_UP ? 2 : 1))];
+  grouped_body<MT, GATE_UP, KSPLIT, TI, TO, NB>(x, w, out, nullptr, 0, 0, rows, blockIdx.x * 16 * NB, n_out, width, lds, 0,
                                                 glu_limit, bias, bias_dtype);
 }
 
 template <int MT, bool GATE_UP, int KSPLIT, typename TI>
-__global__ void __launch_bounds__(256, MT == 1 ? 4 : 1)
+__global__ void __launch_bounds__(256, MT > 1 ? 1 : GATE_UP ? 3 : 4)
 moe_grouped_mfma_kernel(const TI* a, const TI* w, TI* __restrict__ out,
                         const int32_t* __restrict__ offsets, const int32_t* __restrict__ rows,
                         const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_row0,
                         const int32_t* __restrict__ tile_info, int n_out, int width, int act, float glu_limit) {
-  __shared__ float red[KSPLIT > 1 ? 3 * 64 * MT * (GATE_UP ? 2 : 1) * 4 : 1];
+  __shared__ __attribute__((aligned(16))) char lds[4 * IX_TURN_BYTES(GATE_UP ? 2 : 1)];
   if (static_cast<int>(blockIdx.y) >= tile_info[0]) return;
   const int e = tile_expert[blockIdx.y];
   const int n0 = (KSPLIT > 1 ? blockIdx.x : blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
   if (n0 >= n_out) return;  // whole wavefront (KSPLIT == 1) or whole workgroup
-  grouped_body<MT, GATE_UP, KSPLIT, TI, TI>(a, w, out, rows, e, tile_row0[blockIdx.y], offsets[e + 1], n0, n_out, width, red,
+  grouped_body<MT, GATE_UP, KSPLIT, TI, TI>(a, w, out, rows, e, tile_row0[blockIdx.y], offsets[e + 1], n0, n_out, width, lds,
                                     act, glu_limit);
 }
 
@@ -242,14 +288,14 @@ moe_grouped_mfma_kernel(const TI* a, const TI* w, TI* __restrict__ out,
 // tokens with weights and sizes of its own (first, because its reduction may be the longer one and the last
 // workgroups to start set the kernel's end); the rest serve the routed experts' row tiles.
 template <int MT, bool GATE_UP, int NB, typename TI>
-__global__ void __launch_bounds__(256, MT == 1 ? 4 : 1)
+__global__ void __launch_bounds__(256, MT > 1 ? 1 : NB * (GATE_UP ? 2 : 1) > 1 ? 3 : 4)
 moe_grouped_dual_kernel(const TI* a, const TI* w, TI* __restrict__ out,
                         const int32_t* __restrict__ offsets, const int32_t* __restrict__ rows,
                         const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_row0,
                         const int32_t* __restrict__ tile_info, int max_tiles, int n_out, int width,
                         const TI* a_s, const TI* w_s, TI* __restrict__ out_s,
                         int shared_rows, int n_out_s, int width_s, float glu_limit, float glu_limit_s) {
-  __shared__ float red[3 * 64 * MT * NB * (GATE_UP ? 2 : 1) * 4];
+  __shared__ __attribute__((aligned(16))) char lds[4 * IX_TURN_BYTES(NB * (GATE_UP ? 2 : 1))];
   const int n16_s = (n_out_s + 16 * NB - 1) / (16 * NB);  // column blocks of 16 NB out-features
   const int shared_blocks = n16_s * ((shared_rows + 16 * MT - 1) / (16 * MT));
   int idx = blockIdx.x;
@@ -257,7 +303,7 @@ moe_grouped_dual_kernel(const TI* a, const TI* w, TI* __restrict__ out,
     const int tile = idx / n16_s;
     grouped_body<MT, GATE_UP, 4, TI, TI, NB>(a_s, w_s, out_s, nullptr, 0, tile * 16 * MT, shared_rows,
                                              (idx - tile * n16_s) * 16 * NB,
-                                 n_out_s, width_s, red, 0, glu_limit_s);
+                                 n_out_s, width_s, lds, 0, glu_limit_s);
   } else {
     idx -= shared_blocks;
     const int n16_e = (n_out + 16 * NB - 1) / (16 * NB);
@@ -265,7 +311,7 @@ moe_grouped_dual_kernel(const TI* a, const TI* w, TI* __restrict__ out,
     if (tile >= tile_info[0]) return;
     const int e = tile_expert[tile];
     grouped_body<MT, GATE_UP, 4, TI, TI, NB>(a, w, out, rows, e, tile_row0[tile], offsets[e + 1],
-                                             (idx - tile * n16_e) * 16 * NB, n_out, width, red, 0, glu_limit);
+                                             (idx - tile * n16_e) * 16 * NB, n_out, width, lds, 0, glu_limit);
   }
 }
 
@@ -361,8 +407,8 @@ extern "C" int ix_moe_grouped_dual(const void* a, const void* w, void* out, int 
 // way.  A product of the run's type is a workgroup of 16 out-features; with no more of them than the chip has compute
 // units eight wavefronts split its reduction instead of four.  The float32 result (the logits) has so many out-features
 // that 32 a workgroup are better: the rows, which every workgroup reads, weigh less beside the weights.
-// Eight rows: 2,048 features of 2,048 numbers 5.7 us (6.3 with four wavefronts, by way of a grouping of one expert, whose
-// tables a workgroup reads before its weights); a gated unit with biases saves the launch behind it, 6.2 us.
+// Eight rows: 2,048 features of 2,048 numbers 4.9 us, of 5,632 9.6 (11.7 before whole lines were read), 11,264 features of
+// 2,048 10.9 (14.6); a gated unit with biases saves the launch behind it, 6.2 us.
 extern "C" int ix_linear_skinny(const void* x, const void* w, int dtype, void* out, int out_f32, const void* bias,
                                 int bias_dtype, int rows, int64_t n_out, int64_t width, int gate_up, float glu_limit,
                                 hipStream_t stream) {

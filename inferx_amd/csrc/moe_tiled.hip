@@ -30,6 +30,13 @@
 // rows and eight of 682 587 + 348 (684 + 387).  (Weights straight into registers as operands, past LDS: sixteen rows of 64
 // bytes a load are half as fast for one compute unit as eight of 128.  One wavefront a SIMD with 512 registers: no better.)
 // LDS rows are 128 bytes with their 16-byte pieces permuted, so that operand reads and writes fall on distinct banks.
+//
+// An expert of up to 64 rows has one tile, and its weights are read once: past the caches (non-temporal, whole lines).  With
+// more rows that gains nothing (64 experts of 2,560 with 64 rows on average: 404 us up to 64 rows, 423 up to 96).  Results go through LDS,
+// so that a store is 16 bytes a lane of whole lines and not 8 of sixteen rows.  Both products, us, against every load through
+// the caches and results straight from the registers: 60 experts of 1,408, rows of 2,048, beside four of every row: 64 rows
+// in all 116 + 60 (130 + 68), 340 rows 119 + 67 (134 + 73); 2,048 rows unevenly over the 60 163 + 86 (181 + 98); 64 experts of 2,560, rows of
+// 3,584, wide, beside eight of every row: 682 rows 678 + 359 (687 + 372).
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -50,7 +57,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ int tl_at(int row, int piece) { return row * TL_STRIDE + ((piece ^ ((row >> 1) & 7)) << 3); }
 
 // One row tile x 64 NWW weight rows.  NP: pairs of sixteens of activation rows the tile holds, one of each a wavefront.
-template <bool GATE_UP, int NP, int NWW>
+template <bool GATE_UP, int NP, int NWW, bool ONCE>
 __device__ __forceinline__ void
 tiled_body(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restrict__ rows, int n_out, int width,
            int e, int row0, int row_end, int col_block, __bf16* ws, __bf16* xs, int act, float glu_limit) {
@@ -101,7 +108,10 @@ tiled_body(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restr
   auto fetch = [&](int s, int set) {
     const unsigned at = min(place(s) + 8 * (tid & 7), width - 8);
 #pragma unroll
-    for (int i = 0; i < NPW; ++i) wreg[set][i] = *reinterpret_cast<const bf16x8*>(w_expert + (wsrc[i] + at));
+    for (int i = 0; i < NPW; ++i) {
+      const bf16x8* from = reinterpret_cast<const bf16x8*>(w_expert + (wsrc[i] + at));
+      wreg[set][i] = ONCE ? __builtin_nontemporal_load(from) : *from;
+    }
 #pragma unroll
     for (int i = 0; i < NPX; ++i) xreg[set][i] = *reinterpret_cast<const bf16x8*>(a + (xsrc[i] + at));
   };
@@ -246,6 +256,38 @@ tiled_body(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restr
   }
 
   // lane holds weight rows (block) + 4 g + i of activation row row0 + 16 (2 t + xi) + m
+  auto result = [&](int t, int j, float (&v)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[i] = acc[j][t][i];
+      if (GATE_UP) v[i] = ix_glu<true>(v[i], acc[GATE_UP ? j + 2 : j][t][i], glu_limit);
+      else if (act) v[i] = v[i] > 0.f ? v[i] * v[i] : 0.f;  // the square of relu
+    }
+  };
+  if (((n_out & 7) | static_cast<int>(reinterpret_cast<uintptr_t>(out) & 15)) == 0) {
+    // The tile goes through LDS, so that a store is 16 bytes a lane and whole lines.
+    constexpr int OUT_STRIDE = COLS + 8;
+    static_assert(TL_ROWS(NWW) * OUT_STRIDE <= 2 * (TL_XTILE(NWW) + TL_WTILE(NWW)), "the result's tile fits the stages' LDS");
+    __bf16* const tile = ws;
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < NP; ++t)
+#pragma unroll
+      for (int j = 0; j < (GATE_UP ? 2 : 4); ++j) {
+        float v[4];
+        result(t, j, v);
+        *reinterpret_cast<bf16x4*>(tile + (16 * (2 * t + xi) + m) * OUT_STRIDE + (GATE_UP ? 32 : 64) * wi + 16 * j + 4 * g) =
+            bf16x4{(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
+      }
+    __syncthreads();
+    constexpr int LANES = COLS / 8, AT_ONCE = TL_THREADS(NWW) / LANES;  // lanes of a row; rows that the workgroup stores at once
+    const int c = 8 * (tid % LANES);
+    if (n0 + c < n_out)
+      for (int r = tid / LANES; r < min(32 * NP, row_end - row0); r += AT_ONCE)
+        *reinterpret_cast<bf16x8*>(out + static_cast<int64_t>(row0 + r) * n_out + n0 + c) =
+            *reinterpret_cast<const bf16x8*>(tile + r * OUT_STRIDE + c);
+    return;
+  }
   const bool vec = (n_out & 3) == 0;
 #pragma unroll
   for (int t = 0; t < NP; ++t) {
@@ -255,12 +297,7 @@ tiled_body(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restr
     for (int j = 0; j < (GATE_UP ? 2 : 4); ++j) {
       const int nb = n0 + (GATE_UP ? 32 : 64) * wi + 16 * j + 4 * g;
       float v[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[i] = acc[j][t][i];
-        if (GATE_UP) v[i] = ix_glu<true>(v[i], acc[GATE_UP ? j + 2 : j][t][i], glu_limit);
-        else if (act) v[i] = v[i] > 0.f ? v[i] * v[i] : 0.f;  // the square of relu
-      }
+      result(t, j, v);
       __bf16* dst = out + static_cast<int64_t>(r) * n_out + nb;
       if (nb + 4 <= n_out && vec) {
         bf16x4 o = {(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
@@ -281,8 +318,8 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
                          const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_row0,
                          const int32_t* __restrict__ tile_info, int n_out, int width, int n_col_blocks,
                          int act, float glu_limit, int last_tiles, int last_each) {
-  __shared__ __attribute__((aligned(16))) __bf16 ws[2 * TL_WTILE(NWW)];
-  __shared__ __attribute__((aligned(16))) __bf16 xs[2 * TL_XTILE(NWW)];
+  __shared__ __attribute__((aligned(16))) __bf16 ws[2 * (TL_WTILE(NWW) + TL_XTILE(NWW))];
+  __bf16* const xs = ws + 2 * TL_WTILE(NWW);
   // Workgroups go to the chip's eight dies in turn, by their number, and each die has its own L2 and its own share of the
   // memory's bandwidth.  The (row tile, column block) pairs, tile by tile, are cut into eight equal runs, one a die, so that
   // the column blocks of a tile, which read the same activations, share an L2 and no die has more of them than another.
@@ -322,16 +359,20 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
   const int row_end = offsets[e + 1];
   const int held = min(TL_ROWS(NWW), row_end - row0);
   if (held <= 0) return;
-#define BODY(NP) tiled_body<GATE_UP, NP, NWW>(a, w, out, rows, n_out, width, e, row0, row_end, col_block, ws, xs, act, glu_limit)
+  const bool once = row0 == offsets[e] && held == row_end - row0 && held <= 64;  // an expert's only tile, few rows
+#define CALL(NP, ONCE) \
+  tiled_body<GATE_UP, NP, NWW, ONCE>(a, w, out, rows, n_out, width, e, row0, row_end, col_block, ws, xs, act, glu_limit)
+#define BODY(NP) CALL(NP, false)
   switch ((held + 31) >> 5) {  // pairs of sixteens of rows this tile holds
-    case 1: BODY(1); break;
-    case 2: BODY(2); break;
+    case 1: if (once) CALL(1, true); else BODY(1); break;
+    case 2: if (once) CALL(2, true); else BODY(2); break;
     case 3: BODY(3); break;
     case 4: BODY(4); break;
     case 5: BODY(5); break;
     default: BODY((NWW == 4 ? 6 : 5)); break;  // (six in the wide form only)
   }
 #undef BODY
+#undef CALL
 }
 
 // The row-tile map must have been made for tiles of 160 rows, for the wide form of 192.  `wide`: see below.

@@ -274,6 +274,29 @@ def test_grouped_tiled(T, H, E, k, mi, wide):
 
 
 @pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("mi", [8, 72, 76, 264])
+def test_grouped_tiled_rows_read_once_and_results_at_any_place(mi, wide):
+    """Experts of 64 and 65 rows (the most whose weights go past the caches, and one more), of one row, none, a whole tile and
+    one more; results on and off 16-byte boundaries, rows of them whole 16-byte pieces or not: the same bits."""
+    from inferx_amd import ops
+    R, H = ops.moe_tiled_rows(wide), 136
+    counts = [64, 65, 1, 0, R, R + 1]
+    topk_e = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts)).to(torch.int32)[:, None].to(DEV)
+    offsets, rows, dest, tile_map = dispatch(topk_e, len(counts), R)
+    T = sum(counts)
+    x = rnd(T, H, dtype=torch.bfloat16)
+    w = rnd(len(counts), 2 * mi, H, seed=2, dtype=torch.bfloat16, scale=H ** -0.5)
+    got = []
+    for off in (0, 4):  # (the buffer's numbers before and behind the result must stay)
+        buf = torch.full((T * mi + 16,), 7.0, dtype=torch.bfloat16, device=DEV)
+        ops.moe_grouped_tiled(x, w, buf[off:off + T * mi].view(T, mi), offsets, rows, tile_map, True, wide)
+        assert (buf[:off] == 7).all() and (buf[off + T * mi:] == 7).all()
+        got.append(buf[off:off + T * mi].view(T, mi).clone())
+    assert torch.equal(got[0].view(torch.int16), got[1].view(torch.int16))
+    assert rel_err(got[0], grouped_reference(x, w, offsets.cpu(), rows.cpu(), True)) < 1.5e-2
+
+
+@pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("last", [1, 3, 7, 8, 1000])
 def test_grouped_tiled_order_of_the_last_tiles(last, wide):
     """Working the last tiles of the map spread among the others changes no bit, whatever their number."""

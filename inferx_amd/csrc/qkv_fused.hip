@@ -7,7 +7,7 @@
 // with them; its four wavefronts split the reduction and add up through LDS in a fixed order.  The
 // product is formed transposed (A = weight rows, B = token rows), so lane l ends up with features
 // 4*(l/16)+i of token l%16: four consecutive numbers of one output row.  NT: sixteens of tokens (1 or 2); the
-// weights are read once for both.
+// weights are read once for both, as whole lines past the caches that a wavefront turns over in LDS (moe_mfma.hip has why).
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -21,17 +21,23 @@ qkv_rope_skinny_kernel(const __bf16* x, const __bf16* w, const void* __restrict_
                        __bf16* __restrict__ q_out, __bf16* __restrict__ k_cache, __bf16* __restrict__ v_cache,
                        int tokens, int width, int heads, int kv_heads, int head_dim, int page_size,
                        int64_t total_slots) {
-  __shared__ float red[3 * 64 * 8 * NT];
+  __shared__ __attribute__((aligned(16))) char lds[4 * 8192];  // 8 KB a wavefront: a step's weights; the partial sums
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
   const int half = head_dim / 2, per_head = half / 16;
   const int head = blockIdx.x / per_head, jt = blockIdx.x - head * per_head;
-  const int row_lo = head * head_dim + 16 * jt + m;  // weight row (= output feature) of the low half
 
   const int kper = (((width + 3) / 4) + 127) & ~127;
   const int kbegin = wave * kper, kend = min(width, kbegin + kper);
-  const __bf16* wl = w + static_cast<int64_t>(row_lo) * width;
-  const __bf16* wh = wl + static_cast<int64_t>(half) * width;
+  // the sixteen weight rows (= output features) of the low half; load j brings 128 bytes of eight of them, lane l piece
+  // 8 (j / 2) + l % 8 of row 8 (j % 2) + l / 8
+  const char* wl = reinterpret_cast<const char*>(w + static_cast<int64_t>(head * head_dim + 16 * jt) * width);
+  const char* wh = wl + static_cast<int64_t>(half) * width * 2;
+  unsigned wrow[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) wrow[h] = static_cast<unsigned>(8 * h + (lane >> 3)) * static_cast<unsigned>(width) * 2u;
+  char* const turn = lds + wave * 8192;
+  auto turn_at = [&](int r, int p) { return turn + 256 * r + 16 * (p ^ ((r >> 1) | ((r & 1) << 3))); };
   const __bf16* xr[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) xr[t] = x + static_cast<int64_t>(min(16 * t + m, tokens - 1)) * width;
@@ -52,21 +58,38 @@ qkv_rope_skinny_kernel(const __bf16* x, const __bf16* w, const void* __restrict_
     for (int j = 0; j < 4; ++j) {
       int kk = k0 + 32 * j + 8 * g;  // the four lane groups cover 64 contiguous bytes of a row
       kk = kk < kend ? kk : kbegin;  // (past the end: the range's first piece, which exists and was read before)
-      st.fl[j] = *reinterpret_cast<const bf16x8*>(wl + kk);
-      st.fh[j] = *reinterpret_cast<const bf16x8*>(wh + kk);
+      int kw = k0 + 64 * (j >> 1) + 8 * (lane & 7);
+      kw = kw < kend ? kw : kbegin;
+      const unsigned at = wrow[j & 1] + 2u * static_cast<unsigned>(kw);
+      st.fl[j] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(wl + at));
+      st.fh[j] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(wh + at));
 #pragma unroll
       for (int t = 0; t < NT; ++t) st.fx[t][j] = *reinterpret_cast<const bf16x8*>(xr[t] + kk);
     }
   };
   auto multiply = [&](int k0, const Step& st) {
+    // turned over in LDS (a wavefront's LDS operations are carried out in their order)
+    bf16x8 fl[4], fh[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      char* to = turn_at(8 * (j & 1) + (lane >> 3), 8 * (j >> 1) + (lane & 7));
+      *reinterpret_cast<bf16x8*>(to) = st.fl[j];
+      *reinterpret_cast<bf16x8*>(to + 4096) = st.fh[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const char* from = turn_at(m, 4 * j + g);
+      fl[j] = *reinterpret_cast<const bf16x8*>(from);
+      fh[j] = *reinterpret_cast<const bf16x8*>(from + 4096);
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const bool ok = k0 + 32 * j + 8 * g < kend;
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const bf16x8 xv = ok ? st.fx[t][j] : zero;
-        acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(st.fl[j], xv, acc[t][0], 0, 0, 0);
-        acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(st.fh[j], xv, acc[t][1], 0, 0, 0);
+        acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fl[j], xv, acc[t][0], 0, 0, 0);
+        acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fh[j], xv, acc[t][1], 0, 0, 0);
       }
     }
   };
@@ -129,7 +152,7 @@ qkv_rope_skinny_kernel(const __bf16* x, const __bf16* w, const void* __restrict_
     }
   }
   if (wave > 0) {
-    float* dst = red + ((wave - 1) * 64 + lane) * 8 * NT;
+    float* dst = reinterpret_cast<float*>(turn) + lane * 8 * NT;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -141,7 +164,7 @@ qkv_rope_skinny_kernel(const __bf16* x, const __bf16* w, const void* __restrict_
   if (wave > 0) return;
 #pragma unroll
   for (int s = 0; s < 3; ++s) {
-    const float* src = red + (s * 64 + lane) * 8 * NT;
+    const float* src = reinterpret_cast<const float*>(lds + (s + 1) * 8192) + lane * 8 * NT;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll

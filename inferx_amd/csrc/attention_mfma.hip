@@ -6,7 +6,8 @@
 //
 // Unit of work = one wavefront: a tile of up to 16 consecutive queries of one
 // request and one query head, over one slice of that tile's keys (split-KV).
-// There is no LDS and no barrier: a workgroup is four independent wavefronts.
+// There is no barrier: a workgroup is four independent wavefronts (LDS only as TURN
+// below has it).
 //
 // The transposed products are formed so that no operand has to be shuffled:
 //   S^T[key][query]  = K[key][:] . Q[query][:]     (A = K rows, B = Q rows)
@@ -38,15 +39,21 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // head_dim = 16 * NB; a tile holds up to 16 * QT queries; PF: request the next iteration's keys and values
 // before this iteration's are multiplied (pays when few wavefronts are resident: decoding)
+// TURN (decoding with heads of 128 whose keys and values only one wavefront reads): keys come as whole lines past the
+// caches, two rounds ahead, through LDS.  Bound by memory: 64 contexts of 2,048 of 16 heads 165 us = 6.5 TB/s (190 as
+// half lines straight into the operands' registers, one round ahead, each round's pages a load before it).  With the
+// slices' rules (decode_slices in parts/attention.py, min_slice and the order of units below): 64 of 200 to 2,048
+// 78 us (123), 32 of 16 to 700 19.6 (28.2), 32 of 1,500 68 (78), eight of 2,048 27.4 (32.2), one of 517 7.4 (9.2; with
+// the merging, 4.5 us of each).  Few and short contexts are bound by what a wavefront waits for before its first keys.
 // MORE false: without capped scores and a gate (for the plain decoding steps, where a test a round is measurable)
-template <int NB, int QT, bool PF, bool GQ = false, bool MORE = true>
+template <int NB, int QT, bool PF, bool GQ = false, bool MORE = true, bool TURN = false>
 __global__ void __launch_bounds__(256)
 attn_mfma_kernel(const __bf16* __restrict__ q, const __bf16* __restrict__ k_cache, const __bf16* __restrict__ v_cache,
                  const int32_t* __restrict__ block_table, const int32_t* __restrict__ tile_seq,
                  const int32_t* __restrict__ tile_q0, const int32_t* __restrict__ tile_rows,
                  const int32_t* __restrict__ positions, __bf16* __restrict__ out, float* __restrict__ part_o,
                  float* __restrict__ part_ml, int n_tiles, int n_splits, int heads, int kv_heads, int page_size,
-                 int max_blocks, float scale_log2, int span, int page_shift, const float* __restrict__ sink,
+                 int max_blocks, float scale_log2, int span, int page_shift, int min_slice, const float* __restrict__ sink,
                  const float2* __restrict__ turn_back, float cap_slope, float cap2, const __bf16* __restrict__ gate,
                  int64_t gate_stride) {
   // sink (one float per head, or null): exp(sink) joins the softmax's denominator, with no key and no value, not
@@ -59,14 +66,27 @@ attn_mfma_kernel(const __bf16* __restrict__ q, const __bf16* __restrict__ k_cach
   const int lane = threadIdx.x & 63;
   // (wavefronts of a workgroup share nothing: a workgroup is four of them, or fewer where a step has so few that
   // whole compute units would stay idle otherwise)
-  const int unit = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (unit >= n_tiles * n_splits) return;
-  const int tile = unit / n_splits, split = unit - tile * n_splits;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int unit = blockIdx.x * (blockDim.x >> 6) + wave;
   const int group = heads / kv_heads;
-  // GQ: blockIdx.y is the key/value head, column n of the tile is query head kvh * group + n of token tq0
-  const int kvh = GQ ? blockIdx.y : blockIdx.y / group;
+  int tile, split, hy;  // hy: GQ the key/value head, whose query head kvh * group + n is column n of the tile; else the head
+  if constexpr (PF) {
+    // Decoding: the heads of a slice side by side, so that the wavefronts of a workgroup take equally long, and the
+    // workgroups of a long context go to all dies: with a request's slices side by side (and each head by itself) the
+    // longest of 64 requests that are sorted by length fell to one die.  Slices that only long contexts have come last.
+    const int per_slice = GQ ? kv_heads : heads;
+    const int slice = unit / per_slice;
+    if (slice >= n_tiles * n_splits) return;
+    hy = unit - slice * per_slice;
+    split = slice / n_tiles, tile = slice - split * n_tiles;
+  } else {
+    if (unit >= n_tiles * n_splits) return;
+    hy = blockIdx.y;
+    tile = unit / n_splits, split = unit - tile * n_splits;
+  }
+  const int kvh = GQ ? hy : hy / group;
   const int n = lane & 15, g = lane >> 4;
-  const int head = GQ ? kvh * group + min(n, group - 1) : blockIdx.y;
+  const int head = GQ ? kvh * group + min(n, group - 1) : hy;
 
   const int tq0 = tile_q0[tile];
   const int rows = GQ ? group : tile_rows[tile];  // columns of the tile that hold a query
@@ -77,9 +97,19 @@ attn_mfma_kernel(const __bf16* __restrict__ q, const __bf16* __restrict__ k_cach
   const int lo = ix_first_key(pos0, span);
   const int hi = pos0 + (GQ ? 1 : rows);
   const int lo_al = lo & ~(ATTN_KEYS_PER_ITER - 1);
-  const int per = (((hi - lo_al + n_splits - 1) / n_splits) + ATTN_KEYS_PER_ITER - 1) & ~(ATTN_KEYS_PER_ITER - 1);
+  const int per = max((((hi - lo_al + n_splits - 1) / n_splits) + ATTN_KEYS_PER_ITER - 1) & ~(ATTN_KEYS_PER_ITER - 1),
+                      min_slice);
   const int ks = lo_al + split * per;
   const int ke = min(hi, ks + per);
+  if (ks >= ke && split > 0) {  // no keys are left for this slice: the merging kernel reads no more of it than that
+    if (lane < (GQ ? group : tile_rows[tile])) {
+      const int64_t token = tq0 + (GQ ? 0 : lane);
+      const int64_t p = (token * heads + (GQ ? kvh * group + lane : hy)) * n_splits + split;
+      part_ml[2 * p] = -INFINITY;
+      part_ml[2 * p + 1] = 0.f;
+    }
+    return;
+  }
 
   // Q as B operand: lane (n, g) holds Q[query 16 t + n][32 c + 8 g .. +8]
   bf16x8 qf[QT][NC];
@@ -154,47 +184,8 @@ attn_mfma_kernel(const __bf16* __restrict__ q, const __bf16* __restrict__ k_cach
       vf[b] = *reinterpret_cast<const bf16x8*>(vr + static_cast<int64_t>(16 * b + n) * page_size);
   };
 
-  bf16x8 kf_next[PF ? 2 : 1][PF ? NC : 1], vf_next[PF ? NB : 1];
-  int pg[3], pg_next[3];
-  if (ks < ke) {
-    ask_pages(ks, pg);
-    if constexpr (PF) {
-      ask_pages(ks + ATTN_KEYS_PER_ITER, pg_next);
-      load_kv(ks, pg, kf_next, vf_next);
-    }
-  }
-  for (int kb = ks; kb < ke; kb += ATTN_KEYS_PER_ITER) {
-    bf16x8 kf[2][NC], vf[NB];
-    if constexpr (PF) {
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int c = 0; c < NC; ++c) kf[b][c] = kf_next[b][c];
-#pragma unroll
-      for (int b = 0; b < NB; ++b) vf[b] = vf_next[b];
-      if (kb + ATTN_KEYS_PER_ITER < ke) {
-        load_kv(kb + ATTN_KEYS_PER_ITER, pg_next, kf_next, vf_next);
-        ask_pages(kb + 2 * ATTN_KEYS_PER_ITER, pg_next);
-      }
-    } else {
-      ask_pages(kb + ATTN_KEYS_PER_ITER, pg_next);
-      load_kv(kb, pg, kf, vf);
-#pragma unroll
-      for (int i = 0; i < 3; ++i) pg[i] = pg_next[i];
-    }
-    // Values of keys that no query of the tile may read (past the tile's last key in the same page, or on a page
-    // that the window has passed, read from wherever the table's filler points) are made zero: their probability
-    // is zero, but zero times whatever an earlier request left there need not be.  Only rounds at the edges.
-    if (kb + ATTN_KEYS_PER_ITER > hi || kb < lo) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int key = (min(kb + 8 * g, hi - 1) & ~7) + j;
-        if (key >= hi || key < lo) {
-#pragma unroll
-          for (int b = 0; b < NB; ++b) vf[b][j] = (__bf16)0.f;
-        }
-      }
-    }
+  // the products, the softmax and the values of the 32 keys from kb on
+  auto multiply = [&](int kb, const bf16x8 (&kf)[2][NC], const bf16x8 (&vf)[NB]) {
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
       if (QT > 1 && (16 * t >= rows || kb > pos0 + 16 * t + 15)) continue;  // no query of this block reads these keys
@@ -270,6 +261,143 @@ attn_mfma_kernel(const __bf16* __restrict__ q, const __bf16* __restrict__ k_cach
 #pragma unroll
       for (int b = 0; b < NB; ++b) o[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[b], pf, o[t][b], 0, 0, 0);
     }
+  };
+
+  if constexpr (TURN) {
+    // Whole lines, past the caches (every key and value is read once a step), two rounds of 32 keys on their way: a
+    // load brings 1 KB of a page's keys, which the wavefront turns into the matrix cores' operands through 8 KB of LDS
+    // of its own, with no barrier (its LDS operations are carried out in their order).  The pages of the slice's next
+    // 64 sixteens of keys are in one register, so no load waits for a look at the table.  Every load is unconditional
+    // and the loop one straight line: rounds past the end ask for one address only.
+    constexpr int ROW = 2 * NB;  // 16-byte pieces of a key
+    extern __shared__ __attribute__((aligned(16))) char turn_lds[];
+    char* const turn = turn_lds + wave * (32 * 32 * NB);
+    // Piece p of key r of a round lies at piece p ^ (r % 4 + 4 ((r / 8) % 4)): the sixteen keys that are read at one
+    // piece, and the sixteen pieces of a key that are written, fall on different groups of four banks.
+    auto turn_at = [&](int r, int p) { return turn + 32 * NB * r + 16 * (p ^ ((r & 3) | (((r >> 3) & 3) << 2))); };
+    int pages = 0, pages_from = 0;  // lane i: the page of keys pages_from + 16 i ..
+    const int64_t page_stride = static_cast<int64_t>(kv_heads) * page_size * D;
+    const __bf16* const k_head = k_cache + static_cast<int64_t>(kvh) * page_size * D;
+    const __bf16* const v_head = v_cache + static_cast<int64_t>(kvh) * page_size * D;
+    auto look_up = [&](int kb) {
+      pages_from = kb;
+      pages = max(table[page_of(min(kb + 16 * lane, hi - 1))], 0);  // (a page the window has passed: masked)
+    };
+    typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
+    auto fetch = [&](int kb, bf16x8 (&kt)[NB], bf16x8 (&vt)[NB]) {
+      const bool there = kb < ke;
+      kb = min(kb, ks + ((ke - 1 - ks) & ~31));
+      int page[2], off[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int key = min(kb + 16 * b, hi - 1) & ~15;  // (keys past the end: an earlier sixteen once more, masked)
+        page[b] = __builtin_amdgcn_readlane(pages, (min(kb + 16 * b, hi - 1) - pages_from) >> 4);
+        off[b] = key - page_of(key) * page_size;
+      }
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const int b = i / (NB / 2);
+        const __bf16* from = k_head + page[b] * page_stride + off[b] * D;
+        const unsigned at = there ? 8 * (64 * (i - b * (NB / 2)) + lane) : 0;
+        kt[i] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(from + at));
+      }
+      // lane (dd = n, g): values 16 i + dd of eight keys
+      const int64_t vbase = (g >> 1 ? page[1] : page[0]) * page_stride;
+      const int voff = g >> 1 ? off[1] : off[0];
+      const __bf16* vfrom = v_head + vbase + voff + 8 * (g & 1);
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const unsigned at = there ? (16 * i + n) * page_size : 0;
+        vt[i] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(vfrom + at));
+      }
+    };
+    auto use = [&](int kb, const bf16x8 (&kt)[NB], bf16x8 (&vt)[NB]) {
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        const int id = 64 * i + lane;
+        *reinterpret_cast<bf16x8*>(turn_at(id / ROW, id % ROW)) = kt[i];
+      }
+      bf16x8 kf[2][NC];
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+          kf[b][c] = *reinterpret_cast<const bf16x8*>(turn_at(8 * (n >> 2) + 4 * b + (n & 3), 4 * c + g));
+      if (kb + ATTN_KEYS_PER_ITER > hi || kb < lo) {  // values that no query may read: zero, as below
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int key = kb + 8 * g + j;
+          if (key >= hi || key < lo) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) vt[b][j] = (__bf16)0.f;
+          }
+        }
+      }
+      multiply(kb, kf, vt);
+    };
+    bf16x8 kt[2][NB], vt[2][NB];
+    int kb = ks;
+    if (kb < ke) {
+      look_up(kb);
+      fetch(kb, kt[0], vt[0]);
+    }
+    while (kb < ke) {
+      fetch(kb + 32, kt[1], vt[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      use(kb, kt[0], vt[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (kb + 32 >= ke) break;
+      if (kb + 64 < ke && kb + 64 - pages_from >= 1024) look_up(kb + 64);
+      fetch(kb + 64, kt[0], vt[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      use(kb + 32, kt[1], vt[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      kb += 64;
+    }
+  } else {
+  bf16x8 kf_next[PF ? 2 : 1][PF ? NC : 1], vf_next[PF ? NB : 1];
+  int pg[3], pg_next[3];
+  if (ks < ke) {
+    ask_pages(ks, pg);
+    if constexpr (PF) {
+      ask_pages(ks + ATTN_KEYS_PER_ITER, pg_next);
+      load_kv(ks, pg, kf_next, vf_next);
+    }
+  }
+  for (int kb = ks; kb < ke; kb += ATTN_KEYS_PER_ITER) {
+    bf16x8 kf[2][NC], vf[NB];
+    if constexpr (PF) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) kf[b][c] = kf_next[b][c];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) vf[b] = vf_next[b];
+      if (kb + ATTN_KEYS_PER_ITER < ke) {
+        load_kv(kb + ATTN_KEYS_PER_ITER, pg_next, kf_next, vf_next);
+        ask_pages(kb + 2 * ATTN_KEYS_PER_ITER, pg_next);
+      }
+    } else {
+      ask_pages(kb + ATTN_KEYS_PER_ITER, pg_next);
+      load_kv(kb, pg, kf, vf);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) pg[i] = pg_next[i];
+    }
+    // Values of keys that no query of the tile may read (past the tile's last key in the same page, or on a page
+    // that the window has passed, read from wherever the table's filler points) are made zero: their probability
+    // is zero, but zero times whatever an earlier request left there need not be.  Only rounds at the edges.
+    if (kb + ATTN_KEYS_PER_ITER > hi || kb < lo) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int key = (min(kb + 8 * g, hi - 1) & ~7) + j;
+        if (key >= hi || key < lo) {
+#pragma unroll
+          for (int b = 0; b < NB; ++b) vf[b][j] = (__bf16)0.f;
+        }
+      }
+    }
+    multiply(kb, kf, vf);
+  }
   }
 
 #pragma unroll
@@ -332,6 +460,7 @@ attn_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ 
                     int64_t head_gate_stride) {
   __shared__ float wgt[256];
   __shared__ float inv_l;
+  __shared__ int used;  // slices past the last one with keys: nothing was written of them but that
   const int64_t th = blockIdx.x;  // token * heads + head
   const float* ml = part_ml + th * n_splits * 2;
   if (threadIdx.x < 64) {
@@ -339,17 +468,22 @@ attn_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ 
     for (int s = threadIdx.x; s < n_splits; s += 64) mloc = fmaxf(mloc, ml[2 * s]);
     const float M = ix_wave_max(mloc);
     float lloc = 0.f;
+    int last = -1;
     for (int s = threadIdx.x; s < n_splits; s += 64) {
       const float m_s = ml[2 * s];
       const float w = (m_s == -INFINITY) ? 0.f : exp2f(m_s - M);
+      if (m_s != -INFINITY) last = s;
       wgt[s] = w;
       lloc += w * ml[2 * s + 1];
     }
     const float L = ix_wave_sum(lloc);
+    const int n_used = 1 + static_cast<int>(ix_wave_max(static_cast<float>(last)));
+    if (threadIdx.x == 0) used = n_used;
     if (threadIdx.x == 0)
       inv_l = head_gate ? 1.0f / (L * (1.0f + __expf(-(float)head_gate[(th / heads) * head_gate_stride + th % heads]))) : 1.0f / L;
   }
   __syncthreads();
+  const int n = used;
   const float* po = part_o + th * n_splits * head_dim;
   const __bf16* gr = gate ? gate + (th / heads) * gate_stride + (th % heads) * head_dim : nullptr;
   auto gated = [&](float o, int d) { return gr ? o / (1.0f + __expf(-(float)gr[d])) : o; };
@@ -358,7 +492,7 @@ attn_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ 
     for (int d = threadIdx.x; d < half; d += blockDim.x) {
       float u = 0.f, w = 0.f;
 #pragma unroll 8
-      for (int s = 0; s < n_splits; ++s) {
+      for (int s = 0; s < n; ++s) {
         u += wgt[s] * po[s * head_dim + d];
         w += wgt[s] * po[s * head_dim + half + d];
       }
@@ -371,7 +505,7 @@ attn_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ 
   for (int d = threadIdx.x; d < head_dim; d += blockDim.x) {
     float acc = 0.f;
 #pragma unroll 8
-    for (int s = 0; s < n_splits; ++s) acc += wgt[s] * po[s * head_dim + d];
+    for (int s = 0; s < n; ++s) acc += wgt[s] * po[s * head_dim + d];
     out[th * head_dim + d] = (__bf16)gated(acc * inv_l, d);
   }
 }
@@ -385,7 +519,7 @@ int ix_attention_combine(const float* part_o, const float* part_ml, void* out, i
   return ix_check_launch("ix_attention_combine");
 }
 
-template <int NB, int QT, bool PF, bool GQ = false, bool MORE = true>
+template <int NB, int QT, bool PF, bool GQ = false, bool MORE = true, bool TURN = false>
 static void launch_attn(dim3 grid, hipStream_t stream, const void* q, const void* k, const void* v,
                         const int32_t* table, const int32_t* tile_seq, const int32_t* tile_q0,
                         const int32_t* tile_rows, const int32_t* positions, void* out, float* part_o, float* part_ml,
@@ -399,10 +533,18 @@ static void launch_attn(dim3 grid, hipStream_t stream, const void* q, const void
   // workgroups per compute unit of the 256 (one request of 16 heads with its keys in 32 slices: 512 wavefronts)
   const int64_t waves = static_cast<int64_t>(n_tiles) * n_splits * grid.y;
   const int per_group = waves >= 4 * 512 ? 4 : (waves >= 2 * 512 ? 2 : 1);
-  grid.x = static_cast<unsigned>((static_cast<int64_t>(n_tiles) * n_splits + per_group - 1) / per_group);
-  hipLaunchKernelGGL((attn_mfma_kernel<NB, QT, PF, GQ, MORE>), grid, dim3(64 * per_group), 0, stream, (const __bf16*)q, (const __bf16*)k,
+  if (PF) grid = dim3(static_cast<unsigned>((waves + per_group - 1) / per_group));
+  else grid.x = static_cast<unsigned>((static_cast<int64_t>(n_tiles) * n_splits + per_group - 1) / per_group);
+  // Decoding: no slice under 128 keys, or 256 where the launch fills the chip twice over (2,048 wavefronts); what a
+  // wavefront waits for before its first keys (its tile, its position, its pages) is worth about as many.  So a short
+  // context beside long ones is not cut as often as they are.  Eight contexts of 2,048 in slices of 256 and 128 keys:
+  // 26.7 and 29.0 us; eight of 200 to 2,048: 19.5 and 22.1; 4 of 200 to 2,048, 128 keys and equal shares: 13.2 and 14.5.
+  const int min_slice = !PF || waves <= 512 ? 32 : (waves < 2048 ? 128 : 256);
+  hipLaunchKernelGGL((attn_mfma_kernel<NB, QT, PF, GQ, MORE, TURN>), grid, dim3(64 * per_group),
+                     TURN ? per_group * 32 * 32 * NB : 0, stream, (const __bf16*)q, (const __bf16*)k,
                      (const __bf16*)v, table, tile_seq, tile_q0, tile_rows, positions, (__bf16*)out, part_o, part_ml,
-                     n_tiles, n_splits, heads, kv_heads, page_size, max_blocks, scale_log2, span, page_shift, sink,
+                     n_tiles, n_splits, heads, kv_heads, page_size, max_blocks, scale_log2, span, page_shift, min_slice,
+                     sink,
                      reinterpret_cast<const float2*>(turn_back), cap_slope, cap2, (const __bf16*)gate, gate_stride);
 }
 
@@ -433,6 +575,7 @@ static int attention_mfma_any(const void* q, const void* k_cache, const void* v_
              "grouped queries: tiles of 16, at most 16 query heads per key/value head");
   if (n_tiles == 0 || tokens == 0) return 0;
   const int64_t units = static_cast<int64_t>(n_tiles) * n_splits;
+  IX_REQUIRE(units * heads < (int64_t(1) << 31), "too many slices of keys for one launch");
   dim3 grid(static_cast<unsigned>((units + 3) / 4), grouped ? kv_heads : heads);
   const float scale_log2 = scale * 1.4426950408889634f;
   const float cap2 = softcap * 1.4426950408889634f, cap_slope = softcap > 0.f ? 2.0f * scale_log2 / softcap : 0.f;
@@ -445,9 +588,10 @@ static int attention_mfma_any(const void* q, const void* k_cache, const void* v_
   case NB:                                                          \
     if (grouped) {                                                  \
       if (prefetch && more) launch_attn<NB, 1, true, true>(ARGS);   \
-      else if (prefetch) launch_attn<NB, 1, true, true, false>(ARGS); \
+      else if (prefetch) launch_attn<NB, 1, true, true, false, NB == 8>(ARGS); \
       else launch_attn<NB, 1, false, true>(ARGS);                   \
     } else if (prefetch && more) launch_attn<NB, 1, true>(ARGS);    \
+    else if (prefetch && heads == kv_heads) launch_attn<NB, 1, true, false, false, NB == 8>(ARGS); \
     else if (prefetch) launch_attn<NB, 1, true, false, false>(ARGS); \
     else launch_attn<NB, 1, false>(ARGS);                           \
     break;

@@ -260,8 +260,9 @@ class PagedAttention(Mixer):
                     if rows is not None:
                         out.index_copy_(0, rows, outs)
                 return
-            tiles, tile, n_splits, grouped = query_tiles(ctx, self.span, self.num_heads, self.head_dim,
-                                                         self.num_kv_heads)
+            tiles, tile, _, grouped = query_tiles(ctx, self.span, self.num_heads, self.head_dim, self.num_kv_heads)
+            n_splits = decode_slices(tiles.shape[1] * (self.num_kv_heads if grouped else self.num_heads),
+                                     plan_tiles(ctx, tile)[2], self.span)
             work = None
             if n_splits > 1:
                 work = ctx.rt.empty((q.shape[0] * self.num_heads * n_splits * (self.head_dim + 2),), torch.float32)
@@ -497,6 +498,21 @@ def _n_splits(units: int, longest: int, span: int, tile: int) -> int:
     no slice shorter than MIN_KEYS_PER_SPLIT, a power of two (few distinct values, few captured graphs)."""
     keys = min(longest, abs(span) + tile + 32) if span else longest
     n_splits = 1 if units >= 2048 else max(1, min(WAVES_WANTED // max(1, units), -(-keys // MIN_KEYS_PER_SPLIT), 64))
+    return 1 << (n_splits.bit_length() - 1)
+
+
+def decode_slices(units: int, longest: int, span: int) -> int:
+    """Into how many slices at most the wavefront-level kernel cuts the keys of a step of one token per request
+    (bfloat16): as many as make up WAVES_WANTED wavefronts, none under 128 keys (64, up to 32 slices, where one request
+    leaves the chip half empty: 517 keys of 16 heads in 16 and 8 slices 7.4 and 9.0 us), and at least one for every 512
+    keys, since contexts may differ: the kernel gives short ones fewer (a floor under the slices' length), so that no
+    wavefront walks a long context while the others are done.  64 requests of 200 to 2,048 tokens in 2, 4 and 8 slices:
+    85, 78 and 78 us; 64 of 2,048 each: 164, 168 and 172.  A power of two; at most 64, and 16,384 wavefronts (the parts'
+    room)."""
+    keys = min(longest, abs(span) + QUERY_TILE + 32) if span else longest
+    by_keys = max(-(-keys // MIN_KEYS_PER_SPLIT), min(-(-keys // 64), 32) if units <= 16 else 1)
+    by_length = min(-(-keys // 512), 8 * WAVES_WANTED // max(1, units))
+    n_splits = max(1, min(max(WAVES_WANTED // max(1, units), by_length), by_keys, 64))
     return 1 << (n_splits.bit_length() - 1)
 
 

@@ -155,6 +155,30 @@ def test_attention_mfma_grouped_queries(case, n_splits, prefetch):
           f"attention_mfma grouped splits={n_splits}")
 
 
+@pytest.mark.parametrize("heads,kv_heads,page,window", [(16, 16, 16, 0), (16, 16, 48, 300), (28, 4, 32, 0), (28, 4, 16, 64)])
+@pytest.mark.parametrize("n_splits", [1, 16, 33])
+def test_attention_mfma_of_uneven_contexts(heads, kv_heads, page, window, n_splits):
+    """Heads of 128, one token each: contexts around the slices' least length (256 keys where 2,048 wavefronts and more
+    run, 128 or none below) and the 1,024 keys whose pages are looked up at once; slices without keys; numbers that are
+    not finite in the rest of the cache."""
+    from inferx_amd import ops
+    seq_lens = [1, 31, 33, 255, 256, 257, 513, 1023, 1057, 2090] + [96] * 20
+    q_lens = [1] * len(seq_lens)
+    p = build_paged(seq_lens, q_lens, heads, kv_heads, 128, page, torch.bfloat16, seed=8)
+    table = p["table"].tolist()
+    for s, L in enumerate(seq_lens):
+        if L % page:
+            p["k_cache"][table[s][L // page], :, L % page:] = float("nan")
+            p["v_cache"][table[s][L // page], :, :, L % page:] = float("inf")
+    out = torch.full_like(p["q"], float("nan"))
+    T = len(seq_lens)
+    work = torch.full((T * heads * n_splits * 130,), float("nan"), device=DEV) if n_splits > 1 else None
+    ops.attention_mfma(p["q"], p["k_cache"], p["v_cache"], p["table"], tiles_for(q_lens, 1), p["positions"], out,
+                       n_splits, work, 128 ** -0.5, window, 16, True, grouped=heads > kv_heads)
+    close(out, attention_reference(p, seq_lens, q_lens, heads, kv_heads, 128 ** -0.5, window), TOL[torch.bfloat16],
+          f"attention_mfma uneven, splits={n_splits}")
+
+
 PREFILL_CASES = ATTN_CASES + [
     ([1500], [1500], 5, 1, 128, 16, 0),                   # many tiles of one request
     ([777, 300], [130, 300], 4, 2, 112, 16, 0),           # a portion that starts off a tile's edge; odd head blocks

@@ -49,12 +49,11 @@ WIDE_TILES_WIDTH = 3072
 # Measured at the A2.7B shape (24 layers), with against without: decoding at batch 64 11.22 against 11.59 ms a step; a
 # portion of 256 tokens 6.58 against 7.19 ms, of 512 8.16 against 9.17, of 768 9.50 against 9.47, of 1,024 10.88
 # against 10.42; at the 57B shape (8 layers) 512 tokens 9.41 against 10.26 ms, 1,024 13.41 against 13.29.  With the
-# grouped products' stages pipelined and their tiles cut over the dies, ms of a whole prompt: A2.7B shape (8 layers), folded
-# / beside / after: 256 tokens 2.48 / 2.75 / 2.79, 512 2.99 / 3.18 / 3.19, 768 3.33 / 3.50 / 3.60, 1,024 3.78 / 3.97 / 3.99,
-# 1,536 4.48 / 4.47 / 4.68, 2,048 5.35 / 5.11 / 5.35, 4,096 9.37 / 8.56 / 8.87; 57B shape (4 layers), folded / after: 256
-# 3.98 / 4.34, 512 4.52 / 5.15, 768 5.10 / 5.61, 1,024 5.97 / 6.60, 2,048 9.86 / 9.78: the line could now lie higher, and
-# has not been moved.
-FOLD_SHARED_BELOW_TOKENS = 768
+# grouped products as they are now (stages pipelined, tiles cut over the dies, an expert's tiles sharing its weights), us of
+# a whole prompt, without / with: A2.7B shape (8 layers) 300 tokens 2,672 / 2,430, 800 3,462 / 3,261, 1,024 3,883 / 3,603,
+# 1,300 4,416 / 4,198, 1,536 4,505 / 4,512, 2,048 5,150 / 5,237, 4,096 8,361 / 9,009; 57B shape (4 layers) 512 tokens 5,254 /
+# 4,564, 1,024 6,635 / 6,030, 1,500 7,931 / 7,678, 2,048 9,756 / 9,785.
+FOLD_SHARED_BELOW_TOKENS = 1536
 
 
 class MoeFeedForward(FeedForward):

@@ -31,6 +31,16 @@ from .dense_mlp import stack_rows
 from .short_conv import ShortConv
 
 
+# A step that brings some request several tokens goes through the kernel that shares keys and values through LDS where it
+# has a workgroup (a tile of 64 queries of a head) for every compute unit, or no context is long: a workgroup walks all of
+# its keys (1.3 us for 32 of them), while the wavefront-level kernel cuts them into slices.  us, that one / this one, 16
+# heads, window 1,024: whole prompts of 611 and 1,437 105 / 48, eight of 200 37 / 16, one of 300 19.5 / 17.5; portions of 64
+# to 500 tokens on 1,500 (16 to 128 workgroups) 18 to 45 / 44 to 50; 300 tokens beside sixteen single ones (336) 70 / 53.
+PREFILL_TILE = 64
+PREFILL_MIN_WORKGROUPS = 256
+PREFILL_SHORT_KEYS = 384
+
+
 class DifferentialAttention(Mixer):
     graph_safe = True  # every launch reads the step's device arrays only
 
@@ -124,6 +134,14 @@ class DifferentialAttention(Mixer):
         queries of a request, a (head, map) pair per wavefront (a step of one token per request: the query heads of
         a key/value head side by side); else the plain one."""
         page_size = cache.k.shape[2]
+        if (q.dtype == torch.bfloat16 and not ctx.one_token_each
+                and ops.attention_diff_prefill_fits(self.head_dim, self.value_dim, page_size)):
+            tiles, n_tiles, longest = plan_tiles(ctx, PREFILL_TILE)
+            if n_tiles * self.num_heads >= PREFILL_MIN_WORKGROUPS or longest <= PREFILL_SHORT_KEYS:
+                ops.attention_diff_prefill(q, cache.k, cache.v, ctx.block_tables[cache.group], tiles, ctx.positions, out,
+                                           self.scale, self.window, self.keep_first, self.lam, self.norm_eps,
+                                           1.0 - self.diff)
+                return
         if q.dtype == torch.bfloat16 and ops.attention_diff_mfma_fits(self.head_dim, self.value_dim, page_size):
             tiles, n_tiles, longest = plan_tiles(ctx, QUERY_TILE)
             group = self.num_heads // self.num_kv_heads

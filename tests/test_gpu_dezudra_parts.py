@@ -483,6 +483,38 @@ def test_differential_attention_on_the_matrix_cores(H, G, D, V, window, keep, n_
     close(out, want, 1.5e-2, "differential attention (matrix cores)")
 
 
+@pytest.mark.parametrize("page", [16, 48])
+@pytest.mark.parametrize("H,G,D,V,window,keep", [(4, 2, 64, 64, 0, 0), (3, 1, 64, 128, 24, 3), (2, 2, 128, 64, 70, 40),
+                                                 (4, 1, 128, 128, 100, 5), (2, 1, 64, 128, 1, 2), (1, 1, 64, 64, 33, 64)])
+def test_differential_attention_through_lds(H, G, D, V, window, keep, page):
+    """Tiles of up to 64 queries: portions of 21, 64, 65 and 130 queries (whole and ragged sixteens, wavefronts without
+    queries) and single ones; where the window has left whole pages of the last portion's request, they hold
+    not-a-number, as does what lies past its end."""
+    from inferx_amd import ops
+    dtype = torch.bfloat16
+    L = 433
+    runs = [(0, 21), (40, 104), (130, 195), (250, 251), (L - 130, L)]
+    lam, eps, mult = 0.45, 1e-5, 0.7
+    for chosen in ([0, 1, 2, 3, 4], [4]):
+        k, v = rnd((L, 2 * G, D), 1, 1.0, dtype), rnd((L, G, V), 2, 1.0, dtype)
+        kk, vv = k.clone(), v.clone()
+        if chosen == [4] and window:
+            dead, alive = -(-keep // page) * page, (L - 130 + 1 - window) // page * page
+            kk[dead:alive] = float("nan")
+            vv[dead:alive] = float("nan")
+        positions, tiles = [], []
+        for a, b in (runs[i] for i in chosen):
+            tiles += [(0, len(positions) + at, min(64, b - a - at)) for at in range(0, b - a, 64)]
+            positions += range(a, b)
+        q = rnd((len(positions), H, 2, D), 3, 1.0, dtype)
+        kc, vc, table = paged(kk, vv, page, dtype)
+        out = torch.full((len(positions), H, V), float("nan"), dtype=dtype, device=DEV)
+        ops.attention_diff_prefill(q.to(DEV), kc, vc, table, torch.tensor(tiles, dtype=torch.int32, device=DEV).t().contiguous(),
+                                   i32(positions), out, 0.3, window, keep, lam, eps, mult)
+        want = plain_diff_attention(f64(q), f64(k).reshape(L, G, 2, D), f64(v), positions, 0.3, window, keep, lam, eps, mult)
+        close(out, want, 1.5e-2, f"differential attention through LDS, portions {chosen}")
+
+
 @pytest.mark.parametrize("n_splits", [1, 4])
 @pytest.mark.parametrize("H,G,D,V,window,keep", [(4, 2, 32, 32, 24, 3), (16, 1, 64, 32, 0, 0), (6, 2, 16, 96, 44, 3)])
 def test_differential_attention_one_token_each_grouped(H, G, D, V, window, keep, n_splits):

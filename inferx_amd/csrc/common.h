@@ -19,11 +19,13 @@ __device__ __forceinline__ float ix_bf16_to_f32(uint16_t b) {
 }
 
 // round to nearest even; NaN stays NaN
-__device__ __forceinline__ uint16_t ix_f32_to_bf16(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return static_cast<uint16_t>(u >> 16);
+__device__ __forceinline__ uint16_t ix_f32_to_bf16(float f) {  // (one instruction on gfx950, as are two of them together)
+  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
+}
+// two numbers, the first in the lower half
+__device__ __forceinline__ uint32_t ix_f32x2_to_bf16x2(float lo, float hi) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, bf16x2{static_cast<__bf16>(lo), static_cast<__bf16>(hi)});
 }
 
 __device__ __forceinline__ float ix_load(const float* p) { return *p; }

@@ -319,6 +319,24 @@ def test_clamped_gated_unit_with_biases(dtype, tol, limit):
     assert float((act.cpu().double() - want).abs().max()) <= tol * float(want.abs().max())
 
 
+@pytest.mark.parametrize("bias", ["bfloat16", "float32", "bfloat16 off a boundary"])
+def test_clamped_gated_unit_of_many_rows(bias):
+    """More rows than lines of workgroups (512), a width of 257 pieces of eight; a bias of either type, also one that does
+    not lie on 16 bytes."""
+    from inferx_amd import ops
+    T, n, limit = 600, 2056, 7.0
+    gate_up = rnd((T, 2 * n), 1, 3.0, torch.bfloat16)
+    b = rnd((2 * n + 1,), 2, 1.0, torch.float32 if bias == "float32" else torch.bfloat16)
+    dev = b.to(DEV)
+    b, dev = (b[1:], dev[1:]) if bias.endswith("boundary") else (b[:-1], dev[:-1])
+    act = torch.empty(T, n, dtype=torch.bfloat16, device=DEV)
+    ops.glu_bias(gate_up.to(DEV), dev, act, limit)
+    z = gate_up.double() + b.double()
+    g, u = z[:, :n].clamp(max=limit), z[:, n:].clamp(-limit, limit)
+    want = g * torch.sigmoid(1.702 * g) * (u + 1)
+    assert float((act.cpu().double() - want).abs().max()) <= 1e-2 * float(want.abs().max())
+
+
 def test_norm_with_one_number():
     x = rnd((5, 24), 1).double()
     g = torch.tensor(1.3, dtype=torch.float64)

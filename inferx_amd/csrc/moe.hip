@@ -210,9 +210,59 @@ moe_route_logits_mfma_kernel(const __bf16* __restrict__ x, const __bf16* __restr
   }
 }
 
+// Many tokens, float32 activations and weights: the same with v_mfma_f64_16x16x4_f64, whose 64-bit sums (two scores a few
+// 32-bit roundings apart must not change places) cost nothing beside the loads: rounded once, the scores are no further from
+// the 64-bit ones than a wavefront's own sums.  A lane reads four consecutive numbers of its row, the e-th of which meet in
+// one instruction.  511 tokens of 2,048 numbers, 61 rows, within a step: 16 + 6 us with the
+// selection against 60 of a workgroup a token that reads all the router's rows (0.7e-7 from the 64-bit weights, 1.2e-7).
+typedef double route_f64x4 __attribute__((ext_vector_type(4)));
+__global__ void __launch_bounds__(256)
+moe_route_logits_f64_kernel(const float* __restrict__ x, const float* __restrict__ wr, const float* __restrict__ shared_gate_w,
+                            const float* __restrict__ bias, float* __restrict__ logits, int64_t tokens, int width,
+                            int experts) {
+  __shared__ route_f64x4 part[4][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m = lane & 15, g = lane >> 4;
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * 16;
+  const int rows = experts + (shared_gate_w ? 1 : 0);
+  const int r = min(16 * static_cast<int>(blockIdx.y) + m, rows - 1);  // (rows and tokens past the end: the last, not written)
+  const float* xrow = x + min(t0 + m, tokens - 1) * width;
+  const float* wrow = r < experts ? wr + static_cast<int64_t>(r) * width : shared_gate_w;
+  const route_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  route_f64x4 acc[2] = {{0., 0., 0., 0.}, {0., 0., 0., 0.}};
+  for (int kc = 16 * wave; kc < width; kc += 256) {  // uniform over the wavefront
+    route_f32x4 xb[4], wa[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k0 = kc + 64 * u + 4 * g;
+      const bool ok = k0 < width;  // width is a multiple of 4: a lane's piece is whole or absent
+      xb[u] = ok ? *reinterpret_cast<const route_f32x4*>(xrow + k0) : zero;
+      wa[u] = ok ? *reinterpret_cast<const route_f32x4*>(wrow + k0) : zero;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        acc[e & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(wa[u][e]), static_cast<double>(xb[u][e]),
+                                                          acc[e & 1], 0, 0, 0);
+  }
+  part[wave][lane] = acc[0] + acc[1];
+  __syncthreads();
+  if (wave == 0) {
+    const route_f64x4 sum = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+    const int64_t t = t0 + m;  // lane holds rows 16 y + 4 e + g of token t0 + m
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int row = 16 * blockIdx.y + 4 * e + g;
+      if (t < tokens && row < rows)
+        logits[t * (experts + 1) + row] = static_cast<float>(sum[e]) + (bias && row < experts ? bias[row] : 0.f);
+    }
+  }
+}
+
 // `bias` (float32 [experts], or null) is added to the experts' scores before anything else.
 // `logits_scratch`: float32 [tokens, experts + 1], used when tokens <= ROUTE_SMALL_TOKENS, and for more tokens when
-// activations and weights are bfloat16 (may be null: then one kernel per token computes and selects).
+// activations and weights are bfloat16 or all float32 (may be null: then one kernel per token computes and selects).
 #define ROUTE_SMALL_TOKENS 128
 extern "C" int ix_moe_route(const void* x, int dtype, const void* wr, int wr_dtype, const void* shared_gate_w,
                             int sg_dtype, const float* bias, float* topk_w, int32_t* topk_e, float* shared_gate,
@@ -253,6 +303,18 @@ extern "C" int ix_moe_route(const void* x, int dtype, const void* wr, int wr_dty
     hipLaunchKernelGGL(moe_route_logits_mfma_kernel, dim3(static_cast<unsigned>((tokens + 15) / 16), row_blocks),
                        dim3(256), 0, stream, (const __bf16*)x, (const __bf16*)wr, (const __bf16*)shared_gate_w, bias, logits_scratch,
                        tokens, (int)width, experts);
+    hipLaunchKernelGGL(moe_route_select_kernel, dim3(tokens), dim3(64), experts * sizeof(float), stream,
+                       logits_scratch, topk_w, topk_e, shared_gate_w ? shared_gate : nullptr, experts, k, renormalize,
+                       scale, always, n_groups, groups_keep);
+    return ix_check_launch("ix_moe_route");
+  }
+  if (logits_scratch != nullptr && dtype == IX_F32 && wr_dtype == IX_F32 &&
+      (shared_gate_w == nullptr || sg_dtype == IX_F32) && width % 4 == 0 && width < (1 << 30) &&
+      ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(wr) | reinterpret_cast<uintptr_t>(shared_gate_w)) & 15) == 0) {
+    const int row_blocks = (experts + (shared_gate_w ? 1 : 0) + 15) / 16;
+    hipLaunchKernelGGL(moe_route_logits_f64_kernel, dim3(static_cast<unsigned>((tokens + 15) / 16), row_blocks), dim3(256), 0,
+                       stream, (const float*)x, (const float*)wr, (const float*)shared_gate_w, bias, logits_scratch, tokens,
+                       (int)width, experts);
     hipLaunchKernelGGL(moe_route_select_kernel, dim3(tokens), dim3(64), experts * sizeof(float), stream,
                        logits_scratch, topk_w, topk_e, shared_gate_w ? shared_gate : nullptr, experts, k, renormalize,
                        scale, always, n_groups, groups_keep);

@@ -264,7 +264,7 @@ __device__ __forceinline__ conv_u32x4 conv_pack8(const Conv8& y) {
   conv_u32x4 p;
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    p[e] = ix_f32_to_bf16(y.x[2 * e]) | static_cast<uint32_t>(ix_f32_to_bf16(y.x[2 * e + 1])) << 16;
+    p[e] = ix_f32x2_to_bf16x2(y.x[2 * e], y.x[2 * e + 1]);
   return p;
 }
 
@@ -378,15 +378,34 @@ __global__ void __launch_bounds__(CONV_THREADS) short_conv_vec8_kernel(ConvArgs 
   }
 }
 
-// The same for prompt portions without a rotation, at most four taps: a thread owns eight channels of eight
+// The same for prompt portions, at most four taps: a thread owns eight channels of eight
 // consecutive rows, so that taps, bias and nearly every input are read once, and values that eight consecutive places of
 // a page take are written eight at a time.  A row whose inputs all lie in its own portion (its place i >= taps - 1) is
 // formed here; the portion's first rows, a last row that is among them, and the new state belong to one further
 // workgroup per request (blockIdx.x < requests), which alone reads and writes the state.
+//
+// ROT: a rotated channel's partner belongs to the lane rot_dims / 16 further on or back (heads of a size that divides 512
+// lie within a wavefront's 64 lanes), whose sums come by way of a shuffle.  2,048 rows of 2,048 + 512 rotated channels and 512
+// of values that go into pages, four taps: 21 us (47 as a workgroup a row, whose values were stored 2 bytes at a time).
 #define CONV_TILE 8
 #define CONV_TILE_THREADS 128
 
-template <int TAPS>
+// channels c .. c + 7 of row `row`, rotated: `by` the blocks of eight to the partner, `second` which of the two this lane has
+__device__ __forceinline__ void conv_rotate8(const ConvArgs& a, int64_t row, int pair0, int by, bool second, Conv8& y) {
+  const conv_f32x4* cs = reinterpret_cast<const conv_f32x4*>(a.cos_sin + (row * (a.rot_dims / 2) + pair0) * 2);
+  const int from = static_cast<int>(threadIdx.x & 63) + (second ? -by : by);
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    const conv_f32x4 t = cs[h];  // (cos, sin) of two pairs
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const float c = t[2 * e], s = t[2 * e + 1], mine = y.x[2 * h + e], other = __shfl(mine, from, 64);
+      y.x[2 * h + e] = second ? mine * c + other * s : mine * c - other * s;
+    }
+  }
+}
+
+template <int TAPS, bool ROT>
 __global__ void __launch_bounds__(CONV_TILE_THREADS)
 short_conv_tile_kernel(ConvArgs a, const float* __restrict__ wt, const float* __restrict__ bias_f, int vunits,
                        int requests, int tokens) {
@@ -397,6 +416,10 @@ short_conv_tile_kernel(ConvArgs a, const float* __restrict__ wt, const float* __
   const bool live = unit < vunits;
   const int c0 = 8 * (live ? unit : vunits - 1);
   const uint16_t* in = static_cast<const uint16_t*>(a.in);
+  const int half_blocks = a.rot_dims / 16, block = (c0 % a.head_dim) / 8;
+  const bool rotated = ROT && c0 < a.q_channels + a.k_channels && block < 2 * half_blocks;
+  const bool second = block >= half_blocks;
+  const int pair0 = 8 * (second ? block - half_blocks : block);
   if (static_cast<int>(blockIdx.x) < requests) {  // (started first: a chain of reads, worked beside the tiles)
     const int seq = blockIdx.x;
     const int64_t row0 = a.q_start[seq];
@@ -428,6 +451,7 @@ short_conv_tile_kernel(ConvArgs a, const float* __restrict__ wt, const float* __
       const float temp = (a.temp_every > 0.f && c0 < a.q_channels) ? conv_temperature(a, row0 + i) : 1.0f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) y.x[e] *= temp;
+      if (rotated) conv_rotate8(a, row0 + i, pair0, half_blocks, second, y);
       conv_store8(a, row0 + i, c0, y);
     }
 #pragma unroll
@@ -499,6 +523,7 @@ short_conv_tile_kernel(ConvArgs a, const float* __restrict__ wt, const float* __
 #pragma unroll
       for (int e = 0; e < 8; ++e) y.x[e] *= temp;
     }
+    if (rotated) conv_rotate8(a, min(r0 + i, tokens - 1), pair0, half_blocks, second, y);
     vrows[i] = conv_pack8(y);
     if (!formed_s[i] || (is_v && run)) continue;
     if (!paged) {
@@ -572,13 +597,18 @@ extern "C" int ix_short_conv(const void* in, int dtype, int64_t in_stride, const
       value_dim % 8 == 0 && rot_dims % 16 == 0 && in_stride % 8 == 0 && state_stride % 4 == 0 && aligned(in) &&
       aligned(state) && aligned(wt) && aligned(bias_f) && aligned(out_q) && aligned(out_k) && plain_rows_ok &&
       (slots == nullptr || aligned(out_k))) {
-    if (rot_dims == 0 && taps <= 4 && tokens >= 64 && tokens >= 8 * static_cast<int64_t>(requests) && aligned(out_v)) {
+    const bool rotates = rot_dims > 0 && cos_sin != nullptr;
+    if ((!rotates || (512 % head_dim == 0 && aligned(cos_sin))) && taps <= 4 && tokens >= 64 && tokens >= 8 * static_cast<int64_t>(requests) && aligned(out_v)) {
       const int units = channels / 8, tiles = static_cast<int>((tokens + CONV_TILE - 1) / CONV_TILE);
       dim3 tgrid(tiles + requests, (units + CONV_TILE_THREADS - 1) / CONV_TILE_THREADS);
 #define CASE(TAPS)                                                                                                \
   case TAPS:                                                                                                      \
-    hipLaunchKernelGGL(short_conv_tile_kernel<TAPS>, tgrid, dim3(CONV_TILE_THREADS), 0, stream, a, wt,            \
-                       bias ? bias_f : nullptr, units, requests, static_cast<int>(tokens));                         \
+    if (rotates)                                                                                                  \
+      hipLaunchKernelGGL((short_conv_tile_kernel<TAPS, true>), tgrid, dim3(CONV_TILE_THREADS), 0, stream, a, wt,    \
+                         bias ? bias_f : nullptr, units, requests, static_cast<int>(tokens));                       \
+    else                                                                                                          \
+      hipLaunchKernelGGL((short_conv_tile_kernel<TAPS, false>), tgrid, dim3(CONV_TILE_THREADS), 0, stream, a, wt,   \
+                         bias ? bias_f : nullptr, units, requests, static_cast<int>(tokens));                       \
     break;
       switch (taps) { CASE(1) CASE(2) CASE(3) CASE(4) }
 #undef CASE

@@ -209,6 +209,48 @@ def test_short_convolution_rotates_and_appends(dtype, tol, D, V, rot):
         close(got[r], want[r], tol, f"request {r}, {rot} rotated")
 
 
+@pytest.mark.parametrize("taps", [1, 2, 4])
+@pytest.mark.parametrize("D,V,rot", [(64, 128, 64), (128, 64, 32), (16, 24, 16), (512, 8, 512), (24, 16, 16), (96, 64, 96)])
+def test_short_convolution_rotates_portions(D, V, rot, taps):
+    """Portions of many rows (threads that own eight rows of eight channels, a rotated channel's partner in another lane
+    where heads divide 512), continued from what the requests brought before: queries, keys and values in pages, and the
+    new state; portions that begin and end off a tile's edge, one of two rows."""
+    from inferx_amd import ops
+    dtype, page = torch.bfloat16, 16
+    sizes = (3 * D, 2 * D, 2 * V, D, V)
+    C = sizes[0] + sizes[1] + sizes[2]
+    lens, starts = [99, 2, 45, 64], [37, 5, 0, 200]
+    T = sum(lens)
+    w, bias = rnd((C, taps), 3, 0.5, dtype), rnd((C,), 4, 0.5, dtype)
+    x = rnd((T, C), 5, 1.0, dtype)
+    before = rnd((len(lens), taps - 1, C), 6, 1.0)
+    state = before.reshape(len(lens), -1).to(DEV).contiguous() if taps > 1 else torch.zeros((len(lens), 4), device=DEV)
+    q_start = [sum(lens[:r]) for r in range(len(lens) + 1)]
+    positions = [starts[r] + i for r in range(len(lens)) for i in range(lens[r])]
+    per = 20  # pages of a request
+    where = i32([(r * per) * page + starts[r] + i for r in range(len(lens)) for i in range(lens[r])])
+    k_cache = torch.zeros((len(lens) * per, 2, page, D), dtype=dtype, device=DEV)
+    v_cache = torch.zeros((len(lens) * per, 2, V, page), dtype=dtype, device=DEV)
+    inv_freq = torch.tensor([50.0 ** (-2.0 * j / rot) for j in range(rot // 2)], dtype=torch.float32, device=DEV)
+    table = torch.empty((T, rot // 2, 2), dtype=torch.float32, device=DEV)
+    ops.rope_table(table, i32(positions), inv_freq)
+    q = torch.empty((T, sizes[0]), dtype=dtype, device=DEV)
+    rows = ops.StepRows(i32([r for r in range(len(lens)) for _ in range(lens[r])]), i32(q_start), i32(range(len(lens))))
+    ops.short_conv(x.to(DEV), bias.to(DEV), w.to(DEV), state, rows, sizes, q, k_cache, v_cache, slots=where, cos_sin=table,
+                   weight_t=w.to(DEV).float().t().contiguous(), bias_f32=bias.to(DEV).float())
+    flat = where.long()
+    got = torch.cat([q, k_cache.permute(0, 2, 1, 3).reshape(-1, 2 * D)[flat], v_cache.permute(0, 3, 1, 2).reshape(-1, 2 * V)[flat]], 1)
+    for r, n in enumerate(lens):
+        mine = slice(q_start[r], q_start[r] + n)
+        u = np.concatenate([f64(before[r]), f64(x[mine]) + f64(bias)])
+        y = pd.short_conv(u, f64(w))[taps - 1:]
+        at = np.arange(starts[r], starts[r] + n)
+        turned = pd.rotate(y[:, :5 * D].reshape(-1, 5, D), at, rot, 50.0).reshape(-1, 5 * D)
+        close(got[mine], np.concatenate([turned, y[:, 5 * D:]], axis=1), 1.5e-2, f"request {r}")
+        if taps > 1:
+            close(state[r].reshape(taps - 1, C), u[len(u) - (taps - 1):], 1e-6, f"state of request {r}")
+
+
 # ---- the gated delta rule over steps ------------------------------------------------------------------------------
 def plain_delta(q, k, v, a, b, a_log, dt_bias, heads, kv_heads, dim, vdim):
     """The recurrence of `plain_dezudra.delta_mixer`, on its operands (float64 arrays)."""

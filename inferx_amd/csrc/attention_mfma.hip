@@ -29,6 +29,7 @@
 #include "common.h"
 #include "inferx_hip.h"
 
+#include <algorithm>
 #include <mutex>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -451,18 +452,27 @@ attn_mfma_kernel(const __bf16* __restrict__ q, const __bf16* __restrict__ k_cach
 }
 
 // out[t, h, :] = sum_s o_s 2^(m_s - M) / sum_s l_s 2^(m_s - M),  M = max_s m_s
-// One workgroup per (token, head); the slices' weights are worked out once, then every thread
-// sums its columns with independent loads.
-__global__ void __launch_bounds__(128)
+// One workgroup per (token, head).  Slices past the last one with keys were left unwritten but for that; they are not
+// used.  What bounds a launch this small is one trip to memory after the other: the parts of the first slices are asked
+// for together with all slices' reference points, and every thread takes one column (heads of up to 512).
+#define COMBINE_AHEAD 8
+__global__ void __launch_bounds__(512)
 attn_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, __bf16* __restrict__ out,
                     int n_splits, int head_dim, int heads, const float2* __restrict__ turn_back,
                     const __bf16* __restrict__ gate, int64_t gate_stride, const __bf16* __restrict__ head_gate,
                     int64_t head_gate_stride) {
   __shared__ float wgt[256];
   __shared__ float inv_l;
-  __shared__ int used;  // slices past the last one with keys: nothing was written of them but that
+  __shared__ int used;  // slices up to the last one with keys
   const int64_t th = blockIdx.x;  // token * heads + head
   const float* ml = part_ml + th * n_splits * 2;
+  const float* po = part_o + th * n_splits * head_dim;
+  float first[COMBINE_AHEAD];
+  {
+    const int d = min(static_cast<int>(threadIdx.x), head_dim - 1);
+#pragma unroll
+    for (int s = 0; s < COMBINE_AHEAD; ++s) first[s] = po[min(s, n_splits - 1) * head_dim + d];
+  }
   if (threadIdx.x < 64) {
     float mloc = -INFINITY;
     for (int s = threadIdx.x; s < n_splits; s += 64) mloc = fmaxf(mloc, ml[2 * s]);
@@ -478,13 +488,13 @@ attn_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ 
     }
     const float L = ix_wave_sum(lloc);
     const int n_used = 1 + static_cast<int>(ix_wave_max(static_cast<float>(last)));
-    if (threadIdx.x == 0) used = n_used;
-    if (threadIdx.x == 0)
+    if (threadIdx.x == 0) {
+      used = n_used;
       inv_l = head_gate ? 1.0f / (L * (1.0f + __expf(-(float)head_gate[(th / heads) * head_gate_stride + th % heads]))) : 1.0f / L;
+    }
   }
   __syncthreads();
   const int n = used;
-  const float* po = part_o + th * n_splits * head_dim;
   const __bf16* gr = gate ? gate + (th / heads) * gate_stride + (th % heads) * head_dim : nullptr;
   auto gated = [&](float o, int d) { return gr ? o / (1.0f + __expf(-(float)gr[d])) : o; };
   if (turn_back) {  // the result rotated by minus the token's angles: a thread takes element d and d + head_dim / 2
@@ -502,10 +512,17 @@ attn_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ 
     }
     return;
   }
-  for (int d = threadIdx.x; d < head_dim; d += blockDim.x) {
+  for (int d = threadIdx.x; d < head_dim; d += blockDim.x) {  // (once, unless a head is wider than the workgroup)
     float acc = 0.f;
+    int s = 0;
+    if (d == static_cast<int>(threadIdx.x)) {
+#pragma unroll
+      for (int i = 0; i < COMBINE_AHEAD; ++i)
+        if (i < n) acc += wgt[i] * first[i];
+      s = min(COMBINE_AHEAD, n);
+    }
 #pragma unroll 8
-    for (int s = 0; s < n; ++s) acc += wgt[s] * po[s * head_dim + d];
+    for (; s < n; ++s) acc += wgt[s] * po[s * head_dim + d];
     out[th * head_dim + d] = (__bf16)gated(acc * inv_l, d);
   }
 }
@@ -513,7 +530,8 @@ attn_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ 
 int ix_attention_combine(const float* part_o, const float* part_ml, void* out, int64_t tokens, int heads,
                          int n_splits, int head_dim, hipStream_t stream, const float* turn_back, const void* gate,
                          int64_t gate_stride, const void* head_gate, int64_t head_gate_stride) {
-  hipLaunchKernelGGL(attn_combine_kernel, dim3(static_cast<unsigned>(tokens * heads)), dim3(128), 0, stream, part_o,
+  const unsigned threads = static_cast<unsigned>(std::min(512, (head_dim + 63) / 64 * 64));
+  hipLaunchKernelGGL(attn_combine_kernel, dim3(static_cast<unsigned>(tokens * heads)), dim3(threads), 0, stream, part_o,
                      part_ml, (__bf16*)out, n_splits, head_dim, heads, reinterpret_cast<const float2*>(turn_back),
                      (const __bf16*)gate, gate_stride, (const __bf16*)head_gate, head_gate_stride);
   return ix_check_launch("ix_attention_combine");

@@ -274,6 +274,14 @@ latent_attn_mfma_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_
   const int per = ((k_end - k_begin + n_splits - 1) / n_splits + LATM_KEYS - 1) & ~(LATM_KEYS - 1);
   k_begin += static_cast<int>(blockIdx.z) * per;
   k_end = min(k_end, k_begin + per);
+  if (k_begin >= k_end && blockIdx.z > 0) {  // no keys are left for this slice: the merging kernel reads no more of it than that
+    if (g == 0 && wave_on && col_ok) {
+      const int64_t p = (static_cast<int64_t>(row) * heads + head) * n_splits + blockIdx.z;
+      part_ml[2 * p] = -INFINITY;
+      part_ml[2 * p + 1] = 0.f;
+    }
+    return;
+  }
   const int32_t* table = block_table + static_cast<int64_t>(seq_of_token[row]) * max_blocks;
   {  // (every decision in here is the same for the whole workgroup)
     uint4 st[NP];

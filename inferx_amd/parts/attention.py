@@ -477,18 +477,21 @@ def mixed_step_plan(ctx, span: int, heads: int, kv_heads: int, lds_fits: bool = 
     waves = []
     for seqs, grouped in sets:
         ns = n[seqs]
+        tile = 1 if grouped else QUERY_TILE
         alone = lds is None and len(sets) == 1
-        first = q_start[seqs] if alone else np.cumsum(ns) - ns
-        st = _tiles_of(ns, first, seqs, 1 if grouped else QUERY_TILE)
-        rows = positions = None
-        if alone:
-            positions = ctx.positions
-        else:
+        units = int((-(-ns // tile)).sum()) * (kv_heads if grouped else heads)
+        n_splits = _n_splits(units, int(b.seq_lens[seqs].max()), span, QUERY_TILE)
+        # Beside the LDS-sharing kernel, with whole keys, a tile's results go straight to its rows, wherever they lie (seven
+        # prompts of 5 to 150 tokens, 8 layers: two launches and 13 us a layer less).  Slices are merged for all rows of a
+        # launch, which must then be its own.
+        in_place = alone or (lds is not None and n_splits == 1)
+        st = _tiles_of(ns, q_start[seqs] if in_place else np.cumsum(ns) - ns, seqs, tile)
+        rows = None
+        positions = ctx.positions
+        if not in_place:
             rows = to_dev(np.concatenate([np.arange(q_start[i], q_start[i] + n[i]) for i in seqs]))
             positions = ctx.positions.index_select(0, rows)
-        units = st.shape[1] * (kv_heads if grouped else heads)
-        waves.append((rows, to_dev(st), positions, _n_splits(units, int(b.seq_lens[seqs].max()), span, QUERY_TILE),
-                      grouped))
+        waves.append((rows, to_dev(st), positions, n_splits, grouped))
     ctx.memo[key] = (lds, waves)
     return ctx.memo[key]
 

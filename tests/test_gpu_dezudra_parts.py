@@ -335,7 +335,8 @@ def test_delta_rule_keeps_what_was_written_long_ago():
 
 # ---- the norm per head, the gate, the difference --------------------------------------------------------------------
 @pytest.mark.parametrize("dtype,tol", TYPES)
-@pytest.mark.parametrize("heads,vdim", [(3, 12), (2, 64), (1, 200)])
+@pytest.mark.parametrize("heads,vdim", [(3, 12), (2, 64), (1, 200), (2, 65), (1, 511), (2, 512), (1, 1030), (1, 2048), (1, 4096),
+                                        (1, 4100)])
 def test_head_norm_with_gate_and_with_difference(dtype, tol, heads, vdim):
     from inferx_amd import ops
     T = 9

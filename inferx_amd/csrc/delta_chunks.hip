@@ -731,10 +731,13 @@ delta_chunks_chain_kernel(float* work, const int32_t* __restrict__ seq_ids, cons
   }
 }
 
-// O^T = S^T (diag(G) Q)^T + U^T P^T: a lane ends up with four consecutive columns of a row
+// O^T = S^T (diag(G) Q)^T + U^T P^T: a lane ends up with four consecutive columns of a row.  A wavefront takes sixteen columns,
+// a workgroup 64 of a (chunk, head): with 32 a wavefront two workgroups filled a compute unit's registers (and spilled), 528
+// of 128 columns needed a second turn for their last 16, and heads of 64 columns kept two of four wavefronts idle.  33 chunks of 16
+// heads of 128 x 128: 24.7 us (38.8); 32 of 32 of 64 x 64 (the generalized rule): 18.2 (32.8).
 template <int DIM, bool MORE>
-__global__ void __launch_bounds__(DC_THREADS, 2)
-delta_chunks_result_kernel(const float* __restrict__ work, const int32_t* __restrict__ chunk_row0,
+__global__ void __launch_bounds__(DC_THREADS, 3)
+delta_chunks_result_kernel(const float* work, const int32_t* __restrict__ chunk_row0,
                            const int32_t* __restrict__ chunk_rows, float* __restrict__ out, int heads, int vdim) {
   constexpr int LD = DIM + 4, LP = DC_ROWS + 4;
   __shared__ __attribute__((aligned(16))) float q_s[DC_ROWS * LD];
@@ -746,85 +749,65 @@ delta_chunks_result_kernel(const float* __restrict__ work, const int32_t* __rest
   const int n = chunk_rows[chunk];
   const DeltaBlock blk{DIM, vdim, MORE};
   const float* mine = work + (static_cast<int64_t>(chunk) * heads + head) * blk.size();
+  // Everything is asked for before the first of it is used (`work` is a plain pointer: loads through a `const __restrict__`
+  // one were moved behind the barrier); this wavefront's columns of S and U last, they arrive over the barrier (a tile past
+  // the last one: that one, not stored)
+  constexpr int NQ = DC_ROWS * DIM / 4 / DC_THREADS, NPP = DC_ROWS * 16 / DC_THREADS;
+  const int tile = 4 * blockIdx.z + wave, col0 = 16 * min(tile, vdim / 16 - 1);
+  f32x4 qr[NQ], pr[NPP], sa[DIM / 16], ua[4];
 #pragma unroll
-  for (int id = tid; id < DC_ROWS * DIM / 4; id += DC_THREADS) {
-    const int row = id / (DIM / 4), d = 4 * (id % (DIM / 4));
-    *reinterpret_cast<f32x4*>(q_s + row * LD + d) = *reinterpret_cast<const f32x4*>(mine + blk.q() + row * DIM + d);
+  for (int i = 0; i < NQ; ++i) qr[i] = *reinterpret_cast<const f32x4*>(mine + blk.q() + 4 * (tid + DC_THREADS * i));
+#pragma unroll
+  for (int i = 0; i < NPP; ++i) pr[i] = *reinterpret_cast<const f32x4*>(mine + blk.p() + 4 * (tid + DC_THREADS * i));
+#pragma unroll
+  for (int c = 0; c < DIM / 16; ++c)
+    sa[c] = *reinterpret_cast<const f32x4*>(mine + blk.s() + static_cast<int64_t>(col0 + m) * DIM + 16 * c + 4 * g);
+#pragma unroll
+  for (int s = 0; s < 4; ++s) ua[s] = *reinterpret_cast<const f32x4*>(mine + blk.u() + (col0 + m) * 64 + 16 * s + 4 * g);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    const int id = tid + DC_THREADS * i;
+    *reinterpret_cast<f32x4*>(q_s + id / (DIM / 4) * LD + 4 * (id % (DIM / 4))) = qr[i];
   }
 #pragma unroll
-  for (int id = tid; id < DC_ROWS * 16; id += DC_THREADS) {
-    const int row = id >> 4, j = 4 * (id & 15);  // (tiles above the diagonal hold nothing and are not read below)
-    if ((j >> 4) <= (row >> 4))
-      *reinterpret_cast<f32x4*>(p_s + row * LP + j) = *reinterpret_cast<const f32x4*>(mine + blk.p() + row * 64 + j);
+  for (int i = 0; i < NPP; ++i) {  // (tiles above the diagonal hold nothing and are not read below)
+    const int id = tid + DC_THREADS * i;
+    *reinterpret_cast<f32x4*>(p_s + (id >> 4) * LP + 4 * (id & 15)) = pr[i];
   }
   __syncthreads();
-  const int tiles = vdim / 16;
+  if (16 * tile >= vdim) return;
   const f32x4 none = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int t0 = 2 * wave; t0 < tiles; t0 += 8) {
-    f32x4 acc[2][4];  // [tile of columns][tile of rows]
+  f32x4 acc[4];  // [tile of rows]
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+  for (int r = 0; r < 4; ++r) acc[r] = none;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[u][r] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int t1 = min(t0 + 1, tiles - 1);
-    const float* s0 = mine + blk.s() + static_cast<int64_t>(16 * t0 + m) * DIM + 4 * g;
-    const float* s1 = mine + blk.s() + static_cast<int64_t>(16 * t1 + m) * DIM + 4 * g;
-    // (S is asked for at once, U half-way; a sixteen of the reduction is worked before the next one is read from LDS, or the
-    // registers do not hold what the compiler asks for ahead)
-    f32x4 sa[2][DIM / 16], ua[2][4];
+  for (int c = 0; c < DIM / 16; ++c) {
 #pragma unroll
-    for (int c = 0; c < DIM / 16; ++c) {
-      sa[0][c] = *reinterpret_cast<const f32x4*>(s0 + 16 * c);
-      sa[1][c] = *reinterpret_cast<const f32x4*>(s1 + 16 * c);
+    for (int r = 0; r < 4; ++r)
+      acc[r] += dc_mac(sa[c], *reinterpret_cast<const f32x4*>(q_s + (16 * r + m) * LD + 16 * c + 4 * g), none);
+    // (added up here: the optimiser would move the sums behind the branches below and keep every addend until then)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) asm volatile("" : "+v"(acc[r]));
+  }
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const bool odd = __any(dc_odd(ua[s]));
+#pragma unroll
+    for (int r = s; r < 4; ++r) {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(p_s + (16 * r + m) * LP + 16 * s + 4 * g);
+      if (r == s && odd) acc[r] += dc_mac_block_second(ua[s], b, dc_seen(m, 4 * g, true), none);
+      else acc[r] += dc_mac(ua[s], b, none);
     }
     __builtin_amdgcn_sched_barrier(0);
+  }
 #pragma unroll
-    for (int c = 0; c < DIM / 16; ++c) {
-      if (c == DIM / 32) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          ua[0][s] = *reinterpret_cast<const f32x4*>(mine + blk.u() + (16 * t0 + m) * 64 + 16 * s + 4 * g);
-          ua[1][s] = *reinterpret_cast<const f32x4*>(mine + blk.u() + (16 * t1 + m) * 64 + 16 * s + 4 * g);
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const f32x4 b = *reinterpret_cast<const f32x4*>(q_s + (16 * r + m) * LD + 16 * c + 4 * g);
-        acc[0][r] += dc_mac(sa[0][c], b, none);
-        acc[1][r] += dc_mac(sa[1][c], b, none);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const f32x4 a0 = ua[0][s], a1 = ua[1][s];
-      const bool odd = __any(dc_odd(a0) || dc_odd(a1));
-#pragma unroll
-      for (int r = s; r < 4; ++r) {
-        const f32x4 b = *reinterpret_cast<const f32x4*>(p_s + (16 * r + m) * LP + 16 * s + 4 * g);
-        if (r == s && odd) {
-          const f32x4 seen = dc_seen(m, 4 * g, true);
-          acc[0][r] += dc_mac_block_second(a0, b, seen, none);
-          acc[1][r] += dc_mac_block_second(a1, b, seen, none);
-        } else {
-          acc[0][r] += dc_mac(a0, b, none);
-          acc[1][r] += dc_mac(a1, b, none);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      if (t0 + u >= tiles) continue;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = 16 * r + m;
-        if (row < n) {
-          f32x4* to = reinterpret_cast<f32x4*>(out + ((row0 + row) * heads + head) * vdim + 16 * (t0 + u) + 4 * g);
-          if constexpr (MORE) *to += acc[u][r];  // (Q V is there already)
-          else *to = acc[u][r];
-        }
-      }
+  for (int r = 0; r < 4; ++r) {
+    const int row = 16 * r + m;
+    if (row < n) {
+      f32x4* to = reinterpret_cast<f32x4*>(out + ((row0 + row) * heads + head) * vdim + 16 * tile + 4 * g);
+      if constexpr (MORE) *to += acc[r];  // (Q V is there already)
+      else *to = acc[r];
     }
   }
 }
@@ -859,7 +842,7 @@ extern "C" int ix_delta_chunks(const void* q, const void* k, const void* v, int6
   hipLaunchKernelGGL((delta_chunks_chain_kernel<DIM, false>), dim3(heads, vdim / 16, seqs), dim3(DC_THREADS), 0, stream, work, \
                      seq_ids, seq_first, seq_count, state_slots, state, state_stride, heads, vdim);                      \
   if (ix_check_launch("ix_delta_chunks: chain")) return 1;                                                               \
-  hipLaunchKernelGGL((delta_chunks_result_kernel<DIM, false>), dim3(heads, chunks), dim3(DC_THREADS), 0, stream, work, chunk_row0, \
+  hipLaunchKernelGGL((delta_chunks_result_kernel<DIM, false>), dim3(heads, chunks, (vdim + 63) / 64), dim3(DC_THREADS), 0, stream, work, chunk_row0, \
                      chunk_rows, out, heads, vdim)
   if (dim == 32) { RUN(32); }
   else if (dim == 64) { RUN(64); }
@@ -894,7 +877,7 @@ extern "C" int ix_general_delta_chunks(const void* r, const void* k, const void*
   hipLaunchKernelGGL((delta_chunks_chain_kernel<DIM, true>), dim3(heads, vdim / 16, seqs), dim3(DC_THREADS), 0, stream,  \
                      work, seq_ids, seq_first, seq_count, state_slots, state, state_stride, heads, vdim);                \
   if (ix_check_launch("ix_general_delta_chunks: chain")) return 1;                                                       \
-  hipLaunchKernelGGL((delta_chunks_result_kernel<DIM, true>), dim3(heads, chunks), dim3(DC_THREADS), 0, stream, work,    \
+  hipLaunchKernelGGL((delta_chunks_result_kernel<DIM, true>), dim3(heads, chunks, (vdim + 63) / 64), dim3(DC_THREADS), 0, stream, work,    \
                      chunk_row0, chunk_rows, out, heads, vdim)
   if (dim == 32) { RUN(32); }
   else if (dim == 64) { RUN(64); }

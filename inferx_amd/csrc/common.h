@@ -40,6 +40,23 @@ __device__ __forceinline__ float ix_load_rt(const void* base, int dtype, int64_t
                          : ix_bf16_to_f32(static_cast<const uint16_t*>(base)[i]);
 }
 
+// elements i .. i + 3 (i a multiple of 4); in one load where the array lies on such a boundary
+__device__ __forceinline__ float4 ix_load4_rt(const void* base, int dtype, int64_t i) {
+  if (dtype == IX_F32 && (reinterpret_cast<uintptr_t>(base) & 15) == 0)
+    return *reinterpret_cast<const float4*>(static_cast<const float*>(base) + i);
+  if (dtype != IX_F32 && (reinterpret_cast<uintptr_t>(base) & 7) == 0) {
+    const uint2 p = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(base) + i);
+    return make_float4(__uint_as_float(p.x << 16), __uint_as_float(p.x & 0xffff0000u), __uint_as_float(p.y << 16),
+                       __uint_as_float(p.y & 0xffff0000u));
+  }
+  return make_float4(ix_load_rt(base, dtype, i), ix_load_rt(base, dtype, i + 1), ix_load_rt(base, dtype, i + 2),
+                     ix_load_rt(base, dtype, i + 3));
+}
+// four numbers rounded to bfloat16, side by side
+__device__ __forceinline__ uint2 ix_pack4_bf16(const float4& v) {
+  return make_uint2(ix_f32x2_to_bf16x2(v.x, v.y), ix_f32x2_to_bf16x2(v.z, v.w));
+}
+
 // Sum / maximum over the 64 lanes, result in every lane.  Within a row of 16 lanes the partners come through
 // DPP (lanes ^1, ^2, then the half row and the row mirrored: no LDS round trip), across rows through two
 // exchanges.  The order of the additions is fixed.

@@ -72,49 +72,54 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ h, const TD* __restrict__
   }
 }
 
-// bfloat16 delta and output with a width that is a multiple of 4: four columns per thread
-__global__ void add_rmsnorm_vec4_kernel(float* __restrict__ h, const uint16_t* __restrict__ delta,
-                                        const void* __restrict__ w, int w_dtype, uint16_t* __restrict__ out,
-                                        const int32_t* __restrict__ rows, int64_t row_width, int64_t width,
-                                        float eps) {
+// bfloat16 delta and output with a width that is a multiple of 4: NV times four columns per thread, which stay in registers;
+// what a row needs, the weight too, is asked for before its sum of squares is known (one trip to memory a row; read once
+// more after the sum, with the weight a number at a time: 2,048 rows of 2,048 12.6 us, now 10.5).
+template <int NV>
+__global__ void __launch_bounds__(1024)
+add_rmsnorm_vec4_kernel(float* __restrict__ h, const uint16_t* __restrict__ delta, const void* __restrict__ w, int w_dtype,
+                        uint16_t* __restrict__ out, const int32_t* __restrict__ rows, int64_t row_width, int64_t width,
+                        float eps) {
   __shared__ float red[16];
   const int64_t r = blockIdx.x;
   const int64_t row = rows ? rows[r] : r;
   const int64_t first = blockIdx.y * width;
   float* hr = h + row * row_width + first;
   const uint16_t* dr = delta ? delta + row * row_width + first : nullptr;
-  const bool write_back = (rows == nullptr) && (dr != nullptr);
-  auto value = [&](int64_t c) {
-    float4 v = *reinterpret_cast<const float4*>(hr + c);
-    if (dr) {
-      const uint2 d = *reinterpret_cast<const uint2*>(dr + c);
-      v.x += __uint_as_float(d.x << 16);
-      v.y += __uint_as_float(d.x & 0xffff0000u);
-      v.z += __uint_as_float(d.y << 16);
-      v.w += __uint_as_float(d.y & 0xffff0000u);
-    }
-    return v;
-  };
+  float4 v[NV], g[NV];
+  uint2 d[NV];
+#pragma unroll
+  for (int u = 0; u < NV; ++u) {  // (columns past the end: the first ones, not used)
+    const int64_t c = 4 * (threadIdx.x + u * static_cast<int64_t>(blockDim.x)), at = c < width ? c : 0;
+    v[u] = *reinterpret_cast<const float4*>(hr + at);
+    d[u] = dr ? *reinterpret_cast<const uint2*>(dr + at) : make_uint2(0u, 0u);
+    g[u] = ix_load4_rt(w, w_dtype, first + at);
+  }
   float sumsq = 0.f;
-  for (int64_t c = 4 * threadIdx.x; c < width; c += 4 * blockDim.x) {
-    const float4 v = value(c);
-    sumsq += v.x * v.x;
-    sumsq += v.y * v.y;
-    sumsq += v.z * v.z;
-    sumsq += v.w * v.w;
+#pragma unroll
+  for (int u = 0; u < NV; ++u) {
+    if (dr) {
+      v[u].x += __uint_as_float(d[u].x << 16);
+      v[u].y += __uint_as_float(d[u].x & 0xffff0000u);
+      v[u].z += __uint_as_float(d[u].y << 16);
+      v[u].w += __uint_as_float(d[u].y & 0xffff0000u);
+    }
+    if (4 * (threadIdx.x + u * static_cast<int64_t>(blockDim.x)) < width) {
+      sumsq += v[u].x * v[u].x;
+      sumsq += v[u].y * v[u].y;
+      sumsq += v[u].z * v[u].z;
+      sumsq += v[u].w * v[u].w;
+    }
   }
   sumsq = ix_block_sum(sumsq, red);
   const float inv = 1.0f / sqrtf(sumsq / static_cast<float>(width) + eps);
-  uint16_t* outr = out + r * row_width + first;
-  for (int64_t c = 4 * threadIdx.x; c < width; c += 4 * blockDim.x) {
-    const float4 v = value(c);  // h is still as it was: it is written here, after its last reading
-    if (write_back) *reinterpret_cast<float4*>(hr + c) = v;
-    uint2 o;
-    o.x = ix_f32_to_bf16(v.x * inv * ix_load_rt(w, w_dtype, first + c)) |
-          static_cast<uint32_t>(ix_f32_to_bf16(v.y * inv * ix_load_rt(w, w_dtype, first + c + 1))) << 16;
-    o.y = ix_f32_to_bf16(v.z * inv * ix_load_rt(w, w_dtype, first + c + 2)) |
-          static_cast<uint32_t>(ix_f32_to_bf16(v.w * inv * ix_load_rt(w, w_dtype, first + c + 3))) << 16;
-    *reinterpret_cast<uint2*>(outr + c) = o;
+#pragma unroll
+  for (int u = 0; u < NV; ++u) {
+    const int64_t c = 4 * (threadIdx.x + u * static_cast<int64_t>(blockDim.x));
+    if (c >= width) continue;
+    if (dr && !rows) *reinterpret_cast<float4*>(hr + c) = v[u];
+    *reinterpret_cast<uint2*>(out + r * row_width + first + c) =
+        ix_pack4_bf16(make_float4(v[u].x * inv * g[u].x, v[u].y * inv * g[u].y, v[u].z * inv * g[u].z, v[u].w * inv * g[u].w));
   }
 }
 
@@ -131,10 +136,17 @@ extern "C" int ix_add_rmsnorm(void* h, const void* delta, int delta_dtype, const
 #define LAUNCH(TD, TO)                                                                                          \
   hipLaunchKernelGGL((add_rmsnorm_kernel<TD, TO>), grid, block, 0, stream, (float*)h, (const TD*)delta, w, w_dtype, \
                      (TO*)out, rows, row_width, width, eps)
-  if (out_dtype == IX_BF16 && (delta == nullptr || delta_dtype == IX_BF16) && width % 4 == 0 &&
+  if (out_dtype == IX_BF16 && (delta == nullptr || delta_dtype == IX_BF16) && width % 4 == 0 && width <= 16384 &&
       ((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(delta) | reinterpret_cast<uintptr_t>(out)) & 15) == 0) {
-    hipLaunchKernelGGL(add_rmsnorm_vec4_kernel, grid, dim3(width >= 4096 ? 1024 : (width >= 2048 ? 512 : 256)), 0, stream,
-                       (float*)h, (const uint16_t*)delta, w, w_dtype, (uint16_t*)out, rows, row_width, width, eps);
+#define VEC4(NV, THREADS)                                                                                         \
+  hipLaunchKernelGGL(add_rmsnorm_vec4_kernel<NV>, grid, dim3(THREADS), 0, stream, (float*)h, (const uint16_t*)delta, w, \
+                     w_dtype, (uint16_t*)out, rows, row_width, width, eps)
+    if (width <= 1024) VEC4(1, 256);
+    else if (width <= 2048) VEC4(1, 512);
+    else if (width <= 4096) VEC4(2, 512);
+    else if (width <= 8192) VEC4(2, 1024);
+    else VEC4(4, 1024);
+#undef VEC4
     return ix_check_launch("ix_add_rmsnorm");
   }
   if (delta_dtype == IX_F32 && out_dtype == IX_F32) LAUNCH(float, float);

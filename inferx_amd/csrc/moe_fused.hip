@@ -164,6 +164,89 @@ __global__ void moe_combine_add_rmsnorm_vec4_kernel(float* __restrict__ h, const
   }
 }
 
+// The same without a norm of the sum, NV times four columns per thread in registers: the stream, the shared expert's row and
+// the weight are asked for while the row's places among the experts' are looked up, those eight at a time (one after the
+// other, through LDS: 2,048 rows of 2,048 from four experts 20.4 us, now 16.1; eight rows 5.6, now 4.7).
+#define CMB_SLOTS 8
+template <int NV>
+__global__ void __launch_bounds__(1024)
+moe_combine_add_rmsnorm_rows_kernel(float* __restrict__ h, const uint16_t* __restrict__ y, const int32_t* __restrict__ dest,
+                                    const float* __restrict__ topk_w, const uint16_t* __restrict__ shared,
+                                    const float* __restrict__ shared_gate, const void* __restrict__ w, int w_dtype,
+                                    uint16_t* __restrict__ out, const int32_t* __restrict__ rows, int64_t row_width,
+                                    int64_t width, int k, float eps) {
+  __shared__ float red[16];
+  const int64_t r = blockIdx.x;
+  const int64_t row = rows ? rows[r] : r;
+  const int64_t first = blockIdx.y * width;
+  float* hr = h + row * row_width + first;
+  const uint16_t* sr = shared ? shared + row * row_width + first : nullptr;
+  const uint16_t* yr = y + first;
+  int64_t at[NV];
+  float4 v[NV], g[NV];
+  uint2 sh[NV];
+#pragma unroll
+  for (int u = 0; u < NV; ++u) {  // (columns past the end: the first ones, not used)
+    const int64_t c = 4 * (threadIdx.x + u * static_cast<int64_t>(blockDim.x));
+    at[u] = c < width ? c : 0;
+    v[u] = *reinterpret_cast<const float4*>(hr + at[u]);
+    sh[u] = sr ? *reinterpret_cast<const uint2*>(sr + at[u]) : make_uint2(0u, 0u);
+    g[u] = ix_load4_rt(w, w_dtype, first + at[u]);
+  }
+  const float sg = shared ? (shared_gate ? shared_gate[row] : 1.0f) : 0.f;
+  float acc[NV][4] = {};
+  for (int s0 = 0; s0 < k; s0 += CMB_SLOTS) {
+    uint2 part[CMB_SLOTS][NV];
+    float sw[CMB_SLOTS];
+#pragma unroll
+    for (int s = 0; s < CMB_SLOTS; ++s) {
+      if (s0 + s >= k) break;
+      sw[s] = topk_w[row * k + s0 + s];
+      const uint16_t* from = yr + static_cast<int64_t>(dest[row * k + s0 + s]) * row_width;
+#pragma unroll
+      for (int u = 0; u < NV; ++u) part[s][u] = *reinterpret_cast<const uint2*>(from + at[u]);
+    }
+#pragma unroll
+    for (int s = 0; s < CMB_SLOTS; ++s) {
+      if (s0 + s >= k) break;
+#pragma unroll
+      for (int u = 0; u < NV; ++u) {
+        float f[4];
+        bf16x4_to_f32(part[s][u], f);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[u][i] += sw[s] * f[i];
+      }
+    }
+  }
+  float sumsq = 0.f;
+#pragma unroll
+  for (int u = 0; u < NV; ++u) {
+    if (sr) {
+      float f[4];
+      bf16x4_to_f32(sh[u], f);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[u][i] += sg * f[i];
+    }
+    v[u].x += acc[u][0]; v[u].y += acc[u][1]; v[u].z += acc[u][2]; v[u].w += acc[u][3];
+    if (4 * (threadIdx.x + u * static_cast<int64_t>(blockDim.x)) < width) {
+      sumsq += v[u].x * v[u].x;
+      sumsq += v[u].y * v[u].y;
+      sumsq += v[u].z * v[u].z;
+      sumsq += v[u].w * v[u].w;
+    }
+  }
+  sumsq = ix_block_sum(sumsq, red);
+  const float inv = 1.0f / sqrtf(sumsq / static_cast<float>(width) + eps);
+#pragma unroll
+  for (int u = 0; u < NV; ++u) {
+    const int64_t c = 4 * (threadIdx.x + u * static_cast<int64_t>(blockDim.x));
+    if (c >= width) continue;
+    if (!rows) *reinterpret_cast<float4*>(hr + c) = v[u];
+    *reinterpret_cast<uint2*>(out + r * row_width + first + c) =
+        ix_pack4_bf16(make_float4(v[u].x * inv * g[u].x, v[u].y * inv * g[u].y, v[u].z * inv * g[u].z, v[u].w * inv * g[u].w));
+  }
+}
+
 extern "C" int ix_moe_combine_add_rmsnorm(void* h, const void* y, int dtype, const int32_t* dest,
                                           const float* topk_w, const void* shared, const float* shared_gate,
                                           const void* w, int w_dtype, void* out, const int32_t* rows,
@@ -184,7 +267,18 @@ extern "C" int ix_moe_combine_add_rmsnorm(void* h, const void* y, int dtype, con
     hipLaunchKernelGGL(moe_combine_add_rmsnorm_kernel<float>, grid, block, smem, stream, (float*)h, (const float*)y,
                        dest, topk_w, (const float*)shared, shared_gate, w, w_dtype, (float*)out, rows, row_width, width, k, eps,
                        wd, wd_dtype, eps_d);
-  else if (dtype == IX_BF16 && width % 4 == 0 &&
+  else if (dtype == IX_BF16 && width % 4 == 0 && wd == nullptr && width <= 8192 &&
+           ((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(shared) |
+             reinterpret_cast<uintptr_t>(out)) & 15) == 0) {
+#define ROWS(NV, THREADS)                                                                                             \
+  hipLaunchKernelGGL(moe_combine_add_rmsnorm_rows_kernel<NV>, grid, dim3(THREADS), 0, stream, (float*)h, (const uint16_t*)y, \
+                     dest, topk_w, (const uint16_t*)shared, shared_gate, w, w_dtype, (uint16_t*)out, rows, row_width, width, k, eps)
+    if (width <= 1024) ROWS(1, 256);
+    else if (width <= 2048) ROWS(1, 512);
+    else if (width <= 4096) ROWS(2, 512);
+    else ROWS(2, 1024);
+#undef ROWS
+  } else if (dtype == IX_BF16 && width % 4 == 0 &&
            ((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(shared) |
              reinterpret_cast<uintptr_t>(out)) & 15) == 0)
     hipLaunchKernelGGL(moe_combine_add_rmsnorm_vec4_kernel, grid, dim3(width >= 4096 ? 1024 : (width >= 2048 ? 512 : 256)),

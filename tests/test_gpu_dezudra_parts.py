@@ -75,7 +75,7 @@ def run_in_steps(run_step, state_tensors):
 
 # ---- the norm of a branch's result, the add and the next norm in one kernel --------------------------------------
 @pytest.mark.parametrize("dtype,tol", TYPES)
-@pytest.mark.parametrize("width", [40, 258, 1000])
+@pytest.mark.parametrize("width", [40, 258, 1000, 1028, 2052, 4100, 8196])
 def test_normed_branch_add_and_norm(dtype, tol, width):
     from inferx_amd import ops
     T = 7

@@ -490,7 +490,8 @@ def test_routed_and_shared_experts_in_one_launch(T, H, E, k, mi, S):
         assert rel_err(y2, grouped_reference(act2, w2, offsets.cpu(), None, False)) < 1.5e-2
 
 
-@pytest.mark.parametrize("T,H,k,A", [(1, 64, 2, 2), (8, 2048, 4, 32), (21, 96, 3, 70), (5, 1000, 1, 5), (130, 72, 8, 1040)])
+@pytest.mark.parametrize("T,H,k,A", [(1, 64, 2, 2), (8, 2048, 4, 32), (21, 96, 3, 70), (5, 1000, 1, 5), (130, 72, 8, 1040),
+                                      (4, 2052, 9, 40), (3, 4100, 12, 40), (3, 8196, 2, 9)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("with_shared,gated", [(False, False), (True, False), (True, True)])
 def test_expert_sum_add_and_norm_in_one_pass(T, H, k, A, dtype, with_shared, gated):

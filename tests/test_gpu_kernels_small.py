@@ -38,7 +38,8 @@ def test_embed(dtype):
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("wdtype", DTYPES)
-@pytest.mark.parametrize("T,H,eps", [(5, 72, 1e-5), (3, 2048, 1e-6), (2, 5000, 1e-6)])
+@pytest.mark.parametrize("T,H,eps", [(5, 72, 1e-5), (3, 2048, 1e-6), (2, 5000, 1e-6), (2, 1028, 1e-6), (3, 2052, 1e-6),
+                                     (2, 16384, 1e-6), (2, 16388, 1e-6)])
 def test_add_rmsnorm(dtype, wdtype, T, H, eps):
     from inferx_amd import ops
     h0, delta, w = rnd(T, H), rnd(T, H, seed=1, dtype=dtype), rnd(H, seed=2, dtype=wdtype)

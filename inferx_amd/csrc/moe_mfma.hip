@@ -68,7 +68,10 @@ template <> struct MfmaPiece<float> {
 // The work of one wavefront (KSPLIT == 1) or workgroup (KSPLIT > 1): rows [row0, row_end) x out-features
 // [n0, n0 + 16) of expert e.  `lds`: IX_TURN_BYTES for each wavefront; the partial sums of a split reduction go the same
 // way.  NB: blocks of 16 out-features side by side ([n0, n0 + 16 NB)), so that the rows are read once for all of them.
-template <int MT, bool GATE_UP, int KSPLIT, typename TI, typename TO, int NB = 1>
+// HALVES (up to eight rows, MT = NB = 1, width a multiple of two pieces): eight out-features; a block's second eight weight
+// rows are the same features' second half of the reduction, and its second eight columns the rows' second halves, so that
+// the sums meet on the diagonal of the 16 x 16 block and twice as many workgroups share few features.
+template <int MT, bool GATE_UP, int KSPLIT, typename TI, typename TO, int NB = 1, bool HALVES = false>
 __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
                                              TO* __restrict__ out, const int32_t* __restrict__ rows, int e,
                                              int row0, int row_end, int n0, int n_out, int width, char* lds,
@@ -80,9 +83,11 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
   constexpr int NACC = NB * (GATE_UP ? 2 : 1);  // accumulator b + NB h: block b of the gate (h = 0) or up (1) rows
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
-  const int kper = KSPLIT > 1 ? (((width + KSPLIT - 1) / KSPLIT + ROUND - 1) & ~(ROUND - 1)) : width;
+  static_assert(!HALVES || (MT == 1 && NB == 1 && !GATE_UP), "two halves of one block");
+  const int span = HALVES ? width / 2 : width;  // the reduction as the matrix cores see it
+  const int kper = KSPLIT > 1 ? (((span + KSPLIT - 1) / KSPLIT + ROUND - 1) & ~(ROUND - 1)) : span;
   const int kbegin = KSPLIT > 1 ? wave * kper : 0;
-  const int kend = min(width, kbegin + kper);
+  const int kend = min(span, kbegin + kper);
 
   const int64_t w_rows = GATE_UP ? 2 * static_cast<int64_t>(n_out) : n_out;
   // In load j lane l reads piece 8 (j / 2) + l % 8 of row 8 (j % 2) + l / 8: whole lines of 128 bytes.  (A block's rows
@@ -96,7 +101,8 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
     if (u < NB)
 #pragma unroll
       for (int h = 0; h < 2; ++h)
-        wrow[u][h] = static_cast<unsigned>(min(8 * h + (lane >> 3), n_out - 1 - first)) * static_cast<unsigned>(width) * sizeof(TI);
+        wrow[u][h] = (static_cast<unsigned>(min((HALVES ? 0 : 8 * h) + (lane >> 3), n_out - 1 - first)) * static_cast<unsigned>(width) +
+                      (HALVES && h ? span : 0)) * sizeof(TI);
   }
   // Piece p of row r of a round lies at piece p ^ (r / 2 + 8 (r % 2)) of its 256 bytes: the rows that sixteen lanes read at
   // one piece, and the pieces of two rows that they write, fall on sixteen different groups of four banks.
@@ -106,8 +112,8 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
   const TI* xr[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
-    const int r = min(row0 + 16 * t + m, row_end - 1);
-    xr[t] = a + static_cast<int64_t>(rows ? rows[r] : r) * width;
+    const int r = min(row0 + 16 * t + (HALVES ? m & 7 : m), row_end - 1);
+    xr[t] = a + static_cast<int64_t>(rows ? rows[r] : r) * width + (HALVES && m >= 8 ? span : 0);
   }
 
   f32x4 acc[NACC][MT];
@@ -219,6 +225,11 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
     }
   }
 
+  if constexpr (HALVES) {  // lanes of features and rows below eight: the other halves' sums are eight further on in both
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[0][0][i] += __shfl(acc[0][0][i], lane + 40, 64);
+    if (m >= 8 || g >= 2) return;
+  }
   // lane holds out-features n0 + 16 u + 4 g + i of row row0 + 16 t + m
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
@@ -259,13 +270,13 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
 
 // x [rows <= 16 * MT, width] . w^T -> [rows, n_out], the products of a decoding step: 16 NB out-features a workgroup, the
 // reduction split over its KSPLIT wavefronts.
-template <int MT, bool GATE_UP, int KSPLIT, int NB, typename TI, typename TO>
+template <int MT, bool GATE_UP, int KSPLIT, int NB, typename TI, typename TO, bool HALVES = false>
 __global__ void __launch_bounds__(64 * KSPLIT, MT > 1 ? 1 : NB * (GATE_UP ? 2 : 1) > 1 ? 3 : 4)
 linear_skinny_kernel(const TI* x, const TI* w, TO* __restrict__ out, const void* bias, int bias_dtype, int rows, int n_out,
                      int width, float glu_limit) {
   __shared__ __attribute__((aligned(16))) char lds[KSPLIT * IX_TURN_BYTES(NB * (GATE_UP ? 2 : 1))];
-  grouped_body<MT, GATE_UP, KSPLIT, TI, TO, NB>(x, w, out, nullptr, 0, 0, rows, blockIdx.x * 16 * NB, n_out, width, lds, 0,
-                                                glu_limit, bias, bias_dtype);
+  grouped_body<MT, GATE_UP, KSPLIT, TI, TO, NB, HALVES>(x, w, out, nullptr, 0, 0, rows, blockIdx.x * (HALVES ? 8 : 16 * NB),
+                                                        n_out, width, lds, 0, glu_limit, bias, bias_dtype);
 }
 
 template <int MT, bool GATE_UP, int KSPLIT, typename TI>
@@ -408,7 +419,9 @@ extern "C" int ix_moe_grouped_dual(const void* a, const void* w, void* out, int 
 // units eight wavefronts split its reduction instead of four.  The float32 result (the logits) has so many out-features
 // that 32 a workgroup are better: the rows, which every workgroup reads, weigh less beside the weights.
 // Eight rows: 2,048 features of 2,048 numbers 4.9 us, of 5,632 9.6 (11.7 before whole lines were read), 11,264 features of
-// 2,048 10.9 (14.6); a gated unit with biases saves the launch behind it, 6.2 us.
+// 2,048 10.9 (14.6); a gated unit with biases saves the launch behind it, 6.2 us.  With eight features a workgroup (HALVES), one
+// | eight rows, where sixteen took nine rows: 2,048 features of 2,048 3.7 | 4.3 (4.7), of 5,632 6.2 | 8.1 (9.1), 256 of 8,192
+// 5.2 | 7.9 (10.0); float32 5.7 | 6.8 (7.8), 10.8 | 13.1 (15.8), 9.4 | 13.8 (19.7).
 extern "C" int ix_linear_skinny(const void* x, const void* w, int dtype, void* out, int out_f32, const void* bias,
                                 int bias_dtype, int rows, int64_t n_out, int64_t width, int gate_up, float glu_limit,
                                 hipStream_t stream) {
@@ -435,6 +448,18 @@ extern "C" int ix_linear_skinny(const void* x, const void* w, int dtype, void* o
   if (rows <= 16) LAUNCH(1, false, 4, 2, TI, float);            \
   else if (rows <= 32) LAUNCH(2, false, 4, 2, TI, float);       \
   else LAUNCH(4, false, 4, 2, TI, float)
+  // Few features for few rows: eight of them a workgroup where sixteen leave half the compute units without one.
+  const int piece = dtype == IX_F32 ? 4 : 8;
+  if (!out_f32 && !gate_up && rows <= 8 && blocks <= 128 && width % (2 * piece) == 0) {
+    const dim3 grid8(static_cast<unsigned>((n_out + 7) / 8));
+    if (dtype == IX_F32)
+      hipLaunchKernelGGL((linear_skinny_kernel<1, false, 8, 1, float, float, true>), grid8, dim3(512), 0, stream, (const float*)x,
+                         (const float*)w, (float*)out, bias, bias_dtype, rows, (int)n_out, (int)width, glu_limit);
+    else
+      hipLaunchKernelGGL((linear_skinny_kernel<1, false, 8, 1, __bf16, __bf16, true>), grid8, dim3(512), 0, stream, (const __bf16*)x,
+                         (const __bf16*)w, (__bf16*)out, bias, bias_dtype, rows, (int)n_out, (int)width, glu_limit);
+    return ix_check_launch("ix_linear_skinny");
+  }
   if (out_f32 && dtype == IX_F32) { LOGITS(float); }
   else if (out_f32) { LOGITS(__bf16); }
   else if (dtype == IX_F32) { BY_ROWS(float) }

@@ -70,7 +70,8 @@ template <> struct MfmaPiece<float> {
 // way.  NB: blocks of 16 out-features side by side ([n0, n0 + 16 NB)), so that the rows are read once for all of them.
 // HALVES (up to eight rows, MT = NB = 1, width a multiple of two pieces): eight out-features; a block's second eight weight
 // rows are the same features' second half of the reduction, and its second eight columns the rows' second halves, so that
-// the sums meet on the diagonal of the 16 x 16 block and twice as many workgroups share few features.
+// the sums meet on the diagonal of the 16 x 16 block and twice as many workgroups share few features.  Of a gated product
+// (NB = 1) the second eight weight rows are the eight features' up rows, over the whole reduction and for any rows.
 template <int MT, bool GATE_UP, int KSPLIT, typename TI, typename TO, int NB = 1, bool HALVES = false>
 __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
                                              TO* __restrict__ out, const int32_t* __restrict__ rows, int e,
@@ -80,11 +81,12 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
   typedef MfmaPiece<TI> Piece;
   typedef typename Piece::type piece_t;
   constexpr int PN = Piece::N, ROUND = 16 * PN;  // numbers of a piece; of a round of four loads
-  constexpr int NACC = NB * (GATE_UP ? 2 : 1);  // accumulator b + NB h: block b of the gate (h = 0) or up (1) rows
+  constexpr bool UP8 = HALVES && GATE_UP;
+  constexpr int NACC = NB * (GATE_UP && !UP8 ? 2 : 1);  // accumulator b + NB h: block b of the gate (h = 0) or up (1) rows
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m = lane & 15, g = lane >> 4;
-  static_assert(!HALVES || (MT == 1 && NB == 1 && !GATE_UP), "two halves of one block");
-  const int span = HALVES ? width / 2 : width;  // the reduction as the matrix cores see it
+  static_assert(!HALVES || (NB == 1 && (MT == 1 || GATE_UP)), "two halves of one block");
+  const int span = HALVES && !GATE_UP ? width / 2 : width;  // the reduction as the matrix cores see it
   const int kper = KSPLIT > 1 ? (((span + KSPLIT - 1) / KSPLIT + ROUND - 1) & ~(ROUND - 1)) : span;
   const int kbegin = KSPLIT > 1 ? wave * kper : 0;
   const int kend = min(span, kbegin + kper);
@@ -102,8 +104,9 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
 #pragma unroll
       for (int h = 0; h < 2; ++h)
         wrow[u][h] = (static_cast<unsigned>(min((HALVES ? 0 : 8 * h) + (lane >> 3), n_out - 1 - first)) * static_cast<unsigned>(width) +
-                      (HALVES && h ? span : 0)) * sizeof(TI);
+                      (HALVES && !GATE_UP && h ? span : 0)) * sizeof(TI);
   }
+  const char* const wup = UP8 ? wbase[0] + static_cast<int64_t>(n_out) * width * sizeof(TI) : nullptr;
   // Piece p of row r of a round lies at piece p ^ (r / 2 + 8 (r % 2)) of its 256 bytes: the rows that sixteen lanes read at
   // one piece, and the pieces of two rows that they write, fall on sixteen different groups of four banks.
   char* const turn = lds + wave * IX_TURN_BYTES(NACC);
@@ -112,8 +115,8 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
   const TI* xr[MT];
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
-    const int r = min(row0 + 16 * t + (HALVES ? m & 7 : m), row_end - 1);
-    xr[t] = a + static_cast<int64_t>(rows ? rows[r] : r) * width + (HALVES && m >= 8 ? span : 0);
+    const int r = min(row0 + 16 * t + (HALVES && !GATE_UP ? m & 7 : m), row_end - 1);
+    xr[t] = a + static_cast<int64_t>(rows ? rows[r] : r) * width + (HALVES && !GATE_UP && m >= 8 ? span : 0);
   }
 
   f32x4 acc[NACC][MT];
@@ -139,7 +142,7 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
 #pragma unroll
       for (int u = 0; u < NACC; ++u)
         w_[u][j] = __builtin_nontemporal_load(
-            reinterpret_cast<const piece_t*>(wbase[u] + (wrow[u % NB][j & 1] + static_cast<unsigned>(kw) * sizeof(TI))));
+            reinterpret_cast<const piece_t*>((UP8 && (j & 1) ? wup : wbase[u]) + (wrow[u % NB][j & 1] + static_cast<unsigned>(kw) * sizeof(TI))));
 #pragma unroll
       for (int t = 0; t < MT; ++t) x_[t][j] = *reinterpret_cast<const piece_t*>(xr[t] + kk);
     }
@@ -225,7 +228,14 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
     }
   }
 
-  if constexpr (HALVES) {  // lanes of features and rows below eight: the other halves' sums are eight further on in both
+  float ups[UP8 ? MT : 1][4];
+  if constexpr (UP8) {  // lanes of the gate's rows: the up rows' sums are eight rows further on
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ups[t][i] = __shfl_xor(acc[0][t][i], 32, 64);
+    if (g >= 2) return;
+  } else if constexpr (HALVES) {  // lanes of features and rows below eight: the other halves' sums are eight further on in both
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[0][0][i] += __shfl(acc[0][0][i], lane + 40, 64);
     if (m >= 8 || g >= 2) return;
@@ -245,7 +255,7 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
         const int c = min(nb + i, n_out - 1);
         if (bias) v[i] += ix_load_rt(bias, bias_dtype, c);
         if constexpr (GATE_UP) {
-          float up = acc[NB + u][t][i];
+          float up = UP8 ? ups[UP8 ? t : 0][i] : acc[UP8 ? 0 : NB + u][t][i];
           if (bias) up += ix_load_rt(bias, bias_dtype, static_cast<int64_t>(n_out) + c);
           v[i] = ix_glu<sizeof(TI) == 2>(v[i], up, glu_limit);
         }
@@ -271,10 +281,10 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
 // x [rows <= 16 * MT, width] . w^T -> [rows, n_out], the products of a decoding step: 16 NB out-features a workgroup, the
 // reduction split over its KSPLIT wavefronts.
 template <int MT, bool GATE_UP, int KSPLIT, int NB, typename TI, typename TO, bool HALVES = false>
-__global__ void __launch_bounds__(64 * KSPLIT, MT > 1 ? 1 : NB * (GATE_UP ? 2 : 1) > 1 ? 3 : 4)
+__global__ void __launch_bounds__(64 * KSPLIT, MT > 1 ? 1 : NB * (GATE_UP && !HALVES ? 2 : 1) > 1 ? 3 : 4)
 linear_skinny_kernel(const TI* x, const TI* w, TO* __restrict__ out, const void* bias, int bias_dtype, int rows, int n_out,
                      int width, float glu_limit) {
-  __shared__ __attribute__((aligned(16))) char lds[KSPLIT * IX_TURN_BYTES(NB * (GATE_UP ? 2 : 1))];
+  __shared__ __attribute__((aligned(16))) char lds[KSPLIT * IX_TURN_BYTES(NB * (GATE_UP && !HALVES ? 2 : 1))];
   grouped_body<MT, GATE_UP, KSPLIT, TI, TO, NB, HALVES>(x, w, out, nullptr, 0, 0, rows, blockIdx.x * (HALVES ? 8 : 16 * NB),
                                                         n_out, width, lds, 0, glu_limit, bias, bias_dtype);
 }
@@ -457,6 +467,19 @@ extern "C" int ix_linear_skinny(const void* x, const void* w, int dtype, void* o
                          (const float*)w, (float*)out, bias, bias_dtype, rows, (int)n_out, (int)width, glu_limit);
     else
       hipLaunchKernelGGL((linear_skinny_kernel<1, false, 8, 1, __bf16, __bf16, true>), grid8, dim3(512), 0, stream, (const __bf16*)x,
+                         (const __bf16*)w, (__bf16*)out, bias, bias_dtype, rows, (int)n_out, (int)width, glu_limit);
+    return ix_check_launch("ix_linear_skinny");
+  }
+  // A gated product with between one and two blocks of sixteen for a compute unit: some have two of them and most one, and
+  // eights even that out.  One | eight rows of 2,048 numbers, us: 5,632 features 9.5 | 10.5 (10.3 | 11.2), 6,144 9.8 | 10.7 (11.2 |
+  // 12.5); no gain from two blocks a compute unit on (8,192: 12.2 | 13.0 (12.4 | 12.8)), where the rows weigh more.
+  if (!out_f32 && gate_up && rows <= 8 && blocks > 256 && blocks < 448) {
+    const dim3 grid8(static_cast<unsigned>((n_out + 7) / 8));
+    if (dtype == IX_F32)
+      hipLaunchKernelGGL((linear_skinny_kernel<1, true, 4, 1, float, float, true>), grid8, dim3(256), 0, stream, (const float*)x,
+                         (const float*)w, (float*)out, bias, bias_dtype, rows, (int)n_out, (int)width, glu_limit);
+    else
+      hipLaunchKernelGGL((linear_skinny_kernel<1, true, 4, 1, __bf16, __bf16, true>), grid8, dim3(256), 0, stream, (const __bf16*)x,
                          (const __bf16*)w, (__bf16*)out, bias, bias_dtype, rows, (int)n_out, (int)width, glu_limit);
     return ix_check_launch("ix_linear_skinny");
   }

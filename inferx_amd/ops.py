@@ -1813,6 +1813,27 @@ def latent_mfma_fits(q_lat: torch.Tensor, q_rot: torch.Tensor, out: torch.Tensor
                 or (out.stride(0) | out.stride(1)) % 4)
 
 
+HEADS_PRODUCT_TOKENS = 16
+
+
+def heads_product_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether `heads_product` takes these operands."""
+    return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and 0 < x.shape[0] <= HEADS_PRODUCT_TOKENS
+            and w.is_contiguous() and w.shape[1] % 16 == 0 and w.shape[2] % 32 == 0 and x.stride(2) == 1
+            and x.stride(0) % 8 == 0 and x.stride(1) % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+
+def heads_product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
+    """out[t, h] = w[h] . x[t, h] for the few tokens of a decoding step: x [T, heads, width], w [heads, n, width], out
+    [T, heads, n], bfloat16 (see `heads_product_fits`); rows of x and out may have any strides of whole pieces."""
+    T, heads, width = x.shape
+    n = w.shape[1]
+    _need(heads_product_fits(x, w) and w.shape == (heads, n, width), "operands that the kernel does not take")
+    _need(out.shape == (T, heads, n) and out.dtype == x.dtype and out.stride(2) == 1, "out must be bfloat16 [T, heads, n]")
+    _call("ix_heads_product", x.data_ptr(), _i64(x.stride(0)), _i64(x.stride(1)), w.data_ptr(), out.data_ptr(),
+          _i64(out.stride(0)), _i64(out.stride(1)), _i32(T), _i32(heads), _i32(n), _i32(width), _stream())
+
+
 def latent_mfma_splits(tokens: int, heads: int) -> int:
     """Into how many slices a step of one token per request cuts every request's keys: enough workgroups for the
     compute units, whatever the contexts (a captured step keeps its number)."""

@@ -319,6 +319,22 @@ def test_clamped_gated_unit_with_biases(dtype, tol, limit):
     assert float((act.cpu().double() - want).abs().max()) <= tol * float(want.abs().max())
 
 
+@pytest.mark.parametrize("T", [1, 8, 16])
+@pytest.mark.parametrize("H,n,width", [(16, 512, 128), (3, 16, 32), (5, 48, 160), (2, 128, 512), (1, 80, 1056)])
+def test_product_of_every_head(T, H, n, width):
+    """Rows with strides of their own on both sides, what lies between and behind them not-a-number.  The bound is the
+    result's own rounding and that of `width` float32 sums."""
+    from inferx_amd import ops
+    x = torch.full((T, H, width + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
+    x[:, :, :width] = rnd((T, H, width), 1, 1.0, torch.bfloat16).to(DEV)
+    w = rnd((H, n, width), 2, width ** -0.5, torch.bfloat16).to(DEV)
+    out = torch.full((H, T, n), float("nan"), dtype=torch.bfloat16, device=DEV).transpose(0, 1)
+    assert ops.heads_product_fits(x[:, :, :width], w)
+    ops.heads_product(x[:, :, :width], w, out)
+    want = (w.double()[None] * x[:, :, None, :width].double()).sum(-1)
+    assert float(((out.double() - want).abs() - 2.0 ** -8 * want.abs()).max()) <= 4e-5
+
+
 @pytest.mark.parametrize("bias", ["bfloat16", "float32", "bfloat16 off a boundary"])
 def test_clamped_gated_unit_of_many_rows(bias):
     """More rows than lines of workgroups (512), a width of 257 pieces of eight; a bias of either type, also one that does

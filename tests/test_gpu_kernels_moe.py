@@ -343,7 +343,7 @@ def test_grouped_tiled_last_tiles_of_one_expert_together(T, E, mi, pieces, wide)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T", [1, 8, 17, 64])
 # at most 256 blocks of sixteen, and more; at most 128 (both halves of an even reduction in one block for up to eight rows)
-@pytest.mark.parametrize("N,K", [(33, 8), (4096, 1160), (4100, 264), (2048, 1040), (37, 16), (43, 2064)])
+@pytest.mark.parametrize("N,K", [(33, 8), (4096, 1160), (4100, 264), (2048, 1040), (37, 16), (43, 2064), (5637, 72)])
 @pytest.mark.parametrize("form", [None, 0.0, 1.5, -1.0])  # a plain product; gate|up rows by the unit's limit
 @pytest.mark.parametrize("biased", [False, True])
 def test_dense_products_of_few_rows(dtype, T, N, K, form, biased):

@@ -29,6 +29,8 @@
 // 448 + 64 155 | 73 (353 | 137), 256 + 64 118 | 46 (216 | 88), 128 + 64 112 | 39 (163 | 69), 64 + 32 85 | 22 (109 | 25),
 // 32 + 32 85 | 20.5 (86 | 21).  One form of 78 KB of LDS for all sizes took 113 | 35 and 111 | 33 us at the last two;
 // branches past the products that a smaller row does without, 258 | 104 us at 448 + 64.
+// With masks only where a column needs one, and no exchange between a column's lanes unless its maximum has outgrown the
+// reference point: 512 + 64 140 (157 beside it), 256 + 64 104 (119), 128 + 64 98 (113), 64 + 32 71 (86) for 2,048 tokens.
 #include "common.h"
 
 typedef __bf16 lp_bf16x8 __attribute__((ext_vector_type(8)));
@@ -196,26 +198,34 @@ latent_prefill_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_h,
         }
         float p[8], mx = -INFINITY;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int j = k0 + 8 * g + i;
-          p[i] = (j <= my_pos && j > my_lo) ? (i < 4 ? s0[i & 3] : s1[i & 3]) * scale_log2 : -INFINITY;
-          mx = fmaxf(mx, p[i]);
+        for (int i = 0; i < 8; ++i) p[i] = (i < 4 ? s0[i & 3] : s1[i & 3]) * scale_log2;
+        if (!__all(k0 + LP_KEYS - 1 <= my_pos && k0 > my_lo)) {  // (rounds that every column sees need no mask)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const int j = k0 + 8 * g + i;
+            p[i] = (j <= my_pos && j > my_lo) ? p[i] : -INFINITY;
+          }
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
+#pragma unroll
+        for (int i = 0; i < 8; ++i) mx = fmaxf(mx, p[i]);
         // The reference point m of the exponentials follows the running maximum lazily: a column's moves only when its
-        // maximum has outgrown it by more than 2^8, so the sums are seldom rescaled.  Any m gives the same quotient;
-        // weights up to 2^8 keep the relative precision of bfloat16.
+        // maximum has outgrown it by more than 2^8, so the sums are seldom rescaled, and whether any has needs no exchange
+        // between a column's four lanes.  Any m gives the same quotient; weights up to 2^8 keep the relative precision of
+        // bfloat16.
         float alpha = 1.0f;
-        if (mx > m + 8.f) {
-          alpha = exp2f(m - mx);
-          m = mx;
-          l *= alpha;
+        if (__any(mx > m + 8.f)) {
+          mx = fmaxf(mx, __shfl_xor(mx, 16));
+          mx = fmaxf(mx, __shfl_xor(mx, 32));
+          if (mx > m + 8.f) {
+            alpha = exp2f(m - mx);
+            m = mx;
+            l *= alpha;
+          }
         }
         lp_bf16x8 pb;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          const float w = exp2f(p[i] - m);
+          const float w = __builtin_amdgcn_exp2f(p[i] - m);  // (v_exp_f32 as it is: a result below the smallest normal number may be 0)
           l += w;
           pb[i] = static_cast<__bf16>(w);
         }

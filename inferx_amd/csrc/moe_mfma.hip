@@ -431,7 +431,7 @@ extern "C" int ix_moe_grouped_dual(const void* a, const void* w, void* out, int 
 // Eight rows: 2,048 features of 2,048 numbers 4.9 us, of 5,632 9.6 (11.7 before whole lines were read), 11,264 features of
 // 2,048 10.9 (14.6); a gated unit with biases saves the launch behind it, 6.2 us.  With eight features a workgroup (HALVES), one
 // | eight rows, where sixteen took nine rows: 2,048 features of 2,048 3.7 | 4.3 (4.7), of 5,632 6.2 | 8.1 (9.1), 256 of 8,192
-// 5.2 | 7.9 (10.0); float32 5.7 | 6.8 (7.8), 10.8 | 13.1 (15.8), 9.4 | 13.8 (19.7).
+// 5.2 | 7.9 (10.0).
 extern "C" int ix_linear_skinny(const void* x, const void* w, int dtype, void* out, int out_f32, const void* bias,
                                 int bias_dtype, int rows, int64_t n_out, int64_t width, int gate_up, float glu_limit,
                                 hipStream_t stream) {
@@ -458,16 +458,13 @@ extern "C" int ix_linear_skinny(const void* x, const void* w, int dtype, void* o
   if (rows <= 16) LAUNCH(1, false, 4, 2, TI, float);            \
   else if (rows <= 32) LAUNCH(2, false, 4, 2, TI, float);       \
   else LAUNCH(4, false, 4, 2, TI, float)
-  // Few features for few rows: eight of them a workgroup where sixteen leave half the compute units without one.
-  const int piece = dtype == IX_F32 ? 4 : 8;
-  if (!out_f32 && !gate_up && rows <= 8 && blocks <= 128 && width % (2 * piece) == 0) {
-    const dim3 grid8(static_cast<unsigned>((n_out + 7) / 8));
-    if (dtype == IX_F32)
-      hipLaunchKernelGGL((linear_skinny_kernel<1, false, 8, 1, float, float, true>), grid8, dim3(512), 0, stream, (const float*)x,
-                         (const float*)w, (float*)out, bias, bias_dtype, rows, (int)n_out, (int)width, glu_limit);
-    else
-      hipLaunchKernelGGL((linear_skinny_kernel<1, false, 8, 1, __bf16, __bf16, true>), grid8, dim3(512), 0, stream, (const __bf16*)x,
-                         (const __bf16*)w, (__bf16*)out, bias, bias_dtype, rows, (int)n_out, (int)width, glu_limit);
+  // Few features for few rows: eight of them a workgroup where sixteen leave half the compute units without one.  (bfloat16
+  // only: float32 rows are then summed up in another order in portions of up to eight rows than in longer ones, and two
+  // scores of a router 1.8e-6 apart fell the other way from the 64-bit result.)
+  if (dtype == IX_BF16 && !out_f32 && !gate_up && rows <= 8 && blocks <= 128 && width % 16 == 0) {
+    hipLaunchKernelGGL((linear_skinny_kernel<1, false, 8, 1, __bf16, __bf16, true>), dim3(static_cast<unsigned>((n_out + 7) / 8)),
+                       dim3(512), 0, stream, (const __bf16*)x, (const __bf16*)w, (__bf16*)out, bias, bias_dtype, rows,
+                       (int)n_out, (int)width, glu_limit);
     return ix_check_launch("ix_linear_skinny");
   }
   // A gated product with between one and two blocks of sixteen for a compute unit: some have two of them and most one, and

@@ -512,6 +512,7 @@ def decode_slices(units: int, longest: int, span: int) -> int:
     wavefront walks a long context while the others are done.  64 requests of 200 to 2,048 tokens in 2, 4 and 8 slices:
     85, 78 and 78 us; 64 of 2,048 each: 164, 168 and 172.  A power of two; at most 64, and 16,384 wavefronts (the parts'
     room)."""
+    longest = 1 << max(longest - 1, 0).bit_length()  # as captured steps round it: a step and its replay are cut alike
     keys = min(longest, abs(span) + QUERY_TILE + 32) if span else longest
     by_keys = max(-(-keys // MIN_KEYS_PER_SPLIT), min(-(-keys // 64), 32) if units <= 16 else 1)
     by_length = min(-(-keys // 512), 8 * WAVES_WANTED // max(1, units))

@@ -3,36 +3,37 @@
 //
 // What bounds it: the launch and one trip to memory (16 heads of 512 x 128: 2 MB of weights).  A wavefront takes sixteen rows
 // of a head's weights over the whole reduction, as the first operand of v_mfma_f32_16x16x32_bf16, the tokens are the
-// columns; 128 numbers of the reduction are asked for at once.  Eight tokens, 16 heads of 512 x 128: 3.5 us
-// against 10.6 of the library's batched product, which takes a workgroup a head.
+// columns; up to 512 numbers of the reduction are asked for at once, and with few wavefronts each is a workgroup of its own.
+// Eight tokens, 16 heads of 512 x 128 | 128 x 512: 3.2 | 3.7 us against 5.0 | 10.6 of the library's batched product.
 #include "common.h"
 
 typedef __bf16 hp_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 hp_bf16x4 __attribute__((ext_vector_type(4)));
 typedef float hp_f32x4 __attribute__((ext_vector_type(4)));
 
-#define HP_STEPS 4  // pieces of 32 of the reduction that are on their way together
+// STEPS: pieces of 32 of the reduction that are on their way together
+template <int STEPS>
 __global__ void __launch_bounds__(256)
 heads_product_kernel(const __bf16* __restrict__ x, int64_t x_t, int64_t x_h, const __bf16* __restrict__ w,
                      __bf16* __restrict__ out, int64_t out_t, int64_t out_h, int tokens, int heads, int n, int width) {
   const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
   const int per_head = n / 16;
-  const int64_t unit = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int64_t unit = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (unit >= static_cast<int64_t>(heads) * per_head) return;
   const int head = static_cast<int>(unit / per_head), row0 = 16 * static_cast<int>(unit % per_head);
   const __bf16* wr = w + (static_cast<int64_t>(head) * n + row0 + m) * width;
   const __bf16* xr = x + min(m, tokens - 1) * x_t + head * x_h;  // (columns past the last token: that one, not stored)
   hp_f32x4 acc = hp_f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < width; k0 += 32 * HP_STEPS) {
-    hp_bf16x8 wv[HP_STEPS], xv[HP_STEPS];
+  for (int k0 = 0; k0 < width; k0 += 32 * STEPS) {
+    hp_bf16x8 wv[STEPS], xv[STEPS];
 #pragma unroll
-    for (int s = 0; s < HP_STEPS; ++s) {
+    for (int s = 0; s < STEPS; ++s) {
       const int k = min(k0 + 32 * s, width - 32) + 8 * g;
       wv[s] = *reinterpret_cast<const hp_bf16x8*>(wr + k);
       xv[s] = *reinterpret_cast<const hp_bf16x8*>(xr + k);
     }
 #pragma unroll
-    for (int s = 0; s < HP_STEPS; ++s)
+    for (int s = 0; s < STEPS; ++s)
       if (k0 + 32 * s < width) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[s], xv[s], acc, 0, 0, 0);
   }
   // lane holds weight rows row0 + 4 g + i of token m
@@ -49,9 +50,14 @@ extern "C" int ix_heads_product(const void* x, int64_t x_t, int64_t x_h, const v
              "operands must lie on 16-byte boundaries");
   IX_REQUIRE((reinterpret_cast<uintptr_t>(out) & 7) == 0 && (out_t | out_h) % 4 == 0, "out must lie on 8-byte boundaries");
   const int64_t units = static_cast<int64_t>(heads) * (n / 16);
-  IX_REQUIRE((units + 3) / 4 < (int64_t(1) << 31), "too many rows of weights for one launch");
-  const dim3 grid(static_cast<unsigned>((units + 3) / 4));
-  hipLaunchKernelGGL(heads_product_kernel, grid, dim3(256), 0, stream, (const __bf16*)x, x_t, x_h, (const __bf16*)w,
-                     (__bf16*)out, out_t, out_h, tokens, heads, n, width);
+  IX_REQUIRE(units < (int64_t(1) << 31), "too many rows of weights for one launch");
+  const unsigned per_group = units < 1024 ? 1 : 4;
+  const dim3 grid(static_cast<unsigned>((units + per_group - 1) / per_group));
+#define LAUNCH(STEPS)                                                                                                        \
+  hipLaunchKernelGGL(heads_product_kernel<STEPS>, grid, dim3(64 * per_group), 0, stream, (const __bf16*)x, x_t, x_h,          \
+                     (const __bf16*)w, (__bf16*)out, out_t, out_h, tokens, heads, n, width)
+  if (width <= 128) LAUNCH(4);
+  else LAUNCH(16);
+#undef LAUNCH
   return ix_check_launch("ix_heads_product");
 }

@@ -99,10 +99,11 @@ class LatentAttention(Mixer):
             rows.append(rows[-1].new_zeros((odd, self.hidden_size)))
         self.w_in = stack_rows(rows)
         self.w_uk = uk.contiguous().view(H, self.head_dim, self.rank)
-        # [H, rank, head_dim]: the reduction's numbers side by side, for steps of few tokens (the other product, of few rows and
-        # long reductions, is as quick through the library: 5.0 against 5.7 us at eight tokens, 16 heads of 128 x 512)
-        self.w_uk_rows = self.w_uk.transpose(1, 2).contiguous() if rt.dtype == torch.bfloat16 else None
-        self.w_uv_t = uv.contiguous().view(H, self.value_dim, self.rank).transpose(1, 2).contiguous()
+        w_uv = uv.contiguous().view(H, self.value_dim, self.rank)
+        self.w_uv_t = w_uv.transpose(1, 2).contiguous()
+        # the same with the reduction's numbers side by side, for steps of few tokens: [H, rank, head_dim], [H, value_dim, rank]
+        few = rt.dtype == torch.bfloat16
+        self.w_uk_rows, self.w_uv_rows = (self.w_uk.transpose(1, 2).contiguous(), w_uv) if few else (None, None)
         self.w_out = tensors["o.weight"].contiguous()
         self.norm_weight = norm.contiguous()
         if self.position is not None:
@@ -133,7 +134,11 @@ class LatentAttention(Mixer):
         # (without a rotated part nothing is read of it: any rows will do)
         self.attend(ctx, q_lat, q3[:, :, self.head_dim:] if self.rot_dim else q_lat, cache, o_lat.transpose(0, 1), gate)
         y = rt.empty((T, H * self.value_dim))
-        torch.bmm(o_lat, self.w_uv_t, out=y.view(T, H, self.value_dim).transpose(0, 1))
+        o_own, y_heads = o_lat.transpose(0, 1), y.view(T, H, self.value_dim)
+        if self.w_uv_rows is not None and ops.heads_product_fits(o_own, self.w_uv_rows):
+            ops.heads_product(o_own, self.w_uv_rows, y_heads)
+        else:
+            torch.bmm(o_lat, self.w_uv_t, out=y_heads.transpose(0, 1))
         if self.has_gate:
             ops.sigmoid_gate(y, proj[:, at:])
         return rt.linear(y, self.w_out)

@@ -1818,7 +1818,7 @@ HEADS_PRODUCT_TOKENS = 16
 
 def heads_product_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether `heads_product` takes these operands."""
-    return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and 0 < x.shape[0] <= HEADS_PRODUCT_TOKENS
+    return (0 < x.shape[0] <= HEADS_PRODUCT_TOKENS and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and w.is_contiguous() and w.shape[1] % 16 == 0 and w.shape[2] % 32 == 0 and x.stride(2) == 1
             and x.stride(0) % 8 == 0 and x.stride(1) % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 

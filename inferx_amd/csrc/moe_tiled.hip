@@ -338,7 +338,8 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
   const int n_tiles = tile_info[0];
   const unsigned die = blockIdx.x & 7, i = blockIdx.x >> 3;
   const bool spread = last_tiles > 0 && last_tiles < n_tiles;
-  const unsigned light = static_cast<unsigned>(spread ? n_tiles - last_tiles : n_tiles) * n_col_blocks;
+  const int n_light = spread ? n_tiles - last_tiles : n_tiles;
+  const unsigned light = static_cast<unsigned>(n_light) * n_col_blocks;
   const unsigned full = spread ? static_cast<unsigned>(last_tiles) * n_col_blocks : 0u;
   auto cut = [&](unsigned n, unsigned d) { return static_cast<unsigned>(static_cast<uint64_t>(n) * d >> 3); };
   const unsigned light0 = cut(light, die), full0 = cut(full, die);
@@ -364,9 +365,11 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
   const int row_end = offsets[e + 1], first_row = offsets[e];
   if (!is_full && row_end - first_row > TL_ROWS(NWW)) {
     // Row tiles of an expert that has several read the same weights: up to four of them one after the other for a column
-    // block, so that all but the first find the weights in L2.
+    // block, so that all but the first find the weights in L2.  (Tiles of the expert that are among the last ones have
+    // been dealt out above.)
     const int nth = (row0 - first_row) / TL_ROWS(NWW), first = tile - (nth & 3);
-    const unsigned n_here = min(4, (row_end - first_row + TL_ROWS(NWW) - 1) / TL_ROWS(NWW) - (nth & ~3));
+    const int of_expert = (row_end - first_row + TL_ROWS(NWW) - 1) / TL_ROWS(NWW) - (nth & ~3);
+    const unsigned n_here = min(min(4, of_expert), n_light - first);
     const unsigned in = pair - static_cast<unsigned>(first) * n_col_blocks;
     tile = first + static_cast<int>(in % n_here);
     col_block = static_cast<int>(in / n_here);

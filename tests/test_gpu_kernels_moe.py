@@ -340,6 +340,22 @@ def test_grouped_tiled_last_tiles_of_one_expert_together(T, E, mi, pieces, wide)
                 assert float((got - want).abs().max()) <= 2 ** -8 * float(want.abs().max()) + 1e-5, (H, t, c)
 
 
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("last", [0, 1, 2, 3, 4, 6])
+def test_grouped_tiled_experts_of_several_tiles_beside_the_last_ones(last, wide):
+    """Experts of six, one, five and three tiles, which go together up to four at a time; the last ones of the map, worked
+    spread among the others, are some or all of the last expert's, or of the one before it, too: every row is formed."""
+    from inferx_amd import ops
+    R, H, mi = ops.moe_tiled_rows(wide), 72, 1100
+    counts = [5 * R + 3, 2, 5 * R, 2 * R + 1]
+    topk_e = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts)).to(torch.int32)[:, None].to(DEV)
+    offsets, rows, dest, tile_map = dispatch(topk_e, len(counts), R)
+    x, w = rnd(sum(counts), H, dtype=torch.bfloat16), rnd(len(counts), mi, H, seed=2, dtype=torch.bfloat16, scale=H ** -0.5)
+    out = torch.full((sum(counts), mi), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.moe_grouped_tiled(x, w, out, offsets, rows, tile_map, False, wide, last_tiles=last)
+    assert rel_err(out, grouped_reference(x, w, offsets.cpu(), rows.cpu(), False)) < 1e-2
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T", [1, 8, 17, 64])
 # at most 256 blocks of sixteen, and more; at most 128 (both halves of an even reduction in one block for up to eight rows)

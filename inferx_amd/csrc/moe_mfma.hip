@@ -93,7 +93,8 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
 
   const int64_t w_rows = GATE_UP ? 2 * static_cast<int64_t>(n_out) : n_out;
   // In load j lane l reads piece 8 (j / 2) + l % 8 of row 8 (j % 2) + l / 8: whole lines of 128 bytes.  (A block's rows
-  // start at an address that is the same for all lanes; beside it 32 bits are enough.)
+  // start at an address that is the same for all lanes; beside it a lane counts pieces of 16 bytes: in bytes, row 15 of
+  // 143 million numbers is past 32 bits.)
   const char* wbase[NACC];
   unsigned wrow[NB][2];
 #pragma unroll
@@ -103,8 +104,8 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
     if (u < NB)
 #pragma unroll
       for (int h = 0; h < 2; ++h)
-        wrow[u][h] = (static_cast<unsigned>(min((HALVES ? 0 : 8 * h) + (lane >> 3), n_out - 1 - first)) * static_cast<unsigned>(width) +
-                      (HALVES && !GATE_UP && h ? span : 0)) * sizeof(TI);
+        wrow[u][h] = static_cast<unsigned>(min((HALVES ? 0 : 8 * h) + (lane >> 3), n_out - 1 - first)) * static_cast<unsigned>(width / PN) +
+                     (HALVES && !GATE_UP && h ? span / PN : 0);
   }
   const char* const wup = UP8 ? wbase[0] + static_cast<int64_t>(n_out) * width * sizeof(TI) : nullptr;
   // Piece p of row r of a round lies at piece p ^ (r / 2 + 8 (r % 2)) of its 256 bytes: the rows that sixteen lanes read at
@@ -142,7 +143,7 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
 #pragma unroll
       for (int u = 0; u < NACC; ++u)
         w_[u][j] = __builtin_nontemporal_load(
-            reinterpret_cast<const piece_t*>((UP8 && (j & 1) ? wup : wbase[u]) + (wrow[u % NB][j & 1] + static_cast<unsigned>(kw) * sizeof(TI))));
+            reinterpret_cast<const piece_t*>(UP8 && (j & 1) ? wup : wbase[u]) + (wrow[u % NB][j & 1] + static_cast<unsigned>(kw) / PN));
 #pragma unroll
       for (int t = 0; t < MT; ++t) x_[t][j] = *reinterpret_cast<const piece_t*>(xr[t] + kk);
     }

@@ -35,7 +35,7 @@ qkv_rope_skinny_kernel(const __bf16* x, const __bf16* w, const void* __restrict_
   const char* wh = wl + static_cast<int64_t>(half) * width * 2;
   unsigned wrow[2];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) wrow[h] = static_cast<unsigned>(8 * h + (lane >> 3)) * static_cast<unsigned>(width) * 2u;
+  for (int h = 0; h < 2; ++h) wrow[h] = static_cast<unsigned>(8 * h + (lane >> 3)) * static_cast<unsigned>(width / 8);  // (in pieces)
   char* const turn = lds + wave * 8192;
   auto turn_at = [&](int r, int p) { return turn + 256 * r + 16 * (p ^ ((r >> 1) | ((r & 1) << 3))); };
   const __bf16* xr[NT];
@@ -60,9 +60,9 @@ qkv_rope_skinny_kernel(const __bf16* x, const __bf16* w, const void* __restrict_
       kk = kk < kend ? kk : kbegin;  // (past the end: the range's first piece, which exists and was read before)
       int kw = k0 + 64 * (j >> 1) + 8 * (lane & 7);
       kw = kw < kend ? kw : kbegin;
-      const unsigned at = wrow[j & 1] + 2u * static_cast<unsigned>(kw);
-      st.fl[j] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(wl + at));
-      st.fh[j] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(wh + at));
+      const unsigned at = wrow[j & 1] + static_cast<unsigned>(kw) / 8;
+      st.fl[j] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(wl) + at);
+      st.fh[j] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(wh) + at);
 #pragma unroll
       for (int t = 0; t < NT; ++t) st.fx[t][j] = *reinterpret_cast<const bf16x8*>(xr[t] + kk);
     }

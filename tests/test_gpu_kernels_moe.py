@@ -386,6 +386,32 @@ def test_dense_products_of_few_rows(dtype, T, N, K, form, biased):
     assert float((err - eps * want.abs()).max()) <= 4e-5, float(err.max())
 
 
+@pytest.mark.parametrize("which", ["bfloat16", "float32", "q/k/v"])
+def test_streaming_products_of_very_long_rows(which):
+    """Weight rows so long that the sixteenth starts 2^32 bytes behind the first: every row's own first and last number
+    meet the activations' (all others are zero, the sums are small whole numbers)."""
+    from inferx_amd import ops
+    dtype = torch.float32 if which == "float32" else torch.bfloat16
+    K = (1 << 32) // 15 // (4 if which == "float32" else 2) // 16 * 16 + 16
+    T, N = (9 if which == "bfloat16" else 1), (96 if which == "q/k/v" else 16)
+    x, w = torch.zeros(T, K, dtype=dtype, device=DEV), torch.zeros(N, K, dtype=dtype, device=DEV)
+    row = torch.arange(N, device=DEV)
+    x[:, 0], x[:, -1] = 64, 1
+    w[:, 0], w[:, -1] = 1, (row + 1).to(dtype)
+    if which == "q/k/v":
+        q = torch.full((1, 1, 32), float("nan"), dtype=dtype, device=DEV)
+        kc, vc = torch.zeros(1, 1, 16, 32, dtype=dtype, device=DEV), torch.zeros(1, 1, 32, 16, dtype=dtype, device=DEV)
+        ops.qkv_rope_skinny(x, w, None, None, torch.zeros(1, dtype=torch.int32, device=DEV), q, kc, vc, 1, 1, 32)
+        out = torch.cat([q[0, 0], kc[0, 0, 0], vc[0, 0, :, 0]])[None]
+    else:
+        out = torch.full((T, N), float("nan"), dtype=dtype, device=DEV)
+        ops.linear_skinny(x, w, out)
+    want = (65 + row).float().expand(T, N)
+    del x, w
+    torch.cuda.empty_cache()
+    assert torch.equal(out.float(), want), (out.float() - want).nonzero()[:4].tolist()
+
+
 @pytest.mark.parametrize("T,N,K", [(3, 40, 264), (16, 33, 1160), (2, 16, 8), (5, 48, 520)])
 def test_streaming_kernels_read_nothing_past_their_operands(T, N, K):
     """Reduction widths that leave a wavefront a ragged last round: what lies behind the last row of the weights

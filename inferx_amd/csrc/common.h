@@ -52,6 +52,11 @@ __device__ __forceinline__ float4 ix_load4_rt(const void* base, int dtype, int64
   return make_float4(ix_load_rt(base, dtype, i), ix_load_rt(base, dtype, i + 1), ix_load_rt(base, dtype, i + 2),
                      ix_load_rt(base, dtype, i + 3));
 }
+// a sum of squares, continued: one rounding a number, in their order (`+=` leaves the compiler to choose which of the first
+// two squares is rounded by itself)
+__device__ __forceinline__ float ix_add_squares(float sum, const float4& v) {
+  return __builtin_fmaf(v.w, v.w, __builtin_fmaf(v.z, v.z, __builtin_fmaf(v.y, v.y, __builtin_fmaf(v.x, v.x, sum))));
+}
 // four numbers rounded to bfloat16, side by side
 __device__ __forceinline__ uint2 ix_pack4_bf16(const float4& v) {
   return make_uint2(ix_f32x2_to_bf16x2(v.x, v.y), ix_f32x2_to_bf16x2(v.z, v.w));

@@ -556,7 +556,7 @@ head_norm_gate_kernel(const float* __restrict__ x, const float* __restrict__ x2,
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const float o = me + STEP * i < vdim ? v[i] * pre : 0.f;
-    ss += o * o;
+    ss = __builtin_fmaf(o, o, ss);  // (in this order)
   }
   ss = PER_WAVE ? ix_wave_sum(ss) : ix_block_sum(ss, red);
   const float inv = pre * mult / sqrtf(ss / static_cast<float>(vdim) + eps);

@@ -126,12 +126,7 @@ add_rmsnorm_vec4_kernel(float* __restrict__ h, const uint16_t* __restrict__ delt
       v[u].z += __uint_as_float(d[u].y << 16);
       v[u].w += __uint_as_float(d[u].y & 0xffff0000u);
     }
-    if (4 * (threadIdx.x + u * static_cast<int64_t>(blockDim.x)) < width) {
-      sumsq += v[u].x * v[u].x;
-      sumsq += v[u].y * v[u].y;
-      sumsq += v[u].z * v[u].z;
-      sumsq += v[u].w * v[u].w;
-    }
+    if (4 * (threadIdx.x + u * static_cast<int64_t>(blockDim.x)) < width) sumsq = ix_add_squares(sumsq, v[u]);
   }
   sumsq = ix_block_sum(sumsq, red);
   const float inv = 1.0f / sqrtf(sumsq / static_cast<float>(width) + eps);
@@ -163,9 +158,12 @@ extern "C" int ix_add_rmsnorm(void* h, const void* delta, int delta_dtype, const
 #define VEC4(NV, THREADS)                                                                                         \
   hipLaunchKernelGGL(add_rmsnorm_vec4_kernel<NV>, grid, dim3(THREADS), 0, stream, (float*)h, (const uint16_t*)delta, w, \
                      w_dtype, (uint16_t*)out, rows, row_width, width, eps)
+    // (which columns a thread adds up goes by the width alone, as in the experts' sum and norm: 256, 512 or 1,024 threads)
     if (width <= 1024) VEC4(1, 256);
-    else if (width <= 2048) VEC4(1, 512);
-    else if (width <= 4096) VEC4(2, 512);
+    else if (width < 2048) VEC4(2, 256);
+    else if (width == 2048) VEC4(1, 512);
+    else if (width < 4096) VEC4(2, 512);
+    else if (width == 4096) VEC4(1, 1024);
     else if (width <= 8192) VEC4(2, 1024);
     else VEC4(4, 1024);
 #undef VEC4

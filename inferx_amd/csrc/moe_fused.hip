@@ -228,12 +228,7 @@ moe_combine_add_rmsnorm_rows_kernel(float* __restrict__ h, const uint16_t* __res
       for (int i = 0; i < 4; ++i) acc[u][i] += sg * f[i];
     }
     v[u].x += acc[u][0]; v[u].y += acc[u][1]; v[u].z += acc[u][2]; v[u].w += acc[u][3];
-    if (4 * (threadIdx.x + u * static_cast<int64_t>(blockDim.x)) < width) {
-      sumsq += v[u].x * v[u].x;
-      sumsq += v[u].y * v[u].y;
-      sumsq += v[u].z * v[u].z;
-      sumsq += v[u].w * v[u].w;
-    }
+    if (4 * (threadIdx.x + u * static_cast<int64_t>(blockDim.x)) < width) sumsq = ix_add_squares(sumsq, v[u]);
   }
   sumsq = ix_block_sum(sumsq, red);
   const float inv = 1.0f / sqrtf(sumsq / static_cast<float>(width) + eps);
@@ -274,8 +269,10 @@ extern "C" int ix_moe_combine_add_rmsnorm(void* h, const void* y, int dtype, con
   hipLaunchKernelGGL(moe_combine_add_rmsnorm_rows_kernel<NV>, grid, dim3(THREADS), 0, stream, (float*)h, (const uint16_t*)y, \
                      dest, topk_w, (const uint16_t*)shared, shared_gate, w, w_dtype, (uint16_t*)out, rows, row_width, width, k, eps)
     if (width <= 1024) ROWS(1, 256);
-    else if (width <= 2048) ROWS(1, 512);
-    else if (width <= 4096) ROWS(2, 512);
+    else if (width < 2048) ROWS(2, 256);
+    else if (width == 2048) ROWS(1, 512);
+    else if (width < 4096) ROWS(2, 512);
+    else if (width == 4096) ROWS(1, 1024);
     else ROWS(2, 1024);
 #undef ROWS
   } else if (dtype == IX_BF16 && width % 4 == 0 &&

@@ -2,6 +2,7 @@
 temperature sampling, penalties: each kernel alone against a PyTorch reference."""
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -58,6 +59,48 @@ def test_add_rmsnorm(dtype, wdtype, T, H, eps):
     ops.add_rmsnorm(h, delta, w, picked, eps, rows)
     assert torch.equal(h, h0)
     assert rel_err(picked, pm.rms_norm(v, w.double().cpu(), eps)[rows.long().cpu()]) < tol(dtype)
+
+
+def norm_in_its_order(v, w, eps):
+    """v / rms(v) * w in bfloat16, bit for bit: every thread adds the squares of its columns (four at a time) one after the
+    other with one rounding each, 64 threads meet pair by pair, wavefront after wavefront is added; 256, 512 or 1,024
+    threads by the width."""
+    v, w = v.cpu().numpy(), w.float().cpu().numpy()
+    T, W = v.shape
+    n = 1024 if W >= 4096 else 512 if W >= 2048 else 256
+    turns = -(-W // (4 * n))
+    cols = np.zeros((T, turns * 4 * n), dtype=np.float32)
+    cols[:, :W] = v
+    cols = cols.reshape(T, turns, n, 4).astype(np.longdouble)
+    part = np.zeros((T, n), dtype=np.float32)
+    for u in range(turns):
+        for i in range(4):
+            part = (cols[:, u, :, i] ** 2 + part).astype(np.float32)
+    part = part.reshape(T, n // 64, 64)
+    while part.shape[2] > 1:
+        part = part[:, :, 0::2] + part[:, :, 1::2]
+    total = np.zeros(T, dtype=np.float32)
+    for wave in range(n // 64):
+        total = total + part[:, wave, 0]
+    inv = np.float32(1) / np.sqrt(total / np.float32(W) + np.float32(eps))
+    return torch.from_numpy(v * inv[:, None] * w).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("W", [1024, 1028, 2044, 2048, 2052, 4092, 4096, 8192, 16384])
+def test_norms_keep_the_order_of_their_sums(W):
+    """So many rows that an order of its own would show in some bfloat16 results; the sum with a branch, and with two
+    experts' rows."""
+    from inferx_amd import ops
+    T, eps = (1 << 22) // W, 1e-6
+    h, y, w = rnd(T, W), rnd(2 * T, W, seed=1, dtype=torch.bfloat16), rnd(W, seed=2, dtype=torch.bfloat16)
+    out, got = torch.empty(T, W, dtype=torch.bfloat16, device=DEV), h.clone()
+    ops.add_rmsnorm(got, y[:T], w, out, eps)
+    assert torch.equal(got, h + y[:T].float())
+    assert torch.equal(out.cpu(), norm_in_its_order(got, w, eps))
+    if W <= 8192:
+        dest = torch.arange(2 * T, dtype=torch.int32, device=DEV).flip(0).contiguous()
+        ops.moe_combine_add_rmsnorm(h, y, dest, torch.full((T, 2), 0.5, device=DEV), None, None, w, out, eps, None)
+        assert torch.equal(out.cpu(), norm_in_its_order(h, w, eps))
 
 
 @pytest.mark.parametrize("dtype", DTYPES)

@@ -21,24 +21,33 @@ from __future__ import annotations
 import math
 from typing import List, Optional
 
+import numpy as np
 import torch
 
 from .. import ops
 from ..config.spec import PartSpec
-from .attention import MIN_KEYS_PER_SPLIT, QUERY_TILE, WAVES_WANTED, plan_tiles
+from .attention import MIN_KEYS_PER_SPLIT, PREFILL_MIN_ROWS, QUERY_TILE, WAVES_WANTED, _tiles_of, plan_tiles
 from .base import CacheArray, CacheNeed, Mixer, ParamSpec, StateNeed, build_part, register_part
 from .dense_mlp import stack_rows
 from .short_conv import ShortConv
 
 
-# A step that brings some request several tokens goes through the kernel that shares keys and values through LDS where it
-# has a workgroup (a tile of 64 queries of a head) for every compute unit, or no context is long: a workgroup walks all of
-# its keys (1.3 us for 32 of them), while the wavefront-level kernel cuts them into slices.  us, that one / this one, 16
-# heads, window 1,024: whole prompts of 611 and 1,437 105 / 48, eight of 200 37 / 16, one of 300 19.5 / 17.5; portions of 64
-# to 500 tokens on 1,500 (16 to 128 workgroups) 18 to 45 / 44 to 50; 300 tokens beside sixteen single ones (336) 70 / 53.
+# A step that brings some request several tokens goes through the kernel that shares keys and values through LDS, or through
+# the wavefront-level one, which cuts keys into slices where a step has few tiles.  A workgroup of the former (a tile of up to
+# 64 queries of a head, two on a compute unit) walks all of its keys, 1.3 us for 32 of them, however few queries it has.  us,
+# wavefront-level / LDS, 16 heads:
+#   no context long (`turns`: rounds of 32 keys times how often 512 workgroups fill the chip): eight prompts of 200 37 / 16,
+#   one of 300 19.5 / 17.5, 64 tokens on 256 16.2 / 15.0, on 384 16.3 / 18.6; sixteen single tokens on 128 beside 64 15.6 / 13.2,
+#   on 256 15.9 / 17.9; 32 on 64 15.5 / 13.1, on 128 16.0 / 18.0
+#   a workgroup for every compute unit, and the portions' tiles at least a quarter as many as the single tokens': prompts of 611
+#   and 1,437 with a window of 1,024 105 / 48; 300 tokens beside sixteen single ones on 1,000 and 2,000 keys 67 / 51 and 119 / 90,
+#   beside 32 73 / 83 and 132 / 150; 64 beside sixteen 37 / 51 and 64 / 90
+#   single tokens on more than 2,048 keys in a launch of their own, in slices (`portion_plan`), in one LDS launch / two: 1,200
+#   tokens beside sixteen single ones on 1,500, 2,000, 3,000 and 30,000 89 / 84, 106 / 101, 142 / 107 and 1,141 / 306, beside four on
+#   2,000 and 3,000 88 / 90 and 123 / 94
 PREFILL_TILE = 64
 PREFILL_MIN_WORKGROUPS = 256
-PREFILL_SHORT_KEYS = 384
+PREFILL_MAX_FEW_KEYS = 2048
 
 
 class DifferentialAttention(Mixer):
@@ -129,32 +138,75 @@ class DifferentialAttention(Mixer):
         n = 1 if units >= WAVES_WANTED else max(1, min(WAVES_WANTED // max(1, units), -(-span // MIN_KEYS_PER_SPLIT), 64))
         return 1 << (n.bit_length() - 1)
 
+    def portion_plan(self, ctx):
+        """Which tiles the LDS-sharing kernel takes in a step that brings some request several tokens, or None if the
+        wavefront-level kernel takes the step: (tiles, few), few = (rows, tiles, positions, slices, grouped) for a launch of the
+        latter that serves the requests of few tokens by themselves, or None."""
+        key = ("attention_diff_portions", self.num_heads, self.num_kv_heads, self.window, self.keep_first)
+        if key in ctx.memo:
+            return ctx.memo[key]
+        tiles, n_tiles, longest = plan_tiles(ctx, PREFILL_TILE)
+        q_start = ctx.host.q_start.astype(np.int64)
+        n, lens = q_start[1:] - q_start[:-1], ctx.host.seq_lens.astype(np.int64)
+        many, few = np.flatnonzero(n >= PREFILL_MIN_ROWS), np.flatnonzero((n > 0) & (n < PREFILL_MIN_ROWS))
+        workgroups = n_tiles * self.num_heads
+        turns = -(-workgroups // 512) * -(-longest // 32)
+        plan = None
+        if turns <= 4:
+            plan = (tiles, None)
+        elif workgroups < PREFILL_MIN_WORKGROUPS:
+            if turns <= 8 or (turns <= 12 and ctx.num_tokens >= 256):
+                plan = (tiles, None)
+        elif 4 * (n_tiles - len(few)) >= len(few):
+            plan = (tiles, None)
+            keys = int(lens[few].max()) if len(few) else 0
+            if (min(keys, self.window + self.keep_first) if self.window > 0 else keys) > PREFILL_MAX_FEW_KEYS:
+                to_dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(ctx.rt.device)
+                grouped = 2 <= self.num_heads // self.num_kv_heads <= 16
+                own = _tiles_of(n[few], np.cumsum(n[few]) - n[few], few, 1 if grouped else QUERY_TILE)
+                rows = to_dev(np.concatenate([np.arange(q_start[i], q_start[i + 1]) for i in few]))
+                slices = self.key_slices(own.shape[1] * 2 * (self.num_kv_heads if grouped else self.num_heads), keys)
+                plan = (to_dev(_tiles_of(n[many], q_start[many], many, PREFILL_TILE)),
+                        (rows, to_dev(own), ctx.positions.index_select(0, rows), slices, grouped))
+        ctx.memo[key] = plan
+        return plan
+
     def attend(self, ctx, q, cache, out) -> None:
-        """bfloat16 with heads and pages that the matrix-core kernel is built for: that kernel, in tiles of up to 16
-        queries of a request, a (head, map) pair per wavefront (a step of one token per request: the query heads of
-        a key/value head side by side); else the plain one."""
+        """bfloat16 with heads and pages that the matrix-core kernels are built for: those, prompt portions in tiles of 64
+        queries through LDS or, with the few tokens beside them, in tiles of up to 16 queries of a request, a (head, map) pair
+        per wavefront (one token per request: the query heads of a key/value head side by side); else the plain one."""
         page_size = cache.k.shape[2]
+        plan = None
         if (q.dtype == torch.bfloat16 and not ctx.one_token_each
                 and ops.attention_diff_prefill_fits(self.head_dim, self.value_dim, page_size)):
-            tiles, n_tiles, longest = plan_tiles(ctx, PREFILL_TILE)
-            if n_tiles * self.num_heads >= PREFILL_MIN_WORKGROUPS or longest <= PREFILL_SHORT_KEYS:
-                ops.attention_diff_prefill(q, cache.k, cache.v, ctx.block_tables[cache.group], tiles, ctx.positions, out,
-                                           self.scale, self.window, self.keep_first, self.lam, self.norm_eps,
-                                           1.0 - self.diff)
-                return
+            plan = self.portion_plan(ctx)
+        if plan is not None:
+            tiles, few = plan
+            ops.attention_diff_prefill(q, cache.k, cache.v, ctx.block_tables[cache.group], tiles, ctx.positions, out,
+                                       self.scale, self.window, self.keep_first, self.lam, self.norm_eps, 1.0 - self.diff)
+            if few is not None:  # their rows are put side by side: slices are merged for all rows of a launch
+                rows, tiles, positions, n_splits, grouped = few
+                own = q.index_select(0, rows)
+                result = ctx.rt.empty((rows.numel(), self.num_heads, self.value_dim))
+                self._attend_wavefronts(ctx, own, cache, result, tiles, positions, n_splits, grouped)
+                out.index_copy_(0, rows, result)
+            return
         if q.dtype == torch.bfloat16 and ops.attention_diff_mfma_fits(self.head_dim, self.value_dim, page_size):
             tiles, n_tiles, longest = plan_tiles(ctx, QUERY_TILE)
             group = self.num_heads // self.num_kv_heads
             grouped = ctx.one_token_each and 2 <= group <= 16
             n_splits = self.key_slices(n_tiles * 2 * (self.num_kv_heads if grouped else self.num_heads), longest)
-            work = ctx.rt.empty((q.shape[0] * self.num_heads * 2 * n_splits * (self.value_dim + 2),), torch.float32)
-            ops.attention_diff_mfma(q, cache.k, cache.v, ctx.block_tables[cache.group], tiles, ctx.positions, out,
-                                    n_splits, work, self.scale, self.window, self.keep_first, self.lam, self.norm_eps,
-                                    1.0 - self.diff, grouped=grouped)
+            self._attend_wavefronts(ctx, q, cache, out, tiles, ctx.positions, n_splits, grouped)
             return
         ops.attention_diff_plain(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.seq_of_token, ctx.positions,
                                  out, self.scale, self.window, self.keep_first, self.lam, self.norm_eps,
                                  1.0 - self.diff)
+
+    def _attend_wavefronts(self, ctx, q, cache, out, tiles, positions, n_splits: int, grouped: bool) -> None:
+        work = ctx.rt.empty((q.shape[0] * self.num_heads * 2 * n_splits * (self.value_dim + 2),), torch.float32)
+        ops.attention_diff_mfma(q, cache.k, cache.v, ctx.block_tables[cache.group], tiles, positions, out, n_splits, work,
+                                self.scale, self.window, self.keep_first, self.lam, self.norm_eps, 1.0 - self.diff,
+                                grouped=grouped)
 
 
 register_part("mixer", "differential_attention", DifferentialAttention)

@@ -670,6 +670,63 @@ def test_one_key_stands_out_for_every_query_of_a_portion(kernel):
                 f"portion ending at {last}, key {key}: queries {np.flatnonzero((err < 3e-2) != seen).tolist()} of the portion are wrong"
 
 
+def diff_attention_reference(q, k, v, first, window, keep, lam, eps, scale):
+    """q [n, H, 2, D] at positions first.. of one request, k [L, G, 2, D], v [L, G, V]: float64 on the device."""
+    n, H = q.shape[:2]
+    L, G = v.shape[:2]
+    i, j = torch.arange(first, first + n, device=DEV)[:, None], torch.arange(L, device=DEV)[None]
+    seen = (j <= i) & ((i - j < window) | (j < keep)) if window else j <= i
+    kk, vv = k.double().repeat_interleave(H // G, 1), v.double().repeat_interleave(H // G, 1)
+    a = []
+    for m in range(2):
+        s = (q[:, :, m].double().permute(1, 0, 2) @ kk[:, :, m].permute(1, 2, 0).contiguous()) * scale
+        a.append((torch.softmax(s.masked_fill(~seen, float("-inf")), -1) @ vv.permute(1, 0, 2).contiguous()).permute(1, 0, 2))
+    o = a[0] - lam * a[1]
+    return o * torch.rsqrt((o * o).mean(-1, keepdim=True) + eps)
+
+
+@pytest.mark.parametrize("heads,kv,V,window,news,lens,expect", [
+    (16, 4, 64, 0, [2] + [1] * 16, [700] * 17, "wavefronts"),          # more single tokens than portions' tiles
+    (16, 4, 128, 0, [300] + [1] * 16, [1000] + [900] * 16, "lds"),
+    (16, 4, 64, 0, [300] + [1] * 32, [400] + [700] * 32, "wavefronts"),
+    (16, 4, 128, 0, [300] + [1] * 16, [300] + [2049] + [30] * 15, "two launches"),
+    (16, 4, 128, 0, [300] + [1] * 16, [300] + [2048] + [30] * 15, "lds"),
+    (16, 4, 64, 1024, [300] + [1] * 16, [300] + [2500] + [30] * 15, "lds"),  # (a window: 1,024 of them are read)
+    (16, 16, 64, 0, [1, 1000, 3, 15, 1], [2100, 1000, 2500, 20, 7], "two launches"),  # tiles of up to 15 queries, not grouped
+    (16, 2, 64, 2100, [15, 1000, 1, 2], [2500, 1200, 2400, 40], "two launches"),
+    (8, 4, 64, 0, [20, 3, 1], [20, 100, 64], "lds"),                    # short contexts
+    (8, 4, 64, 0, [150, 1], [300, 257], "wavefronts"),
+    (8, 4, 64, 0, [256, 1], [300, 257], "lds"),
+])
+def test_differential_attention_kernels_chosen_by_the_step(heads, kv, V, window, news, lens, expect):
+    """`attend` on steps of portions and single tokens: whichever kernels the step's plan names, the result is float64
+    attention of every request."""
+    from inferx_amd.engine.runtime import CacheBinding, Runtime
+    from inferx_amd.parts.attention_diff import DifferentialAttention
+    from test_gpu_parts import make_ctx
+    D, page, keep, dtype = 64, 16, 4 if window else 0, torch.bfloat16
+    part = DifferentialAttention(64, heads, kv, D, V, 0.5, window=window, keep_first=keep, norm_eps=1e-5)
+    part.lam = 0.4
+    pages = sum(-(-n // page) for n in lens) + 2
+    ctx, batch = make_ctx(Runtime("bfloat16"), news, lens, page, pages)
+    table = torch.from_numpy(batch.block_tables[0].reshape(len(news), -1)).long()
+    kc = torch.full((pages, 2 * kv, page, D), float("nan"), dtype=dtype, device=DEV)
+    vc = torch.full((pages, kv, V, page), float("nan"), dtype=dtype, device=DEV)
+    qs, wants = [], []
+    for s, (n, L) in enumerate(zip(news, lens)):
+        q, k, v = rnd((n, heads, 2, D), 3 * s, 1.0, dtype).to(DEV), rnd((L, 2 * kv, D), 3 * s + 1, 1.0, dtype).to(DEV), rnd((L, kv, V), 3 * s + 2, 1.0, dtype).to(DEV)
+        at = torch.arange(L)
+        own, off = table[s, at // page].to(DEV), (at % page).to(DEV)
+        kc[own, :, off], vc[own, :, :, off] = k, v
+        qs.append(q)
+        wants.append(diff_attention_reference(q, k.view(L, kv, 2, D), v, L - n, window, keep, 0.4, 1e-5, D ** -0.5) * 0.5)
+    out = torch.full((sum(news), heads, V), float("nan"), dtype=dtype, device=DEV)
+    part.attend(ctx, torch.cat(qs), CacheBinding(group=0, arrays=dict(k=kc, v=vc)), out)
+    plan = part.portion_plan(ctx)
+    assert ("wavefronts" if plan is None else "lds" if plan[1] is None else "two launches") == expect
+    close(out, torch.cat(wants).cpu().numpy(), 1.5e-2, expect)
+
+
 # ---- the delta rule in chunks ---------------------------------------------------------------------------------------------
 # rows of the requests of a step (one of them without any), around chunks of 64 and the sixteens within them
 @pytest.mark.parametrize("lengths", [[1, 15, 0, 16], [17, 64, 63], [65, 130], [200]])

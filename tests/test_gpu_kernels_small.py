@@ -86,7 +86,7 @@ def norm_in_its_order(v, w, eps):
     return torch.from_numpy(v * inv[:, None] * w).to(torch.bfloat16)
 
 
-@pytest.mark.parametrize("W", [1024, 1028, 2044, 2048, 2052, 4092, 4096, 8192, 16384])
+@pytest.mark.parametrize("W", [1024, 1028, 2044, 2048, 2052, 4092, 4096, 8192, 16384, 16388, 20480])
 def test_norms_keep_the_order_of_their_sums(W):
     """So many rows that an order of its own would show in some bfloat16 results; the sum with a branch, and with two
     experts' rows."""

@@ -228,10 +228,11 @@ __global__ void silu_mul_kernel(const T* __restrict__ gu, T* __restrict__ out, i
   }
 }
 
-// The gated unit of bfloat16 rows with a width that is a multiple of 8, with or without a bias: eight columns a thread, of
-// one row after the other, 16-byte loads and stores.  Bound by memory where there is no bias (2,048 rows of 5,632, 69 MB:
-// 13 us, 5.4 TB/s; 20,480 columns 39 us).  With one, sixteen loads of 2 bytes a row and thread took 36 us; now a thread loads its columns' once, 16 bytes
-// at a time where they lie on such boundaries: 14 us (without a bias 13).  FAST: `ix_glu`'s quicker exponential.
+// The gated unit of bfloat16 rows with a width that is a multiple of 8, with or without a bias: eight columns a thread, 16-byte
+// loads and stores; a workgroup's threads are the columns of one row (up to 2,048 of them) or of as many as 256 threads hold.
+// Bound by memory (2,048 rows of 5,632, 69 MB: 13 us, 5.4 TB/s; 20,480 columns 39 us).  A thread loads its columns' biases once
+// for up to four rows, 16 bytes at a time where they lie on such boundaries: 14 us (sixteen loads of 2 bytes a row and thread 36).
+// FAST: `ix_glu`'s quicker exponential.
 template <bool FAST>
 __global__ void __launch_bounds__(256)
 glu_rows_kernel(const uint16_t* __restrict__ gu, const void* __restrict__ bias, int bias_dtype,
@@ -259,7 +260,8 @@ glu_rows_kernel(const uint16_t* __restrict__ gu, const void* __restrict__ bias, 
       }
     }
   }
-  for (int64_t t = blockIdx.y; t < tokens; t += gridDim.y) {
+  for (int64_t t = static_cast<int64_t>(blockIdx.y) * blockDim.y + threadIdx.y; t < tokens;
+       t += static_cast<int64_t>(gridDim.y) * blockDim.y) {
     float g[8], u[8];
     unpack(*reinterpret_cast<const uint4*>(gu + t * 2 * width + c), g);
     unpack(*reinterpret_cast<const uint4*>(gu + t * 2 * width + width + c), u);
@@ -282,10 +284,13 @@ template <bool FAST>
 static void launch_glu_rows(const void* gu, const void* bias, int bias_dtype, void* out, int64_t tokens, int64_t width,
                             float limit, hipStream_t stream) {
   const int64_t pieces = width / 8;
-  const unsigned block = static_cast<unsigned>(std::min<int64_t>(256, (pieces + 63) / 64 * 64));
-  const dim3 grid(static_cast<unsigned>((pieces + block - 1) / block), static_cast<unsigned>(std::min<int64_t>(tokens, bias ? 512 : 65535)));  // (a few rows a thread where it has a bias to load)
-  hipLaunchKernelGGL(glu_rows_kernel<FAST>, grid, dim3(block), 0, stream, (const uint16_t*)gu, bias, bias_dtype, (uint16_t*)out,
-                     tokens, width, limit);
+  const dim3 block(static_cast<unsigned>(std::min<int64_t>(256, pieces)), static_cast<unsigned>(std::max<int64_t>(1, 256 / pieces)));
+  const int64_t across = (pieces + block.x - 1) / block.x, down = (tokens + block.y - 1) / block.y;
+  // (with a bias to load, up to four rows a thread as long as 2,048 workgroups are left)
+  const int64_t turns = bias ? std::max<int64_t>(1, std::min<int64_t>(4, across * down / 2048)) : 1;
+  const dim3 grid(static_cast<unsigned>(across), static_cast<unsigned>(std::min<int64_t>((down + turns - 1) / turns, 65535)));
+  hipLaunchKernelGGL(glu_rows_kernel<FAST>, grid, block, 0, stream, (const uint16_t*)gu, bias, bias_dtype, (uint16_t*)out, tokens,
+                     width, limit);
 }
 
 extern "C" int ix_silu_mul(const void* gu, void* out, int dtype, int64_t tokens, int64_t width, hipStream_t stream) {

@@ -353,6 +353,21 @@ def test_clamped_gated_unit_of_many_rows(bias):
     assert float((act.cpu().double() - want).abs().max()) <= 1e-2 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("T,n", [(1, 8), (7000, 8), (131, 136), (20000, 264), (9, 1368), (3, 2040), (2049, 2048)])
+@pytest.mark.parametrize("biased", [False, True])
+def test_gated_unit_of_narrow_rows(T, n, biased):
+    """Several rows a workgroup (32 of 8 columns, one of 1,368), a last one with fewer, one to three turns of rows a thread;
+    what lies behind the result stays."""
+    from inferx_amd import ops
+    gate_up = rnd((T, 2 * n), 1, 3.0, torch.bfloat16).to(DEV)
+    b = rnd((2 * n,), 2, 1.0, torch.bfloat16).to(DEV) if biased else None
+    buf = torch.full((T + 3, n), 9.0, dtype=torch.bfloat16, device=DEV)
+    ops.glu_bias(gate_up, b, buf[:T])
+    z = gate_up.double() + (b.double() if biased else 0.0)
+    want = torch.nn.functional.silu(z[:, :n]) * z[:, n:]
+    assert float((buf[:T].double() - want).abs().max()) <= 1e-2 * float(want.abs().max()) and (buf[T:] == 9.0).all()
+
+
 def test_norm_with_one_number():
     x = rnd((5, 24), 1).double()
     g = torch.tensor(1.3, dtype=torch.float64)

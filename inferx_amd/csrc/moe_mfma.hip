@@ -468,10 +468,12 @@ extern "C" int ix_linear_skinny(const void* x, const void* w, int dtype, void* o
                        (int)n_out, (int)width, glu_limit);
     return ix_check_launch("ix_linear_skinny");
   }
-  // A gated product with between one and two blocks of sixteen for a compute unit: some have two of them and most one, and
-  // eights even that out.  One | eight rows of 2,048 numbers, us: 5,632 features 9.5 | 10.5 (10.3 | 11.2), 6,144 9.8 | 10.7 (11.2 |
-  // 12.5); no gain from two blocks a compute unit on (8,192: 12.2 | 13.0 (12.4 | 12.8)), where the rows weigh more.
-  if (!out_f32 && gate_up && rows <= 8 && blocks > 256 && blocks < 448) {
+  // A gated product with more than one and at most one and a half blocks of sixteen for each of the 256 compute units: some have
+  // two of them and most one; of eights each has up to three.  One | eight rows of 2,048 numbers, us, sixteens and eights,
+  // bfloat16: 257 blocks 9.4 | 10.5 and 8.5 | 9.6, 320 10.2 | 11.0 and 9.1 | 10.1, 384 10.3 | 11.2 and 9.7 | 10.4; with a fourth
+  // eight for some 416 10.6 | 11.5 and 11.3 | 12.5.  float32: 257 18.9 | 19.8 and 16.0 | 17.2, 384 20.5 | 21.2 and 17.9 | 19.1, 416
+  // 20.5 | 21.4 and 21.2 | 23.1.
+  if (!out_f32 && gate_up && rows <= 8 && blocks > 256 && blocks <= 384) {
     const dim3 grid8(static_cast<unsigned>((n_out + 7) / 8));
     if (dtype == IX_F32)
       hipLaunchKernelGGL((linear_skinny_kernel<1, true, 4, 1, float, float, true>), grid8, dim3(256), 0, stream, (const float*)x,

@@ -386,6 +386,24 @@ def test_dense_products_of_few_rows(dtype, T, N, K, form, biased):
     assert float((err - eps * want.abs()).max()) <= 4e-5, float(err.max())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N", [4096, 4097, 6137, 6144, 6145])  # 256 blocks of sixteen, 257 and 384 (eights), 385
+@pytest.mark.parametrize("T", [1, 8, 9])
+def test_gated_products_in_sixteens_and_eights(dtype, T, N):
+    """On both sides of the line the features' sums have one order: a column that both have, alone on its side of it."""
+    from inferx_amd import ops
+    K = 264
+    x, w = rnd(T, K, dtype=dtype), rnd(2 * N, K, seed=1, dtype=dtype, scale=K ** -0.5)
+    out, other = (torch.full((T, n), float("nan"), dtype=dtype, device=DEV) for n in (N, 7168))
+    ops.linear_skinny(x, w, out, True)
+    gate, up = (torch.cat([part, part.new_zeros(7168 - N, K)]) for part in (w[:N], w[N:]))
+    ops.linear_skinny(x, torch.cat([gate, up]), other, True)
+    want = torch.nn.functional.silu(x.double() @ w[:N].double().T) * (x.double() @ w[N:].double().T)
+    assert rel_err(out, want) < (1e-2 if dtype == torch.bfloat16 else 1e-5)
+    if N > 4096:  # (up to 256 blocks eight wavefronts share the reduction, from there on four)
+        assert torch.equal(out, other[:, :N])
+
+
 @pytest.mark.parametrize("which", ["bfloat16", "float32", "q/k/v"])
 def test_streaming_products_of_very_long_rows(which):
     """Weight rows so long that the sixteenth starts 2^32 bytes behind the first: every row's own first and last number

@@ -377,7 +377,7 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
   }
   const int held = min(TL_ROWS(NWW), row_end - row0);
   if (held <= 0) return;
-  const bool once = row0 == first_row && held == row_end - row0 && held <= 64;  // an expert's only tile, few rows
+  const bool once = held == row_end - first_row && held <= 64;  // an expert's only tile, few rows
 #define CALL(NP, ONCE) \
   tiled_body<GATE_UP, NP, NWW, ONCE>(a, w, out, rows, n_out, width, e, row0, row_end, col_block, ws, xs, act, glu_limit)
 #define BODY(NP) CALL(NP, false)

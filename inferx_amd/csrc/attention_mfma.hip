@@ -267,7 +267,7 @@ attn_mfma_kernel(const __bf16* __restrict__ q, const __bf16* __restrict__ k_cach
   if constexpr (TURN) {
     // Whole lines, past the caches (every key and value is read once a step), two rounds of 32 keys on their way: a
     // load brings 1 KB of a page's keys, which the wavefront turns into the matrix cores' operands through 8 KB of LDS
-    // of its own, with no barrier (its LDS operations are carried out in their order).  The pages of the slice's next
+    // of its own, with no workgroup barrier.  The pages of the slice's next
     // 64 sixteens of keys are in one register, so no load waits for a look at the table.  Every load is unconditional
     // and the loop one straight line: rounds past the end ask for one address only.
     constexpr int ROW = 2 * NB;  // 16-byte pieces of a key
@@ -313,11 +313,13 @@ attn_mfma_kernel(const __bf16* __restrict__ q, const __bf16* __restrict__ k_cach
       }
     };
     auto use = [&](int kb, const bf16x8 (&kt)[NB], bf16x8 (&vt)[NB]) {
+      ix_wave_lds_order();
 #pragma unroll
       for (int i = 0; i < NB; ++i) {
         const int id = 64 * i + lane;
         *reinterpret_cast<bf16x8*>(turn_at(id / ROW, id % ROW)) = kt[i];
       }
+      ix_wave_lds_order();
       bf16x8 kf[2][NC];
 #pragma unroll
       for (int b = 0; b < 2; ++b)

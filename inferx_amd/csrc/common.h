@@ -62,6 +62,11 @@ __device__ __forceinline__ uint2 ix_pack4_bf16(const float4& v) {
   return make_uint2(ix_f32x2_to_bf16x2(v.x, v.y), ix_f32x2_to_bf16x2(v.z, v.w));
 }
 
+// What lanes of a wavefront hand each other through LDS needs no workgroup barrier: its LDS operations are carried out in
+// their order.  This keeps the compiler to that order, too, also where it can show that a lane's own addresses differ; it is
+// no instruction.
+__device__ __forceinline__ void ix_wave_lds_order() { __builtin_amdgcn_wave_barrier(); }
+
 // Sum / maximum over the 64 lanes, result in every lane.  Within a row of 16 lanes the partners come through
 // DPP (lanes ^1, ^2, then the half row and the row mirrored: no LDS round trip), across rows through two
 // exchanges.  The order of the additions is fixed.

@@ -148,13 +148,15 @@ __device__ __forceinline__ void grouped_body(const TI* a, const TI* w,
       for (int t = 0; t < MT; ++t) x_[t][j] = *reinterpret_cast<const piece_t*>(xr[t] + kk);
     }
   };
-  // (a wavefront's LDS operations are carried out in their order: what the last round left is read before it is written over)
+  // (what the last round left is read before it is written over)
   auto turn_over = [&](piece_t (&w_)[NACC][4]) {
+    ix_wave_lds_order();
 #pragma unroll
     for (int u = 0; u < NACC; ++u)
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         *reinterpret_cast<piece_t*>(turn_at(8 * (j & 1) + (lane >> 3), 8 * (j >> 1) + (lane & 7)) + 4096 * u) = w_[u][j];
+    ix_wave_lds_order();
   };
   auto multiply = [&](int k0, const piece_t (&x_)[MT][4]) {
     piece_t w_[NACC][4];

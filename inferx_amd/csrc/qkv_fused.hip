@@ -68,14 +68,15 @@ qkv_rope_skinny_kernel(const __bf16* x, const __bf16* w, const void* __restrict_
     }
   };
   auto multiply = [&](int k0, const Step& st) {
-    // turned over in LDS (a wavefront's LDS operations are carried out in their order)
-    bf16x8 fl[4], fh[4];
+    bf16x8 fl[4], fh[4];  // turned over in LDS
+    ix_wave_lds_order();
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       char* to = turn_at(8 * (j & 1) + (lane >> 3), 8 * (j >> 1) + (lane & 7));
       *reinterpret_cast<bf16x8*>(to) = st.fl[j];
       *reinterpret_cast<bf16x8*>(to + 4096) = st.fh[j];
     }
+    ix_wave_lds_order();
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const char* from = turn_at(m, 4 * j + g);

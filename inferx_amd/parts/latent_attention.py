@@ -65,7 +65,7 @@ class LatentAttention(Mixer):
             if getattr(self.position, "begin", 0) != 0 or dims <= 0 or dims % 2 or dims > self.rot_dim:
                 raise ValueError(f"the position encoding must rotate the first {dims} elements of a rotated part of "
                                  f"{self.rot_dim}: an even number within the part, from its start")
-        self.w_in = self.w_uk = self.w_uv_t = self.w_out = self.norm_weight = None
+        self.w_in = self.w_uk = self.w_uv_t = self.w_uk_rows = self.w_uv_rows = self.w_out = self.norm_weight = None
 
     def cache_need(self) -> CacheNeed:
         return CacheNeed((CacheArray("latent", 1, self.rank + self.rot_dim),), self.window)
@@ -101,9 +101,13 @@ class LatentAttention(Mixer):
         self.w_uk = uk.contiguous().view(H, self.head_dim, self.rank)
         w_uv = uv.contiguous().view(H, self.value_dim, self.rank)
         self.w_uv_t = w_uv.transpose(1, 2).contiguous()
-        # the same with the reduction's numbers side by side, for steps of few tokens: [H, rank, head_dim], [H, value_dim, rank]
-        few = rt.dtype == torch.bfloat16
-        self.w_uk_rows, self.w_uv_rows = (self.w_uk.transpose(1, 2).contiguous(), w_uv) if few else (None, None)
+        # The same with the reduction's numbers side by side, [H, rank, head_dim] and [H, value_dim, rank], for steps of few
+        # tokens, kept beside the others where the kernel for them can take the sizes (twice the two weights: 4 MB a layer at 16
+        # heads of 128 and a rank of 512).
+        fits = lambda n, width: rt.dtype == torch.bfloat16 and n % 16 == 0 and width % 32 == 0
+        whole_pieces = self.q_dim % 8 == 0 and self.w_in.shape[0] % 8 == 0  # rows of q lie on 16-byte boundaries
+        self.w_uk_rows = self.w_uk.transpose(1, 2).contiguous() if whole_pieces and fits(self.rank, self.head_dim) else None
+        self.w_uv_rows = w_uv if fits(self.value_dim, self.rank) else None
         self.w_out = tensors["o.weight"].contiguous()
         self.norm_weight = norm.contiguous()
         if self.position is not None:

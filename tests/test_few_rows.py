@@ -17,3 +17,24 @@ def test_products_of_few_rows(dtype, rows, features, reduction, off, streamed):
     w = torch.zeros(features, reduction, dtype=dtype)
     assert rt._skinny_ok(x, w) == streamed
     assert not rt._skinny_ok(x, w.to(torch.float64))
+
+
+@pytest.mark.parametrize("dtype,heads,dim,rot,vdim,rank,gate,uk,uv", [
+    (torch.bfloat16, 4, 64, 32, 48, 96, False, True, True), (torch.float32, 4, 64, 32, 48, 96, False, False, False),
+    (torch.bfloat16, 4, 48, 32, 48, 96, False, False, True),   # a reduction of 48
+    (torch.bfloat16, 4, 64, 32, 40, 96, False, True, False),   # values of 40
+    (torch.bfloat16, 4, 64, 32, 48, 80, False, True, False),   # a rank of 80: rows of weights, but no reduction
+    (torch.bfloat16, 4, 64, 36, 48, 96, False, False, True),   # heads of 100 numbers
+    (torch.bfloat16, 5, 64, 32, 4, 96, True, False, False),    # rows of 20 numbers more: q does not lie on 16 bytes
+    (torch.bfloat16, 4, 64, 0, 48, 70, False, True, True)])    # brought to 96
+def test_latent_attention_keeps_weights_twice_only_where_few_tokens_use_them(dtype, heads, dim, rot, vdim, rank, gate, uk, uv):
+    from inferx_amd.parts.latent_attention import LatentAttention
+    rt = Runtime.__new__(Runtime)
+    rt.dtype = dtype
+    part = LatentAttention(64, heads, dim, rot, vdim, rank, gate=gate)
+    part.bind({p.name: torch.randn(p.shape).to(dtype) for p in part.param_specs()}, rt)
+    assert ((part.w_uk_rows is not None), (part.w_uv_rows is not None)) == (uk, uv)
+    if uk:
+        assert torch.equal(part.w_uk_rows.transpose(1, 2), part.w_uk)
+    if uv:
+        assert torch.equal(part.w_uv_rows.transpose(1, 2), part.w_uv_t)

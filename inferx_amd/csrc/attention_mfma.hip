@@ -556,7 +556,8 @@ static void launch_attn(dim3 grid, hipStream_t stream, const void* q, const void
   if (PF) grid = dim3(static_cast<unsigned>((waves + per_group - 1) / per_group));
   else grid.x = static_cast<unsigned>((static_cast<int64_t>(n_tiles) * n_splits + per_group - 1) / per_group);
   // Decoding: no slice under 128 keys, or 256 where the launch fills the chip twice over (2,048 wavefronts); what a
-  // wavefront waits for before its first keys (its tile, its position, its pages) is worth about as many.  So a short
+  // wavefront waits for before its first keys (its tile, its position, its pages) is worth about as many.  Up to 512 wavefronts,
+  // which leave the chip half empty, only whole rounds are asked for (32).  So a short
   // context beside long ones is not cut as often as they are.  Eight contexts of 2,048 in slices of 256 and 128 keys:
   // 26.7 and 29.0 us; eight of 200 to 2,048: 19.5 and 22.1; 4 of 200 to 2,048, 128 keys and equal shares: 13.2 and 14.5.
   const int min_slice = !PF || waves <= 512 ? 32 : (waves < 2048 ? 128 : 256);

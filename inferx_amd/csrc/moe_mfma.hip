@@ -17,8 +17,8 @@
 // 128 of K (in float32 64: 256 bytes of a row either way).  The matrix cores want
 // 64 contiguous bytes of sixteen rows at once, memory wants whole lines of 128:
 // so a load brings 128 contiguous bytes of eight weight rows, past the caches
-// (non-temporal: a weight is used once a step), and the wavefront turns them over
-// through 4 KB of LDS of its own, with no barrier.  The activations, which every
+// (non-temporal: a tile of rows uses a weight once), and the wavefront turns them over
+// through 4 KB of LDS of its own, with no workgroup barrier.  The activations, which every
 // workgroup reads, come from the caches as operands: in load j lane (m, g) reads
 // the 16 bytes at k0 + 32 j + 8 g of row m (in float32 the j-th numbers of the four
 // groups' pieces meet in one instruction).  KSPLIT = 4 (decoding: few rows, the
@@ -33,6 +33,10 @@
 // shared one of 20,480, rows of 3,584, eight rows on 41 experts 264 + 130 (322 + 166).  The logits of a vocabulary of
 // 151,936, rows of 2,048: one 95 (111), eight 98 (134), sixteen 110 (154), 32 153 (184); of 3,584: sixteen 197 (273).  Two
 // blocks of weights a wavefront (gate|up, logits) take three wavefronts a SIMD, in whose registers nothing is spilled.
+//
+// Past the caches also where several tiles of sixteen rows ask for the same weights (steps of 17 to 48 rows, the shared
+// expert's tiles): they are read again, and it is still faster than lines that stay (us, both products in turn at those sizes,
+// past | through the caches: 17 rows 142 | 155, 32 162 | 175, 33 with the shared expert in pieces 162 | 176, 45 173 | 187).
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));

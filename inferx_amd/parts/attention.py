@@ -506,12 +506,12 @@ def _n_splits(units: int, longest: int, span: int, tile: int) -> int:
 
 def decode_slices(units: int, longest: int, span: int) -> int:
     """Into how many slices at most the wavefront-level kernel cuts the keys of a step of one token per request
-    (bfloat16): as many as make up WAVES_WANTED wavefronts, none under 128 keys (64, up to 32 slices, where one request
-    leaves the chip half empty: 517 keys of 16 heads in 16 and 8 slices 7.4 and 9.0 us), and at least one for every 512
-    keys, since contexts may differ: the kernel gives short ones fewer (a floor under the slices' length), so that no
-    wavefront walks a long context while the others are done.  64 requests of 200 to 2,048 tokens in 2, 4 and 8 slices:
-    85, 78 and 78 us; 64 of 2,048 each: 164, 168 and 172.  A power of two; at most 64, and 16,384 wavefronts (the parts'
-    room)."""
+    (bfloat16).  It goes by the longest context, rounded up to a power of two: as many as make up WAVES_WANTED wavefronts, none
+    under 128 of those keys (64, up to 32 slices, where one request leaves the chip half empty: 517 keys of 16 heads in 16 and 8
+    slices 7.4 and 9.0 us), and at least one for every 512, since contexts may differ: the kernel gives short ones fewer (a
+    floor under the slices' length, 32 keys up to 512 wavefronts, 128 and 256 in larger launches), so that no wavefront walks a
+    long context while the others are done.  64 requests of 200 to 2,048 tokens in 2, 4 and 8 slices: 85, 78 and 78 us; 64 of
+    2,048 each: 164, 168 and 172.  A power of two; at most 64, and 16,384 wavefronts (the parts' room)."""
     longest = 1 << max(longest - 1, 0).bit_length()  # as captured steps round it: a step and its replay are cut alike
     keys = min(longest, abs(span) + QUERY_TILE + 32) if span else longest
     by_keys = max(-(-keys // MIN_KEYS_PER_SPLIT), min(-(-keys // 64), 32) if units <= 16 else 1)

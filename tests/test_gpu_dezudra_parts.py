@@ -670,6 +670,43 @@ def test_one_key_stands_out_for_every_query_of_a_portion(kernel):
                 f"portion ending at {last}, key {key}: queries {np.flatnonzero((err < 3e-2) != seen).tolist()} of the portion are wrong"
 
 
+@pytest.mark.parametrize("V", [64, 128])
+@pytest.mark.parametrize("window,keep", [(37, 5), (70, 40), (64, 16), (0, 0)])
+def test_one_key_stands_out_for_every_query_through_lds(V, window, keep):
+    """As above for the kernel that shares keys through LDS: portions of 150 queries (tiles of 64, 64 and 22, the last one's
+    third and fourth wavefronts without queries); keys at both edges of sixteens, rounds of 32, tiles, the window and the kept
+    first tokens; portions that end at a page's edge, within a page and where the window has left the first keys."""
+    from inferx_amd import ops
+    H, G, D, L, n, page, eps, dtype = 2, 1, 64, 400, 150, 16, 1e-6, torch.bfloat16
+    k, v = rnd((L, 2 * G, D), 1, 0.05), rnd((L, G, V), 2, 1.0, dtype)
+    mark = torch.zeros(D)
+    mark[7] = 40.0
+    kc, vc, table = paged(k.to(dtype), v, page, dtype)
+    q = torch.zeros((n, H, 2, D))
+    q[:, :, 0] = mark
+    for last in (149, 159, 255, 399):
+        first = last - n + 1
+        positions = np.arange(first, last + 1)
+        tiles = torch.tensor([(0, at, min(64, n - at)) for at in range(0, n, 64)], dtype=torch.int32, device=DEV).t().contiguous()
+        edges = [first, last, first + 63, first + 64, first + 127, last - 22, last - 6]
+        keys = {0, 15, 16, 31, 32, 47, 48, keep - 1, keep, keep + 1} | set(edges)
+        keys |= {e - window + d for e in edges for d in (-1, 0, 1)} | {e // 16 * 16 + d for e in edges for d in (-1, 0, 15)}
+        for key in sorted(j for j in keys if 0 <= j <= last):
+            where = (int(table[0, key // page]), 0, key % page)
+            before = kc[where].clone()
+            kc[where] = mark.to(dtype).to(DEV)
+            out = torch.full((n, H, V), float("nan"), dtype=dtype, device=DEV)
+            ops.attention_diff_prefill(q.to(dtype).to(DEV), kc, vc, table, tiles, i32(positions.tolist()), out, 1.0, window, keep,
+                                       0.0, eps, 1.0)
+            kc[where] = before
+            target = f64(v)[key, 0]
+            target = target / np.sqrt(np.mean(target * target) + eps)
+            err = np.abs(f64(out)[:, 0] - target[None, :]).max(axis=1)
+            seen = (key <= positions) & ((positions - key < window) | (key < keep) | (window == 0))
+            assert np.array_equal(err < 3e-2, seen), \
+                f"portion ending at {last}, key {key}: queries {np.flatnonzero((err < 3e-2) != seen).tolist()} of the portion are wrong"
+
+
 def diff_attention_reference(q, k, v, first, window, keep, lam, eps, scale):
     """q [n, H, 2, D] at positions first.. of one request, k [L, G, 2, D], v [L, G, V]: float64 on the device."""
     n, H = q.shape[:2]

@@ -122,6 +122,44 @@ def test_attention_part_whole_and_in_two_steps(dtype, tol, heads, kv, d, window,
     assert err(run([20, 2, 14, 1]), want) < tol
 
 
+@pytest.mark.parametrize("heads,kv", [(16, 16), (8, 2)])
+@pytest.mark.parametrize("sinks,gated", [(False, False), (True, False), (False, True), (True, True)])
+def test_few_tokens_beside_portions_stay_in_their_rows(heads, kv, sinks, gated):
+    """Short requests beside a portion that the LDS-sharing kernel takes: their launches (grouped heads: one for requests of a
+    few tokens, one for the others) read and write the step's rows where they lie, the gate's too."""
+    from inferx_amd.engine.runtime import CacheBinding, Runtime
+    from inferx_amd.parts import attention
+    import attention_util as au
+    d, page = 128, 16
+    q_lens, seq_lens = [3, 200, 1, 9, 15, 150], [60, 200, 90, 9, 47, 340]
+    part = attention.PagedAttention(64, heads, kv, d)
+    pages = sum(-(-L // page) for L in seq_lens) + 2
+    ctx, batch = make_ctx(Runtime("bfloat16"), q_lens, seq_lens, page, pages)
+    p = au.paged_on_device(seq_lens, q_lens, heads, kv, d, page, seed=5, table=batch.block_tables[0], pages=pages)
+    g = torch.Generator().manual_seed(3)
+    T = sum(q_lens)
+    gate = torch.randn(T, heads * d, generator=g).bfloat16() if gated else None
+    sink = torch.randn(heads, generator=g) if sinks else None
+    part.sink = sink.to(DEV) if sinks else None
+    out = torch.full_like(p["q"], float("nan"))
+    part.attend(ctx, p["q"], CacheBinding(group=0, arrays=dict(k=p["k_cache"], v=p["v_cache"])), out,
+                gate=gate.to(DEV) if gated else None)
+    lds, waves = attention.mixed_step_plan(ctx, 0, heads, kv, True, attention.WIDE_PREFILL_TILE)
+    assert lds is not None and [w[4] for w in waves] == ([True, False] if heads > kv else [False])
+    assert all(w[0] is None and w[3] == 1 for w in waves)
+    row = 0
+    for (k, v), q, L, n in zip(p["dense"], p["qs"], seq_lens, q_lens):
+        s = q.double().cpu().permute(1, 0, 2) @ k.double().cpu().repeat_interleave(heads // kv, 1).permute(1, 2, 0) * d ** -0.5
+        s = s.masked_fill(torch.arange(L)[None, None] > torch.arange(L - n, L)[None, :, None], float("-inf"))
+        extra = sink.double()[:, None, None].expand(heads, n, 1) if sinks else torch.full((heads, n, 1), float("-inf")).double()
+        w = torch.softmax(torch.cat([s, extra], 2), 2)[:, :, :L]
+        want = (w @ v.double().cpu().repeat_interleave(heads // kv, 1).permute(1, 0, 2)).permute(1, 0, 2)
+        if gated:
+            want = want * torch.sigmoid(gate[row:row + n].double()).view(n, heads, d)
+        assert err(out[row:row + n], want) < 1.5e-2, f"request of {n} tokens"
+        row += n
+
+
 @pytest.mark.parametrize("heads,kv,d,window,q_lens,seq_lens,expect", [
     (16, 16, 128, 0, [128], [7000], "slices"),                  # few tiles on a long context: keys in slices
     (28, 4, 128, 0, [1, 300, 1, 2], [5000, 6500, 900, 40], "slices, grouped beside"),  # ... beside requests of one

@@ -271,6 +271,12 @@ class MoeFeedForward(FeedForward):
         """Whether the router's scores, selection and grouping of this step fit the one launch for few tokens."""
         return ops.route_one_launch_fits(tokens, self.hidden_size, self.num_experts)
 
+    def _shared_rides_along(self, tokens: int) -> bool:
+        """Whether the shared expert is among the routed ones, in pieces, in a step of so many tokens: up to the line above, and
+        as far as the grouped products' 32-bit places reach."""
+        rows = tokens * (self.top_k + self.shared_pieces)
+        return self.shared_pieces > 0 and tokens < FOLD_SHARED_BELOW_TOKENS and rows * self.expert_width < 1 << 31
+
     takes_lazy_norm = True
 
     def forward(self, ctx, x):
@@ -285,8 +291,8 @@ class MoeFeedForward(FeedForward):
                 x = x.materialize(ctx)
         tile_rows = self._tile_rows(ctx, x)
         one_launch = self._one_launch(ctx, x, tile_rows)
-        if (self.shared_pieces and tile_rows and not one_launch and norm is None
-                and ctx.rt.SKINNY_ROWS < x.shape[0] < FOLD_SHARED_BELOW_TOKENS):
+        if (tile_rows and not one_launch and norm is None and x.shape[0] > ctx.rt.SKINNY_ROWS
+                and self._shared_rides_along(x.shape[0])):
             # a step of middling size: the shared expert rides along as pieces that every token chooses
             topk_w, _, _, offsets, rows, dest, tile_map = self.route_and_dispatch(ctx, x, tile_rows,
                                                                                   always=self.shared_pieces)

@@ -38,3 +38,12 @@ def test_latent_attention_keeps_weights_twice_only_where_few_tokens_use_them(dty
         assert torch.equal(part.w_uk_rows.transpose(1, 2), part.w_uk)
     if uv:
         assert torch.equal(part.w_uv_rows.transpose(1, 2), part.w_uv_t)
+
+
+@pytest.mark.parametrize("pieces,width,tokens,along", [
+    (4, 1408, 33, True), (4, 1408, 1535, True), (4, 1408, 1536, False), (0, 1408, 33, False),
+    (32, 40000, 1535, True), (32, 48000, 767, True), (32, 48000, 1355, True), (32, 48000, 1356, False)])  # 2^31 numbers
+def test_shared_expert_rides_along_as_far_as_the_products_reach(pieces, width, tokens, along):
+    from inferx_amd.parts.moe import MoeFeedForward
+    part = MoeFeedForward(64, 4, 1, width, pieces * width)
+    assert part._shared_rides_along(tokens) == along

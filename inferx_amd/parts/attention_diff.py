@@ -146,30 +146,38 @@ class DifferentialAttention(Mixer):
         if key in ctx.memo:
             return ctx.memo[key]
         tiles, n_tiles, longest = plan_tiles(ctx, PREFILL_TILE)
-        q_start = ctx.host.q_start.astype(np.int64)
-        n, lens = q_start[1:] - q_start[:-1], ctx.host.seq_lens.astype(np.int64)
-        many, few = np.flatnonzero(n >= PREFILL_MIN_ROWS), np.flatnonzero((n > 0) & (n < PREFILL_MIN_ROWS))
         workgroups = n_tiles * self.num_heads
         turns = -(-workgroups // 512) * -(-longest // 32)
         plan = None
-        if turns <= 4:
-            plan = (tiles, None)
-        elif workgroups < PREFILL_MIN_WORKGROUPS:
+        if workgroups < PREFILL_MIN_WORKGROUPS or turns <= 4:
             if turns <= 8 or (turns <= 12 and ctx.num_tokens >= 256):
                 plan = (tiles, None)
-        elif 4 * (n_tiles - len(few)) >= len(few):
-            plan = (tiles, None)
-            keys = int(lens[few].max()) if len(few) else 0
-            if (min(keys, self.window + self.keep_first) if self.window > 0 else keys) > PREFILL_MAX_FEW_KEYS:
-                to_dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(ctx.rt.device)
-                grouped = 2 <= self.num_heads // self.num_kv_heads <= 16
-                own = _tiles_of(n[few], np.cumsum(n[few]) - n[few], few, 1 if grouped else QUERY_TILE)
-                rows = to_dev(np.concatenate([np.arange(q_start[i], q_start[i + 1]) for i in few]))
-                slices = self.key_slices(own.shape[1] * 2 * (self.num_kv_heads if grouped else self.num_heads), keys)
-                plan = (to_dev(_tiles_of(n[many], q_start[many], many, PREFILL_TILE)),
-                        (rows, to_dev(own), ctx.positions.index_select(0, rows), slices, grouped))
+        else:
+            q_start = ctx.host.q_start
+            n = q_start[1:] - q_start[:-1]
+            if n.min() >= PREFILL_MIN_ROWS:
+                plan = (tiles, None)
+            else:
+                few = np.flatnonzero((n > 0) & (n < PREFILL_MIN_ROWS))
+                if 4 * (n_tiles - len(few)) >= len(few):
+                    keys = int(ctx.host.seq_lens[few].max()) if len(few) else 0
+                    read = min(keys, self.window + self.keep_first) if self.window > 0 else keys
+                    plan = (tiles, None) if read <= PREFILL_MAX_FEW_KEYS else self._few_by_themselves(ctx, n, few, keys)
         ctx.memo[key] = plan
         return plan
+
+    def _few_by_themselves(self, ctx, n, few, keys: int):
+        """`portion_plan` with a launch of their own for the requests `few` (n: every request's new tokens, keys: the longest
+        context among `few`): their rows are put side by side, since slices are merged for all rows of a launch."""
+        n, q_start = n.astype(np.int64), ctx.host.q_start.astype(np.int64)
+        to_dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(ctx.rt.device)
+        grouped = 2 <= self.num_heads // self.num_kv_heads <= 16
+        own = _tiles_of(n[few], np.cumsum(n[few]) - n[few], few, 1 if grouped else QUERY_TILE)
+        rows = to_dev(np.concatenate([np.arange(q_start[i], q_start[i + 1]) for i in few]))
+        slices = self.key_slices(own.shape[1] * 2 * (self.num_kv_heads if grouped else self.num_heads), keys)
+        many = np.flatnonzero(n >= PREFILL_MIN_ROWS)
+        return (to_dev(_tiles_of(n[many], q_start[many], many, PREFILL_TILE)),
+                (rows, to_dev(own), ctx.positions.index_select(0, rows), slices, grouped))
 
     def attend(self, ctx, q, cache, out) -> None:
         """bfloat16 with heads and pages that the matrix-core kernels are built for: those, prompt portions in tiles of 64
@@ -184,7 +192,7 @@ class DifferentialAttention(Mixer):
             tiles, few = plan
             ops.attention_diff_prefill(q, cache.k, cache.v, ctx.block_tables[cache.group], tiles, ctx.positions, out,
                                        self.scale, self.window, self.keep_first, self.lam, self.norm_eps, 1.0 - self.diff)
-            if few is not None:  # their rows are put side by side: slices are merged for all rows of a launch
+            if few is not None:
                 rows, tiles, positions, n_splits, grouped = few
                 own = q.index_select(0, rows)
                 result = ctx.rt.empty((rows.numel(), self.num_heads, self.value_dim))

@@ -74,12 +74,14 @@ attn_mfma_kernel(const __bf16* __restrict__ q, const __bf16* __restrict__ k_cach
   if constexpr (PF) {
     // Decoding: the heads of a slice side by side, so that the wavefronts of a workgroup take equally long, and the
     // workgroups of a long context go to all dies: with a request's slices side by side (and each head by itself) the
-    // longest of 64 requests that are sorted by length fell to one die.  Slices that only long contexts have come last.
+    // longest of 64 requests that are sorted by length fell to one die.  Slices that only long contexts have come last, and a
+    // request moves on by one place from slice to slice, or all of its slices would go to the same dies (eight of 16 to 16,000
+    // tokens, 16 heads: 87 us without it, 43 with it; 28 heads on 4 sets 38 and 31).
     const int per_slice = GQ ? kv_heads : heads;
     const int slice = unit / per_slice;
     if (slice >= n_tiles * n_splits) return;
     hy = unit - slice * per_slice;
-    split = slice / n_tiles, tile = slice - split * n_tiles;
+    split = slice / n_tiles, tile = (slice - split * n_tiles + split) % n_tiles;
   } else {
     if (unit >= n_tiles * n_splits) return;
     hy = blockIdx.y;

@@ -179,6 +179,22 @@ def test_attention_mfma_of_uneven_contexts(heads, kv_heads, page, window, n_spli
           f"attention_mfma uneven, splits={n_splits}")
 
 
+@pytest.mark.parametrize("heads,kv_heads,d", [(16, 16, 128), (28, 4, 128), (8, 2, 64)])
+@pytest.mark.parametrize("seq_lens,n_splits", [([45], 1), ([700], 5), ([1, 64, 30], 1), ([3, 2000, 300], 64), ([9] * 130 + [64, 33], 1)])
+def test_attention_mfma_of_one_token_each(heads, kv_heads, d, seq_lens, n_splits):
+    """Short contexts, and fewer requests than slices: a request moves on by one place from slice to
+    slice, and every (request, head, slice) is worked once."""
+    from inferx_amd import ops
+    T = len(seq_lens)
+    p = build_paged(seq_lens, [1] * T, heads, kv_heads, d, 16, torch.bfloat16, seed=3)
+    out = torch.full_like(p["q"], float("nan"))
+    work = torch.full((T * heads * n_splits * (d + 2),), float("nan"), device=DEV) if n_splits > 1 else None
+    ops.attention_mfma(p["q"], p["k_cache"], p["v_cache"], p["table"], tiles_for([1] * T, 1), p["positions"], out, n_splits, work,
+                       d ** -0.5, 0, 16, True, grouped=heads > kv_heads)
+    close(out, attention_reference(p, seq_lens, [1] * T, heads, kv_heads, d ** -0.5, 0), TOL[torch.bfloat16],
+          "attention_mfma one token each")
+
+
 PREFILL_CASES = ATTN_CASES + [
     ([1500], [1500], 5, 1, 128, 16, 0),                   # many tiles of one request
     ([777, 300], [130, 300], 4, 2, 112, 16, 0),           # a portion that starts off a tile's edge; odd head blocks

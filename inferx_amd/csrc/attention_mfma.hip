@@ -100,8 +100,9 @@ attn_mfma_kernel(const __bf16* __restrict__ q, const __bf16* __restrict__ k_cach
   const int lo = ix_first_key(pos0, span);
   const int hi = pos0 + (GQ ? 1 : rows);
   const int lo_al = lo & ~(ATTN_KEYS_PER_ITER - 1);
-  const int per = max((((hi - lo_al + n_splits - 1) / n_splits) + ATTN_KEYS_PER_ITER - 1) & ~(ATTN_KEYS_PER_ITER - 1),
-                      min_slice);
+  // (as many equal slices as the least length allows)
+  const int n_here = min(n_splits, (hi - lo_al + min_slice - 1) / min_slice);
+  const int per = (((hi - lo_al + n_here - 1) / n_here) + ATTN_KEYS_PER_ITER - 1) & ~(ATTN_KEYS_PER_ITER - 1);
   const int ks = lo_al + split * per;
   const int ke = min(hi, ks + per);
   if (ks >= ke && split > 0) {  // no keys are left for this slice: the merging kernel reads no more of it than that
@@ -557,12 +558,14 @@ static void launch_attn(dim3 grid, hipStream_t stream, const void* q, const void
   const int per_group = waves >= 4 * 512 ? 4 : (waves >= 2 * 512 ? 2 : 1);
   if (PF) grid = dim3(static_cast<unsigned>((waves + per_group - 1) / per_group));
   else grid.x = static_cast<unsigned>((static_cast<int64_t>(n_tiles) * n_splits + per_group - 1) / per_group);
-  // Decoding: no slice under 128 keys, or 256 where the launch fills the chip twice over (2,048 wavefronts); what a
-  // wavefront waits for before its first keys (its tile, its position, its pages) is worth about as many.  Up to 512 wavefronts,
-  // which leave the chip half empty, only whole rounds are asked for (32).  So a short
-  // context beside long ones is not cut as often as they are.  Eight contexts of 2,048 in slices of 256 and 128 keys:
-  // 26.7 and 29.0 us; eight of 200 to 2,048: 19.5 and 22.1; 4 of 200 to 2,048, 128 keys and equal shares: 13.2 and 14.5.
-  const int min_slice = !PF || waves <= 512 ? 32 : (waves < 2048 ? 128 : 256);
+  // Decoding: the least length of a slice, in which a context is cut as evenly as its number allows: 128 keys, or 256 where the
+  // launch fills the chip twice over (2,048 wavefronts) and two rounds are on their way; what a wavefront waits for before its
+  // first keys (its tile, its position, its pages) is worth about as many.  Up to 512 wavefronts, which leave the chip half
+  // empty, only whole rounds are asked for (32).  So a short context beside long ones is not cut as often as they are.  Eight
+  // contexts of 2,048 in slices of 256 and 128 keys: 26.7 and 29.0 us; eight of 200 to 2,048: 19.5 and 22.1; 4 of 200 to 2,048, 128
+  // keys and equal shares: 13.2 and 14.5.  32 heads of 64 on 8 sets, 64 contexts of 300 as 256 and 44 keys and evenly 18.3 and 15.7
+  // us, 32 of 517 17.8 and 14.7, eight of 100 to 3,000 at 256 and 128 keys 16.7 and 15.6.
+  const int min_slice = !PF || waves <= 512 ? 32 : (waves < 2048 || !TURN ? 128 : 256);
   hipLaunchKernelGGL((attn_mfma_kernel<NB, QT, PF, GQ, MORE, TURN>), grid, dim3(64 * per_group),
                      TURN ? per_group * 32 * 32 * NB : 0, stream, (const __bf16*)q, (const __bf16*)k,
                      (const __bf16*)v, table, tile_seq, tile_q0, tile_rows, positions, (__bf16*)out, part_o, part_ml,

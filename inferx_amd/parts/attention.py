@@ -261,8 +261,8 @@ class PagedAttention(Mixer):
                         out.index_copy_(0, rows, outs)
                 return
             tiles, tile, _, grouped = query_tiles(ctx, self.span, self.num_heads, self.head_dim, self.num_kv_heads)
-            n_splits = decode_slices(tiles.shape[1] * (self.num_kv_heads if grouped else self.num_heads),
-                                     plan_tiles(ctx, tile)[2], self.span)
+            units, longest = tiles.shape[1] * (self.num_kv_heads if grouped else self.num_heads), plan_tiles(ctx, tile)[2]
+            n_splits = decode_slices(units, longest, self.span, self.head_dim)
             work = None
             if n_splits > 1:
                 work = ctx.rt.empty((q.shape[0] * self.num_heads * n_splits * (self.head_dim + 2),), torch.float32)
@@ -504,18 +504,24 @@ def _n_splits(units: int, longest: int, span: int, tile: int) -> int:
     return 1 << (n_splits.bit_length() - 1)
 
 
-def decode_slices(units: int, longest: int, span: int) -> int:
+def decode_slices(units: int, longest: int, span: int, head_dim: int = 128) -> int:
     """Into how many slices at most the wavefront-level kernel cuts the keys of a step of one token per request
     (bfloat16).  It goes by the longest context, rounded up to a power of two: as many as make up WAVES_WANTED wavefronts, none
     under 128 of those keys (64, up to 32 slices, where one request leaves the chip half empty: 517 keys of 16 heads in 16 and 8
-    slices 7.4 and 9.0 us), and at least one for every 512, since contexts may differ: the kernel gives short ones fewer (a
-    floor under the slices' length, 32 keys up to 512 wavefronts, 128 and 256 in larger launches), so that no wavefront walks a
-    long context while the others are done.  64 requests of 200 to 2,048 tokens in 2, 4 and 8 slices: 85, 78 and 78 us; 64 of
-    2,048 each: 164, 168 and 172.  A power of two; at most 64, and 16,384 wavefronts (the parts' room)."""
+    slices 7.4 and 9.0 us; up to 128 keys stay whole: 100 of 28 heads on 4 sets 7.0 us, in two slices and their merging 7.8),
+    and at least one for every 512, since contexts may differ: the kernel gives short ones fewer (a floor under the slices'
+    length, 32 keys up to 512 wavefronts, 128 and 256 in larger launches), so that no wavefront walks a long context while the
+    others are done.  Where whole contexts are two wavefronts a SIMD already, slices hold as many bytes as 512 keys of heads of
+    128 (256 requests of 32 heads of 64 on 8 sets, 1,000 keys each: 104 us in two slices, 96 whole).  64 requests of 200 to
+    2,048 tokens in 2, 4 and 8 slices: 85, 78 and 78 us; 64 of 2,048 each: 164, 168 and 172.  A power of two; at most 64, and
+    16,384 wavefronts (the parts' room)."""
     longest = 1 << max(longest - 1, 0).bit_length()  # as captured steps round it: a step and its replay are cut alike
     keys = min(longest, abs(span) + QUERY_TILE + 32) if span else longest
+    if keys <= MIN_KEYS_PER_SPLIT:
+        return 1
     by_keys = max(-(-keys // MIN_KEYS_PER_SPLIT), min(-(-keys // 64), 32) if units <= 16 else 1)
-    by_length = min(-(-keys // 512), 8 * WAVES_WANTED // max(1, units))
+    least = max(512, 65536 // head_dim) if units >= WAVES_WANTED else 512
+    by_length = min(-(-keys // least), 8 * WAVES_WANTED // max(1, units))
     n_splits = max(1, min(max(WAVES_WANTED // max(1, units), by_length), by_keys, 64))
     return 1 << (n_splits.bit_length() - 1)
 

@@ -47,3 +47,17 @@ def test_shared_expert_rides_along_as_far_as_the_products_reach(pieces, width, t
     from inferx_amd.parts.moe import MoeFeedForward
     part = MoeFeedForward(64, 4, 1, width, pieces * width)
     assert part._shared_rides_along(tokens) == along
+
+
+@pytest.mark.parametrize("units,longest,span,head_dim,slices", [
+    (16, 517, 0, 128, 16), (16, 65, 0, 128, 1), (4, 128, 0, 128, 1), (4, 129, 0, 128, 4),   # one request
+    (4, 64, 0, 128, 1), (32, 40, 0, 128, 1), (33, 40, 0, 128, 1), (2048, 64, 0, 128, 1), (2048, 65, 0, 128, 1),
+    (128, 2048, 0, 128, 16), (1024, 2048, 0, 128, 4), (1024, 2048, 0, 64, 4), (128, 4096, 1024, 128, 8),
+    (2048, 1000, 0, 64, 1), (2048, 1025, 0, 64, 2), (2048, 1000, 0, 128, 2), (4096, 16000, 0, 128, 4)])
+def test_slices_of_decoding(units, longest, span, head_dim, slices):
+    """Up to 128 keys stay whole; whole contexts that are two wavefronts a SIMD already are cut by their bytes.
+    As a captured step rounds its longest context."""
+    from inferx_amd.parts.attention import decode_slices
+    rounded = 1 << (longest - 1).bit_length()
+    for n in (longest, rounded):
+        assert decode_slices(units, n, span, head_dim) == slices

@@ -606,6 +606,7 @@ static int attention_mfma_any(const void* q, const void* k_cache, const void* v_
   const float scale_log2 = scale * 1.4426950408889634f;
   const float cap2 = softcap * 1.4426950408889634f, cap_slope = softcap > 0.f ? 2.0f * scale_log2 / softcap : 0.f;
   const bool more = softcap > 0.f || gate != nullptr;
+  const bool lines = prefetch != 2;  // (decode_loads in parts/attention.py has the line)
 #define ARGS                                                                                                    \
   grid, stream, q, k_cache, v_cache, block_table, tile_seq, tile_q0, tile_rows, positions, out, part_o, part_ml, \
       n_tiles, n_splits, heads, kv_heads, page_size, max_blocks, scale_log2, span, sink, turn_back, cap_slope,    \
@@ -614,10 +615,11 @@ static int attention_mfma_any(const void* q, const void* k_cache, const void* v_
   case NB:                                                          \
     if (grouped) {                                                  \
       if (prefetch && more) launch_attn<NB, 1, true, true>(ARGS);   \
-      else if (prefetch) launch_attn<NB, 1, true, true, false, NB == 8>(ARGS); \
+      else if (prefetch && lines) launch_attn<NB, 1, true, true, false, NB == 8>(ARGS); \
+      else if (prefetch) launch_attn<NB, 1, true, true, false>(ARGS); \
       else launch_attn<NB, 1, false, true>(ARGS);                   \
     } else if (prefetch && more) launch_attn<NB, 1, true>(ARGS);    \
-    else if (prefetch && heads == kv_heads) launch_attn<NB, 1, true, false, false, NB == 8>(ARGS); \
+    else if (prefetch && lines && heads == kv_heads) launch_attn<NB, 1, true, false, false, NB == 8>(ARGS); \
     else if (prefetch) launch_attn<NB, 1, true, false, false>(ARGS); \
     else launch_attn<NB, 1, false>(ARGS);                           \
     break;

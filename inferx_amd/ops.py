@@ -324,7 +324,8 @@ def attention_mfma(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
     """Paged attention on the matrix cores (bfloat16).  `tiles` int32 [3, n_tiles]: request, first token row and
     number of rows (<= tile_queries, which is 16 or 32) of each query tile.  `workspace` float32 with T * heads * n_splits * (d + 2) entries
     when n_splits > 1.  `grouped`: every tile is ONE token, and the query heads of a key/value head (at most 16)
-    are served together, so that its keys and values are read once for all of them."""
+    are served together, so that its keys and values are read once for all of them.  `prefetch`: tiles of one token each, whose
+    keys and values are asked for ahead (2: heads of 128 in half lines, which short contexts are better with)."""
     T, heads, d = q.shape
     _need(q.dtype == torch.bfloat16, "the matrix-core attention kernel is bfloat16 only")
     _need(out.shape == q.shape and out.dtype == q.dtype, "out mismatch")
@@ -348,7 +349,7 @@ def attention_mfma(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
     args = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), _ptr(tiles[0]),
             _ptr(tiles[1]), _ptr(tiles[2]), _ptr(positions), _ptr(out), _ptr(part_o), _ptr(part_ml), _i64(T),
             _i32(n_tiles), _i32(tile_queries), _i32(n_splits), _i32(heads), _i32(kv_heads), _i32(d), _i32(page_size),
-            _i32(block_table.shape[1]), _f32(scale), _i32(span), _i32(1 if prefetch else 0),
+            _i32(block_table.shape[1]), _f32(scale), _i32(span), _i32(int(prefetch)),
             _i32(1 if grouped else 0))
     if sink is None and turn_back is None and softcap <= 0 and gate is None:
         _call("ix_attention_mfma", *args, _stream())

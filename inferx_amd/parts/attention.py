@@ -267,7 +267,7 @@ class PagedAttention(Mixer):
             if n_splits > 1:
                 work = ctx.rt.empty((q.shape[0] * self.num_heads * n_splits * (self.head_dim + 2),), torch.float32)
             ops.attention_mfma(q, cache.k, cache.v, ctx.block_tables[cache.group], tiles, ctx.positions, out,
-                               n_splits, work, self.scale, self.span, tile, prefetch=True, grouped=grouped, **more)
+                               n_splits, work, self.scale, self.span, tile, prefetch=decode_loads(units, longest), grouped=grouped, **more)
         else:
             if (q.dtype == torch.float32 and turn_back is None and self.value_dim == self.head_dim
                     and page_size % 16 == 0 and self.head_dim % 16 == 0):
@@ -524,6 +524,15 @@ def decode_slices(units: int, longest: int, span: int, head_dim: int = 128) -> i
     by_length = min(-(-keys // least), 8 * WAVES_WANTED // max(1, units))
     n_splits = max(1, min(max(WAVES_WANTED // max(1, units), by_length), by_keys, 64))
     return 1 << (n_splits.bit_length() - 1)
+
+
+def decode_loads(units: int, longest: int) -> int:
+    """How that kernel asks for keys and values of heads of 128: whole lines through LDS (1), or half lines straight into the
+    operands' registers (2) where no context has more than 64 keys and there are few wavefronts, which LDS makes wait longer, or
+    so many that the form of fewer registers has two of them on a SIMD.  30 keys, lines and half lines, us: two and four
+    requests of 28 heads on 4 sets 4.3 and 4.4 (3.9), 16 and 64 of 16 heads 5.0 and 7.3 (5.2, 8.4), 128 and 256 13.0 and 24.3
+    (11.0, 19.4)."""
+    return 2 if 1 << max(longest - 1, 0).bit_length() <= 64 and not 32 < units < WAVES_WANTED else 1
 
 
 def query_tiles(ctx, span: int, heads: int, head_dim: int = 128, kv_heads: Optional[int] = None):

@@ -49,15 +49,15 @@ def test_shared_expert_rides_along_as_far_as_the_products_reach(pieces, width, t
     assert part._shared_rides_along(tokens) == along
 
 
-@pytest.mark.parametrize("units,longest,span,head_dim,slices", [
-    (16, 517, 0, 128, 16), (16, 65, 0, 128, 1), (4, 128, 0, 128, 1), (4, 129, 0, 128, 4),   # one request
-    (4, 64, 0, 128, 1), (32, 40, 0, 128, 1), (33, 40, 0, 128, 1), (2048, 64, 0, 128, 1), (2048, 65, 0, 128, 1),
-    (128, 2048, 0, 128, 16), (1024, 2048, 0, 128, 4), (1024, 2048, 0, 64, 4), (128, 4096, 1024, 128, 8),
-    (2048, 1000, 0, 64, 1), (2048, 1025, 0, 64, 2), (2048, 1000, 0, 128, 2), (4096, 16000, 0, 128, 4)])
-def test_slices_of_decoding(units, longest, span, head_dim, slices):
-    """Up to 128 keys stay whole; whole contexts that are two wavefronts a SIMD already are cut by their bytes.
-    As a captured step rounds its longest context."""
-    from inferx_amd.parts.attention import decode_slices
+@pytest.mark.parametrize("units,longest,span,head_dim,slices,loads", [
+    (16, 517, 0, 128, 16, 1), (16, 65, 0, 128, 1, 1), (4, 128, 0, 128, 1, 1), (4, 129, 0, 128, 4, 1),   # one request
+    (4, 64, 0, 128, 1, 2), (32, 40, 0, 128, 1, 2), (33, 40, 0, 128, 1, 1), (2048, 64, 0, 128, 1, 2), (2048, 65, 0, 128, 1, 1),
+    (128, 2048, 0, 128, 16, 1), (1024, 2048, 0, 128, 4, 1), (1024, 2048, 0, 64, 4, 1), (128, 4096, 1024, 128, 8, 1),
+    (2048, 1000, 0, 64, 1, 1), (2048, 1025, 0, 64, 2, 1), (2048, 1000, 0, 128, 2, 1), (4096, 16000, 0, 128, 4, 1)])
+def test_slices_and_loads_of_decoding(units, longest, span, head_dim, slices, loads):
+    """Up to 128 keys stay whole; whole contexts that are two wavefronts a SIMD already are cut by their bytes; half lines for
+    few or very many wavefronts on up to 64 keys.  As a captured step rounds its longest context."""
+    from inferx_amd.parts.attention import decode_loads, decode_slices
     rounded = 1 << (longest - 1).bit_length()
     for n in (longest, rounded):
-        assert decode_slices(units, n, span, head_dim) == slices
+        assert (decode_slices(units, n, span, head_dim), decode_loads(units, n)) == (slices, loads)

@@ -181,8 +181,9 @@ def test_attention_mfma_of_uneven_contexts(heads, kv_heads, page, window, n_spli
 
 @pytest.mark.parametrize("heads,kv_heads,d", [(16, 16, 128), (28, 4, 128), (8, 2, 64)])
 @pytest.mark.parametrize("seq_lens,n_splits", [([45], 1), ([700], 5), ([1, 64, 30], 1), ([3, 2000, 300], 64), ([9] * 130 + [64, 33], 1)])
-def test_attention_mfma_of_one_token_each(heads, kv_heads, d, seq_lens, n_splits):
-    """Short contexts, and fewer requests than slices: a request moves on by one place from slice to
+@pytest.mark.parametrize("prefetch", [1, 2])
+def test_attention_mfma_of_one_token_each_in_lines_and_half_lines(heads, kv_heads, d, seq_lens, n_splits, prefetch):
+    """Short contexts in either form of loads, and fewer requests than slices: a request moves on by one place from slice to
     slice, and every (request, head, slice) is worked once."""
     from inferx_amd import ops
     T = len(seq_lens)
@@ -190,9 +191,9 @@ def test_attention_mfma_of_one_token_each(heads, kv_heads, d, seq_lens, n_splits
     out = torch.full_like(p["q"], float("nan"))
     work = torch.full((T * heads * n_splits * (d + 2),), float("nan"), device=DEV) if n_splits > 1 else None
     ops.attention_mfma(p["q"], p["k_cache"], p["v_cache"], p["table"], tiles_for([1] * T, 1), p["positions"], out, n_splits, work,
-                       d ** -0.5, 0, 16, True, grouped=heads > kv_heads)
+                       d ** -0.5, 0, 16, prefetch, grouped=heads > kv_heads)
     close(out, attention_reference(p, seq_lens, [1] * T, heads, kv_heads, d ** -0.5, 0), TOL[torch.bfloat16],
-          "attention_mfma one token each")
+          f"attention_mfma one token each, prefetch={prefetch}")
 
 
 PREFILL_CASES = ATTN_CASES + [

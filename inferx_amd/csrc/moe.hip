@@ -262,7 +262,8 @@ moe_route_logits_f64_kernel(const float* __restrict__ x, const float* __restrict
 
 // `bias` (float32 [experts], or null) is added to the experts' scores before anything else.
 // `logits_scratch`: float32 [tokens, experts + 1], used when tokens <= ROUTE_SMALL_TOKENS, and for more tokens when
-// activations and weights are bfloat16 or all float32 (may be null: then one kernel per token computes and selects).
+// activations and weights are bfloat16, or all float32 with many experts or tokens (may be null: then one kernel per token
+// computes and selects).
 #define ROUTE_SMALL_TOKENS 128
 extern "C" int ix_moe_route(const void* x, int dtype, const void* wr, int wr_dtype, const void* shared_gate_w,
                             int sg_dtype, const float* bias, float* topk_w, int32_t* topk_e, float* shared_gate,
@@ -308,7 +309,10 @@ extern "C" int ix_moe_route(const void* x, int dtype, const void* wr, int wr_dty
                        scale, always, n_groups, groups_keep);
     return ix_check_launch("ix_moe_route");
   }
-  if (logits_scratch != nullptr && dtype == IX_F32 && wr_dtype == IX_F32 &&
+  // (With few experts a workgroup a token reads little for itself, and it is one launch with nothing to wait for in between:
+  // that one | the two, us, 1,024 tokens of 2,048 numbers, four experts 8.9 | 16.7, sixteen 12.5 | 17.6, 32 18.5 | 18.7, 64 27.9 |
+  // 22.3; 4,096 tokens, four 19.5 | 20.0, sixteen 30.7 | 24.0.)
+  if (logits_scratch != nullptr && (experts > 32 || tokens > 2048) && dtype == IX_F32 && wr_dtype == IX_F32 &&
       (shared_gate_w == nullptr || sg_dtype == IX_F32) && width % 4 == 0 && width < (1 << 30) &&
       ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(wr) | reinterpret_cast<uintptr_t>(shared_gate_w)) & 15) == 0) {
     const int row_blocks = (experts + (shared_gate_w ? 1 : 0) + 15) / 16;

@@ -49,6 +49,21 @@ def test_route(T, H, E, k, renorm, dtype):
         assert (sums < 0.9999).all()
 
 
+@pytest.mark.parametrize("T,E", [(129, 32), (129, 33), (2048, 32), (2049, 32), (2049, 4), (300, 4)])
+def test_route_of_few_experts_and_many(T, E):
+    """float32 tokens on both sides of the lines between one kernel per token and the scores as a product with 64-bit sums."""
+    from inferx_amd import ops
+    H, k = 60, 3
+    x, wr = rnd(T, H), rnd(E, H, seed=1, scale=0.3)
+    topk_w, topk_e = torch.empty(T, k, device=DEV), torch.empty(T, k, dtype=torch.int32, device=DEV)
+    ops.moe_route(x, wr, None, topk_w, topk_e, None, True, 1.0)
+    want_w, want_e = route_reference(x, wr, k, True)
+    margin = torch.topk(x.double().cpu() @ wr.double().cpu().T, k + 1, dim=-1).values
+    sure = (margin[:, :-1] - margin[:, 1:]).min(-1).values > 1e-5  # (float32 sums of 60 numbers: 1e-6 of scores up to 10)
+    assert int(sure.sum()) > 0.99 * T and torch.equal(topk_e.cpu().long()[sure], want_e[sure])
+    assert rel_err(topk_w[sure.to(DEV)], want_w[sure]) < 1e-5
+
+
 def test_route_refuses_what_it_cannot_do():
     from inferx_amd import ops
     x, wr = rnd(4, 96), rnd(40, 96, seed=1)

@@ -512,16 +512,16 @@ def decode_slices(units: int, longest: int, span: int, head_dim: int = 128) -> i
     and at least one for every 512, since contexts may differ: the kernel gives short ones fewer (a floor under the slices'
     length, 32 keys up to 512 wavefronts, 128 and 256 in larger launches), so that no wavefront walks a long context while the
     others are done.  Where whole contexts are two wavefronts a SIMD already, slices hold as many bytes as 512 keys of heads of
-    128 (256 requests of 32 heads of 64 on 8 sets, 1,000 keys each: 104 us in two slices, 96 whole).  64 requests of 200 to
-    2,048 tokens in 2, 4 and 8 slices: 85, 78 and 78 us; 64 of 2,048 each: 164, 168 and 172.  A power of two; at most 64, and
-    16,384 wavefronts (the parts' room)."""
+    128 at least (256 requests of 32 heads of 64 on 8 sets, 1,000 keys each: 104 us in two slices, 96 whole).  64 requests of
+    200 to 2,048 tokens in 2, 4 and 8 slices: 85, 78 and 78 us; 64 of 2,048 each: 164, 168 and 172.  A power of two; at most 64,
+    and 16,384 wavefronts (the parts' room)."""
     longest = 1 << max(longest - 1, 0).bit_length()  # as captured steps round it: a step and its replay are cut alike
     keys = min(longest, abs(span) + QUERY_TILE + 32) if span else longest
     if keys <= MIN_KEYS_PER_SPLIT:
         return 1
     by_keys = max(-(-keys // MIN_KEYS_PER_SPLIT), min(-(-keys // 64), 32) if units <= 16 else 1)
-    least = max(512, 65536 // head_dim) if units >= WAVES_WANTED else 512
-    by_length = min(-(-keys // least), 8 * WAVES_WANTED // max(1, units))
+    by_length = max(1, keys // max(512, 65536 // head_dim)) if units >= WAVES_WANTED else -(-keys // 512)
+    by_length = min(by_length, 8 * WAVES_WANTED // max(1, units))
     n_splits = max(1, min(max(WAVES_WANTED // max(1, units), by_length), by_keys, 64))
     return 1 << (n_splits.bit_length() - 1)
 

@@ -53,7 +53,7 @@ def test_shared_expert_rides_along_as_far_as_the_products_reach(pieces, width, t
     (16, 517, 0, 128, 16, 1), (16, 65, 0, 128, 1, 1), (4, 128, 0, 128, 1, 1), (4, 129, 0, 128, 4, 1),   # one request
     (4, 64, 0, 128, 1, 2), (32, 40, 0, 128, 1, 2), (33, 40, 0, 128, 1, 1), (2048, 64, 0, 128, 1, 2), (2048, 65, 0, 128, 1, 1),
     (128, 2048, 0, 128, 16, 1), (1024, 2048, 0, 128, 4, 1), (1024, 2048, 0, 64, 4, 1), (128, 4096, 1024, 128, 8, 1),
-    (2048, 1000, 0, 64, 1, 1), (2048, 1025, 0, 64, 2, 1), (2048, 1000, 0, 128, 2, 1), (4096, 16000, 0, 128, 4, 1)])
+    (2048, 1000, 0, 64, 1, 1), (2048, 1025, 0, 64, 2, 1), (2048, 4096, 1024, 64, 1, 1), (2048, 4096, 1024, 128, 2, 1), (2048, 1000, 0, 128, 2, 1), (4096, 16000, 0, 128, 4, 1)])
 def test_slices_and_loads_of_decoding(units, longest, span, head_dim, slices, loads):
     """Up to 128 keys stay whole; whole contexts that are two wavefronts a SIMD already are cut by their bytes; half lines for
     few or very many wavefronts on up to 64 keys.  As a captured step rounds its longest context."""

@@ -32,21 +32,20 @@ from .dense_mlp import stack_rows
 from .short_conv import ShortConv
 
 
-# A step that brings some request several tokens goes through the kernel that shares keys and values through LDS, or through
-# the wavefront-level one, which cuts keys into slices where a step has few tiles.  A workgroup of the former (a tile of up to
-# 64 queries of a head, two on a compute unit) walks all of its keys, 1.3 us for 32 of them, however few queries it has.  us,
-# wavefront-level / LDS, 16 heads:
-#   no context long (`turns`: rounds of 32 keys times how often 512 workgroups fill the chip): eight prompts of 200 37 / 16,
-#   one of 300 19.5 / 17.5, 64 tokens on 256 16.2 / 15.0, on 384 16.3 / 18.6; sixteen single tokens on 128 beside 64 15.6 / 13.2,
-#   on 256 15.9 / 17.9; 32 on 64 15.5 / 13.1, on 128 16.0 / 18.0
-#   a workgroup for every compute unit, and the portions' tiles at least a quarter as many as the single tokens': prompts of 611
-#   and 1,437 with a window of 1,024 105 / 48; 300 tokens beside sixteen single ones on 1,000 and 2,000 keys 67 / 51 and 119 / 90,
-#   beside 32 73 / 83 and 132 / 150; 64 beside sixteen 37 / 51 and 64 / 90
-#   single tokens on more than 2,048 keys in a launch of their own, in slices (`portion_plan`), in one LDS launch / two: 1,200
-#   tokens beside sixteen single ones on 1,500, 2,000, 3,000 and 30,000 89 / 84, 106 / 101, 142 / 107 and 1,141 / 306, beside four on
-#   2,000 and 3,000 88 / 90 and 123 / 94
+# A step that brings some request several tokens goes through the kernel that shares keys and values through LDS, or through the
+# wavefront-level one, which cuts keys into slices where a step has few tiles.  A workgroup of the former (a tile of up to 64
+# queries of a head) walks all of its keys however few queries it has, so which is the quicker goes by the rounds of 32 keys of
+# the longest tile and of all tiles together (`portion_plan`).  The estimates are fitted to 2,776 steps of 0 to 64 single tokens
+# on 100 to 4,000 keys beside portions of 2 to 700 on up to 3,000, 8 to 32 heads, maps and values of 64 and 128: the chosen kernel
+# is 0.6 % from the quicker one on average (the LDS one always 49 %, the other 21 %).  us, wavefront-level / LDS, 16 heads:
+# prompts of 611 and 1,437 with a window of 1,024 105 / 48, eight of 200 37 / 16; 64 tokens on 384 keys 16.3 / 18.6; 64 beside 32
+# single tokens on 1,000 keys, the 64 a prompt of their own 68 / 52, on 1,500 68 / 80; beside sixteen on 2,000 64 / 90.  Where
+# every request brings fewer than sixteen the wavefronts' rounds took a fifth less: sixteen of 5 tokens on 1,000 keys, values of
+# 128, 38 / 51, forty on 600 45 / 56; sixty-four of 10 on 10 18 / 15.
+# Single tokens on more than 2,048 keys go to a launch of their own, in slices, in one LDS launch / two: 1,200 tokens beside
+# sixteen single ones on 1,500, 2,000, 3,000 and 30,000 89 / 84, 106 / 101, 142 / 107 and 1,141 / 306, beside four on 2,000 and
+# 3,000 88 / 90 and 123 / 94.
 PREFILL_TILE = 64
-PREFILL_MIN_WORKGROUPS = 256
 PREFILL_MAX_FEW_KEYS = 2048
 
 
@@ -78,6 +77,8 @@ class DifferentialAttention(Mixer):
         self.conv = ShortConv(self.q_dim, self.k_dim, self.v_dim, self.head_dim, self.value_dim, conv_taps)
         self.w_qkv = self.b_qkv = self.w_out = None
         self.lam = 0.0
+        self.plan_key = ("attention_diff_portions", self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim, self.window,
+                         self.keep_first)
 
     def cache_need(self) -> CacheNeed:
         return CacheNeed((CacheArray("k", 2 * self.num_kv_heads, self.head_dim),
@@ -142,34 +143,45 @@ class DifferentialAttention(Mixer):
         """Which tiles the LDS-sharing kernel takes in a step that brings some request several tokens, or None if the
         wavefront-level kernel takes the step: (tiles, few), few = (rows, tiles, positions, slices, grouped) for a launch of the
         latter that serves the requests of few tokens by themselves, or None."""
-        key = ("attention_diff_portions", self.num_heads, self.num_kv_heads, self.window, self.keep_first)
+        key = self.plan_key
         if key in ctx.memo:
             return ctx.memo[key]
-        tiles, n_tiles, longest = plan_tiles(ctx, PREFILL_TILE)
-        workgroups = n_tiles * self.num_heads
-        turns = -(-workgroups // 512) * -(-longest // 32)
+        tiles, _, longest = plan_tiles(ctx, PREFILL_TILE)
+        reach = self.window + self.keep_first if self.window > 0 else longest
+        H, capped = self.num_heads, reach / 32 + 1
+        q_start = ctx.host.q_start.tolist()
+        shared = own = of_queries = few = 0  # rounds of all tiles of either kernel, the latter's tiles, requests of few tokens
+        keys = most_new = 0                  # the longest context of those, the most tokens of a request
+        for start, end, length in zip(q_start, q_start[1:], ctx.host.seq_lens.tolist()):
+            n = end - start
+            rounds = (2 * length - n) / 64  # of a tile on average
+            rounds = 1 + (rounds if rounds < capped else capped)
+            tiles16 = (n + 15) // 16
+            shared += (n + 63) // 64 * rounds
+            own += tiles16 * rounds
+            of_queries += tiles16
+            most_new = max(most_new, n)
+            if 0 < n < PREFILL_MIN_ROWS:
+                few += 1
+                keys = max(keys, length)
+        most = min(longest, reach + PREFILL_TILE) / 32
+        slices = self.key_slices(of_queries * 2 * H, longest)
+        wide = self.head_dim + self.value_dim
+        through_lds = 9.0 + max(most * (0.64 + 0.0027 * wide), 1.7e-5 * wide * shared * H)
+        own *= 2e-5 if most_new >= PREFILL_MIN_ROWS else 1.6e-5
+        wavefronts = 9.1 + max(most / slices * (1.28 + 0.003 * wide), wide * own * H) + 2e-4 * ctx.num_tokens * H * slices
         plan = None
-        if workgroups < PREFILL_MIN_WORKGROUPS or turns <= 4:
-            if turns <= 8 or (turns <= 12 and ctx.num_tokens >= 256):
-                plan = (tiles, None)
-        else:
-            q_start = ctx.host.q_start
-            n = q_start[1:] - q_start[:-1]
-            if n.min() >= PREFILL_MIN_ROWS:
-                plan = (tiles, None)
-            else:
-                few = np.flatnonzero((n > 0) & (n < PREFILL_MIN_ROWS))
-                if 4 * (n_tiles - len(few)) >= len(few):
-                    keys = int(ctx.host.seq_lens[few].max()) if len(few) else 0
-                    read = min(keys, self.window + self.keep_first) if self.window > 0 else keys
-                    plan = (tiles, None) if read <= PREFILL_MAX_FEW_KEYS else self._few_by_themselves(ctx, n, few, keys)
+        if through_lds < wavefronts:
+            plan = (tiles, None) if not few or min(keys, reach) <= PREFILL_MAX_FEW_KEYS else self._few_by_themselves(ctx, keys)
         ctx.memo[key] = plan
         return plan
 
-    def _few_by_themselves(self, ctx, n, few, keys: int):
-        """`portion_plan` with a launch of their own for the requests `few` (n: every request's new tokens, keys: the longest
-        context among `few`): their rows are put side by side, since slices are merged for all rows of a launch."""
-        n, q_start = n.astype(np.int64), ctx.host.q_start.astype(np.int64)
+    def _few_by_themselves(self, ctx, keys: int):
+        """`portion_plan` with a launch of their own for the requests of few tokens (keys: the longest context among them): their
+        rows are put side by side, since slices are merged for all rows of a launch."""
+        q_start = ctx.host.q_start.astype(np.int64)
+        n = q_start[1:] - q_start[:-1]
+        few = np.flatnonzero((n > 0) & (n < PREFILL_MIN_ROWS))
         to_dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(ctx.rt.device)
         grouped = 2 <= self.num_heads // self.num_kv_heads <= 16
         own = _tiles_of(n[few], np.cumsum(n[few]) - n[few], few, 1 if grouped else QUERY_TILE)

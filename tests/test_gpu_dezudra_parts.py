@@ -723,17 +723,20 @@ def diff_attention_reference(q, k, v, first, window, keep, lam, eps, scale):
 
 
 @pytest.mark.parametrize("heads,kv,V,window,news,lens,expect", [
-    (16, 4, 64, 0, [2] + [1] * 16, [700] * 17, "wavefronts"),          # more single tokens than portions' tiles
+    (16, 4, 64, 0, [2] + [1] * 16, [700] * 17, "wavefronts"),
     (16, 4, 128, 0, [300] + [1] * 16, [1000] + [900] * 16, "lds"),
-    (16, 4, 64, 0, [300] + [1] * 32, [400] + [700] * 32, "wavefronts"),
+    (16, 4, 128, 0, [64] + [1] * 32, [64] + [1000] * 32, "lds"),             # the portion is a prompt of its own
+    (16, 4, 128, 0, [64] + [1] * 16, [1500] + [1000] * 16, "wavefronts"),    # it reads the most keys, for a quarter of the time
     (16, 4, 128, 0, [300] + [1] * 16, [300] + [2049] + [30] * 15, "two launches"),
     (16, 4, 128, 0, [300] + [1] * 16, [300] + [2048] + [30] * 15, "lds"),
     (16, 4, 64, 1024, [300] + [1] * 16, [300] + [2500] + [30] * 15, "lds"),  # (a window: 1,024 of them are read)
     (16, 16, 64, 0, [1, 1000, 3, 15, 1], [2100, 1000, 2500, 20, 7], "two launches"),  # tiles of up to 15 queries, not grouped
     (16, 2, 64, 2100, [15, 1000, 1, 2], [2500, 1200, 2400, 40], "two launches"),
-    (8, 4, 64, 0, [20, 3, 1], [20, 100, 64], "lds"),                    # short contexts
-    (8, 4, 64, 0, [150, 1], [300, 257], "wavefronts"),
-    (8, 4, 64, 0, [256, 1], [300, 257], "lds"),
+    (8, 4, 64, 0, [20, 3, 1], [20, 100, 64], "lds"),                         # short contexts
+    (8, 4, 64, 0, [256, 1], [300, 257], "wavefronts"),                       # few heads: the chip is half empty without slices
+    (16, 4, 128, 0, [64], [2000], "wavefronts"),
+    (16, 16, 128, 0, [5] * 16, [1000] * 16, "wavefronts"),
+    (16, 16, 128, 0, [10] * 64, [10] * 64, "lds"),
 ])
 def test_differential_attention_kernels_chosen_by_the_step(heads, kv, V, window, news, lens, expect):
     """`attend` on steps of portions and single tokens: whichever kernels the step's plan names, the result is float64

@@ -18,30 +18,36 @@
 // rows) and every second sixteen of activation rows, so it reads 4 + 5 operand
 // pieces for 20 products.
 //
-// What bounds it: with few rows per expert the weights (5.8 TB/s with 64 rows of 64 experts of 2,560).  With many the
-// products would, but a workgroup's wavefronts meet at every barrier, and what is not laid under the products there
-// adds to them.  The reduction runs in stages of 64 through two LDS buffers, and a stage in halves of 32: while a half is
-// multiplied, the next half's operands are already on their way from LDS into other registers, also over the end of the
-// stage, and the next stage's writes and the loads of the stages after it stand between the products.  One barrier a
-// stage, between its halves.  Both products, us, against operands read behind the barrier, each use waited for, and row
-// tiles dealt to the dies as wholes: 60 experts of 1,408, rows of 2,048 numbers: 136 rows each 166 + 98 (185 + 104); 23 rows
-// and four experts of 340 rows 143 + 77 (169 + 93); one expert of 5,632 with 2,048 rows 109 + 60 (150 + 82).  64 experts of
-// 2,560, rows of 3,584, wide: 64 rows each 403 + 241 (406 + 241); with eight experts of 512 rows 543 + 305 (579 + 328), 85
-// rows and eight of 682 587 + 348 (684 + 387).  (Weights straight into registers as operands, past LDS: sixteen rows of 64
-// bytes a load are half as fast for one compute unit as eight of 128.  One wavefront a SIMD with 512 registers: no better.)
-// LDS rows are 128 bytes with their 16-byte pieces permuted, so that operand reads and writes fall on distinct banks.
+// What bounds it: with few rows per expert the weights, with many the products; in between each waits for the other
+// in turn.  The reduction runs in stages of 64 through a ring of LDS buffers that the loads fill by themselves
+// (`global_load_lds`, 16 bytes a lane; which piece a lane asks for makes the permutation below): no register holds a
+// piece on its way and no wavefront writes LDS.  (With the pieces through registers, products and operand reads alone
+// ran at 1,580 TFLOP/s, with the writes 1,170, with the loads 950.)  A stage goes in halves of 32: while a half is
+// multiplied, the next half's operands are read from LDS into other registers, also over the end of the stage.  One
+// barrier a stage, between its halves: behind it stage s + 1 has landed for everybody and everybody is done with the
+// buffers of stage s, which take the loads of the stages after those that are on their way (`Ring`).
+//   The rings: what LDS holds, the weights, which come from memory, at least as deep as the activations, which come from
+// L2.  (Four against three stages for tiles of up to 64 rows: no difference; two: 484 against 412 us at 64 experts of 2,560,
+// rows of 3,584, 64 rows each on average.)
+//   Both products, us, against the pieces through registers: 60 experts of 1,408, rows of 2,048, beside four of every row,
+// 340 rows: narrow 128 + 76 (135 + 80), wide 123 + 77 (130 + 83); 2,048 rows unevenly over the 60: wide 166 + 88 (182 + 100);
+// 64 experts of 2,560, rows of 3,584, wide, beside eight of every row: 512 rows 524 + 291 (570 + 316), 682 rows 581 + 326 (607
+// + 351).  Eight experts of 1,920 rows: 1,080 TFLOP/s (970); the library's dense products 1,080.
+//   Built and left out: four wavefronts with 512 registers each and 128 weight rows (a third fewer operand reads; nobody to
+// multiply while one waits: 256 against 238 us for eight experts of 512 rows).
+// LDS rows are 128 bytes with their 16-byte pieces permuted, so that operand reads fall on distinct banks.
 //
-// An expert of up to 64 rows has one tile, and its weights are read once: past the caches (non-temporal, whole lines).  With
-// more rows that gains nothing (64 experts of 2,560 with 64 rows on average: 404 us up to 64 rows, 423 up to 96).  Results go through LDS,
-// so that a store is 16 bytes a lane of whole lines and not 8 of sixteen rows.  Both products, us, against every load through
-// the caches and results straight from the registers: 60 experts of 1,408, rows of 2,048, beside four of every row: 64 rows
-// in all 116 + 60 (130 + 68), 340 rows 119 + 67 (134 + 73); 2,048 rows unevenly over the 60 163 + 86 (181 + 98); 64 experts of 2,560, rows of
-// 3,584, wide, beside eight of every row: 682 rows 678 + 359 (687 + 372).
+// An expert with one tile has its weights read once: past the caches (non-temporal, whole lines; a plain read of memory gives
+// 7.0 TB/s that way and 6.1 through them).  2,048 rows unevenly over 60 experts 254 against 268 us for both products.  Weights
+// that several tiles read stay cached (2,048 rows 289 us past the caches).  Results go through LDS, so that a store is 16
+// bytes a lane of whole lines and not 8 of sixteen rows.
 //
-// Where experts have more rows than a tile (2,048 rows over 60 experts, 137 on average: a third of them), each of an
-// expert's row tiles asked for all its weights again, a column block's 20 us after the other tile's: 1.0 GB past L2 for
-// 0.69 GB of weights at 6.1 TB/s.  Now they go together (see the kernel): steps of 8 layers and 1,024 / 1,300 / 2,048
-// tokens 3,979 / 4,497 / 5,253 -> 3,883 / 4,416 / 5,150 us.
+// Where experts have more rows than a tile, each of an expert's row tiles would ask for all its weights again, a column
+// block's 20 us after the other tile's: they go together (see the kernel).
+//
+// Operands that do not lie on 16-byte boundaries (`DIRECT` false) go through registers, one piece after the other.
+#include <type_traits>
+
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -55,47 +61,86 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // threads per workgroup.  With four, a row tile's activations are read for half as many column blocks.
 #define TL_THREADS(NWW) (128 * (NWW))
 #define TL_STRIDE 64  // elements per LDS row: no padding; the eight 16-byte pieces of a row are stored permuted
-#define TL_XTILE(NWW) (TL_ROWS(NWW) * TL_STRIDE)  // (staged in steps of 16 NWW rows)
-#define TL_WTILE(NWW) (64 * (NWW) * TL_STRIDE)
+#define TL_LDS(NWW) ((NWW) == 4 ? 163840 : 81920)  // bytes: all of a compute unit's, or half
 // piece p of row r lies at piece p ^ ((r >> 1) & 7): the sixteen rows that a quarter of a wavefront reads at one
 // piece index then fall on sixteen different groups of four banks, as do the pieces that sixteen lanes write
 __device__ __forceinline__ int tl_at(int row, int piece) { return row * TL_STRIDE + ((piece ^ ((row >> 1) & 7)) << 3); }
 
+// 16 bytes a lane from base + offset into the workgroup's LDS, lane l's at lds + dst + 16 l (dst and base the same for all
+// lanes).  Straight into LDS the load ends when its data lies there: `wait_loads` and a barrier before others read it.  It is
+// written in assembly because the compiler would wait for every such load before every read of LDS; it has no result in
+// registers that could be taken for there before it is.
+template <bool NT, bool DIRECT>
+__device__ __forceinline__ void to_lds(__bf16* lds, unsigned dst, unsigned offset, const void* base) {
+  if constexpr (!DIRECT) {
+    typedef __bf16 anywhere __attribute__((ext_vector_type(8), aligned(2)));
+    const anywhere v = *reinterpret_cast<const anywhere*>(static_cast<const char*>(base) + offset);
+    *reinterpret_cast<bf16x8*>(reinterpret_cast<char*>(lds) + dst + 16 * (threadIdx.x & 63)) = v;
+  } else {
+    const unsigned at = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) __bf16*)lds)) + dst;
+    if constexpr (NT)
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(at), "v"(offset), "s"(base) : "memory", "m0");
+    else
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(offset), "s"(base) : "memory", "m0");
+  }
+}
+// Until at most N of this wavefront's loads are on their way (they end in the order in which they were issued).
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  static_assert(N < 64, "what the counter holds");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// A barrier that leaves loads on their way alone; what this wavefront has read from LDS or written there is done.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// How many stages' weights (W) and activations (X) LDS holds.
+template <int NP, int NWW> struct Ring {
+  static constexpr int XROWS = NWW == 4 ? 64 * ((NP + 1) / 2) : 32 * NP;  // rows staged: whole loads for every wavefront
+  static constexpr int W = NWW == 4 ? (NP <= 2 ? 4 : 3) : (NP == 1 ? 4 : NP <= 4 ? 3 : 2);
+  static constexpr int X = NWW == 4 ? (NP <= 2 ? 4 : NP <= 4 ? 3 : 2) : (NP == 1 ? 4 : NP == 2 ? 3 : 2);
+  static_assert((W * 64 * NWW + X * XROWS) * 2 * TL_STRIDE <= TL_LDS(NWW), "the rings fit");
+  static_assert(W == X || W == X + 1, "the waits below count on it");
+};
+
 // One row tile x 64 NWW weight rows.  NP: pairs of sixteens of activation rows the tile holds, one of each a wavefront.
-template <bool GATE_UP, int NP, int NWW, bool ONCE>
+template <bool GATE_UP, int NP, int NWW, bool ONCE, bool DIRECT>
 __device__ __forceinline__ void
 tiled_body(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restrict__ rows, int n_out, int width,
-           int e, int row0, int row_end, int col_block, __bf16* ws, __bf16* xs, int act, float glu_limit) {
-  // (a and w are plain pointers on purpose: loads through `const __restrict__` ones may be moved by the
-  // optimiser, which sinks them to their first use and so undoes the prefetch)
+           int e, int row0, int row_end, int col_block, __bf16* lds, int act, float glu_limit) {
+  using R = Ring<NP, NWW>;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15, g = lane >> 4;
   const int wi = wave % NWW, xi = wave / NWW;
-  constexpr int STEP = 16 * NWW;                        // rows that the workgroup's threads stage at once
-  constexpr int NPX = (32 * NP + STEP - 1) / STEP, NPW = 4;  // pieces per thread and stage
-  constexpr int NS = (NWW == 2 ? NP <= 3 : NP <= 4) ? 4 : 2;  // register sets: so many stages are on their way
-  constexpr int WROWS = 64 * NWW, HALF = WROWS / 2;
-  constexpr int COLS = GATE_UP ? HALF : WROWS;          // output columns of this workgroup
+  constexpr int WAVES = 2 * NWW, WROWS = 64 * NWW, HALF = WROWS / 2;
+  constexpr int NPW = WROWS / 8 / WAVES, NPX = R::XROWS / 8 / WAVES;  // loads of a wavefront a stage, eight rows each
+  constexpr int COLS = GATE_UP ? HALF : WROWS;                        // output columns of this workgroup
+  constexpr unsigned WT = WROWS * 2 * TL_STRIDE, XT = R::XROWS * 2 * TL_STRIDE;  // bytes of a stage
   const int n0 = col_block * COLS;
 
   const int64_t w_rows = GATE_UP ? 2 * static_cast<int64_t>(n_out) : n_out;
-  // (32-bit offsets: the entry point has checked that one expert's weights and the activations stay below 2^31)
+  // (32-bit offsets: the entry point has checked that one expert's weights and the activations stay below 2^32 bytes)
   const __bf16* w_expert = w + static_cast<int64_t>(e) * w_rows * width;
-  unsigned wsrc[NPW], xsrc[NPX];  // where the rows of this thread's pieces start
+  unsigned wsrc[NPW], xsrc[NPX];  // where this lane's rows start, in bytes: a wavefront brings rows 8 (wave + WAVES i) to + 7
 #pragma unroll
   for (int i = 0; i < NPW; ++i) {
-    const int r = (tid >> 3) + STEP * i;
+    const int r = 8 * (wave + WAVES * i) + (lane >> 3);
     const int src_row = GATE_UP ? (r < HALF ? 0 : n_out) + min(n0 + (r % HALF), n_out - 1) : min(n0 + r, n_out - 1);
-    wsrc[i] = static_cast<unsigned>(src_row) * static_cast<unsigned>(width);
+    wsrc[i] = 2u * static_cast<unsigned>(src_row) * static_cast<unsigned>(width);
   }
 #pragma unroll
   for (int i = 0; i < NPX; ++i) {
-    const int gr = min(row0 + (tid >> 3) + STEP * i, row_end - 1);  // rows past the end repeat the last one; their results are dropped
-    xsrc[i] = static_cast<unsigned>(rows ? rows[gr] : gr) * static_cast<unsigned>(width);
+    const int gr = min(row0 + 8 * (wave + WAVES * i) + (lane >> 3), row_end - 1);  // rows past the end repeat the last one; their results are dropped
+    xsrc[i] = 2u * static_cast<unsigned>(rows ? rows[gr] : gr) * static_cast<unsigned>(width);
   }
-  const int dst = tl_at(tid >> 3, tid & 7);  // rows STEP further on have the same permutation
+  // The lane's place in its row is piece lane & 7; what belongs there by `tl_at` (the number of a wavefront's eights of rows
+  // is as odd or even as the wavefront's own):
+  static_assert(WAVES % 2 == 0, "as odd or even");
+  const int piece = 8 * ((lane & 7) ^ (4 * (wave & 1) + (lane >> 4)));
 
-  bf16x8 wreg[NS][NPW], xreg[NS][NPX];
   // Experts walk the reduction in the same order but start at different stages (and wrap round): were all
   // workgroups at the same offset of their weight rows at the same time, a row length that is a power of two
   // would send their loads to the same few memory channels (measured with few rows per expert: 4.0 instead of
@@ -110,23 +155,12 @@ tiled_body(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restr
     return k0 + rot < kspan ? k0 + rot : k0 + rot - kspan;
   };
   // (a piece that does not exist, where the width is no multiple of 64, is the row's last one; zeros take its place)
-  auto fetch = [&](int s, int set) {
-    const unsigned at = min(place(s) + 8 * (tid & 7), width - 8);
-#pragma unroll
-    for (int i = 0; i < NPW; ++i) {
-      const bf16x8* from = reinterpret_cast<const bf16x8*>(w_expert + (wsrc[i] + at));
-      wreg[set][i] = ONCE ? __builtin_nontemporal_load(from) : *from;
-    }
-#pragma unroll
-    for (int i = 0; i < NPX; ++i) xreg[set][i] = *reinterpret_cast<const bf16x8*>(a + (xsrc[i] + at));
+  auto at = [&](int s) { return 2u * static_cast<unsigned>(min(place(s) + piece, width - 8)); };
+  auto load_w = [&](unsigned buf, int i, unsigned from) {
+    to_lds<ONCE, DIRECT>(lds, buf + 1024 * (wave + WAVES * i), wsrc[i] + from, w_expert);
   };
-  auto stage = [&](int buf, int set) {
-#pragma unroll
-    for (int i = 0; i < NPW; ++i)
-      *reinterpret_cast<bf16x8*>(ws + buf * TL_WTILE(NWW) + dst + STEP * i * TL_STRIDE) = wreg[set][i];
-#pragma unroll
-    for (int i = 0; i < NPX; ++i)
-      *reinterpret_cast<bf16x8*>(xs + buf * TL_XTILE(NWW) + dst + STEP * i * TL_STRIDE) = xreg[set][i];
+  auto load_x = [&](unsigned buf, int i, unsigned from) {
+    to_lds<false, DIRECT>(lds, R::W * WT + buf + 1024 * (wave + WAVES * i), xsrc[i] + from, a);
   };
 
   f32x4 acc[4][NP];
@@ -139,126 +173,106 @@ tiled_body(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restr
   int xat[2];
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) xat[kk] = tl_at(m, 4 * kk + g);
-  const int wrow = (GATE_UP ? 32 : 64) * wi * TL_STRIDE, xrow = 16 * xi * TL_STRIDE;
+  const __bf16* const ws = lds + (GATE_UP ? 32 : 64) * wi * TL_STRIDE;
+  const __bf16* const xs = lds + R::W * WT / 2 + 16 * xi * TL_STRIDE;
   struct Half { bf16x8 w[4], x[NP]; };
   Half h0, h1;
-  auto read_w = [&](Half& h, int buf, int kk) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {  // gate|up: blocks 32 wi + {0, 16} and their up rows; down: 64 wi + 16 j
-      const int block = GATE_UP ? 16 * (j & 1) + HALF * (j >> 1) : 16 * j;
-      h.w[j] = *reinterpret_cast<const bf16x8*>(ws + buf * TL_WTILE(NWW) + wrow + xat[kk] + block * TL_STRIDE);
+  auto read = [&](Half& h, int i, unsigned wbuf, unsigned xbuf, int kk) {  // the i-th of a half's NP + 4 pieces
+    if (i < 4) {  // gate|up: blocks 32 wi + {0, 16} and their up rows; down: 64 wi + 16 j
+      const int block = GATE_UP ? 16 * (i & 1) + HALF * (i >> 1) : 16 * i;
+      h.w[i] = *reinterpret_cast<const bf16x8*>(ws + wbuf / 2 + xat[kk] + block * TL_STRIDE);
+    } else if (i < NP + 4) {
+      h.x[i - 4] = *reinterpret_cast<const bf16x8*>(xs + xbuf / 2 + xat[kk] + 32 * (i - 4) * TL_STRIDE);
     }
   };
-  auto read_x = [&](Half& h, int buf, int kk) {
+  auto products = [&](const Half& h, int t) {
 #pragma unroll
-    for (int t = 0; t < NP; ++t) h.x[t] = *reinterpret_cast<const bf16x8*>(xs + buf * TL_XTILE(NWW) + xrow + xat[kk] + 32 * t * TL_STRIDE);
-  };
-  auto products = [&](const Half& h) {
-#pragma unroll
-    for (int t = 0; t < NP; ++t)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h.w[j], h.x[t], acc[j][t], 0, 0, 0);
+    for (int j = 0; j < 4; ++j) acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h.w[j], h.x[t], acc[j][t], 0, 0, 0);
   };
 
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    fetch(s, s);
-    __builtin_amdgcn_sched_barrier(0);
+  for (int s = 0; s < R::W; ++s) {
+    const unsigned from = at(s);
+    if (s < R::X)
+#pragma unroll
+      for (int i = 0; i < NPX; ++i) load_x(s * XT, i, from);
+#pragma unroll
+    for (int i = 0; i < NPW; ++i) load_w(s * WT, i, from);
   }
-  stage(0, 0);
-  __builtin_amdgcn_sched_barrier(0);
-  fetch(NS, 0);
-  __builtin_amdgcn_sched_barrier(0);
-  __syncthreads();
-  read_w(h0, 0, 0);
-  read_x(h0, 0, 0);
-  // Stage s is in LDS buffer s & 1, and the operands of its first half are in registers.  While those are multiplied,
-  // the second half's are read, stage s + 1 goes from its registers into the other buffer (whose last readers passed the
-  // previous barrier) and the registers it leaves take the loads of stage s + 1 + NS.  A barrier; while the second half
-  // is multiplied, the first operands of stage s + 1 are read.
-#define TL_STAGE(S, B, SET)                                                       \
-  {                                                                               \
-    stage(1 - (B), ((SET) + 1) % NS);                                             \
-    fetch((S) + 1 + NS, ((SET) + 1) % NS);                                        \
-    read_w(h1, B, 1);                                                             \
-    read_x(h1, B, 1);                                                             \
-    products(h0);                                                                 \
-    TL_ORDER_A                                                                    \
-    __builtin_amdgcn_sched_barrier(0);                                            \
-    __syncthreads();                                                              \
-    read_w(h0, 1 - (B), 0);                                                       \
-    read_x(h0, 1 - (B), 0);                                                       \
-    products(h1);                                                                 \
-    TL_ORDER_B                                                                    \
-    __builtin_amdgcn_sched_barrier(0);                                            \
-  }
-  // what goes between the products: first half NP + 4 reads, NPW + NPX writes and loads; second half NP + 4 reads
-#define TL_ORDER_A                                                                \
-  _Pragma("unroll") for (int t = 0; t < NP; ++t) {                                \
-    __builtin_amdgcn_sched_group_barrier(0x100, (2 * NP + 3) / NP, 0);      \
-    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);                       \
-    __builtin_amdgcn_sched_group_barrier(0x200, (NPW + NPX + NP - 1) / NP, 0);    \
-    __builtin_amdgcn_sched_group_barrier(0x020, (NPW + NPX + NP - 1) / NP, 0);    \
-    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);                       \
-  }
-#define TL_ORDER_B                                                                \
-  _Pragma("unroll") for (int t = 0; t < NP; ++t) {                                \
-    __builtin_amdgcn_sched_group_barrier(0x100, (2 * NP + 3) / NP, 0);      \
-    __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);                           \
-  }
-  // Whole turns only, and no way out of a turn's middle: a way out would join the states of the loads of all
-  // stages, and the loop's first wait would have to be for the worst of them.  A stage that is not whole is left to
-  // the end, too.
-  const bool ragged = (width & (TL_K - 1)) != 0;
-  const int turns = (stages - (ragged ? 1 : 0)) / NS;
-  int s = 0;
-  for (int i = 0; i < turns; ++i, s += NS) {
-    TL_STAGE(s, 0, 0)
-    TL_STAGE(s + 1, 1, 1)
-    if constexpr (NS == 4) {
-      TL_STAGE(s + 2, 0, 2)
-      TL_STAGE(s + 3, 1, 3)
+  wait_loads<NPW * (R::W - 1) + NPX * (R::X - 1)>();
+  lds_barrier();
+  unsigned wbuf = 0, xbuf = 0;  // where the present stage lies in the rings
+#pragma unroll
+  for (int i = 0; i < NP + 4; ++i) read(h0, i, wbuf, xbuf, 0);
+
+  // Stage s, the operands of its first half in registers; LEFT: at least so many stages follow.  Reads and loads go between
+  // the products, as many a step as leave the last ones time to arrive.
+  constexpr int READS = NP > 1 ? (NP + 4 + NP - 2) / (NP - 1) : 5, LOADS = (NPW + NPX + NP - 1) / NP;
+  auto stage = [&](auto left, int s) {
+    constexpr int LEFT = decltype(left)::value;
+#pragma unroll
+    for (int t = 0; t < NP; ++t) {
+      if constexpr (LEFT > 0) products(h0, t);
+#pragma unroll
+      for (int i = READS * t; i < READS * (t + 1); ++i) read(h1, i, wbuf, xbuf, 1);
+      __builtin_amdgcn_sched_barrier(0);
     }
-  }
-#undef TL_STAGE
-#undef TL_ORDER_A
-#undef TL_ORDER_B
-  const bf16x8 zero = {(__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f,
-                       (__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f};
-  auto last = [&](int at, int i) {  // one of the last stages (at most NS: their operands are all on their way)
-    stage(1 - (i & 1), (i + 1) % NS);
-    read_w(h1, i & 1, 1);
-    read_x(h1, i & 1, 1);
-    if (ragged && at == stages - 1) {
+    if constexpr (LEFT == 0) {
+      if (width & (TL_K - 1)) {  // the last stage is not whole
+        const bf16x8 zero = {(__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f,
+                             (__bf16)0.f, (__bf16)0.f, (__bf16)0.f, (__bf16)0.f};
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
-        if (place(at) + 32 * kk + 8 * g >= width) {
-          Half& h = kk ? h1 : h0;
+        for (int kk = 0; kk < 2; ++kk)
+          if (place(s) + 32 * kk + 8 * g >= width) {
+            Half& h = kk ? h1 : h0;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) h.w[j] = zero;
+            for (int j = 0; j < 4; ++j) h.w[j] = zero;
 #pragma unroll
-          for (int t = 0; t < NP; ++t) h.x[t] = zero;
+            for (int t = 0; t < NP; ++t) h.x[t] = zero;
+          }
+      }
+#pragma unroll
+      for (int t = 0; t < NP; ++t) products(h0, t);
+#pragma unroll
+      for (int t = 0; t < NP; ++t) products(h1, t);
+    } else {
+      // Stage s + 1 must have landed.  After its last load there were issued (an iteration issues activations first) the
+      // weights of stages up to s + W - 1 and the activations of stages up to s + X - 1, as far as there are so many.
+      constexpr int LATER_W = R::W - 2 < LEFT - 1 ? R::W - 2 : LEFT - 1, LATER_X = R::X - 2 < LEFT - 1 ? R::X - 2 : LEFT - 1;
+      wait_loads<NPW * LATER_W + NPX * LATER_X>();
+      lds_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      const unsigned wfree = wbuf, xfree = xbuf;  // nobody reads stage s any more
+      wbuf = wbuf + WT == R::W * WT ? 0 : wbuf + WT;
+      xbuf = xbuf + XT == R::X * XT ? 0 : xbuf + XT;
+      const unsigned from_x = LEFT >= R::X ? at(s + R::X) : 0u, from_w = LEFT >= R::W ? at(s + R::W) : 0u;
+#pragma unroll
+      for (int t = 0; t < NP; ++t) {
+        products(h1, t);
+#pragma unroll
+        for (int i = READS * t; i < READS * (t + 1); ++i) read(h0, i, wbuf, xbuf, 0);
+#pragma unroll
+        for (int i = LOADS * t; i < LOADS * (t + 1); ++i) {
+          if (i < NPX) {
+            if constexpr (LEFT >= R::X) load_x(xfree, i, from_x);
+          } else if (i < NPX + NPW) {
+            if constexpr (LEFT >= R::W) load_w(wfree, i - NPX, from_w);
+          }
         }
-    }
-    products(h0);
-    __syncthreads();
-    read_w(h0, 1 - (i & 1), 0);
-    read_x(h0, 1 - (i & 1), 0);
-    products(h1);
-  };
-  const int rest = stages - s;
-  if (rest > 0) {
-    last(s, 0);
-    if (rest > 1) {
-      last(s + 1, 1);
-      if constexpr (NS == 4) {
-        if (rest > 2) {
-          last(s + 2, 2);
-          if (rest > 3) last(s + 3, 3);
-        }
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-  }
+  };
+#define TL_STAGE(LEFT, S) stage(std::integral_constant<int, (LEFT)>{}, (S))
+  for (int s = 0; s < stages - R::W; ++s) TL_STAGE(R::W, s);
+  if constexpr (R::W > 3)
+    if (stages > 3) TL_STAGE(3, stages - 4);
+  if constexpr (R::W > 2)
+    if (stages > 2) TL_STAGE(2, stages - 3);
+  if (stages > 1) TL_STAGE(1, stages - 2);
+  TL_STAGE(0, stages - 1);
+#undef TL_STAGE
+  wait_loads<0>();  // (with fewer stages than the rings hold, the last one again)
 
   // lane holds weight rows (block) + 4 g + i of activation row row0 + 16 (2 t + xi) + m
   auto result = [&](int t, int j, float (&v)[4]) {
@@ -272,8 +286,8 @@ tiled_body(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restr
   if (((n_out & 7) | static_cast<int>(reinterpret_cast<uintptr_t>(out) & 15)) == 0) {
     // The tile goes through LDS, so that a store is 16 bytes a lane and whole lines.
     constexpr int OUT_STRIDE = COLS + 8;
-    static_assert(TL_ROWS(NWW) * OUT_STRIDE <= 2 * (TL_XTILE(NWW) + TL_WTILE(NWW)), "the result's tile fits the stages' LDS");
-    __bf16* const tile = ws;
+    static_assert(TL_ROWS(NWW) * OUT_STRIDE * 2 <= TL_LDS(NWW), "the result's tile fits the stages' LDS");
+    __bf16* const tile = lds;
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < NP; ++t)
@@ -316,25 +330,25 @@ tiled_body(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restr
   }
 }
 
-template <bool GATE_UP, int NWW>
+template <bool GATE_UP, int NWW, bool DIRECT>
 __global__ void __launch_bounds__(TL_THREADS(NWW)) __attribute__((amdgpu_waves_per_eu(2, 2)))
 moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restrict__ offsets,
                          const int32_t* __restrict__ rows,
                          const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_row0,
                          const int32_t* __restrict__ tile_info, int n_out, int width, int n_col_blocks,
                          int act, float glu_limit, int last_tiles, int last_each) {
-  __shared__ __attribute__((aligned(16))) __bf16 ws[2 * (TL_WTILE(NWW) + TL_XTILE(NWW))];
-  __bf16* const xs = ws + 2 * TL_WTILE(NWW);
+  __shared__ __attribute__((aligned(1024))) __bf16 lds[TL_LDS(NWW) / 2];
   // Workgroups go to the chip's eight dies in turn, by their number, and each die has its own L2 and its own share of the
   // memory's bandwidth.  The (row tile, column block) pairs, tile by tile, are cut into eight equal runs, one a die, so that
   // the column blocks of a tile, which read the same activations, share an L2 and no die has more of them than another.
   // The last `last_tiles` row tiles are those of experts that every token uses (the shared expert's pieces): full tiles,
   // bound by the matrix cores, where the others hold few rows and wait for their weights.  They are cut by themselves, and
   // a die works them spread evenly among its others, so that at any time some workgroups multiply while the rest keep
-  // the memory busy: in runs of as many as a tile has column blocks, and `last_each` tiles of one expert together, column
-  // block by column block, as they read the same weights.  (Whole tiles dealt to the dies in turn: some had a tile more,
-  // 163 against 103 us at one expert of 2,048 rows, wide; full ones spread one by one: 151 + 84 against 140 + 79 us at 23
-  // rows of 60 experts and 340 of four, as the others' weights and activations then leave L2 between uses.)
+  // the memory busy: `last_each` tiles of one expert together for a column block, as they read the same weights, and two
+  // column blocks a run.  Both products, us, with runs of one block, two, four and all of a tile's: 64 experts of 2,560, rows of
+  // 3,584, beside eight of every row: 512 rows 810, 827, 832, 852, 682 rows 897, 902, 909, 906; 60 of 1,408, rows of 2,048,
+  // beside four: 100 rows 180, 174, 172, 172, 340 rows 209, 208, 208, 212.  (Whole tiles dealt to the dies in turn: some
+  // had a tile more, 163 against 103 us at one expert of 2,048 rows, wide.)
   const int n_tiles = tile_info[0];
   const unsigned die = blockIdx.x & 7, i = blockIdx.x >> 3;
   const bool spread = last_tiles > 0 && last_tiles < n_tiles;
@@ -348,7 +362,7 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
   bool is_full = false;
   unsigned pair = light0 + i;
   if (n_full > 0) {
-    const unsigned run = n_col_blocks, runs = (n_full + run - 1) / run, period = max(n_mine / runs, run);
+    const unsigned run = 2u * last_each, runs = (n_full + run - 1) / run, period = max(n_mine / runs, run);
     const unsigned r = i / period, off = i % period;  // run r starts at place r * period
     const unsigned len = r < runs ? min(run, n_full - r * run) : 0;
     is_full = off < len;
@@ -377,13 +391,13 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
   }
   const int held = min(TL_ROWS(NWW), row_end - row0);
   if (held <= 0) return;
-  const bool once = held == row_end - first_row && held <= 64;  // an expert's only tile, few rows
+  const bool once = DIRECT && held == row_end - first_row;  // an expert's only tile
 #define CALL(NP, ONCE) \
-  tiled_body<GATE_UP, NP, NWW, ONCE>(a, w, out, rows, n_out, width, e, row0, row_end, col_block, ws, xs, act, glu_limit)
-#define BODY(NP) CALL(NP, false)
+  tiled_body<GATE_UP, NP, NWW, ONCE, DIRECT>(a, w, out, rows, n_out, width, e, row0, row_end, col_block, lds, act, glu_limit)
+#define BODY(NP) if (once) CALL(NP, DIRECT); else CALL(NP, false)
   switch ((held + 31) >> 5) {  // pairs of sixteens of rows this tile holds
-    case 1: if (once) CALL(1, true); else BODY(1); break;
-    case 2: if (once) CALL(2, true); else BODY(2); break;
+    case 1: BODY(1); break;
+    case 2: BODY(2); break;
     case 3: BODY(3); break;
     case 4: BODY(4); break;
     case 5: BODY(5); break;
@@ -419,17 +433,26 @@ extern "C" int ix_moe_grouped_tiled(const void* a, const void* w, void* out, con
   const int64_t groups = 8 * (static_cast<int64_t>(n_col_blocks) * max_tiles / 8 + 2);  // (a die has at most this many pairs)
   IX_REQUIRE(groups < (int64_t(1) << 31), "too many workgroups for one launch");
   dim3 grid(static_cast<unsigned>(groups)), block(TL_THREADS(nww));
-#define LAUNCH(GU, NWW)                                                                                             \
-  hipLaunchKernelGGL((moe_grouped_tiled_kernel<GU, NWW>), grid, block, 0, stream, (const __bf16*)a, (const __bf16*)w, \
-                     (__bf16*)out, offsets, rows, tile_expert, tile_row0, tile_info, (int)n_out, (int)width,         \
-                     n_col_blocks, gate_up == 2 ? 1 : 0, glu_limit, std::min(last_tiles, max_tiles), last_each)
+  const bool direct = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
+#define LAUNCH(GU, NWW, DIRECT)                                                                                     \
+  hipLaunchKernelGGL((moe_grouped_tiled_kernel<GU, NWW, DIRECT>), grid, block, 0, stream, (const __bf16*)a,         \
+                     (const __bf16*)w, (__bf16*)out, offsets, rows, tile_expert, tile_row0, tile_info, (int)n_out,  \
+                     (int)width, n_col_blocks, gate_up == 2 ? 1 : 0, glu_limit, std::min(last_tiles, max_tiles), last_each)
+#define FORM(GU, NWW)                 \
+  if (direct) LAUNCH(GU, NWW, true);  \
+  else LAUNCH(GU, NWW, false)
   if (nww == 4) {
-    if (gate_up == 1) LAUNCH(true, 4);
-    else LAUNCH(false, 4);
+    if (gate_up == 1) {
+      FORM(true, 4);
+    } else {
+      FORM(false, 4);
+    }
+  } else if (gate_up == 1) {
+    FORM(true, 2);
   } else {
-    if (gate_up == 1) LAUNCH(true, 2);
-    else LAUNCH(false, 2);
+    FORM(false, 2);
   }
+#undef FORM
 #undef LAUNCH
   return ix_check_launch("ix_moe_grouped_tiled");
 }

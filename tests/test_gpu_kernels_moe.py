@@ -312,6 +312,36 @@ def test_grouped_tiled_rows_read_once_and_results_at_any_place(mi, wide):
 
 
 @pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("H", [8, 64, 72, 128, 200, 256, 320, 328, 512])
+def test_grouped_tiled_rings_of_every_depth(H, wide):
+    """One to eight stages of the reduction, the last one whole or not, through the rings of every tile height (one to six
+    pairs of sixteens of rows); operands off 16-byte boundaries, which go through registers, give the same bits."""
+    from inferx_amd import ops
+    R, mi = ops.moe_tiled_rows(wide), 136
+    counts = [n for n in (1, 33, 70, 128, 129, 161, R) if n <= R] + [R + 40]
+    topk_e = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts)).to(torch.int32)[:, None].to(DEV)
+    offsets, rows, dest, tile_map = dispatch(topk_e, len(counts), R)
+    T = sum(counts)
+    x = rnd(T, H, dtype=torch.bfloat16)
+    w = rnd(len(counts), mi, H, seed=2, dtype=torch.bfloat16, scale=H ** -0.5)
+
+    def off_by(t, n):
+        buf = torch.empty(t.numel() + n, dtype=t.dtype, device=DEV)
+        buf[n:] = t.reshape(-1)
+        return buf[n:].view(t.shape)
+
+    out = []
+    for a, b in ((x, w), (off_by(x, 1), w), (x, off_by(w, 4))):
+        out.append(torch.full((T, mi), float("nan"), dtype=torch.bfloat16, device=DEV))
+        ops.moe_grouped_tiled(a, b, out[-1], offsets, rows, tile_map, False, wide)
+    want = torch.cat([x[rows.long()][lo:hi].double() @ w[e].double().T
+                      for e, (lo, hi) in enumerate(zip(offsets.tolist(), offsets.tolist()[1:]))])
+    # one rounding of the result and float32 sums of H products
+    assert float((out[0].double() - want).abs().max()) <= 2 ** -8 * float(want.abs().max()) + 1e-5
+    assert all(torch.equal(out[0].view(torch.int16), o.view(torch.int16)) for o in out[1:])
+
+
+@pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("last", [1, 3, 7, 8, 1000])
 def test_grouped_tiled_order_of_the_last_tiles(last, wide):
     """Working the last tiles of the map spread among the others changes no bit, whatever their number."""

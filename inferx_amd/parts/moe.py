@@ -36,24 +36,28 @@ SHARED_BESIDE_TOKENS = 512
 # From this width on the LDS-staged expert products run in their wide form (256 weight rows per workgroup) and the
 # shared expert stays on the main stream (a wide workgroup fills a compute unit's LDS, the library's kernels find
 # no place beside it).  Measured, prompt portions at a width of 3,584 (64 experts of 2,560, 8 per token): 14.9 against
-# 15.5 ms for a mixed step of 1,056 tokens and 8 layers, 2.86 against 3.03 s for 193,000 tokens of long prompts; at a
-# width of 2,048 (60 experts of 1,408, 4 per token) the narrow form beside the shared expert is ahead, 5.19 against
-# 5.30 ms for 2,048 tokens and 8 layers.
+# 15.5 ms for a mixed step of 1,056 tokens and 8 layers, 2.86 against 3.03 s for 193,000 tokens of long prompts.
 WIDE_TILES_WIDTH = 3072
+# From this width on they do where no library product runs beside them: without a shared expert, or with it among the routed
+# ones (below).  Both products at a width of 2,048 (60 experts of 1,408), us, narrow / wide: unevenly routed 512 tokens 209 /
+# 191, 1,024 207 / 208, 2,048 272 / 247, 4,096 403 / 379; with the shared expert among them 64 tokens 170 / 166, 340 208 / 208, 768
+# 255 / 234, 1,500 322 / 317, 2,048 412 / 380.
+WIDE_TILES_ALONE_WIDTH = 2048
 # Between the few rows of a decoding step (where routed and shared experts already share a launch) and the portions
 # from which the shared expert's library products run beside the routed experts, the shared expert is cut into
 # pieces of the routed experts' width, which every token "chooses" with the shared gate's value as their weight:
 # grouping, the two grouped products and the weighted sum then take it along, its weights stream at the rate of the
 # big launches instead of through two library products of few rows and a launch for SwiGLU.  Needs a shared width
 # that is a multiple of the experts' width; keeps the shared expert's weights a second time, in that layout.
-# Measured at the A2.7B shape (24 layers), with against without: decoding at batch 64 11.22 against 11.59 ms a step; a
-# portion of 256 tokens 6.58 against 7.19 ms, of 512 8.16 against 9.17, of 768 9.50 against 9.47, of 1,024 10.88
-# against 10.42; at the 57B shape (8 layers) 512 tokens 9.41 against 10.26 ms, 1,024 13.41 against 13.29.  With the
-# grouped products as they are now (stages pipelined, tiles cut over the dies, an expert's tiles sharing its weights), us of
-# a whole prompt, without / with: A2.7B shape (8 layers) 300 tokens 2,672 / 2,430, 800 3,462 / 3,261, 1,024 3,883 / 3,603,
-# 1,300 4,416 / 4,198, 1,536 4,505 / 4,512, 2,048 5,150 / 5,237, 4,096 8,361 / 9,009; 57B shape (4 layers) 512 tokens 5,254 /
-# 4,564, 1,024 6,635 / 6,030, 1,500 7,931 / 7,678, 2,048 9,756 / 9,785.
+# us of a whole prompt, without / with: A2.7B shape (8 layers) 300 tokens 2,672 / 2,430, 1,024 3,883 / 3,422, 1,536 4,449 /
+# 4,177, 1,800 4,884 / 4,741, 2,048 5,092 / 4,890, 2,176 5,173 / 5,222, 2,560 5,577 / 5,657, 3,072 6,540 / 6,776; 57B shape (4
+# layers) 1,024 tokens 6,290 / 5,550, 1,500 7,522 / 7,263, 2,048 9,178 / 9,040, 2,600 11,127 / 11,257, 4,096 16,078 / 17,077.  The
+# line is eleven whole tiles of the wide form; narrower models, whose products stay in the narrow form, keep theirs (1,300 tokens
+# of the A2.7B shape in that form 4,416 / 4,198, 1,536 4,505 / 4,512).
+# Each piece's result is rounded before the sum adds them in float32: four roundings of a half the size instead of one.  Against
+# 64 bits, fourteen seeds each, without / with: 2,048 tokens 0.02727 / 0.02711, 1,700 0.02628 / 0.02613.
 FOLD_SHARED_BELOW_TOKENS = 1536
+FOLD_SHARED_BELOW_TOKENS_WIDE = 11 * ops.MOE_TILED_ROWS_WIDE + 1
 
 
 class MoeFeedForward(FeedForward):
@@ -180,7 +184,12 @@ class MoeFeedForward(FeedForward):
         per_expert = x.shape[0] * self.top_k / self.num_experts
         if x.shape[0] <= ctx.rt.SKINNY_ROWS or per_expert <= 3:
             return 16
-        return ops.MOE_TILED_F32_ROWS if x.dtype == torch.float32 else ops.moe_tiled_rows(self.wide_tiles)
+        return ops.MOE_TILED_F32_ROWS if x.dtype == torch.float32 else ops.moe_tiled_rows(self._wide(x.shape[0]))
+
+    def _wide(self, tokens: int) -> bool:
+        """Whether the LDS-staged products of this step take their wide form."""
+        alone = self.shared_width == 0 or self._shared_rides_along(tokens)
+        return self.wide_tiles or (alone and self.hidden_size >= WIDE_TILES_ALONE_WIDTH)
 
     def _f32_fits(self, x) -> bool:
         """What the float32 products on the matrix cores ask for beside whole 16-byte pieces: rows on 16-byte boundaries
@@ -210,8 +219,8 @@ class MoeFeedForward(FeedForward):
         if tile_rows == ops.MOE_TILED_F32_ROWS:  # a float32 run, more than a few rows per expert
             ops.moe_grouped_tiled_f32(x, w13, act, offsets, rows, tile_map, self.first_epilogue, self.limit)
             ops.moe_grouped_tiled_f32(act, w2, y, offsets, None, tile_map, False)
-        elif tile_rows == ops.moe_tiled_rows(self.wide_tiles):  # many rows per expert: operands staged through LDS
-            wide = self.wide_tiles
+        elif tile_rows in (ops.MOE_TILED_ROWS, ops.MOE_TILED_ROWS_WIDE):  # many rows per expert: operands staged through LDS
+            wide = tile_rows == ops.MOE_TILED_ROWS_WIDE
             # (a piece of the shared expert holds every token: its tiles are full, and the last ones of the map)
             each = -(-x.shape[0] // tile_rows)
             full = self.shared_pieces * each if with_shared else 0
@@ -275,7 +284,8 @@ class MoeFeedForward(FeedForward):
         """Whether the shared expert is among the routed ones, in pieces, in a step of so many tokens: up to the line above, and
         as far as the grouped products' 32-bit places reach."""
         rows = tokens * (self.top_k + self.shared_pieces)
-        return self.shared_pieces > 0 and tokens < FOLD_SHARED_BELOW_TOKENS and rows * self.expert_width < 1 << 31
+        line = FOLD_SHARED_BELOW_TOKENS_WIDE if self.hidden_size >= WIDE_TILES_ALONE_WIDTH else FOLD_SHARED_BELOW_TOKENS
+        return self.shared_pieces > 0 and tokens < line and rows * self.expert_width < 1 << 31
 
     takes_lazy_norm = True
 
@@ -299,7 +309,7 @@ class MoeFeedForward(FeedForward):
             y = self.experts(ctx, x, offsets, rows, tile_map, tile_rows, with_shared=True)
             return MoeSum(y, dest, topk_w, None, None, self.hidden_size)
         shared = join = None
-        if (not one_launch and self.shared_width > 0 and tile_rows == ops.MOE_TILED_ROWS and not self.wide_tiles
+        if (not one_launch and self.shared_width > 0 and tile_rows == ops.MOE_TILED_ROWS
                 and x.shape[0] >= SHARED_BESIDE_TOKENS and ctx.rt.can_run_beside()):
             # a prompt portion: the shared expert's library products are bound by the matrix cores, the routed
             # experts' kernels by memory, so the two run beside each other on two streams

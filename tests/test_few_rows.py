@@ -49,6 +49,16 @@ def test_shared_expert_rides_along_as_far_as_the_products_reach(pieces, width, t
     assert part._shared_rides_along(tokens) == along
 
 
+@pytest.mark.parametrize("hidden,shared,tokens,wide", [
+    (2048, 5632, 33, True), (2048, 5632, 2112, True), (2048, 5632, 2113, False), (2048, 0, 9000, True), (2048, 1000, 33, False),
+    (2040, 5632, 33, False), (2040, 0, 33, False), (3072, 5632, 2113, True), (3072, 1000, 33, True)])
+def test_wide_expert_products(hidden, shared, tokens, wide):
+    """From a width of 3,072 on always, from 2,048 on where the shared expert is not a product of its own."""
+    from inferx_amd.parts.moe import MoeFeedForward
+    part = MoeFeedForward(hidden, 4, 1, 1408, shared)
+    assert part._wide(tokens) == wide
+
+
 @pytest.mark.parametrize("units,longest,span,head_dim,slices,loads", [
     (16, 517, 0, 128, 16, 1), (16, 65, 0, 128, 1, 1), (4, 128, 0, 128, 1, 1), (4, 129, 0, 128, 4, 1),   # one request
     (4, 64, 0, 128, 1, 2), (32, 40, 0, 128, 1, 2), (33, 40, 0, 128, 1, 1), (2048, 64, 0, 128, 1, 2), (2048, 65, 0, 128, 1, 1),

@@ -48,7 +48,7 @@
 // Operands that do not lie on 16-byte boundaries (`DIRECT` false) go through registers, one piece after the other.
 #include <type_traits>
 
-#include "common.h"
+#include "lds_loads.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
@@ -66,35 +66,16 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // piece index then fall on sixteen different groups of four banks, as do the pieces that sixteen lanes write
 __device__ __forceinline__ int tl_at(int row, int piece) { return row * TL_STRIDE + ((piece ^ ((row >> 1) & 7)) << 3); }
 
-// 16 bytes a lane from base + offset into the workgroup's LDS, lane l's at lds + dst + 16 l (dst and base the same for all
-// lanes).  Straight into LDS the load ends when its data lies there: `wait_loads` and a barrier before others read it.  It is
-// written in assembly because the compiler would wait for every such load before every read of LDS; it has no result in
-// registers that could be taken for there before it is.
+// 16 bytes a lane from base + offset to lds + dst + 16 lane, straight or, from anywhere, through registers.
 template <bool NT, bool DIRECT>
 __device__ __forceinline__ void to_lds(__bf16* lds, unsigned dst, unsigned offset, const void* base) {
-  if constexpr (!DIRECT) {
+  if constexpr (DIRECT) {
+    lds_load16<NT>(lds, dst, offset, base);
+  } else {
     typedef __bf16 anywhere __attribute__((ext_vector_type(8), aligned(2)));
     const anywhere v = *reinterpret_cast<const anywhere*>(static_cast<const char*>(base) + offset);
     *reinterpret_cast<bf16x8*>(reinterpret_cast<char*>(lds) + dst + 16 * (threadIdx.x & 63)) = v;
-  } else {
-    const unsigned at = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) __bf16*)lds)) + dst;
-    if constexpr (NT)
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(at), "v"(offset), "s"(base) : "memory", "m0");
-    else
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(offset), "s"(base) : "memory", "m0");
   }
-}
-// Until at most N of this wavefront's loads are on their way (they end in the order in which they were issued).
-template <int N>
-__device__ __forceinline__ void wait_loads() {
-  static_assert(N < 64, "what the counter holds");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-// A barrier that leaves loads on their way alone; what this wavefront has read from LDS or written there is done.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
 }
 
 // How many stages' weights (W) and activations (X) LDS holds.

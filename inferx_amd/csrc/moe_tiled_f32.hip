@@ -3,12 +3,13 @@
 //
 // What bounds it: at a few dozen rows per expert the weights' way from memory, from about fifty on the matrix cores
 // (32 cycles for 16 x 16 x 4).  A workgroup owns up to 64 rows of one expert (a tile of the grouping kernel's map: with
-// a few hundred tokens all rows of an expert, so that its weights are read once) x 64 weight rows, which for gate|up are
-// 32 gate rows and their 32 up rows; its four wavefronts take sixteen weight rows each (for gate|up eight and eight)
-// and all of the tile's rows.  Stages of 32 of the reduction (128 bytes a row) go through two LDS buffers, three more
-// are on their way in registers, one barrier a stage; 32 KB of LDS and 128 registers leave four workgroups to a compute
-// unit, whose loads and products overlap.  Rows of LDS keep their eight 16-byte pieces permuted (piece p of row r at
-// p ^ ((r >> 1) & 7)), so that sixteen rows read at one piece fall on different banks.
+// a few hundred tokens all rows of an expert, so that its weights are read once) x 128 weight rows, which for gate|up are
+// 64 gate rows and their 64 up rows; its four wavefronts take 32 weight rows each (for gate|up sixteen and sixteen)
+// and all of the tile's rows.  Stages of 32 of the reduction (128 bytes a row) go through a ring of three or four LDS
+// buffers that the loads fill by themselves, with one barrier a stage, as in moe_tiled.hip; half a compute unit's LDS, so
+// that two workgroups share one and one's products overlap with the other's waits.  Rows of LDS keep their eight 16-byte
+// pieces permuted (piece p of row r at p ^ ((r >> 1) & 7)), so that sixteen rows read at one piece fall on different banks.
+// The weights of an expert with one tile are read once: past the caches.
 //
 // A lane reads four consecutive numbers of its row at a time; product j of a piece multiplies the j-th of them, so the
 // four slots of the reduction that one matrix instruction adds up are the pieces' j-th numbers, the same in both
@@ -16,181 +17,235 @@
 // power of two bytes would otherwise all ask the same memory channels at once.  The order of a result's sum so depends
 // on its column alone.
 //
-// Measured at 511 tokens of 60 experts of 1,408 on a width of 2,048, 4 a token (34 rows an expert, 2.1 GB of weights):
-// 387 + 195 us for the two products, against 805 + 563 us of the plain kernel (a workgroup of 64 x 64 on the vector
-// units, LDS filled a number at a time).  The weights alone take 325 us at the rate of a pure read, the products 230.
-// With the tiles cut evenly over the dies, routing to weighted sum: 361 tokens 502 -> 458 us, 511 591 -> 561, 800 797 -> 731.
-#include "common.h"
+// Measured with 60 experts of 1,408 on a width of 2,048, 4 a token, unevenly routed, both products, us, against pieces through
+// registers and LDS writes, 64 weight rows, a die's run of tiles in their order: 170 tokens 389 -> 330, 361 504 -> 390, 511 558
+// -> 463, 800 730 -> 597; 32 rows each 422 -> 382, 64 rows each 676 -> 605 (the weights alone take 324, the last one's products
+// 474).  Of it at 511 tokens the direct loads and 128 rows 50 to 65, the order of the tiles 45 to 60.
+#include <type_traits>
+
+#include "lds_loads.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-#define TF_ROWS 64                 // rows of a tile of the map
-#define TF_WROWS 64                // weight rows per workgroup
-#define TF_K 32                    // numbers of the reduction per stage
-#define TF_TILE (TF_ROWS * TF_K)   // numbers of one LDS buffer
+#define TF_ROWS 64     // rows of a tile of the map
+#define TF_WROWS 128   // weight rows per workgroup
+#define TF_K 32        // numbers of the reduction per stage
+#define TF_LDS 81920   // bytes: half a compute unit's
 __device__ __forceinline__ int tf_at(int row, int piece) { return row * TF_K + ((piece ^ ((row >> 1) & 7)) << 2); }
 
-// NT: sixteens of rows that the tile holds.  Every load is unconditional and the loop one straight line (see
-// moe_tiled.hip): a stage past the end asks for the last stage again, a piece past the row's end for the row's start,
-// with zeros written over it in LDS.
-template <bool GATE_UP, int NT>
+// NT: sixteens of rows that the tile holds.  Every load is unconditional: a stage past the end asks for the last stage
+// again, a piece past the row's end for the row's last one, with zeros in its place among the operands.
+template <bool GATE_UP, int NT, bool ONCE>
 __device__ __forceinline__ void tiled_f32_body(const float* a, const float* w, float* out,
                                                const int32_t* __restrict__ rows, int n_out, int width, int e, int row0,
-                                               int row_end, int col_block, float* ws, float* xs, int act,
-                                               float glu_limit) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+                                               int row_end, int col_block, float* lds, int act, float glu_limit) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15, g = lane >> 4;
   constexpr int COLS = GATE_UP ? TF_WROWS / 2 : TF_WROWS;
-  constexpr int NPX = (NT + 1) / 2;  // pieces of activations per thread and stage (32 rows at a time)
+  constexpr int NPW = TF_WROWS / 32, NPX = (NT + 1) / 2;  // loads of a wavefront a stage, eight rows each
+  constexpr int RING = NT <= 2 ? 4 : 3;                   // stages that LDS holds
+  constexpr unsigned WT = TF_WROWS * 4 * TF_K, XT = 32 * NPX * 4 * TF_K;  // bytes of a stage
+  static_assert(RING * (WT + XT) <= TF_LDS, "the rings fit");
   const int n0 = col_block * COLS;
 
   const int64_t w_rows = GATE_UP ? 2 * static_cast<int64_t>(n_out) : n_out;
   const float* w_expert = w + static_cast<int64_t>(e) * w_rows * width;
-  const int kc_mine = (tid & 7) * 4;
-  int wsrc[2], xsrc[NPX];
+  int64_t wsrc[NPW], xsrc[NPX];  // where this lane's rows start, in numbers
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int r = (tid >> 3) + 32 * i;  // LDS row; wavefront r / 16 multiplies it
-    const int src = GATE_UP ? ((r & 8) ? n_out : 0) + min(n0 + 8 * (r >> 4) + (r & 7), n_out - 1) : min(n0 + r, n_out - 1);
-    wsrc[i] = src * width;
+  for (int i = 0; i < NPW; ++i) {
+    const int r = 8 * (wave + 4 * i) + (lane >> 3);  // LDS row; wavefront r / 32 multiplies it, for gate|up sixteen gate rows, then their up rows
+    const int src = GATE_UP ? ((r & 16) ? n_out : 0) + min(n0 + 16 * (r >> 5) + (r & 15), n_out - 1) : min(n0 + r, n_out - 1);
+    wsrc[i] = static_cast<int64_t>(src) * width;
   }
 #pragma unroll
   for (int i = 0; i < NPX; ++i) {
-    const int gr = min(row0 + (tid >> 3) + 32 * i, row_end - 1);  // rows past the end repeat the last one
-    xsrc[i] = (rows ? rows[gr] : gr) * width;
+    const int gr = min(row0 + 8 * (wave + 4 * i) + (lane >> 3), row_end - 1);  // rows past the end repeat the last one
+    xsrc[i] = static_cast<int64_t>(rows ? rows[gr] : gr) * width;
   }
-  const int dst = tf_at(tid >> 3, tid & 7);  // (32 rows further on: the same permutation)
+  const int piece = 4 * ((lane & 7) ^ (4 * (wave & 1) + (lane >> 4)));  // what belongs at piece lane & 7 of the lane's rows
 
   const int stages = (width + TF_K - 1) / TF_K, kspan = stages * TF_K;
-  const int rot = (width & 255) == 0 ? static_cast<int>((static_cast<unsigned>(col_block) * 3u) % stages) * TF_K : 0;
-  const bool ragged = (width & (TF_K - 1)) != 0;
-  auto place = [&](int k0, bool& ok) {
-    k0 = min(k0, kspan - TF_K);
-    const int k = (k0 + rot < kspan ? k0 + rot : k0 + rot - kspan) + kc_mine;
-    ok = k < width;
-    return ok ? k : 0;
+  const int rot = (width & 255) == 0 ? static_cast<int>((static_cast<unsigned>(col_block) * 6u) % stages) * TF_K : 0;
+  auto place = [&](int s) {  // where stage s starts in a row
+    const int k0 = min(s * TF_K, kspan - TF_K);
+    return k0 + rot < kspan ? k0 + rot : k0 + rot - kspan;
   };
-  f32x4 wreg[3][2], xreg[3][NPX];
-  auto fetch = [&](int k0, f32x4 (&wr)[2], f32x4 (&xr)[NPX]) {
-    bool ok;
-    const int k = place(k0, ok);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) wr[i] = *reinterpret_cast<const f32x4*>(w_expert + wsrc[i] + k);
-#pragma unroll
-    for (int i = 0; i < NPX; ++i) xr[i] = *reinterpret_cast<const f32x4*>(a + xsrc[i] + k);
-    __builtin_amdgcn_sched_barrier(0);
+  auto load = [&](int buf, int i, int at) {  // the i-th of a stage's loads
+    if (i < NPX) lds_load16<false>(lds, RING * WT + buf * XT + 1024 * (wave + 4 * i), a + xsrc[i] + at);
+    else if (i < NPX + NPW) lds_load16<ONCE>(lds, buf * WT + 1024 * (wave + 4 * (i - NPX)), w_expert + wsrc[i - NPX] + at);
   };
-  auto stage = [&](int k0, int buf, const f32x4 (&wr)[2], const f32x4 (&xr)[NPX]) {
+  auto at_stage = [&](int s) { return min(place(s) + piece, width - 4); };
+
+  f32x4 acc[2][NT];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) *reinterpret_cast<f32x4*>(ws + buf * TF_TILE + dst + 32 * TF_K * i) = wr[i];
+  for (int b = 0; b < 2; ++b)
 #pragma unroll
-    for (int i = 0; i < NPX; ++i) *reinterpret_cast<f32x4*>(xs + buf * TF_TILE + dst + 32 * TF_K * i) = xr[i];
-    if (ragged) {
-      bool ok;
-      place(k0, ok);
-      if (!ok) {
+    for (int t = 0; t < NT; ++t) acc[b][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int at16[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) at16[h] = tf_at(m, 4 * h + g);
+  const float* const ws = lds + 32 * wave * TF_K;
+  const float* const xs = lds + RING * WT / 4;
+  struct Half { f32x4 w[2], x[NT]; };
+  Half h0, h1;
+  auto read = [&](Half& h, int i, int buf, int half) {  // the i-th of a half's NT + 2 pieces
+    if (i < 2) h.w[i] = *reinterpret_cast<const f32x4*>(ws + buf * (WT / 4) + at16[half] + 16 * i * TF_K);
+    else if (i < NT + 2) h.x[i - 2] = *reinterpret_cast<const f32x4*>(xs + buf * (XT / 4) + at16[half] + 16 * (i - 2) * TF_K);
+  };
+  auto products = [&](const Half& h, int j) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(h.w[b][j], h.x[t][j], acc[b][t], 0, 0, 0);
+  };
+#pragma unroll
+  for (int s = 0; s < RING; ++s)
+#pragma unroll
+    for (int i = 0; i < NPX + NPW; ++i) load(s, i, at_stage(s));
+  wait_loads<(NPX + NPW) * (RING - 1)>();
+  lds_barrier();
+  int buf = 0;
+#pragma unroll
+  for (int i = 0; i < NT + 2; ++i) read(h0, i, buf, 0);
+  constexpr int READS = (NT + 2 + 1) / 2, LOADS = (NPX + NPW + 2) / 3;
+  auto stage = [&](auto left, int s) {
+    constexpr int LEFT = decltype(left)::value;  // at least so many stages follow
+    if constexpr (LEFT == 0) {
+#pragma unroll
+      for (int i = 0; i < NT + 2; ++i) read(h1, i, buf, 1);
+      if (width & (TF_K - 1)) {  // the last stage is not whole
         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 2; ++i) *reinterpret_cast<f32x4*>(ws + buf * TF_TILE + dst + 32 * TF_K * i) = zero;
+        for (int half = 0; half < 2; ++half)
+          if (place(s) + 16 * half + 4 * g >= width) {
+            Half& h = half ? h1 : h0;
 #pragma unroll
-        for (int i = 0; i < NPX; ++i) *reinterpret_cast<f32x4*>(xs + buf * TF_TILE + dst + 32 * TF_K * i) = zero;
+            for (int b = 0; b < 2; ++b) h.w[b] = zero;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) h.x[t] = zero;
+          }
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) products(h0, j);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) products(h1, j);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        products(h0, j);
+#pragma unroll
+        for (int i = READS * j; i < READS * (j + 1); ++i) read(h1, i, buf, 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      wait_loads<(NPX + NPW) * (RING - 2 < LEFT - 1 ? RING - 2 : LEFT - 1)>();  // stage s + 1 has landed
+      lds_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      const int free = buf;  // nobody reads stage s any more
+      buf = buf + 1 == RING ? 0 : buf + 1;
+      const int at = LEFT >= RING ? at_stage(s + RING) : 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        products(h1, j);
+#pragma unroll
+        for (int i = READS * j; i < READS * (j + 1); ++i) read(h0, i, buf, 0);
+        if constexpr (LEFT >= RING)
+#pragma unroll
+          for (int i = LOADS * j; i < LOADS * (j + 1); ++i) load(free, i, at);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
-  f32x4 acc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  int wat[2], xat[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    wat[h] = tf_at(16 * wave + m, 4 * h + g);
-    xat[h] = tf_at(m, 4 * h + g);
-  }
-  auto multiply = [&](int buf) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const f32x4 wa = *reinterpret_cast<const f32x4*>(ws + buf * TF_TILE + wat[h]);
-      f32x4 xb[NT];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) xb[t] = *reinterpret_cast<const f32x4*>(xs + buf * TF_TILE + xat[h] + 16 * TF_K * t);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wa[j], xb[t][j], acc[t], 0, 0, 0);
-    }
-  };
-
-  fetch(0, wreg[0], xreg[0]);
-  fetch(TF_K, wreg[1], xreg[1]);
-  fetch(2 * TF_K, wreg[2], xreg[2]);
-  stage(0, 0, wreg[0], xreg[0]);
-  fetch(3 * TF_K, wreg[0], xreg[0]);
-  __syncthreads();
-  // stage s lies in LDS buffer s & 1; register set (s + 1) % 3 holds the next one and then takes stage s + 4
-#define TF_STAGE(K0, BUF, SET)                                    \
-  {                                                               \
-    stage((K0) + TF_K, 1 - (BUF), wreg[SET], xreg[SET]);          \
-    fetch((K0) + 4 * TF_K, wreg[SET], xreg[SET]);                 \
-    if ((K0) < kspan) multiply(BUF);                              \
-    __builtin_amdgcn_sched_barrier(0);                            \
-    __syncthreads();                                              \
-  }
-  for (int k0 = 0; k0 < kspan; k0 += 6 * TF_K) {  // whole turns only, as in moe_tiled.hip
-    TF_STAGE(k0, 0, 1)
-    TF_STAGE(k0 + TF_K, 1, 2)
-    TF_STAGE(k0 + 2 * TF_K, 0, 0)
-    TF_STAGE(k0 + 3 * TF_K, 1, 1)
-    TF_STAGE(k0 + 4 * TF_K, 0, 2)
-    TF_STAGE(k0 + 5 * TF_K, 1, 0)
-  }
+#define TF_STAGE(LEFT, S) stage(std::integral_constant<int, (LEFT)>{}, (S))
+  for (int s = 0; s < stages - RING; ++s) TF_STAGE(RING, s);
+  if constexpr (RING > 3)
+    if (stages > 3) TF_STAGE(3, stages - 4);
+  if (stages > 2) TF_STAGE(2, stages - 3);
+  if (stages > 1) TF_STAGE(1, stages - 2);
+  TF_STAGE(0, stages - 1);
 #undef TF_STAGE
+  wait_loads<0>();  // (with fewer stages than the ring holds, the last one again)
 
-  // lane holds the wavefront's weight rows 4 g + i of tile row 16 t + m; for gate|up lanes of g 0, 1 the gate's sums,
-  // those of g 2, 3 (32 lanes on) the same columns' up sums
+  // lane holds weight rows (sixteen) + 4 g + i of tile row 16 t + m
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int r = row0 + 16 * t + m;
-    float v[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[i] = acc[t][i];
-      if constexpr (GATE_UP) v[i] = ix_glu(v[i], __shfl_xor(v[i], 32, 64), glu_limit);
-      else if (act) v[i] = v[i] > 0.f ? v[i] * v[i] : 0.f;  // the square of relu
-    }
-    if (r >= row_end || (GATE_UP && g >= 2)) continue;
-    const int nb = n0 + (GATE_UP ? 8 : 16) * wave + 4 * g;
-    float* o = out + static_cast<int64_t>(r) * n_out + nb;
-    if (nb + 4 <= n_out && (n_out & 3) == 0) {
-      *reinterpret_cast<f32x4*>(o) = f32x4{v[0], v[1], v[2], v[3]};
-    } else {
+    for (int b = 0; b < (GATE_UP ? 1 : 2); ++b) {
+      float v[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (nb + i < n_out) o[i] = v[i];
+      for (int i = 0; i < 4; ++i) {
+        v[i] = acc[b][t][i];
+        if constexpr (GATE_UP) v[i] = ix_glu(v[i], acc[1][t][i], glu_limit);
+        else if (act) v[i] = v[i] > 0.f ? v[i] * v[i] : 0.f;  // the square of relu
+      }
+      if (r >= row_end) continue;
+      const int nb = n0 + (GATE_UP ? 16 : 32) * wave + 16 * b + 4 * g;
+      float* o = out + static_cast<int64_t>(r) * n_out + nb;
+      if (nb + 4 <= n_out && (n_out & 3) == 0) {
+        *reinterpret_cast<f32x4*>(o) = f32x4{v[0], v[1], v[2], v[3]};
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (nb + i < n_out) o[i] = v[i];
+      }
     }
   }
 }
 
 template <bool GATE_UP>
-__global__ void __launch_bounds__(256, 4)
+__global__ void __launch_bounds__(256, 2)
 moe_grouped_tiled_f32_kernel(const float* a, const float* w, float* out, const int32_t* __restrict__ offsets,
                              const int32_t* __restrict__ rows, const int32_t* __restrict__ tile_expert,
                              const int32_t* __restrict__ tile_row0, const int32_t* __restrict__ tile_info, int n_out,
                              int width, int n_col_blocks, int act, float glu_limit) {
-  __shared__ __attribute__((aligned(16))) float ws[2 * TF_TILE];
-  __shared__ __attribute__((aligned(16))) float xs[2 * TF_TILE];
-  // Workgroups go to the chip's eight dies in turn.  The (row tile, column block) pairs, tile by tile, are cut into eight
-  // equal runs, one a die: the column blocks of a tile, which read the same activations, share an L2, and no die has more
-  // of them than another (whole tiles dealt to the dies in turn: of 60, four dies had eight and four seven).
-  const unsigned n_pairs = static_cast<unsigned>(tile_info[0]) * n_col_blocks, die = blockIdx.x & 7;
-  auto cut = [&](unsigned d) { return static_cast<unsigned>(static_cast<uint64_t>(n_pairs) * d >> 3); };
-  const unsigned pair = cut(die) + (blockIdx.x >> 3);
-  if (pair >= cut(die + 1)) return;
-  const int tile = static_cast<int>(pair / n_col_blocks), col_block = static_cast<int>(pair % n_col_blocks);
+  __shared__ __attribute__((aligned(1024))) float lds[TF_LDS / 4];
+  // The tiles with most rows come first, so that what is left at the end is short, and a tile's column blocks go to the
+  // chip's eight dies in turn, so that each has as much of it (a die's run of whole tiles took 133 to 178 us at 511 tokens).  Tiles of as
+  // many sixteens stay together in the map's order; beyond 512 of them the end no longer matters.  (Long and short tiles in
+  // turn leave half the chip idle at times: workgroups are handed out in order, each to a place of its own.)
+  const int n_tiles = tile_info[0];
+  const unsigned pair = blockIdx.x;
+  if (pair >= static_cast<unsigned>(n_tiles) * n_col_blocks) return;
+  int tile = static_cast<int>(pair / n_col_blocks);
+  const int col_block = static_cast<int>(pair % n_col_blocks);
+  if (n_tiles <= 8 * 64) {
+    const int lane = threadIdx.x & 63;
+    unsigned sixteens = 0;  // of the tile 64 c + lane, in four bits for each c
+    int count[5] = {0, 0, 0, 0, 0};
+    for (int c = 0; 64 * c < n_tiles; ++c) {
+      const int t = 64 * c + lane;
+      int n = 0;
+      if (t < n_tiles) n = max(1, (min(TF_ROWS, offsets[tile_expert[t] + 1] - tile_row0[t]) + 15) >> 4);
+      sixteens |= static_cast<unsigned>(n) << (4 * c);
+#pragma unroll
+      for (int k = 1; k <= 4; ++k) count[k] += __popcll(__ballot(n == k));
+    }
+    int place = tile, kind = 4;  // the place among the tiles of so many sixteens
+#pragma unroll
+    for (int k = 4; k > 1; --k)
+      if (kind == k && place >= count[k]) {
+        place -= count[k];
+        kind = k - 1;
+      }
+    for (int c = 0; 64 * c < n_tiles; ++c) {
+      unsigned long long of_kind = __ballot(static_cast<int>(sixteens >> (4 * c) & 15) == kind);
+      const int n = __popcll(of_kind);
+      if (place < n) {
+        for (; place > 0; --place) of_kind &= of_kind - 1;
+        tile = 64 * c + __ffsll(of_kind) - 1;
+        break;
+      }
+      place -= n;
+    }
+    tile = __builtin_amdgcn_readfirstlane(tile);
+  }
   const int e = tile_expert[tile], row0 = tile_row0[tile], row_end = offsets[e + 1];
   const int held = min(TF_ROWS, row_end - row0);
   if (held <= 0) return;
-#define BODY(NT) \
-  tiled_f32_body<GATE_UP, NT>(a, w, out, rows, n_out, width, e, row0, row_end, col_block, ws, xs, act, glu_limit)
+  const bool once = held == row_end - offsets[e];  // an expert's only tile: its weights are read once, past the caches
+#define CALL(NT, ONCE) \
+  tiled_f32_body<GATE_UP, NT, ONCE>(a, w, out, rows, n_out, width, e, row0, row_end, col_block, lds, act, glu_limit)
+#define BODY(NT) if (once) CALL(NT, true); else CALL(NT, false)
   switch ((held + 15) >> 4) {
     case 1: BODY(1); break;
     case 2: BODY(2); break;
@@ -198,6 +253,7 @@ moe_grouped_tiled_f32_kernel(const float* a, const float* w, float* out, const i
     default: BODY(4); break;
   }
 #undef BODY
+#undef CALL
 }
 
 // Shapes as ix_moe_grouped_plain, all float32; the row-tile map must have been made for tiles of 64 rows; operands on
@@ -219,7 +275,7 @@ extern "C" int ix_moe_grouped_tiled_f32(const float* a, const float* w, float* o
   if (max_tiles == 0) return 0;
   const int cols = gate_up == 1 ? TF_WROWS / 2 : TF_WROWS;
   const int n_col_blocks = static_cast<int>((n_out + cols - 1) / cols);
-  const int64_t groups = 8 * (static_cast<int64_t>(n_col_blocks) * max_tiles / 8 + 2);  // (a die has at most this many pairs)
+  const int64_t groups = static_cast<int64_t>(n_col_blocks) * max_tiles;
   IX_REQUIRE(groups < (int64_t(1) << 31), "too many workgroups for one launch");
   dim3 grid(static_cast<unsigned>(groups)), block(256);
   if (gate_up == 1)

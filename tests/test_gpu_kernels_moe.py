@@ -690,6 +690,24 @@ def test_grouped_products_in_float32(counts, K, n, kind, gate_up, limit):
         assert torch.isfinite(shared).all() and rel_err(shared, want(xd @ wd[0].T)) < 1e-5
 
 
+@pytest.mark.parametrize("counts", [[5, 64, 17, 1, 0, 40, 33, 130, 16, 48, 49, 32], [1] * 40 + [70] * 30 + [20] * 30, [2] * 511 + [65]])
+@pytest.mark.parametrize("K", [32, 64, 68, 96, 128, 160, 256])
+def test_grouped_tiled_in_float32_worked_by_their_rows(counts, K):
+    """Tiles of all heights in any order of the map, up to 64, some more and over 512 of them: each is formed, whichever the
+    order in which they are worked; one to eight stages of the reduction through the rings."""
+    from inferx_amd import ops
+    E, A, T, n = len(counts), sum(counts), 70, 132
+    topk_e = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).to(torch.int32)[:, None].to(DEV)
+    offsets, _, _, tile_map = dispatch(topk_e, E, ops.MOE_TILED_F32_ROWS)
+    rows = torch.randint(0, T, (A,), generator=torch.Generator().manual_seed(2)).to(torch.int32).to(DEV)
+    x, w = rnd(T, K, scale=K ** -0.25), rnd(E, n, K, seed=1, scale=K ** -0.25)
+    out = torch.full((A, n), float("nan"), device=DEV)
+    ops.moe_grouped_tiled_f32(x, w, out, offsets, rows, tile_map, False)
+    want = torch.cat([x[rows.long()][lo:hi].double() @ w[e].double().T
+                      for e, (lo, hi) in enumerate(zip(offsets.tolist(), offsets.tolist()[1:]))])
+    assert rel_err(out, want) < 1e-5  # (every product and sum is 32-bit)
+
+
 @pytest.mark.parametrize("T,N,K", [(1, 301, 36), (16, 33, 2048), (17, 384, 100), (32, 70, 4), (64, 1000, 260)])
 def test_linear_skinny_in_float32(T, N, K):
     from inferx_amd import ops

@@ -109,10 +109,29 @@ class Runtime:
         ops.linear_skinny(x, w, out, gate_up, limit, bias)
         return out
 
+    # From 17 rows on a product of so many features goes in tiles.  17 / 32 rows of 2,048 and more, us, few-row kernel / tiles: 6,144
+    # features 12.8 / 10.4 and 16.0 / 11.4, 11,264 17.2 / 14.0 and 21.7 / 14.4, 151,936 in float32 113 / 106 and 152 / 117; 2,048 8.8 / 9.6
+    # and 10.4 / 10.0, 3,584 12.8 / 13.0 and 15.0 / 13.9.
+    TILED_FEATURES = 4096
+
+    def _tiled(self, x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype) -> Optional[torch.Tensor]:
+        """The product in tiles of the few-hundred-row kernel, where it takes it."""
+        rows, features = x.shape[0], w.shape[0]
+        if not (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()
+                and (rows > self.SKINNY_ROWS or (rows > 16 and features >= self.TILED_FEATURES)) and features > 0
+                and x.shape[1] > 0 and x.shape[1] % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0):
+            return None
+        from .. import ops
+        out = self.empty((rows, features), out_dtype)
+        return out if ops.linear_tiled(x, w, out) else None
+
     def linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """x [T, in] . w[out, in]^T -> [T, out] in the run's type, float32 accumulation.
         A weight kept in float32 during a bfloat16 run is multiplied in float32."""
         if w.dtype == x.dtype:
+            out = self._tiled(x, w, x.dtype)
+            if out is not None:
+                return out
             if self._skinny_ok(x, w):
                 return self._skinny(x, w, False)
             if x.dtype == torch.bfloat16 and x.shape[0] > 0 and x.is_contiguous() and w.is_contiguous():
@@ -142,6 +161,9 @@ class Runtime:
 
     def linear_f32(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """As `linear`, result float32 (the logits)."""
+        out = self._tiled(x, w, torch.float32)
+        if out is not None:
+            return out
         if self._skinny_ok(x, w):  # few rows: the vocabulary's weights are the traffic
             from .. import ops
             out = self.empty((x.shape[0], w.shape[0]), torch.float32)

@@ -725,6 +725,24 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
     return True
 
 
+def linear_tiled(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, tile: int = -1) -> bool:
+    """out [T, N] = x [T, K] . w[N, K]^T, bfloat16 operands on 16-byte boundaries, 32-bit accumulation, out bfloat16 or float32,
+    for a few dozen to some hundred rows.  False where the kernel's rule has no tile for the product (nothing was queued then);
+    `tile` from 0 to 8 names one."""
+    T, K = x.shape
+    N = w.shape[0]
+    _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and out.dtype in (torch.bfloat16, torch.float32),
+          "bfloat16 operands and a bfloat16 or float32 result")
+    _need(w.dim() == 2 and w.shape[1] == K and out.shape == (T, N), "shapes do not fit")
+    fn = _functions.get("ix_linear_tiled")
+    if fn is None:
+        fn = _functions["ix_linear_tiled"] = lib().ix_linear_tiled
+    rc = fn(_ptr(x), _ptr(w), _ptr(out), T, N, K, 1 if out.dtype == torch.float32 else 0, tile, _stream())
+    if rc not in (0, 2):
+        raise KernelError(lib().ix_last_error().decode("utf-8", "replace"))
+    return rc == 0
+
+
 def linear_skinny(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate_up: bool = False, glu_limit: float = 0.0,
                   bias: Optional[torch.Tensor] = None) -> None:
     """out [T, N] = x [T, K] . w[N, K]^T for at most 64 rows, all three bfloat16 or all float32.  `gate_up`: w is [2 N, K],

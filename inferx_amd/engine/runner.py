@@ -21,6 +21,7 @@ from typing import Dict, Hashable, List, Optional, Sequence, Tuple
 import numpy as np
 import torch
 
+from .. import ops
 from ..cache.manager import CacheManager, GroupLayout, pages_for_window
 from ..config import config_from_directory
 from ..parts import build_model
@@ -189,7 +190,7 @@ class ModelRunner:
         starts = np.zeros(batch.num_requests, dtype=bool)
         starts[brings] = batch.positions[first[brings]] == 0
         if starts.any():
-            slots = torch.from_numpy(batch.state_slots[starts].astype(np.int64)).to(self.rt.device)
+            slots = ops.upload(batch.state_slots[starts].astype(np.int64), self.rt.device)
             for state in self._states:
                 state.index_fill_(0, slots, 0)
 
@@ -208,7 +209,7 @@ class ModelRunner:
 
     def _upload(self, batch: StepBatch) -> StepContext:
         sizes, flat = _pack(batch)
-        return self._context(torch.from_numpy(flat).to(self.rt.device), sizes, batch)
+        return self._context(ops.upload(flat, self.rt.device), sizes, batch)
 
     # ---- graphs for one-token-per-request steps ---------------------------------
     def _shared_logits(self, rows: int) -> torch.Tensor:

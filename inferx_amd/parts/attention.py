@@ -179,8 +179,8 @@ class PagedAttention(Mixer):
         the slices of the keys follow from `longest`."""
         key = ("attention_tiles_host", QUERY_TILE)
         if key not in ctx.memo:
-            tiles = torch.tensor([list(range(requests)), list(range(requests)), [1] * requests], dtype=torch.int32,
-                                 device=ctx.rt.device)
+            every = np.arange(requests, dtype=np.int32)
+            tiles = ops.upload(np.stack([every, every, np.ones_like(every)]), ctx.rt.device)
             ctx.memo[key] = (tiles, requests, longest)
 
     def forward(self, ctx, x, cache):
@@ -345,7 +345,7 @@ def plan_tiles(ctx, tile: int):
         b = ctx.host
         n = (b.q_start[1:] - b.q_start[:-1]).astype(np.int64)
         tiles_host = _tiles_of(n, b.q_start[:-1].astype(np.int64), np.arange(len(n)), tile)
-        tiles_dev = torch.from_numpy(np.ascontiguousarray(tiles_host)).to(ctx.rt.device)
+        tiles_dev = ops.upload(tiles_host, ctx.rt.device)
         longest = int(b.seq_lens.max()) if len(b.seq_lens) else 0
         base = ctx.memo[("attention_tiles_host", tile)] = (tiles_dev, tiles_host.shape[1], longest)
     return base
@@ -420,10 +420,10 @@ def mixed_step_plan(ctx, span: int, heads: int, kv_heads: int, lds_fits: bool = 
     if key in ctx.memo:
         return ctx.memo[key]
     b = ctx.host
-    dev = ctx.rt.device
     q_start = b.q_start[:-1].astype(np.int64)
     n = (b.q_start[1:] - b.q_start[:-1]).astype(np.int64)
-    to_dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    dev = ctx.rt.device
+    to_dev = lambda a: ops.upload(a, dev)
     long = n >= PREFILL_MIN_ROWS
     seqs = np.flatnonzero(long)
     t = _tiles_of(n[seqs], q_start[seqs], seqs, tile) if (lds_fits and len(seqs)) else None

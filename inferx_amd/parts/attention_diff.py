@@ -128,8 +128,8 @@ class DifferentialAttention(Mixer):
         the slices of the keys follow from `longest`.  (The same plan, under the same key, as plain attention's.)"""
         key = ("attention_tiles_host", QUERY_TILE)
         if key not in ctx.memo:
-            tiles = torch.tensor([list(range(requests)), list(range(requests)), [1] * requests], dtype=torch.int32,
-                                 device=ctx.rt.device)
+            every = np.arange(requests, dtype=np.int32)
+            tiles = ops.upload(np.stack([every, every, np.ones_like(every)]), ctx.rt.device)
             ctx.memo[key] = (tiles, requests, longest)
 
     def key_slices(self, units: int, longest: int) -> int:
@@ -182,7 +182,7 @@ class DifferentialAttention(Mixer):
         q_start = ctx.host.q_start.astype(np.int64)
         n = q_start[1:] - q_start[:-1]
         few = np.flatnonzero((n > 0) & (n < PREFILL_MIN_ROWS))
-        to_dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(ctx.rt.device)
+        to_dev = lambda a: ops.upload(a, ctx.rt.device)
         grouped = 2 <= self.num_heads // self.num_kv_heads <= 16
         own = _tiles_of(n[few], np.cumsum(n[few]) - n[few], few, 1 if grouped else QUERY_TILE)
         rows = to_dev(np.concatenate([np.arange(q_start[i], q_start[i + 1]) for i in few]))

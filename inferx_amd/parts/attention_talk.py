@@ -19,6 +19,7 @@ from __future__ import annotations
 
 from typing import List, Optional
 
+import numpy as np
 import torch
 
 from .. import ops
@@ -141,8 +142,8 @@ class TalkingAttention(Mixer):
         (the plan that `plan_tiles` would make from the host's arrays)."""
         key = ("attention_tiles_host", QUERY_TILE)
         if key not in ctx.memo:
-            tiles = torch.tensor([list(range(requests)), list(range(requests)), [1] * requests], dtype=torch.int32,
-                                 device=ctx.rt.device)
+            every = np.arange(requests, dtype=np.int32)
+            tiles = ops.upload(np.stack([every, every, np.ones_like(every)]), ctx.rt.device)
             ctx.memo[key] = (tiles, requests, longest)
 
     def attend(self, ctx, q, cache, gate, out) -> None:

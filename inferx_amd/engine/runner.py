@@ -291,6 +291,7 @@ class _DecodeGraph:
         # values to the same places; per-request state, though, would be advanced twice, so it is put back.
         kept = [state.clone() for state in runner._states]
         self.logits = runner._shared_logits(S)  # (allocated before the capture, outside the graphs' pool)
+        ctx.logits_place = self.logits
         # Warm-up and capture run on one stream that all of the runner's graphs share: what a library keeps per
         # stream (the dense products' workspace) is there before the capture, and once for all graphs.
         if runner._capture_stream is None:
@@ -313,11 +314,13 @@ class _DecodeGraph:
             else:
                 self.graph.capture_begin(pool=runner._graph_pool)
             try:
-                # The step's logits end in a buffer that all of the runner's graphs share, as the last node of the
-                # graph: what the capture allocated is then free for the next capture (the graphs share a memory
-                # pool), and a graph holds nothing of the size of requests x vocabulary for itself.
+                # The step's logits end in a buffer that all of the runner's graphs share: what the capture allocated is
+                # then free for the next capture (the graphs share a memory pool), and a graph holds nothing of the size of
+                # requests x vocabulary for itself.  The head writes them there (a copy as the graph's last node took 4 us
+                # at one request and 11 at 64), unless its product does not take the place.
                 logits = runner.model.forward(ctx, runner.bindings)
-                self.logits.copy_(logits)
+                if logits.data_ptr() != self.logits.data_ptr():
+                    self.logits.copy_(logits)
                 del logits
             finally:
                 self.graph.capture_end()

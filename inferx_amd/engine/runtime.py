@@ -114,7 +114,8 @@ class Runtime:
     # and 10.4 / 10.0, 3,584 12.8 / 13.0 and 15.0 / 13.9.
     TILED_FEATURES = 4096
 
-    def _tiled(self, x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype) -> Optional[torch.Tensor]:
+    def _tiled(self, x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype,
+               out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
         """The product in tiles of the few-hundred-row kernel, where it takes it."""
         rows, features = x.shape[0], w.shape[0]
         if not (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()
@@ -122,7 +123,8 @@ class Runtime:
                 and x.shape[1] > 0 and x.shape[1] % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0):
             return None
         from .. import ops
-        out = self.empty((rows, features), out_dtype)
+        if out is None:
+            out = self.empty((rows, features), out_dtype)
         return out if ops.linear_tiled(x, w, out) else None
 
     def linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -159,14 +161,15 @@ class Runtime:
             ops.glu_bias(gate_up, bias, act, limit)
         return act
 
-    def linear_f32(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-        """As `linear`, result float32 (the logits)."""
-        out = self._tiled(x, w, torch.float32)
+    def linear_f32(self, x: torch.Tensor, w: torch.Tensor, place: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """As `linear`, result float32 (the logits).  `place`: a float32 tensor of the result's shape that the kernels here write
+        it to; what another product forms is returned where that left it."""
+        out = self._tiled(x, w, torch.float32, place)
         if out is not None:
             return out
         if self._skinny_ok(x, w):  # few rows: the vocabulary's weights are the traffic
             from .. import ops
-            out = self.empty((x.shape[0], w.shape[0]), torch.float32)
+            out = self.empty((x.shape[0], w.shape[0]), torch.float32) if place is None else place
             ops.linear_skinny_f32(x, w, out)
             return out
         if x.dtype == torch.float32 and w.dtype == torch.float32:
@@ -227,3 +230,4 @@ class StepContext:
     host: Any = None                       # the StepBatch (host arrays), for parts that plan on the host
     one_token_each: bool = False           # every request brings exactly one token (a decoding step)
     memo: Dict[Any, Any] = field(default_factory=dict)  # per-step results shared between layers
+    logits_place: Optional[torch.Tensor] = None  # where the head may leave the step's logits (a captured step's buffer)

@@ -70,7 +70,8 @@ class LinearHead(Head):
         self.weight = tensors["weight"].contiguous()
 
     def forward(self, ctx, x):
-        logits = ctx.rt.linear_f32(x, self.weight)
+        place = getattr(ctx, "logits_place", None)
+        logits = ctx.rt.linear_f32(x, self.weight, place) if place is not None else ctx.rt.linear_f32(x, self.weight)
         return logits if self.scale == 1.0 else logits.mul_(self.scale)
 
 

@@ -13,14 +13,15 @@
 //
 // A lane reads four consecutive numbers of its row at a time; product j of a piece multiplies the j-th of them, so the
 // four slots of the reduction that one matrix instruction adds up are the pieces' j-th numbers, the same in both
-// operands.  Workgroups start the reduction at a stage that follows from their column block and wrap round: rows of a
+// operands.  Blocks of weight rows start the reduction at a stage that follows from their number and wrap round: rows of a
 // power of two bytes would otherwise all ask the same memory channels at once.  The order of a result's sum so depends
-// on its column alone.
+// on its column alone (two scores of a later router that are 1e-6 apart fall the other way with another order).
 //
 // Measured with 60 experts of 1,408 on a width of 2,048, 4 a token, unevenly routed, both products, us, against pieces through
-// registers and LDS writes, 64 weight rows, a die's run of tiles in their order: 170 tokens 389 -> 330, 361 504 -> 390, 511 558
-// -> 463, 800 730 -> 597; 32 rows each 422 -> 382, 64 rows each 676 -> 605 (the weights alone take 324, the last one's products
-// 474).  Of it at 511 tokens the direct loads and 128 rows 50 to 65, the order of the tiles 45 to 60.
+// registers and LDS writes, 64 weight rows, a die's run of tiles in their order: 170 tokens 389 -> 348, 361 503 -> 415, 511 562
+// -> 490, 800 747 -> 648; 32 rows each 428 -> 404, 64 rows each 662 -> 641 (the weights alone take 324, the last one's products
+// 474).  Of it at 511 tokens the direct loads and 128 rows 50 to 65, the order of the tiles 45 to 60; that both blocks of a
+// workgroup keep their own order of sums costs 30.
 #include <type_traits>
 
 #include "lds_loads.h"
@@ -30,6 +31,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define TF_ROWS 64     // rows of a tile of the map
 #define TF_WROWS 128   // weight rows per workgroup
 #define TF_K 32        // numbers of the reduction per stage
+#define TF_APART 3     // stages between the starts of neighbouring blocks of 64 weight rows
 #define TF_LDS 81920   // bytes: half a compute unit's
 __device__ __forceinline__ int tf_at(int row, int piece) { return row * TF_K + ((piece ^ ((row >> 1) & 7)) << 2); }
 
@@ -64,12 +66,19 @@ __device__ __forceinline__ void tiled_f32_body(const float* a, const float* w, f
   }
   const int piece = 4 * ((lane & 7) ^ (4 * (wave & 1) + (lane >> 4)));  // what belongs at piece lane & 7 of the lane's rows
 
-  const int stages = (width + TF_K - 1) / TF_K, kspan = stages * TF_K;
-  const int rot = (width & 255) == 0 ? static_cast<int>((static_cast<unsigned>(col_block) * 6u) % stages) * TF_K : 0;
-  auto place = [&](int s) {  // where stage s starts in a row
-    const int k0 = min(s * TF_K, kspan - TF_K);
-    return k0 + rot < kspan ? k0 + rot : k0 + rot - kspan;
+  // Blocks of 64 weight rows start the reduction at a stage that follows from their number and wrap round.  A workgroup
+  // owns two of them, which start TF_APART stages apart: it walks so many stages more, the first of them for the first two
+  // wavefronts only and the last of them for the others.
+  const int stages = (width + TF_K - 1) / TF_K;
+  const bool turned = (width & 255) == 0;  // (then there are eight stages at least)
+  const int total = stages + (turned ? TF_APART : 0);
+  const int begin = turned ? static_cast<int>((static_cast<unsigned>(col_block) * (2u * TF_APART)) % stages) : 0;
+  auto place = [&](int s) {  // where stage s starts in a row (past the end: the last stage again)
+    int k = min(s, total - 1) + begin;
+    k = k < stages ? k : k - stages;
+    return (k < stages ? k : k - stages) * TF_K;
   };
+  auto mine = [&](int s) { return !turned || (wave < 2 ? s < stages : s >= TF_APART); };
   auto load = [&](int buf, int i, int at) {  // the i-th of a stage's loads
     if (i < NPX) lds_load16<false>(lds, RING * WT + buf * XT + 1024 * (wave + 4 * i), a + xsrc[i] + at);
     else if (i < NPX + NPW) lds_load16<ONCE>(lds, buf * WT + 1024 * (wave + 4 * (i - NPX)), w_expert + wsrc[i - NPX] + at);
@@ -125,14 +134,17 @@ __device__ __forceinline__ void tiled_f32_body(const float* a, const float* w, f
             for (int t = 0; t < NT; ++t) h.x[t] = zero;
           }
       }
+      if (mine(s)) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) products(h0, j);
+        for (int j = 0; j < 4; ++j) products(h0, j);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) products(h1, j);
+        for (int j = 0; j < 4; ++j) products(h1, j);
+      }
     } else {
+      const bool own = mine(s);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        products(h0, j);
+        if (own) products(h0, j);
 #pragma unroll
         for (int i = READS * j; i < READS * (j + 1); ++i) read(h1, i, buf, 1);
         __builtin_amdgcn_sched_barrier(0);
@@ -145,7 +157,7 @@ __device__ __forceinline__ void tiled_f32_body(const float* a, const float* w, f
       const int at = LEFT >= RING ? at_stage(s + RING) : 0;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        products(h1, j);
+        if (own) products(h1, j);
 #pragma unroll
         for (int i = READS * j; i < READS * (j + 1); ++i) read(h0, i, buf, 0);
         if constexpr (LEFT >= RING)
@@ -156,12 +168,12 @@ __device__ __forceinline__ void tiled_f32_body(const float* a, const float* w, f
     }
   };
 #define TF_STAGE(LEFT, S) stage(std::integral_constant<int, (LEFT)>{}, (S))
-  for (int s = 0; s < stages - RING; ++s) TF_STAGE(RING, s);
+  for (int s = 0; s < total - RING; ++s) TF_STAGE(RING, s);
   if constexpr (RING > 3)
-    if (stages > 3) TF_STAGE(3, stages - 4);
-  if (stages > 2) TF_STAGE(2, stages - 3);
-  if (stages > 1) TF_STAGE(1, stages - 2);
-  TF_STAGE(0, stages - 1);
+    if (total > 3) TF_STAGE(3, total - 4);
+  if (total > 2) TF_STAGE(2, total - 3);
+  if (total > 1) TF_STAGE(1, total - 2);
+  TF_STAGE(0, total - 1);
 #undef TF_STAGE
   wait_loads<0>();  // (with fewer stages than the ring holds, the last one again)
 

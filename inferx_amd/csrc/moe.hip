@@ -366,9 +366,16 @@ moe_dispatch_wide_kernel(const int32_t* __restrict__ topk_e, int32_t* __restrict
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int i = tid; i < experts; i += DW_THREADS) counts[i] = 0;
   __syncthreads();
-  for (int64_t a = tid; a < assignments; a += DW_THREADS) {
-    const int v = topk_e[a];
-    if (v >= 0 && v < experts) atomicAdd(&counts[v], 1);
+  for (int64_t a0 = tid; a0 < assignments; a0 += DW_ROUNDS * DW_THREADS) {
+    int v[DW_ROUNDS];  // (all asked for before the first is counted: a trip to memory for eight of them)
+#pragma unroll
+    for (int r = 0; r < DW_ROUNDS; ++r) {
+      const int64_t a = a0 + r * DW_THREADS;
+      v[r] = a < assignments ? topk_e[a] : -1;
+    }
+#pragma unroll
+    for (int r = 0; r < DW_ROUNDS; ++r)
+      if (v[r] >= 0 && v[r] < experts) atomicAdd(&counts[v[r]], 1);
   }
   __syncthreads();
   int rows_before = 0, tiles_before = 0;
@@ -415,10 +422,15 @@ moe_dispatch_wide_kernel(const int32_t* __restrict__ topk_e, int32_t* __restrict
     const int64_t a0 = p0 + static_cast<int64_t>(wave) * DW_ROUNDS * 64 + lane;
     uint64_t match[DW_ROUNDS];
     int found = 0;
+    int v[DW_ROUNDS];
 #pragma unroll
     for (int r = 0; r < DW_ROUNDS; ++r) {
       const int64_t a = a0 + 64 * r;
-      match[r] = __ballot(a < assignments && topk_e[a] == e);
+      v[r] = a < assignments ? topk_e[a] : -1;
+    }
+#pragma unroll
+    for (int r = 0; r < DW_ROUNDS; ++r) {
+      match[r] = __ballot(v[r] == e);
       found += __popcll(match[r]);
     }
     if (lane == 0) wave_count[wave] = found;

@@ -1,8 +1,9 @@
 // Loads straight into LDS, and the waits that go with them (gfx950).
 //
 // Such a load ends when its data lies in LDS: `wait_loads` and then a barrier before another wavefront reads it.  They are
-// written in assembly because the compiler would wait for every such load before every read of LDS; they have no result
-// in registers that could be taken for there before it is.  Loads of a wavefront end in the order in which they were issued,
+// written in assembly, as are the waits, so that which reads of LDS wait for which of them is what the kernels say and not what
+// the compiler makes of it; they have no result in registers that could be taken for there before it is, and nothing of them
+// may be on its way when a kernel ends.  Loads of a wavefront end in the order in which they were issued,
 // the compiler's own among them (which it waits for as if these were not there, so at worst for more than it needs).
 #pragma once
 

@@ -253,7 +253,8 @@ using TileN = LinearTile<2, 2, 4, 2, 3>;   // 128 x 64, two workgroups a compute
 // The tile for a product, or -1: the one with the fewest rows of both kinds whose number fits the compute units.  From 96 x 128 on a
 // tile's stages are long enough for the library to be ahead where many of them follow (1,400 x 5,632 x 2,048 55.7 against 52.1 us)
 // or where a fifth of the units have none (850 x 3,584 x 3,584 39.8 against 38.1; 682 x 3,584 x 4,608, 216 tiles, 37.4 against 43.5;
-// up to 2,048 of reduction also with fewer: 144 tiles of 128 x 128 26.3 against 31.4).  Up to 64 rows of what does not fit go in tiles
+// up to 2,048 of reduction also with fewer: 144 tiles of 128 x 128 26.3 against 31.4), or where a product is one stage or three (3,000 x
+// 64 x 700 11.3 against 10.3; 1,500 x 512 x 2,048 11.4 against 14.6).  Up to 64 rows of what does not fit go in tiles
 // of 128 x 64 (a vocabulary's weights: 33 rows of 151,936 x 2,048 116 against 197, 64 rows 125 against 199).
 static int tile_for(int64_t rows, int64_t n_out, int64_t width) {
   const int64_t tiles[8] = {tiles_of<Tile0>(rows, n_out), tiles_of<Tile1>(rows, n_out), tiles_of<Tile2>(rows, n_out),
@@ -263,7 +264,7 @@ static int tile_for(int64_t rows, int64_t n_out, int64_t width) {
   while (tile < 8 && tiles[tile] > LT_UNITS) ++tile;
   if (tile < 5) return tile;
   if (rows <= TileN::X) return 8;
-  if (tile == 8 || width > 4096 || (tile > 5 && width > 2048 && 5 * tiles[tile] < 4 * LT_UNITS)) return -1;
+  if (tile == 8 || width > 4096 || width < 256 || (tile > 5 && width > 2048 && 5 * tiles[tile] < 4 * LT_UNITS)) return -1;
   return tile;
 }
 

@@ -40,7 +40,8 @@ def test_every_tile(tile, f32):
 
 @pytest.mark.parametrize("T,N,K,taken", [
     (33, 2048, 2048, True), (17, 6144, 2048, True), (850, 6144, 2048, True), (1400, 2048, 5632, False), (2048, 6144, 2048, False),
-    (64, 32768, 256, True), (65, 70000, 64, False), (850, 3584, 3584, False), (40, 100, 8, True)])
+    (64, 32768, 256, True), (65, 70000, 64, False), (850, 3584, 3584, False), (40, 100, 8, True),
+    (3000, 700, 64, False), (3000, 700, 256, True)])
 def test_which_products_are_taken(T, N, K, taken):
     from inferx_amd import ops
     x, w = operands(T, N, K)

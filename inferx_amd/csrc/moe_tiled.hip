@@ -311,13 +311,21 @@ tiled_body(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restr
   }
 }
 
+// A second product of the launch: out [rows, n_out] = a [rows, width] . w^T, one set of weights for all rows (with gate|up the two
+// sets of n_out rows).  rows 0: none.
+struct Second {
+  const __bf16 *a, *w;
+  __bf16* out;
+  int rows, n_out, width;
+};
+
 template <bool GATE_UP, int NWW, bool DIRECT>
 __global__ void __launch_bounds__(TL_THREADS(NWW)) __attribute__((amdgpu_waves_per_eu(2, 2)))
 moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restrict__ offsets,
                          const int32_t* __restrict__ rows,
                          const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_row0,
                          const int32_t* __restrict__ tile_info, int n_out, int width, int n_col_blocks,
-                         int act, float glu_limit, int last_tiles, int last_each) {
+                         int act, float glu_limit, int last_tiles, int last_each, Second second) {
   __shared__ __attribute__((aligned(1024))) __bf16 lds[TL_LDS(NWW) / 2];
   // Workgroups go to the chip's eight dies in turn, by their number, and each die has its own L2 and its own share of the
   // memory's bandwidth.  The (row tile, column block) pairs, tile by tile, are cut into eight equal runs, one a die, so that
@@ -332,47 +340,67 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
   // had a tile more, 163 against 103 us at one expert of 2,048 rows, wide.)
   const int n_tiles = tile_info[0];
   const unsigned die = blockIdx.x & 7, i = blockIdx.x >> 3;
-  const bool spread = last_tiles > 0 && last_tiles < n_tiles;
+  // A second product's tiles are worked as the last ones: as many row tiles of one expert.
+  const bool two = NWW == 4 && second.rows > 0, spread = !two && last_tiles > 0 && last_tiles < n_tiles;
+  constexpr int COLS = (GATE_UP ? 32 : 64) * NWW;
+  if (two) last_each = (second.rows + TL_ROWS(NWW) - 1) / TL_ROWS(NWW);
   const int n_light = spread ? n_tiles - last_tiles : n_tiles;
   const unsigned light = static_cast<unsigned>(n_light) * n_col_blocks;
-  const unsigned full = spread ? static_cast<unsigned>(last_tiles) * n_col_blocks : 0u;
+  const unsigned full = two ? static_cast<unsigned>(last_each) * ((second.n_out + COLS - 1) / COLS)
+                            : spread ? static_cast<unsigned>(last_tiles) * n_col_blocks : 0u;
   auto cut = [&](unsigned n, unsigned d) { return static_cast<unsigned>(static_cast<uint64_t>(n) * d >> 3); };
   const unsigned light0 = cut(light, die), full0 = cut(full, die);
   const unsigned n_full = cut(full, die + 1) - full0, n_mine = cut(light, die + 1) - light0 + n_full;
   if (i >= n_mine) return;
   bool is_full = false;
   unsigned pair = light0 + i;
-  if (n_full > 0) {
+  if (two && second.width > width) {
+    // longer ones first: they then end with the others (88 of 88 stages beside some 600 of 22, of 256 places)
+    is_full = i < n_full;
+    pair = is_full ? light + full0 + i : light0 + i - n_full;
+  } else if (n_full > 0) {
     const unsigned run = 2u * last_each, runs = (n_full + run - 1) / run, period = max(n_mine / runs, run);
     const unsigned r = i / period, off = i % period;  // run r starts at place r * period
     const unsigned len = r < runs ? min(run, n_full - r * run) : 0;
     is_full = off < len;
     pair = is_full ? light + full0 + r * run + off : light0 + i - (r < runs ? r * run + len : n_full);
   }
-  int tile = static_cast<int>(pair / n_col_blocks), col_block = static_cast<int>(pair % n_col_blocks);
-  if (is_full && last_each > 1) {  // (the row tiles of an expert one after the other for a column block)
-    const unsigned at = pair - light, per = static_cast<unsigned>(last_each) * n_col_blocks, in = at % per;
-    tile = n_tiles - last_tiles + static_cast<int>(at / per * last_each + in % last_each);
-    col_block = static_cast<int>(in / last_each);
-  }
-  const int e = tile_expert[tile];
-  int row0 = tile_row0[tile];
-  const int row_end = offsets[e + 1], first_row = offsets[e];
-  if (!is_full && row_end - first_row > TL_ROWS(NWW)) {
-    // Row tiles of an expert that has several read the same weights: up to four of them one after the other for a column
-    // block, so that all but the first find the weights in L2.  (Tiles of the expert that are among the last ones have
-    // been dealt out above.)
-    const int nth = (row0 - first_row) / TL_ROWS(NWW), first = tile - (nth & 3);
-    const int of_expert = (row_end - first_row + TL_ROWS(NWW) - 1) / TL_ROWS(NWW) - (nth & ~3);
-    const unsigned n_here = min(min(4, of_expert), n_light - first);
-    const unsigned in = pair - static_cast<unsigned>(first) * n_col_blocks;
-    tile = first + static_cast<int>(in % n_here);
-    col_block = static_cast<int>(in / n_here);
+  int e = 0, row0, row_end, col_block;
+  bool once = false;  // an expert's only tile
+  if (two && is_full) {
+    const int at = static_cast<int>(pair - light);
+    row0 = TL_ROWS(NWW) * (at % last_each);
+    col_block = at / last_each;
+    row_end = second.rows;
+    a = second.a, w = second.w, out = second.out, rows = nullptr, n_out = second.n_out, width = second.width, act = 0;
+  } else {
+    int tile = static_cast<int>(pair / n_col_blocks);
+    col_block = static_cast<int>(pair % n_col_blocks);
+    if (is_full && last_each > 1) {  // (the row tiles of an expert one after the other for a column block)
+      const unsigned at = pair - light, per = static_cast<unsigned>(last_each) * n_col_blocks, in = at % per;
+      tile = n_tiles - last_tiles + static_cast<int>(at / per * last_each + in % last_each);
+      col_block = static_cast<int>(in / last_each);
+    }
+    e = tile_expert[tile];
     row0 = tile_row0[tile];
+    row_end = offsets[e + 1];
+    const int first_row = offsets[e];
+    if (!is_full && row_end - first_row > TL_ROWS(NWW)) {
+      // Row tiles of an expert that has several read the same weights: up to four of them one after the other for a column
+      // block, so that all but the first find the weights in L2.  (Tiles of the expert that are among the last ones have
+      // been dealt out above.)
+      const int nth = (row0 - first_row) / TL_ROWS(NWW), first = tile - (nth & 3);
+      const int of_expert = (row_end - first_row + TL_ROWS(NWW) - 1) / TL_ROWS(NWW) - (nth & ~3);
+      const unsigned n_here = min(min(4, of_expert), n_light - first);
+      const unsigned in = pair - static_cast<unsigned>(first) * n_col_blocks;
+      tile = first + static_cast<int>(in % n_here);
+      col_block = static_cast<int>(in / n_here);
+      row0 = tile_row0[tile];
+    }
+    once = DIRECT && row_end - first_row <= TL_ROWS(NWW);
   }
   const int held = min(TL_ROWS(NWW), row_end - row0);
   if (held <= 0) return;
-  const bool once = DIRECT && held == row_end - first_row;  // an expert's only tile
 #define CALL(NP, ONCE) \
   tiled_body<GATE_UP, NP, NWW, ONCE, DIRECT>(a, w, out, rows, n_out, width, e, row0, row_end, col_block, lds, act, glu_limit)
 #define BODY(NP) if (once) CALL(NP, DIRECT); else CALL(NP, false)
@@ -391,12 +419,15 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
 // The row-tile map must have been made for tiles of 160 rows, for the wide form of 192.  `wide`: see below.
 // gate_up: 0 a plain product, 1 gate|up rows with SwiGLU, 2 a plain product whose results pass the square of relu.
 // glu_limit > 0: the gate|up rows meet in the clamped form (`ix_glu`).  last_tiles: so many tiles at the end of the
-// map are worked spread among the others; `last_each` consecutive ones of them belong to one expert.
+// map are worked spread among the others; `last_each` consecutive ones of them belong to one expert.  a2, w2, out2 (rows2 0: none, and
+// with the wide form only): a product of its own in the same launch, out2 [rows2, n_out2] = a2 [rows2, width2] . w2^T, gate|up
+// as the grouped one; no last tiles then.
 extern "C" int ix_moe_grouped_tiled(const void* a, const void* w, void* out, const int32_t* offsets,
                                     const int32_t* rows, const int32_t* tile_expert, const int32_t* tile_row0,
                                     const int32_t* tile_info, int max_tiles, int64_t a_rows, int64_t n_out,
                                     int64_t width, int gate_up, int wide, float glu_limit, int last_tiles, int last_each,
-                                    hipStream_t stream) {
+                                    const void* a2, const void* w2, void* out2, int64_t rows2, int64_t n_out2,
+                                    int64_t width2, hipStream_t stream) {
   IX_REQUIRE(n_out > 0 && width > 0 && max_tiles >= 0 && last_tiles >= 0 && last_each > 0, "sizes must be positive");
   IX_REQUIRE(last_tiles % last_each == 0, "the last tiles come in equal groups");
   IX_REQUIRE(width % 8 == 0, "the reduction width must be a multiple of 8 for the matrix-core kernel");
@@ -404,21 +435,30 @@ extern "C" int ix_moe_grouped_tiled(const void* a, const void* w, void* out, con
   IX_REQUIRE(a_rows >= 0 && a_rows * width < (int64_t(1) << 31) && (gate_up == 1 ? 2 : 1) * n_out * width < (int64_t(1) << 31),
              "the activations, and one expert's weights, must hold fewer than 2^31 numbers");
   IX_REQUIRE(max_tiles <= 65535, "too many row tiles for one launch");
-  if (max_tiles == 0) return 0;
+  IX_REQUIRE(rows2 >= 0 && (rows2 == 0 || (wide && last_tiles == 0 && gate_up != 2 && n_out2 > 0 && width2 > 0)),
+             "a second product needs the wide form, no last tiles and positive sizes");
+  IX_REQUIRE(width2 % 8 == 0 || rows2 == 0, "the reduction width must be a multiple of 8 for the matrix-core kernel");
+  IX_REQUIRE(rows2 == 0 || (n_out2 < (1 << 30) && width2 < (1 << 30) && rows2 * width2 < (int64_t(1) << 31) &&
+                            (gate_up == 1 ? 2 : 1) * n_out2 * width2 < (int64_t(1) << 31)),
+             "the second product's activations, and its weights, must hold fewer than 2^31 numbers");
+  if (max_tiles == 0 && rows2 == 0) return 0;
   // wide: four wavefronts along the weight rows instead of two (256 weight rows per workgroup, 112 KB of LDS, one
   // workgroup per compute unit): the activations are staged for half as many column blocks.  Same sums in the
   // same order either way.
   const int nww = wide ? 4 : 2;
   const int cols = gate_up == 1 ? 32 * nww : 64 * nww;
   const int n_col_blocks = static_cast<int>((n_out + cols - 1) / cols);
-  const int64_t groups = 8 * (static_cast<int64_t>(n_col_blocks) * max_tiles / 8 + 2);  // (a die has at most this many pairs)
+  const int64_t full2 = rows2 == 0 ? 0 : (rows2 + TL_ROWS(4) - 1) / TL_ROWS(4) * ((n_out2 + cols - 1) / cols);
+  const int64_t groups = 8 * ((static_cast<int64_t>(n_col_blocks) * max_tiles + full2) / 8 + 2);  // (a die has at most this many pairs)
   IX_REQUIRE(groups < (int64_t(1) << 31), "too many workgroups for one launch");
   dim3 grid(static_cast<unsigned>(groups)), block(TL_THREADS(nww));
-  const bool direct = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
+  const uintptr_t second = rows2 == 0 ? 0 : reinterpret_cast<uintptr_t>(a2) | reinterpret_cast<uintptr_t>(w2);
+  const bool direct = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w) | second) & 15) == 0;
 #define LAUNCH(GU, NWW, DIRECT)                                                                                     \
   hipLaunchKernelGGL((moe_grouped_tiled_kernel<GU, NWW, DIRECT>), grid, block, 0, stream, (const __bf16*)a,         \
                      (const __bf16*)w, (__bf16*)out, offsets, rows, tile_expert, tile_row0, tile_info, (int)n_out,  \
-                     (int)width, n_col_blocks, gate_up == 2 ? 1 : 0, glu_limit, std::min(last_tiles, max_tiles), last_each)
+                     (int)width, n_col_blocks, gate_up == 2 ? 1 : 0, glu_limit, std::min(last_tiles, max_tiles), last_each,         \
+                     (Second{(const __bf16*)a2, (const __bf16*)w2, (__bf16*)out2, (int)rows2, (int)n_out2, (int)width2}))
 #define FORM(GU, NWW)                 \
   if (direct) LAUNCH(GU, NWW, true);  \
   else LAUNCH(GU, NWW, false)

@@ -794,11 +794,14 @@ def moe_tiled_rows(wide: bool) -> int:
 
 def moe_grouped_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offsets: torch.Tensor,
                       rows: Optional[torch.Tensor], tile_map: torch.Tensor, gate_up: bool, wide: bool = False,
-                      glu_limit: float = 0.0, last_tiles: int = 0, last_each: int = 1) -> None:
+                      glu_limit: float = 0.0, last_tiles: int = 0, last_each: int = 1,
+                      second: Optional[Tuple[torch.Tensor, torch.Tensor, torch.Tensor]] = None) -> None:
     """Grouped product staged through LDS (bfloat16, many rows per expert); `tile_map` made for tiles of
     `moe_tiled_rows(wide)` rows.  `wide`: 256 instead of 128 weight rows per workgroup (the same sums in the same
     order).  `last_tiles`: so many tiles at the end of the map are worked spread among the others, `last_each`
-    consecutive ones of them belong to one expert (any number gives the same results)."""
+    consecutive ones of them belong to one expert (any number gives the same results).  `second`: (a, w, out) of a dense
+    product out [T, n] = a [T, k] . w^T (gate|up like the grouped one, w then [2 n, k]) in the same launch, with the wide
+    form and without last tiles."""
     E = w.shape[0]
     A, n_out = out.shape
     K = a.shape[1]
@@ -814,9 +817,18 @@ def moe_grouped_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offse
         _need(a.shape[0] >= A, "a has fewer rows than out")
     mt = moe_max_tiles(A, E, moe_tiled_rows(wide))
     _is_i32(tile_map, 2 * mt + 1)
+    a2 = w2 = out2 = None
+    rows2 = n_out2 = width2 = 0
+    if second is not None:
+        a2, w2, out2 = second
+        (rows2, n_out2), width2 = out2.shape, a2.shape[1]
+        _need(a2.dtype == w2.dtype == out2.dtype == torch.bfloat16, "the matrix-core grouped product is bfloat16 only")
+        _need(a2.shape == (rows2, width2) and w2.shape == ((2 if _epilogue(gate_up) == GATE_UP_SWIGLU else 1) * n_out2, width2),
+              "the second product's shapes do not fit")
     _call("ix_moe_grouped_tiled", _ptr(a), _ptr(w), _ptr(out), _ptr(offsets), _ptr(rows), _ptr(tile_map[:mt]),
           _ptr(tile_map[mt:2 * mt]), _ptr(tile_map[2 * mt:]), _i32(mt), _i64(a.shape[0]), _i64(n_out), _i64(K),
-          _i32(_epilogue(gate_up)), _i32(1 if wide else 0), _f32(glu_limit), _i32(last_tiles), _i32(last_each), _stream())
+          _i32(_epilogue(gate_up)), _i32(1 if wide else 0), _f32(glu_limit), _i32(last_tiles), _i32(last_each),
+          _ptr(a2), _ptr(w2), _ptr(out2), _i64(rows2), _i64(n_out2), _i64(width2), _stream())
 
 
 def moe_grouped_tiled_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offsets: torch.Tensor,

@@ -49,15 +49,18 @@ WIDE_TILES_ALONE_WIDTH = 2048
 # grouping, the two grouped products and the weighted sum then take it along, its weights stream at the rate of the
 # big launches instead of through two library products of few rows and a launch for SwiGLU.  Needs a shared width
 # that is a multiple of the experts' width; keeps the shared expert's weights a second time, in that layout.
-# us of a whole prompt, without / with: A2.7B shape (8 layers) 300 tokens 2,672 / 2,430, 1,024 3,883 / 3,422, 1,536 4,449 /
-# 4,177, 1,800 4,884 / 4,741, 2,048 5,092 / 4,890, 2,176 5,173 / 5,222, 2,560 5,577 / 5,657, 3,072 6,540 / 6,776; 57B shape (4
-# layers) 1,024 tokens 6,290 / 5,550, 1,500 7,522 / 7,263, 2,048 9,178 / 9,040, 2,600 11,127 / 11,257, 4,096 16,078 / 17,077.  The
-# line is eleven whole tiles of the wide form; narrower models, whose products stay in the narrow form, keep theirs (1,300 tokens
-# of the A2.7B shape in that form 4,416 / 4,198, 1,536 4,505 / 4,512).
-# Each piece's result is rounded before the sum adds them in float32: four roundings of a half the size instead of one.  Against
-# 64 bits, fourteen seeds each, without / with: 2,048 tokens 0.02727 / 0.02711, 1,700 0.02628 / 0.02613.
+# us of a whole prompt, without / with: A2.7B shape (8 layers) 300 tokens 2,672 / 2,430, 1,024 3,883 / 3,422; 57B shape (4 layers)
+# 1,024 tokens 6,290 / 5,550, 1,500 7,522 / 7,263.
+# Each piece's result is rounded before the sum adds them in float32: four (57B shape: eight) roundings of a half the size (a third)
+# instead of one.
 FOLD_SHARED_BELOW_TOKENS = 1536
-FOLD_SHARED_BELOW_TOKENS_WIDE = 11 * ops.MOE_TILED_ROWS_WIDE + 1
+# From there on, as far as the wide form goes, the shared expert's products are worked in the launches of the grouped ones as they
+# are, each result one sum in 32 bits with one rounding.  A tile of the down product is then as long as those of all pieces, and
+# worked first, so that it ends with the others as long as the pieces are few.  us of a whole prompt, by itself / in pieces / in the
+# launches: A2.7B shape (8 layers) 1,536 tokens 4,449 / 4,185 / 4,110, 1,800 4,884 / 4,675 / 4,520, 2,112 5,130 / 5,105 / 4,915, 57B shape (4
+# layers) 1,536 7,560 / 7,175 / 7,100, 2,048 9,178 / 9,025 / 8,810.  The line is eleven whole tiles of the wide form.
+FOLD_SHARED_WHOLE_BELOW_TOKENS = 11 * ops.MOE_TILED_ROWS_WIDE + 1
+FOLD_SHARED_WHOLE_PIECES = 8
 
 
 class MoeFeedForward(FeedForward):
@@ -188,7 +191,7 @@ class MoeFeedForward(FeedForward):
 
     def _wide(self, tokens: int) -> bool:
         """Whether the LDS-staged products of this step take their wide form."""
-        alone = self.shared_width == 0 or self._shared_rides_along(tokens)
+        alone = self.shared_width == 0 or self._shared_rides_along(tokens) or self._shared_in_the_launches(tokens)
         return self.wide_tiles or (alone and self.hidden_size >= WIDE_TILES_ALONE_WIDTH)
 
     def _f32_fits(self, x) -> bool:
@@ -210,8 +213,9 @@ class MoeFeedForward(FeedForward):
         ops.moe_dispatch(topk_e, offsets, rows, dest, E, tile_rows, tile_map)
         return offsets, rows, dest, tile_map
 
-    def experts(self, ctx, x, offsets, rows, tile_map=None, tile_rows: int = 0, with_shared: bool = False):
-        """`with_shared`: the grouping holds the shared expert's pieces as further experts."""
+    def experts(self, ctx, x, offsets, rows, tile_map=None, tile_rows: int = 0, with_shared: bool = False, shared=None):
+        """`with_shared`: the grouping holds the shared expert's pieces as further experts.  `shared` [T, hidden]: the shared
+        expert's products go into the launches of the wide form and leave their results there."""
         rt, A = ctx.rt, rows.numel()
         w13, w2 = (self.w13_all, self.w2_all) if with_shared else (self.w13, self.w2)
         act = rt.empty((A, self.expert_width))
@@ -224,8 +228,12 @@ class MoeFeedForward(FeedForward):
             # (a piece of the shared expert holds every token: its tiles are full, and the last ones of the map)
             each = -(-x.shape[0] // tile_rows)
             full = self.shared_pieces * each if with_shared else 0
-            ops.moe_grouped_tiled(x, w13, act, offsets, rows, tile_map, self.first_epilogue, wide, self.limit, full, each)
-            ops.moe_grouped_tiled(act, w2, y, offsets, None, tile_map, False, wide, 0.0, full, each)
+            first = second = None
+            if shared is not None:
+                shared_act = rt.empty((x.shape[0], self.shared_width))
+                first, second = (x, self.w_shared_gate_up, shared_act), (shared_act, self.w_shared_down, shared)
+            ops.moe_grouped_tiled(x, w13, act, offsets, rows, tile_map, self.first_epilogue, wide, self.limit, full, each, first)
+            ops.moe_grouped_tiled(act, w2, y, offsets, None, tile_map, False, wide, 0.0, full, each, second)
         elif tile_rows:
             # few rows: the weights are the traffic, the reduction is split over a workgroup's four wavefronts
             ops.moe_grouped_mfma(x, w13, act, offsets, rows, tile_map, tile_rows, self.first_epilogue, 4, self.limit)
@@ -284,8 +292,14 @@ class MoeFeedForward(FeedForward):
         """Whether the shared expert is among the routed ones, in pieces, in a step of so many tokens: up to the line above, and
         as far as the grouped products' 32-bit places reach."""
         rows = tokens * (self.top_k + self.shared_pieces)
-        line = FOLD_SHARED_BELOW_TOKENS_WIDE if self.hidden_size >= WIDE_TILES_ALONE_WIDTH else FOLD_SHARED_BELOW_TOKENS
-        return self.shared_pieces > 0 and tokens < line and rows * self.expert_width < 1 << 31
+        return self.shared_pieces > 0 and tokens < FOLD_SHARED_BELOW_TOKENS and rows * self.expert_width < 1 << 31
+
+    def _shared_in_the_launches(self, tokens: int) -> bool:
+        """Whether the shared expert's products, whole, go into the grouped products' launches in a step of so many tokens."""
+        return (0 < self.shared_pieces <= FOLD_SHARED_WHOLE_PIECES and self.hidden_size >= WIDE_TILES_ALONE_WIDTH
+                and (self.w_shared_down is None or self.w_shared_down.data_ptr() % 16 == 0)
+                and FOLD_SHARED_BELOW_TOKENS <= tokens < FOLD_SHARED_WHOLE_BELOW_TOKENS
+                and max(tokens, 2 * self.hidden_size) * self.shared_width < 1 << 31)
 
     takes_lazy_norm = True
 
@@ -309,6 +323,11 @@ class MoeFeedForward(FeedForward):
             y = self.experts(ctx, x, offsets, rows, tile_map, tile_rows, with_shared=True)
             return MoeSum(y, dest, topk_w, None, None, self.hidden_size)
         shared = join = None
+        if tile_rows == ops.MOE_TILED_ROWS_WIDE and not one_launch and self._shared_in_the_launches(x.shape[0]):
+            shared = ctx.rt.empty((x.shape[0], self.hidden_size))
+            topk_w, _, gate, offsets, rows, dest, tile_map = self.route_and_dispatch(ctx, x, tile_rows, norm)
+            y = self.experts(ctx, x, offsets, rows, tile_map, tile_rows, shared=shared)
+            return MoeSum(y, dest, topk_w, shared, gate, self.hidden_size)
         if (not one_launch and self.shared_width > 0 and tile_rows == ops.MOE_TILED_ROWS
                 and x.shape[0] >= SHARED_BESIDE_TOKENS and ctx.rt.can_run_beside()):
             # a prompt portion: the shared expert's library products are bound by the matrix cores, the routed

@@ -49,6 +49,15 @@ def test_shared_expert_rides_along_as_far_as_the_products_reach(pieces, width, t
     assert part._shared_rides_along(tokens) == along
 
 
+@pytest.mark.parametrize("hidden,pieces,tokens,whole", [
+    (2048, 4, 1535, False), (2048, 4, 1536, True), (2048, 8, 2112, True), (2048, 4, 2113, False), (2048, 9, 1536, False),
+    (2048, 0, 1536, False), (2040, 4, 1536, False)])
+def test_shared_expert_whole_in_the_launches(hidden, pieces, tokens, whole):
+    from inferx_amd.parts.moe import MoeFeedForward
+    part = MoeFeedForward(hidden, 4, 1, 1408, pieces * 1408)
+    assert part._shared_in_the_launches(tokens) == whole and not (whole and part._shared_rides_along(tokens))
+
+
 @pytest.mark.parametrize("hidden,shared,tokens,wide", [
     (2048, 5632, 33, True), (2048, 5632, 2112, True), (2048, 5632, 2113, False), (2048, 0, 9000, True), (2048, 1000, 33, False),
     (2040, 5632, 33, False), (2040, 0, 33, False), (3072, 5632, 2113, True), (3072, 1000, 33, True)])

@@ -385,6 +385,35 @@ def test_grouped_tiled_last_tiles_of_one_expert_together(T, E, mi, pieces, wide)
                 assert float((got - want).abs().max()) <= 2 ** -8 * float(want.abs().max()) + 1e-5, (H, t, c)
 
 
+@pytest.mark.parametrize("gate_up", [False, True])
+@pytest.mark.parametrize("rows,n,k", [(1, 8, 8), (192, 128, 200), (193, 264, 576), (400, 1000, 1160), (600, 44, 64)])
+def test_grouped_tiled_with_a_second_product(rows, n, k, gate_up):
+    """A dense product in the launch of a grouped one, with longer, equal and shorter reductions, one and more row tiles, fewer and
+    more of them than the grouped product has: its results, and the grouped product's bits as without it."""
+    from inferx_amd import ops
+    T, E, top, mi = 300, 6, 2, 136
+    g = torch.Generator().manual_seed(1)
+    topk_e = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).to(torch.int32).to(DEV)
+    offsets, order, dest, tile_map = dispatch(topk_e, E, ops.MOE_TILED_ROWS_WIDE)
+    a2 = rnd(rows, k, seed=3, dtype=torch.bfloat16)
+    w2 = rnd((2 if gate_up else 1) * n, k, seed=4, dtype=torch.bfloat16, scale=k ** -0.5)
+    for H in (72, 200, 576):
+        x = rnd(T, H, dtype=torch.bfloat16)
+        w = rnd(E, (2 if gate_up else 1) * mi, H, seed=2, dtype=torch.bfloat16, scale=H ** -0.5)
+        out = [torch.full((T * top, mi), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+        buf = torch.full((rows * n + 16,), 7.0, dtype=torch.bfloat16, device=DEV)
+        ops.moe_grouped_tiled(x, w, out[0], offsets, order, tile_map, gate_up, True)
+        ops.moe_grouped_tiled(x, w, out[1], offsets, order, tile_map, gate_up, True, second=(a2, w2, buf[8:-8].view(rows, n)))
+        assert torch.isfinite(out[0]).all() and torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+        assert (buf[:8] == 7).all() and (buf[-8:] == 7).all()
+        want = a2.double() @ w2.double().T
+        if gate_up:
+            want = torch.nn.functional.silu(want[:, :n]) * want[:, n:]
+        assert float((buf[8:-8].view(rows, n).double() - want).abs().max()) <= 2 ** -8 * float(want.abs().max()) + 1e-5
+    with pytest.raises(ops.KernelError):  # (last tiles beside it)
+        ops.moe_grouped_tiled(x, w, out[1], offsets, order, tile_map, gate_up, True, last_tiles=1, second=(a2, w2, buf[8:-8].view(rows, n)))
+
+
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("last", [0, 1, 2, 3, 4, 6])
 def test_grouped_tiled_experts_of_several_tiles_beside_the_last_ones(last, wide):

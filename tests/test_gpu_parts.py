@@ -356,6 +356,45 @@ def test_moe_part_with_wide_expert_tiles():
     assert err(wide, pm.moe_block(x.double(), wd, "m.", E, k, False, si)) < 2e-2
 
 
+@pytest.mark.parametrize("T", [1536, 2112])
+@pytest.mark.parametrize("pieces", [4, 8])
+@pytest.mark.parametrize("cancel", [False, True])
+def test_shared_expert_of_long_steps_is_one_sum(T, pieces, cancel):
+    """Steps of 1,536 to 2,112 tokens in the wide form: the shared expert's result is one sum in 32 bits.  `cancel`: two runs of its
+    columns cancel but for 1/64 of them, so that partial results rounded to bfloat16 would show; equal rows of weights give equal
+    activations, so the bound is that of the rounding of the activations and of the result (at most 2^-9 of each number)."""
+    from inferx_amd.config import PartSpec
+    from inferx_amd.engine.runtime import Runtime
+    from inferx_amd.parts import build_part, resolve_delta
+    rt = Runtime("bfloat16")
+    H, E, mi = 2048, 4, 64
+    si = pieces * mi
+    part = build_part("feed_forward", PartSpec("moe", {"hidden_size": H, "num_experts": E, "top_k": 1, "expert_width": mi,
+                                                       "shared_width": si, "shared_gated": False, "init_std": H ** -0.5}))
+    w = tensors_for(part, rt, seed=4)
+    if cancel:
+        for e in range(E):
+            w[f"experts.{e}.down_proj.weight"].zero_()
+        for n in ("gate", "up"):
+            w[f"shared_expert.{n}_proj.weight"][mi:2 * mi] = w[f"shared_expert.{n}_proj.weight"][:mi]
+        down = w["shared_expert.down_proj.weight"]
+        down[:, 2 * mi:] /= 64
+        down[:, mi:2 * mi] = -(down[:, :mi] * (1 + torch.randn(H, mi, generator=torch.Generator().manual_seed(6)) / 64))
+    part.bind({n: v.to(DEV) for n, v in w.items()}, rt)
+    assert part._shared_in_the_launches(T)
+    ctx, _ = make_ctx(rt, [T], [T], 16, 140)
+    x = torch.randn(T, H, generator=torch.Generator().manual_seed(5)).to(rt.dtype)
+    got = resolve_delta(ctx, part.forward(ctx, x.to(DEV))).double()
+    xd, wd = x.to(DEV).double(), {n: v.to(DEV).double() for n, v in w.items()}
+    mlp = lambda p: (torch.nn.functional.silu(xd @ wd[p + "gate_proj.weight"].T) * (xd @ wd[p + "up_proj.weight"].T)) @ wd[p + "down_proj.weight"].T
+    scores = torch.softmax(xd @ wd["gate.weight"].T, -1)
+    weight, chosen = scores.max(-1, keepdim=True)
+    want = mlp("shared_expert.")
+    for e in range(E):
+        want = want + torch.where(chosen == e, weight, 0.0) * mlp(f"experts.{e}.")
+    assert float((got - want).norm() / want.norm()) < 2.0 ** -8
+
+
 def test_shared_expert_beside_the_routed_ones():
     """A prompt portion: the shared expert runs on a second stream beside the routed experts.  The sum is bit for
     bit that of one stream, also when the calls follow one another without a wait (memory of one call is given

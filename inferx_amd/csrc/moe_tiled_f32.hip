@@ -3,13 +3,13 @@
 //
 // What bounds it: at a few dozen rows per expert the weights' way from memory, from about fifty on the matrix cores
 // (32 cycles for 16 x 16 x 4).  A workgroup owns up to 64 rows of one expert (a tile of the grouping kernel's map: with
-// a few hundred tokens all rows of an expert, so that its weights are read once) x 128 weight rows, which for gate|up are
-// 64 gate rows and their 64 up rows; its four wavefronts take 32 weight rows each (for gate|up sixteen and sixteen)
-// and all of the tile's rows.  Stages of 32 of the reduction (128 bytes a row) go through a ring of three or four LDS
-// buffers that the loads fill by themselves, with one barrier a stage, as in moe_tiled.hip; half a compute unit's LDS, so
-// that two workgroups share one and one's products overlap with the other's waits.  Rows of LDS keep their eight 16-byte
-// pieces permuted (piece p of row r at p ^ ((r >> 1) & 7)), so that sixteen rows read at one piece fall on different banks.
-// The weights of an expert with one tile are read once: past the caches.
+// a few hundred tokens all rows of an expert, so that its weights come from memory once) x one or two blocks of 64 weight rows, which for
+// gate|up are 32 gate rows and their 32 up rows; its four wavefronts take sixteen weight rows of each (for gate|up of one block
+// eight and eight, of two sixteen and sixteen) and all of the tile's rows.  Stages of 32 of the reduction (128 bytes a row) go through a
+// ring of three to six LDS buffers that the loads fill by themselves, with one barrier a stage, as in moe_tiled.hip; half a
+// compute unit's LDS, so that two workgroups share one and one's products overlap with the other's waits.  Rows of LDS keep
+// their eight 16-byte pieces permuted (piece p of row r at p ^ ((r >> 1) & 7)), so that sixteen rows read at one piece fall on
+// different banks.  The weights of an expert with one tile go past the caches.
 //
 // A lane reads four consecutive numbers of its row at a time; product j of a piece multiplies the j-th of them, so the
 // four slots of the reduction that one matrix instruction adds up are the pieces' j-th numbers, the same in both
@@ -17,8 +17,13 @@
 // power of two bytes would otherwise all ask the same memory channels at once.  The order of a result's sum so depends
 // on its column alone (two scores of a later router that are 1e-6 apart fall the other way with another order).
 //
-// Measured with 60 experts of 1,408 on a width of 2,048, 4 a token, unevenly routed, both products, us, against pieces through
-// registers and LDS writes, 64 weight rows, a die's run of tiles in their order: 170 tokens 389 -> 348, 361 503 -> 415, 511 562
+// Two blocks read a tile's activations for half as many workgroups; one block has twice the workgroups, each with half the
+// products.  Which of them, by the workgroups that two would give, the sizes' geometric mean of one product's time (509 shapes of 4 to
+// 128 experts, widths of 512 to 2,560, 40 to 1,024 tokens), two blocks against one: up to 128 1.78, 256 1.38, 512 1.21, 768
+// 1.08, 1,024 1.06, 1,500 1.03, more 0.99 (8 experts of 768 on 2,048, 128 tokens, both products: 116 us, 68 with one).
+//
+// Measured with 60 experts of 1,408 on a width of 2,048, 4 a token, unevenly routed, both products, us, two blocks against pieces through
+// registers and LDS writes, one block, a die's run of tiles in their order: 170 tokens 389 -> 348, 361 503 -> 415, 511 562
 // -> 490, 800 747 -> 648; 32 rows each 428 -> 404, 64 rows each 662 -> 641 (the weights alone take 324, the last one's products
 // 474).  Of it at 511 tokens the direct loads and 128 rows 50 to 65, the order of the tiles 45 to 60; that both blocks of a
 // workgroup keep their own order of sums costs 30.
@@ -29,24 +34,24 @@
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define TF_ROWS 64     // rows of a tile of the map
-#define TF_WROWS 128   // weight rows per workgroup
 #define TF_K 32        // numbers of the reduction per stage
 #define TF_APART 3     // stages between the starts of neighbouring blocks of 64 weight rows
 #define TF_LDS 81920   // bytes: half a compute unit's
 __device__ __forceinline__ int tf_at(int row, int piece) { return row * TF_K + ((piece ^ ((row >> 1) & 7)) << 2); }
 
-// NT: sixteens of rows that the tile holds.  Every load is unconditional: a stage past the end asks for the last stage
-// again, a piece past the row's end for the row's last one, with zeros in its place among the operands.
-template <bool GATE_UP, int NT, bool ONCE>
+// BLOCKS: blocks of 64 weight rows that the workgroup owns, one or two.  NT: sixteens of rows that the tile holds.  Every load
+// is unconditional: a stage past the end asks for the last stage again, a piece past the row's end for the row's last one, with
+// zeros in its place among the operands.
+template <bool GATE_UP, int NT, bool ONCE, int BLOCKS>
 __device__ __forceinline__ void tiled_f32_body(const float* a, const float* w, float* out,
                                                const int32_t* __restrict__ rows, int n_out, int width, int e, int row0,
                                                int row_end, int col_block, float* lds, int act, float glu_limit) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15, g = lane >> 4;
-  constexpr int COLS = GATE_UP ? TF_WROWS / 2 : TF_WROWS;
-  constexpr int NPW = TF_WROWS / 32, NPX = (NT + 1) / 2;  // loads of a wavefront a stage, eight rows each
-  constexpr int RING = NT <= 2 ? 4 : 3;                   // stages that LDS holds
-  constexpr unsigned WT = TF_WROWS * 4 * TF_K, XT = 32 * NPX * 4 * TF_K;  // bytes of a stage
+  constexpr int COLS = (GATE_UP ? 32 : 64) * BLOCKS;
+  constexpr int NPW = 2 * BLOCKS, NPX = (NT + 1) / 2;  // loads of a wavefront a stage, eight rows each
+  constexpr int RING = BLOCKS == 2 ? (NT <= 2 ? 4 : 3) : (NT <= 2 ? 6 : 5);  // stages that LDS holds
+  constexpr unsigned WT = 64 * BLOCKS * 4 * TF_K, XT = 32 * NPX * 4 * TF_K;  // bytes of a stage
   static_assert(RING * (WT + XT) <= TF_LDS, "the rings fit");
   const int n0 = col_block * COLS;
 
@@ -55,8 +60,9 @@ __device__ __forceinline__ void tiled_f32_body(const float* a, const float* w, f
   int64_t wsrc[NPW], xsrc[NPX];  // where this lane's rows start, in numbers
 #pragma unroll
   for (int i = 0; i < NPW; ++i) {
-    const int r = 8 * (wave + 4 * i) + (lane >> 3);  // LDS row; wavefront r / 32 multiplies it, for gate|up sixteen gate rows, then their up rows
-    const int src = GATE_UP ? ((r & 16) ? n_out : 0) + min(n0 + 16 * (r >> 5) + (r & 15), n_out - 1) : min(n0 + r, n_out - 1);
+    // LDS row; wavefront r / (16 BLOCKS) multiplies it, for gate|up 8 BLOCKS gate rows, then their up rows
+    const int r = 8 * (wave + 4 * i) + (lane >> 3), of = r / (16 * BLOCKS), in = r % (8 * BLOCKS);
+    const int src = GATE_UP ? ((r & (8 * BLOCKS)) ? n_out : 0) + min(n0 + 8 * BLOCKS * of + in, n_out - 1) : min(n0 + r, n_out - 1);
     wsrc[i] = static_cast<int64_t>(src) * width;
   }
 #pragma unroll
@@ -66,46 +72,46 @@ __device__ __forceinline__ void tiled_f32_body(const float* a, const float* w, f
   }
   const int piece = 4 * ((lane & 7) ^ (4 * (wave & 1) + (lane >> 4)));  // what belongs at piece lane & 7 of the lane's rows
 
-  // Blocks of 64 weight rows start the reduction at a stage that follows from their number and wrap round.  A workgroup
-  // owns two of them, which start TF_APART stages apart: it walks so many stages more, the first of them for the first two
-  // wavefronts only and the last of them for the others.
+  // Blocks of 64 weight rows start the reduction at a stage that follows from their number and wrap round.  The two of a
+  // workgroup that owns two start TF_APART stages apart: it walks so many stages more, the first of them for the first two
+  // wavefronts only and the last of them for the others (and asks for all rows in each, so for 3 stages of every row twice).
   const int stages = (width + TF_K - 1) / TF_K;
   const bool turned = (width & 255) == 0;  // (then there are eight stages at least)
-  const int total = stages + (turned ? TF_APART : 0);
-  const int begin = turned ? static_cast<int>((static_cast<unsigned>(col_block) * (2u * TF_APART)) % stages) : 0;
+  const int total = stages + (BLOCKS == 2 && turned ? TF_APART : 0);
+  const int begin = turned ? static_cast<int>((static_cast<unsigned>(col_block) * (unsigned{BLOCKS} * TF_APART)) % stages) : 0;
   auto place = [&](int s) {  // where stage s starts in a row (past the end: the last stage again)
     int k = min(s, total - 1) + begin;
     k = k < stages ? k : k - stages;
     return (k < stages ? k : k - stages) * TF_K;
   };
-  auto mine = [&](int s) { return !turned || (wave < 2 ? s < stages : s >= TF_APART); };
+  auto mine = [&](int s) { return BLOCKS == 1 || !turned || (wave < 2 ? s < stages : s >= TF_APART); };
   auto load = [&](int buf, int i, int at) {  // the i-th of a stage's loads
     if (i < NPX) lds_load16<false>(lds, RING * WT + buf * XT + 1024 * (wave + 4 * i), a + xsrc[i] + at);
     else if (i < NPX + NPW) lds_load16<ONCE>(lds, buf * WT + 1024 * (wave + 4 * (i - NPX)), w_expert + wsrc[i - NPX] + at);
   };
   auto at_stage = [&](int s) { return min(place(s) + piece, width - 4); };
 
-  f32x4 acc[2][NT];
+  f32x4 acc[BLOCKS][NT];
 #pragma unroll
-  for (int b = 0; b < 2; ++b)
+  for (int b = 0; b < BLOCKS; ++b)
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[b][t] = f32x4{0.f, 0.f, 0.f, 0.f};
   int at16[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) at16[h] = tf_at(m, 4 * h + g);
-  const float* const ws = lds + 32 * wave * TF_K;
+  const float* const ws = lds + 16 * BLOCKS * wave * TF_K;
   const float* const xs = lds + RING * WT / 4;
-  struct Half { f32x4 w[2], x[NT]; };
+  struct Half { f32x4 w[BLOCKS], x[NT]; };
   Half h0, h1;
-  auto read = [&](Half& h, int i, int buf, int half) {  // the i-th of a half's NT + 2 pieces
-    if (i < 2) h.w[i] = *reinterpret_cast<const f32x4*>(ws + buf * (WT / 4) + at16[half] + 16 * i * TF_K);
-    else if (i < NT + 2) h.x[i - 2] = *reinterpret_cast<const f32x4*>(xs + buf * (XT / 4) + at16[half] + 16 * (i - 2) * TF_K);
+  auto read = [&](Half& h, int i, int buf, int half) {  // the i-th of a half's NT + BLOCKS pieces
+    if (i < BLOCKS) h.w[i] = *reinterpret_cast<const f32x4*>(ws + buf * (WT / 4) + at16[half] + 16 * i * TF_K);
+    else if (i < NT + BLOCKS) h.x[i - BLOCKS] = *reinterpret_cast<const f32x4*>(xs + buf * (XT / 4) + at16[half] + 16 * (i - BLOCKS) * TF_K);
   };
   auto products = [&](const Half& h, int j) {
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(h.w[b][j], h.x[t][j], acc[b][t], 0, 0, 0);
+      for (int b = 0; b < BLOCKS; ++b) acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(h.w[b][j], h.x[t][j], acc[b][t], 0, 0, 0);
   };
 #pragma unroll
   for (int s = 0; s < RING; ++s)
@@ -115,13 +121,13 @@ __device__ __forceinline__ void tiled_f32_body(const float* a, const float* w, f
   lds_barrier();
   int buf = 0;
 #pragma unroll
-  for (int i = 0; i < NT + 2; ++i) read(h0, i, buf, 0);
-  constexpr int READS = (NT + 2 + 1) / 2, LOADS = (NPX + NPW + 2) / 3;
+  for (int i = 0; i < NT + BLOCKS; ++i) read(h0, i, buf, 0);
+  constexpr int READS = (NT + BLOCKS + 1) / 2, LOADS = (NPX + NPW + 2) / 3;
   auto stage = [&](auto left, int s) {
     constexpr int LEFT = decltype(left)::value;  // at least so many stages follow
     if constexpr (LEFT == 0) {
 #pragma unroll
-      for (int i = 0; i < NT + 2; ++i) read(h1, i, buf, 1);
+      for (int i = 0; i < NT + BLOCKS; ++i) read(h1, i, buf, 1);
       if (width & (TF_K - 1)) {  // the last stage is not whole
         const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -129,7 +135,7 @@ __device__ __forceinline__ void tiled_f32_body(const float* a, const float* w, f
           if (place(s) + 16 * half + 4 * g >= width) {
             Half& h = half ? h1 : h0;
 #pragma unroll
-            for (int b = 0; b < 2; ++b) h.w[b] = zero;
+            for (int b = 0; b < BLOCKS; ++b) h.w[b] = zero;
 #pragma unroll
             for (int t = 0; t < NT; ++t) h.x[t] = zero;
           }
@@ -169,6 +175,10 @@ __device__ __forceinline__ void tiled_f32_body(const float* a, const float* w, f
   };
 #define TF_STAGE(LEFT, S) stage(std::integral_constant<int, (LEFT)>{}, (S))
   for (int s = 0; s < total - RING; ++s) TF_STAGE(RING, s);
+  if constexpr (RING > 5)
+    if (total > 5) TF_STAGE(5, total - 6);
+  if constexpr (RING > 4)
+    if (total > 4) TF_STAGE(4, total - 5);
   if constexpr (RING > 3)
     if (total > 3) TF_STAGE(3, total - 4);
   if (total > 2) TF_STAGE(2, total - 3);
@@ -177,21 +187,22 @@ __device__ __forceinline__ void tiled_f32_body(const float* a, const float* w, f
 #undef TF_STAGE
   wait_loads<0>();  // (with fewer stages than the ring holds, the last one again)
 
-  // lane holds weight rows (sixteen) + 4 g + i of tile row 16 t + m
+  // lane holds weight rows (sixteen) + 4 g + i of tile row 16 t + m; for gate|up of one block lanes of g 0, 1 the gate's sums,
+  // those of g 2, 3 (32 lanes on) the same columns' up sums
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int r = row0 + 16 * t + m;
 #pragma unroll
-    for (int b = 0; b < (GATE_UP ? 1 : 2); ++b) {
+    for (int b = 0; b < (GATE_UP ? 1 : BLOCKS); ++b) {
       float v[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         v[i] = acc[b][t][i];
-        if constexpr (GATE_UP) v[i] = ix_glu(v[i], acc[1][t][i], glu_limit);
+        if constexpr (GATE_UP) v[i] = ix_glu(v[i], BLOCKS == 2 ? acc[BLOCKS - 1][t][i] : __shfl_xor(v[i], 32, IX_WAVE), glu_limit);
         else if (act) v[i] = v[i] > 0.f ? v[i] * v[i] : 0.f;  // the square of relu
       }
-      if (r >= row_end) continue;
-      const int nb = n0 + (GATE_UP ? 16 : 32) * wave + 16 * b + 4 * g;
+      if (r >= row_end || (GATE_UP && BLOCKS == 1 && g >= 2)) continue;
+      const int nb = n0 + (GATE_UP ? 8 : 16) * BLOCKS * wave + 16 * b + 4 * g;
       float* o = out + static_cast<int64_t>(r) * n_out + nb;
       if (nb + 4 <= n_out && (n_out & 3) == 0) {
         *reinterpret_cast<f32x4*>(o) = f32x4{v[0], v[1], v[2], v[3]};
@@ -204,7 +215,7 @@ __device__ __forceinline__ void tiled_f32_body(const float* a, const float* w, f
   }
 }
 
-template <bool GATE_UP>
+template <bool GATE_UP, int BLOCKS>
 __global__ void __launch_bounds__(256, 2)
 moe_grouped_tiled_f32_kernel(const float* a, const float* w, float* out, const int32_t* __restrict__ offsets,
                              const int32_t* __restrict__ rows, const int32_t* __restrict__ tile_expert,
@@ -256,7 +267,7 @@ moe_grouped_tiled_f32_kernel(const float* a, const float* w, float* out, const i
   if (held <= 0) return;
   const bool once = held == row_end - offsets[e];  // an expert's only tile: its weights are read once, past the caches
 #define CALL(NT, ONCE) \
-  tiled_f32_body<GATE_UP, NT, ONCE>(a, w, out, rows, n_out, width, e, row0, row_end, col_block, lds, act, glu_limit)
+  tiled_f32_body<GATE_UP, NT, ONCE, BLOCKS>(a, w, out, rows, n_out, width, e, row0, row_end, col_block, lds, act, glu_limit)
 #define BODY(NT) if (once) CALL(NT, true); else CALL(NT, false)
   switch ((held + 15) >> 4) {
     case 1: BODY(1); break;
@@ -285,16 +296,25 @@ extern "C" int ix_moe_grouped_tiled_f32(const float* a, const float* w, float* o
   IX_REQUIRE(gate_up >= 0 && gate_up <= 2, "gate_up must be 0, 1 or 2");
   IX_REQUIRE(max_tiles <= 65535, "too many row tiles for one launch");
   if (max_tiles == 0) return 0;
-  const int cols = gate_up == 1 ? TF_WROWS / 2 : TF_WROWS;
-  const int n_col_blocks = static_cast<int>((n_out + cols - 1) / cols);
+  const auto column_blocks = [&](int blocks) {
+    const int cols = (gate_up == 1 ? 32 : 64) * blocks;
+    return (n_out + cols - 1) / cols;
+  };
+  const int blocks = column_blocks(2) * max_tiles <= 1024 ? 1 : 2;  // (see the top of the file)
+  const int n_col_blocks = static_cast<int>(column_blocks(blocks));
   const int64_t groups = static_cast<int64_t>(n_col_blocks) * max_tiles;
   IX_REQUIRE(groups < (int64_t(1) << 31), "too many workgroups for one launch");
   dim3 grid(static_cast<unsigned>(groups)), block(256);
-  if (gate_up == 1)
-    hipLaunchKernelGGL((moe_grouped_tiled_f32_kernel<true>), grid, block, 0, stream, a, w, out, offsets, rows, tile_expert,
-                       tile_row0, tile_info, (int)n_out, (int)width, n_col_blocks, 0, glu_limit);
-  else
-    hipLaunchKernelGGL((moe_grouped_tiled_f32_kernel<false>), grid, block, 0, stream, a, w, out, offsets, rows, tile_expert,
-                       tile_row0, tile_info, (int)n_out, (int)width, n_col_blocks, gate_up == 2 ? 1 : 0, glu_limit);
+#define LAUNCH(GU, BLOCKS)                                                                                                  \
+  hipLaunchKernelGGL((moe_grouped_tiled_f32_kernel<GU, BLOCKS>), grid, block, 0, stream, a, w, out, offsets, rows,          \
+                     tile_expert, tile_row0, tile_info, (int)n_out, (int)width, n_col_blocks, gate_up == 2 ? 1 : 0, glu_limit)
+  if (gate_up == 1) {
+    if (blocks == 2) LAUNCH(true, 2);
+    else LAUNCH(true, 1);
+  } else {
+    if (blocks == 2) LAUNCH(false, 2);
+    else LAUNCH(false, 1);
+  }
+#undef LAUNCH
   return ix_check_launch("ix_moe_grouped_tiled_f32");
 }

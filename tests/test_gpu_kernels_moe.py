@@ -737,6 +737,29 @@ def test_grouped_tiled_in_float32_worked_by_their_rows(counts, K):
     assert rel_err(out, want) < 1e-5  # (every product and sum is 32-bit)
 
 
+@pytest.mark.parametrize("gate_up", [0, 1, 2])
+@pytest.mark.parametrize("K", [4, 32, 68, 96, 128, 160, 196, 256, 512])
+def test_grouped_tiled_in_float32_of_few_and_many_workgroups(K, gate_up):
+    """One block of weight rows a workgroup, and two where (further, empty) experts make many workgroups: float64's results, and the
+    same bits.  Tiles of all heights, one to sixteen stages through rings of three to six buffers, columns past the last block."""
+    from inferx_amd import ops
+    counts, T, n = [5, 64, 17, 1, 0, 40, 33, 130], 70, 388  # (four blocks of 128 and more: 52 workgroups at least, 1,160)
+    E, A = len(counts), sum(counts)
+    topk_e = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).to(torch.int32)[:, None].to(DEV)
+    rows = torch.randint(0, T, (A,), generator=torch.Generator().manual_seed(2)).to(torch.int32).to(DEV)
+    x, few = rnd(T, K, scale=K ** -0.25), rnd(E, (2 if gate_up == 1 else 1) * n, K, seed=1, scale=K ** -0.25)
+    many = torch.cat([few, torch.full((300 - E,) + few.shape[1:], float("nan"), device=DEV)])
+    out = []
+    for w in (few, many):
+        offsets, _, _, tile_map = dispatch(topk_e, w.shape[0], ops.MOE_TILED_F32_ROWS)
+        out.append(torch.full((A, n), float("nan"), device=DEV))
+        ops.moe_grouped_tiled_f32(x, w, out[-1], offsets, rows, tile_map, gate_up)
+    z = torch.cat([x[rows.long()][lo:hi].double() @ few[e].double().T
+                   for e, (lo, hi) in enumerate(zip(offsets.tolist()[:E], offsets.tolist()[1:E + 1]))])
+    want = z if gate_up == 0 else torch.relu(z) ** 2 if gate_up == 2 else torch.nn.functional.silu(z[:, :n]) * z[:, n:]
+    assert rel_err(out[0], want) < 1e-5 and torch.equal(*out)  # (every product and sum is 32-bit)
+
+
 @pytest.mark.parametrize("T,N,K", [(1, 301, 36), (16, 33, 2048), (17, 384, 100), (32, 70, 4), (64, 1000, 260)])
 def test_linear_skinny_in_float32(T, N, K):
     from inferx_amd import ops

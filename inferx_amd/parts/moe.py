@@ -57,8 +57,8 @@ FOLD_SHARED_BELOW_TOKENS = 1536
 # From there on, as far as the wide form goes, the shared expert's products are worked in the launches of the grouped ones as they
 # are, each result one sum in 32 bits with one rounding.  A tile of the down product is then as long as those of all pieces, and
 # worked first, so that it ends with the others as long as the pieces are few.  us of a whole prompt, by itself / in pieces / in the
-# launches: A2.7B shape (8 layers) 1,536 tokens 4,449 / 4,185 / 4,110, 1,800 4,884 / 4,675 / 4,520, 2,112 5,130 / 5,105 / 4,915, 57B shape (4
-# layers) 1,536 7,560 / 7,175 / 7,100, 2,048 9,178 / 9,025 / 8,810.  The line is eleven whole tiles of the wide form.
+# launches: A2.7B shape (8 layers) 1,536 tokens 4,090 / 4,185 / 4,110, 1,800 4,815 / 4,675 / 4,520, 2,112 5,175 / 5,105 / 4,915, 57B shape (4
+# layers) 1,536 7,575 / 7,175 / 7,100, 2,048 9,135 / 9,025 / 8,810.  The line is eleven whole tiles of the wide form.
 FOLD_SHARED_WHOLE_BELOW_TOKENS = 11 * ops.MOE_TILED_ROWS_WIDE + 1
 FOLD_SHARED_WHOLE_PIECES = 8
 

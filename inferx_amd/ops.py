@@ -792,6 +792,13 @@ def moe_tiled_rows(wide: bool) -> int:
     return MOE_TILED_ROWS_WIDE if wide else MOE_TILED_ROWS
 
 
+def moe_tiled_workgroups(assignments: int, experts: int, n_out: int, gate_up: bool) -> float:
+    """About how many workgroups a narrow LDS-staged grouped product has: an expert's last tile is half full on average, and one
+    with a row has a tile."""
+    tiles = max(min(experts, assignments), assignments / MOE_TILED_ROWS + experts / 2)
+    return tiles * -(-n_out // (64 if gate_up else 128))
+
+
 def moe_grouped_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offsets: torch.Tensor,
                       rows: Optional[torch.Tensor], tile_map: torch.Tensor, gate_up: bool, wide: bool = False,
                       glu_limit: float = 0.0, last_tiles: int = 0, last_each: int = 1,

@@ -68,6 +68,20 @@ def test_wide_expert_products(hidden, shared, tokens, wide):
     assert part._wide(tokens) == wide
 
 
+@pytest.mark.parametrize("experts,top,width,shared,tokens,wide", [
+    (60, 4, 1408, 5632, 64, True), (60, 4, 1408, 0, 64, True), (60, 4, 1408, 5632, 2112, True), (8, 6, 768, 0, 203, False),
+    (8, 2, 1408, 1408, 1500, False), (8, 2, 2816, 0, 9000, True), (128, 8, 768, 0, 60, True)])
+def test_wide_expert_products_take_many_workgroups(experts, top, width, shared, tokens, wide):
+    """At a width of 2,048 the narrow form stays where the wide one would leave compute units without work."""
+    from types import SimpleNamespace
+    from inferx_amd import ops
+    from inferx_amd.parts.moe import MoeFeedForward
+    part = MoeFeedForward(2048, experts, top, width, shared)
+    part.w13 = part.w2 = torch.empty(0, dtype=torch.bfloat16)
+    x = torch.empty(tokens, 2048, dtype=torch.bfloat16)
+    assert part._wide(tokens) and part._tile_rows(SimpleNamespace(rt=SimpleNamespace(SKINNY_ROWS=32)), x) == ops.moe_tiled_rows(wide)
+
+
 @pytest.mark.parametrize("units,longest,span,head_dim,slices,loads", [
     (16, 517, 0, 128, 16, 1), (16, 65, 0, 128, 1, 1), (4, 128, 0, 128, 1, 1), (4, 129, 0, 128, 4, 1),   # one request
     (4, 64, 0, 128, 1, 2), (32, 40, 0, 128, 1, 2), (33, 40, 0, 128, 1, 1), (2048, 64, 0, 128, 1, 2), (2048, 65, 0, 128, 1, 1),

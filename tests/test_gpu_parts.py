@@ -381,6 +381,7 @@ def test_shared_expert_of_long_steps_is_one_sum(T, pieces, cancel):
         down[:, 2 * mi:] /= 64
         down[:, mi:2 * mi] = -(down[:, :mi] * (1 + torch.randn(H, mi, generator=torch.Generator().manual_seed(6)) / 64))
     part.bind({n: v.to(DEV) for n, v in w.items()}, rt)
+    part.wide_tiles = True  # (so few workgroups would be narrow ones)
     assert part._shared_in_the_launches(T)
     ctx, _ = make_ctx(rt, [T], [T], 16, 140)
     x = torch.randn(T, H, generator=torch.Generator().manual_seed(5)).to(rt.dtype)

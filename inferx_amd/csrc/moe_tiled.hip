@@ -29,6 +29,10 @@
 //   The rings: what LDS holds, the weights, which come from memory, at least as deep as the activations, which come from
 // L2.  (Four against three stages for tiles of up to 64 rows: no difference; two: 484 against 412 us at 64 experts of 2,560,
 // rows of 3,584, 64 rows each on average.)
+//   A launch of no more narrow workgroups than compute units gives each all of the LDS: three stages of the highest tiles too, of which
+// half of it holds two, and six of the lowest.  Eight experts of 768 on a width of 2,048, 203 tokens of six, both products 36 + 16 us with half,
+// so 29.4 + 13.9 (with the pieces through registers 28.4 + 13.7); four of 2,048 on 2,816, 359 tokens 50 + 34, so 39.5 + 27.6 (35.7 +
+// 23.2).  Four to eight stages are no faster.  Of more workgroups some wait for places: 304 + 304 of them 64 us with half, 96 so.
 //   Both products, us, against the pieces through registers: 60 experts of 1,408, rows of 2,048, beside four of every row,
 // 340 rows: narrow 128 + 76 (135 + 80), wide 123 + 77 (130 + 83); 2,048 rows unevenly over the 60: wide 166 + 88 (182 + 100);
 // 64 experts of 2,560, rows of 3,584, wide, beside eight of every row: 512 rows 524 + 291 (570 + 316), 682 rows 581 + 326 (607
@@ -61,7 +65,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // threads per workgroup.  With four, a row tile's activations are read for half as many column blocks.
 #define TL_THREADS(NWW) (128 * (NWW))
 #define TL_STRIDE 64  // elements per LDS row: no padding; the eight 16-byte pieces of a row are stored permuted
-#define TL_LDS(NWW) ((NWW) == 4 ? 163840 : 81920)  // bytes: all of a compute unit's, or half
+#define TL_LDS(ALL) ((ALL) ? 163840 : 81920)  // bytes: all of a compute unit's, or half
 // piece p of row r lies at piece p ^ ((r >> 1) & 7): the sixteen rows that a quarter of a wavefront reads at one
 // piece index then fall on sixteen different groups of four banks, as do the pieces that sixteen lanes write
 __device__ __forceinline__ int tl_at(int row, int piece) { return row * TL_STRIDE + ((piece ^ ((row >> 1) & 7)) << 3); }
@@ -79,20 +83,22 @@ __device__ __forceinline__ void to_lds(__bf16* lds, unsigned dst, unsigned offse
 }
 
 // How many stages' weights (W) and activations (X) LDS holds.
-template <int NP, int NWW> struct Ring {
+// ALL: a workgroup has all of a compute unit's LDS.
+template <int NP, int NWW, bool ALL> struct Ring {
   static constexpr int XROWS = NWW == 4 ? 64 * ((NP + 1) / 2) : 32 * NP;  // rows staged: whole loads for every wavefront
-  static constexpr int W = NWW == 4 ? (NP <= 2 ? 4 : 3) : (NP == 1 ? 4 : NP <= 4 ? 3 : 2);
-  static constexpr int X = NWW == 4 ? (NP <= 2 ? 4 : NP <= 4 ? 3 : 2) : (NP == 1 ? 4 : NP == 2 ? 3 : 2);
-  static_assert((W * 64 * NWW + X * XROWS) * 2 * TL_STRIDE <= TL_LDS(NWW), "the rings fit");
+  static constexpr int NARROW_ALL = NP == 1 ? 6 : NP == 2 ? 4 : 3;
+  static constexpr int W = NWW == 4 ? (NP <= 2 ? 4 : 3) : ALL ? NARROW_ALL : (NP == 1 ? 4 : NP <= 4 ? 3 : 2);
+  static constexpr int X = NWW == 4 ? (NP <= 2 ? 4 : NP <= 4 ? 3 : 2) : ALL ? NARROW_ALL : (NP == 1 ? 4 : NP == 2 ? 3 : 2);
+  static_assert((W * 64 * NWW + X * XROWS) * 2 * TL_STRIDE <= TL_LDS(ALL), "the rings fit");
   static_assert(W == X || W == X + 1, "the waits below count on it");
 };
 
 // One row tile x 64 NWW weight rows.  NP: pairs of sixteens of activation rows the tile holds, one of each a wavefront.
-template <bool GATE_UP, int NP, int NWW, bool ONCE, bool DIRECT>
+template <bool GATE_UP, int NP, int NWW, bool ALL, bool ONCE, bool DIRECT>
 __device__ __forceinline__ void
 tiled_body(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restrict__ rows, int n_out, int width,
            int e, int row0, int row_end, int col_block, __bf16* lds, int act, float glu_limit) {
-  using R = Ring<NP, NWW>;
+  using R = Ring<NP, NWW, ALL>;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15, g = lane >> 4;
   const int wi = wave % NWW, xi = wave / NWW;
@@ -246,6 +252,10 @@ tiled_body(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restr
   };
 #define TL_STAGE(LEFT, S) stage(std::integral_constant<int, (LEFT)>{}, (S))
   for (int s = 0; s < stages - R::W; ++s) TL_STAGE(R::W, s);
+  if constexpr (R::W > 5)
+    if (stages > 5) TL_STAGE(5, stages - 6);
+  if constexpr (R::W > 4)
+    if (stages > 4) TL_STAGE(4, stages - 5);
   if constexpr (R::W > 3)
     if (stages > 3) TL_STAGE(3, stages - 4);
   if constexpr (R::W > 2)
@@ -267,7 +277,7 @@ tiled_body(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restr
   if (((n_out & 7) | static_cast<int>(reinterpret_cast<uintptr_t>(out) & 15)) == 0) {
     // The tile goes through LDS, so that a store is 16 bytes a lane and whole lines.
     constexpr int OUT_STRIDE = COLS + 8;
-    static_assert(TL_ROWS(NWW) * OUT_STRIDE * 2 <= TL_LDS(NWW), "the result's tile fits the stages' LDS");
+    static_assert(TL_ROWS(NWW) * OUT_STRIDE * 2 <= TL_LDS(ALL), "the result's tile fits the stages' LDS");
     __bf16* const tile = lds;
     __syncthreads();
 #pragma unroll
@@ -319,14 +329,14 @@ struct Second {
   int rows, n_out, width;
 };
 
-template <bool GATE_UP, int NWW, bool DIRECT>
+template <bool GATE_UP, int NWW, bool ALL, bool DIRECT>
 __global__ void __launch_bounds__(TL_THREADS(NWW)) __attribute__((amdgpu_waves_per_eu(2, 2)))
 moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restrict__ offsets,
                          const int32_t* __restrict__ rows,
                          const int32_t* __restrict__ tile_expert, const int32_t* __restrict__ tile_row0,
                          const int32_t* __restrict__ tile_info, int n_out, int width, int n_col_blocks,
                          int act, float glu_limit, int last_tiles, int last_each, Second second) {
-  __shared__ __attribute__((aligned(1024))) __bf16 lds[TL_LDS(NWW) / 2];
+  __shared__ __attribute__((aligned(1024))) __bf16 lds[TL_LDS(ALL) / 2];
   // Workgroups go to the chip's eight dies in turn, by their number, and each die has its own L2 and its own share of the
   // memory's bandwidth.  The (row tile, column block) pairs, tile by tile, are cut into eight equal runs, one a die, so that
   // the column blocks of a tile, which read the same activations, share an L2 and no die has more of them than another.
@@ -402,7 +412,7 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
   const int held = min(TL_ROWS(NWW), row_end - row0);
   if (held <= 0) return;
 #define CALL(NP, ONCE) \
-  tiled_body<GATE_UP, NP, NWW, ONCE, DIRECT>(a, w, out, rows, n_out, width, e, row0, row_end, col_block, lds, act, glu_limit)
+  tiled_body<GATE_UP, NP, NWW, ALL, ONCE, DIRECT>(a, w, out, rows, n_out, width, e, row0, row_end, col_block, lds, act, glu_limit)
 #define BODY(NP) if (once) CALL(NP, DIRECT); else CALL(NP, false)
   switch ((held + 31) >> 5) {  // pairs of sixteens of rows this tile holds
     case 1: BODY(1); break;
@@ -416,7 +426,10 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
 #undef CALL
 }
 
-// The row-tile map must have been made for tiles of 160 rows, for the wide form of 192.  `wide`: see below.
+// The row-tile map must have been made for tiles of 160 rows, for the wide form of 192.  form: 0 narrow; 1 wide, four wavefronts
+// along the weight rows instead of two (256 weight rows a workgroup, all of a compute unit's LDS): the activations are staged for half as
+// many column blocks; 2 narrow with all of a compute unit's LDS, for launches that leave no two workgroups to a compute unit.
+// Same sums in the same order in all of them.
 // gate_up: 0 a plain product, 1 gate|up rows with SwiGLU, 2 a plain product whose results pass the square of relu.
 // glu_limit > 0: the gate|up rows meet in the clamped form (`ix_glu`).  last_tiles: so many tiles at the end of the
 // map are worked spread among the others; `last_each` consecutive ones of them belong to one expert.  a2, w2, out2 (rows2 0: none, and
@@ -425,7 +438,7 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
 extern "C" int ix_moe_grouped_tiled(const void* a, const void* w, void* out, const int32_t* offsets,
                                     const int32_t* rows, const int32_t* tile_expert, const int32_t* tile_row0,
                                     const int32_t* tile_info, int max_tiles, int64_t a_rows, int64_t n_out,
-                                    int64_t width, int gate_up, int wide, float glu_limit, int last_tiles, int last_each,
+                                    int64_t width, int gate_up, int form, float glu_limit, int last_tiles, int last_each,
                                     const void* a2, const void* w2, void* out2, int64_t rows2, int64_t n_out2,
                                     int64_t width2, hipStream_t stream) {
   IX_REQUIRE(n_out > 0 && width > 0 && max_tiles >= 0 && last_tiles >= 0 && last_each > 0, "sizes must be positive");
@@ -435,17 +448,15 @@ extern "C" int ix_moe_grouped_tiled(const void* a, const void* w, void* out, con
   IX_REQUIRE(a_rows >= 0 && a_rows * width < (int64_t(1) << 31) && (gate_up == 1 ? 2 : 1) * n_out * width < (int64_t(1) << 31),
              "the activations, and one expert's weights, must hold fewer than 2^31 numbers");
   IX_REQUIRE(max_tiles <= 65535, "too many row tiles for one launch");
-  IX_REQUIRE(rows2 >= 0 && (rows2 == 0 || (wide && last_tiles == 0 && gate_up != 2 && n_out2 > 0 && width2 > 0)),
+  IX_REQUIRE(form >= 0 && form <= 2, "form must be 0, 1 or 2");
+  IX_REQUIRE(rows2 >= 0 && (rows2 == 0 || (form == 1 && last_tiles == 0 && gate_up != 2 && n_out2 > 0 && width2 > 0)),
              "a second product needs the wide form, no last tiles and positive sizes");
   IX_REQUIRE(width2 % 8 == 0 || rows2 == 0, "the reduction width must be a multiple of 8 for the matrix-core kernel");
   IX_REQUIRE(rows2 == 0 || (n_out2 < (1 << 30) && width2 < (1 << 30) && rows2 * width2 < (int64_t(1) << 31) &&
                             (gate_up == 1 ? 2 : 1) * n_out2 * width2 < (int64_t(1) << 31)),
              "the second product's activations, and its weights, must hold fewer than 2^31 numbers");
   if (max_tiles == 0 && rows2 == 0) return 0;
-  // wide: four wavefronts along the weight rows instead of two (256 weight rows per workgroup, 112 KB of LDS, one
-  // workgroup per compute unit): the activations are staged for half as many column blocks.  Same sums in the
-  // same order either way.
-  const int nww = wide ? 4 : 2;
+  const int nww = form == 1 ? 4 : 2;
   const int cols = gate_up == 1 ? 32 * nww : 64 * nww;
   const int n_col_blocks = static_cast<int>((n_out + cols - 1) / cols);
   const int64_t full2 = rows2 == 0 ? 0 : (rows2 + TL_ROWS(4) - 1) / TL_ROWS(4) * ((n_out2 + cols - 1) / cols);
@@ -454,24 +465,21 @@ extern "C" int ix_moe_grouped_tiled(const void* a, const void* w, void* out, con
   dim3 grid(static_cast<unsigned>(groups)), block(TL_THREADS(nww));
   const uintptr_t second = rows2 == 0 ? 0 : reinterpret_cast<uintptr_t>(a2) | reinterpret_cast<uintptr_t>(w2);
   const bool direct = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w) | second) & 15) == 0;
-#define LAUNCH(GU, NWW, DIRECT)                                                                                     \
-  hipLaunchKernelGGL((moe_grouped_tiled_kernel<GU, NWW, DIRECT>), grid, block, 0, stream, (const __bf16*)a,         \
+#define LAUNCH(GU, NWW, ALL, DIRECT)                                                                                     \
+  hipLaunchKernelGGL((moe_grouped_tiled_kernel<GU, NWW, ALL, DIRECT>), grid, block, 0, stream, (const __bf16*)a,         \
                      (const __bf16*)w, (__bf16*)out, offsets, rows, tile_expert, tile_row0, tile_info, (int)n_out,  \
                      (int)width, n_col_blocks, gate_up == 2 ? 1 : 0, glu_limit, std::min(last_tiles, max_tiles), last_each,         \
                      (Second{(const __bf16*)a2, (const __bf16*)w2, (__bf16*)out2, (int)rows2, (int)n_out2, (int)width2}))
-#define FORM(GU, NWW)                 \
-  if (direct) LAUNCH(GU, NWW, true);  \
-  else LAUNCH(GU, NWW, false)
-  if (nww == 4) {
-    if (gate_up == 1) {
-      FORM(true, 4);
-    } else {
-      FORM(false, 4);
-    }
-  } else if (gate_up == 1) {
-    FORM(true, 2);
+#define FORM(GU)                                       \
+  if (form == 1 && direct) LAUNCH(GU, 4, true, true);  \
+  else if (form == 1) LAUNCH(GU, 4, true, false);      \
+  else if (!direct) LAUNCH(GU, 2, false, false);       \
+  else if (form == 2) LAUNCH(GU, 2, true, true);       \
+  else LAUNCH(GU, 2, false, true)
+  if (gate_up == 1) {
+    FORM(true);
   } else {
-    FORM(false, 2);
+    FORM(false);
   }
 #undef FORM
 #undef LAUNCH

@@ -786,6 +786,7 @@ def _linear_skinny(x, w, out, gate_up, glu_limit, bias, out_f32: bool = False) -
 MOE_TILED_F32_ROWS = 64  # rows per tile of the LDS-staged grouped product in float32
 MOE_TILED_ROWS = 160  # rows per tile of the LDS-staged grouped product
 MOE_TILED_ROWS_WIDE = 192  # ... of its wide form
+MOE_TILED_ALONE = 240  # workgroups up to which a narrow one takes a compute unit's LDS: some less than there are units, as the number is estimated
 
 
 def moe_tiled_rows(wide: bool) -> int:
@@ -832,9 +833,11 @@ def moe_grouped_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offse
         _need(a2.dtype == w2.dtype == out2.dtype == torch.bfloat16, "the matrix-core grouped product is bfloat16 only")
         _need(a2.shape == (rows2, width2) and w2.shape == ((2 if _epilogue(gate_up) == GATE_UP_SWIGLU else 1) * n_out2, width2),
               "the second product's shapes do not fit")
+    few = not wide and moe_tiled_workgroups(A, E, n_out, _epilogue(gate_up) == GATE_UP_SWIGLU) <= MOE_TILED_ALONE
+    form = 1 if wide else 2 if few else 0  # (2: narrow, a workgroup a compute unit)
     _call("ix_moe_grouped_tiled", _ptr(a), _ptr(w), _ptr(out), _ptr(offsets), _ptr(rows), _ptr(tile_map[:mt]),
           _ptr(tile_map[mt:2 * mt]), _ptr(tile_map[2 * mt:]), _i32(mt), _i64(a.shape[0]), _i64(n_out), _i64(K),
-          _i32(_epilogue(gate_up)), _i32(1 if wide else 0), _f32(glu_limit), _i32(last_tiles), _i32(last_each),
+          _i32(_epilogue(gate_up)), _i32(form), _f32(glu_limit), _i32(last_tiles), _i32(last_each),
           _ptr(a2), _ptr(w2), _ptr(out2), _i64(rows2), _i64(n_out2), _i64(width2), _stream())
 
 

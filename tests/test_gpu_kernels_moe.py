@@ -341,6 +341,33 @@ def test_grouped_tiled_rings_of_every_depth(H, wide):
     assert all(torch.equal(out[0].view(torch.int16), o.view(torch.int16)) for o in out[1:])
 
 
+@pytest.mark.parametrize("gate_up", [False, True])
+@pytest.mark.parametrize("H", [8, 64, 72, 128, 192, 256, 264, 320, 384, 448, 512, 584, 1024])
+def test_grouped_tiled_of_few_and_many_workgroups(H, gate_up):
+    """The narrow form with all of a compute unit's LDS, and with half where (further, empty) experts make many workgroups: float64's
+    results, and the same bits.  Tiles of all heights, one to sixteen stages through rings of two to six buffers."""
+    from inferx_amd import ops
+    R, mi = ops.moe_tiled_rows(False), 136
+    counts = [1, 33, 70, 128, 129, R, R + 40]
+    E, T = len(counts), sum(counts)
+    topk_e = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).to(torch.int32)[:, None].to(DEV)
+    x = rnd(T, H, dtype=torch.bfloat16)
+    few = rnd(E, (2 if gate_up else 1) * mi, H, seed=2, dtype=torch.bfloat16, scale=H ** -0.5)
+    many = torch.cat([few, torch.full((300 - E,) + few.shape[1:], float("nan"), dtype=torch.bfloat16, device=DEV)])
+    out = []
+    for w in (few, many):
+        assert (ops.moe_tiled_workgroups(T, w.shape[0], mi, gate_up) <= ops.MOE_TILED_ALONE) == (w is few)
+        offsets, rows, dest, tile_map = dispatch(topk_e, w.shape[0], R)
+        out.append(torch.full((T, mi), float("nan"), dtype=torch.bfloat16, device=DEV))
+        ops.moe_grouped_tiled(x, w, out[-1], offsets, rows, tile_map, gate_up)
+    z = torch.cat([x[rows.long()][lo:hi].double() @ few[e].double().T
+                   for e, (lo, hi) in enumerate(zip(offsets.tolist()[:E], offsets.tolist()[1:E + 1]))])
+    want = torch.nn.functional.silu(z[:, :mi]) * z[:, mi:] if gate_up else z
+    # one rounding of the result and float32 sums of H products
+    assert float((out[0].double() - want).abs().max()) <= 2 ** -8 * float(want.abs().max()) + 1e-5
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+
+
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("last", [1, 3, 7, 8, 1000])
 def test_grouped_tiled_order_of_the_last_tiles(last, wide):

@@ -35,6 +35,6 @@ def kernels(tmp_path):
 @pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
 def test_the_products_kernels_keep_everything_in_registers(tmp_path):
     scratch = kernels(tmp_path)
-    of = {n: b for n, b in scratch.items() if re.search("moe_grouped_tiled|moe_grouped_mfma|moe_grouped_dual|linear_skinny|qkv_rope_skinny|heads_product", n)}
+    of = {n: b for n, b in scratch.items() if re.search("linear_tiled|moe_grouped_tiled|moe_grouped_mfma|moe_grouped_dual|linear_skinny|qkv_rope_skinny|heads_product", n)}
     assert len(of) > 40
     assert not any(of.values()), {n: b for n, b in of.items() if b}

@@ -268,6 +268,17 @@ static int tile_for(int64_t rows, int64_t n_out, int64_t width) {
   return tile;
 }
 
+// (a lane's place in its block of weights, and in the activations, is counted in 32 bits of bytes)
+static bool small_enough(int64_t rows, int64_t n_out, int64_t width) {
+  return rows * width < (int64_t(1) << 31) && 256 * width < (int64_t(1) << 31) && n_out < (int64_t(1) << 31) - 512;
+}
+
+// The rule's tile for a product, 0 to 8, or -1.
+extern "C" int ix_linear_tiled_tile(int64_t rows, int64_t n_out, int64_t width) {
+  if (rows <= 0 || n_out <= 0 || width <= 0 || width % 8 != 0 || !small_enough(rows, n_out, width)) return -1;
+  return tile_for(rows, n_out, width);
+}
+
 // Operands on 16-byte boundaries.  tile: 0 to 8 that one, -1 the rule chooses; then 2 is returned, and nothing queued, where it has
 // no tile for the product.
 extern "C" int ix_linear_tiled(const void* x, const void* w, void* out, int64_t rows, int64_t n_out, int64_t width,
@@ -275,13 +286,11 @@ extern "C" int ix_linear_tiled(const void* x, const void* w, void* out, int64_t 
   IX_REQUIRE(rows > 0 && n_out > 0 && width > 0, "sizes must be positive");
   IX_REQUIRE(width % 8 == 0, "the reduction width must be a multiple of 8");
   IX_REQUIRE(((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0, "operands must lie on 16-byte boundaries");
-  // (a lane's place in its block of weights, and in the activations, is counted in 32 bits of bytes)
-  const bool small = rows * width < (int64_t(1) << 31) && 256 * width < (int64_t(1) << 31) && n_out < (int64_t(1) << 31) - 512;
   if (tile < 0) {
-    tile = small ? tile_for(rows, n_out, width) : -1;
+    tile = ix_linear_tiled_tile(rows, n_out, width);
     if (tile < 0) return 2;
   }
-  IX_REQUIRE(small, "sizes too large");
+  IX_REQUIRE(small_enough(rows, n_out, width), "sizes too large");
   switch (tile) {
     case 0: return linear_tiled<Tile0>(x, w, out, rows, n_out, width, out_f32, stream);
     case 1: return linear_tiled<Tile1>(x, w, out, rows, n_out, width, out_f32, stream);

@@ -123,9 +123,12 @@ class Runtime:
                 and x.shape[1] > 0 and x.shape[1] % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0):
             return None
         from .. import ops
+        tile = ops.linear_tiled_tile(rows, features, x.shape[1])
+        if tile < 0:  # (asked first: nothing is allocated for a product that goes elsewhere)
+            return None
         if out is None:
             out = self.empty((rows, features), out_dtype)
-        return out if ops.linear_tiled(x, w, out) else None
+        return out if ops.linear_tiled(x, w, out, tile) else None
 
     def linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """x [T, in] . w[out, in]^T -> [T, out] in the run's type, float32 accumulation.

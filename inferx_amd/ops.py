@@ -737,6 +737,14 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> bool:
     return True
 
 
+def linear_tiled_tile(rows: int, features: int, width: int) -> int:
+    """The tile that `linear_tiled`'s rule chooses for a product, or -1 where it has none."""
+    fn = _functions.get("ix_linear_tiled_tile")
+    if fn is None:
+        fn = _functions["ix_linear_tiled_tile"] = lib().ix_linear_tiled_tile
+    return fn(rows, features, width)
+
+
 def linear_tiled(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, tile: int = -1) -> bool:
     """out [T, N] = x [T, K] . w[N, K]^T, bfloat16 operands on 16-byte boundaries, 32-bit accumulation, out bfloat16 or float32,
     for a few dozen to some hundred rows.  False where the kernel's rule has no tile for the product (nothing was queued then);

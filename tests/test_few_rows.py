@@ -82,6 +82,22 @@ def test_wide_expert_products_take_many_workgroups(experts, top, width, shared, 
     assert part._wide(tokens) and part._tile_rows(SimpleNamespace(rt=SimpleNamespace(SKINNY_ROWS=32)), x) == ops.moe_tiled_rows(wide)
 
 
+def test_products_that_tiles_do_not_take_are_allocated_once(monkeypatch):
+    from inferx_amd import ops
+    rt = Runtime.__new__(Runtime)
+    made = []
+    monkeypatch.setattr(rt, "empty", lambda shape, dtype=None: made.append(shape) or torch.empty(shape, dtype=dtype or torch.bfloat16), raising=False)
+    monkeypatch.setattr(ops, "gemm_bf16", lambda x, w, out: True)
+    monkeypatch.setattr(ops, "linear_tiled", lambda x, w, out, tile=-1: tile >= 0)
+    for rows, tiled in ((2048, False), (40, True)):
+        x, w = torch.zeros(rows, 2048, dtype=torch.bfloat16), torch.zeros(6144, 2048, dtype=torch.bfloat16)
+        assert (ops.linear_tiled_tile(rows, 6144, 2048) >= 0) == tiled
+        for product in (rt.linear, rt.linear_f32):
+            made.clear()
+            product(x, w)
+            assert made == [(rows, 6144)]
+
+
 @pytest.mark.parametrize("units,longest,span,head_dim,slices,loads", [
     (16, 517, 0, 128, 16, 1), (16, 65, 0, 128, 1, 1), (4, 128, 0, 128, 1, 1), (4, 129, 0, 128, 4, 1),   # one request
     (4, 64, 0, 128, 1, 2), (32, 40, 0, 128, 1, 2), (33, 40, 0, 128, 1, 1), (2048, 64, 0, 128, 1, 2), (2048, 65, 0, 128, 1, 1),

@@ -257,7 +257,7 @@ using TileN = LinearTile<2, 2, 4, 2, 3>;   // 128 x 64, two workgroups a compute
 //   Up to 128 tiles of 32 x 32 with a long reduction: the library cuts it (5,120 to 22,000: 1.05; 663 x 15,872 x 24 38 against 16
 // us, 66 x 8,704 x 192 21.7 against 10.7, 37 x 7,680 x 192 18.6 against 9.9; up to 5,120 0.7, of more tiles 0.8).
 //   Results of no whole fours a row, which are stored one by one: from 64 x 96 on 0.99 (780 x 480 x 6,355 21.8 against 16.9).
-//   64 x 128 with more than 4,096 of reduction where a fifth of the units have none (640 x 5,632 x 2,304, 180 tiles, 33.1 against 29.9;
+//   64 x 128 with more than 4,096 of reduction where a fifth of the units have none (180 of them at 640 x 5,632 x 2,304 33.1 against 29.9;
 // 818 x 5,632 x 2,048, 224 tiles, 31.0 against 32.4), 128 x 128 and 128 x 192 from 2,048 of reduction on (850 x 3,584 x 3,584 39.8 against
 // 38.1; 682 x 3,584 x 4,608, 216 tiles, 37.4 against 43.5).  96 x 128 and larger also where many stages follow, which are long enough for the
 // library to be ahead (1,400 x 5,632 x 2,048 55.7 against 52.1), or up to three (3,000 x 64 x 700 11.3 against 10.3; 1,500 x 512 x

@@ -354,6 +354,11 @@ extern "C" int ix_moe_route(const void* x, int dtype, const void* wr, int wr_dty
 #define DW_THREADS 1024
 #define DW_WAVES (DW_THREADS / 64)
 #define DW_ROUNDS 8
+// MANY: both sweeps ask for eight assignments a thread before they look at the first, one trip to memory for all of them.  From 4,096
+// assignments on; up to there the places that nobody needs cost more: us with / without, 512 assignments 5.2 / 4.9, 2,048 5.7 /
+// 5.3, 4,096 6.0 / 5.8, 8,192 7.0 / 7.3, 16,384 10.6 / 11.9.
+#define DW_MANY 4096
+template <bool MANY>
 __global__ void __launch_bounds__(DW_THREADS)
 moe_dispatch_wide_kernel(const int32_t* __restrict__ topk_e, int32_t* __restrict__ offsets,
                          int32_t* __restrict__ rows, int32_t* __restrict__ dest, int64_t assignments, int experts,
@@ -366,15 +371,16 @@ moe_dispatch_wide_kernel(const int32_t* __restrict__ topk_e, int32_t* __restrict
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int i = tid; i < experts; i += DW_THREADS) counts[i] = 0;
   __syncthreads();
-  for (int64_t a0 = tid; a0 < assignments; a0 += DW_ROUNDS * DW_THREADS) {
-    int v[DW_ROUNDS];  // (all asked for before the first is counted: a trip to memory for eight of them)
+  constexpr int AHEAD = MANY ? DW_ROUNDS : 1;
+  for (int64_t a0 = tid; a0 < assignments; a0 += AHEAD * DW_THREADS) {
+    int v[AHEAD];
 #pragma unroll
-    for (int r = 0; r < DW_ROUNDS; ++r) {
+    for (int r = 0; r < AHEAD; ++r) {
       const int64_t a = a0 + r * DW_THREADS;
       v[r] = a < assignments ? topk_e[a] : -1;
     }
 #pragma unroll
-    for (int r = 0; r < DW_ROUNDS; ++r)
+    for (int r = 0; r < AHEAD; ++r)
       if (v[r] >= 0 && v[r] < experts) atomicAdd(&counts[v[r]], 1);
   }
   __syncthreads();
@@ -423,14 +429,16 @@ moe_dispatch_wide_kernel(const int32_t* __restrict__ topk_e, int32_t* __restrict
     uint64_t match[DW_ROUNDS];
     int found = 0;
     int v[DW_ROUNDS];
+    if constexpr (MANY)
+#pragma unroll
+      for (int r = 0; r < DW_ROUNDS; ++r) {
+        const int64_t a = a0 + 64 * r;
+        v[r] = a < assignments ? topk_e[a] : -1;
+      }
 #pragma unroll
     for (int r = 0; r < DW_ROUNDS; ++r) {
       const int64_t a = a0 + 64 * r;
-      v[r] = a < assignments ? topk_e[a] : -1;
-    }
-#pragma unroll
-    for (int r = 0; r < DW_ROUNDS; ++r) {
-      match[r] = __ballot(v[r] == e);
+      match[r] = __ballot(MANY ? v[r] == e : a < assignments && topk_e[a] == e);
       found += __popcll(match[r]);
     }
     if (lane == 0) wave_count[wave] = found;
@@ -466,8 +474,9 @@ extern "C" int ix_moe_dispatch(const int32_t* topk_e, int32_t* offsets, int32_t*
   IX_REQUIRE(experts > 0 && experts <= IX_MAX_EXPERTS, "number of experts must be between 1 and 1024");
   IX_REQUIRE(tile_rows >= 0, "tile_rows must not be negative");
   IX_REQUIRE(tile_rows == 0 || (tile_expert && tile_row0 && tile_info), "tile map buffers needed");
-  hipLaunchKernelGGL(moe_dispatch_wide_kernel, dim3(experts), dim3(DW_THREADS), 0, stream, topk_e, offsets, rows, dest,
-                     assignments, experts, k, tile_rows, tile_expert, tile_row0, tile_info);
+  hipLaunchKernelGGL(assignments > DW_MANY ? moe_dispatch_wide_kernel<true> : moe_dispatch_wide_kernel<false>, dim3(experts),
+                     dim3(DW_THREADS), 0, stream, topk_e, offsets, rows, dest, assignments, experts, k, tile_rows, tile_expert,
+                     tile_row0, tile_info);
   return ix_check_launch("ix_moe_dispatch");
 }
 

@@ -134,6 +134,18 @@ def test_dispatch_is_a_stable_bijection(T, E, k, tile_rows):
         assert covered == list(range(A))  # tiles cover every row once, in order
 
 
+@pytest.mark.parametrize("A", [1, 1024, 1025, 4095, 4096, 4097, 8192, 8193, 20000])
+@pytest.mark.parametrize("E", [1, 5, 600])
+def test_dispatch_of_few_and_many_assignments(A, E):
+    """Around the sizes at which the kernel's sweeps end and change their form."""
+    topk_e = torch.randint(0, E, (A, 1), generator=torch.Generator().manual_seed(A)).to(torch.int32)
+    offsets, rows, dest, _ = dispatch(topk_e.to(DEV), E)
+    order = torch.sort(topk_e.flatten(), stable=True).indices
+    counts = torch.bincount(topk_e.flatten(), minlength=E)
+    assert torch.equal(offsets.cpu(), torch.cat([torch.zeros(1), counts.cumsum(0)]).to(torch.int32))
+    assert torch.equal(rows.cpu().long(), order) and torch.equal(dest.cpu().long()[order], torch.arange(A))
+
+
 @pytest.mark.parametrize("T,H,E,k,renorm,tile_rows", [(1, 64, 4, 2, False, 16), (8, 2048, 60, 4, False, 16),
                                                        (11, 96, 8, 3, True, 32), (16, 72, 5, 1, False, 0),
                                                        (16, 200, 256, 32, True, 16), (16, 136, 60, 4, True, 16),

@@ -36,7 +36,8 @@ template <int WI_, int XI_, int WB_, int XB_, int RING_> struct LinearTile {
   static_assert(WAVES % 2 == 0 && W % (8 * WAVES) == 0 && X % (8 * WAVES) == 0, "whole loads for every wavefront");
 };
 
-// NT: the weights are read by one row tile only, past the caches.
+// NT: the weights are read by one row tile only and their rows are whole lines: past the caches.  (Rows that share lines would bring those
+// from memory for each of them: tiles of 128 x 64 with a reduction that is not made of whole lines 0.94 of the time through the caches.)
 template <typename T, bool NT, bool F32>
 __global__ void __launch_bounds__(64 * T::WAVES) __attribute__((amdgpu_waves_per_eu(1, 2)))
 linear_tiled_kernel(const __bf16* x, const __bf16* w, void* out, int rows, int n_out, int width, int row_tiles) {
@@ -226,7 +227,7 @@ int linear_tiled(const void* x, const void* w, void* out, int64_t rows, int64_t 
 #define LAUNCH(NT, F)                                                                                                    \
   hipLaunchKernelGGL((linear_tiled_kernel<T, NT, F>), dim3(static_cast<unsigned>(tiles)), dim3(64 * T::WAVES), 0, stream, \
                      (const __bf16*)x, (const __bf16*)w, out, (int)rows, (int)n_out, (int)width, (int)row_tiles)
-  if (row_tiles == 1) {
+  if (row_tiles == 1 && width % LT_K == 0 && (reinterpret_cast<uintptr_t>(w) & 127) == 0) {  // (whole lines)
     if (out_f32) LAUNCH(true, true);
     else LAUNCH(true, false);
   } else {
@@ -262,8 +263,6 @@ using TileN = LinearTile<2, 2, 4, 2, 3>;   // 128 x 64, two workgroups a compute
 // 38.1; 682 x 3,584 x 4,608, 216 tiles, 37.4 against 43.5).  96 x 128 and larger also where many stages follow, which are long enough for the
 // library to be ahead (1,400 x 5,632 x 2,048 55.7 against 52.1), or up to three (3,000 x 64 x 700 11.3 against 10.3; 1,500 x 512 x
 // 2,048 11.4 against 14.6).
-//   128 x 64 of more than 32 rows with a reduction from 2,048 on that is not made of whole stages 1.02 (46 x 3,752 x 43,637 106
-// against 97.5; of whole stages 0.92, up to 32 rows 0.7).
 static int tile_for(int64_t rows, int64_t n_out, int64_t width) {
   const int64_t tiles[8] = {tiles_of<Tile0>(rows, n_out), tiles_of<Tile1>(rows, n_out), tiles_of<Tile2>(rows, n_out),
                             tiles_of<Tile3>(rows, n_out), tiles_of<Tile4>(rows, n_out), tiles_of<Tile5>(rows, n_out),
@@ -271,7 +270,7 @@ static int tile_for(int64_t rows, int64_t n_out, int64_t width) {
   int tile = 0;
   while (tile < 8 && tiles[tile] > LT_UNITS) ++tile;
   if (tile == 0 && width > 5120 && 2 * tiles[0] <= LT_UNITS) return -1;
-  if (tile > 4 && rows <= TileN::X) return rows > 32 && width >= 2048 && width % LT_K != 0 ? -1 : 8;
+  if (tile > 4 && rows <= TileN::X) return 8;
   if (tile > 2 && n_out % 4 != 0) return -1;
   if (tile == 8 || (tile > 4 && (width > 4096 || width < 256))) return -1;
   if (5 * tiles[tile] < 4 * LT_UNITS && ((tile == 4 && width > 4096) || (tile > 5 && width > 2048))) return -1;

@@ -43,7 +43,9 @@
 //
 // An expert with one tile has its weights read once: past the caches (non-temporal, whole lines; a plain read of memory gives
 // 7.0 TB/s that way and 6.1 through them).  2,048 rows unevenly over 60 experts 254 against 268 us for both products.  Weights
-// that several tiles read stay cached (2,048 rows 289 us past the caches).  Results go through LDS, so that a store is 16
+// that several tiles read stay cached (2,048 rows 289 us past the caches), and so do those whose rows are no whole lines: rows and stages
+// share some, which would come from memory for each of them (128 experts of 656 on 2,920, 513 tokens of four, both products 361 us past the
+// caches, 315 through them).  Results go through LDS, so that a store is 16
 // bytes a lane of whole lines and not 8 of sixteen rows.
 //
 // Where experts have more rows than a tile, each of an expert's row tiles would ask for all its weights again, a column
@@ -407,7 +409,8 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
       col_block = static_cast<int>(in / n_here);
       row0 = tile_row0[tile];
     }
-    once = DIRECT && row_end - first_row <= TL_ROWS(NWW);
+    // (rows that are no whole lines share some, which would come from memory for each of them)
+    once = DIRECT && row_end - first_row <= TL_ROWS(NWW) && ((width & 63) | static_cast<int>(reinterpret_cast<uintptr_t>(w) & 127)) == 0;
   }
   const int held = min(TL_ROWS(NWW), row_end - row0);
   if (held <= 0) return;

@@ -9,7 +9,8 @@
 // ring of three to six LDS buffers that the loads fill by themselves, with one barrier a stage, as in moe_tiled.hip; half a
 // compute unit's LDS, so that two workgroups share one and one's products overlap with the other's waits.  Rows of LDS keep
 // their eight 16-byte pieces permuted (piece p of row r at p ^ ((r >> 1) & 7)), so that sixteen rows read at one piece fall on
-// different banks.  The weights of an expert with one tile go past the caches.
+// different banks.  The weights of an expert with one tile go past the caches if their rows are whole lines (42 experts of 2,048 on 2,308, 193
+// tokens of two, gate|up 333 us past them, 269 through them, as rows and stages share lines).
 //
 // A lane reads four consecutive numbers of its row at a time; product j of a piece multiplies the j-th of them, so the
 // four slots of the reduction that one matrix instruction adds up are the pieces' j-th numbers, the same in both
@@ -265,7 +266,8 @@ moe_grouped_tiled_f32_kernel(const float* a, const float* w, float* out, const i
   const int e = tile_expert[tile], row0 = tile_row0[tile], row_end = offsets[e + 1];
   const int held = min(TF_ROWS, row_end - row0);
   if (held <= 0) return;
-  const bool once = held == row_end - offsets[e];  // an expert's only tile: its weights are read once, past the caches
+  // an expert's only tile: its weights are read once, past the caches, if its rows are whole lines
+  const bool once = held == row_end - offsets[e] && ((width & 31) | static_cast<int>(reinterpret_cast<uintptr_t>(w) & 127)) == 0;
 #define CALL(NT, ONCE) \
   tiled_f32_body<GATE_UP, NT, ONCE, BLOCKS>(a, w, out, rows, n_out, width, e, row0, row_end, col_block, lds, act, glu_limit)
 #define BODY(NT) if (once) CALL(NT, true); else CALL(NT, false)

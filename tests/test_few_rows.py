@@ -105,8 +105,8 @@ def test_products_that_tiles_do_not_take_are_allocated_once(monkeypatch):
     # results of no whole fours a row from 64 x 96 on; longer reductions in 64 x 128 for few units; what was left to the library before
     (240, 3510, 480, 2), (240, 5118, 480, -1), (240, 5120, 480, 3), (780, 6355, 480, -1), (500, 3840, 4104, 4), (640, 2400, 4096, 4), (640, 2400, 4104, -1),
     (500, 3838, 4096, -1), (3000, 700, 64, -1), (3000, 700, 256, 5), (850, 3584, 3584, -1), (2048, 6144, 2048, -1),
-    # up to 64 rows that do not fit otherwise: more than 32 of them with stages that are not whole
-    (33, 151936, 2048, 8), (46, 43637, 2056, -1), (46, 43637, 2040, 8), (32, 43637, 2056, 8), (64, 151936, 20480, 8),
+    # up to 64 rows that do not fit otherwise
+    (33, 151936, 2048, 8), (46, 43637, 2056, 8), (64, 151936, 20480, 8), (65, 151936, 2048, -1),
     # sizes that the kernel does not take
     (40, 512, 100, -1), (0, 512, 64, -1), (1 << 20, 64, 4096, -1), (40, 1 << 31, 64, -1)])
 def test_tiles_of_dense_products(rows, features, width, tile):

@@ -22,6 +22,8 @@
 // products.  Which of them, by the workgroups that two would give, the sizes' geometric mean of one product's time (509 shapes of 4 to
 // 128 experts, widths of 512 to 2,560, 40 to 1,024 tokens), two blocks against one: up to 128 1.78, 256 1.38, 512 1.21, 768
 // 1.08, 1,024 1.06, 1,500 1.03, more 0.99 (8 experts of 768 on 2,048, 128 tokens, both products: 116 us, 68 with one).
+// With reductions of 256, 512 and 768 the three stages more that two turned blocks walk weigh too much, so they stay with one (128
+// experts of 256, down to 2,560, 74 tokens of six, 57 us with two blocks, 49 with one; eight of 512 on 512, 1,105 tokens 125 and 109).
 //
 // Measured with 60 experts of 1,408 on a width of 2,048, 4 a token, unevenly routed, both products, us, two blocks against pieces through
 // registers and LDS writes, one block, a die's run of tiles in their order: 170 tokens 389 -> 348, 361 503 -> 415, 511 562
@@ -37,6 +39,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define TF_ROWS 64     // rows of a tile of the map
 #define TF_K 32        // numbers of the reduction per stage
 #define TF_APART 3     // stages between the starts of neighbouring blocks of 64 weight rows
+#define TF_TURNED_WIDTH 1024
 #define TF_LDS 81920   // bytes: half a compute unit's
 __device__ __forceinline__ int tf_at(int row, int piece) { return row * TF_K + ((piece ^ ((row >> 1) & 7)) << 2); }
 
@@ -302,7 +305,8 @@ extern "C" int ix_moe_grouped_tiled_f32(const float* a, const float* w, float* o
     const int cols = (gate_up == 1 ? 32 : 64) * blocks;
     return (n_out + cols - 1) / cols;
   };
-  const int blocks = column_blocks(2) * max_tiles <= 1024 ? 1 : 2;  // (see the top of the file)
+  // (see the top of the file; with short reductions the three stages more that two turned blocks walk weigh too much)
+  const int blocks = column_blocks(2) * max_tiles <= 1024 || (width % 256 == 0 && width < TF_TURNED_WIDTH) ? 1 : 2;
   const int n_col_blocks = static_cast<int>(column_blocks(blocks));
   const int64_t groups = static_cast<int64_t>(n_col_blocks) * max_tiles;
   IX_REQUIRE(groups < (int64_t(1) << 31), "too many workgroups for one launch");

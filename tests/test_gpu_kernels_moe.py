@@ -777,10 +777,10 @@ def test_grouped_tiled_in_float32_worked_by_their_rows(counts, K):
 
 
 @pytest.mark.parametrize("gate_up", [0, 1, 2])
-@pytest.mark.parametrize("K", [4, 32, 68, 96, 128, 160, 196, 256, 512])
+@pytest.mark.parametrize("K", [4, 32, 68, 96, 128, 160, 196, 256, 512, 1024, 1280])
 def test_grouped_tiled_in_float32_of_few_and_many_workgroups(K, gate_up):
     """One block of weight rows a workgroup, and two where (further, empty) experts make many workgroups: float64's results, and the
-    same bits.  Tiles of all heights, one to sixteen stages through rings of three to six buffers, columns past the last block."""
+    same bits.  Tiles of all heights, one to forty stages through rings of three to six buffers, columns past the last block."""
     from inferx_amd import ops
     counts, T, n = [5, 64, 17, 1, 0, 40, 33, 130], 70, 388  # (four blocks of 128 and more: 52 workgroups at least, 1,160)
     E, A = len(counts), sum(counts)

@@ -69,7 +69,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define TL_STRIDE 64  // elements per LDS row: no padding; the eight 16-byte pieces of a row are stored permuted
 #define TL_LDS(ALL) ((ALL) ? 163840 : 81920)  // bytes: all of a compute unit's, or half
 // piece p of row r lies at piece p ^ ((r >> 1) & 7): the sixteen rows that a quarter of a wavefront reads at one
-// piece index then fall on sixteen different groups of four banks, as do the pieces that sixteen lanes write
+// piece index then fall on sixteen different groups of four banks
 __device__ __forceinline__ int tl_at(int row, int piece) { return row * TL_STRIDE + ((piece ^ ((row >> 1) & 7)) << 3); }
 
 // 16 bytes a lane from base + offset to lds + dst + 16 lane, straight or, from anywhere, through registers.

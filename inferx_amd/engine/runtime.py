@@ -110,8 +110,8 @@ class Runtime:
         return out
 
     # From 17 rows on a product of so many features goes in tiles.  17 / 32 rows of 2,048 and more, us, few-row kernel / tiles: 6,144
-    # features 12.8 / 10.4 and 16.0 / 11.4, 11,264 17.2 / 14.0 and 21.7 / 14.4, 151,936 in float32 113 / 106 and 152 / 117; 2,048 8.8 / 9.6
-    # and 10.4 / 10.0, 3,584 12.8 / 13.0 and 15.0 / 13.9.
+    # features 12.8 / 10.4 and 16.0 / 11.4, 151,936 in float32 113 / 106 and 152 / 117; 2,048 8.8 / 9.6 and 10.4 / 10.0, 3,584 12.8 / 13.0
+    # and 15.0 / 13.9.  (Gate|up products of so many rows stay with the few-row kernel, which forms the unit as well.)
     TILED_FEATURES = 4096
 
     def _tiled(self, x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype,

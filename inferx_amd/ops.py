@@ -794,17 +794,20 @@ def _linear_skinny(x, w, out, gate_up, glu_limit, bias, out_f32: bool = False) -
 MOE_TILED_F32_ROWS = 64  # rows per tile of the LDS-staged grouped product in float32
 MOE_TILED_ROWS = 160  # rows per tile of the LDS-staged grouped product
 MOE_TILED_ROWS_WIDE = 192  # ... of its wide form
-MOE_TILED_ALONE = 240  # workgroups up to which a narrow one takes a compute unit's LDS: some less than there are units, as the number is estimated
+# Workgroups up to which a narrow one takes all of a compute unit's LDS: as many as there are units.  Of more some wait for a place: 12
+# tiles, 264 and 192 workgroups, took 85 us for both products where half of it for each takes 66.
+MOE_TILED_ALONE = 256
 
 
 def moe_tiled_rows(wide: bool) -> int:
     return MOE_TILED_ROWS_WIDE if wide else MOE_TILED_ROWS
 
 
-def moe_tiled_workgroups(assignments: int, experts: int, n_out: int, gate_up: bool) -> float:
-    """About how many workgroups a narrow LDS-staged grouped product has: an expert's last tile is half full on average, and one
-    with a row has a tile."""
-    tiles = max(min(experts, assignments), assignments / MOE_TILED_ROWS + experts / 2)
+def moe_tiled_workgroups(assignments: int, experts: int, n_out: int, gate_up: bool, at_most: bool = False) -> float:
+    """About how many workgroups a narrow LDS-staged grouped product has: an expert with a row has a tile, and its last one is half
+    empty on average.  `at_most`: so many as unevenly routed rows seldom exceed."""
+    rows = assignments / MOE_TILED_ROWS
+    tiles = max(min(experts, assignments), 1.25 * rows + 0.55 * experts if at_most else rows + experts / 2)
     return tiles * -(-n_out // (64 if gate_up else 128))
 
 
@@ -841,7 +844,7 @@ def moe_grouped_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offse
         _need(a2.dtype == w2.dtype == out2.dtype == torch.bfloat16, "the matrix-core grouped product is bfloat16 only")
         _need(a2.shape == (rows2, width2) and w2.shape == ((2 if _epilogue(gate_up) == GATE_UP_SWIGLU else 1) * n_out2, width2),
               "the second product's shapes do not fit")
-    few = not wide and moe_tiled_workgroups(A, E, n_out, _epilogue(gate_up) == GATE_UP_SWIGLU) <= MOE_TILED_ALONE
+    few = not wide and moe_tiled_workgroups(A, E, n_out, _epilogue(gate_up) == GATE_UP_SWIGLU, at_most=True) <= MOE_TILED_ALONE
     form = 1 if wide else 2 if few else 0  # (2: narrow, a workgroup a compute unit)
     _call("ix_moe_grouped_tiled", _ptr(a), _ptr(w), _ptr(out), _ptr(offsets), _ptr(rows), _ptr(tile_map[:mt]),
           _ptr(tile_map[mt:2 * mt]), _ptr(tile_map[2 * mt:]), _i32(mt), _i64(a.shape[0]), _i64(n_out), _i64(K),

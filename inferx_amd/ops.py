@@ -803,12 +803,16 @@ def moe_tiled_rows(wide: bool) -> int:
     return MOE_TILED_ROWS_WIDE if wide else MOE_TILED_ROWS
 
 
-def moe_tiled_workgroups(assignments: int, experts: int, n_out: int, gate_up: bool, at_most: bool = False) -> float:
-    """About how many workgroups a narrow LDS-staged grouped product has: an expert with a row has a tile, and its last one is half
+def moe_tiled_tiles(assignments: int, experts: int, at_most: bool = False) -> float:
+    """About how many row tiles a narrow LDS-staged grouped product has: an expert with a row has a tile, and its last one is half
     empty on average.  `at_most`: so many as unevenly routed rows seldom exceed."""
     rows = assignments / MOE_TILED_ROWS
-    tiles = max(min(experts, assignments), 1.25 * rows + 0.55 * experts if at_most else rows + experts / 2)
-    return tiles * -(-n_out // (64 if gate_up else 128))
+    return max(min(experts, assignments), 1.25 * rows + 0.55 * experts if at_most else rows + experts / 2)
+
+
+def moe_tiled_columns(n_out: int, gate_up: bool) -> int:
+    """How many workgroups a row tile of a narrow LDS-staged grouped product has."""
+    return -(-n_out // (64 if gate_up else 128))
 
 
 def moe_grouped_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offsets: torch.Tensor,
@@ -844,7 +848,8 @@ def moe_grouped_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offse
         _need(a2.dtype == w2.dtype == out2.dtype == torch.bfloat16, "the matrix-core grouped product is bfloat16 only")
         _need(a2.shape == (rows2, width2) and w2.shape == ((2 if _epilogue(gate_up) == GATE_UP_SWIGLU else 1) * n_out2, width2),
               "the second product's shapes do not fit")
-    few = not wide and moe_tiled_workgroups(A, E, n_out, _epilogue(gate_up) == GATE_UP_SWIGLU, at_most=True) <= MOE_TILED_ALONE
+    few = not wide and (moe_tiled_tiles(A, E, at_most=True) * moe_tiled_columns(n_out, _epilogue(gate_up) == GATE_UP_SWIGLU)
+                         <= MOE_TILED_ALONE)
     form = 1 if wide else 2 if few else 0  # (2: narrow, a workgroup a compute unit)
     _call("ix_moe_grouped_tiled", _ptr(a), _ptr(w), _ptr(out), _ptr(offsets), _ptr(rows), _ptr(tile_map[:mt]),
           _ptr(tile_map[mt:2 * mt]), _ptr(tile_map[2 * mt:]), _i32(mt), _i64(a.shape[0]), _i64(n_out), _i64(K),

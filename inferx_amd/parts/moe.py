@@ -43,11 +43,13 @@ WIDE_TILES_WIDTH = 3072
 # 191, 1,024 207 / 208, 2,048 272 / 247, 4,096 403 / 379; with the shared expert among them 64 tokens 170 / 166, 340 208 / 208, 768
 # 255 / 234, 1,500 322 / 317, 2,048 412 / 380.
 WIDE_TILES_ALONE_WIDTH = 2048
-# ... and where both products of the narrow form would have so many workgroups: the wide form has half as many, each with twice the
-# work.  Wide against narrow, geometric means over 791 shapes of 4 to 128 experts of 160 to 2,048 on widths of 2,048 and more: up to
-# 512 workgroups 1.32, 1,024 1.11, 1,536 1.06, 2,048 1.06, beyond with 32 rows a tile and more 0.98, with fewer 1.05 (eight experts
-# of 768 on 2,048, 203 tokens of six, both products: 53 against 62 us).
+# ... and where both products of the narrow form would have so many workgroups, as the wide form has half as many, each with twice the
+# work, and, without a shared expert's full tiles among them, so many rows a tile on average.  Wide against narrow, geometric means over 791
+# shapes of 4 to 128 experts of 160 to 2,048 on widths of 2,048 and more: up to 512 workgroups 1.32, 1,024 1.11, 1,536 1.06, 2,048 1.06
+# (eight experts of 768 on 2,048, 203 tokens of six, both products: 53 against 62 us), beyond without a shared expert with less than 32
+# rows a tile 1.07, with more 0.99, with one 1.03 and 0.98 (64 tokens of 60 experts of 1,408, 8 layers, 2,574 us narrow, 2,541 wide).
 WIDE_TILES_ALONE_WORKGROUPS = 2048
+WIDE_TILES_ALONE_ROWS = 32
 # Between the few rows of a decoding step (where routed and shared experts already share a launch) and the portions
 # from which the shared expert's library products run beside the routed experts, the shared expert is cut into
 # pieces of the routed experts' width, which every token "chooses" with the shared gate's value as their weight:
@@ -194,14 +196,16 @@ class MoeFeedForward(FeedForward):
             return 16
         if x.dtype == torch.float32:
             return ops.MOE_TILED_F32_ROWS
-        wide = self.wide_tiles or (self._wide(x.shape[0]) and self._workgroups(x.shape[0]) >= WIDE_TILES_ALONE_WORKGROUPS)
+        wide = self.wide_tiles or (self._wide(x.shape[0]) and self._enough_for_wide(x.shape[0]))
         return ops.moe_tiled_rows(wide)
 
-    def _workgroups(self, tokens: int) -> float:
-        """About how many workgroups both LDS-staged products have in their narrow form, the shared expert's pieces among them."""
-        A, E = tokens * (self.top_k + self.shared_pieces), self.num_experts + self.shared_pieces
-        return (ops.moe_tiled_workgroups(A, E, self.expert_width, self.gated)
-                + ops.moe_tiled_workgroups(A, E, self.hidden_size, False))
+    def _enough_for_wide(self, tokens: int) -> bool:
+        """Whether the LDS-staged products have the workgroups and the rows for their wide form, the shared expert's pieces among them."""
+        rows = tokens * (self.top_k + self.shared_pieces)
+        tiles = ops.moe_tiled_tiles(rows, self.num_experts + self.shared_pieces)
+        columns = ops.moe_tiled_columns(self.expert_width, self.gated) + ops.moe_tiled_columns(self.hidden_size, False)
+        return tiles * columns >= WIDE_TILES_ALONE_WORKGROUPS and (
+            self.shared_pieces > 0 or rows >= WIDE_TILES_ALONE_ROWS * tiles)
 
     def _wide(self, tokens: int) -> bool:
         """Whether the width lets the LDS-staged products of this step take their wide form."""

@@ -69,10 +69,11 @@ def test_wide_expert_products(hidden, shared, tokens, wide):
 
 
 @pytest.mark.parametrize("experts,top,width,shared,tokens,wide", [
-    (60, 4, 1408, 5632, 64, True), (60, 4, 1408, 0, 64, True), (60, 4, 1408, 5632, 2112, True), (8, 6, 768, 0, 203, False),
-    (8, 2, 1408, 1408, 1500, False), (8, 2, 2816, 0, 9000, True), (128, 8, 768, 0, 60, True)])
-def test_wide_expert_products_take_many_workgroups(experts, top, width, shared, tokens, wide):
-    """At a width of 2,048 the narrow form stays where the wide one would leave compute units without work."""
+    (60, 4, 1408, 5632, 64, True), (60, 4, 1408, 5632, 255, True), (60, 4, 1408, 0, 479, False),
+    (60, 4, 1408, 0, 480, True), (60, 4, 1408, 5632, 2112, True), (8, 6, 768, 0, 203, False), (8, 2, 1408, 1408, 1500, False),
+    (8, 2, 2816, 0, 9000, True), (128, 8, 768, 0, 60, False)])
+def test_wide_expert_products_take_many_workgroups_and_rows(experts, top, width, shared, tokens, wide):
+    """At a width of 2,048 the narrow form stays where the wide one would leave compute units without work, or waits for weights."""
     from types import SimpleNamespace
     from inferx_amd import ops
     from inferx_amd.parts.moe import MoeFeedForward

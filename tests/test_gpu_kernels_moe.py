@@ -368,7 +368,7 @@ def test_grouped_tiled_of_few_and_many_workgroups(H, gate_up):
     many = torch.cat([few, torch.full((300 - E,) + few.shape[1:], float("nan"), dtype=torch.bfloat16, device=DEV)])
     out = []
     for w in (few, many):
-        assert (ops.moe_tiled_workgroups(T, w.shape[0], mi, gate_up, at_most=True) <= ops.MOE_TILED_ALONE) == (w is few)
+        assert (ops.moe_tiled_tiles(T, w.shape[0], at_most=True) * ops.moe_tiled_columns(mi, gate_up) <= ops.MOE_TILED_ALONE) == (w is few)
         offsets, rows, dest, tile_map = dispatch(topk_e, w.shape[0], R)
         out.append(torch.full((T, mi), float("nan"), dtype=torch.bfloat16, device=DEV))
         ops.moe_grouped_tiled(x, w, out[-1], offsets, rows, tile_map, gate_up)

@@ -354,10 +354,10 @@ extern "C" int ix_moe_route(const void* x, int dtype, const void* wr, int wr_dty
 #define DW_THREADS 1024
 #define DW_WAVES (DW_THREADS / 64)
 #define DW_ROUNDS 8
-// MANY: both sweeps ask for eight assignments a thread before they look at the first, one trip to memory for all of them.  From 4,096
-// assignments on; up to there the places that nobody needs cost more: us with / without, 512 assignments 5.2 / 4.9, 2,048 5.7 /
-// 5.3, 4,096 6.0 / 5.8, 8,192 7.0 / 7.3, 16,384 10.6 / 11.9.
-#define DW_MANY 4096
+// MANY: both sweeps ask for eight assignments a thread before they look at the first, one trip to memory for all of them.  From more
+// than one a thread on; up to there the places that nobody needs cost more.  In a step, us with / without: 512 assignments 5.5 / 5.4, 2,044
+// 6.6 / 6.9; over and over on the same assignments, which are near then, 512 5.2 / 4.9, 4,096 6.0 / 5.8, 8,192 7.0 / 7.3, 16,384 10.6 / 11.9.
+#define DW_MANY DW_THREADS
 template <bool MANY>
 __global__ void __launch_bounds__(DW_THREADS)
 moe_dispatch_wide_kernel(const int32_t* __restrict__ topk_e, int32_t* __restrict__ offsets,

@@ -27,6 +27,11 @@ __device__ __forceinline__ void lds_load16(void* lds, unsigned dst, const void* 
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(from) : "memory", "m0");
 }
+// 4 bytes a lane to lds + dst + 4 * lane.
+__device__ __forceinline__ void lds_load4(void* lds, unsigned dst, unsigned offset, const void* base) {
+  const unsigned at = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds)) + dst;
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(at), "v"(offset), "s"(base) : "memory", "m0");
+}
 // Until at most N of this wavefront's loads are on their way.
 template <int N>
 __device__ __forceinline__ void wait_loads() {

@@ -363,10 +363,11 @@ __global__ void __launch_bounds__(DW_THREADS)
 moe_dispatch_wide_kernel(const int32_t* __restrict__ topk_e, int32_t* __restrict__ offsets,
                          int32_t* __restrict__ rows, int32_t* __restrict__ dest, int64_t assignments, int experts,
                          int k, int tile_rows, int32_t* __restrict__ tile_expert, int32_t* __restrict__ tile_row0,
-                         int32_t* __restrict__ tile_info) {
+                         int32_t* __restrict__ tile_info, int32_t* __restrict__ queues, int n_queues,
+                         int2* __restrict__ tiles) {
   __shared__ int32_t counts[IX_MAX_EXPERTS];
   __shared__ int32_t wave_count[DW_WAVES];
-  __shared__ int32_t part[2][DW_WAVES];
+  __shared__ int32_t part[4][DW_WAVES];
   const int e = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int i = tid; i < experts; i += DW_THREADS) counts[i] = 0;
@@ -384,41 +385,55 @@ moe_dispatch_wide_kernel(const int32_t* __restrict__ topk_e, int32_t* __restrict
       if (v[r] >= 0 && v[r] < experts) atomicAdd(&counts[v[r]], 1);
   }
   __syncthreads();
-  int rows_before = 0, tiles_before = 0;
-  for (int i = tid; i < e; i += DW_THREADS) {
-    const int c = counts[i];
-    rows_before += c;
-    tiles_before += tile_rows > 0 ? (c + tile_rows - 1) / tile_rows : 0;
+  int rows_before = 0, tiles_before = 0, heavy = 0, all = 0;
+  const int mine = counts[e];
+  for (int i = tid; i < experts; i += DW_THREADS) {
+    const int c = counts[i], tiles = tile_rows > 0 ? (c + tile_rows - 1) / tile_rows : 0;
+    rows_before += i < e ? c : 0;
+    tiles_before += (n_queues > 0 ? c > mine || (c == mine && i < e) : i < e) ? tiles : 0;
+    heavy += c > 128 ? tiles : 0;
+    all += tiles;
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     rows_before += __shfl_xor(rows_before, off, 64);
     tiles_before += __shfl_xor(tiles_before, off, 64);
+    heavy += __shfl_xor(heavy, off, 64);
+    all += __shfl_xor(all, off, 64);
   }
   if (lane == 0) {
     part[0][wave] = rows_before;
     part[1][wave] = tiles_before;
+    part[2][wave] = heavy;
+    part[3][wave] = all;
   }
   __syncthreads();
-  rows_before = tiles_before = 0;
+  rows_before = tiles_before = heavy = all = 0;
 #pragma unroll
   for (int w = 0; w < DW_WAVES; ++w) {
     rows_before += part[0][w];
     tiles_before += part[1][w];
+    heavy += part[2][w];
+    all += part[3][w];
   }
-  const int mine = counts[e];
   const int my_tiles = tile_rows > 0 ? (mine + tile_rows - 1) / tile_rows : 0;
+  if (e == 0 && tid < n_queues) queues[tid] = tid % 9 == 8 ? heavy : 0;
   if (tid == 0) {
     offsets[e] = rows_before;
     if (e == experts - 1) {
       offsets[experts] = rows_before + mine;
-      if (tile_info) tile_info[0] = tiles_before + my_tiles;
+      if (tile_info) tile_info[0] = all;
     }
   }
   if (tile_expert)
     for (int i = tid; i < my_tiles; i += DW_THREADS) {
       tile_expert[tiles_before + i] = e;
       tile_row0[tiles_before + i] = rows_before + i * tile_rows;
+      if (tiles) {
+        const int held = min(tile_rows, mine - i * tile_rows), together = min(4, my_tiles - (i & ~3));
+        tiles[tiles_before + i] = make_int2(rows_before + i * tile_rows, held | e << 8 | (i & 3) << 19 | (together - 1) << 21 |
+                                                                             (my_tiles == 1 ? 1 << 23 : 0));
+      }
     }
   if (mine == 0) return;  // uniform over the workgroup
 
@@ -467,16 +482,24 @@ moe_dispatch_wide_kernel(const int32_t* __restrict__ topk_e, int32_t* __restrict
 }
 
 // tile_expert / tile_row0 need room for min(A, ceil(A / tile_rows) + E) entries; tile_rows 0 skips the map.
+// queues (n_queues, or 0): for so many products that follow by workgroups that stay (moe_tiled_queue.hip), eight zeros and the number of
+// tiles of experts with more than 128 rows each; the map then lists the experts with most rows first, and behind the queues, on a boundary
+// of eight bytes, the same tiles follow as those products want them: first row; rows held (8 bits, so at most 255 a tile), expert (11),
+// its number (2) in a group of up to four (2: less one) tiles of the expert that read the same weights, whether the only one (1).
 extern "C" int ix_moe_dispatch(const int32_t* topk_e, int32_t* offsets, int32_t* rows, int32_t* dest,
                                int64_t assignments, int experts, int k, int tile_rows, int32_t* tile_expert,
-                               int32_t* tile_row0, int32_t* tile_info, hipStream_t stream) {
+                               int32_t* tile_row0, int32_t* tile_info, int32_t* queues, int n_queues, hipStream_t stream) {
   IX_REQUIRE(assignments >= 0 && k > 0, "sizes must be positive");
+  IX_REQUIRE(n_queues >= 0 && n_queues <= 16 && (n_queues == 0 || (queues && tile_rows > 0 && tile_rows < 256 &&
+                                                                  (reinterpret_cast<uintptr_t>(queues) & 7) == 0)),
+             "queues go with a map of tiles of up to 255 rows and lie on a boundary of eight bytes");
   IX_REQUIRE(experts > 0 && experts <= IX_MAX_EXPERTS, "number of experts must be between 1 and 1024");
   IX_REQUIRE(tile_rows >= 0, "tile_rows must not be negative");
   IX_REQUIRE(tile_rows == 0 || (tile_expert && tile_row0 && tile_info), "tile map buffers needed");
   hipLaunchKernelGGL(assignments > DW_MANY ? moe_dispatch_wide_kernel<true> : moe_dispatch_wide_kernel<false>, dim3(experts),
                      dim3(DW_THREADS), 0, stream, topk_e, offsets, rows, dest, assignments, experts, k, tile_rows, tile_expert,
-                     tile_row0, tile_info);
+                     tile_row0, tile_info, queues, 9 * n_queues,
+                     n_queues ? reinterpret_cast<int2*>(queues + (9 * n_queues + 1) / 2 * 2) : nullptr);
   return ix_check_launch("ix_moe_dispatch");
 }
 

@@ -54,23 +54,9 @@
 // Operands that do not lie on 16-byte boundaries (`DIRECT` false) go through registers, one piece after the other.
 #include <type_traits>
 
-#include "lds_loads.h"
+#include "moe_tiled.h"
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// the row-tile map is made for tiles of this many rows (the wide form's hold 192)
-#define TL_ROWS(NWW) ((NWW) == 2 ? 160 : 192)
-#define TL_K 64
-// NWW: wavefronts along the weight rows (2 or 4; two along the activation rows): 64 NWW weight rows and 128 NWW
-// threads per workgroup.  With four, a row tile's activations are read for half as many column blocks.
-#define TL_THREADS(NWW) (128 * (NWW))
-#define TL_STRIDE 64  // elements per LDS row: no padding; the eight 16-byte pieces of a row are stored permuted
 #define TL_LDS(ALL) ((ALL) ? 163840 : 81920)  // bytes: all of a compute unit's, or half
-// piece p of row r lies at piece p ^ ((r >> 1) & 7): the sixteen rows that a quarter of a wavefront reads at one
-// piece index then fall on sixteen different groups of four banks
-__device__ __forceinline__ int tl_at(int row, int piece) { return row * TL_STRIDE + ((piece ^ ((row >> 1) & 7)) << 3); }
 
 // 16 bytes a lane from base + offset to lds + dst + 16 lane, straight or, from anywhere, through registers.
 template <bool NT, bool DIRECT>
@@ -323,14 +309,6 @@ tiled_body(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restr
   }
 }
 
-// A second product of the launch: out [rows, n_out] = a [rows, width] . w^T, one set of weights for all rows (with gate|up the two
-// sets of n_out rows).  rows 0: none.
-struct Second {
-  const __bf16 *a, *w;
-  __bf16* out;
-  int rows, n_out, width;
-};
-
 template <bool GATE_UP, int NWW, bool ALL, bool DIRECT>
 __global__ void __launch_bounds__(TL_THREADS(NWW)) __attribute__((amdgpu_waves_per_eu(2, 2)))
 moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const int32_t* __restrict__ offsets,
@@ -339,79 +317,17 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
                          const int32_t* __restrict__ tile_info, int n_out, int width, int n_col_blocks,
                          int act, float glu_limit, int last_tiles, int last_each, Second second) {
   __shared__ __attribute__((aligned(1024))) __bf16 lds[TL_LDS(ALL) / 2];
-  // Workgroups go to the chip's eight dies in turn, by their number, and each die has its own L2 and its own share of the
-  // memory's bandwidth.  The (row tile, column block) pairs, tile by tile, are cut into eight equal runs, one a die, so that
-  // the column blocks of a tile, which read the same activations, share an L2 and no die has more of them than another.
-  // The last `last_tiles` row tiles are those of experts that every token uses (the shared expert's pieces): full tiles,
-  // bound by the matrix cores, where the others hold few rows and wait for their weights.  They are cut by themselves, and
-  // a die works them spread evenly among its others, so that at any time some workgroups multiply while the rest keep
-  // the memory busy: `last_each` tiles of one expert together for a column block, as they read the same weights, and two
-  // column blocks a run.  Both products, us, with runs of one block, two, four and all of a tile's: 64 experts of 2,560, rows of
-  // 3,584, beside eight of every row: 512 rows 810, 827, 832, 852, 682 rows 897, 902, 909, 906; 60 of 1,408, rows of 2,048,
-  // beside four: 100 rows 180, 174, 172, 172, 340 rows 209, 208, 208, 212.  (Whole tiles dealt to the dies in turn: some
-  // had a tile more, 163 against 103 us at one expert of 2,048 rows, wide.)
-  const int n_tiles = tile_info[0];
-  const unsigned die = blockIdx.x & 7, i = blockIdx.x >> 3;
-  // A second product's tiles are worked as the last ones: as many row tiles of one expert.
-  const bool two = NWW == 4 && second.rows > 0, spread = !two && last_tiles > 0 && last_tiles < n_tiles;
-  constexpr int COLS = (GATE_UP ? 32 : 64) * NWW;
-  if (two) last_each = (second.rows + TL_ROWS(NWW) - 1) / TL_ROWS(NWW);
-  const int n_light = spread ? n_tiles - last_tiles : n_tiles;
-  const unsigned light = static_cast<unsigned>(n_light) * n_col_blocks;
-  const unsigned full = two ? static_cast<unsigned>(last_each) * ((second.n_out + COLS - 1) / COLS)
-                            : spread ? static_cast<unsigned>(last_tiles) * n_col_blocks : 0u;
-  auto cut = [&](unsigned n, unsigned d) { return static_cast<unsigned>(static_cast<uint64_t>(n) * d >> 3); };
-  const unsigned light0 = cut(light, die), full0 = cut(full, die);
-  const unsigned n_full = cut(full, die + 1) - full0, n_mine = cut(light, die + 1) - light0 + n_full;
-  if (i >= n_mine) return;
-  bool is_full = false;
-  unsigned pair = light0 + i;
-  if (two && second.width > width) {
-    // longer ones first: they then end with the others (88 of 88 stages beside some 600 of 22, of 256 places)
-    is_full = i < n_full;
-    pair = is_full ? light + full0 + i : light0 + i - n_full;
-  } else if (n_full > 0) {
-    const unsigned run = 2u * last_each, runs = (n_full + run - 1) / run, period = max(n_mine / runs, run);
-    const unsigned r = i / period, off = i % period;  // run r starts at place r * period
-    const unsigned len = r < runs ? min(run, n_full - r * run) : 0;
-    is_full = off < len;
-    pair = is_full ? light + full0 + r * run + off : light0 + i - (r < runs ? r * run + len : n_full);
-  }
-  int e = 0, row0, row_end, col_block;
-  bool once = false;  // an expert's only tile
-  if (two && is_full) {
-    const int at = static_cast<int>(pair - light);
-    row0 = TL_ROWS(NWW) * (at % last_each);
-    col_block = at / last_each;
-    row_end = second.rows;
+  const TileList<GATE_UP, NWW> list(blockIdx.x & 7, offsets, tile_expert, tile_row0, tile_info, n_col_blocks, width, last_tiles,
+                                    last_each, second);
+  const unsigned i = blockIdx.x >> 3;
+  if (i >= list.n) return;
+  const auto p = list.pair(i);
+  const int e = p.e, row0 = p.row0, row_end = p.row_end, col_block = p.col_block;
+  // An expert's only tile.  (Rows that are no whole lines share some, which would come from memory for each of them.)
+  const bool once = DIRECT && !p.second && row_end - p.first_row <= TL_ROWS(NWW) &&
+                    ((width & 63) | static_cast<int>(reinterpret_cast<uintptr_t>(w) & 127)) == 0;
+  if (p.second)
     a = second.a, w = second.w, out = second.out, rows = nullptr, n_out = second.n_out, width = second.width, act = 0;
-  } else {
-    int tile = static_cast<int>(pair / n_col_blocks);
-    col_block = static_cast<int>(pair % n_col_blocks);
-    if (is_full && last_each > 1) {  // (the row tiles of an expert one after the other for a column block)
-      const unsigned at = pair - light, per = static_cast<unsigned>(last_each) * n_col_blocks, in = at % per;
-      tile = n_tiles - last_tiles + static_cast<int>(at / per * last_each + in % last_each);
-      col_block = static_cast<int>(in / last_each);
-    }
-    e = tile_expert[tile];
-    row0 = tile_row0[tile];
-    row_end = offsets[e + 1];
-    const int first_row = offsets[e];
-    if (!is_full && row_end - first_row > TL_ROWS(NWW)) {
-      // Row tiles of an expert that has several read the same weights: up to four of them one after the other for a column
-      // block, so that all but the first find the weights in L2.  (Tiles of the expert that are among the last ones have
-      // been dealt out above.)
-      const int nth = (row0 - first_row) / TL_ROWS(NWW), first = tile - (nth & 3);
-      const int of_expert = (row_end - first_row + TL_ROWS(NWW) - 1) / TL_ROWS(NWW) - (nth & ~3);
-      const unsigned n_here = min(min(4, of_expert), n_light - first);
-      const unsigned in = pair - static_cast<unsigned>(first) * n_col_blocks;
-      tile = first + static_cast<int>(in % n_here);
-      col_block = static_cast<int>(in / n_here);
-      row0 = tile_row0[tile];
-    }
-    // (rows that are no whole lines share some, which would come from memory for each of them)
-    once = DIRECT && row_end - first_row <= TL_ROWS(NWW) && ((width & 63) | static_cast<int>(reinterpret_cast<uintptr_t>(w) & 127)) == 0;
-  }
   const int held = min(TL_ROWS(NWW), row_end - row0);
   if (held <= 0) return;
 #define CALL(NP, ONCE) \
@@ -437,13 +353,18 @@ moe_grouped_tiled_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
 // glu_limit > 0: the gate|up rows meet in the clamped form (`ix_glu`).  last_tiles: so many tiles at the end of the
 // map are worked spread among the others; `last_each` consecutive ones of them belong to one expert.  a2, w2, out2 (rows2 0: none, and
 // with the wide form only): a product of its own in the same launch, out2 [rows2, n_out2] = a2 [rows2, width2] . w2^T, gate|up
-// as the grouped one; no last tiles then.
+// as the grouped one; no last tiles then.  queue (or null): eight counters that hold 0, and the number of tiles of experts with more
+// than 128 rows, which the map lists first; with them and the tiles as `ix_moe_dispatch` leaves them behind its queues the wide form may
+// be worked by workgroups that stay (moe_tiled_queue.hip).
+int ix_moe_grouped_queue(const void* a, const void* w, void* out, const int32_t* rows, const int32_t* tile_info, const void* tiles,
+                         int32_t* queue, int max_tiles, int64_t n_out, int64_t width, int gate_up, float glu_limit, const void* a2,
+                         const void* w2, void* out2, int64_t rows2, int64_t n_out2, int64_t width2, hipStream_t stream);
 extern "C" int ix_moe_grouped_tiled(const void* a, const void* w, void* out, const int32_t* offsets,
                                     const int32_t* rows, const int32_t* tile_expert, const int32_t* tile_row0,
                                     const int32_t* tile_info, int max_tiles, int64_t a_rows, int64_t n_out,
                                     int64_t width, int gate_up, int form, float glu_limit, int last_tiles, int last_each,
                                     const void* a2, const void* w2, void* out2, int64_t rows2, int64_t n_out2,
-                                    int64_t width2, hipStream_t stream) {
+                                    int64_t width2, int32_t* queue, const void* tiles, hipStream_t stream) {
   IX_REQUIRE(n_out > 0 && width > 0 && max_tiles >= 0 && last_tiles >= 0 && last_each > 0, "sizes must be positive");
   IX_REQUIRE(last_tiles % last_each == 0, "the last tiles come in equal groups");
   IX_REQUIRE(width % 8 == 0, "the reduction width must be a multiple of 8 for the matrix-core kernel");
@@ -465,6 +386,11 @@ extern "C" int ix_moe_grouped_tiled(const void* a, const void* w, void* out, con
   const int64_t full2 = rows2 == 0 ? 0 : (rows2 + TL_ROWS(4) - 1) / TL_ROWS(4) * ((n_out2 + cols - 1) / cols);
   const int64_t groups = 8 * ((static_cast<int64_t>(n_col_blocks) * max_tiles + full2) / 8 + 2);  // (a die has at most this many pairs)
   IX_REQUIRE(groups < (int64_t(1) << 31), "too many workgroups for one launch");
+  if (form == 1 && queue && tiles) {
+    const int rc = ix_moe_grouped_queue(a, w, out, rows, tile_info, tiles, queue, max_tiles, n_out, width, gate_up, glu_limit, a2, w2,
+                                        out2, rows2, n_out2, width2, stream);
+    if (rc != 2) return rc;
+  }
   dim3 grid(static_cast<unsigned>(groups)), block(TL_THREADS(nww));
   const uintptr_t second = rows2 == 0 ? 0 : reinterpret_cast<uintptr_t>(a2) | reinterpret_cast<uintptr_t>(w2);
   const bool direct = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w) | second) & 15) == 0;

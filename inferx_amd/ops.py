@@ -611,16 +611,22 @@ def moe_route_dispatch(x: Optional[torch.Tensor], router_w: torch.Tensor, shared
 
 
 def moe_dispatch(topk_e: torch.Tensor, offsets: torch.Tensor, rows: torch.Tensor, dest: torch.Tensor,
-                 experts: int, tile_rows: int = 0, tile_map: Optional[torch.Tensor] = None) -> None:
+                 experts: int, tile_rows: int = 0, tile_map: Optional[torch.Tensor] = None,
+                 queues: Optional[torch.Tensor] = None) -> None:
     """Group assignments by expert: offsets [E+1], rows [A] (grouped row -> token), dest [A].
     With tile_rows > 0 also the row-tile map for the matrix-core product: `tile_map` int32
-    [2 * max_tiles + 1] = tile_expert | tile_row0 | number of tiles, max_tiles = moe_max_tiles(A, E, tile_rows)."""
+    [2 * max_tiles + 1] = tile_expert | tile_row0 | number of tiles, max_tiles = moe_max_tiles(A, E, tile_rows).
+    `queues`: int32 on an 8-byte boundary, `moe_queues_size(max_tiles)` of them, for the two `moe_grouped_tiled` in the wide form
+    that follow; the map then lists the experts with most rows first."""
     T, k = topk_e.shape
     A = T * k
     _is_i32(topk_e)
     _is_i32(offsets, experts + 1)
     _is_i32(rows, A)
     _is_i32(dest, A)
+    if queues is not None:
+        _need(tile_rows > 0, "queues go with a tile map")
+        _is_i32(queues, moe_queues_size(moe_max_tiles(A, experts, tile_rows)))
     te = tr = ti = None
     if tile_rows > 0:
         mt = moe_max_tiles(A, experts, tile_rows)
@@ -628,7 +634,7 @@ def moe_dispatch(topk_e: torch.Tensor, offsets: torch.Tensor, rows: torch.Tensor
         _is_i32(tile_map, 2 * mt + 1)
         te, tr, ti = tile_map[:mt], tile_map[mt:2 * mt], tile_map[2 * mt:]
     _call("ix_moe_dispatch", _ptr(topk_e), _ptr(offsets), _ptr(rows), _ptr(dest), _i64(A), _i32(experts), _i32(k),
-          _i32(tile_rows), _ptr(te), _ptr(tr), _ptr(ti), _stream())
+          _i32(tile_rows), _ptr(te), _ptr(tr), _ptr(ti), _ptr(queues), _i32(2 if queues is not None else 0), _stream())
 
 
 PLAIN_PRODUCT, GATE_UP_SWIGLU, RELU_SQUARED = 0, 1, 2
@@ -794,9 +800,20 @@ def _linear_skinny(x, w, out, gate_up, glu_limit, bias, out_f32: bool = False) -
 MOE_TILED_F32_ROWS = 64  # rows per tile of the LDS-staged grouped product in float32
 MOE_TILED_ROWS = 160  # rows per tile of the LDS-staged grouped product
 MOE_TILED_ROWS_WIDE = 192  # ... of its wide form
+# What the workgroups of two wide products take their work by: nine numbers each (eight counters and a number of tiles), then two numbers a tile
+MOE_QUEUE = 9
+
+
+def moe_queues_size(max_tiles: int) -> int:
+    return 2 * MOE_QUEUE + 2 * max_tiles
+
+
 # Workgroups up to which a narrow one takes all of a compute unit's LDS: as many as there are units.  Of more some wait for a place: 12
 # tiles, 264 and 192 workgroups, took 85 us for both products where half of it for each takes 66.
 MOE_TILED_ALONE = 256
+
+
+MOE_QUEUE_TILES, MOE_QUEUE_PAIRS = 768, 1536  # the tiles, and the longest list of a die's pairs, that a staying workgroup keeps
 
 
 def moe_tiled_rows(wide: bool) -> int:
@@ -810,6 +827,17 @@ def moe_tiled_tiles(assignments: int, experts: int, at_most: bool = False) -> fl
     return max(min(experts, assignments), 1.25 * rows + 0.55 * experts if at_most else rows + experts / 2)
 
 
+def moe_stays(assignments: int, experts: int, hidden: int, width: int, rows2: int = 0, width2: int = 0) -> bool:
+    """Whether both wide products of `experts` of so many assignments, rows of `hidden`, width `width` (and a second pair of products on
+    `rows2` rows, width `width2`) can be worked by workgroups that stay: whole stages of 64, four at least, and no longer a list than
+    a workgroup keeps."""
+    sizes = (hidden, width) + ((width2,) if rows2 else ())
+    tiles = moe_max_tiles(assignments, experts, MOE_TILED_ROWS_WIDE)
+    pairs = max(tiles * -(-width // 128) + -(-rows2 // MOE_TILED_ROWS_WIDE) * -(-width2 // 128),
+                (tiles + -(-rows2 // MOE_TILED_ROWS_WIDE)) * -(-hidden // 256))
+    return all(n % 64 == 0 and n >= 256 for n in sizes) and tiles <= MOE_QUEUE_TILES and pairs // 8 + 19 <= MOE_QUEUE_PAIRS
+
+
 def moe_tiled_columns(n_out: int, gate_up: bool) -> int:
     """How many workgroups a row tile of a narrow LDS-staged grouped product has."""
     return -(-n_out // (64 if gate_up else 128))
@@ -818,13 +846,16 @@ def moe_tiled_columns(n_out: int, gate_up: bool) -> int:
 def moe_grouped_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offsets: torch.Tensor,
                       rows: Optional[torch.Tensor], tile_map: torch.Tensor, gate_up: bool, wide: bool = False,
                       glu_limit: float = 0.0, last_tiles: int = 0, last_each: int = 1,
-                      second: Optional[Tuple[torch.Tensor, torch.Tensor, torch.Tensor]] = None) -> None:
+                      second: Optional[Tuple[torch.Tensor, torch.Tensor, torch.Tensor]] = None,
+                      queues: Optional[torch.Tensor] = None, nth: int = 0) -> None:
     """Grouped product staged through LDS (bfloat16, many rows per expert); `tile_map` made for tiles of
     `moe_tiled_rows(wide)` rows.  `wide`: 256 instead of 128 weight rows per workgroup (the same sums in the same
     order).  `last_tiles`: so many tiles at the end of the map are worked spread among the others, `last_each`
     consecutive ones of them belong to one expert (any number gives the same results).  `second`: (a, w, out) of a dense
     product out [T, n] = a [T, k] . w^T (gate|up like the grouped one, w then [2 n, k]) in the same launch, with the wide
-    form and without last tiles."""
+    form and without last tiles.  `queues`: what `moe_dispatch` made; with
+    them the wide form's workgroups stay and take one tile after the other (the same results).  `nth`: 0 or 1, whether the
+    first or the second product with them (each once)."""
     E = w.shape[0]
     A, n_out = out.shape
     K = a.shape[1]
@@ -848,13 +879,18 @@ def moe_grouped_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offse
         _need(a2.dtype == w2.dtype == out2.dtype == torch.bfloat16, "the matrix-core grouped product is bfloat16 only")
         _need(a2.shape == (rows2, width2) and w2.shape == ((2 if _epilogue(gate_up) == GATE_UP_SWIGLU else 1) * n_out2, width2),
               "the second product's shapes do not fit")
+    queue = tiles = None
+    if queues is not None:
+        _need(nth in (0, 1), "the queues are for two products")
+        _is_i32(queues, moe_queues_size(mt))
+        queue, tiles = queues[nth * MOE_QUEUE:], queues[2 * MOE_QUEUE:]
     few = not wide and (moe_tiled_tiles(A, E, at_most=True) * moe_tiled_columns(n_out, _epilogue(gate_up) == GATE_UP_SWIGLU)
                          <= MOE_TILED_ALONE)
     form = 1 if wide else 2 if few else 0  # (2: narrow, a workgroup a compute unit)
     _call("ix_moe_grouped_tiled", _ptr(a), _ptr(w), _ptr(out), _ptr(offsets), _ptr(rows), _ptr(tile_map[:mt]),
           _ptr(tile_map[mt:2 * mt]), _ptr(tile_map[2 * mt:]), _i32(mt), _i64(a.shape[0]), _i64(n_out), _i64(K),
           _i32(_epilogue(gate_up)), _i32(form), _f32(glu_limit), _i32(last_tiles), _i32(last_each),
-          _ptr(a2), _ptr(w2), _ptr(out2), _i64(rows2), _i64(n_out2), _i64(width2), _stream())
+          _ptr(a2), _ptr(w2), _ptr(out2), _i64(rows2), _i64(n_out2), _i64(width2), _ptr(queue), _ptr(tiles), _stream())
 
 
 def moe_grouped_tiled_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offsets: torch.Tensor,

@@ -469,6 +469,74 @@ def test_grouped_tiled_experts_of_several_tiles_beside_the_last_ones(last, wide)
     assert rel_err(out, grouped_reference(x, w, offsets.cpu(), rows.cpu(), False)) < 1e-2
 
 
+def with_queue(topk_e, E):
+    """`dispatch` for the wide form's tiles, most rows first, with a queue."""
+    from inferx_amd import ops
+    A, R = topk_e.numel(), ops.MOE_TILED_ROWS_WIDE
+    offsets, rows, dest = (torch.empty(n, dtype=torch.int32, device=DEV) for n in (E + 1, A, A))
+    tile_map = torch.full((2 * ops.moe_max_tiles(A, E, R) + 1,), -7, dtype=torch.int32, device=DEV)
+    mt = ops.moe_max_tiles(A, E, R)
+    queues = torch.full((ops.moe_queues_size(mt),), -7, dtype=torch.int32, device=DEV)
+    ops.moe_dispatch(topk_e, offsets, rows, dest, E, R, tile_map, queues)
+    counts = (offsets[1:] - offsets[:-1]).tolist()
+    tiles = [(e, i) for e in sorted(range(E), key=lambda e: (-counts[e], e)) for i in range(-(-counts[e] // R))]
+    start = [int(offsets[e]) + R * i for e, i in tiles]
+    assert int(tile_map[2 * mt]) == len(tiles)
+    assert list(zip(tile_map[:len(tiles)].tolist(), tile_map[mt:mt + len(tiles)].tolist())) == [(e, r) for (e, _), r in zip(tiles, start)]
+    heavy = sum(-(-n // R) for n in counts if n > 128)
+    want = ([0] * 8 + [heavy]) * 2
+    for (e, i), r in zip(tiles, start):
+        of = -(-counts[e] // R)
+        want += [r, min(R, counts[e] - R * i) | e << 8 | i % 4 << 19 | min(4, of - i // 4 * 4) - 1 << 21 | (of == 1) << 23]
+    assert queues.tolist() == want + [-7] * (queues.numel() - len(want))
+    return offsets, rows, tile_map, queues
+
+
+@pytest.mark.parametrize("epilogue", [False, True, 2])
+@pytest.mark.parametrize("H,mi,few", [(256, 1544, False), (320, 1544, False), (512, 1536, False), (1024, 520, False), (640, 264, True),
+                                      (192, 1544, False), (264, 1544, False), (256, 1540, False)])
+def test_grouped_tiled_by_workgroups_that_stay(H, mi, few, epilogue):
+    """The bits of a workgroup for each tile: tiles of all heights one after the other on a place (and no more tiles than places),
+    four and more stages, column blocks that are whole and not; the shapes that do not go there leave the queue alone."""
+    from inferx_amd import ops
+    counts = [1, 33, 70, 97, 129, 161, 192, 193, 400, 0, 16, 64] * (1 if few else 3)
+    E, T = len(counts), sum(counts)
+    g = torch.Generator().manual_seed(1)
+    topk_e = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=g)].to(torch.int32)[:, None].to(DEV)
+    offsets, rows, tile_map, queues = with_queue(topk_e, E)
+    x = rnd(T, H, dtype=torch.bfloat16)
+    w = rnd(E, (2 if epilogue == 1 else 1) * mi, H, seed=2, dtype=torch.bfloat16, scale=H ** -0.5)
+    want = torch.full((T, mi), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.moe_grouped_tiled(x, w, want, offsets, rows, tile_map, epilogue, True)
+    assert torch.isfinite(want).all()
+    buf = torch.full((T * mi + 16,), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.moe_grouped_tiled(x, w, buf[8:-8].view(T, mi), offsets, rows, tile_map, epilogue, True, queues=queues, nth=1)
+    assert torch.equal(buf[8:-8].view(T, mi).view(torch.int16), want.view(torch.int16))
+    assert (buf[:8] == 7).all() and (buf[-8:] == 7).all()
+    assert (int(queues[9:17].sum()) > 0) == (H % 64 == 0 and H >= 256 and mi % 8 == 0)
+
+
+@pytest.mark.parametrize("gate_up", [False, True])
+@pytest.mark.parametrize("rows,n,k", [(1, 8, 256), (193, 264, 576), (700, 2000, 2048), (600, 2000, 320), (400, 1000, 192)])
+def test_grouped_tiled_with_a_second_product_by_workgroups_that_stay(rows, n, k, gate_up):
+    """A second product of shorter, equal and longer reductions among the tiles: the bits of both as by a workgroup for each."""
+    from inferx_amd import ops
+    T, E, top, mi, H = 900, 20, 3, 1160, 576
+    g = torch.Generator().manual_seed(1)
+    topk_e = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).to(torch.int32).to(DEV)
+    offsets, order, tile_map, queues = with_queue(topk_e, E)
+    x, a2 = rnd(T, H, dtype=torch.bfloat16), rnd(rows, k, seed=3, dtype=torch.bfloat16)
+    w = rnd(E, (2 if gate_up else 1) * mi, H, seed=2, dtype=torch.bfloat16, scale=H ** -0.5)
+    w2 = rnd((2 if gate_up else 1) * n, k, seed=4, dtype=torch.bfloat16, scale=k ** -0.5)
+    out = [torch.full((T * top, mi), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    out2 = [torch.full((rows, n), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    for i in (0, 1):
+        ops.moe_grouped_tiled(x, w, out[i], offsets, order, tile_map, gate_up, True, second=(a2, w2, out2[i]), queues=queues if i else None)
+    assert (int(queues[:8].sum()) > 0) == (k >= 256)
+    for a, b in (out, out2):
+        assert torch.isfinite(a).all() and torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T", [1, 8, 17, 64])
 # at most 256 blocks of sixteen, and more; at most 128 (both halves of an even reduction in one block for up to eight rows)

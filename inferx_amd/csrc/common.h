@@ -190,8 +190,14 @@ __device__ __forceinline__ float ix_glu(float g, float u, float limit) {
   } else if (limit < 0.f) {
     steep = 1.5957691216057308f * fmaf(0.044715f * g, g, 1.0f);  // 2 sqrt(2 / pi) (1 + 0.044715 g^2)
   }
-  const float e = FAST ? __expf(-steep * g) : expf(-steep * g);
-  return g / (1.0f + e) * u;
+  if constexpr (FAST) {
+    // (A workgroup's 48 results a lane take longer than the matrix cores' last two stages, so their instructions count: the divide
+    // is a reciprocal and one step of Newton's, which leaves it an ulp off at most; the largest exponent keeps that step finite.)
+    const float d = 1.0f + __expf(fminf(-steep * g, 88.0f)), r = __builtin_amdgcn_rcpf(d);
+    return g * __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r) * u;
+  } else {
+    return g / (1.0f + expf(-steep * g)) * u;
+  }
 }
 
 // The first key that a query at position `pos` reads, by how far its attention looks back: `span` 0 every earlier

@@ -102,6 +102,11 @@ class Runtime:
             return x.shape[1] % 4 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0 and w.numel() > 0
         return x.dtype == torch.bfloat16 and x.shape[1] % 8 == 0
 
+    def pairs_ok(self, x: torch.Tensor, w: torch.Tensor) -> bool:
+        """Whether x . w^T may share a launch with another product of as few rows."""
+        from .. import ops
+        return x.dtype == torch.bfloat16 and x.shape[0] <= ops.LINEAR_PAIR_ROWS and self._skinny_ok(x, w)
+
     def _skinny(self, x: torch.Tensor, w: torch.Tensor, gate_up: bool, limit: float = 0.0,
                 bias: Optional[torch.Tensor] = None) -> torch.Tensor:
         from .. import ops

@@ -827,6 +827,27 @@ def _linear_skinny(x, w, out, gate_up, glu_limit, bias, out_f32: bool = False) -
           _f32(glu_limit), _stream())
 
 
+LINEAR_PAIR_ROWS = 16
+
+
+def linear_skinny_pair(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, x2: torch.Tensor, w2: torch.Tensor, out2: torch.Tensor,
+                       gate_up: bool = False, glu_limit: float = 0.0, bias: Optional[torch.Tensor] = None) -> None:
+    """`linear_skinny(x, w, out, gate_up, glu_limit, bias)` and out2 = x2 . w2^T in one launch: bfloat16, up to LINEAR_PAIR_ROWS rows,
+    neither of them reading what the other writes."""
+    T, K = x.shape
+    _need(all(t.dtype == torch.bfloat16 for t in (x, w, out, x2, w2, out2)), "all bfloat16")
+    _need(0 < T <= LINEAR_PAIR_ROWS and x2.shape[0] == T, f"between 1 and {LINEAR_PAIR_ROWS} rows, the same for both")
+    _need_pieces(x)
+    _need_pieces(x2)
+    _need(w.dim() == 2 and w.shape[1] == K and out.shape == (T, w.shape[0] // 2 if gate_up else w.shape[0])
+          and (not gate_up or w.shape[0] % 2 == 0), "shapes do not fit")
+    _need(w2.dim() == 2 and w2.shape[1] == x2.shape[1] and out2.shape == (T, w2.shape[0]), "the second product's shapes do not fit")
+    _need(bias is None or bias.numel() == w.shape[0], "one bias per row of the weights")
+    _call("ix_linear_skinny_pair", _ptr(x), _ptr(w), _ptr(out), _ptr(bias), _i32(_dt(bias) if bias is not None else F32),
+          _i64(out.shape[1]), _i64(K), _i32(1 if gate_up else 0), _f32(glu_limit), _ptr(x2), _ptr(w2), _ptr(out2), _i64(w2.shape[0]),
+          _i64(w2.shape[1]), _i32(T), _stream())
+
+
 MOE_TILED_F32_ROWS = 64  # rows per tile of the LDS-staged grouped product in float32
 MOE_TILED_ROWS = 160  # rows per tile of the LDS-staged grouped product
 MOE_TILED_ROWS_WIDE = 192  # ... of its wide form

@@ -219,6 +219,10 @@ class PositionEncoding(Part):
 
 
 class Mixer(Part):
+    # True: `forward` takes a further argument, `beside`, whose `first(w)` and `last(y, w)` form the mixer's first product (of x) and
+    # its last one in place of `rt.linear` (see `FeedForward.beside`)
+    takes_beside = False
+
     def forward(self, ctx, x, cache):
         """`cache`: the `CacheBinding` of this execution (its arrays of pages, its state), or None if the mixer
         keeps nothing."""
@@ -267,6 +271,11 @@ class FeedForward(Part):
 
     def forward(self, ctx, x):
         raise NotImplementedError
+
+    def beside(self, ctx, x):
+        """This feed-forward, on rows x that a mixer reads too, to be worked in the launches of that mixer's first and last products; or
+        None where it is worked by itself.  Its `result(ctx)` is what `forward` would return."""
+        return None
 
 
 class BranchGain(Part):

@@ -116,6 +116,11 @@ class ParallelBlock(Block):
 
     def forward(self, ctx, h, pending, caches):
         x = self.norm.forward(ctx, h, pending)
+        # (in a step of few rows the feed-forward's products may share the launches of the mixer's first and last)
+        beside = self.feed_forward.beside(ctx, x) if self.mixer.takes_beside and self.feed_forward is not None else None
+        if beside is not None:
+            a = self.mixer.forward(ctx, x, caches.get("mixer"), beside)
+            return BranchSum(a, beside.result(ctx))
         a = self.mixer.forward(ctx, x, caches.get("mixer"))
         if self.feed_forward is None:
             return a

@@ -68,9 +68,58 @@ class DenseMlp(FeedForward):
     def forward(self, ctx, x):
         """The result without the last product's bias: whoever adds the result to the stream adds `out_bias()` with
         it (`BiasedDelta`), so that the bias costs no pass of its own."""
-        rt = ctx.rt
-        y = rt.linear(rt.gated_linear(x, self.w_gate_up, self.form, self.b_gate_up), self.w_down)
+        y = self.down(ctx, self.activated(ctx, x))
         return y if self.b_down is None else BiasedDelta(y, self.b_down)
+
+    def activated(self, ctx, x):
+        return ctx.rt.gated_linear(x, self.w_gate_up, self.form, self.b_gate_up)
+
+    def down(self, ctx, act):
+        return ctx.rt.linear(act, self.w_down)
+
+
+    def beside(self, ctx, x):
+        """In a step of few rows: this feed-forward as the companion of a mixer that reads the same rows, or None."""
+        rt = ctx.rt
+        if x.dtype != torch.bfloat16 or not (rt.pairs_ok(x, self.w_gate_up) and self.w_down.dtype == x.dtype and self.width % 8 == 0):
+            return None
+        return Beside(rt, self, x)
+
+
+class Beside:
+    """A dense feed-forward worked in the launches of a mixer that reads the same rows: its first product with the mixer's `first`,
+    its second with the mixer's `last`, which do not need each other.  For steps of few rows, where every launch counts; the same
+    results as one after the other."""
+
+    def __init__(self, rt, mlp, x):
+        self.rt, self.mlp, self.x, self.act, self.out = rt, mlp, x, None, None
+
+    def first(self, w):
+        """x . w^T"""
+        from .. import ops
+        rt, mlp, x = self.rt, self.mlp, self.x
+        if not rt.pairs_ok(x, w):
+            return rt.linear(x, w)
+        proj, self.act = rt.empty((x.shape[0], w.shape[0])), rt.empty((x.shape[0], mlp.width))
+        ops.linear_skinny_pair(x, mlp.w_gate_up, self.act, x, w, proj, True, mlp.form, mlp.b_gate_up)
+        return proj
+
+    def last(self, y, w):
+        """y . w^T"""
+        from .. import ops
+        rt, mlp = self.rt, self.mlp
+        if self.act is None or not rt.pairs_ok(y, w):
+            return rt.linear(y, w)
+        out, self.out = rt.empty((y.shape[0], w.shape[0])), rt.empty((y.shape[0], mlp.w_down.shape[0]))
+        ops.linear_skinny_pair(self.act, mlp.w_down, self.out, y, w, out)
+        return out
+
+    def result(self, ctx):
+        """The feed-forward's result, as its `forward` gives it."""
+        mlp = self.mlp
+        if self.out is None:
+            self.out = mlp.down(ctx, self.act if self.act is not None else mlp.activated(ctx, self.x))
+        return self.out if mlp.b_down is None else BiasedDelta(self.out, mlp.b_down)
 
 
 class PolyNormMlp(FeedForward):

@@ -113,10 +113,12 @@ class LatentAttention(Mixer):
         if self.position is not None:
             self.position.bind({}, rt)
 
-    def forward(self, ctx, x, cache):
+    takes_beside = True
+
+    def forward(self, ctx, x, cache, beside=None):
         rt, T, H = ctx.rt, x.shape[0], self.num_heads
         table = self.position.prepare(ctx) if self.position is not None else None
-        proj = rt.linear(x, self.w_in)  # q of all heads | d | gate
+        proj = rt.linear(x, self.w_in) if beside is None else beside.first(self.w_in)  # q of all heads | d | gate
         at = H * self.q_dim + self.rank + self.rot_dim
         q, dkv = proj[:, :H * self.q_dim], proj[:, H * self.q_dim:at]
         gate = proj[:, at:at + H] if self.head_gate else None
@@ -145,7 +147,7 @@ class LatentAttention(Mixer):
             torch.bmm(o_lat, self.w_uv_t, out=y_heads.transpose(0, 1))
         if self.has_gate:
             ops.sigmoid_gate(y, proj[:, at:])
-        return rt.linear(y, self.w_out)
+        return rt.linear(y, self.w_out) if beside is None else beside.last(y, self.w_out)
 
     def attend(self, ctx, q_lat, q_rot, cache, out, gate=None) -> None:
         latent, table = cache.arrays["latent"], ctx.block_tables[cache.group]

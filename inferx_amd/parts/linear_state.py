@@ -75,9 +75,11 @@ class GeneralizedDelta(Mixer):
         self.norm_weight = tensors["norm.weight"].contiguous()
         self.w_out = tensors["o.weight"].contiguous()
 
-    def forward(self, ctx, x, cache):
+    takes_beside = True
+
+    def forward(self, ctx, x, cache, beside=None):
         rt, T, C, H, D = ctx.rt, x.shape[0], self.channels, self.num_heads, self.head_dim
-        proj = rt.linear(x, self.w_in)  # r | k | v | gate | rate's logits
+        proj = rt.linear(x, self.w_in) if beside is None else beside.first(self.w_in)  # r | k | v | gate | rate's logits
         r, k, v, gate, rate = (proj[:, i * C:(i + 1) * C] for i in range(5))
         low = rt.linear_f32(x, self.w_w1)
         ops.tanh_(low)
@@ -100,7 +102,7 @@ class GeneralizedDelta(Mixer):
         y = rt.empty((T, C))
         ops.head_norm_gate(o, y, self.norm_eps, weight=self.norm_weight, gate=gate, weight_per_head=True,
                            gate_sigmoid=True)
-        return rt.linear(y, self.w_out)
+        return rt.linear(y, self.w_out) if beside is None else beside.last(y, self.w_out)
 
 
 CHUNKED_MIN_ROWS = 16  # portions of at least this many rows are worked in chunks
@@ -250,9 +252,11 @@ class LightningAttention(Mixer):
         self.w_out = tensors["o.weight"].contiguous()
         self.decay = torch.tensor(self.decay_values, dtype=torch.float64).to(torch.float32).to(rt.device)
 
-    def forward(self, ctx, x, cache):
+    takes_beside = True
+
+    def forward(self, ctx, x, cache, beside=None):
         rt, T, H = ctx.rt, x.shape[0], self.num_heads
-        proj = rt.linear(x, self.w_in)  # q | k | v | gate
+        proj = rt.linear(x, self.w_in) if beside is None else beside.first(self.w_in)  # q | k | v | gate
         Q, V = self.qk_dim, self.v_dim
         q, k, v, gate = proj[:, :Q], proj[:, Q:2 * Q], proj[:, 2 * Q:2 * Q + V], proj[:, 2 * Q + V:]
         o = rt.empty((T, H, self.value_dim), torch.float32)
@@ -260,7 +264,7 @@ class LightningAttention(Mixer):
         y = rt.empty((T, V))
         # one norm over all heads together: "one head" of all heads' value columns
         ops.head_norm_gate(o.view(T, 1, V), y, self.norm_eps, weight=self.norm_weight, gate=gate, gate_sigmoid=True)
-        return rt.linear(y, self.w_out)
+        return rt.linear(y, self.w_out) if beside is None else beside.last(y, self.w_out)
 
 
 class Retention(Mixer):
@@ -303,10 +307,12 @@ class Retention(Mixer):
         if self.position is not None:
             self.position.bind({}, rt)
 
-    def forward(self, ctx, x, cache):
+    takes_beside = True
+
+    def forward(self, ctx, x, cache, beside=None):
         rt, T, H = ctx.rt, x.shape[0], self.num_heads
         table = self.position.prepare(ctx) if self.position is not None else None
-        proj = rt.linear(x, self.w_in)  # q | k | v | gate
+        proj = rt.linear(x, self.w_in) if beside is None else beside.first(self.w_in)  # q | k | v | gate
         Q, V = self.qk_dim, self.v_dim
         q, k, v, gate = proj[:, :Q], proj[:, Q:2 * Q], proj[:, 2 * Q:2 * Q + V], proj[:, 2 * Q + V:]
         o = rt.empty((T, H, self.value_dim), torch.float32)
@@ -314,7 +320,7 @@ class Retention(Mixer):
                       k_scale=self.head_dim ** -0.5)
         y = rt.empty((T, V))
         ops.head_norm_gate(o, y, self.norm_eps, gate=gate)
-        return rt.linear(y, self.w_out)
+        return rt.linear(y, self.w_out) if beside is None else beside.last(y, self.w_out)
 
 
 register_part("mixer", "retention", Retention)

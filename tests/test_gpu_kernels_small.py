@@ -482,3 +482,31 @@ def test_random_weights_are_the_same_bits_on_the_host_and_on_the_device():
         host = counter_normal(11, "model.layers.2.mlp.experts.5.up_proj.weight", shape, std)
         device = counter_normal(11, "model.layers.2.mlp.experts.5.up_proj.weight", shape, std, device="cuda:0")
         assert torch.equal(host, device.cpu())
+
+
+@pytest.mark.parametrize("rows", [1, 7, 8, 9, 16])
+@pytest.mark.parametrize("gate_up", [False, True])
+@pytest.mark.parametrize("n,k,n2,k2", [(2048, 2048, 2048, 5632), (704, 264, 37, 264), (5632, 2048, 3648, 2048), (33, 8, 100, 1160)])
+def test_two_products_of_few_rows_in_one_launch(n, k, n2, k2, gate_up, rows):
+    """Both as in launches of their own (the same bits where the reduction is cut as there), with nothing written beside them."""
+    from inferx_amd import ops
+    bf = torch.bfloat16
+    x, x2 = rnd(rows, k, dtype=bf), rnd(rows, k2, seed=1, dtype=bf)
+    w, w2 = rnd((2 if gate_up else 1) * n, k, seed=2, dtype=bf, scale=k ** -0.5), rnd(n2, k2, seed=3, dtype=bf, scale=k2 ** -0.5)
+    bias = rnd(w.shape[0], seed=4, dtype=bf)
+    bufs = [torch.full((rows * m + 16,), 7.0, dtype=bf, device=DEV) for m in (n, n2)]
+    out, out2 = bufs[0][8:-8].view(rows, n), bufs[1][8:-8].view(rows, n2)
+    ops.linear_skinny_pair(x, w, out, x2, w2, out2, gate_up, 7.0 if gate_up else 0.0, bias)
+    assert all((b[:8] == 7).all() and (b[-8:] == 7).all() for b in bufs)
+    z = x.double() @ w.double().T + bias.double()
+    if gate_up:
+        g, u = z[:, :n].clamp(max=7), z[:, n:].clamp(-7, 7)
+        z = g * torch.sigmoid(1.702 * g) * (u + 1)
+    for got, want in ((out, z), (out2, x2.double() @ w2.double().T)):
+        # one rounding of the result and float32 sums
+        assert float((got.double() - want).abs().max()) <= 2 ** -8 * float(want.abs().max()) + 1e-5
+    if not gate_up and n2 == 2048:
+        one, two = torch.empty_like(out), torch.empty_like(out2)
+        ops.linear_skinny(x, w, one, bias=bias)
+        ops.linear_skinny(x2, w2, two)
+        assert torch.equal(out, one) and torch.equal(out2, two)

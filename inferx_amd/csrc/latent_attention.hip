@@ -17,12 +17,13 @@
 //   cos_sin  float32 [T, pairs, 2]: element 2i of a rotated part is paired with 2i + 1, i < pairs; the rest passes
 //            (`halves`: element i is paired with i + pairs instead, the first 2 * pairs numbers of the part)
 //   cache    [pages * page_size, rank + rot_dim]; slots[t] is the token's row
+//   own_c, own_r (or null): [tokens, rank] and [tokens, rot_dim], which get the same numbers
 template <typename T>
 __global__ void __launch_bounds__(256)
 latent_prepare_kernel(T* __restrict__ q, int64_t q_stride, const T* __restrict__ dkv, int64_t dkv_stride,
                       const void* __restrict__ norm_w, int nw_dtype, float eps, const float* __restrict__ cos_sin,
                       int pairs, const int32_t* __restrict__ slots, T* __restrict__ cache, int heads, int q_dim,
-                      int rot_dim, int rank, int halves) {
+                      int rot_dim, int rank, int halves, T* __restrict__ own_c, T* __restrict__ own_r) {
   __shared__ float red[16];
   const int64_t t = blockIdx.x;
   const int tid = threadIdx.x;
@@ -45,18 +46,22 @@ latent_prepare_kernel(T* __restrict__ q, int64_t q_stride, const T* __restrict__
   }
   ss = ix_block_sum(ss, red);
   if (!dst) return;
+  auto put = [&](int i, float x) {
+    ix_store(dst + i, x);
+    if (own_c) ix_store(i < rank ? own_c + t * rank + i : own_r + t * rot_dim + (i - rank), x);
+  };
   const float inv = 1.0f / sqrtf(ss / static_cast<float>(rank) + eps);
   for (int i = tid; i < rank; i += blockDim.x)
-    ix_store(dst + i, ix_load(row + i) * inv * ix_load_rt(norm_w, nw_dtype, i));
+    put(i, ix_load(row + i) * inv * ix_load_rt(norm_w, nw_dtype, i));
   if (halves) {
     for (int i = tid; i < rot_dim; i += blockDim.x) {
       const float x = ix_load(row + rank + i);
       if (i < 2 * pairs) {
         const int p = i < pairs ? i : i - pairs;
         const float other = ix_load(row + rank + (i < pairs ? i + pairs : i - pairs)), c = cs[2 * p], s = cs[2 * p + 1];
-        ix_store(dst + rank + i, i < pairs ? x * c - other * s : x * c + other * s);
+        put(rank + i, i < pairs ? x * c - other * s : x * c + other * s);
       } else {
-        ix_store(dst + rank + i, x);
+        put(rank + i, x);
       }
     }
     return;
@@ -66,11 +71,11 @@ latent_prepare_kernel(T* __restrict__ q, int64_t q_stride, const T* __restrict__
     const float u = ix_load(row + rank + i);
     if (p < pairs) {
       const float v = ix_load(row + rank + i + 1), c = cs[2 * p], s = cs[2 * p + 1];
-      ix_store(dst + rank + i, u * c - v * s);
-      ix_store(dst + rank + i + 1, v * c + u * s);
+      put(rank + i, u * c - v * s);
+      put(rank + i + 1, v * c + u * s);
     } else {
-      ix_store(dst + rank + i, u);
-      if (i + 1 < rot_dim) ix_store(dst + rank + i + 1, ix_load(row + rank + i + 1));
+      put(rank + i, u);
+      if (i + 1 < rot_dim) put(rank + i + 1, ix_load(row + rank + i + 1));
     }
   }
 }
@@ -78,19 +83,21 @@ latent_prepare_kernel(T* __restrict__ q, int64_t q_stride, const T* __restrict__
 extern "C" int ix_latent_prepare(void* q, int64_t q_stride, const void* dkv, int64_t dkv_stride, int dtype, const void* norm_w,
                                  int nw_dtype, float eps, const float* cos_sin, int pairs, const int32_t* slots,
                                  void* cache, int64_t tokens, int heads, int q_dim, int rot_dim, int rank, int halves,
-                                 hipStream_t stream) {
+                                 void* own_c, void* own_r, hipStream_t stream) {
   IX_REQUIRE(tokens >= 0 && heads > 0 && rank > 0 && rot_dim >= 0 && q_dim >= rot_dim, "sizes must be positive");
   IX_REQUIRE(pairs >= 0 && 2 * pairs <= rot_dim && (pairs == 0 || cos_sin != nullptr),
              "the rotated pairs must fit into the rotated part");
+  IX_REQUIRE(own_c == nullptr || (slots != nullptr && (own_r != nullptr || rot_dim == 0)), "rows of their own are copies of the cache's");
   if (tokens == 0) return 0;
   dim3 grid(static_cast<unsigned>(tokens)), block(256);
   if (dtype == IX_F32)
     hipLaunchKernelGGL(latent_prepare_kernel<float>, grid, block, 0, stream, (float*)q, q_stride, (const float*)dkv, dkv_stride,
-                       norm_w, nw_dtype, eps, cos_sin, pairs, slots, (float*)cache, heads, q_dim, rot_dim, rank, halves);
+                       norm_w, nw_dtype, eps, cos_sin, pairs, slots, (float*)cache, heads, q_dim, rot_dim, rank, halves,
+                       (float*)own_c, (float*)own_r);
   else if (dtype == IX_BF16)
     hipLaunchKernelGGL(latent_prepare_kernel<bf16_t>, grid, block, 0, stream, (bf16_t*)q, q_stride, (const bf16_t*)dkv,
                        dkv_stride, norm_w, nw_dtype, eps, cos_sin, pairs, slots, (bf16_t*)cache, heads, q_dim, rot_dim,
-                       rank, halves);
+                       rank, halves, (bf16_t*)own_c, (bf16_t*)own_r);
   else
     IX_REQUIRE(false, "dtype must be float32 or bfloat16");
   return ix_check_launch("ix_latent_prepare");

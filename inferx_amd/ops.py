@@ -1910,11 +1910,12 @@ def stream_norm(h: torch.Tensor, y: Optional[torch.Tensor], mix: Optional[torch.
 # ---- attention over a compressed cache ------------------------------------------------------------------------------
 def latent_prepare(q: torch.Tensor, dkv: torch.Tensor, norm_w: torch.Tensor, eps: float,
                    cos_sin: Optional[torch.Tensor], slots: Optional[torch.Tensor], cache: torch.Tensor, heads: int,
-                   rot_dim: int, rank: int, halves: bool = False) -> None:
+                   rot_dim: int, rank: int, halves: bool = False,
+                   own: Optional[Tuple[torch.Tensor, torch.Tensor]] = None) -> None:
     """Per token: the last `rot_dim` numbers of every head of q [T, heads * q_dim] are rotated in place (pairs
     (2i, 2i + 1), i < cos_sin.shape[1]; float32 table [T, pairs, 2]; with `halves` the pairs (i, i + pairs)); the first `rank` numbers of the dkv row pass an
     RMS norm with `norm_w` (float32 sums), its last rot_dim are rotated likewise, and [c | kr] goes to row slots[t] of
-    `cache` [pages, 1, page_size, rank + rot_dim]."""
+    `cache` [pages, 1, page_size, rank + rot_dim], and c and kr to `own`, contiguous [T, rank] and [T, rot_dim], as well."""
     T = q.shape[0]
     _need(q.dim() == 2 and q.stride(1) == 1 and q.is_cuda and q.shape[1] % heads == 0, "q must be rows of heads * q_dim")
     q_dim = q.shape[1] // heads
@@ -1931,9 +1932,37 @@ def latent_prepare(q: torch.Tensor, dkv: torch.Tensor, norm_w: torch.Tensor, eps
           and cache.is_contiguous(), "the cache must be [pages, 1, page_size, rank + rot_dim] of q's type")
     if slots is not None:
         _is_i32(slots, T)
+    own_c, own_r = own if own is not None else (None, None)
+    if own is not None:
+        _need(slots is not None and own_c.dtype == q.dtype and own_r.dtype == q.dtype and own_c.is_contiguous()
+              and own_r.is_contiguous() and tuple(own_c.shape) == (T, rank) and tuple(own_r.shape) == (T, rot_dim),
+              "rows of their own are [T, rank] and [T, rot_dim] of q's type, copies of what the cache gets")
     _call("ix_latent_prepare", q.data_ptr(), _i64(q.stride(0)), dkv.data_ptr(), _i64(dkv.stride(0)), _i32(_dt(q)), _ptr(norm_w),
           _i32(_dt(norm_w)), _f32(eps), _ptr(cos_sin), _i32(pairs), _ptr(slots), _ptr(cache), _i64(T), _i32(heads),
-          _i32(q_dim), _i32(rot_dim), _i32(rank), _i32(1 if halves else 0), _stream())
+          _i32(q_dim), _i32(rot_dim), _i32(rank), _i32(1 if halves else 0), _ptr(own_c), _ptr(own_r), _stream())
+
+
+LATENT_WHOLE_SIZES = (128, 64, 128)  # numbers of a key, its rotated part and a value
+LATENT_WHOLE_QUERIES = 64
+
+
+def latent_whole(q: torch.Tensor, kv: torch.Tensor, rot: torch.Tensor, tiles: torch.Tensor, out: torch.Tensor,
+                 scale: float) -> None:
+    """Attention of requests that bring their whole contexts, on keys and values of each head's own (latent_whole.hip): q
+    [T, heads, 192] with the rotated part behind, kv [T, heads * 256] (all heads' keys of 128, then their values of 128), rot
+    [T, 64], tiles int32 [3, n] (first row, up to 64 rows, position of the first; a request's rows are its positions from 0 on)
+    -> out [T, heads, 128].  Bfloat16; scale positive."""
+    T, heads = q.shape[0], q.shape[1]
+    dim, rd, vd = LATENT_WHOLE_SIZES
+    _need(all(t.dtype == torch.bfloat16 and t.is_cuda for t in (q, kv, rot, out)), "bfloat16 on the device")
+    _need(q.dim() == 3 and q.shape[2] == dim + rd and q.stride(2) == 1 and tuple(out.shape) == (T, heads, vd) and out.stride(2) == 1
+          and tuple(kv.shape) == (T, heads * (dim + vd)) and kv.is_contiguous() and tuple(rot.shape) == (T, rd)
+          and rot.is_contiguous(), "q [T, heads, 192], kv [T, heads * 256], rot [T, 64], out [T, heads, 128]")
+    _need((q.data_ptr() | kv.data_ptr() | rot.data_ptr()) % 16 == 0 and out.data_ptr() % 8 == 0, "operands on 16-byte boundaries")
+    _need(tiles.dim() == 2 and tiles.shape[0] == 3 and scale > 0, "tiles must be int32 [3, n], scale positive")
+    _is_i32(tiles)
+    _call("ix_latent_whole", q.data_ptr(), _i64(q.stride(0)), _i64(q.stride(1)), _ptr(kv), _ptr(rot), _ptr(tiles), _i32(tiles.shape[1]),
+          out.data_ptr(), _i64(out.stride(0)), _i64(out.stride(1)), _i64(T), _i32(heads), _f32(scale), _stream())
 
 
 def _head_gate(gate: Optional[torch.Tensor], tokens: int, heads: int, dtype):

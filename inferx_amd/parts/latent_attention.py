@@ -4,10 +4,14 @@ maps, and one rotated key part that all heads share.
     q        = x . Wq^T                          per head [dim plain | rot_dim rotated]
     d        = x . Wdkv^T                        rank + rot_dim numbers
     c        = rmsnorm(d[:rank]) * w_c           the latent (float32 sums); kr = rotate(d[rank:])
-    k_h, v_h = Wuk_h c,  Wuv_h c                 never formed: the maps move to the query's side
+    k_h, v_h = Wuk_h c,  Wuv_h c                 not formed: the maps move to the query's side
     ql_h     = Wuk_h^T q_h[:dim]                 a product per head before the attention
     p_h      = softmax_j<=i((ql_h . c[j] + rotate(q_h[dim:]) . kr[j]) * scale)
     y        = concat_h(Wuv_h (sum_j p_h[j] c[j])) . Wo^T        a product per head after it
+
+Where every request of a step brings its whole context, the keys and values are formed after all, for the step only (see
+`whole_contexts`): the products that move queries and results fall away, and the attention reads 192 + 128 numbers a key and
+head instead of 576 + 512.
 
 Only [c | kr] is kept per token (`CacheNeed` of one array, one "head" of rank + rot_dim numbers), whatever the
 number of heads.  The rotation pairs element 2i with 2i + 1 over the first `rotary_dim` numbers of the rotated part
@@ -27,12 +31,19 @@ from __future__ import annotations
 
 from typing import List, Optional
 
+import numpy as np
 import torch
 
 from .. import ops
 from ..config.spec import PartSpec
+from .attention import _tiles_of
 from .base import CacheArray, CacheNeed, Mixer, ParamSpec, build_part, register_part
 from .dense_mlp import stack_rows
+
+# From so many tokens of a step on, whole contexts get keys and values of each head's own.  Four layers, two of them with this
+# mixer (16 heads of 128 + 64, a latent of 512), us, on the latents / on keys and values: one prompt of 64 tokens 931 / 913, of 256
+# 872 / 840, of 1,100 1,318 / 1,135, of 6,000 5,347 / 4,282; 8 of 20 886 / 856, 32 of 160 3,522 / 3,393.
+WHOLE_TOKENS = 64
 
 
 class LatentAttention(Mixer):
@@ -65,7 +76,7 @@ class LatentAttention(Mixer):
             if getattr(self.position, "begin", 0) != 0 or dims <= 0 or dims % 2 or dims > self.rot_dim:
                 raise ValueError(f"the position encoding must rotate the first {dims} elements of a rotated part of "
                                  f"{self.rot_dim}: an even number within the part, from its start")
-        self.w_in = self.w_uk = self.w_uv_t = self.w_uk_rows = self.w_uv_rows = self.w_out = self.norm_weight = None
+        self.w_in = self.w_kv = self.w_uk = self.w_uv_t = self.w_uk_rows = self.w_uv_rows = self.w_out = self.norm_weight = None
 
     def cache_need(self) -> CacheNeed:
         return CacheNeed((CacheArray("latent", 1, self.rank + self.rot_dim),), self.window)
@@ -98,6 +109,9 @@ class LatentAttention(Mixer):
             odd = -sum(t.shape[0] for t in rows) % 8
             rows.append(rows[-1].new_zeros((odd, self.hidden_size)))
         self.w_in = stack_rows(rows)
+        if rt.dtype == torch.bfloat16 and (self.head_dim, self.rot_dim, self.value_dim) == ops.LATENT_WHOLE_SIZES:
+            self.w_kv = torch.cat([uk, uv])  # (the two maps one behind the other, for whole contexts' keys and values)
+            uk, uv = self.w_kv[:uk.shape[0]], self.w_kv[uk.shape[0]:]
         self.w_uk = uk.contiguous().view(H, self.head_dim, self.rank)
         w_uv = uv.contiguous().view(H, self.value_dim, self.rank)
         self.w_uv_t = w_uv.transpose(1, 2).contiguous()
@@ -123,10 +137,16 @@ class LatentAttention(Mixer):
         q, dkv = proj[:, :H * self.q_dim], proj[:, H * self.q_dim:at]
         gate = proj[:, at:at + H] if self.head_gate else None
         latent = cache.arrays["latent"]
+        tiles = self.whole_contexts(ctx, q, cache)
+        own = (rt.empty((T, self.rank)), rt.empty((T, self.rot_dim))) if tiles is not None else None
         ops.latent_prepare(q, dkv, self.norm_weight, self.eps, table,
                            ctx.slots[cache.group] if cache.writes else None, latent, H, self.rot_dim, self.rank,
-                           self.halves)
+                           self.halves, own)
         q3 = q.unflatten(1, (H, self.q_dim))
+        if own is not None:
+            y = rt.empty((T, H * self.value_dim))
+            ops.latent_whole(q3, rt.linear(own[0], self.w_kv), own[1], tiles, y.view(T, H, self.value_dim), self.scale)
+            return self.last(rt, y, proj[:, at:], beside)
         q_own = q3[:, :, :self.head_dim]
         if self.w_uk_rows is not None and ops.heads_product_fits(q_own, self.w_uk_rows):
             q_lat = rt.empty((T, H, self.rank))
@@ -145,9 +165,30 @@ class LatentAttention(Mixer):
             ops.heads_product(o_own, self.w_uv_rows, y_heads)
         else:
             torch.bmm(o_lat, self.w_uv_t, out=y_heads.transpose(0, 1))
+        return self.last(rt, y, proj[:, at:], beside)
+
+    def last(self, rt, y, gate, beside):
         if self.has_gate:
-            ops.sigmoid_gate(y, proj[:, at:])
+            ops.sigmoid_gate(y, gate)
         return rt.linear(y, self.w_out) if beside is None else beside.last(y, self.w_out)
+
+    def whole_contexts(self, ctx, q, cache):
+        """Where every request of the step brings its whole context and the sizes are those of the kernel that works on keys and
+        values of each head's own: its tiles, the ones that read most keys first; otherwise None."""
+        if (ctx.host is None or ctx.one_token_each or ctx.num_tokens < WHOLE_TOKENS or self.window or self.head_gate
+                or not cache.writes or self.scale <= 0
+                or self.w_kv is None or self.w_in.shape[0] % 8
+                or ctx.num_tokens * self.num_heads * 512 >= 1 << 32):
+            return None
+        if "whole_contexts" not in ctx.memo:
+            b, plan = ctx.host, None
+            n, first = (b.q_start[1:] - b.q_start[:-1]).astype(np.int64), b.q_start[:-1].astype(np.int64)
+            if np.all((n == b.seq_lens) | (n == 0)):
+                seq, row, rows = _tiles_of(n, first, np.arange(len(n)), ops.LATENT_WHOLE_QUERIES)
+                plan = np.stack([row, rows, row - first[seq]]).astype(np.int32)
+                plan = ops.upload(np.ascontiguousarray(plan[:, np.argsort(-(plan[1] + plan[2]), kind="stable")]), ctx.rt.device)
+            ctx.memo["whole_contexts"] = plan
+        return ctx.memo["whole_contexts"]
 
     def attend(self, ctx, q_lat, q_rot, cache, out, gate=None) -> None:
         latent, table = cache.arrays["latent"], ctx.block_tables[cache.group]

@@ -408,6 +408,43 @@ def test_latent_attention_of_prompts(H, rank, rot, page, window, gated):
     assert torch.isfinite(out).all() and err <= 2e-2, f"{err:.2e}"
 
 
+@pytest.mark.parametrize("H", [1, 3, 16])
+@pytest.mark.parametrize("lengths", [[1, 63, 64, 65], [33, 200, 1, 129], [20], [577, 31]])
+def test_latent_attention_of_whole_contexts(H, lengths):
+    """Requests that end within a tile, a step of 32 keys or a wavefront's share of them; the tensors around the operands and
+    another request's rows are NaN, and reach nothing.  Against float64 on the same numbers: the weights' and the results'
+    rounding to bfloat16, 2^-9 each of at most the values' size (4), and as much again for the exponentials and sums."""
+    from inferx_amd import ops
+    T, dim, rd, vd = sum(lengths) + 70, 128, 64, 128
+    scale = (dim + rd) ** -0.5
+    q = torch.full((T, H * (dim + rd) + 64), float("nan"), dtype=torch.bfloat16, device=DEV)
+    kv = torch.full((T, H * (dim + vd)), float("nan"), dtype=torch.bfloat16, device=DEV)
+    rot = torch.full((T, rd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    n = sum(lengths)
+    q[:n, :H * (dim + rd)] = rnd((n, H * (dim + rd)), 1, 2.0, torch.bfloat16).to(DEV)
+    kv[:n] = rnd((n, H * (dim + vd)), 2, 1.0, torch.bfloat16).to(DEV).clamp(-4, 4)
+    rot[:n] = rnd((n, rd), 3, 2.0, torch.bfloat16).to(DEV)
+    tiles, at = [], 0
+    for length in lengths + [70]:
+        tiles += [(at + i, min(64, length - i), i) for i in range(0, length, 64)]
+        at += length
+    out = torch.full((T, H, vd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    q3 = q[:, :H * (dim + rd)].unflatten(1, (H, dim + rd))
+    ops.latent_whole(q3, kv, rot, torch.tensor(tiles, dtype=torch.int32, device=DEV).t().contiguous(), out, scale)
+    at = 0
+    for length in lengths:
+        r = slice(at, at + length)
+        k = torch.cat([kv[r, :H * dim].unflatten(1, (H, dim)), rot[r, None].expand(length, H, rd)], 2).cpu().double()
+        v = kv[r, H * dim:].unflatten(1, (H, vd)).cpu().double()
+        s = torch.einsum("qhd,khd->hqk", q3[r].cpu().double(), k) * scale
+        s = s.masked_fill(torch.ones(length, length, dtype=torch.bool).triu(1), float("-inf"))
+        want = torch.einsum("hqk,khd->qhd", s.softmax(2), v)
+        err = float((out[r].cpu().double() - want).abs().max())
+        assert err <= 4 * 4 * 2.0 ** -9, f"{length}: {err:.2e}"
+        at += length
+    assert torch.isnan(out[n:]).all()
+
+
 # the smallest sizes of the kernel's three forms and their largest (128, 320 with a latent of 256, 576), one row of each
 # with fewer numbers than the form has room for
 @pytest.mark.parametrize("rank,rot", [(16, 16), (96, 0), (112, 16), (128, 32), (144, 48), (256, 64), (272, 16), (512, 0), (512, 64)])

@@ -43,8 +43,8 @@
 //
 // What bounds it: row by row, the chain of dependent sums of a row (0.33 us a row whatever the chip is doing).  In chunks
 // the chain is 64 times shorter and its step two small products (3.6 us a chunk).  Measured with 16 heads of 128 x 128, one
-// request, all three launches against row by row: 51 against 46 us at 128 rows, 59 against 72 at 200, 81 against 172 at
-// 500, 155 against 474 at 1,437, 190 against 672 at 2,048 (with 32-bit sums throughout 151).  The generalized rule, 32 heads
+// request, all three launches against row by row: 44 against 46 us at 128 rows, 51 against 72 at 200, 68 against 172 at
+// 500, 141 against 474 at 1,437, 177 against 672 at 2,048.  The generalized rule, 32 heads
 // of 64 x 64: 42 against 43 us at 160 rows, 46 against 66 at 256, 169 against 492 at 2,048 (with 32-bit sums 130).
 //
 // A lane's operand of a 16 x 16 x 4 product is one number of row (column) l % 16 at reduction index l / 16.  Operands
@@ -159,6 +159,7 @@ __device__ __forceinline__ void dc_invert_diagonal(const float* a_s, float (*t_s
 #pragma unroll
     for (int j = 0; j < i; ++j) s = fmaf(-ar[j], x[j], s);
     x[i] = s;
+    if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // (not all of the block's numbers at once: that would be 120 registers)
   }
 #pragma unroll
   for (int i = 0; i < 16; ++i) t_s[b][i][col] = i == col ? 0.f : x[i];
@@ -206,21 +207,30 @@ __device__ __forceinline__ void dc_solve(const float* a_s, const float (*t_s)[16
     }
 #pragma unroll
     for (int u = 0; u < NT; ++u) x[u][b] += y[u];
+    __builtin_amdgcn_sched_barrier(0);  // (the next block's operands: not before)
   }
 }
 
+// A chunk and head takes a workgroup some 30 us whatever else the chip is doing (sums and inner products one behind the other), so
+// three of them share a compute unit: rows stay in LDS as they came, with their factors beside them, and a wavefront solves for
+// two tiles at a time.  All three launches, us, with two workgroups to a compute unit (rows in 32 bits, four tiles) / as it is: 16
+// heads of 128 x 128, 33 chunks (528 workgroups, 16 more than went at once) 177 / 159, 32 chunks 183 / 177, 16 requests of 300
+// rows 355 / 303.
 template <int DIM>
-__global__ void __launch_bounds__(DC_THREADS, 2)
+__global__ void __launch_bounds__(DC_THREADS, 3)
 delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, int64_t q_stride, int64_t k_stride,
                             int64_t v_stride, const float* __restrict__ ab, const float* __restrict__ a_log,
                             const float* __restrict__ dt_bias, const int32_t* __restrict__ chunk_row0,
                             const int32_t* __restrict__ chunk_rows, float* __restrict__ work, int heads, int kv_heads,
                             int vdim) {
-  constexpr int LD = DIM + 4, LA = DC_ROWS + 4;
-  __shared__ __attribute__((aligned(16))) float k_s[DC_ROWS * LD];
-  // the queries, and once they are done with A in their place (two workgroups fit a compute unit so)
-  __shared__ __attribute__((aligned(16))) float qa_s[DC_ROWS * (LD > LA ? LD : LA)];
-  float *const q_s = qa_s, *const a_s = qa_s;
+  constexpr int LD = DIM + 8, LA = DC_ROWS + 4;
+  // Rows as they came, and the factors that make them unit rows: half the room of the products.
+  __shared__ __attribute__((aligned(16))) bf16_t k_s[DC_ROWS * LD];
+  // the queries, and once they are done with A in their place
+  __shared__ __attribute__((aligned(16))) unsigned char qa_s[DC_ROWS * (2 * LD > 4 * LA ? 2 * LD : 4 * LA)];
+  bf16_t* const q_s = reinterpret_cast<bf16_t*>(qa_s);
+  float* const a_s = reinterpret_cast<float*>(qa_s);
+  __shared__ float f_s[2][DC_ROWS];  // the keys' factors, the queries'
   __shared__ __attribute__((aligned(16))) float t_s[4][16][20];  // inverses of the blocks on the diagonal of I + A
   __shared__ double c_s[DC_ROWS];                                // log G_i
   __shared__ double beta_s[DC_ROWS], g_s[DC_ROWS], rest_s[DC_ROWS];  // beta_i, G_i, G_n / G_i (products with them round once)
@@ -246,27 +256,24 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
       for (int i = 0; i < QUARTER / 8; ++i) raw[which][i] = *reinterpret_cast<const uint4*>(rows[which] + 8 * i);
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
-      float x[QUARTER];
+      bf16_t* dst = (which ? q_s : k_s) + row * LD + part * QUARTER;
       double sum = 0.;  // (a row's factor is one error for all its numbers)
 #pragma unroll
       for (int i = 0; i < QUARTER / 8; ++i) {
         const uint32_t u[4] = {raw[which][i].x, raw[which][i].y, raw[which][i].z, raw[which][i].w};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          x[8 * i + 2 * e] = __uint_as_float(u[e] << 16);
-          x[8 * i + 2 * e + 1] = __uint_as_float(u[e] & 0xffff0000u);
+          const double lo = __uint_as_float(u[e] << 16), hi = __uint_as_float(u[e] & 0xffff0000u);
+          sum += lo * lo;
+          sum += hi * hi;
         }
+        *reinterpret_cast<uint4*>(dst + 8 * i) = raw[which][i];
       }
-#pragma unroll
-      for (int i = 0; i < QUARTER; ++i) sum += static_cast<double>(x[i]) * static_cast<double>(x[i]);
       float ss = static_cast<float>(sum);
       ss += ix_dpp<IX_DPP_XOR1>(ss);
       ss += ix_dpp<IX_DPP_XOR2>(ss);
-      const float f = row < n ? (which ? 1.0f / sqrtf(static_cast<float>(DIM)) : 1.0f) / sqrtf(ss + 1e-6f) : 0.f;
-      float* dst = (which ? q_s : k_s) + row * LD + part * QUARTER;
-#pragma unroll
-      for (int i = 0; i < QUARTER; i += 4)
-        *reinterpret_cast<f32x4*>(dst + i) = f32x4{x[i] * f, x[i + 1] * f, x[i + 2] * f, x[i + 3] * f};
+      if (part == 0)
+        f_s[which][row] = row < n ? (which ? 1.0f / sqrtf(static_cast<float>(DIM)) : 1.0f) / sqrtf(ss + 1e-6f) : 0.f;
     }
   }
   if (wave == 0) {
@@ -291,16 +298,23 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
   }
   __syncthreads();
 
+  // four numbers of a unit row
+  auto unit4 = [&](const bf16_t* at, float f) {
+    const uint2 u = *reinterpret_cast<const uint2*>(at);
+    return f32x4{__uint_as_float(u.x << 16) * f, __uint_as_float(u.x & 0xffff0000u) * f, __uint_as_float(u.y << 16) * f,
+                 __uint_as_float(u.y & 0xffff0000u) * f};
+  };
   // ---- q_i . k_j, then k_i . k_j: the ten tiles on and below the diagonal of each
-  auto score = [&](const float* rows, int pair, auto&& put) {
+  auto score = [&](const bf16_t* rows, const float* factors, int pair, auto&& put) {
     const int rt = pair < 1 ? 0 : (pair < 3 ? 1 : (pair < 6 ? 2 : 3)), ct = pair - rt * (rt + 1) / 2;
-    const float* ar = rows + (16 * rt + dc_turn(m)) * LD + 4 * g;
-    const float* br = k_s + (16 * ct + m) * LD + 4 * g;
+    const bf16_t* ar = rows + (16 * rt + dc_turn(m)) * LD + 4 * g;
+    const bf16_t* br = k_s + (16 * ct + m) * LD + 4 * g;
+    const float fa = factors[16 * rt + dc_turn(m)], fb = f_s[0][16 * ct + m];
     f64x4 s0 = f64x4{0., 0., 0., 0.}, s1 = s0;
 #pragma unroll
     for (int c = 0; c < DIM / 16; c += 2) {
-      s0 = dc_mac64(*reinterpret_cast<const f32x4*>(ar + 16 * c), *reinterpret_cast<const f32x4*>(br + 16 * c), s0);
-      s1 = dc_mac64(*reinterpret_cast<const f32x4*>(ar + 16 * c + 16), *reinterpret_cast<const f32x4*>(br + 16 * c + 16), s1);
+      s0 = dc_mac64(unit4(ar + 16 * c, fa), unit4(br + 16 * c, fb), s0);
+      s1 = dc_mac64(unit4(ar + 16 * c + 16, fa), unit4(br + 16 * c + 16, fb), s1);
     }
     const int j = 16 * ct + m;
 #pragma unroll
@@ -312,11 +326,11 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
   };
 #pragma unroll 1
   for (int pair = wave; pair < 10; pair += 4)
-    score(q_s, pair, [&](int i, int j, double x) { mine[blk.p() + i * 64 + j] = j <= i ? static_cast<float>(beta_s[j] * x) : 0.f; });
+    score(q_s, f_s[1], pair, [&](int i, int j, double x) { mine[blk.p() + i * 64 + j] = j <= i ? static_cast<float>(beta_s[j] * x) : 0.f; });
   // ---- what the chain and the result take as they are
   for (int id = tid; id < DIM * 16; id += DC_THREADS) {
     const int row = id / (DIM / 4), d = 4 * (id % (DIM / 4));
-    f32x4 x = *reinterpret_cast<const f32x4*>(q_s + row * LD + d);
+    f32x4 x = unit4(q_s + row * LD + d, f_s[1][row]);
 #pragma unroll
     for (int e = 0; e < 4; ++e) x[e] = static_cast<float>(x[e] * g_s[row]);
     *reinterpret_cast<f32x4*>(mine + blk.q() + row * DIM + d) = x;
@@ -324,42 +338,66 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
   __syncthreads();
 #pragma unroll 1
   for (int pair = 3 - wave; pair < 10; pair += 4)  // (the wavefronts that had three tiles above have two)
-    score(k_s, pair, [&](int i, int j, double x) { a_s[i * LA + j] = j < i ? static_cast<float>(beta_s[j] * x) : 0.f; });
+    score(k_s, f_s[0], pair, [&](int i, int j, double x) { a_s[i * LA + j] = j < i ? static_cast<float>(beta_s[j] * x) : 0.f; });
   for (int id = tid; id < DIM * 16; id += DC_THREADS) {
     const int d = id >> 4, jq = 4 * (id & 15);
     f32x4 x;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] = k_s[(jq + e) * LD + d];
+    for (int e = 0; e < 4; ++e) x[e] = ix_load(k_s + (jq + e) * LD + d) * f_s[0][jq + e];
     *reinterpret_cast<f32x4*>(mine + blk.kt() + d * 64 + jq) = x;
   }
   if (tid < DC_ROWS) reinterpret_cast<double*>(mine + blk.rest())[tid] = rest_s[tid] * beta_s[tid];
   for (int d = tid; d < DIM; d += DC_THREADS) mine[blk.g() + d] = static_cast<float>(g_s[DC_ROWS - 1]);
   __syncthreads();
 
-  // ---- the diagonal blocks' inverses: lane (block, column), sixteen steps of substitution
-  if (wave == 0) dc_invert_diagonal<LA>(a_s, t_s, g, m);
-  __syncthreads();
-
-  // ---- (I + A) [W | Uv] = [diag(G) K | V], four tiles of sixteen columns at a time and wavefront
+  // a wavefront's first tiles of V are asked for before W's, behind which they arrive
   const int tiles = (DIM + vdim) / 16;
-#pragma unroll 1
-  for (int t0 = 4 * wave; t0 < tiles; t0 += 16) {
-    f32x4 x[4][4];  // [tile][block of rows]
+  auto ask_v = [&](int t0, unsigned short (&x)[2][4][4]) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int t = min(t0 + u, tiles - 1);
+    for (int u = 0; u < 2; ++u) {
+      const bf16_t* from = v + row0 * v_stride + head * vdim + 16 * min(t0 + u, tiles - 1) - DIM + m;
 #pragma unroll
       for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int row = 16 * b + 4 * g + e;
-          if (16 * t < DIM) x[u][b][e] = static_cast<float>(g_s[row] * k_s[row * LD + 16 * t + m]);
-          else x[u][b][e] = ix_load(v + (row0 + min(row, n - 1)) * v_stride + head * vdim + 16 * t - DIM + m);
-        }
+        for (int e = 0; e < 4; ++e) x[u][b][e] = from[min(16 * b + 4 * g + e, n - 1) * v_stride].bits;
     }
-    dc_solve<LA, 4>(a_s, t_s, m, g, x);
+  };
+  // ---- the diagonal blocks' inverses: lane (block, column), sixteen steps of substitution
+  if (wave == 0) dc_invert_diagonal<LA>(a_s, t_s, g, m);
+  __builtin_amdgcn_sched_barrier(0);
+  unsigned short vx[2][4][4];
+  const int v0 = 2 * wave + (DIM / 16 - 2 * wave + 7) / 8 * 8;  // the first of its tiles that are V's
+  if (v0 < tiles) ask_v(v0, vx);
+  __builtin_amdgcn_sched_barrier(0);
+  __syncthreads();
+
+  // ---- (I + A) [W | Uv] = [diag(G) K | V], two tiles of sixteen columns at a time and wavefront (with four
+  // a compute unit's registers hold two workgroups)
+#pragma unroll 1
+  for (int t0 = 2 * wave; t0 < tiles; t0 += 8) {
+    f32x4 x[2][4];  // [tile][block of rows]
+    if (16 * t0 < DIM) {  // (DIM / 16 is even: both tiles are W's or both V's)
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int row = 16 * b + 4 * g + e;
+            x[u][b][e] = static_cast<float>(g_s[row] * (ix_load(k_s + row * LD + 16 * (t0 + u) + m) * f_s[0][row]));
+          }
+    } else {
+      if (t0 != v0) ask_v(t0, vx);
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[u][b][e] = ix_bf16_to_f32(vx[u][b][e]);
+    }
+    dc_solve<LA, 2>(a_s, t_s, m, g, x);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
       const int t = t0 + u;
       if (t >= tiles) continue;
 #pragma unroll

@@ -220,7 +220,7 @@ extern "C" int ix_latent_attention_plain(const void* ql, int64_t ql_t, int64_t q
 // column; a lane's accumulators all belong to its column, so rescaling is a multiplication by the lane's factor.
 //
 // One token per request (steps that bring more go through latent_prefill.hip): a workgroup takes one token and one slice
-// of its keys, a wavefront sixteen heads, a column one head; slices leave (max, sum, unnormalised sums) for
+// of its keys, a wavefront sixteen heads, a column one head (up to sixteen heads in all: the kernel after this one); slices leave (max, sum, unnormalised sums) for
 // `attn_combine_kernel`.  The next round's rows are on their way from memory while a round is multiplied.
 typedef __bf16 lat_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 lat_bf16x4 __attribute__((ext_vector_type(4)));
@@ -415,6 +415,172 @@ latent_attn_mfma_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_
   }
 }
 
+// The same for up to sixteen heads, which are one wavefront's columns: all four wavefronts share out the products instead.  A
+// wavefront multiplies sixteen of a round's keys over every other 32 numbers of a row; the halves of the scores meet in LDS, each
+// wavefront works the weights of all 32 keys from them (the same numbers in each) and sums up a quarter of the latent, whose rows
+// it reads transposed (ds_read_b64_tr_b16: of sixteen lanes, lanes 4 e .. 4 e + 3 name sixteen numbers of key e, and lane i
+// gets the i-th number of the four keys).
+// Eight tokens, 16 heads, 512 + 64 numbers, up to 216 keys in slices of 32: 7.7 us, with one wavefront at work and the rows written
+// transposed 11.2.
+__device__ __forceinline__ lat_bf16x4 lat_read_turned(const __bf16* at) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(lat_bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)at));
+}
+
+template <int NW, int NR>  // rank + rot_dim <= 32 NW, rank <= 16 NR, both even
+__global__ void __launch_bounds__(256)
+latent_attn_few_kernel(const __bf16* __restrict__ ql, int64_t ql_t, int64_t ql_h, const __bf16* __restrict__ qr,
+                       int64_t qr_t, int64_t qr_h, const __bf16* __restrict__ cache,
+                       const int32_t* __restrict__ block_table, const int32_t* __restrict__ seq_of_token,
+                       const int32_t* __restrict__ positions, __bf16* __restrict__ out, int64_t out_t, int64_t out_h,
+                       float* __restrict__ part_o, float* __restrict__ part_ml, int n_splits, int tokens, int heads,
+                       int rank, int rot_dim, int page_size, int max_blocks, float scale_log2,
+                       int window, const __bf16* __restrict__ head_gate, int64_t gate_stride) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char latm_lds[];
+  constexpr int NP = (4 * NW + 7) / 8;  // 16-byte pieces of a round's rows that a thread moves
+  constexpr int SP = LATM_KEYS + 4;     // scores per column in LDS
+  const int width = rank + rot_dim;
+  const int kstride = ((width + 63) & ~63) + LATM_KPAD;
+  auto key_place = [&](int r, int piece) { return r * kstride + ((piece ^ (((r >> 3) & 1) << 2)) << 3); };
+  const int p8 = width / 8, nw = width / 32, nr = rank / 16;
+  float* const sp = reinterpret_cast<float*>(latm_lds);                 // [2][16][SP]: the halves of the scores
+  __bf16* const k_s = reinterpret_cast<__bf16*>(sp + 2 * 16 * SP);      // [32][kstride]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), keys16 = wave & 1, part = wave >> 1;
+  const int n = lane & 15, g = lane >> 4;
+  const int row = blockIdx.x, head = n;
+  const bool col_ok = head < heads;
+
+  lat_bf16x8 qf[NW / 2];  // steps part, part + 2, ..
+#pragma unroll
+  for (int s = 0; s < NW / 2; ++s) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) qf[s][e] = static_cast<__bf16>(0.f);
+    if (2 * s + part < nw && col_ok) {
+      const int i = 32 * (2 * s + part) + 8 * g;
+      const __bf16* src = i < rank ? ql + row * ql_t + head * ql_h + i : qr + row * qr_t + head * qr_h + (i - rank);
+      qf[s] = *reinterpret_cast<const lat_bf16x8*>(src);
+    }
+  }
+  lat_f32x4 acc[NR / 4];  // tiles wave, wave + 4, ..
+#pragma unroll
+  for (int d = 0; d < NR / 4; ++d) acc[d] = lat_f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -1e30f, l = 0.f;
+
+  const int my_pos = positions[row];
+  const int k_lo = window > 0 ? max(my_pos + 1 - window, 0) : 0;
+  int k_begin = k_lo & ~(LATM_KEYS - 1), k_end = my_pos + 1;
+  const int per = ((k_end - k_begin + n_splits - 1) / n_splits + LATM_KEYS - 1) & ~(LATM_KEYS - 1);
+  k_begin += static_cast<int>(blockIdx.z) * per;
+  k_end = min(k_end, k_begin + per);
+  if (k_begin >= k_end && blockIdx.z > 0) {  // (as above)
+    if (g == 0 && wave == 0 && col_ok) {
+      const int64_t p = (static_cast<int64_t>(row) * heads + head) * n_splits + blockIdx.z;
+      part_ml[2 * p] = -INFINITY;
+      part_ml[2 * p + 1] = 0.f;
+    }
+    return;
+  }
+  const int32_t* table = block_table + static_cast<int64_t>(seq_of_token[row]) * max_blocks;
+  uint4 st[NP];
+  const int my_key = tid >> 3, my_sub = tid & 7;  // a thread moves pieces my_sub, my_sub + 8, .. of one key's row
+  auto ask = [&](int k0) {
+    const int j = k0 + my_key;
+    const bool there = j < k_end && j >= k_lo;
+    const int64_t at = there ? (static_cast<int64_t>(table[j / page_size]) * page_size + j % page_size) * width : 0;
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      const int pc = my_sub + 8 * u;
+      st[u] = uint4{0u, 0u, 0u, 0u};  // rows past the last key enter LDS as zeros
+      if (there && pc < p8) st[u] = *reinterpret_cast<const uint4*>(cache + at + 8 * pc);
+    }
+  };
+  if (k_begin < k_end) ask(k_begin);
+  for (int k0 = k_begin; k0 < k_end; k0 += LATM_KEYS) {  // (every decision in here is the same for the whole workgroup)
+    __syncthreads();  // the round before has been read
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+      const int pc = my_sub + 8 * u;
+      if (pc < p8) *reinterpret_cast<uint4*>(k_s + key_place(my_key, pc)) = st[u];
+    }
+    __syncthreads();
+    if (k0 + LATM_KEYS < k_end) ask(k0 + LATM_KEYS);
+    {
+      const int ka = 8 * (n >> 2) + (n & 3) + 4 * keys16;  // the key of this lane's row of the first operand
+      lat_f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < NW / 2; ++i)
+        if (2 * i + part < nw)
+          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              *reinterpret_cast<const lat_bf16x8*>(k_s + key_place(ka, 4 * (2 * i + part) + g)), qf[i], s, 0, 0, 0);
+      *reinterpret_cast<lat_f32x4*>(sp + (part * 16 + n) * SP + 8 * g + 4 * keys16) = s;
+    }
+    __syncthreads();
+    float p[8], mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 8; i += 4) {
+      const lat_f32x4 s = *reinterpret_cast<const lat_f32x4*>(sp + n * SP + 8 * g + i) +
+                          *reinterpret_cast<const lat_f32x4*>(sp + (16 + n) * SP + 8 * g + i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int j = k0 + 8 * g + i + e;
+        p[i + e] = (j >= k_lo && j < k_end) ? s[e] * scale_log2 : -INFINITY;
+        mx = fmaxf(mx, p[i + e]);
+      }
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float m_new = fmaxf(m, mx), alpha = exp2f(m - m_new);
+    m = m_new;
+    float sum = 0.f;
+    lat_bf16x8 pb;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      p[i] = exp2f(p[i] - m_new);
+      sum += p[i];
+      pb[i] = static_cast<__bf16>(p[i]);
+    }
+    l = l * alpha + sum;
+    const bool rescale = !__all(alpha == 1.0f);
+#pragma unroll
+    for (int d = 0; d < NR / 4; ++d) {
+      const int tile = wave + 4 * d;
+      if (tile < nr) {
+        if (rescale) acc[d] *= alpha;
+        // this lane names numbers 4 (n % 4) .. of the tile's sixteen, of key 8 g + n / 4 and of the one four keys on
+        const __bf16* at = k_s + key_place(8 * g + (n >> 2), 2 * tile + ((n >> 1) & 1)) + 4 * (n & 1);
+        const lat_bf16x8 a = __builtin_shufflevector(lat_read_turned(at), lat_read_turned(at + 4 * kstride), 0, 1, 2, 3, 4, 5, 6, 7);
+        acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb, acc[d], 0, 0, 0);
+      }
+    }
+  }
+
+  float lt = l + __shfl_xor(l, 16);
+  lt += __shfl_xor(lt, 32);
+  if (!col_ok) return;
+  if (n_splits > 1) {
+    const int64_t p = (static_cast<int64_t>(row) * heads + head) * n_splits + blockIdx.z;
+#pragma unroll
+    for (int d = 0; d < NR / 4; ++d)
+      if (wave + 4 * d < nr) *reinterpret_cast<lat_f32x4*>(part_o + p * rank + 16 * (wave + 4 * d) + 4 * g) = acc[d];
+    if (g == 0 && wave == 0) {
+      part_ml[2 * p] = lt > 0.f ? m : -INFINITY;
+      part_ml[2 * p + 1] = lt;
+    }
+  } else {
+    const float inv = head_gate ? 1.0f / (lt * (1.0f + __expf(-(float)head_gate[row * gate_stride + head]))) : 1.0f / lt;
+#pragma unroll
+    for (int d = 0; d < NR / 4; ++d) {
+      if (wave + 4 * d < nr) {
+        lat_bf16x4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = static_cast<__bf16>(acc[d][i] * inv);
+        *reinterpret_cast<lat_bf16x4*>(out + row * out_t + head * out_h + 16 * (wave + 4 * d) + 4 * g) = o;
+      }
+    }
+  }
+}
+
 int ix_latent_prefill(const void* ql, int64_t ql_t, int64_t ql_h, const void* qr, int64_t qr_t, int64_t qr_h,
                       const void* cache, const int32_t* block_table, const int32_t* seq_of_token, const int32_t* positions,
                       void* out, int64_t out_t, int64_t out_h, int tokens, int heads, int rank, int rot_dim, int page_size,
@@ -449,13 +615,15 @@ extern "C" int ix_latent_attention_mfma(const void* ql, int64_t ql_t, int64_t ql
     return ix_latent_prefill(ql, ql_t, ql_h, qr, qr_t, qr_h, cache, block_table, seq_of_token, positions, out, out_t, out_h,
                              static_cast<int>(tokens), heads, rank, rot_dim, page_size, max_blocks,
                              scale * 1.4426950408889634f, window, head_gate, gate_stride, stream);
-  const size_t lds = (static_cast<size_t>(LATM_KEYS) * (((width + 63) & ~63) + LATM_KPAD) + static_cast<size_t>(rank) * LATM_VSTRIDE) * 2;
+  const bool few = heads <= 16;
+  const size_t rows_lds = static_cast<size_t>(LATM_KEYS) * (((width + 63) & ~63) + LATM_KPAD) * 2;
+  const size_t lds = rows_lds + (few ? 2 * 16 * (LATM_KEYS + 4) * sizeof(float) : static_cast<size_t>(rank) * LATM_VSTRIDE * 2);
   const dim3 grid(static_cast<unsigned>(tokens), (heads + 63) / 64, n_splits);
   const float scale_log2 = scale * 1.4426950408889634f;
 #define LAUNCH(NW, NR)                                                                                                  \
   do {                                                                                                                  \
-    auto kernel = latent_attn_mfma_kernel<NW, NR>;                                                                      \
-    if (lds > 48 * 1024) {                                                                                              \
+    auto kernel = few ? latent_attn_few_kernel<NW, NR> : latent_attn_mfma_kernel<NW, NR>;                               \
+    if (lds > 48 * 1024) { /* (never with few heads) */                                                                                              \
       static bool raised = false;                                                                                       \
       if (!raised) {                                                                                                    \
         /* (a refusal shows as the launch's own error) */                                                              \

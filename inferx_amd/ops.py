@@ -1911,11 +1911,14 @@ def stream_norm(h: torch.Tensor, y: Optional[torch.Tensor], mix: Optional[torch.
 def latent_prepare(q: torch.Tensor, dkv: torch.Tensor, norm_w: torch.Tensor, eps: float,
                    cos_sin: Optional[torch.Tensor], slots: Optional[torch.Tensor], cache: torch.Tensor, heads: int,
                    rot_dim: int, rank: int, halves: bool = False,
-                   own: Optional[Tuple[torch.Tensor, torch.Tensor]] = None) -> None:
+                   own: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
+                   product: Optional[Tuple[torch.Tensor, torch.Tensor]] = None) -> None:
     """Per token: the last `rot_dim` numbers of every head of q [T, heads * q_dim] are rotated in place (pairs
     (2i, 2i + 1), i < cos_sin.shape[1]; float32 table [T, pairs, 2]; with `halves` the pairs (i, i + pairs)); the first `rank` numbers of the dkv row pass an
     RMS norm with `norm_w` (float32 sums), its last rot_dim are rotated likewise, and [c | kr] goes to row slots[t] of
-    `cache` [pages, 1, page_size, rank + rot_dim], and c and kr to `own`, contiguous [T, rank] and [T, rot_dim], as well."""
+    `cache` [pages, 1, page_size, rank + rot_dim], and c and kr to `own`, contiguous [T, rank] and [T, rot_dim], as well.
+    `product` = (w, out): also out[t, h] = w[h] . the numbers of q[t, h] before the rotated part, as `heads_product` (operands that
+    `heads_product_fits` takes, rank the rows of w; not with `own`)."""
     T = q.shape[0]
     _need(q.dim() == 2 and q.stride(1) == 1 and q.is_cuda and q.shape[1] % heads == 0, "q must be rows of heads * q_dim")
     q_dim = q.shape[1] // heads
@@ -1932,6 +1935,17 @@ def latent_prepare(q: torch.Tensor, dkv: torch.Tensor, norm_w: torch.Tensor, eps
           and cache.is_contiguous(), "the cache must be [pages, 1, page_size, rank + rot_dim] of q's type")
     if slots is not None:
         _is_i32(slots, T)
+    if product is not None:
+        w, moved = product
+        _need(own is None and heads_product_fits(q.unflatten(1, (heads, q_dim))[:, :, :q_dim - rot_dim], w)
+              and tuple(w.shape) == (heads, rank, q_dim - rot_dim), "a product that the kernel does not take")
+        _need(tuple(moved.shape) == (T, heads, rank) and moved.dtype == q.dtype and moved.stride(2) == 1,
+              "the product's result must be bfloat16 [T, heads, rank]")
+        _call("ix_latent_prepare_product", q.data_ptr(), _i64(q.stride(0)), dkv.data_ptr(), _i64(dkv.stride(0)), _ptr(norm_w),
+              _i32(_dt(norm_w)), _f32(eps), _ptr(cos_sin), _i32(pairs), _ptr(slots), _ptr(cache), _i64(T), _i32(heads),
+              _i32(q_dim), _i32(rot_dim), _i32(rank), _i32(1 if halves else 0), _ptr(w), moved.data_ptr(), _i64(moved.stride(0)),
+              _i64(moved.stride(1)), _stream())
+        return
     own_c, own_r = own if own is not None else (None, None)
     if own is not None:
         _need(slots is not None and own_c.dtype == q.dtype and own_r.dtype == q.dtype and own_c.is_contiguous()
@@ -2053,11 +2067,13 @@ def latent_attention_mfma(q_lat: torch.Tensor, q_rot: torch.Tensor, cache: torch
                           seq_of_token: torch.Tensor, positions: torch.Tensor, out: torch.Tensor, rank: int,
                           rot_dim: int, scale: float, one_token_each: bool = False, n_splits: int = 1,
                           work: Optional[Tuple[torch.Tensor, torch.Tensor]] = None, window: int = 0,
-                          head_gate: Optional[torch.Tensor] = None) -> None:
+                          head_gate: Optional[torch.Tensor] = None, merge: bool = True) -> None:
     """`latent_attention_plain` on the matrix cores (see `latent_mfma_fits`).  `one_token_each`: every request brings
     one token; its keys may then be cut into `n_splits` slices, with `work` = float32 ([T * heads * n_splits, rank],
-    [T * heads * n_splits, 2]) and a contiguous `out` [T, heads, rank]."""
+    [T * heads * n_splits, 2]) and a contiguous `out` [T, heads, rank].  Without `merge` the slices' parts are left in `work`
+    for `latent_merge_product`, and `out` and the gate are not touched."""
     T, heads = q_lat.shape[0], q_lat.shape[1]
+    _need(merge or n_splits > 1, "there is nothing to merge")
     ql_t, ql_h = _head_rows(q_lat, T, heads, rank, "q_lat")
     qr_t, qr_h = _head_rows(q_rot, T, heads, rot_dim, "q_rot")
     o_t, o_h = _head_rows(out, T, heads, rank, "out")
@@ -2077,7 +2093,22 @@ def latent_attention_mfma(q_lat: torch.Tensor, q_rot: torch.Tensor, cache: torch
               and part_ml.dtype == torch.float32 and part_ml.numel() >= T * heads * n_splits * 2
               and part_ml.is_contiguous() and out.is_contiguous(), "the slices' workspace or a result that is not contiguous")
     _call("ix_latent_attention_mfma", q_lat.data_ptr(), _i64(ql_t), _i64(ql_h), q_rot.data_ptr(), _i64(qr_t), _i64(qr_h),
-          _ptr(cache), _ptr(block_table), _ptr(seq_of_token), _ptr(positions), out.data_ptr(), _i64(o_t), _i64(o_h),
+          _ptr(cache), _ptr(block_table), _ptr(seq_of_token), _ptr(positions), out.data_ptr() if merge else None, _i64(o_t), _i64(o_h),
           _ptr(part_o), _ptr(part_ml), _i32(n_splits), _i64(T), _i32(heads), _i32(rank), _i32(rot_dim),
           _i32(cache.shape[2]), _i32(block_table.shape[1]), _f32(scale), _i32(1 if one_token_each else 0), _i32(window),
           *_head_gate(head_gate, T, heads, q_lat.dtype), _stream())
+
+
+def latent_merge_product(work: Tuple[torch.Tensor, torch.Tensor], n_splits: int, w: torch.Tensor, out: torch.Tensor,
+                         head_gate: Optional[torch.Tensor] = None) -> None:
+    """out[t, h] = w[h] . what the slices' parts in `work` come to (see `latent_attention_mfma`): w [heads, n, rank] and out
+    [T, heads, n] bfloat16, rank a multiple of 8 up to 512; with `head_gate` times its sigmoid."""
+    T, heads, n = out.shape
+    rank = w.shape[2]
+    part_o, part_ml = work
+    _need(w.dtype == torch.bfloat16 and out.dtype == torch.bfloat16 and tuple(w.shape) == (heads, n, rank) and w.data_ptr() % 16 == 0
+          and out.stride(2) == 1 and rank % 8 == 0 and rank <= 512, "w [heads, n, rank], out [T, heads, n], bfloat16")
+    _need(part_o.dtype == torch.float32 and part_o.numel() >= T * heads * n_splits * rank and part_ml.dtype == torch.float32
+          and part_ml.numel() >= T * heads * n_splits * 2, "the slices' parts")
+    _call("ix_latent_merge_product", _ptr(part_o), _ptr(part_ml), _i32(n_splits), _ptr(w), out.data_ptr(), _i64(out.stride(0)),
+          _i64(out.stride(1)), _i64(T), _i32(heads), _i32(rank), _i32(n), *_head_gate(head_gate, T, heads, out.dtype), _stream())

@@ -139,32 +139,33 @@ class LatentAttention(Mixer):
         latent = cache.arrays["latent"]
         tiles = self.whole_contexts(ctx, q, cache)
         own = (rt.empty((T, self.rank)), rt.empty((T, self.rot_dim))) if tiles is not None else None
+        q3 = q.unflatten(1, (H, self.q_dim))
+        q_own = q3[:, :, :self.head_dim]
+        few = own is None and self.w_uk_rows is not None and ops.heads_product_fits(q_own, self.w_uk_rows)
+        q_lat = rt.empty((T, H, self.rank)) if few else None
         ops.latent_prepare(q, dkv, self.norm_weight, self.eps, table,
                            ctx.slots[cache.group] if cache.writes else None, latent, H, self.rot_dim, self.rank,
-                           self.halves, own)
-        q3 = q.unflatten(1, (H, self.q_dim))
+                           self.halves, own, (self.w_uk_rows, q_lat) if few else None)
+        y = rt.empty((T, H * self.value_dim))
+        y_heads = y.view(T, H, self.value_dim)
         if own is not None:
-            y = rt.empty((T, H * self.value_dim))
-            ops.latent_whole(q3, rt.linear(own[0], self.w_kv), own[1], tiles, y.view(T, H, self.value_dim), self.scale)
+            ops.latent_whole(q3, rt.linear(own[0], self.w_kv), own[1], tiles, y_heads, self.scale)
             return self.last(rt, y, proj[:, at:], beside)
-        q_own = q3[:, :, :self.head_dim]
-        if self.w_uk_rows is not None and ops.heads_product_fits(q_own, self.w_uk_rows):
-            q_lat = rt.empty((T, H, self.rank))
-            ops.heads_product(q_own, self.w_uk_rows, q_lat)
-        else:
+        if q_lat is None:
             q_lat = torch.bmm(q_own.transpose(0, 1), self.w_uk).transpose(0, 1)  # [T, H, rank]
         if ctx.one_token_each:  # (the slices of a token's keys meet in a contiguous [T, H, rank])
             o_lat = rt.empty((T, H, self.rank)).transpose(0, 1)
         else:
             o_lat = rt.empty((H, T, self.rank))
+        o_own = o_lat.transpose(0, 1)
+        fits = self.w_uv_rows is not None and ops.heads_product_fits(o_own, self.w_uv_rows)
         # (without a rotated part nothing is read of it: any rows will do)
-        self.attend(ctx, q_lat, q3[:, :, self.head_dim:] if self.rot_dim else q_lat, cache, o_lat.transpose(0, 1), gate)
-        y = rt.empty((T, H * self.value_dim))
-        o_own, y_heads = o_lat.transpose(0, 1), y.view(T, H, self.value_dim)
-        if self.w_uv_rows is not None and ops.heads_product_fits(o_own, self.w_uv_rows):
-            ops.heads_product(o_own, self.w_uv_rows, y_heads)
-        else:
-            torch.bmm(o_lat, self.w_uv_t, out=y_heads.transpose(0, 1))
+        if not self.attend(ctx, q_lat, q3[:, :, self.head_dim:] if self.rot_dim else q_lat, cache, o_own, gate,
+                           y_heads if fits else None):
+            if fits:
+                ops.heads_product(o_own, self.w_uv_rows, y_heads)
+            else:
+                torch.bmm(o_lat, self.w_uv_t, out=y_heads.transpose(0, 1))
         return self.last(rt, y, proj[:, at:], beside)
 
     def last(self, rt, y, gate, beside):
@@ -190,12 +191,14 @@ class LatentAttention(Mixer):
             ctx.memo["whole_contexts"] = plan
         return ctx.memo["whole_contexts"]
 
-    def attend(self, ctx, q_lat, q_rot, cache, out, gate=None) -> None:
+    def attend(self, ctx, q_lat, q_rot, cache, out, gate=None, y=None) -> bool:
+        """The weighted sums of latents into `out`; or, where slices of keys are merged and `y` is given (few tokens), their
+        products with the value maps into that: then True."""
         latent, table = cache.arrays["latent"], ctx.block_tables[cache.group]
         if not ops.latent_mfma_fits(q_lat, q_rot, out, self.rank, self.rot_dim):  # float32 runs, other sizes
             ops.latent_attention_plain(q_lat, q_rot, latent, table, ctx.seq_of_token, ctx.positions, out, self.rank,
                                        self.rot_dim, self.scale, self.window, gate)
-            return
+            return False
         rt, T, H = ctx.rt, q_lat.shape[0], self.num_heads
         splits, work = 1, None
         if ctx.one_token_each:
@@ -203,7 +206,12 @@ class LatentAttention(Mixer):
             if splits > 1:
                 work = (rt.empty((T * H * splits, self.rank), torch.float32), rt.empty((T * H * splits, 2), torch.float32))
         ops.latent_attention_mfma(q_lat, q_rot, latent, table, ctx.seq_of_token, ctx.positions, out, self.rank,
-                                  self.rot_dim, self.scale, ctx.one_token_each, splits, work, self.window, gate)
+                                  self.rot_dim, self.scale, ctx.one_token_each, splits, work, self.window, gate,
+                                  y is None or splits == 1)
+        if y is None or splits == 1:
+            return False
+        ops.latent_merge_product(work, splits, self.w_uv_rows, y, gate)
+        return True
 
 
 register_part("mixer", "latent_attention", LatentAttention)

@@ -408,6 +408,54 @@ def test_latent_attention_of_prompts(H, rank, rot, page, window, gated):
     assert torch.isfinite(out).all() and err <= 2e-2, f"{err:.2e}"
 
 
+@pytest.mark.parametrize("T,H,dim,rot,rank", [(1, 1, 32, 0, 16), (8, 16, 128, 64, 512), (16, 3, 160, 32, 96)])
+@pytest.mark.parametrize("halves", [False, True])
+def test_latent_rows_and_the_queries_way_to_them_in_one_launch(T, H, dim, rot, rank, halves):
+    """The same numbers as in two launches."""
+    from inferx_amd import ops
+    q = rnd((T, H * (dim + rot) + rank + rot), 1, 1.0, torch.bfloat16).to(DEV)
+    w, norm = rnd((H, rank, dim), 2, 0.1, torch.bfloat16).to(DEV), rnd((rank,), 3, 1.0, torch.bfloat16).to(DEV)
+    angles = rnd((T, rot // 2, 1), 4, 3.0) if rot else None
+    table = torch.cat([angles.cos(), angles.sin()], 2).float().contiguous().to(DEV) if rot else None
+    slots = torch.arange(T, dtype=torch.int32, device=DEV).flip(0)
+    got = []
+    for fused in (False, True):
+        mine, cache = q.clone(), torch.zeros((2, 1, 16, rank + rot), dtype=torch.bfloat16, device=DEV)
+        out = torch.full((T, H, rank), float("nan"), dtype=torch.bfloat16, device=DEV)
+        rows, d = mine[:, :H * (dim + rot)], mine[:, H * (dim + rot):]
+        ops.latent_prepare(rows, d, norm, 1e-6, table, slots, cache, H, rot, rank, halves, None, (w, out) if fused else None)
+        if not fused:
+            ops.heads_product(rows.unflatten(1, (H, dim + rot))[:, :, :dim], w, out)
+        got.append((mine, cache, out))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T,H,rank,n,splits", [(1, 1, 32, 16, 2), (8, 16, 512, 128, 32), (16, 3, 96, 144, 9), (2, 5, 264, 40, 70)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_slices_of_latents_merged_and_multiplied_in_one_launch(T, H, rank, n, splits, gated):
+    """Some tokens have keys in the first slices only, and NaN where the others' parts would be.  Against float64 on the same
+    numbers: float32 sums of `rank` terms and a result rounded to bfloat16."""
+    from inferx_amd import ops
+    o, m = rnd((T, H, splits, rank), 1, 1.0), rnd((T, H, splits), 2, 3.0)
+    l = rnd((T, H, splits), 3, 1.0).abs() + 0.1
+    for t in range(T):
+        used = 1 + (t * 5) % splits
+        o[t, :, used:], m[t, :, used:], l[t, :, used:] = float("nan"), float("-inf"), 0.0
+    w, gate = rnd((H, n, rank), 4, 0.1, torch.bfloat16), rnd((T, H + 3), 5, 1.0, torch.bfloat16)
+    work = (o.float().contiguous().to(DEV), torch.stack([m, l], 3).float().contiguous().to(DEV))
+    wide = torch.full((T, H * n + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
+    out = wide[:, :H * n].unflatten(1, (H, n))
+    ops.latent_merge_product(work, splits, w.to(DEV), out, gate.to(DEV)[:, 3:] if gated else None)
+    f = torch.exp2(m.double() - m.double().amax(2, keepdim=True))
+    x = (f[..., None] * o.double().nan_to_num()).sum(2) / (f * l.double()).sum(2)[..., None]
+    if gated:
+        x = x * torch.sigmoid(gate[:, 3:].double())[..., None]
+    want = torch.einsum("thr,hnr->thn", x, w.double())
+    bound = 2.0 ** -8 * want.abs() + 2.0 ** -20 * torch.einsum("thr,hnr->thn", x.abs(), w.double().abs())
+    assert ((out.cpu().double() - want).abs() <= bound).all() and torch.isnan(wide[:, H * n:]).all()
+
+
 @pytest.mark.parametrize("H", [1, 3, 16])
 @pytest.mark.parametrize("lengths", [[1, 63, 64, 65], [33, 200, 1, 129], [20], [577, 31]])
 def test_latent_attention_of_whole_contexts(H, lengths):

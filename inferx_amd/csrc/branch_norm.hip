@@ -79,12 +79,18 @@ branch_norm_kernel(float* __restrict__ h, BranchTerms m, const void* __restrict_
   }
 }
 
-__device__ __forceinline__ float4 bn_load4(const void* base, int dtype, int64_t i) {  // i a multiple of 4
-  if (dtype == IX_F32) return *reinterpret_cast<const float4*>(static_cast<const float*>(base) + i);
+// four numbers as they lie in memory (16 bytes of float32, 8 of bfloat16), i a multiple of 4, and opened
+__device__ __forceinline__ uint4 bn_ask4(const void* base, int dtype, int64_t i) {
+  if (dtype == IX_F32) return *reinterpret_cast<const uint4*>(static_cast<const float*>(base) + i);
   const uint2 p = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(base) + i);
-  return make_float4(__uint_as_float(p.x << 16), __uint_as_float(p.x & 0xffff0000u), __uint_as_float(p.y << 16),
-                     __uint_as_float(p.y & 0xffff0000u));
+  return make_uint4(p.x, p.y, 0u, 0u);
 }
+__device__ __forceinline__ float4 bn_open4(const uint4& x, int dtype) {
+  if (dtype == IX_F32) return make_float4(__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z), __uint_as_float(x.w));
+  return make_float4(__uint_as_float(x.x << 16), __uint_as_float(x.x & 0xffff0000u), __uint_as_float(x.y << 16),
+                     __uint_as_float(x.y & 0xffff0000u));
+}
+__device__ __forceinline__ float4 bn_load4(const void* base, int dtype, int64_t i) { return bn_open4(bn_ask4(base, dtype, i), dtype); }
 __device__ __forceinline__ void bn_add4(float4& v, float f, const float4& d) {
   v.x += f * d.x;
   v.y += f * d.y;
@@ -121,7 +127,18 @@ branch_norm_vec4_kernel(float* __restrict__ h, BranchTerms m, const void* __rest
     const int64_t c = 4 * (threadIdx.x + static_cast<int64_t>(u) * blockDim.x);
     v[u] = wa[u] = wb[u] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (c >= width) continue;
+    // Everything is asked for before anything is opened: opened within the branch that asks for it, one number's way from memory
+    // came after the other's (2,048 rows of 2,048 numbers, two branches and a bias, 11.6 us, 12.5 so; eight rows 4.7 and 4.9).
     const float4 old = *reinterpret_cast<const float4*>(hr + c);
+    uint4 ra, rb, rbias, rshared, rw1, rw2, ragain, rstep;
+    if (m.a) ra = bn_ask4(m.a, IX_BF16, row * width + c);
+    if (m.b) rb = bn_ask4(m.b, IX_BF16, row * width + c);
+    if (m.shared) rshared = bn_ask4(m.shared, IX_BF16, row * width + c);
+    if (w1) rw1 = bn_ask4(w1, w1_dtype, c);
+    if (w2) rw2 = bn_ask4(w2, w2_dtype, c);
+    if (m.bias) rbias = bn_ask4(m.bias, m.bias_dtype, c);
+    if (again) ragain = bn_ask4(m.again, m.again_dtype, id * width + c);
+    if (m.step) rstep = bn_ask4(m.step, m.step_dtype, c);
     float4 d = make_float4(0.f, 0.f, 0.f, 0.f);
     if (m.y) {
       const int32_t* dest = m.dest + row * m.k;
@@ -136,18 +153,15 @@ branch_norm_vec4_kernel(float* __restrict__ h, BranchTerms m, const void* __rest
           if (s0 + s < m.k) bn_add4(d, weight[s0 + s], e[s]);
       }
     }
-    if (m.a) bn_add4(d, 1.0f, bn_load4(m.a, IX_BF16, row * width + c));
-    if (m.b) bn_add4(d, 1.0f, bn_load4(m.b, IX_BF16, row * width + c));
-    if (m.bias) bn_add4(d, 1.0f, bn_load4(m.bias, m.bias_dtype, c));
-    if (m.shared) bn_add4(d, sg, bn_load4(m.shared, IX_BF16, row * width + c));
-    if (w1) wa[u] = bn_load4(w1, w1_dtype, c);
-    if (w2) wb[u] = bn_load4(w2, w2_dtype, c);
+    if (m.a) bn_add4(d, 1.0f, bn_open4(ra, IX_BF16));
+    if (m.b) bn_add4(d, 1.0f, bn_open4(rb, IX_BF16));
+    if (m.bias) bn_add4(d, 1.0f, bn_open4(rbias, m.bias_dtype));
+    if (m.shared) bn_add4(d, sg, bn_open4(rshared, IX_BF16));
+    if (w1) wa[u] = bn_open4(rw1, w1_dtype);
+    if (w2) wb[u] = bn_open4(rw2, w2_dtype);
     v[u] = make_float4(old.x + d.x, old.y + d.y, old.z + d.z, old.w + d.w);
-    if (again) {
-      const float4 t = bn_load4(m.again, m.again_dtype, id * width + c);
-      bn_add4(v[u], m.again_scale, t);
-    }
-    if (m.step) bn_add4(v[u], 1.0f, bn_load4(m.step, m.step_dtype, c));
+    if (again) bn_add4(v[u], m.again_scale, bn_open4(ragain, m.again_dtype));
+    if (m.step) bn_add4(v[u], 1.0f, bn_open4(rstep, m.step_dtype));
     if (!rows) *reinterpret_cast<float4*>(hr + c) = v[u];
     sumsq += v[u].x * v[u].x;
     sumsq += v[u].y * v[u].y;

@@ -478,6 +478,31 @@ def attention_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
           _i32(span), _stream())
 
 
+ATTENTION_KEYS_QUERIES = 64
+
+
+def attention_prefill_keys(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor,
+                           tiles: torch.Tensor, positions: torch.Tensor, out: torch.Tensor, scale: float) -> None:
+    """Paged attention for prompt portions (bfloat16, heads of 128, no window) with a tile's keys shared out among the wavefronts
+    (attention_prefill_keys.hip): `tiles` as for attention_mfma, of up to 64 queries of one request, the ones that read most keys
+    first; scale positive."""
+    T, heads, d = q.shape
+    _need(q.dtype == torch.bfloat16 and d == 128, "bfloat16 and heads of 128 only")
+    _need(out.shape == q.shape and out.dtype == q.dtype, "out mismatch")
+    _check_caches(q, k_cache, v_cache)
+    page_size = k_cache.shape[2]
+    _need(block_table.dim() == 2, "block table must be [requests, pages]")
+    _is_i32(block_table)
+    _is_i32(positions, T)
+    _is_i32(tiles)
+    _need(tiles.dim() == 2 and tiles.shape[0] == 3 and tiles.is_contiguous(), "tiles must be int32 [3, n_tiles]")
+    _need(page_size & (page_size - 1) == 0 and page_size >= 16, "this kernel takes pages of a power of two of keys, 16 at least")
+    _need(scale > 0, "scale must be positive")
+    _call("ix_attention_prefill_keys", _ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), _ptr(tiles), _i32(tiles.shape[1]),
+          _ptr(positions), _ptr(out), _i32(heads), _i32(k_cache.shape[1]), _i32(page_size), _i32(block_table.shape[1]), _f32(scale),
+          _stream())
+
+
 ROUTE_SMALL_TOKENS = 128
 
 

@@ -233,9 +233,12 @@ class PagedAttention(Mixer):
                 tile = WIDE_PREFILL_TILE if self.head_dim % 32 == 0 else PREFILL_TILE
                 lds_fits = (self.head_dim <= 128 and page_size & (page_size - 1) == 0
                             and (not special or (turn_back is None and tile == WIDE_PREFILL_TILE)))
-                lds, waves = mixed_step_plan(ctx, self.span, self.num_heads, self.num_kv_heads, lds_fits, tile)
+                by_keys = self.head_dim == 128 and self.span == 0 and lds_fits and not special and self.scale > 0
+                lds, waves = mixed_step_plan(ctx, self.span, self.num_heads, self.num_kv_heads, lds_fits, tile, by_keys)
                 table = ctx.block_tables[cache.group]
-                if lds is not None:
+                if lds is not None and lds[1] is None:
+                    ops.attention_prefill_keys(q, cache.k, cache.v, table, lds[0], ctx.positions, out, self.scale)
+                elif lds is not None:
                     tiles, pairs, slices = lds
                     work = None
                     if slices > 1:
@@ -398,10 +401,39 @@ def serves_group_together(heads: int, kv_heads: int) -> bool:
     return 2 <= heads // kv_heads <= 16
 
 
-def mixed_step_plan(ctx, span: int, heads: int, kv_heads: int, lds_fits: bool = True, tile: int = PREFILL_TILE):
+def _rounds(t: np.ndarray, b) -> np.ndarray:
+    """Rounds of 64 keys that each of the tiles `t` reads where there is no window."""
+    new = (b.q_start[1:] - b.q_start[:-1]).astype(np.int64)
+    first = t[1].astype(np.int64) - b.q_start[:-1].astype(np.int64)[t[0]]
+    return -(-(b.seq_lens.astype(np.int64)[t[0]] - new[t[0]] + first + t[2]) // 64)
+
+
+def keys_pay(rounds: np.ndarray, heads: int, cus: int, slices: int) -> bool:
+    """Whether the kernel that shares out a tile's keys among its wavefronts (ops.attention_prefill_keys, tiles of 64 queries) beats
+    the one with tiles of 128, which would cut its keys into `slices`.  `rounds`: of the tiles of 64, falling.
+
+    With tiles of 128 the step takes as long as the longest tile: 9.3 us and 1.15 a round, 16 at least; with slices 21 and 1.17 a
+    round of a slice.  With tiles of 64 up to two workgroups follow each other on a compute unit, the ones started last on those
+    that are done first: 5.5 us a workgroup and 1.35 for each two rounds.  With more workgroups than that every compute unit is busy to
+    the end either way, and tiles of 128 read keys half as often (16 heads, 4,096 tokens 99 us against 114, 4 prompts of 1,024 42
+    against 53).  Measured, tiles of 128 / of 64, us, 16 heads: a prompt of 128 tokens 16.1 / 9.0, of 512 18.9 / 13.3, of 1,536
+    37.3 / 27.2, of 2,048 46.4 / 36.8; 28 heads on 4: of 1,024 28.8 / 26.7, two portions of 333 on 1,024 keys 48.4 / 40.3, 1,024
+    tokens on 4,096 keys 100 / 109."""
+    units = len(rounds) * heads
+    if units == 0 or units > 2 * cus:
+        return False
+    us = np.repeat(5.5 + 1.35 * (-(-rounds // 2)), heads)
+    ours = us[0] if units <= cus else max(us[0], (us[cus:] + us[2 * cus - units:cus][::-1]).max())
+    theirs = max(16.0, 9.3 + 1.15 * rounds[0]) if slices == 1 else 21.0 + 1.17 * rounds[0] / slices
+    return bool(1.05 * ours < theirs)
+
+
+def mixed_step_plan(ctx, span: int, heads: int, kv_heads: int, lds_fits: bool = True, tile: int = PREFILL_TILE,
+                    by_keys: bool = False):
     """Who serves which requests of a step in which some request brings more than one token: (lds, waves).
 
-    lds = (tiles, pairs, slices) for the LDS-sharing kernel, rows as in the step, or None.  It takes the requests
+    lds = (tiles, pairs, slices) for the LDS-sharing kernel, rows as in the step, or None.  With `by_keys` pairs may be None:
+    then the kernel that shares out a tile's keys takes the tiles, which are its own (see keys_pay).  It takes the requests
     that bring at least PREFILL_MIN_ROWS tokens, in tiles of `tile` queries (64 or 128), if they bring
     PREFILL_MIN_TOKENS together and make enough workgroups (below); slices: into how many workgroups each tile's
     keys are cut.
@@ -416,7 +448,7 @@ def mixed_step_plan(ctx, span: int, heads: int, kv_heads: int, lds_fits: bool = 
     a tile's 64 at work and once per query head (measured at 32 decoding requests with 4,096 keys beside two
     portions of 512, 28 query heads on 4: 487 us per layer; 162 + 57 us in two launches)."""
     reach = abs(span)  # keys that a query reads at most, or 0 for all
-    key = ("attention_mixed", span, heads, kv_heads, lds_fits, tile)
+    key = ("attention_mixed", span, heads, kv_heads, lds_fits, tile, by_keys)
     if key in ctx.memo:
         return ctx.memo[key]
     b = ctx.host
@@ -467,7 +499,16 @@ def mixed_step_plan(ctx, span: int, heads: int, kv_heads: int, lds_fits: bool = 
         # fills a compute unit)
         pairs = _pairs_by_work(t, b, span, pair=not wide and slices == 1 and t.shape[1] * heads >= 2 * cus,
                                slices=slices)
-        lds = (to_dev(t), to_dev(pairs), slices)
+        mine = None
+        if by_keys and wide and t.shape[1] * heads <= cus:
+            mine = _tiles_of(n[seqs], q_start[seqs], seqs, ops.ATTENTION_KEYS_QUERIES)
+            rounds = _rounds(mine, b)
+            order = np.argsort(-rounds, kind="stable")
+            mine = np.ascontiguousarray(mine[:, order]) if keys_pay(rounds[order], heads, cus, slices) else None
+        if mine is not None:
+            lds = (to_dev(mine), None, 1)
+        else:
+            lds = (to_dev(t), to_dev(pairs), slices)
         served = long.copy()
     group = heads // kv_heads
     together = serves_group_together(heads, kv_heads)

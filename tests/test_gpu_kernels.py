@@ -260,6 +260,26 @@ def test_attention_prefill_with_key_slices(tile, index, n_splits, paired):
           f"attention_prefill slices={n_splits}")
 
 
+@pytest.mark.parametrize("seq_lens,q_lens,heads,kv_heads,page", [
+    ([1, 63, 64, 65, 33], [1, 63, 64, 65, 33], 3, 1, 16),            # ends within a tile, a step of 32 keys, a wavefront's share
+    ([700, 129, 300, 95], [100, 129, 1, 64], 28, 4, 32),             # portions on contexts, tiles off their edges
+    ([1500, 20], [1500, 17], 2, 2, 64),
+    ([97, 160], [97, 31], 16, 16, 128)])
+def test_attention_prefill_with_keys_shared_out(seq_lens, q_lens, heads, kv_heads, page):
+    """A tile's keys among the wavefronts; numbers that are not finite in the rest of the cache."""
+    from inferx_amd import ops
+    p = build_paged(seq_lens, q_lens, heads, kv_heads, 128, page, torch.bfloat16, seed=11)
+    table = p["table"].tolist()
+    for s, L in enumerate(seq_lens):
+        if L % page:
+            p["k_cache"][table[s][L // page], :, L % page:] = float("nan")
+            p["v_cache"][table[s][L // page], :, :, L % page:] = float("inf")
+    out = torch.full_like(p["q"], float("nan"))
+    ops.attention_prefill_keys(p["q"], p["k_cache"], p["v_cache"], p["table"], tiles_for(q_lens, 64), p["positions"], out, 128 ** -0.5)
+    close(out, attention_reference(p, seq_lens, q_lens, heads, kv_heads, 128 ** -0.5, 0), TOL[torch.bfloat16],
+          "attention_prefill_keys")
+
+
 @pytest.mark.parametrize("tile", [64, 128])
 def test_attention_prefill_finds_far_keys(tile):
     """Each of a few queries of a long portion matches one key far before it: its output must be that key's value

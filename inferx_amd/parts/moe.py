@@ -50,12 +50,12 @@ WIDE_TILES_ALONE_WIDTH = 2048
 # rows a tile 1.07, with more 0.99, with one 1.03 and 0.98 (64 tokens of 60 experts of 1,408, 8 layers, 2,574 us narrow, 2,541 wide).
 WIDE_TILES_ALONE_WORKGROUPS = 2048
 WIDE_TILES_ALONE_ROWS = 32
-# The wide form's workgroups stay and take tile after tile (where the shapes allow it: `ops.moe_stays`) from so many tokens on, or from so
-# wide rows on.  With less of both a tile is short and waits for its weights alone, and one workgroup a tile, with a stage more
-# on its way, is as good or better.  Whole steps, us, a workgroup for each tile / staying: A2.7B shape, 4 layers, decoding 34 requests 1,098
-# / 1,115, 64 1,213 / 1,252, prompts of 64 tokens 880 / 908, 100 952 / 944, 256 1,176 / 1,118, 512 1,393 / 1,300, 1,024 1,772 / 1,683; 57B
-# shape, 2 layers, portions of 40 tokens 1,600 / 1,560, 128 1,763 / 1,736, 256 1,979 / 1,845.
-STAY_TOKENS, STAY_WIDTH = 96, 3072
+# The wide form's workgroups stay and take tile after tile (where the shapes allow it: `ops.moe_stays`) from so many tokens on.  With
+# fewer a tile is short and waits for its weights alone, and one workgroup a tile, with a stage more on its way, is as good or
+# better.  Whole steps, us, a workgroup for each tile / staying: A2.7B shape, 4 layers, decoding 34 requests 1,098 / 1,115, 64 1,213 /
+# 1,252, prompts of 64 tokens 880 / 908, 100 952 / 944, 256 1,176 / 1,118, 512 1,393 / 1,300, 1,024 1,772 / 1,683; 57B shape, 4 layers,
+# portions of 44 tokens 2,941 / 2,968, 72 3,041 / 3,053, 96 3,071 / 3,067, 128 3,194 / 3,159; 2 layers, 256 1,979 / 1,845.
+STAY_TOKENS = 96
 # Between the few rows of a decoding step (where routed and shared experts already share a launch) and the portions
 # from which the shared expert's library products run beside the routed experts, the shared expert is cut into
 # pieces of the routed experts' width, which every token "chooses" with the shared gate's value as their weight:
@@ -241,7 +241,7 @@ class MoeFeedForward(FeedForward):
         if tile_rows:
             mt, T = ops.moe_max_tiles(A, E, tile_rows), topk_e.shape[0]
             n, second_rows = 2 * mt + 1, T if not always and self._shared_in_the_launches(T) else 0
-            stays = (tile_rows == ops.MOE_TILED_ROWS_WIDE and (T >= STAY_TOKENS or self.hidden_size >= STAY_WIDTH)
+            stays = (tile_rows == ops.MOE_TILED_ROWS_WIDE and T >= STAY_TOKENS
                      and ops.moe_stays(A, E, self.hidden_size, self.expert_width, second_rows, self.shared_width))
             # (the queues of the wide form's two products lie behind the map, on a boundary of eight bytes)
             tile_map = rt.empty((n + 1 + ops.moe_queues_size(mt) if stays else n,), torch.int32)

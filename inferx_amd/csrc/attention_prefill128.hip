@@ -308,8 +308,11 @@ attn_prefill128_kernel(const __bf16* __restrict__ q, const __bf16* k_cache, cons
           for (int b = 0; b < NB2; ++b) va[g][b] = *reinterpret_cast<const bf16x8*>(vs + v_at[g] + 32 * b * VS);
         __builtin_amdgcn_sched_barrier(0);
         // this lane: query qn, keys kb + 32 b + 8 c + 4 h + e for element 4 c + e of s[b]
-        // keys that every query of the wavefront sees need no mask (uniform)
-        const bool inner = wq0 + 32 <= rows && kb + PW_KEYS - 1 <= wfirst && kb >= wlast_lo;
+        // Keys that every query of the wavefront sees need no mask (uniform).  Rows past the tile's last one may see whatever they
+        // like: nothing of them is stored.  (Masked in every round for their sake, a portion's last tile took twice as long, and all
+        // waited for it: two portions of 333 tokens on 2,000 and 1,000 keys, 28 heads on 4, 75 us, 52 so; 400 on
+        // 8,000 135, 97.)
+        const bool inner = kb + PW_KEYS - 1 <= wfirst && kb >= wlast_lo;
         float mx = -INFINITY;
         const float sl = CAP ? 1.0f : scale_log2;  // (capped scores are in units of log2 already)
         if constexpr (CAP) {

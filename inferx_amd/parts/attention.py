@@ -417,8 +417,8 @@ def keys_pay(rounds: np.ndarray, heads: int, cus: int, slices: int) -> bool:
     that are done first: 5.5 us a workgroup and 1.35 for each two rounds.  With more workgroups than that every compute unit is busy to
     the end either way, and tiles of 128 read keys half as often (16 heads, 4,096 tokens 99 us against 114, 4 prompts of 1,024 42
     against 53).  Measured, tiles of 128 / of 64, us, 16 heads: a prompt of 128 tokens 16.1 / 9.0, of 512 18.9 / 13.3, of 1,536
-    37.3 / 27.2, of 2,048 46.4 / 36.8; 28 heads on 4: of 1,024 28.8 / 26.7, two portions of 333 on 1,024 keys 48.4 / 40.3, 1,024
-    tokens on 4,096 keys 100 / 109."""
+    37.3 / 27.2, of 2,048 46.4 / 36.8; 28 heads on 4: of 1,024 28.8 / 26.7, a portion of 333 on 3,000 keys 47.2 / 43.4; not
+    taken: two portions of 333 on 1,024 keys 34.4 / 40.1, 1,024 tokens on 4,096 keys 100 / 109."""
     units = len(rounds) * heads
     if units == 0 or units > 2 * cus:
         return False

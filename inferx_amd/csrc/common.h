@@ -192,9 +192,11 @@ __device__ __forceinline__ float ix_glu(float g, float u, float limit) {
   }
   if constexpr (FAST) {
     // (A workgroup's 48 results a lane take longer than the matrix cores' last two stages, so their instructions count: the divide
-    // is a reciprocal and one step of Newton's, which leaves it an ulp off at most; the largest exponent keeps that step finite.)
-    const float d = 1.0f + __expf(fminf(-steep * g, 88.0f)), r = __builtin_amdgcn_rcpf(d);
-    return g * __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r) * u;
+    // is a reciprocal, one step of Newton's and Markstein's correction of the quotient, which rounds it as a division does; the
+    // largest exponent keeps both finite, and what is not finite is put right by itself.)
+    const float d = 1.0f + __expf(fminf(-steep * g, 88.0f)), y = __builtin_amdgcn_rcpf(d);
+    const float r = __builtin_fmaf(__builtin_fmaf(-d, y, 1.0f), y, y), q = g * r;
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, g), r, q), d, g) * u;
   } else {
     return g / (1.0f + expf(-steep * g)) * u;
   }

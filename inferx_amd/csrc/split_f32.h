@@ -43,7 +43,7 @@ __device__ __forceinline__ void split8(const f32x4& a, const f32x4& b, bf16x8 (&
 }
 
 // The sum of n products in their order.
-static __device__ __attribute__((noinline)) float plain_dot(const float* x, const float* w, int n) {
+__device__ __attribute__((noinline)) float plain_dot(const float* x, const float* w, int n) {
   float sum = 0.f;
   for (int i = 0; i < n; ++i) sum = __builtin_fmaf(x[i], w[i], sum);
   return sum;

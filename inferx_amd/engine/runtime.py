@@ -135,9 +135,8 @@ class Runtime:
             out = self.empty((rows, features), out_dtype)
         return out if ops.linear_tiled(x, w, out, tile) else None
 
-    def _split(self, x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
-               parts: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
-        """The float32 product on the bfloat16 matrix cores, where that kernel takes it.  `parts`: x's, if they are there already."""
+    def _split(self, x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+        """The float32 product on the bfloat16 matrix cores, where that kernel takes it."""
         if not (x.dtype == torch.float32 and w.dtype == torch.float32 and x.shape[0] > self.SKINNY_ROWS and x.is_cuda
                 and x.is_contiguous() and w.is_contiguous() and w.numel() > 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0):
             return None
@@ -147,12 +146,12 @@ class Runtime:
             return None
         if out is None:
             out = self.empty((x.shape[0], w.shape[0]), torch.float32)
-        ops.linear_split(x, w, out, tile, parts)
+        ops.linear_split(x, w, out, tile)
         return out
 
-    def linear(self, x: torch.Tensor, w: torch.Tensor, parts: Optional[torch.Tensor] = None) -> torch.Tensor:
+    def linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """x [T, in] . w[out, in]^T -> [T, out] in the run's type, float32 accumulation.
-        A weight kept in float32 during a bfloat16 run is multiplied in float32.  `parts`: see `_split`."""
+        A weight kept in float32 during a bfloat16 run is multiplied in float32."""
         if w.dtype == x.dtype:
             out = self._tiled(x, w, x.dtype)
             if out is not None:
@@ -166,18 +165,18 @@ class Runtime:
                 out = self.empty((x.shape[0], w.shape[0]))
                 if ops.gemm_bf16(x, w, out):
                     return out
-            out = self._split(x, w, parts=parts)
+            out = self._split(x, w)
             return torch.matmul(x, w.t()) if out is None else out
         return torch.matmul(x.to(torch.float32), w.to(torch.float32).t()).to(self.dtype)
 
     def gated_linear(self, x: torch.Tensor, w_gate_up: torch.Tensor, limit: float = 0.0,
-                     bias: Optional[torch.Tensor] = None, parts: Optional[torch.Tensor] = None) -> torch.Tensor:
+                     bias: Optional[torch.Tensor] = None) -> torch.Tensor:
         """silu(x . Wg^T) * (x . Wu^T) for w_gate_up = [Wg; Wu] of shape [2 n, in] -> [T, n].  `bias` (2 n numbers) is
         added to both products first; with `limit` other than 0 they meet in another form (see `ops.glu_bias`)."""
         from .. import ops
         if self._skinny_ok(x, w_gate_up):
             return self._skinny(x, w_gate_up, True, limit, bias)
-        gate_up = self.linear(x, w_gate_up, parts)
+        gate_up = self.linear(x, w_gate_up)
         act = self.empty((x.shape[0], w_gate_up.shape[0] // 2))
         if bias is None and limit == 0:
             ops.silu_mul(gate_up, act)

@@ -992,30 +992,6 @@ def moe_grouped_tiled_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, o
           _i32(_epilogue(gate_up)), _f32(glu_limit), _stream())
 
 
-def moe_grouped_split(a: torch.Tensor, parts: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offsets: torch.Tensor,
-                      rows: Optional[torch.Tensor], tile_map: torch.Tensor, gate_up, glu_limit: float = 0.0) -> None:
-    """As `moe_grouped_tiled_f32`, on the bfloat16 matrix cores (every number as the sum of three), for widths in multiples of 32;
-    `parts`: `split_rows` of a."""
-    E = w.shape[0]
-    A, n_out = out.shape
-    K = a.shape[1]
-    _need(a.dtype == w.dtype == out.dtype == torch.float32, "this grouped product is float32 only")
-    _need_pieces(a, w, out)
-    _need(w.dim() == 3 and w.shape[2] == K and w.shape[1] == (2 * n_out if _epilogue(gate_up) == GATE_UP_SWIGLU else n_out),
-          "expert weight shape does not fit")
-    _need(parts.dtype == torch.bfloat16 and parts.numel() == 3 * a.numel(), "the parts of other rows")
-    _is_i32(offsets, E + 1)
-    if rows is not None:
-        _is_i32(rows, A)
-    else:
-        _need(a.shape[0] >= A, "a has fewer rows than out")
-    mt = moe_max_tiles(A, E, MOE_TILED_F32_ROWS)
-    _is_i32(tile_map, 2 * mt + 1)
-    _call("ix_moe_grouped_split", _ptr(a), _ptr(parts), _ptr(w), _ptr(out), _ptr(offsets), _ptr(rows), _ptr(tile_map[:mt]),
-          _ptr(tile_map[mt:2 * mt]), _ptr(tile_map[2 * mt:]), _i32(mt), _i64(n_out), _i64(K), _i32(_epilogue(gate_up)),
-          _f32(glu_limit), _stream())
-
-
 def moe_grouped_plain(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offsets: torch.Tensor,
                       rows: Optional[torch.Tensor], gate_up: bool, glu_limit: float = 0.0) -> None:
     """Grouped product over device offsets.  gate_up: a [T, H] gathered through `rows`,

@@ -76,12 +76,6 @@ FOLD_SHARED_WHOLE_BELOW_TOKENS = 11 * ops.MOE_TILED_ROWS_WIDE + 1
 FOLD_SHARED_WHOLE_PIECES = 8
 
 
-# From so many rows an expert on, on average, a float32 run's grouped products go to the bfloat16 matrix cores.  Both products of 60 experts of
-# 1,408 on a width of 2,048, us, float32 instructions / there with the splits of the activations: 150 tokens of four 296 / 307, 256 359 / 339, 400 427 / 376,
-# 511 498 / 437; whole prompts of 256 tokens, 2 layers, 1,541 / 1,551, 400 1,945 / 1,913, 700 2,822 / 2,744.
-SPLIT_ROWS_PER_EXPERT = 20
-
-
 class MoeFeedForward(FeedForward):
     graph_safe = True
 
@@ -249,17 +243,14 @@ class MoeFeedForward(FeedForward):
         ops.moe_dispatch(topk_e, offsets, rows, dest, E, tile_rows, tile_map, queues)
         return offsets, rows, dest, tile_map
 
-    def experts(self, ctx, x, offsets, rows, tile_map=None, tile_rows: int = 0, with_shared: bool = False, shared=None, parts=None):
-        """`parts`: those of x (`ops.split_rows`), with which a float32 run's products go to the bfloat16 matrix cores.  `with_shared`: the grouping holds the shared expert's pieces as further experts.  `shared` [T, hidden]: the shared
+    def experts(self, ctx, x, offsets, rows, tile_map=None, tile_rows: int = 0, with_shared: bool = False, shared=None):
+        """`with_shared`: the grouping holds the shared expert's pieces as further experts.  `shared` [T, hidden]: the shared
         expert's products go into the launches of the wide form and leave their results there."""
         rt, A = ctx.rt, rows.numel()
         w13, w2 = (self.w13_all, self.w2_all) if with_shared else (self.w13, self.w2)
         act = rt.empty((A, self.expert_width))
         y = rt.empty((A, self.hidden_size))
-        if parts is not None:  # a float32 run, many rows per expert
-            ops.moe_grouped_split(x, parts, w13, act, offsets, rows, tile_map, self.first_epilogue, self.limit)
-            ops.moe_grouped_split(act, ops.split_rows(act), w2, y, offsets, None, tile_map, False)
-        elif tile_rows == ops.MOE_TILED_F32_ROWS:  # a float32 run, more than a few rows per expert
+        if tile_rows == ops.MOE_TILED_F32_ROWS:  # a float32 run, more than a few rows per expert
             ops.moe_grouped_tiled_f32(x, w13, act, offsets, rows, tile_map, self.first_epilogue, self.limit)
             ops.moe_grouped_tiled_f32(act, w2, y, offsets, None, tile_map, False)
         elif tile_rows in (ops.MOE_TILED_ROWS, ops.MOE_TILED_ROWS_WIDE):  # many rows per expert: operands staged through LDS
@@ -300,16 +291,9 @@ class MoeFeedForward(FeedForward):
         ops.moe_grouped_dual(act, self.w2, y, offsets, None, tile_map, tile_rows, sact, self.w_shared_down, sout, False)
         return y, sout
 
-    def shared(self, ctx, x, parts=None):
+    def shared(self, ctx, x):
         rt = ctx.rt
-        return rt.linear(rt.gated_linear(x, self.w_shared_gate_up, limit=self.shared_limit, parts=parts), self.w_shared_down)
-
-    def _parts(self, x, tile_rows: int):
-        """The parts of a float32 run's rows where its grouped products go to the bfloat16 matrix cores, or None."""
-        if (tile_rows == ops.MOE_TILED_F32_ROWS and x.shape[0] * self.top_k >= SPLIT_ROWS_PER_EXPERT * self.num_experts
-                and self.hidden_size % 32 == 0 and self.expert_width % 32 == 0):
-            return ops.split_rows(x)
-        return None
+        return rt.linear(rt.gated_linear(x, self.w_shared_gate_up, limit=self.shared_limit), self.w_shared_down)
 
     def route_and_dispatch(self, ctx, x, tile_rows: int, norm=None, always: int = 0):
         """`route` then `dispatch`; for the few tokens of a decoding step in one launch, and the norm before the
@@ -385,12 +369,11 @@ class MoeFeedForward(FeedForward):
         if one_launch:
             y, shared = self.experts_and_shared(ctx, x, offsets, rows, tile_map, tile_rows)
         else:
-            parts = self._parts(x, tile_rows)
-            y = self.experts(ctx, x, offsets, rows, tile_map, tile_rows, parts=parts)
+            y = self.experts(ctx, x, offsets, rows, tile_map, tile_rows)
             if join is not None:
                 join()
             elif self.shared_width > 0:
-                shared = self.shared(ctx, x, parts)
+                shared = self.shared(ctx, x)
         return MoeSum(y, dest, topk_w, shared, gate, self.hidden_size)
 
 

@@ -75,65 +75,3 @@ def test_the_rule_and_the_runtime():
             assert ((got.double() - x.double() @ w.double().T).abs() <= bound(x, w) * 4).all()  # (the library rounds once for four)
     place = torch.empty(511, 4096, device=DEV)
     assert rt.linear_f32(rnd(511, 2048), rnd(4096, 2048, seed=1), place) is place
-
-
-def grouped(counts, seed=1):
-    """offsets, rows, tile map of experts with so many rows, the rows in any order."""
-    from inferx_amd import ops
-    E, A, R = len(counts), sum(counts), ops.MOE_TILED_F32_ROWS
-    g = torch.Generator().manual_seed(seed)
-    topk_e = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(A, generator=g)].to(torch.int32)[:, None].to(DEV)
-    offsets, rows, dest = (torch.empty(n, dtype=torch.int32, device=DEV) for n in (E + 1, A, A))
-    tile_map = torch.empty(2 * ops.moe_max_tiles(A, E, R) + 1, dtype=torch.int32, device=DEV)
-    ops.moe_dispatch(topk_e, offsets, rows, dest, E, R, tile_map)
-    return offsets, rows, tile_map
-
-
-@pytest.mark.parametrize("epilogue", [0, 1, 2])
-@pytest.mark.parametrize("K,n", [(32, 7), (64, 64), (96, 130), (128, 200), (256, 72), (512, 1028), (2048, 96)])
-def test_grouped_split(K, n, epilogue):
-    """Tiles of one and two blocks of rows, whole and not, experts of none, one and several tiles; one to sixty-four stages."""
-    from inferx_amd import ops
-    counts = [1, 32, 33, 64, 65, 0, 130, 5]
-    offsets, rows, tile_map = grouped(counts)
-    A = sum(counts)
-    x, w = rnd(A, K), rnd(len(counts), (2 if epilogue == 1 else 1) * n, K, seed=1, scale=K ** -0.5)
-    buf = torch.full((A * n + 16,), 7.0, device=DEV)
-    out = buf[8:-8].view(A, n)
-    ops.moe_grouped_split(x, ops.split_rows(x), w, out, offsets, rows, tile_map, epilogue)
-    assert (buf[:8] == 7).all() and (buf[-8:] == 7).all()
-    for e, (lo, hi) in enumerate(zip(offsets.tolist(), offsets.tolist()[1:])):
-        xe = x[rows[lo:hi].long()]
-        z, err = xe.double() @ w[e].double().T, bound(xe, w[e])
-        if epilogue == 1:  # silu has slopes up to 1.1
-            want = torch.nn.functional.silu(z[:, :n]) * z[:, n:]
-            err = 1.1 * err[:, :n] * z[:, n:].abs() + z[:, :n].abs() * err[:, n:] + 1.1 * err[:, :n] * err[:, n:]
-        else:
-            want = z.clamp(min=0) ** 2 if epilogue == 2 else z
-            err = 2 * z.abs() * err + err ** 2 if epilogue == 2 else err
-        assert ((out[lo:hi].double() - want).abs() <= err + 8 * 2.0 ** -24 * want.abs() + 1e-37).all()
-    again = torch.empty_like(out)
-    ops.moe_grouped_split(x, ops.split_rows(x), w, again, offsets, rows, tile_map, epilogue)
-    assert torch.equal(out, again)
-    gathered = x[rows.long()].contiguous()
-    ops.moe_grouped_split(gathered, ops.split_rows(gathered), w, again, offsets, None, tile_map, epilogue)
-    assert torch.equal(out, again)
-
-
-@pytest.mark.parametrize("gate_up", [False, True])
-def test_grouped_split_of_infinities(gate_up):
-    from inferx_amd import ops
-    counts = [3, 40]
-    offsets, rows, tile_map = grouped(counts)
-    x, w = rnd(43, 64), rnd(2, 24, 64, seed=1)
-    x[3, 5], x[4, 7], x[6, 1] = float("inf"), float("nan"), 3.4e38
-    w[1, 9, 11], w[0, 12, 0] = float("-inf"), float("nan")
-    out = torch.empty(43, 12 if gate_up else 24, device=DEV)
-    ops.moe_grouped_split(x, ops.split_rows(x), w, out, offsets, rows, tile_map, gate_up)
-    for e, (lo, hi) in enumerate(zip(offsets.tolist(), offsets.tolist()[1:])):
-        z = x[rows[lo:hi].long()] @ w[e].t()
-        want = z[:, :12] / (1 + torch.exp(-z[:, :12])) * z[:, 12:] if gate_up else z
-        assert torch.equal(torch.isnan(out[lo:hi]), torch.isnan(want))
-        assert torch.equal(out[lo:hi][torch.isinf(want)], want[torch.isinf(want)])
-        ok = torch.isfinite(want)
-        assert torch.allclose(out[lo:hi][ok], want[ok], rtol=1e-4, atol=1e-4)

@@ -135,20 +135,6 @@ class Runtime:
             out = self.empty((rows, features), out_dtype)
         return out if ops.linear_tiled(x, w, out, tile) else None
 
-    def _split(self, x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
-        """The float32 product on the bfloat16 matrix cores, where that kernel takes it."""
-        if not (x.dtype == torch.float32 and w.dtype == torch.float32 and x.shape[0] > self.SKINNY_ROWS and x.is_cuda
-                and x.is_contiguous() and w.is_contiguous() and w.numel() > 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0):
-            return None
-        from .. import ops
-        tile = ops.linear_split_tile(x.shape[0], w.shape[0], x.shape[1])
-        if tile < 0:
-            return None
-        if out is None:
-            out = self.empty((x.shape[0], w.shape[0]), torch.float32)
-        ops.linear_split(x, w, out, tile)
-        return out
-
     def linear(self, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         """x [T, in] . w[out, in]^T -> [T, out] in the run's type, float32 accumulation.
         A weight kept in float32 during a bfloat16 run is multiplied in float32."""
@@ -165,8 +151,7 @@ class Runtime:
                 out = self.empty((x.shape[0], w.shape[0]))
                 if ops.gemm_bf16(x, w, out):
                     return out
-            out = self._split(x, w)
-            return torch.matmul(x, w.t()) if out is None else out
+            return torch.matmul(x, w.t())
         return torch.matmul(x.to(torch.float32), w.to(torch.float32).t()).to(self.dtype)
 
     def gated_linear(self, x: torch.Tensor, w_gate_up: torch.Tensor, limit: float = 0.0,
@@ -196,8 +181,7 @@ class Runtime:
             ops.linear_skinny_f32(x, w, out)
             return out
         if x.dtype == torch.float32 and w.dtype == torch.float32:
-            out = self._split(x, w, place)
-            return torch.matmul(x, w.t()) if out is None else out
+            return torch.matmul(x, w.t())
         if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16:
             if x.shape[0] > 0 and x.is_contiguous() and w.is_contiguous():
                 from .. import ops

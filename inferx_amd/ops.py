@@ -794,36 +794,6 @@ def linear_tiled(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, tile: int 
     return rc == 0
 
 
-def linear_split_tile(rows: int, features: int, width: int) -> int:
-    """The tile in which `linear_split` forms a float32 product, or -1 where its rule leaves it to others."""
-    fn = _functions.get("ix_linear_split_tile")
-    if fn is None:
-        fn = _functions["ix_linear_split_tile"] = lib().ix_linear_split_tile
-    return fn(rows, features, width)
-
-
-def split_rows(x: torch.Tensor) -> torch.Tensor:
-    """The three bfloat16 parts of float32 rows x [T, K], K a multiple of 32: [T, K / 32, 3, 32]."""
-    T, K = x.shape
-    _need(x.dtype == torch.float32 and K % 32 == 0, "float32 rows of a multiple of 32 numbers")
-    parts = torch.empty((T, K // 32, 3, 32), dtype=torch.bfloat16, device=x.device)
-    _call("ix_split_rows", _ptr(x), _ptr(parts), _i64(T), _i64(K), _stream())
-    return parts
-
-
-def linear_split(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, tile: int, parts: Optional[torch.Tensor] = None) -> None:
-    """out [T, N] = x [T, K] . w[N, K]^T, all float32 on 16-byte boundaries, K a multiple of 64, on the bfloat16 matrix cores: every number as
-    the sum of three.  `tile`: 0 to 2.  `parts`: `split_rows` of x, if they are there already."""
-    T, K = x.shape
-    N = w.shape[0]
-    _need(x.dtype == w.dtype == out.dtype == torch.float32, "float32 operands and result")
-    _need(w.dim() == 2 and w.shape[1] == K and out.shape == (T, N), "shapes do not fit")
-    if parts is None:
-        parts = split_rows(x)
-    _need(parts.dtype == torch.bfloat16 and parts.numel() == 3 * T * K, "the parts of other rows")
-    _call("ix_linear_split", _ptr(x), _ptr(parts), _ptr(w), _ptr(out), _i64(T), _i64(N), _i64(K), _i32(tile), _stream())
-
-
 def linear_skinny(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate_up: bool = False, glu_limit: float = 0.0,
                   bias: Optional[torch.Tensor] = None) -> None:
     """out [T, N] = x [T, K] . w[N, K]^T for at most 64 rows, all three bfloat16 or all float32.  `gate_up`: w is [2 N, K],

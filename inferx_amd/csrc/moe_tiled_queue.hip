@@ -38,6 +38,7 @@
 #define TQ_LIST 1536                                 // ... of so many
 static_assert(TQ_LIST_AT + 4 * TQ_LIST <= TQ_LDS, "everything fits LDS");
 #define TQ_SECOND 32768  // bit of a list's entry: of the second product
+#define TQ_USED (1 << 30)  // bit of a counter: a launch has been worked by it (and it is at its start again)
 
 // Activations of a tile of NP pairs of sixteens of rows.  (LOADS: of a wavefront a stage, eight rows each.)
 template <int NP> struct XRing {
@@ -389,7 +390,7 @@ __device__ __forceinline__ bool queue_body(Run& run, __bf16* lds, float glu_limi
   return true;
 }
 
-// queue: a counter a die, 0 before the launch, and the number of tiles of experts with more than 128 rows.
+// queue: a counter a die, 0 before the first launch with it, and the number of tiles of experts with more than 128 rows.
 // tiles: the map's, most rows first (see ix_moe_dispatch); places for max_tiles of them.
 template <bool GATE_UP>
 __global__ void __launch_bounds__(TQ_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -433,10 +434,15 @@ moe_grouped_queue_kernel(const __bf16* a, const __bf16* w, __bf16* out, const in
   };
   int got = 0;
   auto fetch = [&]() {
-    if (tid == 0) got = TQ_PLACES / 8 + __hip_atomic_fetch_add(queue + die, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) got = __hip_atomic_fetch_add(queue + die, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
+  // A die's workgroups ask once a pair, n times in all: whoever asks last leaves the counter as the next launch with it needs it.
   auto fetched = [&]() {
-    if (tid == 0) *next_at = got;
+    if (tid == 0) {
+      const int before = got & (TQ_USED - 1);
+      *next_at = TQ_PLACES / 8 + before;
+      if (before == static_cast<int>(n) - 1) __hip_atomic_store(queue + die, TQ_USED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   };
   auto take = [&](Work& next) {
     const unsigned i = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(*next_at));

@@ -900,8 +900,8 @@ def moe_grouped_tiled(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, offse
     consecutive ones of them belong to one expert (any number gives the same results).  `second`: (a, w, out) of a dense
     product out [T, n] = a [T, k] . w^T (gate|up like the grouped one, w then [2 n, k]) in the same launch, with the wide
     form and without last tiles.  `queues`: what `moe_dispatch` made; with
-    them the wide form's workgroups stay and take one tile after the other (the same results).  `nth`: 0 or 1, whether the
-    first or the second product with them (each once)."""
+    them the wide form's workgroups stay and take one tile after the other (the same results).  `nth`: 0 or 1, which of the
+    queues (a launch leaves its queue as it found it; launches that may overlap need one each)."""
     E = w.shape[0]
     A, n_out = out.shape
     K = a.shape[1]

@@ -537,6 +537,22 @@ def test_grouped_tiled_with_a_second_product_by_workgroups_that_stay(rows, n, k,
         assert torch.isfinite(a).all() and torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
+@pytest.mark.parametrize("counts", [[193, 400, 70, 1, 64, 0, 130] * 3, [5, 200]])  # more pairs than places, and fewer
+def test_workgroups_that_stay_can_be_launched_again(counts):
+    """A launch leaves its counters at their start: the same product again, and another of another number of pairs, by the same queue."""
+    from inferx_amd import ops
+    E, T, H, mi = len(counts), sum(counts), 256, 1544
+    topk_e = torch.repeat_interleave(torch.arange(E), torch.tensor(counts)).to(torch.int32)[:, None].to(DEV)
+    offsets, rows, tile_map, queues = with_queue(topk_e, E)
+    x = rnd(T, H, dtype=torch.bfloat16)
+    for epilogue, n in ((True, mi), (True, mi), (False, 520), (False, 520)):
+        w = rnd(E, (2 if epilogue else 1) * n, H, seed=2, dtype=torch.bfloat16, scale=H ** -0.5)
+        got, want = (torch.full((T, n), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+        ops.moe_grouped_tiled(x, w, want, offsets, rows, tile_map, epilogue, True)
+        ops.moe_grouped_tiled(x, w, got, offsets, rows, tile_map, epilogue, True, queues=queues)
+        assert torch.isfinite(want).all() and torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T", [1, 8, 17, 64])
 # at most 256 blocks of sixteen, and more; at most 128 (both halves of an even reduction in one block for up to eight rows)

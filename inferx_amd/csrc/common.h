@@ -192,10 +192,10 @@ __device__ __forceinline__ float ix_glu(float g, float u, float limit) {
   }
   if constexpr (FAST) {
     // (A workgroup's 48 results a lane take longer than the matrix cores' last two stages, so their instructions count: the divide
-    // is a reciprocal, one step of Newton's and Markstein's correction of the quotient, which rounds it as a division does; the
-    // largest exponent keeps both finite, and what is not finite is put right by itself.)
-    const float d = 1.0f + __expf(fminf(-steep * g, 88.0f)), y = __builtin_amdgcn_rcpf(d);
-    const float r = __builtin_fmaf(__builtin_fmaf(-d, y, 1.0f), y, y), q = g * r;
+    // is a reciprocal, one step of Newton's and Markstein's correction of the quotient, which rounds it as a division does.  The
+    // reciprocal is an eighth's, whose own stays normal up to the largest sum; infinities and NaN come out as a division has them.)
+    const float d = 1.0f + __expf(-steep * g), eighth = d * 0.125f, y = __builtin_amdgcn_rcpf(eighth);
+    const float r = __builtin_fmaf(__builtin_fmaf(-eighth, y, 1.0f), y, y) * 0.125f, q = g * r;
     return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, g), r, q), d, g) * u;
   } else {
     return g / (1.0f + expf(-steep * g)) * u;

@@ -537,6 +537,50 @@ def test_grouped_tiled_with_a_second_product_by_workgroups_that_stay(rows, n, k,
         assert torch.isfinite(a).all() and torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
+@pytest.mark.parametrize("kind", ["unit", "few rows", "few rows of experts", "tiles", "wide tiles", "staying"])
+def test_gates_at_the_ends_of_their_range(kind):
+    """The gated unit where the exponential's sum is largest, past the largest and not a number: what the division of 32-bit numbers
+    gives, up to the exponential's own error and one rounding to bfloat16."""
+    from inferx_amd import ops
+    bf, H, T = torch.bfloat16, 256, 64
+    gates = [float("-inf"), float("nan"), float("inf"), -3e38, -1e30, -100.0, -88.5, -88.0, -87.5, -87.0, -30.0, -0.0, 1e-3, 90.0, 3e38]
+    g = torch.tensor(gates).repeat_interleave(3).to(bf)
+    u = torch.tensor([1.0, -1e30, 0.5]).repeat(len(gates)).to(bf)
+    n = -(-len(g) // 8) * 8
+    g, u = (torch.cat([t, t.new_ones(n - len(t))]) for t in (g, u))
+    w = torch.zeros(2 * n, H, dtype=bf)
+    w[:, 0] = torch.cat([g, u])
+    x = torch.zeros(T, H, dtype=bf, device=DEV)
+    x[:, 0] = 1
+    w = w.to(DEV)
+    if kind == "unit":
+        out = torch.empty(T, n, dtype=bf, device=DEV)
+        ops.silu_mul(torch.cat([g, u]).to(DEV)[None].repeat(T, 1), out)
+    elif kind == "few rows":
+        out = torch.empty(8, n, dtype=bf, device=DEV)
+        ops.linear_skinny(x[:8], w, out, True)
+    else:
+        topk_e = torch.zeros(T, 1, dtype=torch.int32, device=DEV)
+        out = torch.empty(T, n, dtype=bf, device=DEV)
+        if kind in ("wide tiles", "staying"):
+            offsets, rows, tile_map, queues = with_queue(topk_e, 1)
+            ops.moe_grouped_tiled(x, w[None], out, offsets, rows, tile_map, True, True, queues=queues if kind == "staying" else None)
+        else:
+            R = 16 if kind == "few rows of experts" else ops.MOE_TILED_ROWS
+            offsets, rows, dest = (torch.empty(m, dtype=torch.int32, device=DEV) for m in (2, T, T))
+            tile_map = torch.empty(2 * ops.moe_max_tiles(T, 1, R) + 1, dtype=torch.int32, device=DEV)
+            ops.moe_dispatch(topk_e, offsets, rows, dest, 1, R, tile_map)
+            if R == 16:
+                ops.moe_grouped_mfma(x, w[None], out, offsets, rows, tile_map, R, True, 4)
+            else:
+                ops.moe_grouped_tiled(x, w[None], out, offsets, rows, tile_map, True, False)
+    want = (g.float() / (1 + torch.exp(-g.float())) * u.float()).to(bf).float().expand(out.shape)
+    got = out.cpu().float()
+    ends = ~torch.isfinite(want)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got[ends].nan_to_num(), want[ends].nan_to_num())
+    assert ((got - want).abs()[~ends] <= 2.0 ** -7 * want.abs()[~ends]).all()
+
+
 @pytest.mark.parametrize("counts", [[193, 400, 70, 1, 64, 0, 130] * 3, [5, 200]])  # more pairs than places, and fewer
 def test_workgroups_that_stay_can_be_launched_again(counts):
     """A launch leaves its counters at their start: the same product again, and another of another number of pairs, by the same queue."""

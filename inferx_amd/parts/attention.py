@@ -401,16 +401,14 @@ def serves_group_together(heads: int, kv_heads: int) -> bool:
     return 2 <= heads // kv_heads <= 16
 
 
-def _rounds(t: np.ndarray, b) -> np.ndarray:
-    """Rounds of 64 keys that each of the tiles `t` reads where there is no window."""
-    new = (b.q_start[1:] - b.q_start[:-1]).astype(np.int64)
-    first = t[1].astype(np.int64) - b.q_start[:-1].astype(np.int64)[t[0]]
-    return -(-(b.seq_lens.astype(np.int64)[t[0]] - new[t[0]] + first + t[2]) // 64)
+def _keys_us(rounds: int) -> float:
+    """What a workgroup of ops.attention_prefill_keys takes for a tile that reads so many rounds of 64 keys (see keys_pay)."""
+    return 5.5 + 1.35 * -(-rounds // 2)
 
 
-def keys_pay(rounds: np.ndarray, heads: int, cus: int, slices: int) -> bool:
+def keys_pay(rounds: List[int], heads: int, cus: int, slices: int) -> bool:
     """Whether the kernel that shares out a tile's keys among its wavefronts (ops.attention_prefill_keys, tiles of 64 queries) beats
-    the one with tiles of 128, which would cut its keys into `slices`.  `rounds`: of the tiles of 64, falling.
+    the one with tiles of 128, which would cut its keys into `slices`.  `rounds`: of 64 keys, of the tiles of 64, falling.
 
     With tiles of 128 the step takes as long as the longest tile: 9.3 us and 1.15 a round, 16 at least; with slices 21 and 1.17 a
     round of a slice.  With tiles of 64 up to two workgroups follow each other on a compute unit, the ones started last on those
@@ -422,10 +420,36 @@ def keys_pay(rounds: np.ndarray, heads: int, cus: int, slices: int) -> bool:
     units = len(rounds) * heads
     if units == 0 or units > 2 * cus:
         return False
-    us = np.repeat(5.5 + 1.35 * (-(-rounds // 2)), heads)
-    ours = us[0] if units <= cus else max(us[0], (us[cus:] + us[2 * cus - units:cus][::-1]).max())
     theirs = max(16.0, 9.3 + 1.15 * rounds[0]) if slices == 1 else 21.0 + 1.17 * rounds[0] / slices
-    return bool(1.05 * ours < theirs)
+    ours = _keys_us(rounds[0])  # of the first workgroup, which ends no later than any that nobody follows
+    if 1.05 * ours < theirs:
+        for tile in range(cus // heads, len(rounds)):
+            # its last workgroup, which follows the longest one that any of its workgroups does
+            last = min((tile + 1) * heads, units) - 1
+            ours = max(ours, _keys_us(rounds[tile]) + _keys_us(rounds[(2 * cus - 1 - last) // heads]))
+    return 1.05 * ours < theirs
+
+
+def _keys_tiles(new: List[int], seen: List[int], first_row: List[int], seqs: List[int], heads: int, cus: int,
+                slices: int) -> Optional[np.ndarray]:
+    """The tiles of ops.attention_prefill_keys for requests that bring `new` tokens and have `seen` with them, those that read most
+    keys first (int32 [3, tiles] = request, first row, rows), or None where the kernel with tiles of 128 takes them.  In plain
+    numbers, and the tiles only where they may be taken, as the step's first layer waits for its plan.  On the host, us, the whole plan
+    with both kernels' tiles made as arrays and the choice after that / so: one prompt of 512 tokens 103 / 29, of 2,048 109 / 57, 512
+    tokens on 8,000 keys (not taken) 111 / 70, two portions of 333 beside 16 tokens (not taken) 174 / 136."""
+    size, units = ops.ATTENTION_KEYS_QUERIES, heads * sum(-(-n // ops.ATTENTION_KEYS_QUERIES) for n in new)
+    longest = -(-max(seen) // 64)
+    if units > 2 * cus or not keys_pay([longest], 1, cus, slices):
+        return None
+    if units > cus:  # two workgroups follow each other at least, of the shortest tiles that there are
+        shortest = -(-min(L - n + min(size, n) for n, L in zip(new, seen)) // 64)
+        if not keys_pay([longest, shortest, shortest], 1, 2, slices):
+            return None
+    tiles = sorted(((-(-(L - n + min(at + size, n)) // 64), s, row + at, min(size, n - at))
+                    for n, L, row, s in zip(new, seen, first_row, seqs) for at in range(0, n, size)), key=lambda t: -t[0])
+    if not keys_pay([t[0] for t in tiles], heads, cus, slices):
+        return None
+    return np.ascontiguousarray(np.array(tiles, dtype=np.int32).T[1:])
 
 
 def mixed_step_plan(ctx, span: int, heads: int, kv_heads: int, lds_fits: bool = True, tile: int = PREFILL_TILE,
@@ -458,7 +482,8 @@ def mixed_step_plan(ctx, span: int, heads: int, kv_heads: int, lds_fits: bool = 
     to_dev = lambda a: ops.upload(a, dev)
     long = n >= PREFILL_MIN_ROWS
     seqs = np.flatnonzero(long)
-    t = _tiles_of(n[seqs], q_start[seqs], seqs, tile) if (lds_fits and len(seqs)) else None
+    new, seen = n[seqs].tolist(), b.seq_lens[seqs].tolist()
+    n_tiles = sum(-(-m // tile) for m in new) if lds_fits else 0
     # The LDS-sharing kernel walks a tile's keys in one workgroup.  With few tiles that leaves compute units idle
     # however long the context is (128 queries of 16 heads on 30,000 keys: 638 us in 32 workgroups).  Then, from
     # about 6,000 keys on, every tile's keys are cut into slices with a workgroup each, about a thousand in all and
@@ -469,45 +494,42 @@ def mixed_step_plan(ctx, span: int, heads: int, kv_heads: int, lds_fits: bool = 
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
     slices = 1
     wide = tile == WIDE_PREFILL_TILE
-    if t is not None and wide:
+    if n_tiles and wide:
         # Tiles of 128 queries: a workgroup fills a compute unit, so what counts is a workgroup per compute unit.
         # With fewer (tile, head) pairs than that, the keys are cut into as many slices as make them up, none under
         # eight rounds of 64 keys, 32 at most (64 tokens of 16 heads on 8,192 keys: 25 us in 16 slices against 141
         # in one; 1,024 tokens of 28 heads on 30,000 keys, 224 pairs: one slice is best).
-        keys = int(b.seq_lens[seqs].max())
+        keys = max(seen)
         rounds = -(-(min(keys, reach + tile) if reach else keys) // 64)
-        slices = max(1, min(cus // (t.shape[1] * heads), rounds // PREFILL_SLICE_ROUNDS, 32))
+        slices = max(1, min(cus // (n_tiles * heads), rounds // PREFILL_SLICE_ROUNDS, 32))
         slices = 1 << (slices.bit_length() - 1)
-    elif t is not None and t.shape[1] * heads < 8 * cus:
-        keys = int(b.seq_lens[seqs].max())
+    elif n_tiles and n_tiles * heads < 8 * cus:
+        keys = max(seen)
         rounds = -(-(min(keys, reach + PREFILL_TILE) if reach else keys) // 64)
         if rounds >= PREFILL_SLICED_MIN_ROUNDS:
             # (with two to eight workgroups per compute unit a few slices still even out what the compute units
             # get: 2,048 queries of 28 heads on 30,000 keys, 896 workgroups, 1.53 against 1.73 ms in four slices)
-            want = (4 if t.shape[1] * heads < 2 * cus else 16) * cus
-            slices = max(1, min(want // (t.shape[1] * heads), rounds // PREFILL_SLICE_ROUNDS, 64))
+            want = (4 if n_tiles * heads < 2 * cus else 16) * cus
+            slices = max(1, min(want // (n_tiles * heads), rounds // PREFILL_SLICE_ROUNDS, 64))
             slices = 1 << (slices.bit_length() - 1)
     lds = None
     served = np.zeros(len(n), dtype=bool)
-    if t is not None and int(n[long].sum()) >= PREFILL_MIN_TOKENS and \
-            (wide or slices > 1 or t.shape[1] * heads >= PREFILL_MIN_WORKGROUPS):
-        # Two workgroups fit a compute unit.  Pairs only when that still leaves two per compute unit: with fewer,
-        # a workgroup per tile keeps two wavefronts on a SIMD instead of one (measured: two portions of 512 on 28
-        # heads, 448 tiles, 15.2 against 15.8 ms for a step of 8 layers; 2,048 tokens on 16 heads, 512 tiles, 15.5
-        # against 15.4 ms for 24 layers).
-        # (tiles of 128 queries are never paired: the workgroups are started in the order of falling work, and one
-        # fills a compute unit)
-        pairs = _pairs_by_work(t, b, span, pair=not wide and slices == 1 and t.shape[1] * heads >= 2 * cus,
-                               slices=slices)
-        mine = None
-        if by_keys and wide and t.shape[1] * heads <= cus:
-            mine = _tiles_of(n[seqs], q_start[seqs], seqs, ops.ATTENTION_KEYS_QUERIES)
-            rounds = _rounds(mine, b)
-            order = np.argsort(-rounds, kind="stable")
-            mine = np.ascontiguousarray(mine[:, order]) if keys_pay(rounds[order], heads, cus, slices) else None
-        if mine is not None:
-            lds = (to_dev(mine), None, 1)
+    if n_tiles and sum(new) >= PREFILL_MIN_TOKENS and (
+            wide or slices > 1 or n_tiles * heads >= PREFILL_MIN_WORKGROUPS):
+        own = None
+        if by_keys and wide and n_tiles * heads <= cus:
+            own = _keys_tiles(new, seen, q_start[seqs].tolist(), seqs.tolist(), heads, cus, slices)
+        if own is not None:
+            lds = (to_dev(own), None, 1)
         else:
+            # Two workgroups fit a compute unit.  Pairs only when that still leaves two per compute unit: with fewer,
+            # a workgroup per tile keeps two wavefronts on a SIMD instead of one (measured: two portions of 512 on 28
+            # heads, 448 tiles, 15.2 against 15.8 ms for a step of 8 layers; 2,048 tokens on 16 heads, 512 tiles, 15.5
+            # against 15.4 ms for 24 layers).
+            # (tiles of 128 queries are never paired: the workgroups are started in the order of falling work, and one
+            # fills a compute unit)
+            t = _tiles_of(n[seqs], q_start[seqs], seqs, tile)
+            pairs = _pairs_by_work(t, b, span, pair=not wide and slices == 1 and n_tiles * heads >= 2 * cus, slices=slices)
             lds = (to_dev(t), to_dev(pairs), slices)
         served = long.copy()
     group = heads // kv_heads

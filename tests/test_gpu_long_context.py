@@ -151,7 +151,8 @@ STEP_CASES = [
     (28, 4, 128, 0, [200], [32048], "portion in slices"),
     (16, 16, 128, 0, [2048] * 8, [30000, 2048, 9000, 30000, 16000, 30000, 22000, 30000], "portion in tiles"),
     (16, 16, 80, 0, [2048] * 4, [30000, 2048, 9000, 16000], "portions in pairs"),
-    (28, 4, 128, 0, [1] * 32 + [512, 512], [4096] * 32 + [4096, 8192], "portions beside grouped tokens"),
+    (28, 4, 128, 0, [1] * 32 + [512, 512], [4096] * 32 + [4096, 8192],
+     "portions' keys shared out beside grouped tokens"),
     (16, 16, 128, 4096, [2048, 1], [20000, 30000], "portion and a token, window"),
 ]
 
@@ -163,7 +164,7 @@ def test_steps_on_long_contexts_through_the_part(heads, kv, d, window, q_lens, s
     from inferx_amd.config import PartSpec
     from inferx_amd.engine.runtime import CacheBinding, Runtime
     from inferx_amd.parts import attention, build_part
-    from test_gpu_parts import make_ctx
+    from test_gpu_parts import make_ctx, plan_of
     rt = Runtime("bfloat16")
     page = 16
     part = build_part("mixer", PartSpec("attention", {"hidden_size": 64, "num_heads": heads, "num_kv_heads": kv,
@@ -180,15 +181,14 @@ def test_steps_on_long_contexts_through_the_part(heads, kv, d, window, q_lens, s
         _, _, n_splits, grouped = attention.query_tiles(ctx, window, heads, d, kv)
         assert grouped == expect.startswith("grouped") and f"{n_splits} slices" in expect, (n_splits, grouped)
     else:
-        tile = attention.WIDE_PREFILL_TILE if d % 32 == 0 else attention.PREFILL_TILE
-        lds, waves = attention.mixed_step_plan(ctx, window, heads, kv, True, tile)
+        lds, waves = plan_of(ctx)
         if expect == "portion in slices":
             assert lds[2] > 1 and not waves
         elif expect == "portion in tiles":
             assert lds[2] == 1 and int(lds[1][1].max()) < 0 and not waves
         elif expect == "portions in pairs":
             assert lds[2] == 1 and int(lds[1][1].max()) >= 0 and not waves
-        elif expect == "portions beside grouped tokens":
-            assert lds is not None and len(waves) == 1 and waves[0][4]
+        elif expect == "portions' keys shared out beside grouped tokens":
+            assert lds[1] is None and len(waves) == 1 and waves[0][4]
         else:
             assert lds is not None and len(waves) == 1

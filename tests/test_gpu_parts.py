@@ -40,6 +40,12 @@ def make_ctx(rt, q_lens, seq_lens, page_size, pages, groups=1):
                        one_token_each=batch.one_token_each), batch
 
 
+def plan_of(ctx):
+    """The plan that `PagedAttention.attend` followed, as it left it in the step's context."""
+    plan, = [plan for key, plan in ctx.memo.items() if isinstance(key, tuple) and key[0] == "attention_mixed"]
+    return plan
+
+
 def tensors_for(part, rt, seed=0, std=None):
     out = {}
     for i, p in enumerate(part.param_specs()):
@@ -144,8 +150,8 @@ def test_few_tokens_beside_portions_stay_in_their_rows(heads, kv, sinks, gated):
     out = torch.full_like(p["q"], float("nan"))
     part.attend(ctx, p["q"], CacheBinding(group=0, arrays=dict(k=p["k_cache"], v=p["v_cache"])), out,
                 gate=gate.to(DEV) if gated else None)
-    lds, waves = attention.mixed_step_plan(ctx, 0, heads, kv, True, attention.WIDE_PREFILL_TILE)
-    assert lds is not None and [w[4] for w in waves] == ([True, False] if heads > kv else [False])
+    lds, waves = plan_of(ctx)
+    assert lds is not None and (lds[1] is None) == (not sinks and not gated) and [w[4] for w in waves] == ([True, False] if heads > kv else [False])
     assert all(w[0] is None and w[3] == 1 for w in waves)
     row = 0
     for (k, v), q, L, n in zip(p["dense"], p["qs"], seq_lens, q_lens):
@@ -162,8 +168,10 @@ def test_few_tokens_beside_portions_stay_in_their_rows(heads, kv, sinks, gated):
 
 @pytest.mark.parametrize("heads,kv,d,window,q_lens,seq_lens,expect", [
     (16, 16, 128, 0, [128], [7000], "slices"),                  # few tiles on a long context: keys in slices
-    (28, 4, 128, 0, [1, 300, 1, 2], [5000, 6500, 900, 40], "slices, grouped beside"),  # ... beside requests of one
+    (28, 4, 128, 0, [1, 300, 1, 2], [5000, 9000, 900, 40], "slices, grouped beside"),  # ... beside requests of one
                                                                 # and two tokens, served per key/value head
+    (28, 4, 128, 0, [1, 300, 1, 2], [5000, 6500, 900, 40], "keys, grouped beside"),  # ... a tile's keys shared out
+    (16, 16, 128, 0, [700], [700], "keys"),
     (16, 16, 48, 0, [130, 1], [400, 77], "one kernel"),         # few tiles of 64, short context
     (16, 16, 64, 0, [130, 1], [400, 77], "portion and tokens"), # (a head of two 32s: a tile of 128 and a token beside)
     (16, 16, 112, 0, [2100], [2100], "pairs"),                  # many tiles of 64, in pairs
@@ -214,13 +222,11 @@ def test_attention_kernels_chosen_by_the_step(heads, kv, d, window, q_lens, seq_
     out = torch.full_like(q, float("nan"))
     part.attend(ctx, q, CacheBinding(group=0, arrays=dict(k=k_cache.to(DEV), v=v_cache.to(DEV))), out)
     assert err(out, torch.cat(wants)) < 1.5e-2
-    # the plan that attend() followed (memoised in the step's context)
     from inferx_amd.parts import attention
     if expect == "grouped":
         assert attention.query_tiles(ctx, window, heads, d, kv)[3]
     else:
-        tile = attention.WIDE_PREFILL_TILE if d % 32 == 0 else attention.PREFILL_TILE
-        lds, waves = attention.mixed_step_plan(ctx, window, heads, kv, True, tile)
+        lds, waves = plan_of(ctx)
         if expect == "one kernel":
             assert lds is None and len(waves) == 1 and waves[0][0] is None and not waves[0][4]
         elif expect == "two launches":
@@ -233,6 +239,8 @@ def test_attention_kernels_chosen_by_the_step(heads, kv, d, window, q_lens, seq_
             assert lds is not None and lds[2] == 1 and len(waves) == 1 and waves[0][4] == (heads > kv)
         elif expect == "slices":
             assert lds[2] > 1 and not waves
+        elif expect.startswith("keys"):
+            assert lds[1] is None and [w[4] for w in waves] == ([True] if "beside" in expect else [])
         else:
             assert lds[2] > 1 and len(waves) == 1 and waves[0][4]
 

@@ -358,7 +358,9 @@ extern "C" int ix_moe_route(const void* x, int dtype, const void* wr, int wr_dty
 // than one a thread on; up to there the places that nobody needs cost more.  In a step, us with / without: 512 assignments 5.5 / 5.4, 2,044
 // 6.6 / 6.9; over and over on the same assignments, which are near then, 512 5.2 / 4.9, 4,096 6.0 / 5.8, 8,192 7.0 / 7.3, 16,384 10.6 / 11.9.
 #define DW_MANY DW_THREADS
-template <bool MANY>
+// QUEUES: experts by their rows, and the sums over all of them, for the products that follow by workgroups that stay; where none do, the
+// sums would cost 0.6 us (64 tokens of 60 experts, in a step, 6.1 us with them, 5.5 without).
+template <bool MANY, bool QUEUES>
 __global__ void __launch_bounds__(DW_THREADS)
 moe_dispatch_wide_kernel(const int32_t* __restrict__ topk_e, int32_t* __restrict__ offsets,
                          int32_t* __restrict__ rows, int32_t* __restrict__ dest, int64_t assignments, int experts,
@@ -367,7 +369,7 @@ moe_dispatch_wide_kernel(const int32_t* __restrict__ topk_e, int32_t* __restrict
                          int2* __restrict__ tiles) {
   __shared__ int32_t counts[IX_MAX_EXPERTS];
   __shared__ int32_t wave_count[DW_WAVES];
-  __shared__ int32_t part[4][DW_WAVES];
+  __shared__ int32_t part[QUEUES ? 3 : 2][DW_WAVES];
   const int e = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   for (int i = tid; i < experts; i += DW_THREADS) counts[i] = 0;
@@ -385,51 +387,58 @@ moe_dispatch_wide_kernel(const int32_t* __restrict__ topk_e, int32_t* __restrict
       if (v[r] >= 0 && v[r] < experts) atomicAdd(&counts[v[r]], 1);
   }
   __syncthreads();
-  int rows_before = 0, tiles_before = 0, heavy = 0, all = 0;
   const int mine = counts[e];
-  for (int i = tid; i < experts; i += DW_THREADS) {
+  // (the first expert has no rows before it, and adds up the tiles of experts with many rows instead, and all of them)
+  const bool sums = QUEUES && e == 0;
+  int rows_before = 0, tiles_before = 0, all = 0;
+  for (int i = tid; i < (QUEUES ? experts : e); i += DW_THREADS) {
     const int c = counts[i], tiles = tile_rows > 0 ? (c + tile_rows - 1) / tile_rows : 0;
-    rows_before += i < e ? c : 0;
-    tiles_before += (n_queues > 0 ? c > mine || (c == mine && i < e) : i < e) ? tiles : 0;
-    heavy += c > 128 ? tiles : 0;
-    all += tiles;
+    if constexpr (QUEUES) {
+      rows_before += sums ? (c > 128 ? tiles : 0) : i < e ? c : 0;
+      tiles_before += c > mine || (c == mine && i < e) ? tiles : 0;
+      all += tiles;
+    } else {
+      rows_before += c;
+      tiles_before += tiles;
+    }
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     rows_before += __shfl_xor(rows_before, off, 64);
     tiles_before += __shfl_xor(tiles_before, off, 64);
-    heavy += __shfl_xor(heavy, off, 64);
-    all += __shfl_xor(all, off, 64);
+    if (sums) all += __shfl_xor(all, off, 64);
   }
   if (lane == 0) {
     part[0][wave] = rows_before;
     part[1][wave] = tiles_before;
-    part[2][wave] = heavy;
-    part[3][wave] = all;
+    if constexpr (QUEUES) part[2][wave] = all;
   }
   __syncthreads();
-  rows_before = tiles_before = heavy = all = 0;
+  rows_before = tiles_before = all = 0;
 #pragma unroll
   for (int w = 0; w < DW_WAVES; ++w) {
     rows_before += part[0][w];
     tiles_before += part[1][w];
-    heavy += part[2][w];
-    all += part[3][w];
+    if (sums) all += part[2][w];
   }
   const int my_tiles = tile_rows > 0 ? (mine + tile_rows - 1) / tile_rows : 0;
-  if (e == 0 && tid < n_queues) queues[tid] = tid % 9 == 8 ? heavy : 0;
+  if (sums) {
+    if (tid < n_queues) queues[tid] = tid % 9 == 8 ? rows_before : 0;
+    if (tid == 0) tile_info[0] = all;
+    rows_before = 0;
+  }
   if (tid == 0) {
     offsets[e] = rows_before;
     if (e == experts - 1) {
       offsets[experts] = rows_before + mine;
-      if (tile_info) tile_info[0] = all;
+      if (!QUEUES && tile_info) tile_info[0] = tiles_before + my_tiles;
     }
   }
   if (tile_expert)
     for (int i = tid; i < my_tiles; i += DW_THREADS) {
       tile_expert[tiles_before + i] = e;
       tile_row0[tiles_before + i] = rows_before + i * tile_rows;
-      if (tiles) {
+      if constexpr (QUEUES) {
         const int held = min(tile_rows, mine - i * tile_rows), together = min(4, my_tiles - (i & ~3));
         tiles[tiles_before + i] = make_int2(rows_before + i * tile_rows, held | e << 8 | (i & 3) << 19 | (together - 1) << 21 |
                                                                              (my_tiles == 1 ? 1 << 23 : 0));
@@ -496,8 +505,10 @@ extern "C" int ix_moe_dispatch(const int32_t* topk_e, int32_t* offsets, int32_t*
   IX_REQUIRE(experts > 0 && experts <= IX_MAX_EXPERTS, "number of experts must be between 1 and 1024");
   IX_REQUIRE(tile_rows >= 0, "tile_rows must not be negative");
   IX_REQUIRE(tile_rows == 0 || (tile_expert && tile_row0 && tile_info), "tile map buffers needed");
-  hipLaunchKernelGGL(assignments > DW_MANY ? moe_dispatch_wide_kernel<true> : moe_dispatch_wide_kernel<false>, dim3(experts),
-                     dim3(DW_THREADS), 0, stream, topk_e, offsets, rows, dest, assignments, experts, k, tile_rows, tile_expert,
+  const bool many = assignments > DW_MANY;
+  auto* const kernel = n_queues ? (many ? moe_dispatch_wide_kernel<true, true> : moe_dispatch_wide_kernel<false, true>)
+                                : (many ? moe_dispatch_wide_kernel<true, false> : moe_dispatch_wide_kernel<false, false>);
+  hipLaunchKernelGGL(kernel, dim3(experts), dim3(DW_THREADS), 0, stream, topk_e, offsets, rows, dest, assignments, experts, k, tile_rows, tile_expert,
                      tile_row0, tile_info, queues, 9 * n_queues,
                      n_queues ? reinterpret_cast<int2*>(queues + (9 * n_queues + 1) / 2 * 2) : nullptr);
   return ix_check_launch("ix_moe_dispatch");

@@ -44,7 +44,7 @@
 // What bounds it: row by row, the chain of dependent sums of a row (0.33 us a row whatever the chip is doing).  In chunks
 // the chain is 64 times shorter and its step two small products (3.6 us a chunk).  Measured with 16 heads of 128 x 128, one
 // request, all three launches against row by row: 44 against 46 us at 128 rows, 51 against 72 at 200, 68 against 172 at
-// 500, 141 against 474 at 1,437, 177 against 672 at 2,048.  The generalized rule, 32 heads
+// 500, 141 against 474 at 1,437, 176 against 672 at 2,048.  The generalized rule, 32 heads
 // of 64 x 64: 42 against 43 us at 160 rows, 46 against 66 at 256, 169 against 492 at 2,048 (with 32-bit sums 130).
 //
 // A lane's operand of a 16 x 16 x 4 product is one number of row (column) l % 16 at reduction index l / 16.  Operands
@@ -214,8 +214,8 @@ __device__ __forceinline__ void dc_solve(const float* a_s, const float (*t_s)[16
 // A chunk and head takes a workgroup some 30 us whatever else the chip is doing (sums and inner products one behind the other), so
 // three of them share a compute unit: rows stay in LDS as they came, with their factors beside them, and a wavefront solves for
 // two tiles at a time.  All three launches, us, with two workgroups to a compute unit (rows in 32 bits, four tiles) / as it is: 16
-// heads of 128 x 128, 33 chunks (528 workgroups, 16 more than went at once) 177 / 159, 32 chunks 183 / 177, 16 requests of 300
-// rows 355 / 303.
+// heads of 128 x 128, 33 chunks of two requests (528 workgroups, 16 more than went at once) 178 / 160, 32 of one 184 / 176, 16
+// requests of 300 rows 356 / 298.  A lane has 168 registers so and needs 132.
 template <int DIM>
 __global__ void __launch_bounds__(DC_THREADS, 3)
 delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, int64_t q_stride, int64_t k_stride,
@@ -353,13 +353,16 @@ delta_chunks_prepare_kernel(const bf16_t* q, const bf16_t* k, const bf16_t* v, i
   // a wavefront's first tiles of V are asked for before W's, behind which they arrive
   const int tiles = (DIM + vdim) / 16;
   auto ask_v = [&](int t0, unsigned short (&x)[2][4][4]) {
+    // (hidden: the rows' places would otherwise be kept in registers from one time to the next, twenty of them in scratch memory)
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const bf16_t* from = v + row0 * v_stride + head * vdim + 16 * min(t0 + u, tiles - 1) - DIM + m;
+      const bf16_t* from = v + row0 * v_stride + head * vdim + 16 * min(t0 + u, tiles - 1) - DIM + (ln & 15);
 #pragma unroll
       for (int b = 0; b < 4; ++b)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x[u][b][e] = from[min(16 * b + 4 * g + e, n - 1) * v_stride].bits;
+        for (int e = 0; e < 4; ++e) x[u][b][e] = from[min(16 * b + 4 * (ln >> 4) + e, n - 1) * v_stride].bits;
     }
   };
   // ---- the diagonal blocks' inverses: lane (block, column), sixteen steps of substitution

@@ -35,6 +35,15 @@ def kernels(tmp_path):
 @pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
 def test_the_products_kernels_keep_everything_in_registers(tmp_path):
     scratch = kernels(tmp_path)
-    of = {n: b for n, b in scratch.items() if re.search("linear_tiled|moe_grouped_tiled|moe_grouped_mfma|moe_grouped_dual|linear_skinny|qkv_rope_skinny|heads_product", n)}
+    of = {n: b for n, b in scratch.items() if re.search("linear_tiled|moe_grouped_tiled|moe_grouped_mfma|moe_grouped_dual|linear_skinny|qkv_rope_skinny|heads_product|moe_grouped_queue", n)}
     assert len(of) > 40
     assert not any(of.values()), {n: b for n, b in of.items() if b}
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+@pytest.mark.parametrize("names,count", [("attn_prefill_keys", 1), ("latent_whole", 1), ("latent_attn_few", 3), ("latent_merge_product", 1),
+                                         ("latent_prepare_product", 2), ("delta_chunks_|general_chunks_", 18)])
+def test_kernels_of_counted_registers_keep_everything_in_them(tmp_path, names, count):
+    """Those whose waits are counted by hand, or whose launch bounds give a lane just the registers that it needs."""
+    of = {n: b for n, b in kernels(tmp_path).items() if re.search(names, n)}
+    assert len(of) == count and not any(of.values()), of

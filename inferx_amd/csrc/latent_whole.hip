@@ -288,7 +288,9 @@ extern "C" int ix_latent_whole(const void* q, int64_t q_t, int64_t q_h, const vo
                                int n_tiles, void* out, int64_t out_t, int64_t out_h, int64_t tokens, int heads, float scale,
                                hipStream_t stream) {
   IX_REQUIRE(n_tiles >= 0 && heads > 0 && tokens >= 0, "sizes must be positive");
-  IX_REQUIRE(tokens < (1 << 24) && tokens * heads * 512 < (int64_t(1) << 32), "places within keys and values must fit 32 bits");
+  // (a row's number and its bytes are multiplied as numbers of 24 bits)
+  IX_REQUIRE(tokens < (1 << 24) && heads < (1 << 15), "up to 2^24 tokens and 2^15 heads, less one each");
+  IX_REQUIRE(tokens * heads * 512 < (int64_t(1) << 32), "places within keys and values must fit 32 bits");
   IX_REQUIRE((q_t | q_h) % 8 == 0 && (out_t | out_h) % 4 == 0, "rows of queries on 16-byte, of results on 8-byte boundaries");
   IX_REQUIRE(static_cast<int64_t>(n_tiles) * heads < (int64_t(1) << 31), "too many workgroups for one launch");
   if (n_tiles == 0) return 0;

@@ -179,7 +179,7 @@ class LatentAttention(Mixer):
         if (ctx.host is None or ctx.one_token_each or ctx.num_tokens < WHOLE_TOKENS or self.window or self.head_gate
                 or not cache.writes or self.scale <= 0
                 or self.w_kv is None or self.w_in.shape[0] % 8
-                or ctx.num_tokens * self.num_heads * 512 >= 1 << 32):
+                or self.num_heads >= 1 << 15 or ctx.num_tokens * self.num_heads * 512 >= 1 << 32):
             return None
         if "whole_contexts" not in ctx.memo:
             b, plan = ctx.host, None

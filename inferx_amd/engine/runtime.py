@@ -105,7 +105,8 @@ class Runtime:
     def pairs_ok(self, x: torch.Tensor, w: torch.Tensor) -> bool:
         """Whether x . w^T may share a launch with another product of as few rows."""
         from .. import ops
-        return x.dtype == torch.bfloat16 and x.shape[0] <= ops.LINEAR_PAIR_ROWS and self._skinny_ok(x, w)
+        return (x.dtype == torch.bfloat16 and x.shape[0] <= ops.LINEAR_PAIR_ROWS and w.shape[0] < ops.LINEAR_PAIR_FEATURES
+                and self._skinny_ok(x, w))
 
     def _skinny(self, x: torch.Tensor, w: torch.Tensor, gate_up: bool, limit: float = 0.0,
                 bias: Optional[torch.Tensor] = None) -> torch.Tensor:

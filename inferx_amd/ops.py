@@ -822,7 +822,7 @@ def _linear_skinny(x, w, out, gate_up, glu_limit, bias, out_f32: bool = False) -
           _f32(glu_limit), _stream())
 
 
-LINEAR_PAIR_ROWS = 16
+LINEAR_PAIR_ROWS, LINEAR_PAIR_FEATURES = 16, 1 << 24  # up to so many rows, fewer rows of weights
 
 
 def linear_skinny_pair(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, x2: torch.Tensor, w2: torch.Tensor, out2: torch.Tensor,

@@ -19,6 +19,16 @@ def test_products_of_few_rows(dtype, rows, features, reduction, off, streamed):
     assert not rt._skinny_ok(x, w.to(torch.float64))
 
 
+@pytest.mark.parametrize("dtype,rows,features,reduction,pairs", [
+    (torch.bfloat16, 1, 8, 8, True), (torch.bfloat16, 16, 8, 8, True), (torch.bfloat16, 17, 8, 8, False), (torch.bfloat16, 4, 8, 12, False),
+    (torch.float32, 4, 8, 8, False), (torch.bfloat16, 1, (1 << 24) - 1, 8, True), (torch.bfloat16, 1, 1 << 24, 8, False)])
+def test_products_that_may_share_a_launch(dtype, rows, features, reduction, pairs):
+    """Sizes that the launch of two refuses go through launches of their own."""
+    rt = Runtime.__new__(Runtime)
+    x, w = torch.empty(rows, reduction, dtype=dtype, device="meta"), torch.empty(features, reduction, dtype=dtype, device="meta")
+    assert rt.pairs_ok(x, w) == pairs
+
+
 @pytest.mark.parametrize("dtype,heads,dim,rot,vdim,rank,gate,uk,uv", [
     (torch.bfloat16, 4, 64, 32, 48, 96, False, True, True), (torch.float32, 4, 64, 32, 48, 96, False, False, False),
     (torch.bfloat16, 4, 48, 32, 48, 96, False, False, True),   # a reduction of 48

@@ -520,16 +520,24 @@ extern "C" int ix_linear_skinny(const void* x, const void* w, int dtype, void* o
 // Two products of the same few rows' layer that do not need each other, in one launch: out [rows, n_out] = x . w^T as ix_linear_skinny
 // forms it (gate_up, bias, glu_limit) and out2 [rows, n_out2] = x2 [rows, width2] . w2^T, all bfloat16, up to 16 rows.
 //
-// What it saves is a launch's start and its first loads' way from memory, during which the other product's weights arrive.  Eight rows, in a
-// step, us, two launches / one: gate|up of 5,632 beside 3,648 to 10,240 features of 2,048 numbers 19.7 / 14.9, down of 5,632 beside 2,048
-// features of 2,048 12.2 / 9.4.
+// What it saves is a launch's start and its first loads' way from memory, during which the other product's weights arrive: never slower
+// than two launches (one, eight and sixteen rows, 19 pairs of 768 to 14,336 features of 768 to 18,944 numbers, weights from memory).
+// Eights or sixteens, us, one | eight rows, two launches / sixteens / eights:
+//   gated, up to 600 blocks of sixteen together: 88 + 228 of 2,048 numbers 10.7 / 7.6 / 6.7 | 11.9 / 8.7 / 7.4, 176 + 384 14.6 / 11.2 /
+//   10.3 | 16.3 / 11.9 / 10.4, 352 + 228 15.6 / 13.4 / 12.5 | 16.8 / 13.8 / 12.8; more: 256 + 384 16.7 / 11.7 / 11.9 | 17.8 / 12.5 / 12.6,
+//   384 + 384 18.0 / 14.9 / 14.8 | 19.8 / 14.4 / 15.3, 352 + 640 21.0 / 16.9 / 17.1 | 22.4 / 17.3 / 17.7
+//   plain, up to 128 blocks each, as alone: 128 of 5,632 and 128 of 2,048 numbers 9.9 / 8.4 / 7.3 | 11.8 / 9.5 / 9.2, of 11,264 13.6 / 13.5 /
+//   10.8 | 17.5 / 15.8 / 14.0; more: 224 of 18,944 and 224 of 3,584 32.5 / 30.1 / 28.5 | 37.2 / 32.5 / 38.0, 256 of 11,008 and 256 of
+//   4,096 26.2 / 22.7 / 24.7 | 28.5 / 24.5 / 32.1
 extern "C" int ix_linear_skinny_pair(const void* x, const void* w, void* out, const void* bias, int bias_dtype, int64_t n_out,
                                      int64_t width, int gate_up, float glu_limit, const void* x2, const void* w2, void* out2,
                                      int64_t n_out2, int64_t width2, int rows, hipStream_t stream) {
   IX_REQUIRE(rows > 0 && rows <= 16 && n_out > 0 && width > 0 && n_out2 > 0 && width2 > 0, "between 1 and 16 rows, positive sizes");
   IX_REQUIRE(width % 8 == 0 && width2 % 8 == 0, "rows of the reduction must be multiples of 16 bytes");
   IX_REQUIRE(n_out < (1 << 24) && n_out2 < (1 << 24) && width < (1 << 30) && width2 < (1 << 30), "sizes too large");
-  const bool eights = rows <= 8 && (gate_up || (width % 16 == 0 && width2 % 16 == 0));
+  const int64_t sixteens = (n_out + 15) / 16, sixteens2 = (n_out2 + 15) / 16;
+  const bool eights = rows <= 8 && (gate_up ? sixteens + sixteens2 <= 600
+                                            : sixteens <= 128 && sixteens2 <= 128 && width % 16 == 0 && width2 % 16 == 0);
   const int per = eights ? 8 : 16, per2 = eights && !gate_up ? 8 : 16;
   const int blocks = static_cast<int>((n_out + per - 1) / per), blocks2 = static_cast<int>((n_out2 + per2 - 1) / per2);
 #define LAUNCH(GU, KS, H, H2)                                                                                                    \

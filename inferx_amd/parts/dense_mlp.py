@@ -77,7 +77,6 @@ class DenseMlp(FeedForward):
     def down(self, ctx, act):
         return ctx.rt.linear(act, self.w_down)
 
-
     def beside(self, ctx, x):
         """In a step of few rows: this feed-forward as the companion of a mixer that reads the same rows, or None."""
         rt = ctx.rt
@@ -88,8 +87,8 @@ class DenseMlp(FeedForward):
 
 class Beside:
     """A dense feed-forward worked in the launches of a mixer that reads the same rows: its first product with the mixer's `first`,
-    its second with the mixer's `last`, which do not need each other.  For steps of few rows, where every launch counts; the same
-    results as one after the other."""
+    its second with the mixer's `last`, which do not need each other.  For steps of few rows, where every launch counts; the results
+    of one after the other, up to the order of their 32-bit sums (the reduction may be cut among fewer or more wavefronts)."""
 
     def __init__(self, rt, mlp, x):
         self.rt, self.mlp, self.x, self.act, self.out = rt, mlp, x, None, None

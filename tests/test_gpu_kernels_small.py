@@ -510,3 +510,21 @@ def test_two_products_of_few_rows_in_one_launch(n, k, n2, k2, gate_up, rows):
         ops.linear_skinny(x, w, one, bias=bias)
         ops.linear_skinny(x2, w2, two)
         assert torch.equal(out, one) and torch.equal(out2, two)
+
+
+@pytest.mark.parametrize("gate_up,n,k,n2,k2", [(False, 2064, 5632, 2048, 2048), (False, 2048, 2048, 2064, 5632), (False, 4096, 1104, 4096, 1040),
+                                               (True, 5632, 264, 3968, 264), (True, 5632, 264, 3984, 264)])
+def test_pairs_of_products_take_eights_only_where_they_are_quicker(gate_up, n, k, n2, k2):
+    """With more than 128 blocks of sixteen features in either plain product, eight rows are worked as the first of sixteen are: the
+    same bits.  (Eights of plain products cut the reduction in two more.)  Gated ones, whose sums do not change, on both sides of 600."""
+    from inferx_amd import ops
+    bf = torch.bfloat16
+    x, x2 = rnd(16, k, dtype=bf), rnd(16, k2, seed=1, dtype=bf)
+    w, w2 = rnd((2 if gate_up else 1) * n, k, seed=2, dtype=bf, scale=k ** -0.5), rnd(n2, k2, seed=3, dtype=bf, scale=k2 ** -0.5)
+    got = []
+    for rows in (16, 8):
+        out, out2 = torch.full((rows, n), float("nan"), dtype=bf, device=DEV), torch.full((rows, n2), float("nan"), dtype=bf, device=DEV)
+        ops.linear_skinny_pair(x[:rows], w, out, x2[:rows], w2, out2, gate_up)
+        got.append((out[:8], out2[:8]))
+    for a, b in zip(*got):
+        assert torch.isfinite(a).all() and torch.equal(a, b)

@@ -859,7 +859,9 @@ def moe_queues_size(max_tiles: int) -> int:
 MOE_TILED_ALONE = 256
 
 
-MOE_QUEUE_TILES, MOE_QUEUE_PAIRS = 768, 1536  # the tiles, and the longest list of a die's pairs, that a staying workgroup keeps
+# The tiles, and the longest list of a die's pairs, that a staying workgroup keeps.  Of the list, more than an eighth of the pairs: the
+# roundings of three runs of pairs, and the sixteen that may go in halves.
+MOE_QUEUE_TILES, MOE_QUEUE_PAIRS, MOE_QUEUE_MORE = 768, 1536, 3 + 16
 
 
 def moe_tiled_rows(wide: bool) -> int:
@@ -881,7 +883,7 @@ def moe_stays(assignments: int, experts: int, hidden: int, width: int, rows2: in
     tiles = moe_max_tiles(assignments, experts, MOE_TILED_ROWS_WIDE)
     pairs = max(tiles * -(-width // 128) + -(-rows2 // MOE_TILED_ROWS_WIDE) * -(-width2 // 128),
                 (tiles + -(-rows2 // MOE_TILED_ROWS_WIDE)) * -(-hidden // 256))
-    return all(n % 64 == 0 and n >= 256 for n in sizes) and tiles <= MOE_QUEUE_TILES and pairs // 8 + 19 <= MOE_QUEUE_PAIRS
+    return all(n % 64 == 0 and n >= 256 for n in sizes) and tiles <= MOE_QUEUE_TILES and pairs // 8 + MOE_QUEUE_MORE <= MOE_QUEUE_PAIRS
 
 
 def moe_tiled_columns(n_out: int, gate_up: bool) -> int:

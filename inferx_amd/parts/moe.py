@@ -50,12 +50,19 @@ WIDE_TILES_ALONE_WIDTH = 2048
 # rows a tile 1.07, with more 0.99, with one 1.03 and 0.98 (64 tokens of 60 experts of 1,408, 8 layers, 2,574 us narrow, 2,541 wide).
 WIDE_TILES_ALONE_WORKGROUPS = 2048
 WIDE_TILES_ALONE_ROWS = 32
-# The wide form's workgroups stay and take tile after tile (where the shapes allow it: `ops.moe_stays`) from so many tokens on.  With
-# fewer a tile is short and waits for its weights alone, and one workgroup a tile, with a stage more on its way, is as good or
-# better.  Whole steps, us, a workgroup for each tile / staying: A2.7B shape, 4 layers, decoding 34 requests 1,098 / 1,115, 64 1,213 /
-# 1,252, prompts of 64 tokens 880 / 908, 100 952 / 944, 256 1,176 / 1,118, 512 1,393 / 1,300, 1,024 1,772 / 1,683; 57B shape, 4 layers,
-# portions of 44 tokens 2,941 / 2,968, 72 3,041 / 3,053, 96 3,071 / 3,067, 128 3,194 / 3,159; 2 layers, 256 1,979 / 1,845.
+# The wide form's workgroups stay and take tile after tile (where the shapes allow it: `ops.moe_stays`) from so many tokens on.  Whole
+# steps, us, a workgroup for each tile / staying: A2.7B shape, 8 layers, prompts of 48 tokens 1,367 / 1,429, 72 1,450 / 1,455, 100 1,587 /
+# 1,543, 256 1,973 / 1,910, 768 2,775 / 2,647; 64 experts of 1,408 on 2,048 with two pieces, 8 layers, 72 1,487 / 1,541, 100 1,554 / 1,552,
+# 192 1,832 / 1,734; 57B shape, 4 layers, portions of 48 2,880 / 2,883, 96 2,998 / 3,002, 128 3,113 / 3,092; 2 layers, 256 1,979 / 1,845.
 STAY_TOKENS = 96
+# ... as long as the weights of the first product are no more than so many MiB a compute unit, and so many more for each row that a tile
+# has.  A tile of few rows waits for its weights alone, and one workgroup a tile has a stage more of them on its way: what that
+# gains grows with the weights, while staying gains a tile's start and end.  Whole steps again, 100 | 256 | 384 | 768 tokens: 256
+# experts of 2,048 on 4,096 (32 MiB; 4, 9, 13 and 27 rows a tile), 3 layers, 4,375 / 4,679 | 5,585 / 6,057 | 5,922 / 6,407 | 6,660 / 6,841
+# and 1,200 tokens (42 rows) 7,245 / 7,275; 160 of 1,536 on 5,120 (19 MiB; 5, 13, 19, 38), 3 layers, 3,390 / 3,416 | 3,892 / 3,978 | 4,052 /
+# 4,078 | 4,506 / 4,409; 128 of 1,536 on 4,096 (12 MiB; 7, 18, 27, 54), 4 layers, 2,842 / 2,833 | 3,332 / 3,321 | 3,622 / 3,543 | 4,044 /
+# 3,942; 256 of 768 on 2,048 (6 MiB; 4, 9, 13, 27), 6 layers, 1,212 / 1,186 | 1,474 / 1,394 | 1,655 / 1,575 | 2,028 / 1,942.
+STAY_MIB, STAY_MIB_A_ROW = 8.0, 0.625
 # Between the few rows of a decoding step (where routed and shared experts already share a launch) and the portions
 # from which the shared expert's library products run beside the routed experts, the shared expert is cut into
 # pieces of the routed experts' width, which every token "chooses" with the shared gate's value as their weight:
@@ -226,6 +233,12 @@ class MoeFeedForward(FeedForward):
                 and (2 if self.gated else 1) * self.expert_width * self.hidden_size < 1 << 31
                 and ops.moe_max_tiles(A, self.num_experts, 16) < 65536)
 
+    def _staying_pays(self, tokens: int, assignments: int, experts: int) -> bool:
+        """Whether the wide form's workgroups had better stay than be as many as tiles."""
+        tiles = ops.moe_tiled_tiles(assignments, experts)
+        weights = tiles * (4 if self.gated else 2) * self.expert_width * self.hidden_size / ops.MOE_TILED_ALONE
+        return tokens >= STAY_TOKENS and weights <= (STAY_MIB + STAY_MIB_A_ROW * assignments / tiles) * 2 ** 20
+
     def dispatch(self, ctx, topk_e, tile_rows: int = 0, always: int = 0):
         rt, A, E = ctx.rt, topk_e.numel(), self.num_experts + always
         offsets = rt.empty((E + 1,), torch.int32)
@@ -235,7 +248,7 @@ class MoeFeedForward(FeedForward):
         if tile_rows:
             mt, T = ops.moe_max_tiles(A, E, tile_rows), topk_e.shape[0]
             n, second_rows = 2 * mt + 1, T if not always and self._shared_in_the_launches(T) else 0
-            stays = (tile_rows == ops.MOE_TILED_ROWS_WIDE and T >= STAY_TOKENS
+            stays = (tile_rows == ops.MOE_TILED_ROWS_WIDE and self._staying_pays(T, A, E)
                      and ops.moe_stays(A, E, self.hidden_size, self.expert_width, second_rows, self.shared_width))
             # (the queues of the wide form's two products lie behind the map, on a boundary of eight bytes)
             tile_map = rt.empty((n + 1 + ops.moe_queues_size(mt) if stays else n,), torch.int32)

@@ -2072,6 +2072,18 @@ def latent_attention_mfma(q_lat: torch.Tensor, q_rot: torch.Tensor, cache: torch
           *_head_gate(head_gate, T, heads, q_lat.dtype), _stream())
 
 
+def latent_merge_pays(tokens: int, heads: int, n: int, rank: int) -> bool:
+    """Whether `latent_merge_product` beats merging the slices' parts and `heads_product`, each in a launch of its own.
+
+    It reads a head's map once a token, the other way reads it once: one launch pays as long as every token and head has a compute
+    unit, and two workgroups to a unit with maps of 32 KB.  us, two launches / one, 200 | 2,000 keys, values of 128 from a rank of 512 (128 KB):
+    1 token of 16 heads 6.1 / 5.7 | 7.6 / 6.9, 8 of 16 6.9 / 6.1 | 9.6 / 9.4, 16 of 16 7.7 / 6.9 | 8.1 / 7.7, 8 of 32 8.2 / 7.7 | 9.8 / 9.7, 4 of 64
+    9.3 / 8.1 | 11.0 / 12.0; 16 of 32 10.6 / 11.7 | 10.0 / 11.3, 16 of 64 13.8 / 18.6 | 12.4 / 16.4, 16 of 128 15.9 / 28.3 | 15.4 / 26.2.  Values
+    of 64 from 256 (32 KB): 16 of 16 6.9 / 5.4 | 8.0 / 6.4, 16 of 32 7.7 / 7.4 | 9.5 / 8.7, 4 of 128 8.4 / 7.9 | 14.2 / 12.9; 8 of 128 10.8 / 13.3 |
+    14.8 / 16.2."""
+    return tokens * heads <= (512 if n * rank <= 1 << 14 else 256)
+
+
 def latent_merge_product(work: Tuple[torch.Tensor, torch.Tensor], n_splits: int, w: torch.Tensor, out: torch.Tensor,
                          head_gate: Optional[torch.Tensor] = None) -> None:
     """out[t, h] = w[h] . what the slices' parts in `work` come to (see `latent_attention_mfma`): w [heads, n, rank] and out

@@ -192,8 +192,8 @@ class LatentAttention(Mixer):
         return ctx.memo["whole_contexts"]
 
     def attend(self, ctx, q_lat, q_rot, cache, out, gate=None, y=None) -> bool:
-        """The weighted sums of latents into `out`; or, where slices of keys are merged and `y` is given (few tokens), their
-        products with the value maps into that: then True."""
+        """The weighted sums of latents into `out`; or, where slices of keys are merged, `y` is given (few tokens) and one launch for
+        both pays, their products with the value maps into that: then True."""
         latent, table = cache.arrays["latent"], ctx.block_tables[cache.group]
         if not ops.latent_mfma_fits(q_lat, q_rot, out, self.rank, self.rot_dim):  # float32 runs, other sizes
             ops.latent_attention_plain(q_lat, q_rot, latent, table, ctx.seq_of_token, ctx.positions, out, self.rank,
@@ -205,13 +205,12 @@ class LatentAttention(Mixer):
             splits = ops.latent_mfma_splits(T, H)
             if splits > 1:
                 work = (rt.empty((T * H * splits, self.rank), torch.float32), rt.empty((T * H * splits, 2), torch.float32))
+        together = y is not None and splits > 1 and ops.latent_merge_pays(T, H, self.value_dim, self.rank)
         ops.latent_attention_mfma(q_lat, q_rot, latent, table, ctx.seq_of_token, ctx.positions, out, self.rank,
-                                  self.rot_dim, self.scale, ctx.one_token_each, splits, work, self.window, gate,
-                                  y is None or splits == 1)
-        if y is None or splits == 1:
-            return False
-        ops.latent_merge_product(work, splits, self.w_uv_rows, y, gate)
-        return True
+                                  self.rot_dim, self.scale, ctx.one_token_each, splits, work, self.window, gate, not together)
+        if together:
+            ops.latent_merge_product(work, splits, self.w_uv_rows, y, gate)
+        return together
 
 
 register_part("mixer", "latent_attention", LatentAttention)

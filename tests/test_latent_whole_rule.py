@@ -1,4 +1,5 @@
-"""Which steps latent attention works on keys and values of each head's own, and the tiles it makes for them, on the CPU."""
+"""Which steps latent attention works on keys and values of each head's own, the tiles it makes for them, and when slices of keys are
+merged in the launch of the value maps, on the CPU."""
 import types
 
 import numpy as np
@@ -63,3 +64,22 @@ def test_sizes_that_places_within_keys_and_values_hold(heads, tokens, fits):
     assert (part.whole_contexts(step([tokens], [tokens]), None, WRITES) is not None) == fits
     refused = build.load().ix_latent_whole(None, 0, 0, None, None, None, 0, None, 0, 0, tokens, heads, 1.0, None)  # no tiles
     assert (refused == 0) == fits
+
+
+@pytest.mark.parametrize("tokens,heads,n,rank,slices,together", [
+    (1, 16, 128, 512, 32, True), (16, 16, 128, 512, 16, True), (16, 17, 128, 512, 16, False), (2, 128, 128, 512, 32, True),
+    (16, 128, 128, 512, 8, False), (16, 32, 64, 256, 16, True), (16, 33, 64, 256, 16, False), (16, 32, 64, 264, 16, False),
+    (8, 16, 128, 512, 1, False)])
+def test_slices_are_merged_where_their_products_are_formed_only_for_few_pairs(monkeypatch, tokens, heads, n, rank, slices, together):
+    """One workgroup a token and head reads the head's whole map."""
+    part, done = LatentAttention(64, heads, 128, 64, n, rank), []
+    monkeypatch.setattr(ops, "latent_mfma_fits", lambda *a: True)
+    monkeypatch.setattr(ops, "latent_mfma_splits", lambda *a: slices)
+    monkeypatch.setattr(ops, "latent_attention_mfma", lambda *a: done.append(a[-1]))
+    monkeypatch.setattr(ops, "latent_merge_product", lambda *a: done.append("merged"))
+    meta = lambda *shape, dtype=torch.bfloat16: torch.empty(shape, dtype=dtype, device="meta")
+    ctx = step([1] * tokens, [100] * tokens, one_token_each=True, block_tables=[None], seq_of_token=None, positions=None)
+    ctx.rt.empty = lambda shape, dtype: meta(*shape, dtype=dtype)
+    cache = types.SimpleNamespace(arrays={"latent": None}, group=0)
+    got = part.attend(ctx, meta(tokens, heads, rank), None, cache, meta(tokens, heads, rank), None, meta(tokens, heads, n))
+    assert got == together and done == ([False, "merged"] if together else [True])

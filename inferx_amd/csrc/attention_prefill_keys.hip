@@ -6,8 +6,8 @@
 // one request and one head, so there are twice as many tiles with half the work, and its four wavefronts (one a SIMD, 512 registers
 // each) take the steps of 32 keys w, w + 4, .. of them: the structure of latent_whole.hip, where it is explained, on the pages of
 // the cache.  Keys and values are loaded for 64 queries instead of 128, which is what bounds it where there are tiles enough.
-// Tiles of 128 / this, us: 16 heads, a prompt of 128 tokens 16.1 / 9.0, of 1,024 32.8 (in two slices) / 19.4, of 2,048 46.4 / 36.8, of
-// 4,096 98.9 / 113.6 (there the caller stays with tiles of 128).  Error against 64 bits, of the norm, same sizes: 1.90e-3 / 1.87e-3,
+// Tiles of 128 / this, us: 16 heads, a prompt of 130 tokens 11.9 / 9.7, of 1,024 32.5 (in two slices) / 20.0, of 2,048 48.4 / 39.3 (in a
+// step, where weights have passed through the caches since, 54.4 / 46.6), of 4,096 98.9 / 113.6 (there the caller stays with tiles of 128).  Error against 64 bits, of the norm, same sizes: 1.90e-3 / 1.87e-3,
 // 2,048 tokens 2.09e-3 / 2.04e-3.
 #include "common.h"
 #include "lds_loads.h"

@@ -406,32 +406,36 @@ def _keys_us(rounds: int) -> float:
     return 5.5 + 1.35 * -(-rounds // 2)
 
 
-def keys_pay(rounds: List[int], heads: int, cus: int, slices: int) -> bool:
+def keys_pay(rounds: List[int], heads: int, cus: int, slices: int, load: float) -> bool:
     """Whether the kernel that shares out a tile's keys among its wavefronts (ops.attention_prefill_keys, tiles of 64 queries) beats
-    the one with tiles of 128, which would cut its keys into `slices`.  `rounds`: of 64 keys, of the tiles of 64, falling.
+    the one with tiles of 128, which would cut its keys into `slices` and have `load` workgroups a compute unit without slices.
+    `rounds`: of 64 keys, of the tiles of 64, falling.
 
-    With tiles of 128 the step takes as long as the longest tile: 9.3 us and 1.15 a round, 16 at least; with slices 21 and 1.17 a
-    round of a slice.  With tiles of 64 up to two workgroups follow each other on a compute unit, the ones started last on those
-    that are done first: 5.5 us a workgroup and 1.35 for each two rounds.  With more workgroups than that every compute unit is busy to
-    the end either way, and tiles of 128 read keys half as often (16 heads, 4,096 tokens 99 us against 114, 4 prompts of 1,024 42
-    against 53).  Measured, tiles of 128 / of 64, us, 16 heads: a prompt of 128 tokens 16.1 / 9.0, of 512 18.9 / 13.3, of 1,536
-    37.3 / 27.2, of 2,048 46.4 / 36.8; 28 heads on 4: of 1,024 28.8 / 26.7, a portion of 333 on 3,000 keys 47.2 / 43.4; not
-    taken: two portions of 333 on 1,024 keys 34.4 / 40.1, 1,024 tokens on 4,096 keys 100 / 109."""
+    With tiles of 128 the step takes as long as the longest tile: 9.3 us and 1.15 a round, a tenth more of these with a workgroup on every
+    compute unit; with slices 21 and 1.17 a round of a slice.  With tiles of 64 up to two workgroups follow each other on a compute
+    unit, the ones started last on those that are done first: 5.5 us a workgroup and 1.35 for each two rounds, and 4.5 from one to the
+    other.  With more workgroups than that every compute unit is busy to the end either way, and tiles of 128 read keys half as often (16
+    heads, 4,096 tokens 99 us against 114).  Heads that share keys and values take as long as others (32 on 8 and on 32: within 3 %).
+    Measured, tiles of 128 / of 64, us, 16 heads: a prompt of 130 tokens 11.9 / 9.7, of 512 18.5 / 13.6, of 1,536 38.6 / 28.7, of
+    2,048 48.4 / 39.3; 28 heads on 4: of 1,024 30.5 / 28.5, a portion of 333 on 2,000 keys 41.5 / 35.5, on 500 26.0 / 18.8; not
+    taken: four prompts of 256 16.7 / 19.6, eight of 100 14.0 / 17.0, two portions of 333 on 1,024 keys 36.6 / 41.9, 1,024 tokens
+    on 2,048 72.1 / 71.6; 64 heads on 8: one prompt of 384 18.3 / 19.7.  Of 239 steps of ten numbers of heads none that goes here was
+    slower, and none that stays away more than 10 % quicker here."""
     units = len(rounds) * heads
     if units == 0 or units > 2 * cus:
         return False
-    theirs = max(16.0, 9.3 + 1.15 * rounds[0]) if slices == 1 else 21.0 + 1.17 * rounds[0] / slices
+    theirs = 9.3 + 1.15 * (1 + 0.1 * load) * rounds[0] if slices == 1 else 21.0 + 1.17 * rounds[0] / slices
     ours = _keys_us(rounds[0])  # of the first workgroup, which ends no later than any that nobody follows
     if 1.05 * ours < theirs:
         for tile in range(cus // heads, len(rounds)):
             # its last workgroup, which follows the longest one that any of its workgroups does
             last = min((tile + 1) * heads, units) - 1
-            ours = max(ours, _keys_us(rounds[tile]) + _keys_us(rounds[(2 * cus - 1 - last) // heads]))
+            ours = max(ours, _keys_us(rounds[tile]) + 4.5 + _keys_us(rounds[(2 * cus - 1 - last) // heads]))
     return 1.05 * ours < theirs
 
 
-def _keys_tiles(new: List[int], seen: List[int], first_row: List[int], seqs: List[int], heads: int, cus: int,
-                slices: int) -> Optional[np.ndarray]:
+def _keys_tiles(new: List[int], seen: List[int], first_row: List[int], seqs: List[int], heads: int, cus: int, slices: int,
+                load: float) -> Optional[np.ndarray]:
     """The tiles of ops.attention_prefill_keys for requests that bring `new` tokens and have `seen` with them, those that read most
     keys first (int32 [3, tiles] = request, first row, rows), or None where the kernel with tiles of 128 takes them.  In plain
     numbers, and the tiles only where they may be taken, as the step's first layer waits for its plan.  On the host, us, the whole plan
@@ -439,15 +443,15 @@ def _keys_tiles(new: List[int], seen: List[int], first_row: List[int], seqs: Lis
     tokens on 8,000 keys (not taken) 111 / 70, two portions of 333 beside 16 tokens (not taken) 174 / 136."""
     size, units = ops.ATTENTION_KEYS_QUERIES, heads * sum(-(-n // ops.ATTENTION_KEYS_QUERIES) for n in new)
     longest = -(-max(seen) // 64)
-    if units > 2 * cus or not keys_pay([longest], 1, cus, slices):
+    if units > 2 * cus or not keys_pay([longest], 1, cus, slices, load):
         return None
     if units > cus:  # two workgroups follow each other at least, of the shortest tiles that there are
         shortest = -(-min(L - n + min(size, n) for n, L in zip(new, seen)) // 64)
-        if not keys_pay([longest, shortest, shortest], 1, 2, slices):
+        if not keys_pay([longest, shortest, shortest], 1, 2, slices, load):
             return None
     tiles = sorted(((-(-(L - n + min(at + size, n)) // 64), s, row + at, min(size, n - at))
                     for n, L, row, s in zip(new, seen, first_row, seqs) for at in range(0, n, size)), key=lambda t: -t[0])
-    if not keys_pay([t[0] for t in tiles], heads, cus, slices):
+    if not keys_pay([t[0] for t in tiles], heads, cus, slices, load):
         return None
     return np.ascontiguousarray(np.array(tiles, dtype=np.int32).T[1:])
 
@@ -518,7 +522,7 @@ def mixed_step_plan(ctx, span: int, heads: int, kv_heads: int, lds_fits: bool = 
             wide or slices > 1 or n_tiles * heads >= PREFILL_MIN_WORKGROUPS):
         own = None
         if by_keys and wide and n_tiles * heads <= cus:
-            own = _keys_tiles(new, seen, q_start[seqs].tolist(), seqs.tolist(), heads, cus, slices)
+            own = _keys_tiles(new, seen, q_start[seqs].tolist(), seqs.tolist(), heads, cus, slices, n_tiles * heads / cus)
         if own is not None:
             lds = (to_dev(own), None, 1)
         else:

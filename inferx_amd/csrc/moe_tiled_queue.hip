@@ -8,9 +8,9 @@
 // the next pair's first two stages follow it in the ring, with the row numbers, and behind the last operand
 // read everything else of the next pair's start is asked for, so that the results are formed and stored while it arrives.
 // By time stamps a pair takes 26 to 40 us now of the 29 to 45 from one start on a place to the next; the rest of it is the reduction, which the
-// memory's rate bounds for few rows and the card's power for many.  Launches of 2,048 tokens in 60 experts of 1,408 beside a shared one: 256 + 132
-// -> 231 + 128 us; 64 experts of 2,560 beside eight pieces, 512 tokens: 538 + 302 -> 484 + 284; whole steps 3 to 6 % (a prompt of 2,048
-// 4,630 -> 4,448 us at 8 layers, 16 decodes beside two portions of 333 4,702 -> 4,434 at 4).  Pairs dealt out beforehand, every 32nd to
+// memory's rate bounds for few rows and the card's power for many.  Gate|up + down in a step, a workgroup for each pair -> so: 2,048 tokens in 60
+// experts of 1,408 beside a shared one 261 + 135 -> 247 + 130 us, 340 tokens beside four pieces 127 + 76 -> 122 + 72; 64 experts of 2,560
+// beside eight pieces, 512 tokens 547 + 305 -> 520 + 297, 682 tokens 603 + 341 -> 588 + 334.  Pairs dealt out beforehand, every 32nd to
 // a workgroup, instead of from a counter would lose most of that: they take 27 to 100 us.  Taken at the start of the pair before
 // instead of at its end, the next pair waited behind one of 100 us while other places were empty (down 126 -> 134 us).
 //
